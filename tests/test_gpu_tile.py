@@ -1,0 +1,122 @@
+"""The tiled products of prompt-sized steps (csrc/gemm_tile.hip) against 64-bit ones, at the edges of their tiles: rows and columns
+that fill no tile, the shortest K, the last part of a split K shorter than the others, every tile shape the rule chooses."""
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from tokenmill_amd.hip.library import library
+
+pytestmark = pytest.mark.gpu
+P, I = ctypes.c_void_p, ctypes.c_int
+
+# (rows, result columns, K): with those below they reach every tile
+SILU = [(65, 8, 256), (77, 4864, 320), (129, 1000, 256), (200, 4864, 256), (257, 4864, 448), (333, 4864, 256), (512, 4864, 896), (1000, 6000, 448),
+        (700, 4864, 448), (1000, 4864, 896), (2048, 4864, 896), (4001, 4864, 896), (2000, 4096, 1792), (1025, 40, 256)]
+
+
+def _operands(M, N, K, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    a = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    return a, w, a.double() @ w.double().T
+
+
+def _stream():
+    return P(torch.cuda.current_stream().cuda_stream)
+
+
+def test_the_sizes_below_reach_every_tile():
+    lib = library()
+    shapes = {lib.tm_gemm_tile_shape(M, 2 * n, K, 1) for M, n, K in SILU}
+    shapes |= {lib.tm_gemm_tile_shape(M, N, K, lib.tm_tile_linear_parts(M, N, K)) for M, N, K in PARTS}
+    shapes |= {lib.tm_gemm_tile_shape(M, (H + 2 * KVH) * D, K, 1) for M, H, KVH, D, K in QKV}
+    assert shapes == set(range(11))
+
+
+@pytest.mark.parametrize("M,n,K", SILU)
+def test_gate_up_silu(M, n, K):
+    a, w, ref = _operands(M, 2 * n, K, M + n)
+    out = torch.full((M, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+    assert library().tm_tile_gate_up_silu(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), P(out.data_ptr()), I(n), _stream()) == 0
+    gate, up = ref.chunk(2, 1)
+    want = torch.nn.functional.silu(gate) * up
+    # gate and up are rounded to bfloat16 (by at most 2^-8 of themselves; silu' <= 1.1), and the result is; 32-bit sums of K terms
+    # of size 1 / sqrt(K) add less than 2^-18
+    bound = 2.0 ** -8 * (1.1 * gate.abs() * up.abs() + 2 * want.abs()) * 1.02 + 2.0 ** -18 * (1.1 * up.abs() + gate.abs() + 1)
+    assert ((out.double() - want).abs() <= bound).all()
+
+
+QKV = [(65, 14, 2, 64, 256), (333, 14, 2, 64, 896), (1000, 28, 4, 128, 256), (2500, 14, 2, 64, 256), (70, 3, 1, 192, 256)]
+
+
+@pytest.mark.parametrize("stored", [True, False])
+@pytest.mark.parametrize("bias_dtype", [torch.float32, torch.bfloat16, None])
+@pytest.mark.parametrize("M,H,KVH,D,K", QKV)
+def test_qkv_with_rotation_and_cache_write(M, H, KVH, D, K, bias_dtype, stored):
+    N, page = (H + 2 * KVH) * D, 16
+    a, w, ref = _operands(M, N, K, M + H)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    bias = torch.randn(N, generator=g, device="cuda").to(bias_dtype) if bias_dtype else None
+    angle = torch.rand(300, D // 2, generator=g, device="cuda") * 6.28
+    cos, sin = angle.cos(), angle.sin()
+    pos = torch.randint(0, 300, (M,), generator=g, device="cuda", dtype=torch.int32)
+    pages = -(-M // page) + 2
+    slots = torch.randperm(pages * page, generator=g, device="cuda")[:M].int()
+    slots[1::7] = -1
+    q = torch.full((M, H * D), 7.0, device="cuda", dtype=torch.bfloat16)
+    k = torch.full((pages, page, KVH, D), 7.0, device="cuda", dtype=torch.bfloat16)
+    v = torch.full((pages, KVH, D, page), 7.0, device="cuda", dtype=torch.bfloat16)
+    code = -1 if bias is None else (0 if bias_dtype == torch.float32 else 1)
+    assert library().tm_tile_qkv_rope(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), P(bias.data_ptr() if bias is not None else None), I(code),
+                                      P(q.data_ptr()), I(H), I(KVH), I(D), P(cos.data_ptr()), P(sin.data_ptr()), P(pos.data_ptr()),
+                                      P(slots.data_ptr() if stored else None), P(k.data_ptr()), P(v.data_ptr()), I(page), _stream()) == 0
+    x = (ref + (bias.double() if bias is not None else 0)).view(M, H + 2 * KVH, D)
+    lo, hi = x[..., :D // 2], x[..., D // 2:]
+    c, s = (t.double()[pos.long()][:, None] for t in (cos, sin))
+    turned = torch.cat([lo * c - hi * s, hi * c + lo * s], -1)
+    size = torch.cat([lo.abs() + hi.abs()] * 2, -1)             # each of the pair is rounded, then the result is
+    bound = 2.0 ** -8 * (size + turned.abs()) * 1.02 + 2.0 ** -17
+    assert ((q.double().view(M, H, D) - turned[:, :H]).abs() <= bound[:, :H]).all()
+    kept = (slots >= 0) & stored
+    at = slots[kept].long()
+    keys, values = k.view(-1, KVH, D), v.permute(0, 3, 1, 2).reshape(-1, KVH, D)
+    assert ((keys[at].double() - turned[kept, H:H + KVH]).abs() <= bound[kept, H:H + KVH]).all()
+    assert ((values[at].double() - x[kept, H + KVH:]).abs() <= 2.0 ** -8 * x[kept, H + KVH:].abs() * 1.02 + 2.0 ** -17).all()
+    others = torch.ones(pages * page, dtype=torch.bool, device="cuda")
+    others[at] = False
+    assert (keys[others] == 7).all() and (values[others] == 7).all()
+
+
+PARTS = [(65, 896, 896), (77, 896, 4864), (130, 3584, 960), (333, 896, 4864), (1000, 1016, 4864), (2048, 896, 896), (2048, 896, 4864),
+         (4000, 896, 4864), (1000, 3584, 3584)]
+
+
+@pytest.mark.parametrize("M,N,K", PARTS)
+def test_partial_sums_of_a_split_k(M, N, K):
+    lib = library()
+    parts = lib.tm_tile_linear_parts(M, N, K)
+    assert 1 <= parts <= 8
+    a, w, ref = _operands(M, N, K, M + K)
+    out = torch.full((parts, M, N), float("nan"), device="cuda")
+    assert lib.tm_tile_linear_split(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), I(N), P(out.data_ptr()), _stream()) == 0
+    # 32-bit sums of products of size 1 / sqrt(K): the rounding of each of K additions to a sum of at most about 5
+    assert (out.double().sum(0) - ref).abs().max() <= 2.0 ** -24 * 5 * 4 * K ** 0.5
+
+
+def test_what_the_kernels_do_not_take_is_refused():
+    lib = library()
+    a, w, _ = _operands(65, 128, 320, 1)
+    out = torch.zeros(65, 64, device="cuda", dtype=torch.bfloat16)
+
+    def run(a_ptr, lda, K, n):
+        return lib.tm_tile_gate_up_silu(P(a_ptr), I(lda), I(65), I(K), P(w.data_ptr()), P(out.data_ptr()), I(n), _stream())
+
+    assert run(a.data_ptr(), 320, 320, 64) == 0
+    assert run(a.data_ptr() + 2, 320, 320, 64) == 1             # rows off their 16-byte places
+    assert run(a.data_ptr(), 324, 320, 64) == 1
+    assert run(a.data_ptr(), 320, 300, 64) == 1                 # k that is not whole steps
+    assert run(a.data_ptr(), 320, 192, 64) == 1                 # fewer steps than the ring has buffers
+    assert run(a.data_ptr(), 320, 320, 60) == 1

@@ -36,6 +36,19 @@ int tm_gemm_f32_mfma_fits(const void* A, int lda, const void* W, const void* bia
 int tm_gemm_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,
                      hipStream_t stream);
 
+// Products of prompt-sized steps on the bfloat16 matrix unit (gemm_tile.hip), W row-major [rows, K]; K a multiple of 64, rows of
+// whole 16-byte pieces (tm_gemm_tile_takes): silu(gate) * up of gate|up; q|k|v with bias, rotation over the whole head (head
+// sizes that are multiples of 64) and cache write; 32-bit partial sums [parts][M][N] of a product whose K is split
+// (tm_tile_linear_parts says over how many parts, 0: the library's product is the better one).
+int tm_gemm_tile_takes(const void* A, int lda, const void* W, int M, int N, int K);
+int tm_gemm_tile_shape(int M, int N, int K, int splits);        // which of its tiles it runs with (for tests)
+int tm_tile_gate_up_silu(const void* A, int lda, int M, int K, const void* W, void* act, int I, hipStream_t stream);
+int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void* W, const void* bias, int bias_dtype, void* q, int H, int KVH, int D,
+                     const float* cos_t, const float* sin_t, const int* positions, const int* slots, void* k_pool, void* v_pool,
+                     int page, hipStream_t stream);
+int tm_tile_linear_parts(int M, int N, int K);
+int tm_tile_linear_split(const void* A, int lda, int M, int K, const void* W, int N, float* parts, hipStream_t stream);
+
 int tm_attn_paged_generic(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
                           const void* v_pool, const int* block_tables, int table_width, const int* seq_of_token,
                           const int* positions, int T, int H, int KVH, int D, int page, float scale, int window,

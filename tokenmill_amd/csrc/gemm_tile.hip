@@ -1,0 +1,530 @@
+// Matrix products of prompt-sized steps on the bfloat16 matrix unit, each with its layer's own epilogue: C = A W^T (+ bias)
+// stored in bfloat16; gate|up with SiLU*up; q|k|v with bias, rotation and cache write; 32-bit partial sums of a product whose
+// K is split over groups of blocks.
+//
+// A block of four wavefronts computes a tile of BM rows by BN matrix rows, BM x BN / 4 a wavefront, k in steps of 64. Both
+// operands come straight into LDS (16 bytes a lane, no registers in between) into a ring of ST buffers, ST - 1 to ST steps
+// ahead of the products; a wavefront waits for its own loads of a step by count and meets the others at one barrier a step.
+// The operand fragments of half a step (32 k) are read from LDS while the half before is multiplied. The blocks stay: each
+// walks tiles b, b + gridDim.x, ... as ONE stream of steps, so the loads of the next tile are on their way while a tile's
+// epilogue stores, and the ring never runs empty inside a launch.
+//
+// LDS. A load instruction of a wavefront fills 1,024 bytes in lane order: eight rows of 128 bytes. Lane l brings row l / 8 and,
+// of its eight 16-byte pieces, the one whose place in the row is l % 8 after the XOR below, so an operand load (lane (r, g):
+// piece g of row r) meets no bank twice and the global side still reads whole 128-byte lines.
+//
+// Which matrix row an LDS row holds is the epilogue's choice: 64 LDS rows are a "unit", for SiLU 32 gate rows and the 32 up
+// rows that meet them, for q|k|v 32 channels of a head and the 32 they are rotated with, else 64 consecutive rows. A pair of
+// 16-row matrix tiles takes its rows in the order 8 (r / 4) + r % 4 (+ 4), so that a lane ends with eight consecutive
+// columns of a row of C: 16-byte stores.
+#include "common.h"
+#include "api.h"
+#include "fused_common.h"
+
+#include <type_traits>
+
+enum { GT_SILU = 0, GT_QKV = 1, GT_PARTS = 2 };
+
+struct TileArgs {
+    const bf16_t* A;            // [M, K], rows lda apart
+    const bf16_t* W;            // [rows, K]
+    const void* bias;           // [rows] or null
+    void* C;                    // [M, N] rows ldc apart; PARTS: float [split][M][N]
+    int M, N, K, lda, ldc;      // N: matrix rows (SiLU: twice I)
+    int bias_f32;
+    int tiles_m, tiles_n, splits, band;
+    int I;                      // SiLU: columns of the result
+    // q|k|v
+    int H, KVH, D, page_shift;
+    const float* cos_t;         // [positions, D / 2]
+    const float* sin_t;
+    const int* positions;       // [M]
+    const int* slots;           // [M]; < 0: not stored; or null
+    bf16_t* k_pool;             // [pages, page, KVH, D]
+    bf16_t* v_pool;             // [pages, KVH, D, page]
+};
+
+// 16 bytes a lane from base + voff (bytes) to LDS at lds (bytes, wave-uniform) + 16 * lane
+__device__ __forceinline__ void gt_load_lds(uint32_t lds, uint32_t voff, const void* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base));
+}
+
+// two values rounded to bfloat16 and back, by one conversion
+__device__ __forceinline__ void gt_round2(float& a, float& b) {
+    const uint32_t u = fd_pack(a, b);
+    a = __uint_as_float(u << 16);
+    b = __uint_as_float(u & 0xffff0000u);
+}
+
+template <int N>
+__device__ __forceinline__ void gt_wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
+// Tile t of the launch -> (row tile, column tile, part of K). The blocks of one XCD (b % 8) walk a run of neighbouring tiles,
+// up to 16 row tiles of a column tile first, so that what an XCD's blocks read at a time overlaps in its L2.
+__device__ __forceinline__ bool gt_place(const TileArgs& a, int p, int& tm, int& tn, int& sp) {
+    const int total = a.tiles_m * a.tiles_n * a.splits;
+    const int chunk = (total + 7) / 8;
+    const int t = (p % 8) * chunk + p / 8;
+    if (p / 8 >= chunk || t >= total) return false;
+    sp = t / (a.tiles_m * a.tiles_n);
+    const int in = t - sp * a.tiles_m * a.tiles_n;
+    const int band = in / (a.band * a.tiles_n);
+    const int rows = a.tiles_m - a.band * band < a.band ? a.tiles_m - a.band * band : a.band;
+    const int q = in - band * a.band * a.tiles_n;
+    tn = q / rows;
+    tm = a.band * band + q - tn * rows;
+    return true;
+}
+
+// the matrix row that row q of unit u holds
+template <int EPI>
+__device__ __forceinline__ int gt_matrix_row(const TileArgs& a, int u, int q) {
+    int n;
+    if (EPI == GT_SILU) {
+        n = 32 * u + (q & 31);
+        n = n < a.I ? n : a.I - 1;
+        if (q >= 32) n += a.I;
+        return n;
+    }
+    if (EPI == GT_QKV) {
+        const int per_head = a.D / 64, head = u / per_head;
+        n = head * a.D + 32 * (u - head * per_head) + (q & 31) + (q >= 32 ? a.D / 2 : 0);
+    } else {
+        n = 64 * u + q;
+    }
+    return n < a.N ? n : a.N - 1;
+}
+
+// MT, NT: 16-row tiles of A and of the matrix a wavefront multiplies; WM x WN = 4 wavefronts; ST: buffers of the ring
+template <int EPI, int MT, int NT, int WM, int WN, int ST, int OCC>
+__global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
+    extern __shared__ __align__(16) unsigned char gt_smem[];
+    constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, ROWS = BM + BN;
+    constexpr int STAGE = ROWS * 128, NL = ROWS / 32;               // bytes of a buffer; loads a wavefront makes for it
+    static_assert(BM % 32 == 0 && BN % 64 == 0 && NT % 4 == 0, "");
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)gt_smem;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;
+    const int r = lane % 16, g = lane / 16;
+    const int wm = wave / WN, wn = wave % WN;
+    const int ksteps = a.K / 64;
+    const int per = (ksteps + a.splits - 1) / a.splits;             // k-steps of a part
+
+    // --- the loading side: runs ahead of the products over the block's tiles ---
+    uint32_t voff[NL];
+    const bf16_t *lA = a.A, *lW = a.W;
+    int l_p = blockIdx.x;
+    bool l_more = true;
+    auto next_load_tile = [&]() {
+        int tm, tn, sp;
+        if (!l_more || !gt_place(a, l_p, tm, tn, sp)) {             // no further tile: the same bytes again, never multiplied
+            l_more = false;
+            lA = a.A;
+            lW = a.W;
+            return;
+        }
+        l_p += gridDim.x;
+        const int k0 = sp * per;
+        lA = a.A + (size_t)k0 * 64;
+        lW = a.W + (size_t)k0 * 64;
+        const int in8 = lane / 8, at = lane % 8;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int R = (wave + 4 * i) * 8 + in8;                 // row of the buffer
+            if (i < BM / 32) {
+                int m = tm * BM + R;
+                m = m < a.M ? m : a.M - 1;
+                voff[i] = (uint32_t)m * (uint32_t)a.lda * 2u + (uint32_t)((at ^ ((R >> 1) & 7)) * 16);
+            } else {
+                const int Rb = R - BM;
+                const int n = gt_matrix_row<EPI>(a, tn * (BN / 64) + Rb / 64, Rb % 64);
+                voff[i] = (uint32_t)n * (uint32_t)a.K * 2u + (uint32_t)((at ^ (((Rb >> 1) & 1) | (((Rb >> 3) & 3) << 1))) * 16);
+            }
+        }
+    };
+    auto issue_one = [&](uint32_t dst, int i) { gt_load_lds(dst + i * 4096, voff[i], i < BM / 32 ? (const void*)lA : (const void*)lW); };
+    auto issued = [&]() {
+        lA += l_more ? 64 : 0;
+        lW += l_more ? 64 : 0;
+    };
+
+    // --- the multiplying side ---
+    int tm, tn, sp;
+    int p = blockIdx.x;
+    if (!gt_place(a, p, tm, tn, sp)) return;
+    next_load_tile();
+#pragma unroll
+    for (int s = 0; s < ST; ++s) {                                  // (every part of K has at least ST steps)
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + s * STAGE + wave * 1024);
+#pragma unroll
+        for (int i = 0; i < NL; ++i) issue_one(dst, i);
+        issued();
+    }
+
+    f32x4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    FFrag fa[2][MT], fb[2][NT];
+    const int rb = 8 * (r / 4) + r % 4;
+    const int offA = (wm * MT * 16 + r) * 128 + ((g ^ ((r >> 1) & 7)) << 4);
+    const int offB = (BM + wn * NT * 16 + rb) * 128 + ((g ^ (((rb >> 1) & 1) | (((rb >> 3) & 3) << 1))) << 4);
+    // One half of a step: the products of half `half`, and spread between them the reads of the other half's operands (from
+    // buffer `from`) and, with dst, the loads of the step ST ahead. The order is the program's: the barriers between the groups
+    // keep the compiler from gathering the reads.
+    constexpr int READS = MT + NT, PRODUCTS = MT * NT;
+    auto half_step = [&](auto HALF, int from, auto LOADS, uint32_t dst) {
+        constexpr int half = decltype(HALF)::value, other = 1 - half;
+        const unsigned char* pa = gt_smem + from * STAGE + (offA ^ (other * 64));
+        const unsigned char* pb = gt_smem + from * STAGE + (offB ^ (other * 64));
+#pragma unroll
+        for (int q = 0; q < READS; ++q) {
+            if (q == 0) fa[other][0].u = *(const u32x4_t*)pa;
+            else if (q <= NT) fb[other][q - 1].u = *(const u32x4_t*)(pb + ((q - 1) / 2) * 4096 + ((q - 1) & 1) * 512);
+            else fa[other][q - NT].u = *(const u32x4_t*)(pa + (q - NT) * 2048);
+            if constexpr (decltype(LOADS)::value) {
+#pragma unroll
+                for (int i = q * NL / READS; i < (q + 1) * NL / READS; ++i) issue_one(dst, i);
+            }
+#pragma unroll
+            for (int n = q * PRODUCTS / READS; n < (q + 1) * PRODUCTS / READS; ++n)
+                acc[n / NT][n % NT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[half][n % NT].b, fa[half][n / NT].b, acc[n / NT][n % NT], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    gt_wait_loads<(ST - 1) * NL>();
+    __builtin_amdgcn_s_barrier();
+    int buf = 0;
+    while (true) {
+        // the first half's operands of a tile: read here, not behind the tile before, whose epilogue needs the registers
+        fa[0][0].u = *(const u32x4_t*)(gt_smem + buf * STAGE + offA);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) fb[0][j].u = *(const u32x4_t*)(gt_smem + buf * STAGE + offB + (j / 2) * 4096 + (j & 1) * 512);
+#pragma unroll
+        for (int i = 1; i < MT; ++i) fa[0][i].u = *(const u32x4_t*)(gt_smem + buf * STAGE + offA + i * 2048);
+        const int k0 = sp * per;
+        const int steps = ksteps - k0 < per ? ksteps - k0 : per;
+        // what the epilogue's addresses hang on: asked for now where there are registers for it, so that the end of the tile waits
+        // for one trip and not for two
+        int pos[EPI == GT_QKV ? MT : 1], slot[EPI == GT_QKV ? MT : 1];
+        auto read_places = [&]() {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const int m = tm * BM + (wm * MT + i) * 16 + r;
+                pos[i] = a.positions[m < a.M ? m : a.M - 1];
+                slot[i] = a.slots ? a.slots[m < a.M ? m : a.M - 1] : -1;
+            }
+        };
+        if constexpr (EPI == GT_QKV && MT <= 5) read_places();
+        // the loads are ST steps ahead: those of the last ST steps are the next tile's
+#pragma unroll 1
+        for (int part = 0; part < 2; ++part) {
+            if (part) next_load_tile();
+#pragma unroll 1
+            for (int s = part ? ST : steps - ST; s > 0; --s) {
+                half_step(std::integral_constant<int, 0>{}, buf, std::false_type{}, 0u);
+                // the next step's rows have arrived (this wavefront's, then everybody's), and this step's have been read
+                gt_wait_loads<(ST - 2) * NL>();
+                __builtin_amdgcn_s_barrier();
+                const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + wave * 1024);
+                buf = buf + 1 == ST ? 0 : buf + 1;
+                asm volatile("" ::: "memory");
+                half_step(std::integral_constant<int, 1>{}, buf, std::true_type{}, dst);
+                issued();
+            }
+        }
+        // --- the tile's results ---
+        if constexpr (EPI == GT_QKV && MT > 5) read_places();
+#pragma unroll
+        for (int un = 0; un < NT / 4; ++un) {
+            const int u = tn * (BN / 64) + wn * (NT / 4) + un;      // the unit
+            // a lane's columns: eight from c0 on and eight from c1 on (indices into the matrix's rows)
+            int c0, c1, head = 0, d0 = 0;
+            bool ok0, ok1;
+            if (EPI == GT_SILU) {
+                c0 = 32 * u + 8 * g;
+                c1 = a.I + c0;
+                ok0 = ok1 = c0 < a.I;
+            } else if (EPI == GT_QKV) {
+                const int per_head = a.D / 64;
+                head = u / per_head;
+                d0 = 32 * (u - head * per_head) + 8 * g;
+                c0 = head * a.D + d0;
+                c1 = c0 + a.D / 2;
+                ok0 = ok1 = c1 < a.N;
+            } else {
+                c0 = 64 * u + 8 * g;
+                c1 = c0 + 32;
+                ok0 = c0 < a.N;
+                ok1 = c1 < a.N;
+            }
+            // q|k|v: the bias and (a few rows at a time) the rows' cosines and sines, all asked for before the first is used
+            constexpr int AHEAD = EPI != GT_QKV ? 1 : MT <= 5 ? MT : 4;
+            f32x4_t bias[4], cs[AHEAD][2], sn[AHEAD][2];
+            if constexpr (EPI == GT_QKV) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int at = (ok0 ? (e < 2 ? c0 : c1) : 0) + 4 * (e & 1);
+                    bias[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                    if (!a.bias) continue;
+                    if (a.bias_f32) {
+                        bias[e] = *(const f32x4_t*)((const float*)a.bias + at);
+                    } else {
+                        const uint2 u = *(const uint2*)((const bf16_t*)a.bias + at);
+                        bias[e] = f32x4_t{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                                          __uint_as_float(u.y & 0xffff0000u)};
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (EPI == GT_QKV) {
+                    if (i % AHEAD == 0 && head < a.H + a.KVH) {
+#pragma unroll
+                        for (int k = 0; k < AHEAD && i + k < MT; ++k) {
+                            const size_t at = (size_t)pos[i + k] * (a.D / 2) + d0;
+#pragma unroll
+                            for (int e = 0; e < 2; ++e) {
+                                cs[k][e] = *(const f32x4_t*)(a.cos_t + at + 4 * e);
+                                sn[k][e] = *(const f32x4_t*)(a.sin_t + at + 4 * e);
+                            }
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                const int m = tm * BM + (wm * MT + i) * 16 + r;
+                float x[8], y[8];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    x[e] = acc[i][4 * un][e];
+                    x[4 + e] = acc[i][4 * un + 1][e];
+                    y[e] = acc[i][4 * un + 2][e];
+                    y[4 + e] = acc[i][4 * un + 3][e];
+                }
+                if (m >= a.M) continue;
+                if (EPI == GT_PARTS) {
+                    float* dst = (float*)a.C + ((size_t)sp * a.M + m) * a.N;
+                    if (ok0) {
+                        *(f32x4_t*)(dst + c0) = f32x4_t{x[0], x[1], x[2], x[3]};
+                        *(f32x4_t*)(dst + c0 + 4) = f32x4_t{x[4], x[5], x[6], x[7]};
+                    }
+                    if (ok1) {
+                        *(f32x4_t*)(dst + c1) = f32x4_t{y[0], y[1], y[2], y[3]};
+                        *(f32x4_t*)(dst + c1 + 4) = f32x4_t{y[4], y[5], y[6], y[7]};
+                    }
+                } else if (EPI == GT_SILU) {
+                    if (!ok0) continue;
+                    float v[8];
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        gt_round2(x[e], x[e + 1]);
+                        gt_round2(y[e], y[e + 1]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = x[e] * __builtin_amdgcn_rcpf(1.f + __expf(-x[e])) * y[e];
+                    *(u32x4_t*)((bf16_t*)a.C + (size_t)m * a.ldc + c0) =
+                        u32x4_t{fd_pack(v[0], v[1]), fd_pack(v[2], v[3]), fd_pack(v[4], v[5]), fd_pack(v[6], v[7])};
+                } else {
+                    if (!ok0) continue;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        x[e] += bias[e / 4][e % 4];
+                        y[e] += bias[2 + e / 4][e % 4];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        gt_round2(x[e], x[e + 1]);
+                        gt_round2(y[e], y[e + 1]);
+                    }
+                    const int row_slot = slot[EPI == GT_QKV ? i : 0];
+                    if (head < a.H + a.KVH) {
+                        float y1[8], y2[8];
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) rotate_pair(x[e], y[e], cs[i % AHEAD][e / 4][e % 4], sn[i % AHEAD][e / 4][e % 4], y1[e], y2[e]);
+                        bf16_t* dst = nullptr;
+                        if (head < a.H) dst = (bf16_t*)a.C + (size_t)m * a.ldc + head * a.D + d0;
+                        else if (row_slot >= 0) dst = a.k_pool + ((size_t)row_slot * a.KVH + (head - a.H)) * a.D + d0;
+                        if (dst) {
+                            *(u32x4_t*)dst = u32x4_t{fd_pack(y1[0], y1[1]), fd_pack(y1[2], y1[3]), fd_pack(y1[4], y1[5]), fd_pack(y1[6], y1[7])};
+                            *(u32x4_t*)(dst + a.D / 2) =
+                                u32x4_t{fd_pack(y2[0], y2[1]), fd_pack(y2[2], y2[3]), fd_pack(y2[4], y2[5]), fd_pack(y2[6], y2[7])};
+                        }
+                    } else if (row_slot >= 0) {
+                        const int vh = head - a.H - a.KVH;
+                        const int pg = row_slot >> a.page_shift, in_page = row_slot & ((1 << a.page_shift) - 1);
+                        bf16_t* dst = a.v_pool + ((((size_t)pg * a.KVH + vh) * a.D + d0) << a.page_shift) + in_page;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            dst[(size_t)e << a.page_shift] = f32_to_bf16(x[e]);
+                            dst[(size_t)(a.D / 2 + e) << a.page_shift] = f32_to_bf16(y[e]);
+                        }
+                    }
+                }
+            }
+        }
+        p += gridDim.x;
+        if (!gt_place(a, p, tm, tn, sp)) break;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    gt_wait_loads<0>();                                             // nothing of the ring is in flight when the block ends
+}
+
+// --- which tile, how many parts of K ---------------------------------------------------------------------------------------
+
+// The tiles there are: 16-row tiles a wavefront (of A, of the matrix), wavefronts (down, across), buffers, blocks a CU; then the
+// microseconds a 64-wide step and an epilogue of one block take when a CU has one, and of two when it has two. A large tile
+// moves the fewest bytes per product, small ones are for launches that would leave CUs idle, the one with eight buffers for
+// matrices that come from HBM under few rows (q|k|v of the 0.5B shape at 77 rows, in a step: 12.6 us with four, 8.9 with
+// eight). Fitted to 1,900 timings on an MI355X with cold matrices (the 0.5B and 7B shapes' four matrices, 70 to 6,500 rows, K in
+// one to eight parts): the shape these figures choose takes 3% longer than the best one on average. Large tiles stand at this
+// card's limit (products of 16,384^3 reach 1.55 PFLOP/s; 224 x 256 tiles 1.6 once the ring runs), small ones at the latency
+// of a step.
+#define GT_SHAPES(X)                                       \
+    X(0, 8, 8, 2, 2, 2, 1, 1.206, 10.0, 0, 0)              \
+    X(1, 7, 8, 2, 2, 2, 1, 1.133, 8.79, 0, 0)              \
+    X(2, 6, 8, 2, 2, 2, 1, 1.096, 7.59, 0, 0)              \
+    X(3, 5, 8, 2, 2, 3, 1, 0.784, 7.50, 0, 0)              \
+    X(4, 4, 8, 2, 2, 3, 1, 0.755, 6.15, 0, 0)              \
+    X(5, 3, 8, 2, 2, 3, 1, 0.685, 4.61, 0, 0)              \
+    X(6, 4, 4, 2, 2, 4, 1, 0.483, 3.58, 0, 0)              \
+    X(7, 2, 4, 2, 2, 3, 2, 0.400, 1.48, 0.581, 3.28)       \
+    X(8, 1, 4, 4, 1, 4, 2, 0.232, 1.01, 0.342, 1.94)       \
+    X(9, 1, 4, 4, 1, 8, 1, 0.213, 1.16, 0, 0)              \
+    X(10, 1, 4, 2, 2, 4, 2, 0.318, 1.02, 0.273, 0.61)
+struct GtShape { int BM, BN, ST, OCC; double step, epi, step2, epi2; };
+#define GT_SHAPE(id, MT, NT, WM, WN, ST, OCC, s1, e1, s2, e2) {16 * MT * WM, 16 * NT * WN, ST, OCC, s1, e1, s2, e2},
+static const GtShape gt_shapes[] = {GT_SHAPES(GT_SHAPE)};
+constexpr int GT_N_SHAPES = sizeof(gt_shapes) / sizeof(gt_shapes[0]);
+constexpr int GT_CUS = 256;
+constexpr double GT_BYTES_US = 14e6;        // what the CUs take out of the second-level caches together
+
+// Microseconds a launch takes beyond its start: rounds of blocks, or the operands' way into the CUs.
+static double gt_cost(const GtShape& t, int M, int N, int K, int splits) {
+    const int per = (K / 64 + splits - 1) / splits;
+    const long long tiles = (long long)((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN) * splits;
+    const bool pairs = t.OCC > 1 && tiles > GT_CUS;
+    const long long slots = pairs ? 2 * GT_CUS : GT_CUS;
+    const double compute = (double)((tiles + slots - 1) / slots) * (pairs ? per * t.step2 + t.epi2 : per * t.step + t.epi);
+    const double bytes = (double)tiles * (t.BM + t.BN) * per * 128 / GT_BYTES_US;
+    return compute > bytes ? compute : bytes;
+}
+
+// Every part of K has to fill the ring.
+static bool gt_splits_ok(const GtShape& t, int K, int splits) {
+    const int steps = K / 64, per = (steps + splits - 1) / splits;
+    return steps - (splits - 1) * per >= t.ST;
+}
+
+static int gt_choose(int M, int N, int K, int splits, double* cost = nullptr) {
+    int best = -1;
+    double least = 0;
+    for (int i = 0; i < GT_N_SHAPES; ++i) {
+        if (!gt_splits_ok(gt_shapes[i], K, splits)) continue;
+        const double c = gt_cost(gt_shapes[i], M, N, K, splits);
+        if (best < 0 || c < least) best = i, least = c;
+    }
+    if (cost) *cost = least;
+    return best;
+}
+
+template <int EPI, int MT, int NT, int WM, int WN, int ST, int OCC>
+static int gt_launch(TileArgs& a, hipStream_t stream) {
+    constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, LDS = (BM + BN) * 128 * ST;
+    static_assert(LDS * OCC <= 160 * 1024, "");
+    static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_tile_kernel<EPI, MT, NT, WM, WN, ST, OCC>,
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if (allowed != hipSuccess) return TM_ERR_LAUNCH;
+    a.tiles_m = (a.M + BM - 1) / BM;
+    a.tiles_n = EPI == GT_SILU ? (2 * ((a.I + 31) / 32 * 32) + BN - 1) / BN : (a.N + BN - 1) / BN;
+    // row tiles an XCD's blocks take beside each other: all of them where K is short enough for their rows to stay in its L2
+    const int most = a.K > 2048 ? 6 : 16, bands = (a.tiles_m + most - 1) / most;
+    a.band = (a.tiles_m + bands - 1) / bands;
+    const int chunk = (a.tiles_m * a.tiles_n * a.splits + 7) / 8;
+    const int grid = 8 * chunk < GT_CUS * OCC ? 8 * chunk : GT_CUS * OCC;
+    gemm_tile_kernel<EPI, MT, NT, WM, WN, ST, OCC><<<grid, 256, LDS, stream>>>(a);
+    TM_CHECK_LAUNCH();
+    return TM_OK;
+}
+
+template <int EPI>
+static int gt_go(TileArgs& a, int shape, hipStream_t stream) {
+    switch (shape) {
+#define GT_CASE(id, MT, NT, WM, WN, ST, OCC, s1, e1, s2, e2) case id: return gt_launch<EPI, MT, NT, WM, WN, ST, OCC>(a, stream);
+        GT_SHAPES(GT_CASE)
+    }
+    return TM_ERR_ARG;
+}
+
+// Which of the tiles above a product runs with.
+extern "C" int tm_gemm_tile_shape(int M, int N, int K, int splits) {
+    return M > 0 && N > 0 && K >= 256 && splits > 0 ? gt_choose(M, N, K, splits) : -1;
+}
+
+static bool gt_aligned(const void* p) { return p && ((uintptr_t)p % 16) == 0; }
+
+// Whole 16-byte pieces everywhere, k in whole steps, rows that 32-bit offsets reach.
+extern "C" int tm_gemm_tile_takes(const void* A, int lda, const void* W, int M, int N, int K) {
+    return M > 0 && N > 0 && N % 8 == 0 && K >= 256 && K % 64 == 0 && lda >= K && lda % 8 == 0 && gt_aligned(A) && gt_aligned(W) &&
+           (long long)M * lda * 2 < (1ll << 32) && (long long)N * K * 2 < (1ll << 32) && (long long)M * N < (1ll << 40);
+}
+
+// act[m, i] = silu(gate) * up with gate|up = A W^T, W [2 I, K] (gate rows, then up rows)
+extern "C" int tm_tile_gate_up_silu(const void* A, int lda, int M, int K, const void* W, void* act, int I, hipStream_t stream) {
+    if (I <= 0 || I % 8 || !gt_aligned(act) || !tm_gemm_tile_takes(A, lda, W, M, 2 * I, K)) return TM_ERR_ARG;
+    TileArgs a{};
+    a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = act;
+    a.M = M; a.N = 2 * I; a.K = K; a.lda = lda; a.ldc = I; a.I = I; a.splits = 1;
+    return gt_go<GT_SILU>(a, gt_choose(M, 2 * I, K, 1), stream);
+}
+
+// q (rotated, [M, H D]), and k and v to the cache, of q|k|v = A W^T + bias; head sizes of whole units (64), rotated over the
+// whole head; slots (null: nothing is stored) as in tm_rope_kv_write
+extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void* W, const void* bias, int bias_dtype, void* q, int H,
+                                int KVH, int D, const float* cos_t, const float* sin_t, const int* positions, const int* slots,
+                                void* k_pool, void* v_pool, int page, hipStream_t stream) {
+    const int N = (H + 2 * KVH) * D;
+    if (H <= 0 || KVH <= 0 || D <= 0 || D % 64 || !gt_aligned(q) || !cos_t || !sin_t || !positions || page <= 0 || (page & (page - 1)) ||
+        (bias && bias_dtype != TM_NONE && !gt_aligned(bias)) || !gt_aligned(cos_t) || !gt_aligned(sin_t) || (slots && (!gt_aligned(k_pool) || !v_pool)) || !tm_gemm_tile_takes(A, lda, W, M, N, K))
+        return TM_ERR_ARG;
+    TileArgs a{};
+    a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = q;
+    a.bias = bias_dtype == TM_NONE ? nullptr : bias; a.bias_f32 = bias_dtype == TM_F32;
+    a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = H * D; a.splits = 1;
+    a.H = H; a.KVH = KVH; a.D = D; a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots;
+    a.k_pool = (bf16_t*)k_pool; a.v_pool = (bf16_t*)v_pool;
+    while ((1 << a.page_shift) < page) ++a.page_shift;
+    return gt_go<GT_QKV>(a, gt_choose(M, N, K, 1), stream);
+}
+
+// Parts that a plain product's K is split into, whose 32-bit sums the next norm adds; 0: the library's product is the better one.
+// Few tiles leave CUs idle for the library and for one part alike; a part costs a write and a read of its sums.
+extern "C" int tm_tile_linear_parts(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || N % 8 || K < 256 || K % 64) return 0;
+    if ((long long)((M + 127) / 128) * ((N + 127) / 128) > GT_CUS) return 0;
+    int best = 0;
+    double least = 0;
+    for (int splits = 1; splits <= 8; ++splits) {
+        double c;
+        if (gt_choose(M, N, K, splits, &c) < 0) continue;
+        c += (double)splits * M * N * 4 / 5e6;                      // the norm reads them
+        if (!best || c < least) best = splits, least = c;
+    }
+    return best;
+}
+
+// parts[p][m][n], p < tm_tile_linear_parts(M, N, K): the partial sums of A W^T
+extern "C" int tm_tile_linear_split(const void* A, int lda, int M, int K, const void* W, int N, float* parts, hipStream_t stream) {
+    const int splits = tm_tile_linear_parts(M, N, K);
+    if (splits < 1 || !gt_aligned(parts) || !tm_gemm_tile_takes(A, lda, W, M, N, K)) return TM_ERR_ARG;
+    TileArgs a{};
+    a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = parts;
+    a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = N; a.splits = splits;
+    return gt_go<GT_PARTS>(a, gt_choose(M, N, K, splits), stream);
+}

@@ -109,10 +109,10 @@ enum {
     TM_QKV_FROM_NORM = 0,       // q|k|v by the kernel that starts at the norm (at most 16 tokens)
     TM_QKV_PANEL,               // ... by the kernel that keeps the normed input in LDS (17 to 64 tokens)
     TM_QKV_STREAM,              // ... by the kernel that streams the packed matrix for up to 64 tokens
-    TM_QKV_PLAIN,               // ... by a product, then rotation and cache write
+    TM_QKV_PLAIN,               // ... by a product over the row-major matrix, with rotation and cache write behind it or in its epilogue
     TM_GATE_UP_FROM_NORM,
     TM_GATE_UP_STREAM,
-    TM_GATE_UP_PLAIN,           // a product with the SiLU*up epilogue, or a product and then SiLU*up
+    TM_GATE_UP_PLAIN,           // any other product with the SiLU*up epilogue, or a product and then SiLU*up
     TM_PREFILL_SPLIT_KEYS,      // bfloat16 attention of prompt portions: wavefronts split a tile's key blocks
     TM_PREFILL_SHARED_KEYS,     // ... a tile's keys and values staged through LDS for all heads of a kv head
     TM_PROGRAM_COUNTERS

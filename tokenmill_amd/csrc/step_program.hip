@@ -90,6 +90,21 @@ bool stream_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype, int 
            aligned(x, 16) && tm_gemm_stream_fits(M, L.K);
 }
 
+// the products of prompt-sized steps with their epilogues (gemm_tile.hip), over the row-major matrix: wherever the kernels for
+// few rows do not run. Against the library's product and the kernel behind it, in us a layer: gate|up with SiLU*up, 0.5B
+// shape, 77 / 512 / 2,048 rows 16.4 / 22.2 / 65.0 to 6.9 / 13.2 / 35-40; 7B shape, 3,001 rows 724 to 590; q|k|v with rotation
+// and cache write, 0.5B shape 14.3 / 15.0 / 20.1 to 5.7 / 6.5 / 12.7.
+bool tile_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype) {
+    return dtype == TM_BF16 && L.dtype == TM_BF16 && !L.act && M > TM_SKINNY_ROWS && tm_gemm_tile_takes(x, ldx, L.w, M, L.N, L.K);
+}
+
+// Parts of K for an output or down projection of M rows beyond the stream kernels' whose 32-bit sums the next norm adds up; 0: none.
+int tile_parts(const TmLinear& L, int M) {
+    if (M <= TM_STREAM_ROWS || L.dtype != TM_BF16 || L.bias || L.act) return 0;
+    const int parts = tm_tile_linear_parts(M, L.N, L.K);
+    return parts <= TM_MAX_SUMS ? parts : 0;
+}
+
 // The product rule. x_dtype: type of x (the model's activations); the matrix has its own (L.dtype).
 struct Products {
     hipStream_t stream;
@@ -221,6 +236,7 @@ struct Run {
     int project(const TmLinear& L, const void* x_, int ldx, int M) {
         // 17 to 64 rows over a matrix with few rows of output: K split over groups of blocks, whose partial sums the
         // next norm adds up (or, where the caller wants the result itself, a small kernel)
+        // (the stream kernels take at most 64 rows: `sums` has room for TM_MAX_SUMS of them then)
         const int groups = (sums && L.N == p->hidden && L.packed_parts == 1 && stream_ok(L, x_, ldx, M, dtype, products.skinny_rows))
                                ? tm_stream_linear_parts(L.N, L.K) : 1;
         if (groups >= 2 && groups <= TM_MAX_SUMS) {
@@ -229,6 +245,13 @@ struct Run {
             delta = nullptr;
             pending_sums = groups;
             return accumulate && resid ? TM_OK : settle();
+        }
+        if (const int parts = (sums && accumulate && resid && L.N == p->hidden && tile_ok(L, x_, ldx, M, dtype)) ? tile_parts(L, M) : 0) {
+            const int rc = tm_tile_linear_split(x_, ldx, M, L.K, L.w, L.N, sums, stream);
+            if (rc) return rc;
+            delta = nullptr;
+            pending_sums = parts;
+            return TM_OK;
         }
         if (accumulate && resid && products.accumulates(L, dtype, x_, ldx, M)) {
             delta = nullptr;
@@ -333,8 +356,16 @@ struct Run {
                     q = qkv;
                     q_stride = HD;
                     ++p->taken[TM_QKV_STREAM];
+                } else if (tables_fusable && a.D % 64 == 0 && tile_ok(a.qkv, xn, hidden, T, dtype) && is_pow2(a.page) && bias_ok &&
+                           aligned(a.cos_t, 16) && aligned(a.sin_t, 16) && (!a.write || aligned(a.k_pool, 16))) {
+                    // 4. more tokens: rotation and cache write in the epilogue of a product over the row-major matrix
+                    rc = tm_tile_qkv_rope(xn, hidden, T, hidden, a.qkv.w, a.qkv.bias, a.qkv.bias_dtype, qkv, a.H, a.KVH, a.D, a.cos_t,
+                                          a.sin_t, s->positions, slots, kp, vp, a.page, stream);
+                    q = qkv;
+                    q_stride = HD;
+                    ++p->taken[TM_QKV_PLAIN];
                 } else {
-                    // 4. product, then rotation and cache write
+                    // 5. product, then rotation and cache write
                     if ((rc = linear(a.qkv, xn, hidden, T, qkv, QKV, dtype))) return rc;
                     if (a.rot > 0 || a.write)
                         rc = tm_rope_kv_write(qkv, dtype, T, a.H, a.KVH, a.D, a.rot, a.rot > 0 ? a.cos_t : nullptr,
@@ -440,6 +471,9 @@ struct Run {
                     ++p->taken[TM_GATE_UP_STREAM];
                 } else if (plain && T <= TM_SKINNY_ROWS && skinny_ok(f.gate_up, xn, hidden, dtype)) {   // (a matrix without a packed copy)
                     rc = tm_gemm_skinny(xn, hidden, f.gate_up.w, nullptr, TM_NONE, act, f.I, T, f.I, hidden, TM_BF16, 1, nullptr, 0, stream);
+                    ++p->taken[TM_GATE_UP_PLAIN];
+                } else if (plain && f.I % 8 == 0 && tile_ok(f.gate_up, xn, hidden, T, dtype)) {
+                    rc = tm_tile_gate_up_silu(xn, hidden, T, hidden, f.gate_up.w, act, f.I, stream);
                     ++p->taken[TM_GATE_UP_PLAIN];
                 } else {
                     if ((rc = linear(f.gate_up, xn, hidden, T, gu, 2 * f.I, dtype))) return rc;
@@ -564,6 +598,19 @@ void tm_program_counters(const TmProgram* p, long long* out) {
     for (int i = 0; i < TM_PROGRAM_COUNTERS; ++i) out[i] = p ? p->taken[i] : 0;
 }
 
+// Most parts that a product's K is split into in a step of T tokens (their sums [T, hidden] are kept until the next norm).
+static int program_sums(const TmProgram* p, int T) {
+    if (p->dtype != TM_BF16) return 0;
+    if (T <= TM_STREAM_ROWS) return TM_MAX_SUMS;
+    int most = 0;
+    for (const Op& op : p->ops) {
+        const TmLinear* L = op.kind == OP_ATTENTION ? &op.att.o : op.kind == OP_FEED_FORWARD ? &op.ffn.down : nullptr;
+        const int parts = L ? tile_parts(*L, T) : 0;
+        if (parts > most) most = parts;
+    }
+    return most;
+}
+
 // Bytes of workspace a step of T tokens with R logit rows needs, of which ``num_decode`` are single tokens
 // whose contexts reach ``max_decode_context``.
 size_t tm_program_workspace_bytes(const TmProgram* p, int T, int R, int num_decode, int max_decode_context) {
@@ -580,8 +627,7 @@ size_t tm_program_workspace_bytes(const TmProgram* p, int T, int R, int num_deco
     const size_t chunks = (size_t)tm_decode_chunks(max_decode_context > 0 ? max_decode_context : 1);
     n += align_up((size_t)num_decode * p->max_heads_d * chunks * 4); // split decode attention: partial values
     n += align_up((size_t)num_decode * p->max_heads * chunks * 2 * 4);   // ... and their (max, sum)
-    if (T <= TM_STREAM_ROWS && p->dtype == TM_BF16)
-        n += align_up((size_t)TM_MAX_SUMS * T * p->hidden * 4);      // partial sums of a product whose K is split over blocks
+    n += align_up((size_t)program_sums(p, T) * T * p->hidden * 4);   // partial sums of a product whose K is split over blocks
     const size_t rows = (size_t)(T > R ? T : R);
     n += align_up(rows * p->max_wide_in * 4);                        // 32-bit copies around the product of a 32-bit matrix
     n += align_up(rows * p->max_wide_out * 4);
@@ -629,7 +675,8 @@ int tm_program_run(const TmProgram* p, int first, int count, const TmStep* s, Tm
     const size_t chunks = (size_t)tm_decode_chunks(s->max_decode_context > 0 ? s->max_decode_context : 1);
     r.part_o = (float*)take((size_t)s->num_decode * p->max_heads_d * chunks * 4);
     r.part_ml = (float*)take((size_t)s->num_decode * p->max_heads * chunks * 2 * 4);
-    r.sums = (T <= TM_STREAM_ROWS && p->dtype == TM_BF16) ? (float*)take((size_t)TM_MAX_SUMS * T * p->hidden * 4) : nullptr;
+    const int parts = program_sums(p, T);
+    r.sums = parts ? (float*)take((size_t)parts * T * p->hidden * 4) : nullptr;
     const size_t rows = (size_t)(T > R ? T : R);
     if (p->max_wide_in) r.products.wide_in = (float*)take(rows * p->max_wide_in * 4);
     if (p->max_wide_out) r.products.wide_out = (float*)take(rows * p->max_wide_out * 4);
