@@ -1,0 +1,145 @@
+"""The 32-bit path's kernels for few rows (csrc/gemv_f32.hip, csrc/attention_decode_f32.hip) against 64-bit computations: rows and
+columns that fill no tile, the shortest K, K in parts, contexts at the edges of chunks, windows, kept keys, caps, sinks, gates."""
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from tokenmill_amd.hip.library import library
+
+pytestmark = pytest.mark.gpu
+P, I, F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+
+
+def _ptr(t):
+    return P(t.data_ptr() if t is not None else None)
+
+
+def _stream():
+    return P(torch.cuda.current_stream().cuda_stream)
+
+
+def _operands(M, N, K, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    a = torch.randn(M, K, generator=g, device="cuda")
+    w = torch.randn(N, K, generator=g, device="cuda") * K ** -0.5
+    return a, w, a.double() @ w.double().T
+
+
+# 32-bit sums: a wavefront's chain of K / (4 x 8) additions or fewer and the wavefronts' sums, each rounding a sum of at most about 5
+def _bound(K):
+    return 2.0 ** -24 * 5 * (16 + K ** 0.5)
+
+
+@pytest.mark.parametrize("N,K", [(4, 16), (20, 48), (896, 896), (1152, 4864), (8200, 896), (9000, 112)])
+@pytest.mark.parametrize("M", [1, 7, 16])
+def test_products_plain_and_in_parts(M, N, K):
+    lib = library()
+    a, w, ref = _operands(M, N, K, M + N + K)
+    bias = torch.randn(N, device="cuda")
+    out = torch.full((M, N), float("nan"), device="cuda")
+    assert lib.tm_gemv_f32_mfma(_ptr(a), I(K), _ptr(w), _ptr(bias), _ptr(out), I(N), I(M), I(N), I(K), _stream()) == 0
+    assert (out.double() - ref - bias.double()).abs().max() <= _bound(K)
+    parts = lib.tm_gemv_f32_parts(N, K)
+    sums = torch.full((parts, M, N), float("nan"), device="cuda")
+    assert lib.tm_gemv_f32_mfma_split(_ptr(a), I(K), _ptr(w), _ptr(sums), I(M), I(N), I(K), _stream()) == 0
+    assert (sums.double().sum(0) - ref).abs().max() <= _bound(K)
+
+
+def test_a_long_k_is_split():
+    assert library().tm_gemv_f32_parts(896, 4864) == 4 and library().tm_gemv_f32_parts(896, 896) == 1
+
+
+@pytest.mark.parametrize("n,K", [(4, 16), (36, 64), (4864, 896)])
+@pytest.mark.parametrize("M", [1, 16])
+def test_gate_up_silu(M, n, K):
+    a, w, ref = _operands(M, 2 * n, K, M + n)
+    out = torch.full((M, n), float("nan"), device="cuda")
+    assert library().tm_gemv_f32_gate_up_silu(_ptr(a), I(K), _ptr(w), _ptr(out), I(M), I(n), I(K), _stream()) == 0
+    gate, up = ref.chunk(2, 1)
+    want = torch.nn.functional.silu(gate) * up
+    assert ((out.double() - want).abs() <= _bound(K) * (1.1 * up.abs() + gate.abs() + 1) + 2.0 ** -20 * want.abs()).all()
+
+
+@pytest.mark.parametrize("M,H,KVH,D,K", [(1, 14, 2, 64, 896), (16, 3, 1, 128, 64), (5, 4, 2, 32, 16)])
+def test_qkv_with_rotation_and_cache_write(M, H, KVH, D, K):
+    N, page = (H + 2 * KVH) * D, 16
+    a, w, ref = _operands(M, N, K, M + H)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    bias = torch.randn(N, generator=g, device="cuda")
+    angle = torch.rand(300, D // 2, generator=g, device="cuda") * 6.28
+    cos, sin = angle.cos(), angle.sin()
+    pos = torch.randint(0, 300, (M,), generator=g, device="cuda", dtype=torch.int32)
+    slots = torch.randperm(3 * page, generator=g, device="cuda")[:M].int()
+    slots[1::3] = -1
+    q = torch.empty(M, H * D, device="cuda")
+    k, v = torch.full((3, page, KVH, D), 7.0, device="cuda"), torch.full((3, KVH, D, page), 7.0, device="cuda")
+    assert library().tm_gemv_f32_qkv_rope(_ptr(a), I(K), _ptr(w), _ptr(bias), _ptr(q), I(M), I(K), I(H), I(KVH), I(D), _ptr(cos), _ptr(sin),
+                                          _ptr(pos), _ptr(slots), _ptr(k), _ptr(v), I(page), _stream()) == 0
+    x = (ref + bias.double()).view(M, H + 2 * KVH, D)
+    lo, hi = x[..., :D // 2], x[..., D // 2:]
+    c, s = (t.double()[pos.long()][:, None] for t in (cos, sin))
+    turned = torch.cat([lo * c - hi * s, hi * c + lo * s], -1)
+    bound = 2 * _bound(K) + 2.0 ** -21
+    assert (q.double().view(M, H, D) - turned[:, :H]).abs().max() <= bound
+    kept = slots >= 0
+    at = slots[kept].long()
+    keys, values = k.view(-1, KVH, D), v.permute(0, 3, 1, 2).reshape(-1, KVH, D)
+    assert (keys[at].double() - turned[kept, H:H + KVH]).abs().max() <= bound
+    assert (values[at].double() - x[kept, H + KVH:]).abs().max() <= bound
+    others = torch.ones(3 * page, dtype=torch.bool, device="cuda")
+    others[at] = False
+    assert (keys[others] == 7).all() and (values[others] == 7).all()
+
+
+CONTEXTS = [1, 16, 17, 127, 128, 129, 700, 1024, 1500]
+
+
+@pytest.mark.parametrize("extras", ["plain", "window", "window+keep", "cap+sink+gate"])
+@pytest.mark.parametrize("H,KVH,D,page", [(14, 2, 64, 16), (5, 5, 32, 64), (16, 1, 128, 16)])
+def test_attention_of_single_tokens(H, KVH, D, page, extras):
+    g = torch.Generator(device="cuda").manual_seed(H + D)
+    S, W = len(CONTEXTS), -(-max(CONTEXTS) // page)
+    window, keep = (150 if "window" in extras else 0), (20 if "keep" in extras else 0)
+    cap = 3.0 if "cap" in extras else 0.0
+    sink = torch.randn(H, generator=g, device="cuda") if "sink" in extras else None
+    gate = torch.randn(S, H * D, generator=g, device="cuda") if "gate" in extras else None
+    q = torch.randn(S, H * D, generator=g, device="cuda") * 2
+    pages = S * W + 1
+    k, v = torch.randn(pages, page, KVH, D, generator=g, device="cuda"), torch.randn(pages, KVH, D, page, generator=g, device="cuda")
+    k[0], v[0] = float("nan"), float("nan")                     # what released and padding entries of a table point at
+    table = torch.zeros(S, W, dtype=torch.int32, device="cuda")
+    out = torch.full((S, H * D), float("nan"), device="cuda")
+    wants = []
+    for s, ctx in enumerate(CONTEXTS):
+        ids = torch.arange(1 + s * W, 1 + s * W + -(-ctx // page), device="cuda", dtype=torch.int32)
+        seen = torch.arange(ctx, device="cuda")
+        lo = max(0, ctx - window) if window else 0
+        seen = seen[(seen >= lo) | (seen < keep)]
+        for j in range(len(ids)):                               # pages that no seen key lies in have been given back
+            if not ((seen // page) == j).any():
+                ids[j] = 0
+        table[s, :len(ids)] = ids
+        at = ids[(seen // page).long()].long()
+        kk, vv = k[at, seen % page].double(), v[at, :, :, seen % page].double()         # [keys, KVH, D]
+        v[ids[-1].long(), :, :, (ctx - 1) % page + 1:] = float("nan")                   # places beyond the newest key
+        k[ids[-1].long(), (ctx - 1) % page + 1:] = float("nan")
+        for h in range(H):
+            sc = kk[:, h // (H // KVH)] @ q[s, h * D:(h + 1) * D].double() * D ** -0.5
+            if cap:
+                sc = cap * torch.tanh(sc / cap)
+            e = torch.exp(sc - sc.max())
+            total = e.sum() + (torch.exp(sink[h].double() - sc.max()) if sink is not None else 0)
+            o = (e / total) @ vv[:, h // (H // KVH)]
+            wants.append(o * torch.sigmoid(gate[s, h * D:(h + 1) * D].double()) if gate is not None else o)
+    ctxs = torch.tensor(CONTEXTS, dtype=torch.int32, device="cuda")
+    chunks = -(-W * page // 128) + 1
+    part_o, part_ml = (torch.full((S * H * chunks * n,), float("nan"), device="cuda") for n in (D, 2))
+    assert library().tm_attn_decode_f32(_ptr(q), I(H * D), _ptr(out), I(H * D), _ptr(k), _ptr(v), _ptr(table), I(W), _ptr(ctxs), _ptr(part_o),
+                                        _ptr(part_ml), I(chunks), I(S), I(H), I(KVH), I(D), I(page), F(D ** -0.5), I(window), I(keep), F(cap),
+                                        _ptr(sink), _ptr(gate), I(H * D), _stream()) == 0
+    want = torch.stack(wants).view(S, H * D)
+    # scores of size up to about 10 with 32-bit dot products: 2^-20 absolute, which the exponential makes relative; values of size up to 5
+    assert (out.double() - want).abs().max() <= 2.0 ** -17

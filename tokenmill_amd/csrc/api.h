@@ -49,6 +49,26 @@ int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void* W, const 
 int tm_tile_linear_parts(int M, int N, int K);
 int tm_tile_linear_split(const void* A, int lda, int M, int K, const void* W, int N, float* parts, hipStream_t stream);
 
+// The true 32-bit path's products of at most 16 rows on the 32-bit matrix unit (gemv_f32.hip): K a multiple of 16, N of 4, 16-byte
+// pieces (tm_gemv_f32_mfma_takes). A plain product; 32-bit partial sums [parts][M][N] (tm_gemv_f32_parts says how many);
+// silu(gate) * up; q|k|v with bias, rotation over the whole head (head sizes that are multiples of 32) and cache write.
+int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, const void* bias, int M, int N, int K);
+int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K, hipStream_t stream);
+int tm_gemv_f32_parts(int N, int K);
+int tm_gemv_f32_mfma_split(const float* A, int lda, const float* W, float* parts, int M, int N, int K, hipStream_t stream);
+int tm_gemv_f32_gate_up_silu(const float* A, int lda, const float* W, float* act, int M, int I, int K, hipStream_t stream);
+int tm_gemv_f32_qkv_rope(const float* A, int lda, const float* W, const float* bias, float* q, int M, int K, int H, int KVH, int D,
+                         const float* cos_t, const float* sin_t, const int* positions, const int* slots, float* k_pool, float* v_pool,
+                         int page, hipStream_t stream);
+
+// Attention of single tokens in 32-bit (attention_decode_f32.hip): as tm_attn_decode_mfma_cap with chunks of 128 keys; part_o float
+// [S, H, max_chunks, D], part_ml [S, H, max_chunks, 2].
+int tm_attn_decode_f32_takes(const void* q, int q_stride, const void* k_pool, const void* v_pool, int H, int KVH, int D, int page);
+int tm_attn_decode_f32(const float* q, int q_stride, float* out, int out_stride, const float* k_pool, const float* v_pool,
+                       const int* block_tables, int table_width, const int* context_lens, float* part_o, float* part_ml, int max_chunks, int S,
+                       int H, int KVH, int D, int page, float scale, int window, int keep, float softcap, const float* sink, const float* cgate,
+                       int ldcg, hipStream_t stream);
+
 int tm_attn_paged_generic(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
                           const void* v_pool, const int* block_tables, int table_width, const int* seq_of_token,
                           const int* positions, int T, int H, int KVH, int D, int page, float scale, int window,

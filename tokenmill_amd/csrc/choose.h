@@ -39,6 +39,7 @@ constexpr int TM_GEMV_F32_ROWS = 16;
 
 // --- decode attention ---------------------------------------------------------------------------------
 constexpr int TM_DECODE_CHUNK = 256;        // keys per block of the split decode attention
+constexpr int TM_DECODE_F32_CHUNK = 128;    // the same in the 32-bit path, whose contexts are always split below that many pairs
 constexpr int TM_DECODE_SPLIT_PAIRS = 192;  // below this many (request, kv head) pairs the split kernels run
 
 inline int tm_decode_chunks(int max_context) { return (max_context + TM_DECODE_CHUNK - 1) / TM_DECODE_CHUNK; }

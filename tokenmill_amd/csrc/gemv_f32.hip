@@ -1,0 +1,256 @@
+// The true 32-bit path's products of at most 16 rows (decode steps), on the 32-bit matrix unit: a plain product (with bias, or as
+// 32-bit partial sums of a K split over blocks, which the next norm adds), gate|up with SiLU*up, q|k|v with bias, rotation and
+// cache write.
+//
+// Such a product is bound by reading its matrix once (35 MB for gate|up of the 0.5B shape) and, where that is small, by the trips to
+// memory. A block takes RT tiles of 16 matrix rows (SiLU and q|k|v: one, of 8 rows and the 8 that meet them, twice the blocks);
+// its wavefronts split K into runs of steps of 16 k and ask for several steps of matrix and activations at once, in the matrix
+// instruction's own layout (lane (r, g): 16 bytes of row r at 4 g), so nothing goes through LDS but the wavefronts' sums at the
+// end, added in wavefront order. The activations come from the second-level cache. Which k goes where depends on the matrix
+// alone: a row's result does not depend on the other rows. Non-temporal loads cost a tenth here: a line's two halves are
+// asked for by two instructions.
+// Before, a wavefront had 256 k of four rows, a lane 4 k each, and summed over the lanes by shuffles, 6 x 32 of them a wavefront:
+// 19.0 us a product of the 0.5B shape on average, with SiLU*up and rotation in kernels behind it; now gate|up takes 12 us (2.9
+// TB/s), down 7, q|k|v and o 5, the head 126 (4.3 TB/s).
+#include "common.h"
+#include "api.h"
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+enum { GM_PLAIN = 0, GM_SILU = 1, GM_QKV = 2 };
+
+struct GemvArgs {
+    const float* A;             // [M, K], rows lda apart
+    const float* W;             // [rows, K]
+    const float* bias;          // [rows] or null
+    float* C;                   // [M, N] rows ldc apart; SiLU: [M, I]; q|k|v: q [M, H D]
+    float* parts;               // [gridDim.y][M][N] instead of C, or null
+    int lda, ldc, M, N, K;
+    int I;
+    int H, KVH, D, page_shift;
+    const float* cos_t;         // [positions, D / 2]
+    const float* sin_t;
+    const int* positions;
+    const int* slots;           // or null
+    float* k_pool;              // [pages, page, KVH, D]
+    float* v_pool;              // [pages, KVH, D, page]
+};
+
+// AHEAD: steps of 16 k a wavefront asks for at once
+template <int EPI, int RT, int WAVES, int AHEAD>
+__global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArgs a) {
+    static_assert(EPI == GM_PLAIN || RT == 1, "");
+    __shared__ __align__(16) f32x4_t red[WAVES][RT][TM_WAVE];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;
+    const int r = lane % 16, g = lane / 16;
+    const int u = blockIdx.x;
+    // the first rows of the tiles
+    int n0[RT], head = 0, j0 = 0;
+    int far = 0;                                                // SiLU, q|k|v: how far on the rows of the tile's second half are
+    if constexpr (EPI == GM_SILU) {                             // 8 gate rows and the 8 up rows that meet them
+        n0[0] = 8 * u;
+        far = a.I;
+    } else if constexpr (EPI == GM_QKV) {                       // 8 channels of a head and the 8 they are rotated with
+        const int per_head = a.D / 16;
+        head = u / per_head;
+        j0 = 8 * (u - head * per_head);
+        n0[0] = head * a.D + j0;
+        far = a.D / 2;
+    } else {
+#pragma unroll
+        for (int t = 0; t < RT; ++t) n0[t] = (u * RT + t) * 16;
+    }
+    const int steps = a.K / 16;
+    const int per_block = (steps + gridDim.y - 1) / gridDim.y;
+    const int b0 = blockIdx.y * per_block, b1 = b0 + per_block < steps ? b0 + per_block : steps;
+    const int per = (per_block + WAVES - 1) / WAVES;
+    const int s0 = b0 + wave * per, s1 = s0 + per < b1 ? s0 + per : b1;
+    const float* pa = a.A + (size_t)(r < a.M ? r : a.M - 1) * a.lda + 4 * g;
+    const float* pw[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        // (rows beyond the matrix, or the half: its last one, never stored)
+        const int end = EPI == GM_SILU ? a.I : a.N, at = n0[t] + (EPI == GM_PLAIN ? r : r % 8);
+        const int n = (at < end ? at : end - 1) + (EPI != GM_PLAIN && r >= 8 ? far : 0);
+        pw[t] = a.W + (size_t)n * a.K + 4 * g;
+    }
+    // what the epilogue waits for otherwise
+    int pos = 0, slot = -1;
+    if constexpr (EPI == GM_QKV) {
+        pos = a.positions[r < a.M ? r : a.M - 1];
+        slot = a.slots ? a.slots[r < a.M ? r : a.M - 1] : -1;
+    }
+    f32x4_t sum[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) sum[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < s1; s += AHEAD) {
+        f32x4_t w[RT][AHEAD], x[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const int at = 16 * (s + i < s1 ? s + i : s1 - 1);  // (no load under a test: beyond the end the last step again)
+#pragma unroll
+            for (int t = 0; t < RT; ++t) w[t][i] = *(const f32x4_t*)(pw[t] + at);
+            x[i] = *(const f32x4_t*)(pa + at);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // four sums a tile, of every fourth k, that join the running one here: short chains of roundings
+        f32x4_t acc[RT][4];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[t][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            if (s + i >= s1) break;                             // the same for the whole wavefront
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int t = 0; t < RT; ++t)
+                    acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i][e], x[i][e], acc[t][e], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < RT; ++t) sum[t] += (acc[t][0] + acc[t][1]) + (acc[t][2] + acc[t][3]);
+    }
+#pragma unroll
+    for (int t = 0; t < RT; ++t) red[wave][t][lane] = sum[t];
+    __syncthreads();
+    // lane (r, g): row r of A, rows 4 g .. + 3 of the tile
+    if (EPI == GM_PLAIN ? wave >= RT : wave > 0 || g >= 2) return;
+    auto total = [&](int t, int of) {
+        f32x4_t v = red[0][t][of];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) v += red[w][t][of];
+        return v;
+    };
+    if constexpr (EPI == GM_PLAIN) {
+        const int n = n0[0] + 16 * wave + 4 * g;
+        if (r >= a.M || n >= a.N) return;                       // N is a multiple of 4: a piece is whole or absent
+        f32x4_t v = total(wave, lane);
+        if (a.parts) {
+            *(f32x4_t*)(a.parts + ((size_t)blockIdx.y * a.M + r) * a.N + n) = v;
+            return;
+        }
+        if (a.bias) v += *(const f32x4_t*)(a.bias + n);
+        *(f32x4_t*)(a.C + (size_t)r * a.ldc + n) = v;
+    } else if constexpr (EPI == GM_SILU) {
+        const int c = n0[0] + 4 * g;
+        if (r >= a.M || c >= a.I) return;
+        const f32x4_t gt = total(0, lane), up = total(0, lane + 32);
+        f32x4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = gt[e] / (1.f + expf(-gt[e])) * up[e];
+        *(f32x4_t*)(a.C + (size_t)r * a.ldc + c) = v;
+    } else {
+        if (r >= a.M) return;
+        f32x4_t x = total(0, lane), y = total(0, lane + 32);
+        if (a.bias) {
+            x += *(const f32x4_t*)(a.bias + n0[0] + 4 * g);
+            y += *(const f32x4_t*)(a.bias + n0[0] + far + 4 * g);
+        }
+        const int d = j0 + 4 * g;
+        if (head < a.H + a.KVH) {
+            const size_t at = (size_t)pos * (a.D / 2) + d;
+            const f32x4_t c = *(const f32x4_t*)(a.cos_t + at), s = *(const f32x4_t*)(a.sin_t + at);
+            f32x4_t y1, y2;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float p, q;
+                rotate_pair(x[e], y[e], c[e], s[e], p, q);
+                y1[e] = p;
+                y2[e] = q;
+            }
+            float* dst = nullptr;
+            if (head < a.H) dst = a.C + (size_t)r * a.ldc + head * a.D + d;
+            else if (slot >= 0) dst = a.k_pool + ((size_t)slot * a.KVH + (head - a.H)) * a.D + d;
+            if (dst) {
+                *(f32x4_t*)dst = y1;
+                *(f32x4_t*)(dst + a.D / 2) = y2;
+            }
+        } else if (slot >= 0) {
+            const int vh = head - a.H - a.KVH;
+            const int pg = slot >> a.page_shift, in_page = slot & ((1 << a.page_shift) - 1);
+            float* dst = a.v_pool + ((((size_t)pg * a.KVH + vh) * a.D + d) << a.page_shift) + in_page;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                dst[(size_t)e << a.page_shift] = x[e];
+                dst[(size_t)(a.D / 2 + e) << a.page_shift] = y[e];
+            }
+        }
+    }
+}
+
+static bool gm_aligned16(const void* p) { return p && ((uintptr_t)p % 16) == 0; }
+
+// Whole 16-byte pieces, k in whole steps of 16.
+extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, const void* bias, int M, int N, int K) {
+    return M > 0 && M <= 16 && N > 0 && N % 4 == 0 && K >= 16 && K % 16 == 0 && lda >= K && lda % 4 == 0 && gm_aligned16(A) && gm_aligned16(W) &&
+           (!bias || gm_aligned16(bias));
+}
+
+// Up to a block a CU, eight wavefronts split K and ask for four steps at a time; more blocks than that have four wavefronts with
+// seven (0.5B shape, eight rows: down 7.1 us against 8.2 to 9.0 for the other combinations of 4, 8, 16 and 4, 7; gate|up 12.1
+// against 12.0 to 13.7, head 126 against 127 to 131).
+#define GM_LAUNCH(EPI, RT, units, split)                                                                                    \
+    do {                                                                                                                    \
+        if ((units) * (split) <= 256) gemv_mfma_f32_kernel<EPI, RT, 8, 4><<<dim3(units, split), 512, 0, stream>>>(a);       \
+        else gemv_mfma_f32_kernel<EPI, RT, 4, 7><<<dim3(units, split), 256, 0, stream>>>(a);                                \
+    } while (0)
+
+extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,
+                                hipStream_t stream) {
+    if (!tm_gemv_f32_mfma_takes(A, lda, W, bias, M, N, K) || !gm_aligned16(C) || ldc < N || ldc % 4) return TM_ERR_ARG;
+    GemvArgs a{};
+    a.A = A; a.W = W; a.bias = bias; a.C = C; a.lda = lda; a.ldc = ldc; a.M = M; a.N = N; a.K = K;
+    // two tiles a block read the activations once for both, where that still gives every CU a block
+    const int two = (N + 31) / 32, one = (N + 15) / 16;
+    if (two >= 256) GM_LAUNCH(GM_PLAIN, 2, two, 1);
+    else GM_LAUNCH(GM_PLAIN, 1, one, 1);
+    TM_CHECK_LAUNCH();
+    return TM_OK;
+}
+
+// Parts that K is split into where 16-row tiles are too few for the chip (a part keeps at least 32 steps of 16 k, two a wavefront).
+extern "C" int tm_gemv_f32_parts(int N, int K) {
+    const int units = (N + 15) / 16;
+    int parts = 1;
+    while (parts < 8 && units * parts * 2 <= 256 && K / 16 / (parts * 2) >= 32) parts *= 2;
+    return parts;
+}
+
+// parts[p][m][n], p < tm_gemv_f32_parts(N, K)
+extern "C" int tm_gemv_f32_mfma_split(const float* A, int lda, const float* W, float* parts, int M, int N, int K, hipStream_t stream) {
+    if (!tm_gemv_f32_mfma_takes(A, lda, W, nullptr, M, N, K) || !gm_aligned16(parts)) return TM_ERR_ARG;
+    GemvArgs a{};
+    a.A = A; a.W = W; a.parts = parts; a.lda = lda; a.M = M; a.N = N; a.K = K;
+    const int units = (N + 15) / 16;
+    GM_LAUNCH(GM_PLAIN, 1, units, tm_gemv_f32_parts(N, K));
+    TM_CHECK_LAUNCH();
+    return TM_OK;
+}
+
+// act[m, i] = silu(gate) * up, W [2 I, K]
+extern "C" int tm_gemv_f32_gate_up_silu(const float* A, int lda, const float* W, float* act, int M, int I, int K, hipStream_t stream) {
+    if (I <= 0 || I % 4 || !gm_aligned16(act) || !tm_gemv_f32_mfma_takes(A, lda, W, nullptr, M, 2 * I, K)) return TM_ERR_ARG;
+    GemvArgs a{};
+    a.A = A; a.W = W; a.C = act; a.lda = lda; a.ldc = I; a.M = M; a.N = 2 * I; a.K = K; a.I = I;
+    GM_LAUNCH(GM_SILU, 1, (I + 7) / 8, 1);
+    TM_CHECK_LAUNCH();
+    return TM_OK;
+}
+
+// as tm_tile_qkv_rope, in 32-bit; head sizes that are multiples of 32
+extern "C" int tm_gemv_f32_qkv_rope(const float* A, int lda, const float* W, const float* bias, float* q, int M, int K, int H, int KVH, int D,
+                                    const float* cos_t, const float* sin_t, const int* positions, const int* slots, float* k_pool,
+                                    float* v_pool, int page, hipStream_t stream) {
+    const int N = (H + 2 * KVH) * D;
+    if (H <= 0 || KVH <= 0 || D <= 0 || D % 32 || !gm_aligned16(q) || !gm_aligned16(cos_t) || !gm_aligned16(sin_t) || !positions || page <= 0 ||
+        (page & (page - 1)) || (slots && (!gm_aligned16(k_pool) || !v_pool)) || !tm_gemv_f32_mfma_takes(A, lda, W, bias, M, N, K))
+        return TM_ERR_ARG;
+    GemvArgs a{};
+    a.A = A; a.W = W; a.bias = bias; a.C = q; a.lda = lda; a.ldc = H * D; a.M = M; a.N = N; a.K = K;
+    a.H = H; a.KVH = KVH; a.D = D; a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots; a.k_pool = k_pool; a.v_pool = v_pool;
+    while ((1 << a.page_shift) < page) ++a.page_shift;
+    GM_LAUNCH(GM_QKV, 1, N / 16, 1);
+    TM_CHECK_LAUNCH();
+    return TM_OK;
+}

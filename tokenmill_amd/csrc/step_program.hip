@@ -98,6 +98,12 @@ bool tile_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype) {
     return dtype == TM_BF16 && L.dtype == TM_BF16 && !L.act && M > TM_SKINNY_ROWS && tm_gemm_tile_takes(x, ldx, L.w, M, L.N, L.K);
 }
 
+// the 32-bit path's products of few rows with their epilogues (gemv_f32.hip)
+bool gemv32_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype) {
+    return dtype == TM_F32 && L.dtype == TM_F32 && !L.act && (!L.bias || L.bias_dtype == TM_F32) && M <= TM_GEMV_F32_ROWS &&
+           tm_gemv_f32_mfma_takes(x, ldx, L.w, L.bias, M, L.N, L.K);
+}
+
 // Parts of K for an output or down projection of M rows beyond the stream kernels' whose 32-bit sums the next norm adds up; 0: none.
 int tile_parts(const TmLinear& L, int M) {
     if (M <= TM_STREAM_ROWS || L.dtype != TM_BF16 || L.bias || L.act) return 0;
@@ -146,6 +152,8 @@ struct Products {
                                          out_dtype, ep, nullptr, 0, stream);
         if (dtype != TM_BF16) {
             const bool plain32 = out_dtype == TM_F32 && (L.bias_dtype == TM_NONE || L.bias_dtype == TM_F32);
+            if (plain32 && M <= TM_GEMV_F32_ROWS && ldc % 4 == 0 && aligned(out, 16) && tm_gemv_f32_mfma_takes(x, ldx, L.w, L.bias, M, L.N, L.K))
+                return then_act(tm_gemv_f32_mfma((const float*)x, ldx, (const float*)L.w, (const float*)L.bias, (float*)out, ldc, M, L.N, L.K, stream));
             if (plain32 && M <= TM_GEMV_F32_ROWS && L.K % 4 == 0 && ldx % 4 == 0 && aligned(x, 16) && aligned(L.w, 16))
                 return then_act(tm_gemv_f32((const float*)x, ldx, (const float*)L.w, (const float*)L.bias, (float*)out, ldc, M, L.N, L.K, stream));
             if (plain32 && tm_gemm_f32_mfma_fits(x, ldx, L.w, L.bias, out, ldc, M, L.N, L.K))
@@ -190,6 +198,12 @@ struct Products {
         return tm_gemm_skinny(x, ldx, L.w, L.bias, L.bias_dtype, nullptr, L.N, M, L.N, L.K, TM_BF16, 0, accum, ldacc, stream);
     }
 };
+
+// chunks that the decode attention's partial results have room for
+int program_chunks(const TmProgram* p, int max_decode_context) {
+    const int n = max_decode_context > 0 ? max_decode_context : 1;
+    return p->dtype == TM_F32 ? (n + TM_DECODE_F32_CHUNK - 1) / TM_DECODE_F32_CHUNK : tm_decode_chunks(n);
+}
 
 struct Run {
     const TmProgram* p;
@@ -252,6 +266,16 @@ struct Run {
             delta = nullptr;
             pending_sums = parts;
             return TM_OK;
+        }
+        if (sums && accumulate && resid && L.N == p->hidden && !L.bias && gemv32_ok(L, x_, ldx, M, dtype)) {
+            const int parts32 = tm_gemv_f32_parts(L.N, L.K);
+            if (parts32 >= 2) {
+                const int rc = tm_gemv_f32_mfma_split((const float*)x_, ldx, (const float*)L.w, sums, M, L.N, L.K, stream);
+                if (rc) return rc;
+                delta = nullptr;
+                pending_sums = parts32;
+                return TM_OK;
+            }
         }
         if (accumulate && resid && products.accumulates(L, dtype, x_, ldx, M)) {
             delta = nullptr;
@@ -364,8 +388,16 @@ struct Run {
                     q = qkv;
                     q_stride = HD;
                     ++p->taken[TM_QKV_PLAIN];
+                } else if (tables_fusable && a.D % 32 == 0 && gemv32_ok(a.qkv, xn, hidden, T, dtype) && is_pow2(a.page) &&
+                           aligned(a.cos_t, 16) && aligned(a.sin_t, 16) && (!a.write || aligned(a.k_pool, 16))) {
+                    // 5. the same in 32-bit, for few tokens
+                    rc = tm_gemv_f32_qkv_rope((const float*)xn, hidden, (const float*)a.qkv.w, (const float*)a.qkv.bias, (float*)qkv, T, hidden,
+                                              a.H, a.KVH, a.D, a.cos_t, a.sin_t, s->positions, slots, (float*)kp, (float*)vp, a.page, stream);
+                    q = qkv;
+                    q_stride = HD;
+                    ++p->taken[TM_QKV_PLAIN];
                 } else {
-                    // 5. product, then rotation and cache write
+                    // 6. product, then rotation and cache write
                     if ((rc = linear(a.qkv, xn, hidden, T, qkv, QKV, dtype))) return rc;
                     if (a.rot > 0 || a.write)
                         rc = tm_rope_kv_write(qkv, dtype, T, a.H, a.KVH, a.D, a.rot, a.rot > 0 ? a.cos_t : nullptr,
@@ -415,6 +447,14 @@ struct Run {
                                              s->context_lens + (S - nd), split ? part_o : nullptr, split ? part_ml : nullptr,
                                              tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep,
                                              a.softcap, a.sink, cg_dec, cgate_ld, stream);
+                done_decode = true;
+            } else if (nd && dtype == TM_F32 && nd * a.KVH < TM_DECODE_SPLIT_PAIRS &&
+                       tm_attn_decode_f32_takes(q_dec, q_stride, a.k_pool, a.v_pool, a.H, a.KVH, a.D, a.page)) {
+                // (beyond that many pairs the generic kernel's blocks of one (token, head) pair fill the chip)
+                rc = tm_attn_decode_f32((const float*)q_dec, q_stride, (float*)out_dec, HD, (const float*)a.k_pool, (const float*)a.v_pool,
+                                        tables + (size_t)(S - nd) * W, W, s->context_lens + (S - nd), part_o, part_ml,
+                                        program_chunks(p, s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep, a.softcap,
+                                        a.sink, (const float*)cg_dec, cgate_ld, stream);
                 done_decode = true;
             }
             if (rc) return rc;
@@ -474,6 +514,9 @@ struct Run {
                     ++p->taken[TM_GATE_UP_PLAIN];
                 } else if (plain && f.I % 8 == 0 && tile_ok(f.gate_up, xn, hidden, T, dtype)) {
                     rc = tm_tile_gate_up_silu(xn, hidden, T, hidden, f.gate_up.w, act, f.I, stream);
+                    ++p->taken[TM_GATE_UP_PLAIN];
+                } else if (plain && f.I % 4 == 0 && gemv32_ok(f.gate_up, xn, hidden, T, dtype)) {
+                    rc = tm_gemv_f32_gate_up_silu((const float*)xn, hidden, (const float*)f.gate_up.w, (float*)act, T, f.I, hidden, stream);
                     ++p->taken[TM_GATE_UP_PLAIN];
                 } else {
                     if ((rc = linear(f.gate_up, xn, hidden, T, gu, 2 * f.I, dtype))) return rc;
@@ -600,12 +643,12 @@ void tm_program_counters(const TmProgram* p, long long* out) {
 
 // Most parts that a product's K is split into in a step of T tokens (their sums [T, hidden] are kept until the next norm).
 static int program_sums(const TmProgram* p, int T) {
-    if (p->dtype != TM_BF16) return 0;
-    if (T <= TM_STREAM_ROWS) return TM_MAX_SUMS;
+    if (p->dtype == TM_BF16 && T <= TM_STREAM_ROWS) return TM_MAX_SUMS;
+    if (p->dtype == TM_F32 && T > TM_GEMV_F32_ROWS) return 0;
     int most = 0;
     for (const Op& op : p->ops) {
         const TmLinear* L = op.kind == OP_ATTENTION ? &op.att.o : op.kind == OP_FEED_FORWARD ? &op.ffn.down : nullptr;
-        const int parts = L ? tile_parts(*L, T) : 0;
+        const int parts = !L ? 0 : p->dtype == TM_F32 ? tm_gemv_f32_parts(L->N, L->K) : tile_parts(*L, T);
         if (parts > most) most = parts;
     }
     return most;
@@ -624,7 +667,7 @@ size_t tm_program_workspace_bytes(const TmProgram* p, int T, int R, int num_deco
     n += align_up((size_t)T * p->max_act * es);                      // silu(gate) * up
     n += align_up((size_t)T * p->hidden * es);                       // a product's output still to be added
     n += align_up((size_t)(R > 0 ? R : 1) * p->hidden * es);         // normed rows for the head
-    const size_t chunks = (size_t)tm_decode_chunks(max_decode_context > 0 ? max_decode_context : 1);
+    const size_t chunks = (size_t)program_chunks(p, max_decode_context);
     n += align_up((size_t)num_decode * p->max_heads_d * chunks * 4); // split decode attention: partial values
     n += align_up((size_t)num_decode * p->max_heads * chunks * 2 * 4);   // ... and their (max, sum)
     n += align_up((size_t)program_sums(p, T) * T * p->hidden * 4);   // partial sums of a product whose K is split over blocks
@@ -672,7 +715,7 @@ int tm_program_run(const TmProgram* p, int first, int count, const TmStep* s, Tm
     r.act = take((size_t)T * p->max_act * es);
     r.delta_buf = take((size_t)T * p->hidden * es);
     r.hnorm = take((size_t)(R > 0 ? R : 1) * p->hidden * es);
-    const size_t chunks = (size_t)tm_decode_chunks(s->max_decode_context > 0 ? s->max_decode_context : 1);
+    const size_t chunks = (size_t)program_chunks(p, s->max_decode_context);
     r.part_o = (float*)take((size_t)s->num_decode * p->max_heads_d * chunks * 4);
     r.part_ml = (float*)take((size_t)s->num_decode * p->max_heads * chunks * 2 * 4);
     const int parts = program_sums(p, T);
