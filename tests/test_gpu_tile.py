@@ -106,6 +106,71 @@ def test_partial_sums_of_a_split_k(M, N, K):
     assert (out.double().sum(0) - ref).abs().max() <= 2.0 ** -24 * 5 * 4 * K ** 0.5
 
 
+def _operands32(M, N, K, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    a, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") * K ** -0.5
+    return a, w, a.double() @ w.double().T
+
+
+# 32-bit sums in blocks of 128 k: a chain of 128 additions in a block, then K / 128 of sums of at most about 5
+def _bound32(K):
+    return 2.0 ** -24 * 5 * (6 + (K / 128) ** 0.5) * 2
+
+
+@pytest.mark.parametrize("M,n,K", [(17, 8, 128), (65, 40, 160), (333, 1000, 896), (1000, 4864, 896)])
+def test_gate_up_silu_in_32_bit(M, n, K):
+    a, w, ref = _operands32(M, 2 * n, K, M + n)
+    out = torch.full((M, n), float("nan"), device="cuda")
+    assert library().tm_tile_f32_gate_up_silu(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), P(out.data_ptr()), I(n), _stream()) == 0
+    gate, up = ref.chunk(2, 1)
+    want = torch.nn.functional.silu(gate) * up
+    assert ((out.double() - want).abs() <= _bound32(K) * (1.1 * up.abs() + gate.abs() + 1) + 2.0 ** -20 * want.abs()).all()
+
+
+@pytest.mark.parametrize("M,H,KVH,D,K", [(17, 3, 1, 64, 128), (333, 14, 2, 64, 896), (130, 4, 2, 128, 224)])
+def test_qkv_in_32_bit(M, H, KVH, D, K):
+    N, page = (H + 2 * KVH) * D, 16
+    a, w, ref = _operands32(M, N, K, M + H)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    bias = torch.randn(N, generator=g, device="cuda")
+    angle = torch.rand(300, D // 2, generator=g, device="cuda") * 6.28
+    cos, sin = angle.cos(), angle.sin()
+    pos = torch.randint(0, 300, (M,), generator=g, device="cuda", dtype=torch.int32)
+    pages = -(-M // page) + 2
+    slots = torch.randperm(pages * page, generator=g, device="cuda")[:M].int()
+    slots[1::7] = -1
+    q = torch.empty(M, H * D, device="cuda")
+    k, v = torch.full((pages, page, KVH, D), 7.0, device="cuda"), torch.full((pages, KVH, D, page), 7.0, device="cuda")
+    assert library().tm_tile_f32_qkv_rope(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), P(bias.data_ptr()), P(q.data_ptr()), I(H), I(KVH), I(D),
+                                          P(cos.data_ptr()), P(sin.data_ptr()), P(pos.data_ptr()), P(slots.data_ptr()), P(k.data_ptr()),
+                                          P(v.data_ptr()), I(page), _stream()) == 0
+    x = (ref + bias.double()).view(M, H + 2 * KVH, D)
+    lo, hi = x[..., :D // 2], x[..., D // 2:]
+    c, s = (t.double()[pos.long()][:, None] for t in (cos, sin))
+    turned = torch.cat([lo * c - hi * s, hi * c + lo * s], -1)
+    bound = 2 * _bound32(K) + 2.0 ** -20
+    assert (q.double().view(M, H, D) - turned[:, :H]).abs().max() <= bound
+    kept = slots >= 0
+    at = slots[kept].long()
+    keys, values = k.view(-1, KVH, D), v.permute(0, 3, 1, 2).reshape(-1, KVH, D)
+    assert (keys[at].double() - turned[kept, H:H + KVH]).abs().max() <= bound
+    assert (values[at].double() - x[kept, H + KVH:]).abs().max() <= bound
+    others = torch.ones(pages * page, dtype=torch.bool, device="cuda")
+    others[at] = False
+    assert (keys[others] == 7).all() and (values[others] == 7).all()
+
+
+@pytest.mark.parametrize("splits", [0, 1, 3])
+@pytest.mark.parametrize("M,N,K", [(17, 8, 384), (333, 896, 896), (1000, 896, 4864)])
+def test_products_and_partial_sums_in_32_bit(M, N, K, splits):
+    lib = library()
+    splits = splits or lib.tm_tile_f32_parts(M, N, K)
+    a, w, ref = _operands32(M, N, K, M + K)
+    out = torch.full((splits, M, N), float("nan"), device="cuda")
+    assert lib.tm_tile_f32_linear_split(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), I(N), P(out.data_ptr()), I(splits), _stream()) == 0
+    assert (out.double().sum(0) - ref).abs().max() <= _bound32(K)
+
+
 def test_what_the_kernels_do_not_take_is_refused():
     lib = library()
     a, w, _ = _operands(65, 128, 320, 1)

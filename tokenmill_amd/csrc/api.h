@@ -49,6 +49,15 @@ int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void* W, const 
 int tm_tile_linear_parts(int M, int N, int K);
 int tm_tile_linear_split(const void* A, int lda, int M, int K, const void* W, int N, float* parts, hipStream_t stream);
 
+// The same for the true 32-bit path (K a multiple of 32, tm_tile_f32_takes); tm_tile_f32_linear_split with one part stores the product.
+int tm_tile_f32_takes(const void* A, int lda, const void* W, int M, int N, int K);
+int tm_tile_f32_gate_up_silu(const void* A, int lda, int M, int K, const void* W, void* act, int I, hipStream_t stream);
+int tm_tile_f32_qkv_rope(const void* A, int lda, int M, int K, const void* W, const void* bias, void* q, int H, int KVH, int D,
+                         const float* cos_t, const float* sin_t, const int* positions, const int* slots, void* k_pool, void* v_pool,
+                         int page, hipStream_t stream);
+int tm_tile_f32_parts(int M, int N, int K);
+int tm_tile_f32_linear_split(const void* A, int lda, int M, int K, const void* W, int N, float* parts, int splits, hipStream_t stream);
+
 // The true 32-bit path's products of at most 16 rows on the 32-bit matrix unit (gemv_f32.hip): K a multiple of 16, N of 4, 16-byte
 // pieces (tm_gemv_f32_mfma_takes). A plain product; 32-bit partial sums [parts][M][N] (tm_gemv_f32_parts says how many);
 // silu(gate) * up; q|k|v with bias, rotation over the whole head (head sizes that are multiples of 32) and cache write.

@@ -26,8 +26,8 @@
 enum { GT_SILU = 0, GT_QKV = 1, GT_PARTS = 2 };
 
 struct TileArgs {
-    const bf16_t* A;            // [M, K], rows lda apart
-    const bf16_t* W;            // [rows, K]
+    const void* A;              // [M, K], rows lda apart
+    const void* W;              // [rows, K]
     const void* bias;           // [rows] or null
     void* C;                    // [M, N] rows ldc apart; PARTS: float [split][M][N]
     int M, N, K, lda, ldc;      // N: matrix rows (SiLU: twice I)
@@ -40,17 +40,37 @@ struct TileArgs {
     const float* sin_t;
     const int* positions;       // [M]
     const int* slots;           // [M]; < 0: not stored; or null
-    bf16_t* k_pool;             // [pages, page, KVH, D]
-    bf16_t* v_pool;             // [pages, KVH, D, page]
+    void* k_pool;               // [pages, page, KVH, D]
+    void* v_pool;               // [pages, KVH, D, page]
 };
+
+// An operand fragment: 16 bytes of a row, 8 bfloat16 or 4 float32 values
+union GtFrag {
+    u32x4_t u;
+    bf16x8_t b;
+    f32x4_t f;
+};
+
+// eight results of a row in the tensors' type, 16-byte stores
+template <typename T>
+__device__ __forceinline__ void gt_store8(T* dst, const float (&v)[8]) {
+    if constexpr (sizeof(T) == 4) {
+        *(f32x4_t*)dst = f32x4_t{v[0], v[1], v[2], v[3]};
+        *(f32x4_t*)(dst + 4) = f32x4_t{v[4], v[5], v[6], v[7]};
+    } else {
+        *(u32x4_t*)dst = u32x4_t{fd_pack(v[0], v[1]), fd_pack(v[2], v[3]), fd_pack(v[4], v[5]), fd_pack(v[6], v[7])};
+    }
+}
 
 // 16 bytes a lane from base + voff (bytes) to LDS at lds (bytes, wave-uniform) + 16 * lane
 __device__ __forceinline__ void gt_load_lds(uint32_t lds, uint32_t voff, const void* base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base));
 }
 
-// two values rounded to bfloat16 and back, by one conversion
+// two values rounded to the tensors' type and back, by one conversion
+template <typename T>
 __device__ __forceinline__ void gt_round2(float& a, float& b) {
+    if constexpr (sizeof(T) == 4) return;
     const uint32_t u = fd_pack(a, b);
     a = __uint_as_float(u << 16);
     b = __uint_as_float(u & 0xffff0000u);
@@ -98,7 +118,7 @@ __device__ __forceinline__ int gt_matrix_row(const TileArgs& a, int u, int q) {
 }
 
 // MT, NT: 16-row tiles of A and of the matrix a wavefront multiplies; WM x WN = 4 wavefronts; ST: buffers of the ring
-template <int EPI, int MT, int NT, int WM, int WN, int ST, int OCC>
+template <typename T, int EPI, int MT, int NT, int WM, int WN, int ST, int OCC>
 __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     extern __shared__ __align__(16) unsigned char gt_smem[];
     constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, ROWS = BM + BN;
@@ -108,26 +128,27 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;
     const int r = lane % 16, g = lane / 16;
     const int wm = wave / WN, wn = wave % WN;
-    const int ksteps = a.K / 64;
+    constexpr int ES = sizeof(T), KSTEP = 128 / ES;                 // a step is 128 bytes of every row
+    const int ksteps = a.K / KSTEP;
     const int per = (ksteps + a.splits - 1) / a.splits;             // k-steps of a part
 
     // --- the loading side: runs ahead of the products over the block's tiles ---
     uint32_t voff[NL];
-    const bf16_t *lA = a.A, *lW = a.W;
+    const unsigned char *lA = (const unsigned char*)a.A, *lW = (const unsigned char*)a.W;
     int l_p = blockIdx.x;
     bool l_more = true;
     auto next_load_tile = [&]() {
         int tm, tn, sp;
         if (!l_more || !gt_place(a, l_p, tm, tn, sp)) {             // no further tile: the same bytes again, never multiplied
             l_more = false;
-            lA = a.A;
-            lW = a.W;
+            lA = (const unsigned char*)a.A;
+            lW = (const unsigned char*)a.W;
             return;
         }
         l_p += gridDim.x;
         const int k0 = sp * per;
-        lA = a.A + (size_t)k0 * 64;
-        lW = a.W + (size_t)k0 * 64;
+        lA = (const unsigned char*)a.A + (size_t)k0 * 128;
+        lW = (const unsigned char*)a.W + (size_t)k0 * 128;
         const int in8 = lane / 8, at = lane % 8;
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
@@ -135,18 +156,18 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
             if (i < BM / 32) {
                 int m = tm * BM + R;
                 m = m < a.M ? m : a.M - 1;
-                voff[i] = (uint32_t)m * (uint32_t)a.lda * 2u + (uint32_t)((at ^ ((R >> 1) & 7)) * 16);
+                voff[i] = (uint32_t)m * (uint32_t)a.lda * ES + (uint32_t)((at ^ ((R >> 1) & 7)) * 16);
             } else {
                 const int Rb = R - BM;
                 const int n = gt_matrix_row<EPI>(a, tn * (BN / 64) + Rb / 64, Rb % 64);
-                voff[i] = (uint32_t)n * (uint32_t)a.K * 2u + (uint32_t)((at ^ (((Rb >> 1) & 1) | (((Rb >> 3) & 3) << 1))) * 16);
+                voff[i] = (uint32_t)n * (uint32_t)a.K * ES + (uint32_t)((at ^ (((Rb >> 1) & 1) | (((Rb >> 3) & 3) << 1))) * 16);
             }
         }
     };
     auto issue_one = [&](uint32_t dst, int i) { gt_load_lds(dst + i * 4096, voff[i], i < BM / 32 ? (const void*)lA : (const void*)lW); };
     auto issued = [&]() {
-        lA += l_more ? 64 : 0;
-        lW += l_more ? 64 : 0;
+        lA += l_more ? 128 : 0;
+        lW += l_more ? 128 : 0;
     };
 
     // --- the multiplying side ---
@@ -162,12 +183,32 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
         issued();
     }
 
-    f32x4_t acc[MT][NT];
+    // 32-bit operands: the accumulators hold the sum of a block of 128 k, which joins the running total at the block's end (one
+    // chain of roundings over all of K loses several times what a blocked sum does)
+    constexpr int TM_ = ES == 4 ? MT : 1, TN_ = ES == 4 ? NT : 1;
+    f32x4_t acc[MT][NT], total[TM_][TN_];
+    auto join = [&]() {
+        if constexpr (ES == 4) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+            for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    FFrag fa[2][MT], fb[2][NT];
+                for (int j = 0; j < NT; ++j) {
+                    total[i][j] += acc[i][j];
+                    acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    };
+    auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                if constexpr (ES == 4) total[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            }
+    };
+    clear();
+    GtFrag fa[2][MT], fb[2][NT];
     const int rb = 8 * (r / 4) + r % 4;
     const int offA = (wm * MT * 16 + r) * 128 + ((g ^ ((r >> 1) & 7)) << 4);
     const int offB = (BM + wn * NT * 16 + rb) * 128 + ((g ^ (((rb >> 1) & 1) | (((rb >> 3) & 3) << 1))) << 4);
@@ -175,6 +216,14 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     // buffer `from`) and, with dst, the loads of the step ST ahead. The order is the program's: the barriers between the groups
     // keep the compiler from gathering the reads.
     constexpr int READS = MT + NT, PRODUCTS = MT * NT;
+    auto multiply = [&](const GtFrag& w, const GtFrag& x, f32x4_t& c) {
+        if constexpr (ES == 4) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(w.f[e], x.f[e], c, 0, 0, 0);
+        } else {
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.b, x.b, c, 0, 0, 0);
+        }
+    };
     auto half_step = [&](auto HALF, int from, auto LOADS, uint32_t dst) {
         constexpr int half = decltype(HALF)::value, other = 1 - half;
         const unsigned char* pa = gt_smem + from * STAGE + (offA ^ (other * 64));
@@ -190,7 +239,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
             }
 #pragma unroll
             for (int n = q * PRODUCTS / READS; n < (q + 1) * PRODUCTS / READS; ++n)
-                acc[n / NT][n % NT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[half][n % NT].b, fa[half][n / NT].b, acc[n / NT][n % NT], 0, 0, 0);
+                multiply(fb[half][n % NT], fa[half][n / NT], acc[n / NT][n % NT]);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -219,6 +268,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
             }
         };
         if constexpr (EPI == GT_QKV && MT <= 5) read_places();
+        int block = 0;
         // the loads are ST steps ahead: those of the last ST steps are the next tile's
 #pragma unroll 1
         for (int part = 0; part < 2; ++part) {
@@ -234,9 +284,16 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                 asm volatile("" ::: "memory");
                 half_step(std::integral_constant<int, 1>{}, buf, std::true_type{}, dst);
                 issued();
+                if constexpr (ES == 4) {
+                    if (++block == 4) {
+                        block = 0;
+                        join();
+                    }
+                }
             }
         }
         // --- the tile's results ---
+        join();
         if constexpr (EPI == GT_QKV && MT > 5) read_places();
 #pragma unroll
         for (int un = 0; un < NT / 4; ++un) {
@@ -300,10 +357,11 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                 float x[8], y[8];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    x[e] = acc[i][4 * un][e];
-                    x[4 + e] = acc[i][4 * un + 1][e];
-                    y[e] = acc[i][4 * un + 2][e];
-                    y[4 + e] = acc[i][4 * un + 3][e];
+                    const int at = 4 * un;
+                    x[e] = ES == 4 ? total[ES == 4 ? i : 0][ES == 4 ? at : 0][e] : acc[i][at][e];
+                    x[4 + e] = ES == 4 ? total[ES == 4 ? i : 0][ES == 4 ? at + 1 : 0][e] : acc[i][at + 1][e];
+                    y[e] = ES == 4 ? total[ES == 4 ? i : 0][ES == 4 ? at + 2 : 0][e] : acc[i][at + 2][e];
+                    y[4 + e] = ES == 4 ? total[ES == 4 ? i : 0][ES == 4 ? at + 3 : 0][e] : acc[i][at + 3][e];
                 }
                 if (m >= a.M) continue;
                 if (EPI == GT_PARTS) {
@@ -321,13 +379,15 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                     float v[8];
 #pragma unroll
                     for (int e = 0; e < 8; e += 2) {
-                        gt_round2(x[e], x[e + 1]);
-                        gt_round2(y[e], y[e + 1]);
+                        gt_round2<T>(x[e], x[e + 1]);
+                        gt_round2<T>(y[e], y[e + 1]);
                     }
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) v[e] = x[e] * __builtin_amdgcn_rcpf(1.f + __expf(-x[e])) * y[e];
-                    *(u32x4_t*)((bf16_t*)a.C + (size_t)m * a.ldc + c0) =
-                        u32x4_t{fd_pack(v[0], v[1]), fd_pack(v[2], v[3]), fd_pack(v[4], v[5]), fd_pack(v[6], v[7])};
+                    for (int e = 0; e < 8; ++e) {
+                        if constexpr (ES == 4) v[e] = x[e] / (1.f + expf(-x[e])) * y[e];
+                        else v[e] = x[e] * __builtin_amdgcn_rcpf(1.f + __expf(-x[e])) * y[e];     // (far closer than the bfloat16 it becomes)
+                    }
+                    gt_store8((T*)a.C + (size_t)m * a.ldc + c0, v);
                 } else {
                     if (!ok0) continue;
 #pragma unroll
@@ -337,30 +397,29 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                     }
 #pragma unroll
                     for (int e = 0; e < 8; e += 2) {
-                        gt_round2(x[e], x[e + 1]);
-                        gt_round2(y[e], y[e + 1]);
+                        gt_round2<T>(x[e], x[e + 1]);
+                        gt_round2<T>(y[e], y[e + 1]);
                     }
                     const int row_slot = slot[EPI == GT_QKV ? i : 0];
                     if (head < a.H + a.KVH) {
                         float y1[8], y2[8];
 #pragma unroll
                         for (int e = 0; e < 8; ++e) rotate_pair(x[e], y[e], cs[i % AHEAD][e / 4][e % 4], sn[i % AHEAD][e / 4][e % 4], y1[e], y2[e]);
-                        bf16_t* dst = nullptr;
-                        if (head < a.H) dst = (bf16_t*)a.C + (size_t)m * a.ldc + head * a.D + d0;
-                        else if (row_slot >= 0) dst = a.k_pool + ((size_t)row_slot * a.KVH + (head - a.H)) * a.D + d0;
+                        T* dst = nullptr;
+                        if (head < a.H) dst = (T*)a.C + (size_t)m * a.ldc + head * a.D + d0;
+                        else if (row_slot >= 0) dst = (T*)a.k_pool + ((size_t)row_slot * a.KVH + (head - a.H)) * a.D + d0;
                         if (dst) {
-                            *(u32x4_t*)dst = u32x4_t{fd_pack(y1[0], y1[1]), fd_pack(y1[2], y1[3]), fd_pack(y1[4], y1[5]), fd_pack(y1[6], y1[7])};
-                            *(u32x4_t*)(dst + a.D / 2) =
-                                u32x4_t{fd_pack(y2[0], y2[1]), fd_pack(y2[2], y2[3]), fd_pack(y2[4], y2[5]), fd_pack(y2[6], y2[7])};
+                            gt_store8(dst, y1);
+                            gt_store8(dst + a.D / 2, y2);
                         }
                     } else if (row_slot >= 0) {
                         const int vh = head - a.H - a.KVH;
                         const int pg = row_slot >> a.page_shift, in_page = row_slot & ((1 << a.page_shift) - 1);
-                        bf16_t* dst = a.v_pool + ((((size_t)pg * a.KVH + vh) * a.D + d0) << a.page_shift) + in_page;
+                        T* dst = (T*)a.v_pool + ((((size_t)pg * a.KVH + vh) * a.D + d0) << a.page_shift) + in_page;
 #pragma unroll
                         for (int e = 0; e < 8; ++e) {
-                            dst[(size_t)e << a.page_shift] = f32_to_bf16(x[e]);
-                            dst[(size_t)(a.D / 2 + e) << a.page_shift] = f32_to_bf16(y[e]);
+                            Elem<T>::store(dst + ((size_t)e << a.page_shift), x[e]);
+                            Elem<T>::store(dst + ((size_t)(a.D / 2 + e) << a.page_shift), y[e]);
                         }
                     }
                 }
@@ -368,10 +427,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
         }
         p += gridDim.x;
         if (!gt_place(a, p, tm, tn, sp)) break;
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        clear();
     }
     gt_wait_loads<0>();                                             // nothing of the ring is in flight when the block ends
 }
@@ -434,11 +490,11 @@ static int gt_choose(int M, int N, int K, int splits, double* cost = nullptr) {
     return best;
 }
 
-template <int EPI, int MT, int NT, int WM, int WN, int ST, int OCC>
+template <typename T, int EPI, int MT, int NT, int WM, int WN, int ST, int OCC>
 static int gt_launch(TileArgs& a, hipStream_t stream) {
     constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, LDS = (BM + BN) * 128 * ST;
     static_assert(LDS * OCC <= 160 * 1024, "");
-    static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_tile_kernel<EPI, MT, NT, WM, WN, ST, OCC>,
+    static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_tile_kernel<T, EPI, MT, NT, WM, WN, ST, OCC>,
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (allowed != hipSuccess) return TM_ERR_LAUNCH;
     a.tiles_m = (a.M + BM - 1) / BM;
@@ -448,7 +504,7 @@ static int gt_launch(TileArgs& a, hipStream_t stream) {
     a.band = (a.tiles_m + bands - 1) / bands;
     const int chunk = (a.tiles_m * a.tiles_n * a.splits + 7) / 8;
     const int grid = 8 * chunk < GT_CUS * OCC ? 8 * chunk : GT_CUS * OCC;
-    gemm_tile_kernel<EPI, MT, NT, WM, WN, ST, OCC><<<grid, 256, LDS, stream>>>(a);
+    gemm_tile_kernel<T, EPI, MT, NT, WM, WN, ST, OCC><<<grid, 256, LDS, stream>>>(a);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
@@ -456,7 +512,7 @@ static int gt_launch(TileArgs& a, hipStream_t stream) {
 template <int EPI>
 static int gt_go(TileArgs& a, int shape, hipStream_t stream) {
     switch (shape) {
-#define GT_CASE(id, MT, NT, WM, WN, ST, OCC, s1, e1, s2, e2) case id: return gt_launch<EPI, MT, NT, WM, WN, ST, OCC>(a, stream);
+#define GT_CASE(id, MT, NT, WM, WN, ST, OCC, s1, e1, s2, e2) case id: return gt_launch<bf16_t, EPI, MT, NT, WM, WN, ST, OCC>(a, stream);
         GT_SHAPES(GT_CASE)
     }
     return TM_ERR_ARG;
@@ -479,7 +535,7 @@ extern "C" int tm_gemm_tile_takes(const void* A, int lda, const void* W, int M, 
 extern "C" int tm_tile_gate_up_silu(const void* A, int lda, int M, int K, const void* W, void* act, int I, hipStream_t stream) {
     if (I <= 0 || I % 8 || !gt_aligned(act) || !tm_gemm_tile_takes(A, lda, W, M, 2 * I, K)) return TM_ERR_ARG;
     TileArgs a{};
-    a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = act;
+    a.A = A; a.W = W; a.C = act;
     a.M = M; a.N = 2 * I; a.K = K; a.lda = lda; a.ldc = I; a.I = I; a.splits = 1;
     return gt_go<GT_SILU>(a, gt_choose(M, 2 * I, K, 1), stream);
 }
@@ -494,11 +550,11 @@ extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void
         (bias && bias_dtype != TM_NONE && !gt_aligned(bias)) || !gt_aligned(cos_t) || !gt_aligned(sin_t) || (slots && (!gt_aligned(k_pool) || !v_pool)) || !tm_gemm_tile_takes(A, lda, W, M, N, K))
         return TM_ERR_ARG;
     TileArgs a{};
-    a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = q;
+    a.A = A; a.W = W; a.C = q;
     a.bias = bias_dtype == TM_NONE ? nullptr : bias; a.bias_f32 = bias_dtype == TM_F32;
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = H * D; a.splits = 1;
     a.H = H; a.KVH = KVH; a.D = D; a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots;
-    a.k_pool = (bf16_t*)k_pool; a.v_pool = (bf16_t*)v_pool;
+    a.k_pool = k_pool; a.v_pool = v_pool;
     while ((1 << a.page_shift) < page) ++a.page_shift;
     return gt_go<GT_QKV>(a, gt_choose(M, N, K, 1), stream);
 }
@@ -524,7 +580,81 @@ extern "C" int tm_tile_linear_split(const void* A, int lda, int M, int K, const 
     const int splits = tm_tile_linear_parts(M, N, K);
     if (splits < 1 || !gt_aligned(parts) || !tm_gemm_tile_takes(A, lda, W, M, N, K)) return TM_ERR_ARG;
     TileArgs a{};
-    a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = parts;
+    a.A = A; a.W = W; a.C = parts;
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = N; a.splits = splits;
     return gt_go<GT_PARTS>(a, gt_choose(M, N, K, splits), stream);
+}
+
+// --- the same in 32-bit ---------------------------------------------------------------------------------------------------
+//
+// The 32-bit matrix unit takes sixteen times as long over a product, so a step of a tile of 64 x 64 (1,024 cycles of it) hides
+// every load and read, and small tiles leave the fewest CUs idle in a last round: three blocks a CU, one shape (gate|up of 1,000 /
+// 4,096 rows 154 / 537 us; two blocks a CU 159 / 566, 128 x 64 160 / 523, 64 x 128 160 / 524, 128 x 128 189 / 562; 111 / 455 at the
+// unit's peak). Against the kernel of gemm_f32_mfma.hip (16 k at a time through registers), 0.5B shape, 1,000 rows, in us a layer:
+// gate|up with SiLU*up 192 to 154, q|k|v with rotation 50 to 33, o and down 197 to 92.
+
+#define GT_F32 float, EPI, 1, 4, 4, 1, 3, 3
+constexpr int GT_F32_TILE = 64, GT_F32_STEP = 32, GT_F32_RING = 3;
+
+template <int EPI>
+static int gt_go_f32(TileArgs& a, hipStream_t stream) {
+    return gt_launch<GT_F32>(a, stream);
+}
+
+extern "C" int tm_tile_f32_takes(const void* A, int lda, const void* W, int M, int N, int K) {
+    return M > 0 && N > 0 && N % 8 == 0 && K >= GT_F32_STEP * GT_F32_RING && K % GT_F32_STEP == 0 && lda >= K && lda % 4 == 0 && gt_aligned(A) &&
+           gt_aligned(W) && (long long)M * lda * 4 < (1ll << 32) && (long long)N * K * 4 < (1ll << 32);
+}
+
+extern "C" int tm_tile_f32_gate_up_silu(const void* A, int lda, int M, int K, const void* W, void* act, int I, hipStream_t stream) {
+    if (I <= 0 || I % 8 || !gt_aligned(act) || !tm_tile_f32_takes(A, lda, W, M, 2 * I, K)) return TM_ERR_ARG;
+    TileArgs a{};
+    a.A = A; a.W = W; a.C = act;
+    a.M = M; a.N = 2 * I; a.K = K; a.lda = lda; a.ldc = I; a.I = I; a.splits = 1;
+    return gt_go_f32<GT_SILU>(a, stream);
+}
+
+extern "C" int tm_tile_f32_qkv_rope(const void* A, int lda, int M, int K, const void* W, const void* bias, void* q, int H, int KVH, int D,
+                                    const float* cos_t, const float* sin_t, const int* positions, const int* slots, void* k_pool,
+                                    void* v_pool, int page, hipStream_t stream) {
+    const int N = (H + 2 * KVH) * D;
+    if (H <= 0 || KVH <= 0 || D <= 0 || D % 64 || !gt_aligned(q) || (bias && !gt_aligned(bias)) || !gt_aligned(cos_t) || !gt_aligned(sin_t) || !positions ||
+        page <= 0 || (page & (page - 1)) || (slots && (!gt_aligned(k_pool) || !v_pool)) || !tm_tile_f32_takes(A, lda, W, M, N, K))
+        return TM_ERR_ARG;
+    TileArgs a{};
+    a.A = A; a.W = W; a.C = q; a.bias = bias; a.bias_f32 = 1;
+    a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = H * D; a.splits = 1;
+    a.H = H; a.KVH = KVH; a.D = D; a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots; a.k_pool = k_pool; a.v_pool = v_pool;
+    while ((1 << a.page_shift) < page) ++a.page_shift;
+    return gt_go_f32<GT_QKV>(a, stream);
+}
+
+// Parts of K for a product whose sums the next norm adds: as many as even out the CUs' shares and give them two blocks to choose from
+// (a step takes 0.55 us where a CU has one block, 0.445 of its time where it has more); a part more costs the norm a read. Down of
+// the 0.5B shape at 1,000 rows: 86 us in one part, 77 in four, 69 in eight.
+extern "C" int tm_tile_f32_parts(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || N % 8 || K < GT_F32_STEP * GT_F32_RING || K % GT_F32_STEP) return 0;
+    const long long tiles = (long long)((M + GT_F32_TILE - 1) / GT_F32_TILE) * ((N + GT_F32_TILE - 1) / GT_F32_TILE);
+    const int steps = K / GT_F32_STEP;
+    int best = 1;
+    double least = 0;
+    for (int splits = 1; splits <= 8; ++splits) {
+        const int per = (steps + splits - 1) / splits;
+        if (steps - (splits - 1) * per < GT_F32_RING) continue;
+        const long long rounds = (tiles * splits + GT_CUS - 1) / GT_CUS;
+        const double c = (rounds > 1 ? rounds * (per * 0.445 + 1) : per * 0.55 + 1) + (double)splits * M * N * 4 / 5e6;
+        if (splits == 1 || c < least) best = splits, least = c;
+    }
+    return best;
+}
+
+// parts[p][m][n], p < splits: the partial sums of A W^T (splits 1: the product itself)
+extern "C" int tm_tile_f32_linear_split(const void* A, int lda, int M, int K, const void* W, int N, float* parts, int splits, hipStream_t stream) {
+    if (splits < 1 || !gt_aligned(parts) || !tm_tile_f32_takes(A, lda, W, M, N, K)) return TM_ERR_ARG;
+    const int steps = K / GT_F32_STEP, per = (steps + splits - 1) / splits;
+    if (steps - (splits - 1) * per < GT_F32_RING) return TM_ERR_ARG;
+    TileArgs a{};
+    a.A = A; a.W = W; a.C = parts;
+    a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = N; a.splits = splits;
+    return gt_go_f32<GT_PARTS>(a, stream);
 }

@@ -104,6 +104,12 @@ bool gemv32_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype) {
            tm_gemv_f32_mfma_takes(x, ldx, L.w, L.bias, M, L.N, L.K);
 }
 
+// the 32-bit path's products of more rows (gemm_tile.hip)
+bool tile32_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype) {
+    return dtype == TM_F32 && L.dtype == TM_F32 && !L.act && (!L.bias || L.bias_dtype == TM_F32) && M > TM_GEMV_F32_ROWS &&
+           tm_tile_f32_takes(x, ldx, L.w, M, L.N, L.K);
+}
+
 // Parts of K for an output or down projection of M rows beyond the stream kernels' whose 32-bit sums the next norm adds up; 0: none.
 int tile_parts(const TmLinear& L, int M) {
     if (M <= TM_STREAM_ROWS || L.dtype != TM_BF16 || L.bias || L.act) return 0;
@@ -156,6 +162,8 @@ struct Products {
                 return then_act(tm_gemv_f32_mfma((const float*)x, ldx, (const float*)L.w, (const float*)L.bias, (float*)out, ldc, M, L.N, L.K, stream));
             if (plain32 && M <= TM_GEMV_F32_ROWS && L.K % 4 == 0 && ldx % 4 == 0 && aligned(x, 16) && aligned(L.w, 16))
                 return then_act(tm_gemv_f32((const float*)x, ldx, (const float*)L.w, (const float*)L.bias, (float*)out, ldc, M, L.N, L.K, stream));
+            if (plain32 && !L.bias && !L.act && ldc == L.N && aligned(out, 16) && tile32_ok(L, x, ldx, M, dtype))
+                return tm_tile_f32_linear_split(x, ldx, M, L.K, L.w, L.N, (float*)out, 1, stream);
             if (plain32 && tm_gemm_f32_mfma_fits(x, ldx, L.w, L.bias, out, ldc, M, L.N, L.K))
                 return then_act(tm_gemm_f32_mfma((const float*)x, ldx, (const float*)L.w, (const float*)L.bias, (float*)out, ldc, M, L.N, L.K, stream));
             return then_act(tm_gemm_nt_tiled(x, ldx, L.w, L.bias, L.bias_dtype, out, ldc, M, L.N, L.K, dtype, out_dtype, stream));
@@ -265,6 +273,14 @@ struct Run {
             if (rc) return rc;
             delta = nullptr;
             pending_sums = parts;
+            return TM_OK;
+        }
+        if (sums && accumulate && resid && L.N == p->hidden && !L.bias && tile32_ok(L, x_, ldx, M, dtype)) {
+            const int parts32 = tm_tile_f32_parts(M, L.N, L.K);
+            const int rc = tm_tile_f32_linear_split(x_, ldx, M, L.K, L.w, L.N, sums, parts32, stream);
+            if (rc) return rc;
+            delta = nullptr;
+            pending_sums = parts32;
             return TM_OK;
         }
         if (sums && accumulate && resid && L.N == p->hidden && !L.bias && gemv32_ok(L, x_, ldx, M, dtype)) {
@@ -396,8 +412,16 @@ struct Run {
                     q = qkv;
                     q_stride = HD;
                     ++p->taken[TM_QKV_PLAIN];
+                } else if (tables_fusable && a.D % 64 == 0 && tile32_ok(a.qkv, xn, hidden, T, dtype) && is_pow2(a.page) && bias_ok &&
+                           aligned(a.cos_t, 16) && aligned(a.sin_t, 16) && (!a.write || aligned(a.k_pool, 16))) {
+                    // 6. ... and for more
+                    rc = tm_tile_f32_qkv_rope(xn, hidden, T, hidden, a.qkv.w, a.qkv.bias, qkv, a.H, a.KVH, a.D, a.cos_t, a.sin_t, s->positions,
+                                              slots, kp, vp, a.page, stream);
+                    q = qkv;
+                    q_stride = HD;
+                    ++p->taken[TM_QKV_PLAIN];
                 } else {
-                    // 6. product, then rotation and cache write
+                    // 7. product, then rotation and cache write
                     if ((rc = linear(a.qkv, xn, hidden, T, qkv, QKV, dtype))) return rc;
                     if (a.rot > 0 || a.write)
                         rc = tm_rope_kv_write(qkv, dtype, T, a.H, a.KVH, a.D, a.rot, a.rot > 0 ? a.cos_t : nullptr,
@@ -517,6 +541,9 @@ struct Run {
                     ++p->taken[TM_GATE_UP_PLAIN];
                 } else if (plain && f.I % 4 == 0 && gemv32_ok(f.gate_up, xn, hidden, T, dtype)) {
                     rc = tm_gemv_f32_gate_up_silu((const float*)xn, hidden, (const float*)f.gate_up.w, (float*)act, T, f.I, hidden, stream);
+                    ++p->taken[TM_GATE_UP_PLAIN];
+                } else if (plain && f.I % 8 == 0 && tile32_ok(f.gate_up, xn, hidden, T, dtype)) {
+                    rc = tm_tile_f32_gate_up_silu(xn, hidden, T, hidden, f.gate_up.w, act, f.I, stream);
                     ++p->taken[TM_GATE_UP_PLAIN];
                 } else {
                     if ((rc = linear(f.gate_up, xn, hidden, T, gu, 2 * f.I, dtype))) return rc;
@@ -644,11 +671,10 @@ void tm_program_counters(const TmProgram* p, long long* out) {
 // Most parts that a product's K is split into in a step of T tokens (their sums [T, hidden] are kept until the next norm).
 static int program_sums(const TmProgram* p, int T) {
     if (p->dtype == TM_BF16 && T <= TM_STREAM_ROWS) return TM_MAX_SUMS;
-    if (p->dtype == TM_F32 && T > TM_GEMV_F32_ROWS) return 0;
     int most = 0;
     for (const Op& op : p->ops) {
         const TmLinear* L = op.kind == OP_ATTENTION ? &op.att.o : op.kind == OP_FEED_FORWARD ? &op.ffn.down : nullptr;
-        const int parts = !L ? 0 : p->dtype == TM_F32 ? tm_gemv_f32_parts(L->N, L->K) : tile_parts(*L, T);
+        const int parts = !L ? 0 : p->dtype == TM_BF16 ? tile_parts(*L, T) : T <= TM_GEMV_F32_ROWS ? tm_gemv_f32_parts(L->N, L->K) : tm_tile_f32_parts(T, L->N, L->K);
         if (parts > most) most = parts;
     }
     return most;
