@@ -106,6 +106,66 @@ def test_partial_sums_of_a_split_k(M, N, K):
     assert (out.double().sum(0) - ref).abs().max() <= 2.0 ** -24 * 5 * 4 * K ** 0.5
 
 
+# (tokens, experts, choices a token, K, width): experts without a token, with one, with tiles that are full and that are not
+EXPERTS = [(40, 3, 1, 192, 16), (200, 5, 2, 256, 208), (700, 4, 2, 320, 576), (130, 16, 3, 192, 192)]
+
+
+@pytest.mark.parametrize("tile_rows", [64, 128])
+@pytest.mark.parametrize("kind", ["silu", "clamped", "relu2"])
+@pytest.mark.parametrize("T,E,top,K,F", EXPERTS)
+def test_experts(T, E, top, K, F, kind, tile_rows):
+    from tokenmill_amd.hip import ops
+    lib = library()
+    g = torch.Generator(device="cuda").manual_seed(T + F)
+    gated = kind != "relu2"
+    x = torch.randn(T, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(E, F * (2 if gated else 1), K, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    down = (torch.randn(E, K, F, generator=g, device="cuda") * F ** -0.5).bfloat16()
+    table = torch.rand(50, E, generator=g, device="cuda").argsort(1)[:, :top].int().contiguous()
+    if E == 16:
+        table[:, 0] = 7                                         # most of the tokens in one expert
+        table[:, 1:] = torch.tensor([2, 5], device="cuda", dtype=torch.int32)
+    ids = torch.randint(0, 50, (T,), generator=g, device="cuda", dtype=torch.int32)
+    slot_pair, _, tiles, n_tiles, _ = ops.moe_route(ids, table, E, tile_rows)
+    weight = torch.rand(T * top, generator=g, device="cuda")
+    limit, alpha = 1.5, 1.7
+    act = torch.full((T * top, F), float("nan"), device="cuda", dtype=torch.bfloat16)
+    part = torch.full((T * top, K), float("nan"), device="cuda")
+    assert lib.tm_tile_experts_takes(P(x.data_ptr()), I(K), ctypes.c_longlong(T), P(w.data_ptr()), P(act.data_ptr()), I(tile_rows), I(K), I(w.shape[1]))
+    common = (P(tiles.data_ptr()), P(n_tiles.data_ptr()), I(tiles.shape[0]), I(tile_rows))
+    if kind == "clamped":
+        rc = lib.tm_moe_clamped_mfma(P(x.data_ptr()), I(K), P(slot_pair.data_ptr()), I(top), P(weight.data_ptr()), P(w.data_ptr()), P(act.data_ptr()),
+                                     *common, I(K), I(F), ctypes.c_float(limit), ctypes.c_float(alpha), _stream())
+    else:
+        first = lib.tm_moe_gate_up_mfma if gated else lib.tm_moe_up_act_mfma
+        rc = first(P(x.data_ptr()), I(K), P(slot_pair.data_ptr()), I(top), P(w.data_ptr()), P(act.data_ptr()), *common, I(K), I(F), _stream())
+    assert rc == 0
+    takes_down = bool(lib.tm_tile_experts_takes(P(act.data_ptr()), I(F), ctypes.c_longlong(T * top), P(down.data_ptr()), P(part.data_ptr()), I(tile_rows), I(F), I(K)))
+    assert takes_down == (F % 64 == 0 and F >= 192)
+    assert lib.tm_moe_down_mfma(P(act.data_ptr()), P(down.data_ptr()), P(part.data_ptr()), *common, I(F), I(K), _stream()) == 0
+    pairs = slot_pair.long()
+    expert = table[ids.long()].flatten().long()[pairs]
+    rows = x.double()[pairs // top]
+    h = torch.empty(T * top, w.shape[1], dtype=torch.float64, device="cuda")
+    for e in range(E):
+        h[expert == e] = rows[expert == e] @ w[e].double().T
+    if kind == "relu2":
+        want, slope = h.clamp(min=0) ** 2, 2 * h.abs()
+    else:
+        a, b = h.chunk(2, 1)
+        if kind == "silu":
+            want, slope = torch.nn.functional.silu(a) * b, 1.1 * b.abs() + a.abs()
+        else:
+            a, b = a * weight.double()[pairs, None], b * weight.double()[pairs, None]
+            a, b = a.clamp(max=limit), b.clamp(-limit, limit)
+            want, slope = a * torch.sigmoid(alpha * a) * (b + 1), 1.5 * (b.abs() + 1) + a.abs()
+    # the result is rounded to bfloat16 (by at most 2^-8 of itself); 32-bit sums of K terms of size 1 / sqrt(K) are off by less than 2^-18
+    assert ((act.double() - want).abs() <= 2.0 ** -8 * want.abs() * 1.01 + 2.0 ** -18 * (slope + 1)).all()
+    for e in range(E):
+        ref = act[expert == e].double() @ down[e].double().T
+        assert ((part[expert == e].double() - ref).abs() <= 2.0 ** -18 * (1 + act[expert == e].double().abs().amax(1, keepdim=True))).all()
+
+
 def _operands32(M, N, K, seed):
     g = torch.Generator(device="cuda").manual_seed(seed)
     a, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") * K ** -0.5

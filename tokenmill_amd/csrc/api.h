@@ -58,6 +58,13 @@ int tm_tile_f32_qkv_rope(const void* A, int lda, int M, int K, const void* W, co
 int tm_tile_f32_parts(int M, int N, int K);
 int tm_tile_f32_linear_split(const void* A, int lda, int M, int K, const void* W, int N, float* parts, int splits, hipStream_t stream);
 
+// The experts' products of grouped_mfma.hip in tiles of 64 slots, for steps whose route has tiles of 64 or 128 rows (kind 0: silu(gate) * up,
+// 1: clamped gate, 2: relu squared, 3: down, 32-bit).
+int tm_tile_experts_takes(const void* A, int lda, long long rows, const void* W, const void* C, int tile_rows, int K, int N);
+int tm_tile_experts(int kind, const void* A, int lda, const int* row_src, int src_div, const void* W, void* C, const int* tiles,
+                    const int* n_tiles, int max_tiles, int tile_rows, int K, int F, const float* pair_weight, float limit, float alpha,
+                    hipStream_t stream);
+
 // The true 32-bit path's products of at most 16 rows on the 32-bit matrix unit (gemv_f32.hip): K a multiple of 16, N of 4, 16-byte
 // pieces (tm_gemv_f32_mfma_takes). A plain product; 32-bit partial sums [parts][M][N] (tm_gemv_f32_parts says how many);
 // silu(gate) * up; q|k|v with bias, rotation over the whole head (head sizes that are multiples of 32) and cache write.

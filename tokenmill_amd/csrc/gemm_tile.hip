@@ -23,7 +23,7 @@
 
 #include <type_traits>
 
-enum { GT_SILU = 0, GT_QKV = 1, GT_PARTS = 2 };
+enum { GT_SILU = 0, GT_QKV = 1, GT_PARTS = 2, GT_EXPERT_SILU = 3, GT_EXPERT_CLAMPED = 4, GT_EXPERT_RELU2 = 5, GT_EXPERT_DOWN = 6 };
 
 struct TileArgs {
     const void* A;              // [M, K], rows lda apart
@@ -42,6 +42,21 @@ struct TileArgs {
     const int* slots;           // [M]; < 0: not stored; or null
     void* k_pool;               // [pages, page, KVH, D]
     void* v_pool;               // [pages, KVH, D, page]
+    // experts: a matrix a group (W [groups, rows, K]); row tiles (group, first slot, slots) from the route, n_tiles[0] of them with up
+    // to tile_rows slots, which blocks take BM at a time; slot i reads row row_src[i] / src_div of A (row_src null: row i)
+    const int* tiles;
+    const int* n_tiles;
+    const int* row_src;
+    int src_div, tile_rows;
+    const float* pair_weight;   // clamped gate: [pairs], multiplies the products of slot i by pair_weight[row_src[i]]; or null
+    float limit, alpha;
+};
+
+// Where a tile lies.
+struct GtPlace {
+    int tn, sp;                 // column tile, part of K
+    int m0, end;                // its rows: m0 .. end - 1 at most
+    int group;
 };
 
 // An operand fragment: 16 bytes of a row, 8 bfloat16 or 4 float32 values
@@ -81,28 +96,52 @@ __device__ __forceinline__ void gt_wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
 
-// Tile t of the launch -> (row tile, column tile, part of K). The blocks of one XCD (b % 8) walk a run of neighbouring tiles,
-// up to 16 row tiles of a column tile first, so that what an XCD's blocks read at a time overlaps in its L2.
-__device__ __forceinline__ bool gt_place(const TileArgs& a, int p, int& tm, int& tn, int& sp) {
-    const int total = a.tiles_m * a.tiles_n * a.splits;
+// Tile p of the launch. The blocks of one XCD (b % 8) walk a run of neighbouring tiles, `band` row tiles of a column tile first,
+// so that what an XCD's blocks read at a time overlaps in its L2. False: no further tile.
+template <bool GROUPED>
+__device__ __forceinline__ bool gt_place(const TileArgs& a, int BM, int p, GtPlace& at) {
+    const int per_entry = GROUPED ? a.tile_rows / BM : 1;
+    const int tiles_m = GROUPED ? __builtin_amdgcn_readfirstlane(a.n_tiles[0]) * per_entry : a.tiles_m;
+    const int total = tiles_m * a.tiles_n * a.splits;
     const int chunk = (total + 7) / 8;
     const int t = (p % 8) * chunk + p / 8;
     if (p / 8 >= chunk || t >= total) return false;
-    sp = t / (a.tiles_m * a.tiles_n);
-    const int in = t - sp * a.tiles_m * a.tiles_n;
+    at.sp = t / (tiles_m * a.tiles_n);
+    const int in = t - at.sp * tiles_m * a.tiles_n;
     const int band = in / (a.band * a.tiles_n);
-    const int rows = a.tiles_m - a.band * band < a.band ? a.tiles_m - a.band * band : a.band;
+    const int rows = tiles_m - a.band * band < a.band ? tiles_m - a.band * band : a.band;
     const int q = in - band * a.band * a.tiles_n;
-    tn = q / rows;
-    tm = a.band * band + q - tn * rows;
+    at.tn = q / rows;
+    const int tm = a.band * band + q - at.tn * rows;
+    if (GROUPED) {
+        const int* e = a.tiles + 3 * (tm / per_entry);
+        const int first = __builtin_amdgcn_readfirstlane(e[1]);
+        at.group = __builtin_amdgcn_readfirstlane(e[0]);
+        at.m0 = first + tm % per_entry * BM;
+        at.end = first + __builtin_amdgcn_readfirstlane(e[2]);
+    } else {
+        at.group = 0;
+        at.m0 = tm * BM;
+        at.end = a.M;
+    }
     return true;
+}
+
+// ... or the next one behind it (the block's tiles are gridDim.x apart) that has a row
+template <bool GROUPED>
+__device__ __forceinline__ bool gt_next(const TileArgs& a, int BM, int& p, GtPlace& at) {
+    while (gt_place<GROUPED>(a, BM, p, at)) {
+        if (!GROUPED || at.m0 < at.end) return true;
+        p += gridDim.x;
+    }
+    return false;
 }
 
 // the matrix row that row q of unit u holds
 template <int EPI>
 __device__ __forceinline__ int gt_matrix_row(const TileArgs& a, int u, int q) {
     int n;
-    if (EPI == GT_SILU) {
+    if (EPI == GT_SILU || EPI == GT_EXPERT_SILU || EPI == GT_EXPERT_CLAMPED) {
         n = 32 * u + (q & 31);
         n = n < a.I ? n : a.I - 1;
         if (q >= 32) n += a.I;
@@ -122,6 +161,7 @@ template <typename T, int EPI, int MT, int NT, int WM, int WN, int ST, int OCC>
 __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     extern __shared__ __align__(16) unsigned char gt_smem[];
     constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, ROWS = BM + BN;
+    constexpr bool GROUPED = EPI >= GT_EXPERT_SILU, GATED = EPI == GT_SILU || EPI == GT_EXPERT_SILU || EPI == GT_EXPERT_CLAMPED;
     constexpr int STAGE = ROWS * 128, NL = ROWS / 32;               // bytes of a buffer; loads a wavefront makes for it
     static_assert(BM % 32 == 0 && BN % 64 == 0 && NT % 4 == 0, "");
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)gt_smem;
@@ -138,28 +178,29 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     int l_p = blockIdx.x;
     bool l_more = true;
     auto next_load_tile = [&]() {
-        int tm, tn, sp;
-        if (!l_more || !gt_place(a, l_p, tm, tn, sp)) {             // no further tile: the same bytes again, never multiplied
+        GtPlace at_;
+        if (!l_more || !gt_next<GROUPED>(a, BM, l_p, at_)) {             // no further tile: the same bytes again, never multiplied
             l_more = false;
             lA = (const unsigned char*)a.A;
             lW = (const unsigned char*)a.W;
             return;
         }
         l_p += gridDim.x;
-        const int k0 = sp * per;
+        const int k0 = at_.sp * per;
         lA = (const unsigned char*)a.A + (size_t)k0 * 128;
-        lW = (const unsigned char*)a.W + (size_t)k0 * 128;
+        lW = (const unsigned char*)a.W + (size_t)k0 * 128 + (GROUPED ? (size_t)at_.group * a.N * a.K * ES : 0);
         const int in8 = lane / 8, at = lane % 8;
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
             const int R = (wave + 4 * i) * 8 + in8;                 // row of the buffer
             if (i < BM / 32) {
-                int m = tm * BM + R;
-                m = m < a.M ? m : a.M - 1;
+                int m = at_.m0 + R;
+                m = m < at_.end ? m : at_.end - 1;
+                if (GROUPED && a.row_src) m = a.row_src[m] / a.src_div;
                 voff[i] = (uint32_t)m * (uint32_t)a.lda * ES + (uint32_t)((at ^ ((R >> 1) & 7)) * 16);
             } else {
                 const int Rb = R - BM;
-                const int n = gt_matrix_row<EPI>(a, tn * (BN / 64) + Rb / 64, Rb % 64);
+                const int n = gt_matrix_row<EPI>(a, at_.tn * (BN / 64) + Rb / 64, Rb % 64);
                 voff[i] = (uint32_t)n * (uint32_t)a.K * ES + (uint32_t)((at ^ (((Rb >> 1) & 1) | (((Rb >> 3) & 3) << 1))) * 16);
             }
         }
@@ -171,9 +212,9 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     };
 
     // --- the multiplying side ---
-    int tm, tn, sp;
+    GtPlace at_;
     int p = blockIdx.x;
-    if (!gt_place(a, p, tm, tn, sp)) return;
+    if (!gt_next<GROUPED>(a, BM, p, at_)) return;
     next_load_tile();
 #pragma unroll
     for (int s = 0; s < ST; ++s) {                                  // (every part of K has at least ST steps)
@@ -254,7 +295,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
         for (int j = 0; j < NT; ++j) fb[0][j].u = *(const u32x4_t*)(gt_smem + buf * STAGE + offB + (j / 2) * 4096 + (j & 1) * 512);
 #pragma unroll
         for (int i = 1; i < MT; ++i) fa[0][i].u = *(const u32x4_t*)(gt_smem + buf * STAGE + offA + i * 2048);
-        const int k0 = sp * per;
+        const int k0 = at_.sp * per;
         const int steps = ksteps - k0 < per ? ksteps - k0 : per;
         // what the epilogue's addresses hang on: asked for now where there are registers for it, so that the end of the tile waits
         // for one trip and not for two
@@ -262,7 +303,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
         auto read_places = [&]() {
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                const int m = tm * BM + (wm * MT + i) * 16 + r;
+                const int m = at_.m0 + (wm * MT + i) * 16 + r;
                 pos[i] = a.positions[m < a.M ? m : a.M - 1];
                 slot[i] = a.slots ? a.slots[m < a.M ? m : a.M - 1] : -1;
             }
@@ -297,11 +338,11 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
         if constexpr (EPI == GT_QKV && MT > 5) read_places();
 #pragma unroll
         for (int un = 0; un < NT / 4; ++un) {
-            const int u = tn * (BN / 64) + wn * (NT / 4) + un;      // the unit
+            const int u = at_.tn * (BN / 64) + wn * (NT / 4) + un;      // the unit
             // a lane's columns: eight from c0 on and eight from c1 on (indices into the matrix's rows)
             int c0, c1, head = 0, d0 = 0;
             bool ok0, ok1;
-            if (EPI == GT_SILU) {
+            if (GATED) {
                 c0 = 32 * u + 8 * g;
                 c1 = a.I + c0;
                 ok0 = ok1 = c0 < a.I;
@@ -353,7 +394,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
-                const int m = tm * BM + (wm * MT + i) * 16 + r;
+                const int m = at_.m0 + (wm * MT + i) * 16 + r;
                 float x[8], y[8];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -363,9 +404,9 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                     y[e] = ES == 4 ? total[ES == 4 ? i : 0][ES == 4 ? at + 2 : 0][e] : acc[i][at + 2][e];
                     y[4 + e] = ES == 4 ? total[ES == 4 ? i : 0][ES == 4 ? at + 3 : 0][e] : acc[i][at + 3][e];
                 }
-                if (m >= a.M) continue;
-                if (EPI == GT_PARTS) {
-                    float* dst = (float*)a.C + ((size_t)sp * a.M + m) * a.N;
+                if (m >= at_.end) continue;
+                if (EPI == GT_PARTS || EPI == GT_EXPERT_DOWN) {
+                    float* dst = (float*)a.C + ((size_t)(GROUPED ? 0 : at_.sp) * a.M + m) * a.N;
                     if (ok0) {
                         *(f32x4_t*)(dst + c0) = f32x4_t{x[0], x[1], x[2], x[3]};
                         *(f32x4_t*)(dst + c0 + 4) = f32x4_t{x[4], x[5], x[6], x[7]};
@@ -374,6 +415,24 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                         *(f32x4_t*)(dst + c1) = f32x4_t{y[0], y[1], y[2], y[3]};
                         *(f32x4_t*)(dst + c1 + 4) = f32x4_t{y[4], y[5], y[6], y[7]};
                     }
+                } else if (EPI == GT_EXPERT_RELU2) {
+                    T* dst = (T*)a.C + (size_t)m * a.ldc;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        x[e] = fmaxf(x[e], 0.f) * fmaxf(x[e], 0.f);
+                        y[e] = fmaxf(y[e], 0.f) * fmaxf(y[e], 0.f);
+                    }
+                    if (ok0) gt_store8(dst + c0, x);
+                    if (ok1) gt_store8(dst + c1, y);
+                } else if (EPI == GT_EXPERT_SILU || EPI == GT_EXPERT_CLAMPED) {
+                    if (!ok0) continue;
+                    float v[8];
+                    const float w = EPI == GT_EXPERT_CLAMPED && a.pair_weight ? a.pair_weight[a.row_src[m]] : 1.f;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        v[e] = EPI == GT_EXPERT_CLAMPED ? clamped_glu_f32(w * x[e], w * y[e], a.alpha, a.limit)
+                                                        : x[e] / (1.0f + __expf(-x[e])) * y[e];
+                    gt_store8((T*)a.C + (size_t)m * a.ldc + c0, v);
                 } else if (EPI == GT_SILU) {
                     if (!ok0) continue;
                     float v[8];
@@ -426,7 +485,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
             }
         }
         p += gridDim.x;
-        if (!gt_place(a, p, tm, tn, sp)) break;
+        if (!gt_next<GROUPED>(a, BM, p, at_)) break;
         clear();
     }
     gt_wait_loads<0>();                                             // nothing of the ring is in flight when the block ends
@@ -497,11 +556,14 @@ static int gt_launch(TileArgs& a, hipStream_t stream) {
     static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_tile_kernel<T, EPI, MT, NT, WM, WN, ST, OCC>,
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (allowed != hipSuccess) return TM_ERR_LAUNCH;
-    a.tiles_m = (a.M + BM - 1) / BM;
-    a.tiles_n = EPI == GT_SILU ? (2 * ((a.I + 31) / 32 * 32) + BN - 1) / BN : (a.N + BN - 1) / BN;
+    // (experts: M is the most row tiles the route can give, tiles of a.tile_rows rows)
+    constexpr bool GROUPED = EPI >= GT_EXPERT_SILU, GATED = EPI == GT_SILU || EPI == GT_EXPERT_SILU || EPI == GT_EXPERT_CLAMPED;
+    a.tiles_m = GROUPED ? a.M * (a.tile_rows / BM) : (a.M + BM - 1) / BM;
+    a.tiles_n = GATED ? (2 * ((a.I + 31) / 32 * 32) + BN - 1) / BN : (a.N + BN - 1) / BN;
     // row tiles an XCD's blocks take beside each other: all of them where K is short enough for their rows to stay in its L2
     const int most = a.K > 2048 ? 6 : 16, bands = (a.tiles_m + most - 1) / most;
-    a.band = (a.tiles_m + bands - 1) / bands;
+    // experts: two row tiles, mostly of one expert, beside all its columns (against four: 80 to 106 us where BM is 128)
+    a.band = GROUPED ? 2 : (a.tiles_m + bands - 1) / bands;
     const int chunk = (a.tiles_m * a.tiles_n * a.splits + 7) / 8;
     const int grid = 8 * chunk < GT_CUS * OCC ? 8 * chunk : GT_CUS * OCC;
     gemm_tile_kernel<T, EPI, MT, NT, WM, WN, ST, OCC><<<grid, 256, LDS, stream>>>(a);
@@ -657,4 +719,44 @@ extern "C" int tm_tile_f32_linear_split(const void* A, int lda, int M, int K, co
     a.A = A; a.W = W; a.C = parts;
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = N; a.splits = splits;
     return gt_go_f32<GT_PARTS>(a, stream);
+}
+
+// --- the products of experts -----------------------------------------------------------------------------------------------
+//
+// A tile of the route (128 slots, or 64) by 256 matrix rows: these products stand at what the CUs take out of the second-level
+// caches, so the larger tile wins although an expert's last one is seldom full (16 experts of 187 slots on average: 3 tiles of 64
+// or 2 of 128 slots). Against grouped_mfma.hip (128 slots by 64 or 128 rows, 32 k a step through registers and padded LDS rows),
+// 3,000 pairs of 16 experts of 2,048 x 2,048, gate|up with silu and down, in us: 144 + 84 to 80 + 45; 64 x 256 123 + 62, 64 x 128
+// 117 + 67, 128 x 128 99 + 50. The matrices alone take 54 + 27 to read.
+
+template <int EPI>
+static int gt_expert(const void* A, int lda, const int* row_src, int src_div, const void* W, void* C, int ldc, const int* tiles, const int* n_tiles,
+                     int max_tiles, int tile_rows, int K, int N, int I, const float* pair_weight, float limit, float alpha, hipStream_t stream) {
+    TileArgs a{};
+    a.A = A; a.W = W; a.C = C; a.M = max_tiles; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.splits = 1; a.I = I;
+    a.tiles = tiles; a.n_tiles = n_tiles; a.row_src = row_src; a.src_div = src_div; a.tile_rows = tile_rows;
+    a.pair_weight = pair_weight; a.limit = limit; a.alpha = alpha;
+    return tile_rows % 128 == 0 ? gt_launch<bf16_t, EPI, 4, 8, 2, 2, 3, 1>(a, stream) : gt_launch<bf16_t, EPI, 2, 8, 2, 2, 3, 1>(a, stream);
+}
+
+// Whole 16-byte pieces, k in whole steps that fill the ring, tiles of whole 64 rows; `rows`: the most rows of A there are.
+extern "C" int tm_tile_experts_takes(const void* A, int lda, long long rows, const void* W, const void* C, int tile_rows, int K, int N) {
+    return tile_rows % 64 == 0 && tile_rows > 0 && K >= 192 && K % 64 == 0 && N % 16 == 0 && lda % 8 == 0 && gt_aligned(A) && gt_aligned(W) &&
+           gt_aligned(C) && rows * lda * 2 < (1ll << 32) && (long long)N * K * 2 < (1ll << 32);
+}
+
+// The products of tm_moe_gate_up_mfma (kind 0), tm_moe_clamped_mfma (1), tm_moe_up_act_mfma (2: N rows an expert) and
+// tm_moe_down_mfma (3); their operands, checked by them.
+extern "C" int tm_tile_experts(int kind, const void* A, int lda, const int* row_src, int src_div, const void* W, void* C, const int* tiles,
+                               const int* n_tiles, int max_tiles, int tile_rows, int K, int F, const float* pair_weight, float limit, float alpha,
+                               hipStream_t stream) {
+#define GT_EXPERT_GO(EPI, N, I) gt_expert<EPI>(A, lda, row_src, src_div, W, C, F, tiles, n_tiles, max_tiles, tile_rows, K, N, I, pair_weight, limit, alpha, stream)
+    switch (kind) {
+        case 0: return GT_EXPERT_GO(GT_EXPERT_SILU, 2 * F, F);
+        case 1: return GT_EXPERT_GO(GT_EXPERT_CLAMPED, 2 * F, F);
+        case 2: return GT_EXPERT_GO(GT_EXPERT_RELU2, F, 0);
+        case 3: return GT_EXPERT_GO(GT_EXPERT_DOWN, F, 0);
+    }
+#undef GT_EXPERT_GO
+    return TM_ERR_ARG;
 }

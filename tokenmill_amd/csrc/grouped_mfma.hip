@@ -212,6 +212,8 @@ extern "C" int tm_moe_gate_up_mfma(const void* x, int ldx, const int* slot_pair,
         ldx % 8 || !gm_aligned(x) || !gm_aligned(W))
         return TM_ERR_ARG;
     if (max_tiles == 0) return TM_OK;
+    if (tile_rows >= 64 && tm_tile_experts_takes(x, ldx, (long long)max_tiles * tile_rows, W, act, tile_rows, K, 2 * F))
+        return tm_tile_experts(0, x, ldx, slot_pair, top, W, act, tiles, n_tiles, max_tiles, tile_rows, K, F, nullptr, 0.f, 0.f, stream);
     dim3 grid(max_tiles, (F + GM_BN - 1) / GM_BN);
     if (grid.y > 65535) return TM_ERR_ARG;
 #define GM_GO(RT_, BK_, BN_)                                                                                                             \
@@ -233,6 +235,8 @@ extern "C" int tm_moe_clamped_mfma(const void* x, int ldx, const int* slot_pair,
         ldx % 8 || !gm_aligned(x) || !gm_aligned(W) || !(limit > 0.f))
         return TM_ERR_ARG;
     if (max_tiles == 0) return TM_OK;
+    if (tile_rows >= 64 && tm_tile_experts_takes(x, ldx, (long long)max_tiles * tile_rows, W, act, tile_rows, K, 2 * F))
+        return tm_tile_experts(1, x, ldx, slot_pair, top, W, act, tiles, n_tiles, max_tiles, tile_rows, K, F, pair_weight, limit, alpha, stream);
     dim3 grid(max_tiles, (F + GM_BN - 1) / GM_BN);
     if (grid.y > 65535) return TM_ERR_ARG;
 #define GM_GO(RT_, BK_)                                                                                                                  \
@@ -253,6 +257,8 @@ extern "C" int tm_moe_up_act_mfma(const void* x, int ldx, const int* slot_pair, 
         ldx % 8 || !gm_aligned(x) || !gm_aligned(W))
         return TM_ERR_ARG;
     if (max_tiles == 0) return TM_OK;
+    if (tile_rows >= 64 && tm_tile_experts_takes(x, ldx, (long long)max_tiles * tile_rows, W, act, tile_rows, K, F))
+        return tm_tile_experts(2, x, ldx, slot_pair, top, W, act, tiles, n_tiles, max_tiles, tile_rows, K, F, nullptr, 0.f, 0.f, stream);
     dim3 grid(max_tiles, (F + GM_BN - 1) / GM_BN);
     if (grid.y > 65535) return TM_ERR_ARG;
 #define GM_GO(RT_, BK_, BN_)                                                                                                             \
@@ -273,6 +279,8 @@ extern "C" int tm_moe_down_mfma(const void* act, const void* W, float* part, con
     if (!act || !W || !part || !tiles || !n_tiles || F <= 0 || N <= 0 || max_tiles < 0 || F % 8 || !gm_aligned(act) || !gm_aligned(W))
         return TM_ERR_ARG;
     if (max_tiles == 0) return TM_OK;
+    if (tile_rows >= 64 && tm_tile_experts_takes(act, F, (long long)max_tiles * tile_rows, W, part, tile_rows, F, N))
+        return tm_tile_experts(3, act, F, nullptr, 1, W, part, tiles, n_tiles, max_tiles, tile_rows, F, N, nullptr, 0.f, 0.f, stream);
     dim3 grid(max_tiles, (N + GM_BN - 1) / GM_BN);
     if (grid.y > 65535) return TM_ERR_ARG;
 #define GM_GO(RT_, BK_, BN_)                                                                                                              \
