@@ -91,7 +91,10 @@ def test_qkv_with_rotation_and_cache_write(M, H, KVH, D, K, bias_dtype, stored):
 
 
 PARTS = [(65, 896, 896), (77, 896, 4864), (130, 3584, 960), (333, 896, 4864), (1000, 1016, 4864), (2048, 896, 896), (2048, 896, 4864),
-         (4000, 896, 4864), (1000, 3584, 3584)]
+         (4000, 896, 4864), (1000, 3584, 3584),
+         # few rows: the tile with a ring of five, its shortest parts, one part, K below the ring, K beyond its range
+         (1, 896, 896), (8, 3584, 3584), (17, 1000, 320), (16, 896, 4864), (33, 40, 256), (64, 2048, 2048), (64, 520, 12800),
+         (40, 264, 12864), (5, 8200, 640)]
 
 
 @pytest.mark.parametrize("M,N,K", PARTS)

@@ -30,8 +30,21 @@ inline int tm_from_norm_rows(int hidden) { const int s = tm_skinny_rows(hidden);
 constexpr int TM_PANEL_QKV_ROWS = 64;
 // up to this many rows the products stream the packed matrix once for several row tiles, with their epilogues
 constexpr int TM_STREAM_ROWS = 64;
-// (a plain product of 17 to 64 rows, such as the output and down projections, is streamed where splitting its K over
-// groups of blocks pays: tm_stream_linear_parts in gemm_stream.hip; else it is the library's)
+// ... except gate|up where a 64-column tile for each CU covers the matrix: the tiled product over the row-major matrix then
+// runs in one round with 64 KB of the matrix on their way into each CU. Streamed to tiled, cold matrices, 17 / 64 rows, us:
+// 896 -> 2 x 4,864 9.0 / 11.9 to 6.9 / 8.1; 2,048 -> 2 x 5,632 14.4 / 20.8 to 13.0 / 14.2; 3,072 -> 2 x 8,192 (256 tiles)
+// 22.7 / 34.6 to 20.4 / 21.5; beyond a tile a CU 1,536 -> 2 x 8,960 16.2 / 19.4 to 15.9 / 22.8, 3,584 -> 2 x 18,944 48.4 / 52.9
+// to 62.1 / 66.6.
+constexpr int TM_TILE_FEW_COLUMNS = 64 * 256;
+// Output and down projections run tiled, K in parts, beyond so many rows: beyond the rows of the kernels that start at the norm
+// at widths from 3,072, else beyond 16. Against the streamed product (the library's for 896 -> 896) with the norm that adds the
+// parts, 8 / 64 rows, us: 896 -> 896 10.4 (of the product alone) to 7.2 / 7.8; 4,864 -> 896 10.5 / 14.7 to 8.6 / 10.5; 2,048 ->
+// 2,048 10.4 / 14.5 to 8.9 / 10.3; 3,584 -> 3,584 12.9 / 19.0 to 11.5 / 13.4; 18,944 -> 3,584 31.0 / 38.6 to 29.4 / 34.9;
+// 5,120 -> 5,120 18.0 / 25.1 to 16.8 / 20.0. In a step of 9 rows the down projections of widths 1,536 and 2,048 (K 8,960 and
+// 11,008) were 1.3 and 1.9 us slower tiled, with 24 rows level: hence 16 there.
+inline int tm_split_rows(int hidden) { return hidden < 3072 ? TM_SKINNY_ROWS : 4; }
+// (what that does not take, such as a projection with a bias, is streamed where splitting its K over groups of blocks pays:
+// tm_stream_linear_parts in gemm_stream.hip; else it is the library's)
 // most rows one launch of the skinny product takes at all
 constexpr int TM_SKINNY_MAX_ROWS = 64;
 // most rows the 32-bit matrix-vector product takes

@@ -94,8 +94,8 @@ bool stream_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype, int 
 // few rows do not run. Against the library's product and the kernel behind it, in us a layer: gate|up with SiLU*up, 0.5B
 // shape, 77 / 512 / 2,048 rows 16.4 / 22.2 / 65.0 to 6.9 / 13.2 / 35-40; 7B shape, 3,001 rows 724 to 590; q|k|v with rotation
 // and cache write, 0.5B shape 14.3 / 15.0 / 20.1 to 5.7 / 6.5 / 12.7.
-bool tile_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype) {
-    return dtype == TM_BF16 && L.dtype == TM_BF16 && !L.act && M > TM_SKINNY_ROWS && tm_gemm_tile_takes(x, ldx, L.w, M, L.N, L.K);
+bool tile_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype, int beyond = TM_SKINNY_ROWS) {
+    return dtype == TM_BF16 && L.dtype == TM_BF16 && !L.act && M > beyond && tm_gemm_tile_takes(x, ldx, L.w, M, L.N, L.K);
 }
 
 // the 32-bit path's products of few rows with their epilogues (gemv_f32.hip)
@@ -110,9 +110,9 @@ bool tile32_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype) {
            tm_tile_f32_takes(x, ldx, L.w, M, L.N, L.K);
 }
 
-// Parts of K for an output or down projection of M rows beyond the stream kernels' whose 32-bit sums the next norm adds up; 0: none.
+// Parts of K for an output or down projection of M rows whose 32-bit sums the next norm adds up; 0: none.
 int tile_parts(const TmLinear& L, int M) {
-    if (M <= TM_STREAM_ROWS || L.dtype != TM_BF16 || L.bias || L.act) return 0;
+    if (L.dtype != TM_BF16 || L.bias || L.act) return 0;
     const int parts = tm_tile_linear_parts(M, L.N, L.K);
     return parts <= TM_MAX_SUMS ? parts : 0;
 }
@@ -256,8 +256,17 @@ struct Run {
     // resid += round(x W^T + b) in the product's epilogue where a kernel does that and the caller lets it; else the
     // product goes to delta_buf and is added by the next norm (or handed back).
     int project(const TmLinear& L, const void* x_, int ldx, int M) {
-        // 17 to 64 rows over a matrix with few rows of output: K split over groups of blocks, whose partial sums the
-        // next norm adds up (or, where the caller wants the result itself, a small kernel)
+        // K in parts, whose 32-bit sums the next norm adds up
+        if (const int parts = (sums && accumulate && resid && L.N == p->hidden && tile_ok(L, x_, ldx, M, dtype, tm_split_rows(p->hidden)))
+                                  ? tile_parts(L, M) : 0) {
+            const int rc = tm_tile_linear_split(x_, ldx, M, L.K, L.w, L.N, sums, stream);
+            if (rc) return rc;
+            delta = nullptr;
+            pending_sums = parts;
+            return TM_OK;
+        }
+        // up to 64 rows of what that does not take (a bias; a caller that wants the result itself, which a small kernel adds up),
+        // over the packed matrix
         // (the stream kernels take at most 64 rows: `sums` has room for TM_MAX_SUMS of them then)
         const int groups = (sums && L.N == p->hidden && L.packed_parts == 1 && stream_ok(L, x_, ldx, M, dtype, products.skinny_rows))
                                ? tm_stream_linear_parts(L.N, L.K) : 1;
@@ -267,13 +276,6 @@ struct Run {
             delta = nullptr;
             pending_sums = groups;
             return accumulate && resid ? TM_OK : settle();
-        }
-        if (const int parts = (sums && accumulate && resid && L.N == p->hidden && tile_ok(L, x_, ldx, M, dtype)) ? tile_parts(L, M) : 0) {
-            const int rc = tm_tile_linear_split(x_, ldx, M, L.K, L.w, L.N, sums, stream);
-            if (rc) return rc;
-            delta = nullptr;
-            pending_sums = parts;
-            return TM_OK;
         }
         if (sums && accumulate && resid && L.N == p->hidden && !L.bias && tile32_ok(L, x_, ldx, M, dtype)) {
             const int parts32 = tm_tile_f32_parts(M, L.N, L.K);
@@ -529,6 +531,9 @@ struct Run {
                 if (plain && two_parts && packed_ok(f.gate_up, xn, hidden, T, dtype, from_norm_rows)) {
                     rc = tm_gemm_skinny_packed(xn, hidden, f.gate_up.packed, 16, nullptr, TM_NONE, act, f.I, T, f.I, hidden, TM_BF16, 1,
                                                nullptr, 0, stream);
+                    ++p->taken[TM_GATE_UP_PLAIN];
+                } else if (plain && f.I % 8 == 0 && tile_ok(f.gate_up, xn, hidden, T, dtype) && (T > TM_STREAM_ROWS || 2 * f.I <= TM_TILE_FEW_COLUMNS)) {
+                    rc = tm_tile_gate_up_silu(xn, hidden, T, hidden, f.gate_up.w, act, f.I, stream);
                     ++p->taken[TM_GATE_UP_PLAIN];
                 } else if (plain && two_parts && f.I % 4 == 0 && stream_ok(f.gate_up, xn, hidden, T, dtype, from_norm_rows)) {
                     rc = tm_stream_gate_up_silu(xn, hidden, T, hidden, f.gate_up.packed, act, f.I, stream);
