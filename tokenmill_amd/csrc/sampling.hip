@@ -62,11 +62,13 @@ __global__ __launch_bounds__(SM_NT) void argmax_rows_kernel(const float* __restr
 // candidates are reduced. Ties go to the lower index in both stages (the first maximum).
 #define AM_NT 256
 // clear (may be null): clear_per_row 64-bit words per row that the row's blocks set to zero between them
-// (the sampler's histograms: no launch of its own for that).
+// (the sampler's histograms: no launch of its own for that). wave_v (may be null): the maximum of every wavefront's share
+// (the entries threadIdx.x + j AM_NT of the chunk), NaN if it has none.
+// Bound by reading the logits once; eight loads of a lane in flight (64 rows of 151,936: 20.0 us with one, 13.2 with eight).
 __global__ __launch_bounds__(AM_NT) void argmax_partial_kernel(const float* __restrict__ logits, int V, int chunk,
                                                                float* __restrict__ part_v, int* __restrict__ part_i,
                                                                unsigned long long* __restrict__ clear,
-                                                               int clear_per_row) {
+                                                               int clear_per_row, float* __restrict__ wave_v) {
     __shared__ ArgMax smem[AM_NT / TM_WAVE];
     const int row = blockIdx.x, c = blockIdx.y, NB = gridDim.y;
     if (clear) {
@@ -77,9 +79,13 @@ __global__ __launch_bounds__(AM_NT) void argmax_partial_kernel(const float* __re
     const int lo = c * chunk, hi = lo + chunk < V ? lo + chunk : V;
     const float* src = logits + (size_t)row * V;
     ArgMax best{-INFINITY, -1};
-    for (int i = lo + threadIdx.x; i < hi; i += AM_NT) {
-        const float v = src[i];
-        if (v == v) best = better(best, ArgMax{v, i});
+    for (int i = lo + threadIdx.x; i < hi; i += 8 * AM_NT) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = src[i + j * AM_NT < hi ? i + j * AM_NT : i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (i + j * AM_NT < hi && v[j] == v[j]) best = better(best, ArgMax{v[j], i + j * AM_NT});
     }
 #pragma unroll
     for (int off = TM_WAVE / 2; off > 0; off >>= 1) {
@@ -87,7 +93,10 @@ __global__ __launch_bounds__(AM_NT) void argmax_partial_kernel(const float* __re
         best = better(best, o);
     }
     const int wave = threadIdx.x / TM_WAVE, lane = threadIdx.x % TM_WAVE;
-    if (lane == 0) smem[wave] = best;
+    if (lane == 0) {
+        smem[wave] = best;
+        if (wave_v) wave_v[((size_t)row * NB + c) * (AM_NT / TM_WAVE) + wave] = best.i < 0 ? NAN : best.v;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         ArgMax r = smem[0];
@@ -129,7 +138,7 @@ extern "C" int tm_argmax_rows(const float* logits, int R, int V, int* out, float
         return TM_OK;
     }
     const int chunk = (V + NB - 1) / NB;
-    argmax_partial_kernel<<<dim3(R, NB), AM_NT, 0, stream>>>(logits, V, chunk, work_v, work_i, nullptr, 0);
+    argmax_partial_kernel<<<dim3(R, NB), AM_NT, 0, stream>>>(logits, V, chunk, work_v, work_i, nullptr, 0, nullptr);
     TM_CHECK_LAUNCH();
     argmax_final_kernel<<<R, TM_WAVE, 0, stream>>>(work_v, work_i, NB, out);
     TM_CHECK_LAUNCH();
@@ -185,7 +194,7 @@ extern "C" int tm_argmax_rows_static(const float* logits, int R, int V, int* out
     int* part_i = (int*)(base + (size_t)AM_STATIC_PAIRS * sizeof(float));   // [R, NB]
     // Nothing has to start at zero: the first kernel writes every (row, chunk) entry that the second reads.
     const int chunk = (V + NB - 1) / NB;
-    argmax_partial_kernel<<<dim3(R, NB), AM_NT, 0, stream>>>(logits, V, chunk, part_v, part_i, nullptr, 0);
+    argmax_partial_kernel<<<dim3(R, NB), AM_NT, 0, stream>>>(logits, V, chunk, part_v, part_i, nullptr, 0, nullptr);
     TM_CHECK_LAUNCH();
     argmax_final_kernel<<<R, TM_WAVE, 0, stream>>>(part_v, part_i, NB, out);
     TM_CHECK_LAUNCH();
@@ -198,9 +207,10 @@ extern "C" int tm_argmax_rows_static(const float* logits, int R, int V, int* out
 // A row of a wide vocabulary is cut into the chunks of the two-stage argmax (one block each), so a
 // step's few rows still fill the chip; every stage is a launch over (row, chunk):
 //   1. the chunk maxima (argmax_partial_kernel, which also clears the row's histograms) and the row
-//      maximum (sample_rowmax_kernel): zmax for the softmax, and the token of a greedy row;
+//      maximum (sample_bound_kernel): zmax for the softmax, and the token of a greedy row; and, for top-k, a
+//      key that at least k entries reach, from the maxima of the chunks' wavefronts;
 //   2. top-k, if some row asks for it: three launches, one per level of a radix descent (11, 11 and
-//      10 bits of the order-preserving key of logit / temperature) that add the chunk's counts to
+//      10 bits of the order-preserving key of logit / temperature) that add the counts of the entries from that key up to
 //      the row's histogram of that level; the blocks of the next level find the bucket that holds
 //      the k-th largest entry from the histograms before it;
 //   3. top-p over what top-k kept, if some row asks for it: the same descent with fixed-point
@@ -246,7 +256,7 @@ __device__ __forceinline__ RowParams row_params(int r, int V, const float* tempe
     rp.need_k = !rp.greedy && rp.k < V;
     rp.p = top_p[r];
     rp.need_p = !rp.greedy && rp.p < 1.f;
-    rp.zmax = rowmax[r] * rp.inv_t;
+    rp.zmax = rowmax ? rowmax[r] * rp.inv_t : 0.f;
     return rp;
 }
 
@@ -259,7 +269,7 @@ __device__ __forceinline__ RowParams row_params(int r, int V, const float* tempe
 // drop: weight in the histogram that belongs to entries top-k does not keep after all, ties beyond its budget).
 __device__ void pick_bucket(const unsigned long long* __restrict__ hist, int bins, bool by_mass, double frac,
                             unsigned long long drop, unsigned long long& limit, unsigned long long& above,
-                            uint32_t& bucket, unsigned long long* s_scan /* SR_NT */, unsigned long long* s_res /* 2 */) {
+                            uint32_t& bucket, unsigned long long* s_scan /* SR_NT / 64 */, unsigned long long* s_res /* 2 */) {
     const int t = threadIdx.x, per = bins / SR_NT;
     unsigned long long local[SR_BINS / SR_NT];
     unsigned long long sum = 0;
@@ -268,16 +278,22 @@ __device__ void pick_bucket(const unsigned long long* __restrict__ hist, int bin
         local[j] = j < per ? hist[bins - 1 - (t * per + j)] : 0ull;
         sum += local[j];
     }
-    __syncthreads();                                     // s_scan and s_res may still be read from the call before
-    s_scan[t] = sum;
-    __syncthreads();
-    for (int off = 1; off < SR_NT; off <<= 1) {          // inclusive scan over the threads
-        const unsigned long long add = t >= off ? s_scan[t - off] : 0ull;
-        __syncthreads();
-        s_scan[t] += add;
-        __syncthreads();
+    const int wave = t / TM_WAVE, lane = t % TM_WAVE;
+    unsigned long long incl = sum;                       // inclusive scan over the threads
+#pragma unroll
+    for (int off = 1; off < TM_WAVE; off <<= 1) {
+        const unsigned long long up = __shfl_up(incl, off, TM_WAVE);
+        if (lane >= off) incl += up;
     }
-    const unsigned long long incl = s_scan[t], excl = incl - sum, total = s_scan[SR_NT - 1];
+    __syncthreads();                                     // s_scan and s_res may still be read from the call before
+    if (lane == TM_WAVE - 1) s_scan[wave] = incl;
+    __syncthreads();
+    unsigned long long total = 0;
+    for (int v = 0; v < SR_NT / TM_WAVE; ++v) {
+        if (v < wave) incl += s_scan[v];
+        total += s_scan[v];
+    }
+    const unsigned long long excl = incl - sum;
     if (frac >= 0.0) limit = (unsigned long long)((double)(total > drop ? total - drop : 0ull) * frac);
     auto reached = [&](unsigned long long run) { return by_mass ? run > limit : run >= limit; };
     if (t == SR_NT - 1 && !reached(above + total)) {     // never: bucket 0, everything above it counts
@@ -307,15 +323,32 @@ __device__ void pick_bucket(const unsigned long long* __restrict__ hist, int bin
     above = s_res[1];
 }
 
+// Where a descent stands after some of its levels, left by the launch of each level for the next one: a block then walks one
+// histogram, not all before it (64 rows of 151,936 with both filters: a launch of the top-p descent 28.6 to 12.3 us, with the shares below).
+struct Descent {
+    unsigned long long limit, above;
+    uint32_t prefix, pad;
+};
+
 // The key of the k-th largest entry (by count) or the smallest key the nucleus keeps (by mass) from a
-// row's three finished histograms; `above` = count / weight of the entries with a larger key.
+// row's three finished histograms; `above` = count / weight of the entries with a larger key. saved (may be null):
+// [levels - 1] is where the descent stood one level earlier, for levels of two or more.
 __device__ uint32_t descend(const unsigned long long* __restrict__ hist3, int levels, bool by_mass, double frac,
                             unsigned long long& limit, unsigned long long& above, uint32_t& mask,
-                            unsigned long long* s_scan, unsigned long long* s_res, unsigned long long drop = 0ull) {
+                            unsigned long long* s_scan, unsigned long long* s_res, const Descent* __restrict__ saved,
+                            unsigned long long drop = 0ull) {
     uint32_t prefix = 0;
+    int first = 0;
     mask = 0;
     above = 0;
-    for (int level = 0; level < levels; ++level) {
+    if (saved && levels >= 2) {
+        first = levels - 1;
+        prefix = saved[first].prefix;
+        above = saved[first].above;
+        limit = saved[first].limit;
+        for (int level = 0; level < first; ++level) mask |= (uint32_t)(level_bins(level) - 1) << level_shift(level);
+    }
+    for (int level = first; level < levels; ++level) {
         uint32_t bucket;
         pick_bucket(hist3 + (size_t)level * SR_BINS, level_bins(level), by_mass, level == 0 ? frac : -1.0, drop, limit,
                     above, bucket, s_scan, s_res);
@@ -335,11 +368,11 @@ struct KEdge {
     unsigned long long dropped;
 };
 __device__ KEdge k_edge(const unsigned long long* __restrict__ hist_k, const RowParams& rp,
-                        unsigned long long* s_scan, unsigned long long* s_res) {
+                        unsigned long long* s_scan, unsigned long long* s_res, const Descent* __restrict__ saved) {
     unsigned long long limit = (unsigned long long)rp.k, above = 0;
     uint32_t mask;
     KEdge e;
-    e.key = descend(hist_k, 3, false, -1.0, limit, above, mask, s_scan, s_res);
+    e.key = descend(hist_k, 3, false, -1.0, limit, above, mask, s_scan, s_res, saved);
     const long long budget = (long long)rp.k - (long long)above;         // above: entries strictly larger
     e.budget = budget > 0x7fffffffLL ? 0x7fffffff : (budget < 0 ? 0 : (int)budget);
     const unsigned long long ties = hist_k[2 * SR_BINS + (e.key & (uint32_t)(level_bins(2) - 1))];
@@ -348,22 +381,65 @@ __device__ KEdge k_edge(const unsigned long long* __restrict__ hist_k, const Row
     return e;
 }
 
-__global__ __launch_bounds__(TM_WAVE) void sample_rowmax_kernel(const float* __restrict__ part_v,
-                                                                const int* __restrict__ part_i, int NB,
-                                                                float* __restrict__ rowmax, int* __restrict__ rowarg) {
-    const int row = blockIdx.x;
+// What the launches of a row hand on.
+struct RowState {
+    Descent k[3], p[3];         // [level], level 1 and 2
+    KEdge edge;                 // where top-k ends, from the first level of the top-p descent
+    uint32_t bound;             // at least k entries have this key or a larger one (0: not known)
+};
+
+// A wavefront's share of a chunk in which every entry's key is below `floor` (block-wide thread layout of the chunk maxima).
+__device__ __forceinline__ bool share_below(const float* __restrict__ wave_v, size_t chunk_at, float inv_t, uint32_t floor) {
+    const float z = wave_v[chunk_at * (AM_NT / TM_WAVE) + threadIdx.x / TM_WAVE] * inv_t;
+    return z == z && order_key(z) < floor;
+}
+static_assert(AM_NT == SR_NT, "the wavefronts' shares of a chunk are the same in all launches");
+
+// The k-th largest of the wavefronts' maxima bounds the k-th largest entry from below: each maximum is an entry of its own.
+// Shares below it take no part in top-k, and the ones below top-k's end none in what follows: with k = 50 two thirds of the
+// shares of a row of 151,936 are passed over without a read, and next to no entry reaches the histograms' atomics.
+#define SR_MAX_SHARES (256 * (AM_NT / TM_WAVE))
+__global__ __launch_bounds__(SR_NT) void sample_bound_kernel(const float* __restrict__ part_v, const int* __restrict__ part_i,
+                                                             const float* __restrict__ wave_v, int NB, int V,
+                                                             const float* __restrict__ temperature, const int* __restrict__ top_k,
+                                                             const float* __restrict__ top_p, float* __restrict__ rowmax,
+                                                             int* __restrict__ rowarg, RowState* __restrict__ state) {
+    __shared__ uint32_t s_key[SR_MAX_SHARES];
+    __shared__ ArgMax s_best[SR_NT / TM_WAVE];
+    __shared__ uint32_t s_bound;
+    const int row = blockIdx.x, n = NB * (AM_NT / TM_WAVE);
     ArgMax best{-INFINITY, -1};
-    for (int c = threadIdx.x; c < NB; c += TM_WAVE)
-        best = better(best, ArgMax{part_v[(size_t)row * NB + c], part_i[(size_t)row * NB + c]});
+    for (int c = threadIdx.x; c < NB; c += SR_NT) best = better(best, ArgMax{part_v[(size_t)row * NB + c], part_i[(size_t)row * NB + c]});
 #pragma unroll
     for (int off = TM_WAVE / 2; off > 0; off >>= 1) {
         ArgMax o{__shfl_xor(best.v, off, TM_WAVE), __shfl_xor(best.i, off, TM_WAVE)};
         best = better(best, o);
     }
+    if (threadIdx.x % TM_WAVE == 0) s_best[threadIdx.x / TM_WAVE] = best;
+    const RowParams rp = row_params(row, V, temperature, top_k, top_p, nullptr);
+    for (int i = threadIdx.x; i < n; i += SR_NT) {
+        const float z = wave_v[(size_t)row * n + i] * rp.inv_t;
+        s_key[i] = z == z ? order_key(z) : 0u;           // (no number's key is 0)
+    }
+    if (threadIdx.x == 0) s_bound = 0u;
+    __syncthreads();
     if (threadIdx.x == 0) {
+        for (int v = 1; v < SR_NT / TM_WAVE; ++v) best = better(best, s_best[v]);
         rowmax[row] = best.i < 0 ? 0.f : best.v;
         rowarg[row] = best.i < 0 ? 0 : best.i;
     }
+    if (rp.need_k && rp.k <= n)
+        for (int i = threadIdx.x; i < n; i += SR_NT) {
+            const uint32_t key = s_key[i];
+            int larger = 0, level = 0;
+            for (int j = 0; j < n; ++j) {
+                larger += s_key[j] > key;
+                level += s_key[j] == key;
+            }
+            if (larger < rp.k && larger + level >= rp.k) s_bound = key;    // (threads that write it write one value)
+        }
+    __syncthreads();
+    if (threadIdx.x == 0) state[row].bound = s_bound;
 }
 
 // One level of a descent: the chunk's entries that match the buckets picked so far, into the row's
@@ -374,9 +450,11 @@ __global__ __launch_bounds__(SR_NT) void sample_hist_kernel(const float* __restr
                                                             const int* __restrict__ top_k,
                                                             const float* __restrict__ top_p,
                                                             const float* __restrict__ rowmax,
-                                                            unsigned long long* __restrict__ hist_all, int level) {
+                                                            unsigned long long* __restrict__ hist_all, int level,
+                                                            const float* __restrict__ wave_v,
+                                                            RowState* __restrict__ row_state, int stages) {
     __shared__ unsigned long long s_hist[SR_BINS];
-    __shared__ unsigned long long s_scan[SR_NT];
+    __shared__ unsigned long long s_scan[SR_NT / TM_WAVE];
     __shared__ unsigned long long s_res[2];
     const int r = blockIdx.x, c = blockIdx.y;
     const RowParams rp = row_params(r, V, temperature, top_k, top_p, rowmax);
@@ -385,30 +463,43 @@ __global__ __launch_bounds__(SR_NT) void sample_hist_kernel(const float* __restr
     unsigned long long* hist_p = hist_k + 3 * SR_BINS;
     uint32_t floor_key = 0, prefix = 0, mask = 0;
     unsigned long long limit = 0, above = 0;
+    RowState& state = row_state[r];
+    const bool writes = c == 0 && threadIdx.x == 0;
     if (BY_MASS) {
         unsigned long long dropped = 0;
         if (rp.need_k) {
-            const KEdge e = k_edge(hist_k, rp, s_scan, s_res);
+            const KEdge e = level > 0 ? state.edge : k_edge(hist_k, rp, s_scan, s_res, (stages & 1) ? state.k : nullptr);
             floor_key = e.key;
             dropped = e.dropped;
+            if (level == 0 && writes) state.edge = e;
         }
-        prefix = descend(hist_p, level, true, (double)rp.p, limit, above, mask, s_scan, s_res, dropped);
+        prefix = descend(hist_p, level, true, (double)rp.p, limit, above, mask, s_scan, s_res, state.p, dropped);
     } else {
         limit = (unsigned long long)rp.k;
-        prefix = descend(hist_k, level, false, -1.0, limit, above, mask, s_scan, s_res);
+        prefix = descend(hist_k, level, false, -1.0, limit, above, mask, s_scan, s_res, state.k);
+        floor_key = state.bound;
     }
+    if (level > 0 && writes) (BY_MASS ? state.p : state.k)[level] = Descent{limit, above, prefix, 0u};
+    const bool skip = share_below(wave_v, (size_t)r * gridDim.y + c, rp.inv_t, floor_key > prefix ? floor_key : prefix);
+    if (__syncthreads_and(skip)) return;                 // nothing of this chunk counts
     for (int b = threadIdx.x; b < SR_BINS; b += SR_NT) s_hist[b] = 0ull;
     __syncthreads();
     const float* row = logits + (size_t)r * V;
     const int lo = c * chunk, hi = lo + chunk < V ? lo + chunk : V;
     const int shift = level_shift(level);
     const uint32_t digit_mask = (uint32_t)(level_bins(level) - 1);
-    for (int i = lo + threadIdx.x; i < hi; i += SR_NT) {
-        const float z = row[i] * rp.inv_t;
-        if (!(z == z)) continue;
-        const uint32_t key = order_key(z);
-        if (key < floor_key || (key & mask) != prefix) continue;
-        atomicAdd(&s_hist[(key >> shift) & digit_mask], BY_MASS ? fix_weight(expf(z - rp.zmax)) : 1ull);
+    for (int i = lo + threadIdx.x; i < hi && !skip; i += 8 * SR_NT) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = row[i + j * SR_NT < hi ? i + j * SR_NT : i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float z = v[j] * rp.inv_t;
+            if (i + j * SR_NT >= hi || !(z == z)) continue;
+            const uint32_t key = order_key(z);
+            if (key < floor_key || (key & mask) != prefix) continue;
+            atomicAdd(&s_hist[(key >> shift) & digit_mask], BY_MASS ? fix_weight(expf(z - rp.zmax)) : 1ull);
+        }
     }
     __syncthreads();
     unsigned long long* dst = (BY_MASS ? hist_p : hist_k) + (size_t)level * SR_BINS;
@@ -468,8 +559,10 @@ __global__ __launch_bounds__(SR_NT) void sample_chunk_mass_kernel(const float* _
                                                                   const unsigned long long* __restrict__ hist_all,
                                                                   float* __restrict__ chunk_weight,
                                                                   int* __restrict__ chunk_ties,
-                                                                  RowKeep* __restrict__ row_keep) {
-    __shared__ unsigned long long s_scan[SR_NT];
+                                                                  RowKeep* __restrict__ row_keep,
+                                                                  const float* __restrict__ wave_v,
+                                                                  const RowState* __restrict__ row_state, int stages) {
+    __shared__ unsigned long long s_scan[SR_NT / TM_WAVE];
     __shared__ unsigned long long s_res[2];
     __shared__ float s_w[SR_NT / TM_WAVE];
     __shared__ int s_n[SR_NT / TM_WAVE];
@@ -481,7 +574,7 @@ __global__ __launch_bounds__(SR_NT) void sample_chunk_mass_kernel(const float* _
     RowKeep keep{0u, 0, 0};
     unsigned long long dropped = 0;
     if (rp.need_k) {
-        const KEdge e = k_edge(hist_k, rp, s_scan, s_res);
+        const KEdge e = rp.need_p && (stages & 2) ? row_state[r].edge : k_edge(hist_k, rp, s_scan, s_res, (stages & 1) ? row_state[r].k : nullptr);
         keep.p_key = e.key;
         keep.ties_matter = 1;
         keep.tie_budget = e.budget;
@@ -493,7 +586,8 @@ __global__ __launch_bounds__(SR_NT) void sample_chunk_mass_kernel(const float* _
         // here is vocabulary order; the first always stays): limit = p * mass, above = mass of larger keys
         unsigned long long limit = 0, above = 0;
         uint32_t mask;
-        const uint32_t pk = descend(hist_p, 3, true, (double)rp.p, limit, above, mask, s_scan, s_res, dropped);
+        const uint32_t pk = descend(hist_p, 3, true, (double)rp.p, limit, above, mask, s_scan, s_res,
+                                    (stages & 2) ? row_state[r].p : nullptr, dropped);
         if (!rp.need_k || pk >= keep.p_key) {
             const unsigned long long w = fix_weight(expf(key_value(pk) - rp.zmax));
             const unsigned long long room = limit > above ? limit - above : 0ull;
@@ -510,10 +604,17 @@ __global__ __launch_bounds__(SR_NT) void sample_chunk_mass_kernel(const float* _
     const int lo = c * chunk, hi = lo + chunk < V ? lo + chunk : V;
     float w = 0.f;
     int ties = 0;
-    for (int i = lo + threadIdx.x; i < hi; i += SR_NT) {
-        bool tie;
-        w += entry_weight(row[i], rp, keep, tie);
-        ties += tie;
+    const bool skip = share_below(wave_v, (size_t)r * NB + c, rp.inv_t, keep.p_key);
+    for (int i = lo + threadIdx.x; i < hi && !skip; i += 8 * SR_NT) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = row[i + j * SR_NT < hi ? i + j * SR_NT : i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            bool tie = false;
+            if (i + j * SR_NT < hi) w += entry_weight(v[j], rp, keep, tie);
+            ties += tie;
+        }
     }
     block_sums(w, ties, s_w, s_n);
     if (threadIdx.x == 0) {
@@ -701,8 +802,8 @@ __global__ __launch_bounds__(SR_NT) void sample_pick_kernel(const float* __restr
 static size_t sample_hist_bytes(int R) { return (size_t)R * SR_HIST_PER_ROW * sizeof(unsigned long long); }
 extern "C" size_t tm_sample_work_bytes(int R, int V) {
     const size_t NB = (size_t)tm_argmax_work_chunks(V);
-    const size_t per_chunk = (size_t)R * NB * 4;         // part_v, part_i, chunk_weight, chunk_ties
-    return sample_hist_bytes(R) + 4 * per_chunk + (size_t)R * (sizeof(RowKeep) + 8);
+    const size_t per_chunk = (size_t)R * NB * 4;         // part_v, part_i, chunk_weight, chunk_ties, wave_v
+    return sample_hist_bytes(R) + (size_t)R * sizeof(RowState) + (4 + AM_NT / TM_WAVE) * per_chunk + (size_t)R * (sizeof(RowKeep) + 8);
 }
 
 // stages: bit 0 = some row may use top-k, bit 1 = some row may use top-p (3 if the caller does not
@@ -718,32 +819,34 @@ extern "C" int tm_sample_rows(const float* logits, int R, int V, const float* te
     unsigned char* w = (unsigned char*)work;
     unsigned long long* hist = (unsigned long long*)w;
     w += sample_hist_bytes(R);
+    RowState* state = (RowState*)w;     w += (size_t)R * sizeof(RowState);
     float* part_v = (float*)w;          w += (size_t)R * NB * 4;
     int* part_i = (int*)w;              w += (size_t)R * NB * 4;
+    float* wave_v = (float*)w;          w += (size_t)R * NB * (AM_NT / TM_WAVE) * 4;
     float* chunk_weight = (float*)w;    w += (size_t)R * NB * 4;
     int* chunk_ties = (int*)w;          w += (size_t)R * NB * 4;
     RowKeep* row_keep = (RowKeep*)w;    w += (size_t)R * sizeof(RowKeep);
     float* rowmax = (float*)w;          w += (size_t)R * 4;
     int* rowarg = (int*)w;
     const dim3 grid(R, NB);
-    argmax_partial_kernel<<<grid, AM_NT, 0, stream>>>(logits, V, chunk, part_v, part_i, hist, SR_HIST_PER_ROW);
+    argmax_partial_kernel<<<grid, AM_NT, 0, stream>>>(logits, V, chunk, part_v, part_i, hist, SR_HIST_PER_ROW, wave_v);
     TM_CHECK_LAUNCH();
-    sample_rowmax_kernel<<<R, TM_WAVE, 0, stream>>>(part_v, part_i, NB, rowmax, rowarg);
+    sample_bound_kernel<<<R, SR_NT, 0, stream>>>(part_v, part_i, wave_v, NB, V, temperature, top_k, top_p, rowmax, rowarg, state);
     TM_CHECK_LAUNCH();
     if (stages & 1)
         for (int level = 0; level < 3; ++level) {
             sample_hist_kernel<false><<<grid, SR_NT, 0, stream>>>(logits, V, chunk, temperature, top_k, top_p, rowmax,
-                                                                 hist, level);
+                                                                 hist, level, wave_v, state, stages);
             TM_CHECK_LAUNCH();
         }
     if (stages & 2)
         for (int level = 0; level < 3; ++level) {
             sample_hist_kernel<true><<<grid, SR_NT, 0, stream>>>(logits, V, chunk, temperature, top_k, top_p, rowmax,
-                                                                hist, level);
+                                                                hist, level, wave_v, state, stages);
             TM_CHECK_LAUNCH();
         }
     sample_chunk_mass_kernel<<<grid, SR_NT, 0, stream>>>(logits, V, chunk, temperature, top_k, top_p, rowmax, hist,
-                                                         chunk_weight, chunk_ties, row_keep);
+                                                         chunk_weight, chunk_ties, row_keep, wave_v, state, stages);
     TM_CHECK_LAUNCH();
     sample_pick_kernel<<<R, SR_NT, 0, stream>>>(logits, V, chunk, NB, temperature, top_k, top_p, rowmax, rowarg,
                                                 chunk_weight, chunk_ties, row_keep, u, out);
