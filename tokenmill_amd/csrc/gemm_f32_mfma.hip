@@ -1,6 +1,6 @@
 // C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]), everything float32, on the 32-bit matrix unit
 // (v_mfma_f32_16x16x4_f32: 32-bit products and sums, no reduced-precision inputs): the matrix product
-// of prompt-sized steps of the true 32-bit path                (reference src/infer/model/layers.py:144,
+// of more than 16 rows of the true 32-bit path that the tiled kernel does not take (K % 16 == 0 is enough here) (reference src/infer/model/layers.py:144,
 // 150,163-164 run with float32 parameters, src/infer/model/loader.py:32-35).
 //
 // A block of four wavefronts computes a BM x BN tile of C; A and W tiles of 16 k go through LDS, the

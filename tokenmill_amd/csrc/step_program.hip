@@ -90,8 +90,8 @@ bool stream_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype, int 
            aligned(x, 16) && tm_gemm_stream_fits(M, L.K);
 }
 
-// the products of prompt-sized steps with their epilogues (gemm_tile.hip), over the row-major matrix: wherever the kernels for
-// few rows do not run. Against the library's product and the kernel behind it, in us a layer: gate|up with SiLU*up, 0.5B
+// the products of prompt-sized steps with their epilogues (gemm_tile.hip), over the row-major matrix: beyond the rows of the
+// kernels for few rows (the rules for steps of up to 64 tokens stand in choose.h). Against the library's product and the kernel behind it, in us a layer: gate|up with SiLU*up, 0.5B
 // shape, 77 / 512 / 2,048 rows 16.4 / 22.2 / 65.0 to 6.9 / 13.2 / 35-40; 7B shape, 3,001 rows 724 to 590; q|k|v with rotation
 // and cache write, 0.5B shape 14.3 / 15.0 / 20.1 to 5.7 / 6.5 / 12.7.
 bool tile_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype, int beyond = TM_SKINNY_ROWS) {
@@ -382,7 +382,7 @@ struct Run {
                     if ((rc = normed(a.norm))) return rc;
                     xn = x;
                 }
-                // 2. the normed input kept in LDS (17 to 48 tokens)
+                // 2. the normed input kept in LDS (up to TM_PANEL_QKV_ROWS tokens)
                 if (tables_fusable && a.D % 32 == 0 && a.qkv.dtype == TM_BF16 && panel_ok(a.qkv, xn, hidden, T, dtype, from_norm_rows, TM_PANEL_QKV_ROWS) &&
                     is_pow2(a.page) && bias_ok) {
                     rc = tm_panel_qkv_rope(xn, hidden, T, hidden, a.qkv.packed, a.qkv.bias, a.qkv.bias_dtype, qkv, a.H, a.KVH, a.D,
