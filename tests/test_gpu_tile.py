@@ -49,6 +49,26 @@ def test_gate_up_silu(M, n, K):
     assert ((out.double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** 127])
+def test_the_activation_is_the_one_of_the_other_products(scale):
+    """Rows of A with one entry give gate and up without a rounding, so the activation alone is compared, bit for bit with the kernel
+    behind a plain product: every bfloat16 gate there is, or, at the large scale, infinities too (and infinities times zero)."""
+    M = n = K = 256
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a = (torch.eye(K, device="cuda") * scale).bfloat16()
+    w = (torch.randn(2 * n, K, generator=g, device="cuda") * 3).bfloat16()
+    if scale == 1:
+        every = torch.arange(65536, device="cuda").sub(32768).to(torch.int16).view(torch.bfloat16)
+        w[:n] = torch.where(every.isfinite() & (every.float().abs() >= 2.0 ** -100), every, torch.zeros_like(every)).view(n, K)
+    out, want = torch.empty(2, M, n, device="cuda", dtype=torch.bfloat16)
+    lib = library()
+    assert lib.tm_tile_gate_up_silu(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), P(out.data_ptr()), I(n), _stream()) == 0
+    both = (w.float().T * scale).bfloat16().contiguous()
+    assert lib.tm_silu_mul(P(both.data_ptr()), P(want.data_ptr()), I(1), I(M), I(n), _stream()) == 0
+    assert both.isinf().any() == (scale > 1)
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.nan_to_num(0.0), want.nan_to_num(0.0))
+
+
 QKV = [(65, 14, 2, 64, 256), (333, 14, 2, 64, 896), (1000, 28, 4, 128, 256), (2500, 14, 2, 64, 256), (70, 3, 1, 192, 256)]
 
 

@@ -91,6 +91,19 @@ __device__ __forceinline__ void gt_round2(float& a, float& b) {
     b = __uint_as_float(u & 0xffff0000u);
 }
 
+// x / (1 + exp(-x)). Of a bfloat16 x the division is a reciprocal, one correction of the quotient by its remainder and the unit's
+// own last step for infinities; a quarter of both sides keeps the reciprocal of the largest divisors normal. The same bits as
+// the division for every bfloat16 x, in seven instructions for eleven: at one wavefront a SIMD an epilogue's instructions are
+// its time (2,048 rows of 896 -> 2 x 4,864, in a step: 4.3 us more than the one-instruction exponential and reciprocal, whose
+// error is 3e-6 of the value at the far end where this one's is 1.3e-7; with the division itself 6.1 us more).
+template <typename T>
+__device__ __forceinline__ float gt_silu(float x) {
+    const float e = expf(-x);
+    if constexpr (sizeof(T) == 4) return x / (1.f + e);
+    const float n = 0.25f * x, d = fmaf(e, 0.25f, 0.25f), r = __builtin_amdgcn_rcpf(d), q = n * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
+}
+
 template <int N>
 __device__ __forceinline__ void gt_wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
@@ -442,10 +455,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                         gt_round2<T>(y[e], y[e + 1]);
                     }
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        if constexpr (ES == 4) v[e] = x[e] / (1.f + expf(-x[e])) * y[e];
-                        else v[e] = x[e] * __builtin_amdgcn_rcpf(1.f + __expf(-x[e])) * y[e];     // (far closer than the bfloat16 it becomes)
-                    }
+                    for (int e = 0; e < 8; ++e) v[e] = gt_silu<T>(x[e]) * y[e];
                     gt_store8((T*)a.C + (size_t)m * a.ldc + c0, v);
                 } else {
                     if (!ok0) continue;
