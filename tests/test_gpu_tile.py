@@ -129,6 +129,21 @@ def test_partial_sums_of_a_split_k(M, N, K):
     assert (out.double().sum(0) - ref).abs().max() <= 2.0 ** -24 * 5 * 4 * K ** 0.5
 
 
+# an output and a down projection of the shipped shapes and what lies around the line between the two tiles of few rows
+@pytest.mark.parametrize("N,K", [(896, 896), (896, 4864), (2048, 11008), (3584, 3584), (3584, 18944), (5120, 27648), (3072, 12864), (2944, 12864)])
+def test_few_rows_do_not_change_a_row_of_a_split_product(N, K):
+    lib = library()
+    parts = lib.tm_tile_linear_parts(1, N, K)
+    a, w, _ = _operands(64, N, K, N + K)
+    sums = {}
+    for M in (1, 5, 16, 17, 32, 33, 48, 64):
+        assert lib.tm_tile_linear_parts(M, N, K) == parts
+        out = torch.full((parts, M, N), float("nan"), device="cuda")
+        assert lib.tm_tile_linear_split(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), I(N), P(out.data_ptr()), _stream()) == 0
+        sums[M] = out
+    assert all(torch.equal(out, sums[64][:, :M]) for M, out in sums.items())
+
+
 # (tokens, experts, choices a token, K, width): experts without a token, with one, with tiles that are full and that are not
 EXPERTS = [(40, 3, 1, 192, 16), (200, 5, 2, 256, 208), (700, 4, 2, 320, 576), (130, 16, 3, 192, 192)]
 

@@ -635,20 +635,26 @@ extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void
 // Few tiles leave CUs idle for the library and for one part alike; a part costs a write and a read of its sums.
 // Up to 64 rows there is one row of tiles: 64 columns wide, with a ring of five buffers, two blocks a CU, and as many parts as
 // give each CU a block, each at least as deep as the ring. Of the tiles above and 1 to 8 parts, 8 to 64 rows, this was the best
-// or within 4% of it at ten matrices from 896 x 896 to 5,120 x 27,648, but for 64 rows of 18,944 -> 3,584 and 27,648 -> 5,120
-// (34.9 and 62.2 us to 32.2 and 57.5 with 64 x 128 tiles, eight and six parts: the cost above chooses beyond 32 rows of those).
-constexpr int GT_FEW_ROWS = 64, GT_FEW_RING = 5, GT_FEW_STEPS = 200;
-static bool gt_few(int M, int K) { return M <= GT_FEW_ROWS && (M <= 32 || K / 64 <= GT_FEW_STEPS); }
+// or within 4% of it at ten matrices from 896 x 896 to 5,120 x 27,648, but for long K with columns enough for 128 wide tiles to
+// give three CUs in four a block: those take 64 x 128 tiles, in as many parts (with the norm, 5 / 17 / 32 / 48 / 64 rows, us:
+// 18,944 -> 3,584 64 wide in four parts 29.1 / 29.5 / 30.5 / 32.3 / 34.6, 128 wide in eight 29.4 / 29.8 / 30.3 / 31.2 / 32.1;
+// 27,648 -> 5,120 in three and six 53.6 / 54.0 / 55.2 / 59.2 / 63.1 and 54.0 / 54.5 / 55.8 / 56.8 / 58.3; 13,952 -> 2,048, which
+// 128 wide tiles would leave half the CUs without, stays at eight parts of 64, 15.8 to 18.3).
+// How K is cut hangs on N and K alone: a row's result does not change with the number of rows.
+constexpr int GT_FEW_ROWS = 64, GT_FEW_RING = 5, GT_FEW_WIDE_RING = 3;
+static bool gt_few(int M, int K) { return M <= GT_FEW_ROWS && K >= 64 * GT_FEW_RING; }
+static bool gt_few_wide(int N, int K) { return K / 64 > 200 && (N + 127) / 128 * 8 >= GT_CUS * 3 / 4; }
 static int gt_few_parts(int N, int K) {
-    int parts = GT_CUS / ((N + 63) / 64);
+    const int columns = gt_few_wide(N, K) ? 128 : 64, ring = gt_few_wide(N, K) ? GT_FEW_WIDE_RING : GT_FEW_RING;
+    int parts = GT_CUS / ((N + columns - 1) / columns);
     parts = parts < 1 ? 1 : parts > 8 ? 8 : parts;
-    while (parts > 1 && K / 64 - (parts - 1) * ((K / 64 + parts - 1) / parts) < GT_FEW_RING) --parts;
+    while (parts > 1 && K / 64 - (parts - 1) * ((K / 64 + parts - 1) / parts) < ring) --parts;
     return parts;
 }
 
 extern "C" int tm_tile_linear_parts(int M, int N, int K) {
     if (M <= 0 || N <= 0 || N % 8 || K < 256 || K % 64) return 0;
-    if (gt_few(M, K) && K >= 64 * GT_FEW_RING) return (N + 63) / 64 <= 2 * GT_CUS ? gt_few_parts(N, K) : 0;
+    if (gt_few(M, K)) return (N + 63) / 64 <= 2 * GT_CUS ? gt_few_parts(N, K) : 0;
     if ((long long)((M + 127) / 128) * ((N + 127) / 128) > GT_CUS) return 0;
     int best = 0;
     double least = 0;
@@ -668,7 +674,9 @@ extern "C" int tm_tile_linear_split(const void* A, int lda, int M, int K, const 
     TileArgs a{};
     a.A = A; a.W = W; a.C = parts;
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = N; a.splits = splits;
-    if (gt_few(M, K) && K >= 64 * GT_FEW_RING) return gt_launch<bf16_t, GT_PARTS, 1, 4, 4, 1, GT_FEW_RING, 2>(a, stream);
+    if (gt_few(M, K))
+        return gt_few_wide(N, K) ? gt_launch<bf16_t, GT_PARTS, 2, 4, 2, 2, GT_FEW_WIDE_RING, 2>(a, stream)
+                                 : gt_launch<bf16_t, GT_PARTS, 1, 4, 4, 1, GT_FEW_RING, 2>(a, stream);
     return gt_go<GT_PARTS>(a, gt_choose(M, N, K, splits), stream);
 }
 
