@@ -269,6 +269,20 @@ def test_products_and_partial_sums_in_32_bit(M, N, K, splits):
     assert (out.double().sum(0) - ref).abs().max() <= _bound32(K)
 
 
+@pytest.mark.parametrize("N,K", [(896, 896), (896, 4864), (2048, 5504), (3584, 3584), (5120, 1120), (8, 96)])
+def test_the_rows_do_not_change_a_row_of_a_split_product_in_32_bit(N, K):
+    lib = library()
+    parts = lib.tm_tile_f32_parts(1, N, K)
+    a, w, _ = _operands32(700, N, K, N + K)
+    sums = {}
+    for M in (17, 64, 65, 200, 333, 700):
+        assert lib.tm_tile_f32_parts(M, N, K) == parts
+        out = torch.full((parts, M, N), float("nan"), device="cuda")
+        assert lib.tm_tile_f32_linear_split(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), I(N), P(out.data_ptr()), I(parts), _stream()) == 0
+        sums[M] = out
+    assert all(torch.equal(out, sums[700][:, :M]) for M, out in sums.items())
+
+
 def test_what_the_kernels_do_not_take_is_refused():
     lib = library()
     a, w, _ = _operands(65, 128, 320, 1)

@@ -724,23 +724,21 @@ extern "C" int tm_tile_f32_qkv_rope(const void* A, int lda, int M, int K, const 
     return gt_go_f32<GT_QKV>(a, stream);
 }
 
-// Parts of K for a product whose sums the next norm adds: as many as even out the CUs' shares and give them two blocks to choose from
-// (a step takes 0.55 us where a CU has one block, 0.445 of its time where it has more); a part more costs the norm a read. Down of
-// the 0.5B shape at 1,000 rows: 86 us in one part, 77 in four, 69 in eight.
+// Parts of K for a product whose sums the next norm adds: as many as give each CU a block of one row of tiles, eight at most, seven
+// steps at least to a part; from N and K alone, so that a row's result does not change with the number of rows (the sums of a
+// part and the norm's addition of the parts are in a fixed order). Few rows want many parts and many rows few, whose sums the
+// norm reads; with the norm, 17 / 100 / 300 / 1,000 / 4,096 rows, us: 4,864 -> 896 in one part 85 / 86 / 87 / 89 / 298, in
+// eight 16 / 19 / 39 / 76 / 290; 896 -> 896 in one 21 / 22 / 22 / 25 / 68, four 10 / 11 / 17 / 28 / 72, seven 9 / 10 / 15 / 31 /
+// 84; 2,048 -> 2,048 in one 40 / 40 / 43 / 74 / 268, eight 11 / 18 / 34 / 87 / 353; 3,584 -> 3,584 in one 65 / 66 / 119 / 224 /
+// 791, four 23 / 37 / 79 / 210 / 842. (The rows decide only whether there is a product.)
 extern "C" int tm_tile_f32_parts(int M, int N, int K) {
     if (M <= 0 || N <= 0 || N % 8 || K < GT_F32_STEP * GT_F32_RING || K % GT_F32_STEP) return 0;
-    const long long tiles = (long long)((M + GT_F32_TILE - 1) / GT_F32_TILE) * ((N + GT_F32_TILE - 1) / GT_F32_TILE);
     const int steps = K / GT_F32_STEP;
-    int best = 1;
-    double least = 0;
-    for (int splits = 1; splits <= 8; ++splits) {
-        const int per = (steps + splits - 1) / splits;
-        if (steps - (splits - 1) * per < GT_F32_RING) continue;
-        const long long rounds = (tiles * splits + GT_CUS - 1) / GT_CUS;
-        const double c = (rounds > 1 ? rounds * (per * 0.445 + 1) : per * 0.55 + 1) + (double)splits * M * N * 4 / 5e6;
-        if (splits == 1 || c < least) best = splits, least = c;
-    }
-    return best;
+    int parts = GT_CUS / ((N + GT_F32_TILE - 1) / GT_F32_TILE);
+    parts = parts < steps / 7 ? parts : steps / 7;
+    parts = parts < 1 ? 1 : parts > 8 ? 8 : parts;
+    while (parts > 1 && steps - (parts - 1) * ((steps + parts - 1) / parts) < GT_F32_RING) --parts;
+    return parts;
 }
 
 // parts[p][m][n], p < splits: the partial sums of A W^T (splits 1: the product itself)
