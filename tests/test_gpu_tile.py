@@ -283,6 +283,24 @@ def test_the_rows_do_not_change_a_row_of_a_split_product_in_32_bit(N, K):
     assert all(torch.equal(out, sums[700][:, :M]) for M, out in sums.items())
 
 
+@pytest.mark.parametrize("N,K", [(9728, 896), (896, 896), (896, 4864), (3584, 18944)])
+def test_products_in_32_bit_lose_less_than_the_kernel_of_one_block_size(N, K):
+    """rms error against 64 bits beside that of gemm_f32_mfma.hip, whose sums run in blocks of 128 k: in blocks of half that, or in
+    parts, the chains are shorter. At K = 896 (one part) the roundings' variance goes with 128 / 4 + 7 and 64 / 4 + 14 additions, 39
+    to 30, and what the matrix unit rounds inside an addition goes with the block: a tenth less at least."""
+    lib = library()
+    M, parts = 333, lib.tm_tile_f32_parts(333, N, K) if N < K or N == K else 1
+    a, w, ref = _operands32(M, N, K, 9)
+    out, before = torch.empty(parts, M, N, device="cuda"), torch.empty(M, N, device="cuda")
+    assert lib.tm_tile_f32_linear_split(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), I(N), P(out.data_ptr()), I(parts), _stream()) == 0
+    assert lib.tm_gemm_f32_mfma(P(a.data_ptr()), I(K), P(w.data_ptr()), None, P(before.data_ptr()), I(N), I(M), I(N), I(K), _stream()) == 0
+    total = out[0]
+    for part in out[1:]:
+        total = total + part                                    # in 32-bit, in the order of the norm
+    now, then = ((t.double() - ref).square().mean().sqrt() for t in (total, before))
+    assert now <= 0.9 * then
+
+
 def test_what_the_kernels_do_not_take_is_refused():
     lib = library()
     a, w, _ = _operands(65, 128, 320, 1)
