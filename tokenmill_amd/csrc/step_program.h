@@ -110,11 +110,20 @@ enum {
     TM_QKV_PANEL,               // ... by the kernel that keeps the normed input in LDS (17 to 64 tokens)
     TM_QKV_STREAM,              // ... by the kernel that streams the packed matrix for up to 64 tokens
     TM_QKV_PLAIN,               // ... by a product over the row-major matrix, with rotation and cache write behind it or in its epilogue
+                                // (the latter are counted once more below)
     TM_GATE_UP_FROM_NORM,
     TM_GATE_UP_STREAM,
     TM_GATE_UP_PLAIN,           // any other product with the SiLU*up epilogue, or a product and then SiLU*up
     TM_PREFILL_SPLIT_KEYS,      // bfloat16 attention of prompt portions: wavefronts split a tile's key blocks
     TM_PREFILL_SHARED_KEYS,     // ... a tile's keys and values staged through LDS for all heads of a kv head
+    TM_QKV_TILED,               // of TM_QKV_PLAIN, the tiled products (gemm_tile.hip), in either type
+    TM_QKV_FEW_F32,             // ... and the 32-bit products of few rows (gemv_f32.hip)
+    TM_GATE_UP_TILED,           // the same of TM_GATE_UP_PLAIN
+    TM_GATE_UP_FEW_F32,
+    TM_PROJECT_TILED,           // output and down projections whose K is split: tiled
+    TM_PROJECT_STREAM,          // ... over the packed matrix (gemm_stream.hip)
+    TM_PROJECT_FEW_F32,         // ... 32-bit, few rows
+    TM_DECODE_F32_SPLIT,        // 32-bit attention of single tokens in chunks (attention_decode_f32.hip)
     TM_PROGRAM_COUNTERS
 };
 void tm_program_counters(const TmProgram* p, long long* out);

@@ -263,6 +263,7 @@ struct Run {
             if (rc) return rc;
             delta = nullptr;
             pending_sums = parts;
+            ++p->taken[TM_PROJECT_TILED];
             return TM_OK;
         }
         // up to 64 rows of what that does not take (a bias; a caller that wants the result itself, which a small kernel adds up),
@@ -275,6 +276,7 @@ struct Run {
             if (rc) return rc;
             delta = nullptr;
             pending_sums = groups;
+            ++p->taken[TM_PROJECT_STREAM];
             return accumulate && resid ? TM_OK : settle();
         }
         if (sums && accumulate && resid && L.N == p->hidden && !L.bias && tile32_ok(L, x_, ldx, M, dtype)) {
@@ -283,6 +285,7 @@ struct Run {
             if (rc) return rc;
             delta = nullptr;
             pending_sums = parts32;
+            ++p->taken[TM_PROJECT_TILED];
             return TM_OK;
         }
         if (sums && accumulate && resid && L.N == p->hidden && !L.bias && gemv32_ok(L, x_, ldx, M, dtype)) {
@@ -292,6 +295,7 @@ struct Run {
                 if (rc) return rc;
                 delta = nullptr;
                 pending_sums = parts32;
+                ++p->taken[TM_PROJECT_FEW_F32];
                 return TM_OK;
             }
         }
@@ -406,6 +410,7 @@ struct Run {
                     q = qkv;
                     q_stride = HD;
                     ++p->taken[TM_QKV_PLAIN];
+                    ++p->taken[TM_QKV_TILED];
                 } else if (tables_fusable && a.D % 32 == 0 && gemv32_ok(a.qkv, xn, hidden, T, dtype) && is_pow2(a.page) &&
                            aligned(a.cos_t, 16) && aligned(a.sin_t, 16) && (!a.write || aligned(a.k_pool, 16))) {
                     // 5. the same in 32-bit, for few tokens
@@ -414,6 +419,7 @@ struct Run {
                     q = qkv;
                     q_stride = HD;
                     ++p->taken[TM_QKV_PLAIN];
+                    ++p->taken[TM_QKV_FEW_F32];
                 } else if (tables_fusable && a.D % 64 == 0 && tile32_ok(a.qkv, xn, hidden, T, dtype) && is_pow2(a.page) && bias_ok &&
                            aligned(a.cos_t, 16) && aligned(a.sin_t, 16) && (!a.write || aligned(a.k_pool, 16))) {
                     // 6. ... and for more
@@ -422,6 +428,7 @@ struct Run {
                     q = qkv;
                     q_stride = HD;
                     ++p->taken[TM_QKV_PLAIN];
+                    ++p->taken[TM_QKV_TILED];
                 } else {
                     // 7. product, then rotation and cache write
                     if ((rc = linear(a.qkv, xn, hidden, T, qkv, QKV, dtype))) return rc;
@@ -482,6 +489,7 @@ struct Run {
                                         program_chunks(p, s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep, a.softcap,
                                         a.sink, (const float*)cg_dec, cgate_ld, stream);
                 done_decode = true;
+                ++p->taken[TM_DECODE_F32_SPLIT];
             }
             if (rc) return rc;
             if (tp && !done_prefill && nd && !done_decode) {
@@ -535,6 +543,7 @@ struct Run {
                 } else if (plain && f.I % 8 == 0 && tile_ok(f.gate_up, xn, hidden, T, dtype) && (T > TM_STREAM_ROWS || 2 * f.I <= TM_TILE_FEW_COLUMNS)) {
                     rc = tm_tile_gate_up_silu(xn, hidden, T, hidden, f.gate_up.w, act, f.I, stream);
                     ++p->taken[TM_GATE_UP_PLAIN];
+                    ++p->taken[TM_GATE_UP_TILED];
                 } else if (plain && two_parts && f.I % 4 == 0 && stream_ok(f.gate_up, xn, hidden, T, dtype, from_norm_rows)) {
                     rc = tm_stream_gate_up_silu(xn, hidden, T, hidden, f.gate_up.packed, act, f.I, stream);
                     ++p->taken[TM_GATE_UP_STREAM];
@@ -544,12 +553,15 @@ struct Run {
                 } else if (plain && f.I % 8 == 0 && tile_ok(f.gate_up, xn, hidden, T, dtype)) {
                     rc = tm_tile_gate_up_silu(xn, hidden, T, hidden, f.gate_up.w, act, f.I, stream);
                     ++p->taken[TM_GATE_UP_PLAIN];
+                    ++p->taken[TM_GATE_UP_TILED];
                 } else if (plain && f.I % 4 == 0 && gemv32_ok(f.gate_up, xn, hidden, T, dtype)) {
                     rc = tm_gemv_f32_gate_up_silu((const float*)xn, hidden, (const float*)f.gate_up.w, (float*)act, T, f.I, hidden, stream);
                     ++p->taken[TM_GATE_UP_PLAIN];
+                    ++p->taken[TM_GATE_UP_FEW_F32];
                 } else if (plain && f.I % 8 == 0 && tile32_ok(f.gate_up, xn, hidden, T, dtype)) {
                     rc = tm_tile_f32_gate_up_silu(xn, hidden, T, hidden, f.gate_up.w, act, f.I, stream);
                     ++p->taken[TM_GATE_UP_PLAIN];
+                    ++p->taken[TM_GATE_UP_TILED];
                 } else {
                     if ((rc = linear(f.gate_up, xn, hidden, T, gu, 2 * f.I, dtype))) return rc;
                     rc = tm_silu_mul(gu, act, dtype, T, f.I, stream);

@@ -61,10 +61,10 @@ TmHook = CFUNCTYPE(None, c_void_p, c_int, c_int, c_int)
 LABELS = ("embed", "qkv", "attention", "o_proj", "gate_up", "down", "norm", "head")
 RUN_LABELS, RUN_TUNE_AT_ONCE = 1, 2
 
-# how q|k|v, the feed-forward's activation and the attention of prompt portions were computed, in the order of the
-# header's counters
+# how q|k|v, the feed-forward's activation, the projections and the attention were computed, in the order of the header's counters
 COUNTERS = ("qkv_from_norm", "qkv_panel", "qkv_stream", "qkv_plain", "gate_up_from_norm",
-            "gate_up_stream", "gate_up_plain", "prefill_split_keys", "prefill_shared_keys")
+            "gate_up_stream", "gate_up_plain", "prefill_split_keys", "prefill_shared_keys", "qkv_tiled", "qkv_few_f32",
+            "gate_up_tiled", "gate_up_few_f32", "project_tiled", "project_stream", "project_few_f32", "decode_f32_split")
 
 
 def bound():

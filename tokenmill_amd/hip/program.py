@@ -200,7 +200,7 @@ class StepProgram:
     # --- run -------------------------------------------------------------------------------------------------
 
     def counters(self) -> dict[str, int]:
-        """How often each way of computing q|k|v and the feed-forward's activation has been taken."""
+        """How often each way of computing an operation has been taken (``abi.COUNTERS``)."""
         out = (ctypes.c_longlong * len(abi.COUNTERS))()
         self._lib.tm_program_counters(self._handle, out)
         return dict(zip(abi.COUNTERS, out))
