@@ -73,6 +73,9 @@ BF16 = [
     ((3072, 24, 4, 2048), 64, {"qkv_stream": 1, **GATE_UP, "project_tiled": 2}),
     ((4096, 32, 8, 2048), 4, {"qkv_stream": 1, "gate_up_stream": 1, "project_stream": 2}),
     ((4096, 32, 8, 2048), 5, {"qkv_stream": 1, "gate_up_stream": 1, "project_tiled": 2}),
+    ((5120, 40, 8, 2048), 5, {"qkv_stream": 1, "gate_up_stream": 1, "project_stream": 2}),
+    ((5120, 40, 8, 2048), 64, {"qkv_stream": 1, **GATE_UP, "project_stream": 2}),
+    ((5120, 40, 8, 2048), 65, TILED),
 ]
 
 

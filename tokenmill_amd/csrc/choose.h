@@ -37,12 +37,15 @@ constexpr int TM_STREAM_ROWS = 64;
 // to 62.1 / 66.6.
 constexpr int TM_TILE_FEW_COLUMNS = 64 * 256;
 // Output and down projections run tiled, K in parts, beyond so many rows: beyond the rows of the kernels that start at the norm
-// at widths from 3,072, else beyond 16. Against the streamed product (the library's for 896 -> 896) with the norm that adds the
-// parts, 8 / 64 rows, us: 896 -> 896 10.4 (of the product alone) to 7.2 / 7.8; 4,864 -> 896 10.5 / 14.7 to 8.6 / 10.5; 2,048 ->
-// 2,048 10.4 / 14.5 to 8.9 / 10.3; 3,584 -> 3,584 12.9 / 19.0 to 11.5 / 13.4; 18,944 -> 3,584 31.0 / 38.6 to 29.4 / 34.9;
-// 5,120 -> 5,120 18.0 / 25.1 to 16.8 / 20.0. In a step of 9 rows the down projections of widths 1,536 and 2,048 (K 8,960 and
-// 11,008) were 1.3 and 1.9 us slower tiled, with 24 rows level: hence 16 there.
-inline int tm_split_rows(int hidden) { return hidden < 3072 ? TM_SKINNY_ROWS : 4; }
+// at widths from 3,072, beyond 16 at smaller ones, and at widths above 4,096 only beyond the streamed products' 64. Against the
+// streamed product (the library's for 896 -> 896) with the norm that adds the parts, 8 / 64 rows, us: 896 -> 896 10.4 (of the
+// product alone) to 7.2 / 7.8; 4,864 -> 896 10.5 / 14.7 to 8.6 / 10.5; 2,048 -> 2,048 10.4 / 14.5 to 8.9 / 10.3; 3,584 -> 3,584
+// 12.9 / 19.0 to 11.5 / 13.4; 18,944 -> 3,584 31.0 / 38.6 to 29.5 / 32.1. In a step of 9 rows the down projections of widths
+// 1,536 and 2,048 (K 8,960 and 11,008) were 1.3 and 1.9 us slower tiled, with 24 rows level: hence 16 there. A layer of whole
+// steps of 5 / 17 / 40 / 64 single tokens, streamed to tiled: width 3,584 122.7 / 130.1 / 144.2 / 156.1 to 122.7 / 127.7 / 140.0 /
+// 150.4; 4,096 (14,336 wide inside) 119.2 / 132.9 / 153.9 / 169.1 to 119.2 / 131.4 / 149.3 / 160.9; 5,120 198.5 / 210.7 / 232.0 /
+// 253.2 to 201.3 / 214.2 / 234.0 / 251.6 (the products level, the sums of more parts to add): hence the line behind 4,096.
+inline int tm_split_rows(int hidden) { return hidden < 3072 ? TM_SKINNY_ROWS : hidden <= 4096 ? 4 : TM_STREAM_ROWS; }
 // (what that does not take, such as a projection with a bias, is streamed where splitting its K over groups of blocks pays:
 // tm_stream_linear_parts in gemm_stream.hip; else it is the library's)
 // most rows one launch of the skinny product takes at all
