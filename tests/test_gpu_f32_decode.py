@@ -143,3 +143,37 @@ def test_attention_of_single_tokens(H, KVH, D, page, extras):
     want = torch.stack(wants).view(S, H * D)
     # scores of size up to about 10 with 32-bit dot products: 2^-20 absolute, which the exponential makes relative; values of size up to 5
     assert (out.double() - want).abs().max() <= 2.0 ** -17
+
+
+def test_the_grid_of_the_attention_does_not_grow_with_the_longest_context_there_can_be():
+    """A block for each of 256 chunks of 64 requests of two kv heads would be 32,768, next to all of which find no key."""
+    blocks = library().tm_attn_decode_f32_blocks
+    assert blocks(64, 2, 256) == 16 and blocks(1, 2, 256) == 256 and blocks(8, 2, 6) == 6 and blocks(5000, 8, 256) == 1
+
+
+def test_attention_of_single_tokens_walks_the_chunks_of_long_contexts():
+    """More chunks than the grid has blocks for a pair: the same bits as for each request alone, whose grid has one for each."""
+    S, H, KVH, D, page, most = 32, 32, 16, 32, 16, 2000
+    g = torch.Generator(device="cuda").manual_seed(3)
+    W, chunks = -(-most // page), -(-most // 128)
+    assert library().tm_attn_decode_f32_blocks(S, KVH, chunks) == 4 and library().tm_attn_decode_f32_blocks(1, KVH, chunks) == chunks
+    q = torch.randn(S, H * D, generator=g, device="cuda")
+    k, v = torch.randn(2, S * W * page * KVH * D, generator=g, device="cuda")
+    table = torch.arange(S * W, device="cuda", dtype=torch.int32).view(S, W)
+    ctxs = torch.randint(1, most + 1, (S,), generator=g, device="cuda", dtype=torch.int32)
+    ctxs[:3] = torch.tensor([most, 1, 512])
+
+    def run(rows, window, keep):
+        n = len(rows)
+        out = torch.full((n, H * D), float("nan"), device="cuda")
+        part_o, part_ml = (torch.full((n * H * chunks * e,), float("nan"), device="cuda") for e in (D, 2))
+        qs, ts, cs = q[rows].contiguous(), table[rows].contiguous(), ctxs[rows].contiguous()
+        assert library().tm_attn_decode_f32(_ptr(qs), I(H * D), _ptr(out), I(H * D), _ptr(k), _ptr(v), _ptr(ts), I(W), _ptr(cs), _ptr(part_o),
+                                            _ptr(part_ml), I(chunks), I(n), I(H), I(KVH), I(D), I(page), F(D ** -0.5), I(window), I(keep), F(0.0),
+                                            _ptr(None), _ptr(None), I(H * D), _stream()) == 0
+        return out
+
+    for window, keep in ((0, 0), (300, 20)):
+        together = run(list(range(S)), window, keep)
+        assert together.isfinite().all()
+        assert torch.equal(together, torch.cat([run([s], window, keep) for s in range(S)]))

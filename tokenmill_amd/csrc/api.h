@@ -80,6 +80,7 @@ int tm_gemv_f32_qkv_rope(const float* A, int lda, const float* W, const float* b
 // Attention of single tokens in 32-bit (attention_decode_f32.hip): as tm_attn_decode_mfma_cap with chunks of 128 keys; part_o float
 // [S, H, max_chunks, D], part_ml [S, H, max_chunks, 2].
 int tm_attn_decode_f32_takes(const void* q, int q_stride, const void* k_pool, const void* v_pool, int H, int KVH, int D, int page);
+int tm_attn_decode_f32_blocks(int S, int KVH, int max_chunks);     // blocks its grid has for a (request, kv head) pair
 int tm_attn_decode_f32(const float* q, int q_stride, float* out, int out_stride, const float* k_pool, const float* v_pool,
                        const int* block_tables, int table_width, const int* context_lens, float* part_o, float* part_ml, int max_chunks, int S,
                        int H, int KVH, int D, int page, float scale, int window, int keep, float softcap, const float* sink, const float* cgate,
