@@ -207,10 +207,26 @@ struct Products {
     }
 };
 
-// chunks that the decode attention's partial results have room for
-int program_chunks(const TmProgram* p, int max_decode_context) {
-    const int n = max_decode_context > 0 ? max_decode_context : 1;
+// The attention of `num_decode` single tokens whose contexts reach `context`: does its matrix-unit kernel take it in chunks, whose
+// partial results need room? (What the tensors' places add to the question, an operation asks where it runs.)
+bool decode_in_chunks(const TmProgram* p, const TmAttentionOp& a, int num_decode, int context) {
+    if (num_decode <= 0) return false;
+    if (p->dtype == TM_F32)         // (beyond that many pairs the generic kernel's blocks of one (token, head) pair fill the chip)
+        return num_decode * a.KVH < TM_DECODE_SPLIT_PAIRS && tm_attn_decode_f32_takes(nullptr, a.H * a.D, a.k_pool, a.v_pool, a.H, a.KVH, a.D, a.page);
+    return tm_decode_splits(num_decode, a.KVH, context);
+}
+
+// chunks of such a step
+int context_chunks(const TmProgram* p, int context) {
+    const int n = context > 0 ? context : 1;
     return p->dtype == TM_F32 ? (n + TM_DECODE_F32_CHUNK - 1) / TM_DECODE_F32_CHUNK : tm_decode_chunks(n);
+}
+
+// chunks that the decode attention's partial results have room for: none where no operation of the program takes them
+int program_chunks(const TmProgram* p, int num_decode, int context) {
+    for (const Op& op : p->ops)
+        if (op.kind == OP_ATTENTION && decode_in_chunks(p, op.att, num_decode, context)) return context_chunks(p, context);
+    return 0;
 }
 
 struct Run {
@@ -475,18 +491,17 @@ struct Run {
             const char* q_dec = (const char*)q + (size_t)tp * q_stride * es;
             char* out_dec = (char*)attn + (size_t)tp * HD * es;
             if (nd && dtype == TM_BF16 && head_mfma && page_ok && a.H / a.KVH <= 16 && q_ok) {
-                const bool split = tm_decode_splits(nd, a.KVH, s->max_decode_context);
+                const bool split = decode_in_chunks(p, a, nd, s->max_decode_context);
                 rc = tm_attn_decode_mfma_cap(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
                                              s->context_lens + (S - nd), split ? part_o : nullptr, split ? part_ml : nullptr,
                                              tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep,
                                              a.softcap, a.sink, cg_dec, cgate_ld, stream);
                 done_decode = true;
-            } else if (nd && dtype == TM_F32 && nd * a.KVH < TM_DECODE_SPLIT_PAIRS &&
+            } else if (nd && dtype == TM_F32 && decode_in_chunks(p, a, nd, s->max_decode_context) &&
                        tm_attn_decode_f32_takes(q_dec, q_stride, a.k_pool, a.v_pool, a.H, a.KVH, a.D, a.page)) {
-                // (beyond that many pairs the generic kernel's blocks of one (token, head) pair fill the chip)
                 rc = tm_attn_decode_f32((const float*)q_dec, q_stride, (float*)out_dec, HD, (const float*)a.k_pool, (const float*)a.v_pool,
                                         tables + (size_t)(S - nd) * W, W, s->context_lens + (S - nd), part_o, part_ml,
-                                        program_chunks(p, s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep, a.softcap,
+                                        context_chunks(p, s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep, a.softcap,
                                         a.sink, (const float*)cg_dec, cgate_ld, stream);
                 done_decode = true;
                 ++p->taken[TM_DECODE_F32_SPLIT];
@@ -710,7 +725,7 @@ size_t tm_program_workspace_bytes(const TmProgram* p, int T, int R, int num_deco
     n += align_up((size_t)T * p->max_act * es);                      // silu(gate) * up
     n += align_up((size_t)T * p->hidden * es);                       // a product's output still to be added
     n += align_up((size_t)(R > 0 ? R : 1) * p->hidden * es);         // normed rows for the head
-    const size_t chunks = (size_t)program_chunks(p, max_decode_context);
+    const size_t chunks = (size_t)program_chunks(p, num_decode, max_decode_context);
     n += align_up((size_t)num_decode * p->max_heads_d * chunks * 4); // split decode attention: partial values
     n += align_up((size_t)num_decode * p->max_heads * chunks * 2 * 4);   // ... and their (max, sum)
     n += align_up((size_t)program_sums(p, T) * T * p->hidden * 4);   // partial sums of a product whose K is split over blocks
@@ -758,7 +773,7 @@ int tm_program_run(const TmProgram* p, int first, int count, const TmStep* s, Tm
     r.act = take((size_t)T * p->max_act * es);
     r.delta_buf = take((size_t)T * p->hidden * es);
     r.hnorm = take((size_t)(R > 0 ? R : 1) * p->hidden * es);
-    const size_t chunks = (size_t)program_chunks(p, s->max_decode_context);
+    const size_t chunks = (size_t)program_chunks(p, s->num_decode, s->max_decode_context);
     r.part_o = (float*)take((size_t)s->num_decode * p->max_heads_d * chunks * 4);
     r.part_ml = (float*)take((size_t)s->num_decode * p->max_heads * chunks * 2 * 4);
     const int parts = program_sums(p, T);
