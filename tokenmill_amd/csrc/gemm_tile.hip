@@ -79,7 +79,7 @@ __device__ __forceinline__ void gt_store8(T* dst, const float (&v)[8]) {
 
 // 16 bytes a lane from base + voff (bytes) to LDS at lds (bytes, wave-uniform) + 16 * lane
 __device__ __forceinline__ void gt_load_lds(uint32_t lds, uint32_t voff, const void* base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base));
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "m0", "memory");
 }
 
 // two values rounded to the tensors' type and back, by one conversion
@@ -303,6 +303,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
 
     gt_wait_loads<(ST - 1) * NL>();
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");                                  // (the barrier alone holds no read back from before it)
     int buf = 0;
     while (true) {
         // the first half's operands of a tile: read here, not behind the tile before, whose epilogue needs the registers
