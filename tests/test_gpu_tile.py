@@ -1,5 +1,6 @@
 """The tiled products of prompt-sized steps (csrc/gemm_tile.hip) against 64-bit ones, at the edges of their tiles: rows and columns
-that fill no tile, the shortest K, the last part of a split K shorter than the others, every tile shape the rule chooses."""
+that fill no tile, the shortest K, the last part of a split K shorter than the others, every tile shape the rule chooses with
+every epilogue, rows of A that lie apart."""
 from __future__ import annotations
 
 import ctypes
@@ -12,9 +13,10 @@ from tokenmill_amd.hip.library import library
 pytestmark = pytest.mark.gpu
 P, I = ctypes.c_void_p, ctypes.c_int
 
-# (rows, result columns, K): with those below they reach every tile
+# (rows, result columns, K): every tile
 SILU = [(65, 8, 256), (77, 4864, 320), (129, 1000, 256), (200, 4864, 256), (257, 4864, 448), (333, 4864, 256), (512, 4864, 896), (1000, 6000, 448),
-        (700, 4864, 448), (1000, 4864, 896), (2048, 4864, 896), (4001, 4864, 896), (2000, 4096, 1792), (1025, 40, 256)]
+        (700, 4864, 448), (1000, 4864, 896), (2048, 4864, 896), (4001, 4864, 896), (2000, 4096, 1792), (1025, 40, 256), (33, 2816, 1024),
+        (700, 2816, 1024)]
 
 
 def _operands(M, N, K, seed):
@@ -28,12 +30,14 @@ def _stream():
     return P(torch.cuda.current_stream().cuda_stream)
 
 
-def test_the_sizes_below_reach_every_tile():
+def test_the_sizes_reach_every_tile_with_every_epilogue():
     lib = library()
-    shapes = {lib.tm_gemm_tile_shape(M, 2 * n, K, 1) for M, n, K in SILU}
-    shapes |= {lib.tm_gemm_tile_shape(M, N, K, lib.tm_tile_linear_parts(M, N, K)) for M, N, K in PARTS}
-    shapes |= {lib.tm_gemm_tile_shape(M, (H + 2 * KVH) * D, K, 1) for M, H, KVH, D, K in QKV}
-    assert shapes == set(range(11))
+    few = [size for size in PARTS if size[0] <= 64 and size[2] >= 320]          # these run one of two tiles of their own
+    assert {K // 64 > 200 and N >= 3072 for M, N, K in few} == {True, False}
+    for shapes in ({lib.tm_gemm_tile_shape(M, 2 * n, K, 1) for M, n, K in SILU},
+                   {lib.tm_gemm_tile_shape(M, (H + 2 * KVH) * D, K, 1) for M, H, KVH, D, K, page in QKV},
+                   {lib.tm_gemm_tile_shape(M, N, K, lib.tm_tile_linear_parts(M, N, K)) for M, N, K in PARTS if (M, N, K) not in few}):
+        assert shapes == set(range(11))
 
 
 @pytest.mark.parametrize("M,n,K", SILU)
@@ -69,14 +73,17 @@ def test_the_activation_is_the_one_of_the_other_products(scale):
     assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.nan_to_num(0.0), want.nan_to_num(0.0))
 
 
-QKV = [(65, 14, 2, 64, 256), (333, 14, 2, 64, 896), (1000, 28, 4, 128, 256), (2500, 14, 2, 64, 256), (70, 3, 1, 192, 256)]
+# (rows, heads, kv heads, head size, K, page): every tile
+QKV = [(65, 14, 2, 64, 256, 16), (333, 14, 2, 64, 896, 16), (1000, 28, 4, 128, 256, 16), (2500, 14, 2, 64, 256, 16), (70, 3, 1, 192, 256, 16),
+       (66, 28, 4, 128, 512, 4), (400, 28, 4, 128, 512, 64), (600, 28, 4, 128, 512, 128), (1001, 28, 4, 128, 512, 1), (1500, 28, 4, 128, 512, 32),
+       (2000, 28, 4, 128, 512, 16), (2500, 28, 4, 128, 512, 16), (3001, 28, 4, 128, 512, 64), (3200, 28, 4, 128, 512, 16), (199, 28, 4, 128, 512, 16)]
 
 
 @pytest.mark.parametrize("stored", [True, False])
 @pytest.mark.parametrize("bias_dtype", [torch.float32, torch.bfloat16, None])
-@pytest.mark.parametrize("M,H,KVH,D,K", QKV)
-def test_qkv_with_rotation_and_cache_write(M, H, KVH, D, K, bias_dtype, stored):
-    N, page = (H + 2 * KVH) * D, 16
+@pytest.mark.parametrize("M,H,KVH,D,K,page", QKV)
+def test_qkv_with_rotation_and_cache_write(M, H, KVH, D, K, page, bias_dtype, stored):
+    N = (H + 2 * KVH) * D
     a, w, ref = _operands(M, N, K, M + H)
     g = torch.Generator(device="cuda").manual_seed(M)
     bias = torch.randn(N, generator=g, device="cuda").to(bias_dtype) if bias_dtype else None
@@ -111,10 +118,11 @@ def test_qkv_with_rotation_and_cache_write(M, H, KVH, D, K, bias_dtype, stored):
 
 
 PARTS = [(65, 896, 896), (77, 896, 4864), (130, 3584, 960), (333, 896, 4864), (1000, 1016, 4864), (2048, 896, 896), (2048, 896, 4864),
-         (4000, 896, 4864), (1000, 3584, 3584),
-         # few rows: the tile with a ring of five, its shortest parts, one part, K below the ring, K beyond its range
+         (4000, 896, 4864), (1000, 3584, 3584), (500, 3584, 18944), (650, 3584, 18944), (520, 3584, 18944), (265, 3584, 18944),
+         (200, 3584, 18944), (135, 3584, 18944), (135, 3584, 3584), (100, 3584, 3584),
+         # few rows: the tile with a ring of five, its shortest parts, one part, K below the ring, the wide tile of long K
          (1, 896, 896), (8, 3584, 3584), (17, 1000, 320), (16, 896, 4864), (33, 40, 256), (64, 2048, 2048), (64, 520, 12800),
-         (40, 264, 12864), (5, 8200, 640)]
+         (40, 264, 12864), (5, 8200, 640), (48, 3584, 18944), (3, 3072, 12864)]
 
 
 @pytest.mark.parametrize("M,N,K", PARTS)
@@ -127,6 +135,38 @@ def test_partial_sums_of_a_split_k(M, N, K):
     assert lib.tm_tile_linear_split(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), I(N), P(out.data_ptr()), _stream()) == 0
     # 32-bit sums of products of size 1 / sqrt(K): the rounding of each of K additions to a sum of at most about 5
     assert (out.double().sum(0) - ref).abs().max() <= 2.0 ** -24 * 5 * 4 * K ** 0.5
+
+
+@pytest.mark.parametrize("M,K", [(40, 640), (77, 256), (300, 896)])
+def test_rows_of_a_that_lie_apart(M, K):
+    """The same bits as of rows side by side, from every epilogue and in both types."""
+    lib, N, H, KVH, D = library(), 512, 2, 1, 128
+    for dt in (torch.bfloat16, torch.float32):
+        bf = dt is torch.bfloat16
+        g = torch.Generator(device="cuda").manual_seed(M)
+        wide = torch.randn(M, K + 24, generator=g, device="cuda").to(dt)
+        w = (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(dt)
+        cos, sin = torch.rand(2, M, D // 2, generator=g, device="cuda")
+        pos = torch.arange(M, device="cuda", dtype=torch.int32)
+        got = []
+        for a in (wide[:, :K], wide[:, :K].contiguous()):
+            lead = (P(a.data_ptr()), I(a.stride(0)), I(M), I(K), P(w.data_ptr()))
+            act, q = torch.empty(M, N // 2, device="cuda", dtype=dt), torch.empty(M, H * D, device="cuda", dtype=dt)
+            k, v = torch.zeros(2, M * KVH * D, device="cuda", dtype=dt)
+            n = lib.tm_tile_linear_parts(M, N, K) if bf else 2
+            sums = torch.empty(n, M, N, device="cuda")
+            tail = (P(q.data_ptr()), I(H), I(KVH), I(D), P(cos.data_ptr()), P(sin.data_ptr()), P(pos.data_ptr()), P(pos.data_ptr()), P(k.data_ptr()),
+                    P(v.data_ptr()), I(1), _stream())
+            if bf:
+                assert lib.tm_tile_gate_up_silu(*lead, P(act.data_ptr()), I(N // 2), _stream()) == 0
+                assert lib.tm_tile_qkv_rope(*lead, P(None), I(-1), *tail) == 0
+                assert lib.tm_tile_linear_split(*lead, I(N), P(sums.data_ptr()), _stream()) == 0
+            else:
+                assert lib.tm_tile_f32_gate_up_silu(*lead, P(act.data_ptr()), I(N // 2), _stream()) == 0
+                assert lib.tm_tile_f32_qkv_rope(*lead, P(None), *tail) == 0
+                assert lib.tm_tile_f32_linear_split(*lead, I(N), P(sums.data_ptr()), I(n), _stream()) == 0
+            got.append((act, q, k, v, sums))
+        assert all(torch.equal(x, y) for x, y in zip(*got)) and all(x.isfinite().all() for x in got[0])
 
 
 # an output and a down projection of the shipped shapes and what lies around the line between the two tiles of few rows
