@@ -41,3 +41,24 @@ def test_top_k_at_the_bound(where, k, p):
     got = tokens(logits, k, p, us)
     assert all(a == b or m < 1e-4 for a, b, m in zip(got, want, margins))
     assert sum(a == b for a, b in zip(got, want)) >= R - 2
+
+
+@pytest.mark.parametrize("k", [2, 50, 244, 245, 246, 980])
+def test_top_k_at_the_bound_of_the_widest_rows(k):
+    """A million entries have 245 chunks, whose maxima are the keys that the bound is looked up among. Entries of whole steps tie
+    by the thousand, and every token is among the k that are kept."""
+    R, wide = 4, 1_000_000
+    g = torch.Generator().manual_seed(k)
+    logits = (torch.randn(R, wide, generator=g) * 3).round() / 4
+    logits[1, :900_000] = float("nan")                          # most shares without a number
+    logits[2] = logits[2].sort().values                         # the largest all in the last shares
+    us = [P.uniform_from_counter(3, r) for r in range(R)]
+    kept = torch.zeros(R, wide, dtype=torch.bool)
+    for r in range(R):
+        kept[r, logits[r].nan_to_num(float("-inf")).sort(descending=True, stable=True).indices[:k]] = True
+    for u in (us, [0.0] * R, [1.0 - 2.0 ** -24] * R):
+        got = tokens(logits, k, 1.0, u)
+        assert all(kept[r, t] for r, t in enumerate(got))
+        z = torch.where(kept, logits.double() / 0.9, torch.tensor(float("-inf"), dtype=torch.float64)).softmax(1).cumsum(1)
+        for r, t in enumerate(got):                             # the token in whose share of the mass u lies, to 32-bit sums of k weights
+            assert (z[r, t - 1] if t else 0.0) - 1e-5 <= u[r] <= z[r, t] + 1e-5

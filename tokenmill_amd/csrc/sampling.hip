@@ -393,53 +393,58 @@ __device__ __forceinline__ bool share_below(const float* __restrict__ wave_v, si
     const float z = wave_v[chunk_at * (AM_NT / TM_WAVE) + threadIdx.x / TM_WAVE] * inv_t;
     return z == z && order_key(z) < floor;
 }
-static_assert(AM_NT == SR_NT, "the wavefronts' shares of a chunk are the same in all launches");
+static_assert(AM_NT == SR_NT && SR_NT == 256, "the wavefronts' shares of a chunk are the same in all launches");
 
-// The k-th largest of the wavefronts' maxima bounds the k-th largest entry from below: each maximum is an entry of its own.
-// Shares below it take no part in top-k, and the ones below top-k's end none in what follows: with k = 50 two thirds of the
-// shares of a row of 151,936 are passed over without a read, and next to no entry reaches the histograms' atomics.
-#define SR_MAX_SHARES (256 * (AM_NT / TM_WAVE))
+// The k-th largest of the shares' maxima bounds the k-th largest entry from below: each maximum is an entry of its own. Shares
+// below it take no part in top-k, and the ones below top-k's end none in what follows: with k = 50 two thirds of the shares of a
+// row of 151,936 are passed over without a read, and next to no entry reaches the histograms' atomics. A share is a wavefront's,
+// or, in rows of more than 64 chunks, a whole chunk's: one key a thread, and every thread counts the keys larger than its own,
+// n steps (2.5 us for 152 keys; with all 980 wavefronts of a row of 1,000,000 it was 60 us, more than the bound saves: a row
+// sampled with k = 50 68.9 us without a bound, 116.1 with that, 57.9 so).
 __global__ __launch_bounds__(SR_NT) void sample_bound_kernel(const float* __restrict__ part_v, const int* __restrict__ part_i,
                                                              const float* __restrict__ wave_v, int NB, int V,
                                                              const float* __restrict__ temperature, const int* __restrict__ top_k,
                                                              const float* __restrict__ top_p, float* __restrict__ rowmax,
                                                              int* __restrict__ rowarg, RowState* __restrict__ state) {
-    __shared__ uint32_t s_key[SR_MAX_SHARES];
+    __shared__ uint32_t s_key[SR_NT];
     __shared__ ArgMax s_best[SR_NT / TM_WAVE];
     __shared__ uint32_t s_bound;
-    const int row = blockIdx.x, n = NB * (AM_NT / TM_WAVE);
+    constexpr int WAVES = AM_NT / TM_WAVE;
+    const int row = blockIdx.x, t = threadIdx.x;
+    const bool by_wave = NB * WAVES <= SR_NT;
+    const int n = by_wave ? NB * WAVES : NB;             // (a row has at most SR_NT chunks)
+    const RowParams rp = row_params(row, V, temperature, top_k, top_p, nullptr);
     ArgMax best{-INFINITY, -1};
-    for (int c = threadIdx.x; c < NB; c += SR_NT) best = better(best, ArgMax{part_v[(size_t)row * NB + c], part_i[(size_t)row * NB + c]});
+    if (t < NB) best = ArgMax{part_v[(size_t)row * NB + t], part_i[(size_t)row * NB + t]};
+    uint32_t key = 0u;                                   // (no number's key is 0)
+    if (t < n) {
+        const float z = (by_wave ? wave_v[(size_t)row * n + t] : best.i < 0 ? NAN : best.v) * rp.inv_t;
+        if (z == z) key = order_key(z);
+    }
 #pragma unroll
     for (int off = TM_WAVE / 2; off > 0; off >>= 1) {
         ArgMax o{__shfl_xor(best.v, off, TM_WAVE), __shfl_xor(best.i, off, TM_WAVE)};
         best = better(best, o);
     }
-    if (threadIdx.x % TM_WAVE == 0) s_best[threadIdx.x / TM_WAVE] = best;
-    const RowParams rp = row_params(row, V, temperature, top_k, top_p, nullptr);
-    for (int i = threadIdx.x; i < n; i += SR_NT) {
-        const float z = wave_v[(size_t)row * n + i] * rp.inv_t;
-        s_key[i] = z == z ? order_key(z) : 0u;           // (no number's key is 0)
-    }
-    if (threadIdx.x == 0) s_bound = 0u;
+    if (t % TM_WAVE == 0) s_best[t / TM_WAVE] = best;
+    s_key[t] = key;
+    if (t == 0) s_bound = 0u;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (t == 0) {
         for (int v = 1; v < SR_NT / TM_WAVE; ++v) best = better(best, s_best[v]);
         rowmax[row] = best.i < 0 ? 0.f : best.v;
         rowarg[row] = best.i < 0 ? 0 : best.i;
     }
-    if (rp.need_k && rp.k <= n)
-        for (int i = threadIdx.x; i < n; i += SR_NT) {
-            const uint32_t key = s_key[i];
-            int larger = 0, level = 0;
-            for (int j = 0; j < n; ++j) {
-                larger += s_key[j] > key;
-                level += s_key[j] == key;
-            }
-            if (larger < rp.k && larger + level >= rp.k) s_bound = key;    // (threads that write it write one value)
+    if (rp.need_k && rp.k <= n && t < n) {
+        int larger = 0, level = 0;
+        for (int j = 0; j < n; ++j) {
+            larger += s_key[j] > key;
+            level += s_key[j] == key;
         }
+        if (larger < rp.k && larger + level >= rp.k) s_bound = key;        // (threads that write it write one value)
+    }
     __syncthreads();
-    if (threadIdx.x == 0) state[row].bound = s_bound;
+    if (t == 0) state[row].bound = s_bound;
 }
 
 // One level of a descent: the chunk's entries that match the buckets picked so far, into the row's
