@@ -49,3 +49,28 @@ def test_shapes_that_the_32_bit_kernel_does_not_take_hold_no_room_for_it(heads, 
 def test_one_chunk():
     """In 32-bit a single chunk passes through the partial results too, in bfloat16 it does not."""
     assert _grows_by(F32, 14, 2, 64, 8, 100) == _chunked(14, 64, 8, 1) and _grows_by(BF16, 14, 2, 64, 8, 256) == 0
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+def test_partial_sums_have_the_room_of_the_projection_with_most_parts(dtype):
+    """However many layers there are and whichever comes first: 896 -> 896 and 4,864 -> 896 are cut into different numbers of parts."""
+    lib, place = abi.bound(), 4096
+    parts = lambda T, K: (lib.tm_tile_linear_parts if dtype == BF16 else lib.tm_tile_f32_parts)(T, HIDDEN, K)      # noqa: E731
+
+    def program(layers):
+        p = lib.tm_program_create(dtype, HIDDEN)
+        for inside in layers:
+            lin = lambda n, k: abi.TmLinear(w=place, N=n, K=k, dtype=dtype, bias_dtype=-1)                          # noqa: E731
+            assert lib.tm_program_add_feed_forward(p, abi.TmFfnOp(gate_up=lin(2 * inside, HIDDEN), down=lin(HIDDEN, inside), I=inside)) >= 0
+        return p
+
+    first, many, other = program([4864, 896]), program([896, 4864] * 12), program([896])
+    for T in (65, 300, 1000, 2048):
+        assert parts(T, 4864) > parts(T, 896) or dtype == BF16
+        sizes = [lib.tm_program_workspace_bytes(p, T, 1, 0, 0) for p in (first, many, other)]
+        size, up = 4 if dtype == F32 else 2, lambda n: -(-n // 256) * 256
+        widest = up(T * 2 * 4864 * size) + up(T * 4864 * size) - up(T * 2 * 896 * size) - up(T * 896 * size)
+        more = max(parts(T, 4864), parts(T, 896)) - parts(T, 896)
+        assert sizes[0] == sizes[1] == sizes[2] + widest + up(more * T * HIDDEN * 4)
+    for p in (first, many, other):
+        lib.tm_program_destroy(p)

@@ -48,6 +48,9 @@ struct TmProgram {
     // a matrix the checkpoint stores in 32-bit stays 32-bit in a bfloat16 model: its product runs in 32-bit on a
     // widened copy of the activations; the widest input and output of such products
     int max_wide_in = 0, max_wide_out = 0;
+    // the output and down projections, one of each kind that the rules for their partial sums tell apart: a step asks for those
+    // sums' room three times, and the rule weighs 88 ways to cut a matrix (24 layers: 30 us of the host a time, of two kinds 1.3)
+    std::vector<TmLinear> projections;
     TmHook hook = nullptr;
     void* hook_user = nullptr;
     TmTune tune{0, 3, 0};
@@ -623,6 +626,12 @@ bool linear_fits(TmProgram* p, const TmLinear& L) {
     return true;
 }
 
+void note_projection(TmProgram* p, const TmLinear& L) {
+    for (const TmLinear& o : p->projections)
+        if (o.N == L.N && o.K == L.K && o.dtype == L.dtype && !o.bias == !L.bias && o.act == L.act) return;
+    p->projections.push_back(L);
+}
+
 }  // namespace
 
 extern "C" {
@@ -668,6 +677,7 @@ int tm_program_add_attention(TmProgram* p, const TmAttentionOp* a) {
     op.kind = OP_ATTENTION;
     op.att = *a;
     p->ops.push_back(op);
+    note_projection(p, a->o);
     if (!a->outside && a->qkv.N > p->max_qkv) p->max_qkv = a->qkv.N;
     if (a->H > p->max_heads) p->max_heads = a->H;
     if (a->H * a->D > p->max_heads_d) p->max_heads_d = a->H * a->D;
@@ -682,6 +692,7 @@ int tm_program_add_feed_forward(TmProgram* p, const TmFfnOp* f) {
     op.kind = OP_FEED_FORWARD;
     op.ffn = *f;
     p->ops.push_back(op);
+    note_projection(p, f->down);
     if (2 * f->I > p->max_gu) p->max_gu = 2 * f->I;
     if (f->I > p->max_act) p->max_act = f->I;
     return (int)p->ops.size() - 1;
@@ -704,9 +715,8 @@ void tm_program_counters(const TmProgram* p, long long* out) {
 static int program_sums(const TmProgram* p, int T) {
     if (p->dtype == TM_BF16 && T <= TM_STREAM_ROWS) return TM_MAX_SUMS;
     int most = 0;
-    for (const Op& op : p->ops) {
-        const TmLinear* L = op.kind == OP_ATTENTION ? &op.att.o : op.kind == OP_FEED_FORWARD ? &op.ffn.down : nullptr;
-        const int parts = !L ? 0 : p->dtype == TM_BF16 ? tile_parts(*L, T) : T <= TM_GEMV_F32_ROWS ? tm_gemv_f32_parts(L->N, L->K) : tm_tile_f32_parts(T, L->N, L->K);
+    for (const TmLinear& L : p->projections) {
+        const int parts = p->dtype == TM_BF16 ? tile_parts(L, T) : T <= TM_GEMV_F32_ROWS ? tm_gemv_f32_parts(L.N, L.K) : tm_tile_f32_parts(T, L.N, L.K);
         if (parts > most) most = parts;
     }
     return most;
