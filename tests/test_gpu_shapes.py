@@ -170,9 +170,10 @@ def test_the_measured_configuration_against_the_plain_implementation(layer_model
         del eng
         torch.cuda.empty_cache()
     # Up to 16 rows every kernel fixes its order of additions by the sizes alone: padding a step to its bucket
-    # changes no bit. Beyond that the products are the library's, which may pick another algorithm for the 48
-    # rows of a bucket than for the 40 of the eager step: then the logits agree up to rounding, and a token can
-    # differ where two candidates are a near-tie (after which the two runs generate different sequences, each
+    # changes no bit. Beyond that the layers' products do too (up to 64 rows), but the output head is the
+    # library's, which may pick another algorithm for the 48 rows of a bucket than for the 40 of the eager step, and
+    # 48 requests of four kv heads are enough pairs for the one-block attention where 40 are not: then the logits
+    # agree up to rounding, and a token can differ where two candidates are a near-tie (after which the two runs generate different sequences, each
     # of which must be right by itself). Such requests are a minority, and each is checked against the plain
     # implementation, beside a sample spread over the batch (the first is one that crosses 2,304 keys).
     if n_requests <= 16:

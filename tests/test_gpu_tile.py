@@ -169,6 +169,31 @@ def test_rows_of_a_that_lie_apart(M, K):
         assert all(torch.equal(x, y) for x, y in zip(*got)) and all(x.isfinite().all() for x in got[0])
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_the_rows_do_not_change_a_row_of_gate_up_or_of_qkv(dt):
+    """Whichever tile the number of rows chooses: K is not split, and a row's sums run over k in one order."""
+    lib, most, K, n, H, KVH, D = library(), 3200, 896, 2048, 14, 2, 64
+    g = torch.Generator(device="cuda").manual_seed(4)
+    a = torch.randn(most, K, generator=g, device="cuda").to(dt)
+    w = (torch.randn(2 * n, K, generator=g, device="cuda") * K ** -0.5).to(dt)
+    cos, sin = torch.rand(2, most, D // 2, generator=g, device="cuda")
+    pos = torch.arange(most, device="cuda", dtype=torch.int32)
+    f32, tiles, got = dt is torch.float32, set(), []
+    for M in (most, 17, 65, 130, 200, 333, 512, 700, 1000, 1500, 2048):
+        act, q = torch.empty(M, n, device="cuda", dtype=dt), torch.empty(M, H * D, device="cuda", dtype=dt)
+        k, v = torch.zeros(2, most, KVH * D, device="cuda", dtype=dt)
+        lead = (P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()))
+        tail = (P(q.data_ptr()), I(H), I(KVH), I(D), P(cos.data_ptr()), P(sin.data_ptr()), P(pos.data_ptr()), P(pos.data_ptr()), P(k.data_ptr()),
+                P(v.data_ptr()), I(1), _stream())
+        assert (lib.tm_tile_f32_gate_up_silu if f32 else lib.tm_tile_gate_up_silu)(*lead, P(act.data_ptr()), I(n), _stream()) == 0
+        assert (lib.tm_tile_f32_qkv_rope(*lead, P(None), *tail) if f32 else lib.tm_tile_qkv_rope(*lead, P(None), I(-1), *tail)) == 0
+        got.append((act, q, k[:M], v[:M]))
+        tiles.add(lib.tm_gemm_tile_shape(M, 2 * n, K, 1))
+    assert len(tiles) >= 6
+    for few in got[1:]:
+        assert all(torch.equal(x, y[:x.shape[0]]) for x, y in zip(few, got[0]))
+
+
 # an output and a down projection of the shipped shapes and what lies around the line between the two tiles of few rows
 @pytest.mark.parametrize("N,K", [(896, 896), (896, 4864), (2048, 11008), (3584, 3584), (3584, 18944), (5120, 27648), (3072, 12864), (2944, 12864)])
 def test_few_rows_do_not_change_a_row_of_a_split_product(N, K):

@@ -58,7 +58,7 @@ int tm_tile_f32_qkv_rope(const void* A, int lda, int M, int K, const void* W, co
 int tm_tile_f32_parts(int M, int N, int K);
 int tm_tile_f32_linear_split(const void* A, int lda, int M, int K, const void* W, int N, float* parts, int splits, hipStream_t stream);
 
-// The experts' products of grouped_mfma.hip in tiles of 64 slots, for steps whose route has tiles of 64 or 128 rows (kind 0: silu(gate) * up,
+// The experts' products of grouped_mfma.hip in tiles of 128 or 64 slots, for steps whose route has tiles of 64 or 128 rows (kind 0: silu(gate) * up,
 // 1: clamped gate, 2: relu squared, 3: down, 32-bit).
 int tm_tile_experts_takes(const void* A, int lda, long long rows, const void* W, const void* C, int tile_rows, int K, int N);
 int tm_tile_experts(int kind, const void* A, int lda, const int* row_src, int src_div, const void* W, void* C, const int* tiles,

@@ -32,7 +32,7 @@ constexpr int TM_PANEL_QKV_ROWS = 64;
 constexpr int TM_STREAM_ROWS = 64;
 // ... except gate|up where a 64-column tile for each CU covers the matrix: the tiled product over the row-major matrix then
 // runs in one round with 64 KB of the matrix on their way into each CU. Streamed to tiled, cold matrices, 17 / 64 rows, us:
-// 896 -> 2 x 4,864 9.0 / 11.9 to 6.9 / 8.1; 2,048 -> 2 x 5,632 14.4 / 20.8 to 13.0 / 14.2; 3,072 -> 2 x 8,192 (256 tiles)
+// 896 -> 2 x 4,864 9.0 / 11.9 to 7.4 / 7.7; 2,048 -> 2 x 5,632 14.4 / 20.8 to 13.0 / 14.2; 3,072 -> 2 x 8,192 (256 tiles)
 // 22.7 / 34.6 to 20.4 / 21.5; beyond a tile a CU 1,536 -> 2 x 8,960 16.2 / 19.4 to 15.9 / 22.8, 3,584 -> 2 x 18,944 48.4 / 52.9
 // to 62.1 / 66.6.
 constexpr int TM_TILE_FEW_COLUMNS = 64 * 256;

@@ -1,6 +1,6 @@
-// Matrix products of prompt-sized steps on the bfloat16 matrix unit, each with its layer's own epilogue: C = A W^T (+ bias)
-// stored in bfloat16; gate|up with SiLU*up; q|k|v with bias, rotation and cache write; 32-bit partial sums of a product whose
-// K is split over groups of blocks.
+// Matrix products of prompt-sized steps on the bfloat16 matrix unit, each with its layer's own epilogue: gate|up with SiLU*up;
+// q|k|v with bias, rotation and cache write; 32-bit partial sums of a product A W^T whose K is split over groups of blocks (or is
+// not, one part); the products of experts. The same kernel on the 32-bit matrix unit is the true 32-bit path's.
 //
 // A block of four wavefronts computes a tile of BM rows by BN matrix rows, BM x BN / 4 a wavefront, k in steps of 64. Both
 // operands come straight into LDS (16 bytes a lane, no registers in between) into a ring of ST buffers, ST - 1 to ST steps
@@ -642,7 +642,8 @@ extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void
 // or within 4% of it at ten matrices from 896 x 896 to 5,120 x 27,648, but for long K with columns enough for 128 wide tiles to
 // give three CUs in four a block: those take 64 x 128 tiles, in as many parts (with the norm, 5 / 17 / 32 / 48 / 64 rows, us:
 // 18,944 -> 3,584 64 wide in four parts 29.1 / 29.5 / 30.5 / 32.3 / 34.6, 128 wide in eight 29.4 / 29.8 / 30.3 / 31.2 / 32.1;
-// 27,648 -> 5,120 in three and six 53.6 / 54.0 / 55.2 / 59.2 / 63.1 and 54.0 / 54.5 / 55.8 / 56.8 / 58.3; 13,952 -> 2,048, which
+// 27,648 -> 5,120, which choose.h streams in such steps, in three and six 53.6 / 54.0 / 55.2 / 59.2 / 63.1 and 54.0 / 54.5 / 55.8 / 56.8 /
+// 58.3; 13,952 -> 2,048, which
 // 128 wide tiles would leave half the CUs without, stays at eight parts of 64, 15.8 to 18.3).
 // How K is cut hangs on N and K alone: a row's result does not change with the number of rows.
 constexpr int GT_FEW_ROWS = 64, GT_FEW_RING = 5, GT_FEW_WIDE_RING = 3;
@@ -690,7 +691,7 @@ extern "C" int tm_tile_linear_split(const void* A, int lda, int M, int K, const 
 // every load and read, and small tiles leave the fewest CUs idle in a last round: three blocks a CU, one shape (gate|up of 1,000 /
 // 4,096 rows 154 / 537 us; two blocks a CU 159 / 566, 128 x 64 160 / 523, 64 x 128 160 / 524, 128 x 128 189 / 562; 111 / 455 at the
 // unit's peak). Against the kernel of gemm_f32_mfma.hip (16 k at a time through registers), 0.5B shape, 1,000 rows, in us a layer:
-// gate|up with SiLU*up 192 to 154, q|k|v with rotation 50 to 33, o and down 197 to 92.
+// gate|up with SiLU*up 192 to 154, q|k|v with rotation 50 to 33, o and down 197 to 88.
 
 #define GT_F32 float, EPI, 1, 4, 4, 1, 3, 3
 constexpr int GT_F32_TILE = 64, GT_F32_STEP = 32, GT_F32_RING = 3;

@@ -94,9 +94,9 @@ bool stream_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype, int 
 }
 
 // the products of prompt-sized steps with their epilogues (gemm_tile.hip), over the row-major matrix: beyond the rows of the
-// kernels for few rows (the rules for steps of up to 64 tokens stand in choose.h). Against the library's product and the kernel behind it, in us a layer: gate|up with SiLU*up, 0.5B
-// shape, 77 / 512 / 2,048 rows 16.4 / 22.2 / 65.0 to 6.9 / 13.2 / 35-40; 7B shape, 3,001 rows 724 to 590; q|k|v with rotation
-// and cache write, 0.5B shape 14.3 / 15.0 / 20.1 to 5.7 / 6.5 / 12.7.
+// kernels for few rows (the rules for steps of up to 64 tokens stand in choose.h). Against the library's product and the kernel
+// behind it, in us a layer of a step: gate|up with SiLU*up, 0.5B shape, 77 / 512 / 2,048 rows 16.4 / 22.2 / 65.0 to 7.1 / 14.3 / 39-43;
+// 7B shape, 3,001 rows 724 to 595; q|k|v with rotation and cache write, 0.5B shape 14.3 / 15.0 / 20.1 to 5.7 / 6.5 / 12.7.
 bool tile_ok(const TmLinear& L, const void* x, int ldx, int M, int dtype, int beyond = TM_SKINNY_ROWS) {
     return dtype == TM_BF16 && L.dtype == TM_BF16 && !L.act && M > beyond && tm_gemm_tile_takes(x, ldx, L.w, M, L.N, L.K);
 }
