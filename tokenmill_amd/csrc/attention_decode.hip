@@ -147,8 +147,8 @@ __device__ __forceinline__ void attend_keys64(const Keys64<D>& kv, const Bf16x8B
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) m = fmaxf(m, sc[t][i]);
-    m = fmaxf(m, __shfl_xor(m, 16, TM_WAVE));
-    m = fmaxf(m, __shfl_xor(m, 32, TM_WAVE));
+    m = lane_max<16>(m);
+    m = lane_max<32>(m);
     const float neg_m = (m == -INFINITY) ? 0.f : -m;
     l = 0.f;
     float pr[4][4];
@@ -159,8 +159,8 @@ __device__ __forceinline__ void attend_keys64(const Keys64<D>& kv, const Bf16x8B
             pr[t][i] = __builtin_amdgcn_exp2f(sc[t][i] + neg_m);
             l += pr[t][i];
         }
-    l += __shfl_xor(l, 16, TM_WAVE);
-    l += __shfl_xor(l, 32, TM_WAVE);
+    l = lane_sum<16>(l);
+    l = lane_sum<32>(l);
     // O^T[d][head] = V^T[d][keys] P^T[keys][head], 32 keys (tiles 2b, 2b+1) per instruction
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};

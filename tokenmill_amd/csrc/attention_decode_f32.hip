@@ -85,8 +85,8 @@ __global__ __launch_bounds__(64 * DF_WAVES) void attn_decode_f32_kernel(const fl
                     for (int c = 0; c < NDT; ++c) vf[b][c][i] = 0.f;
             }
         }
-        m = fmaxf(m, __shfl_xor(m, 16, TM_WAVE));
-        m = fmaxf(m, __shfl_xor(m, 32, TM_WAVE));
+        m = lane_max<16>(m);
+        m = lane_max<32>(m);
         const float ref = m == -INFINITY ? 0.f : m;                         // (a wavefront whose keys nobody sees: weights of zero)
         float l = 0.f;
         f32x4_t o[NDT];
@@ -105,8 +105,8 @@ __global__ __launch_bounds__(64 * DF_WAVES) void attn_decode_f32_kernel(const fl
 #pragma unroll
                 for (int c = 0; c < NDT; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][c][i], pr[i], o[c], 0, 0, 0);
         }
-        l += __shfl_xor(l, 16, TM_WAVE);
-        l += __shfl_xor(l, 32, TM_WAVE);
+        l = lane_sum<16>(l);
+        l = lane_sum<32>(l);
         __syncthreads();                                                // (the sums of the chunk before have been read)
         if (g == 0) {
             m_s[wave][r] = m;

@@ -282,8 +282,8 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
         for (int hh = 0; hh < HPW; ++hh) {
             if (hh >= nh) continue;                                  // block-uniform
             float lsum = st.l[hh];
-            lsum += __shfl_xor(lsum, 16, TM_WAVE);
-            lsum += __shfl_xor(lsum, 32, TM_WAVE);
+            lsum = lane_sum<16>(lsum);
+            lsum = lane_sum<32>(lsum);
             // a gate per channel: this thread's pieces, on their way while the partials meet
             constexpr int GP = (16 * (D / 2) + 64 * KS - 1) / (64 * KS);
             uint32_t gv[GP];

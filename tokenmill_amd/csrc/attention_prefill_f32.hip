@@ -109,8 +109,8 @@ __global__ __launch_bounds__(64 * AF_SPLIT) void attn_prefill_f32_kernel(
             }
         }
         float bm = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-        bm = fmaxf(bm, __shfl_xor(bm, 16, TM_WAVE));
-        bm = fmaxf(bm, __shfl_xor(bm, 32, TM_WAVE));
+        bm = lane_max<16>(bm);
+        bm = lane_max<32>(bm);
         const float m_new = fmaxf(m, bm);
         // a column that has seen no key yet keeps m = -inf; its weights and its correction are zeros
         // (every lane stays in step: the matrix instructions below are wave-wide)
@@ -133,8 +133,8 @@ __global__ __launch_bounds__(64 * AF_SPLIT) void attn_prefill_f32_kernel(
         }
     }
     // o[dt][i] = sum for d = 16 dt + 4 g + i of token r; the column's sum is spread over its four lanes
-    l += __shfl_xor(l, 16, TM_WAVE);
-    l += __shfl_xor(l, 32, TM_WAVE);
+    l = lane_sum<16>(l);
+    l = lane_sum<32>(l);
     // the four wavefronts' partial results meet in LDS; a wavefront that had no key block brings m = -inf, l = 0, o = 0
     __shared__ float m_s[AF_SPLIT][16], l_s[AF_SPLIT][16];
     __shared__ __attribute__((aligned(16))) float o_s[AF_SPLIT][16][D + 4];

@@ -308,8 +308,8 @@ __global__ __launch_bounds__(64 * WAVES, SharedPlan<D>::WAVES_PER_SIMD) void att
         for (int hh = 0; hh < HPW; ++hh) {
             if (hh >= nh) continue;                                  // wave-uniform
             float lsum = st.l[hh];
-            lsum += __shfl_xor(lsum, 16, TM_WAVE);
-            lsum += __shfl_xor(lsum, 32, TM_WAVE);
+            lsum = lane_sum<16>(lsum);
+            lsum = lane_sum<32>(lsum);
             if (r >= valid) continue;
             if (sink) lsum += __builtin_amdgcn_exp2f(sink[h0 + hh] * 1.4426950408889634f - st.m[hh]);      // a term of the denominator without a key
             const float inv = 1.f / lsum;

@@ -23,12 +23,10 @@ __device__ __forceinline__ float bf16_to_f32(bf16_t v) {
     return __uint_as_float(((uint32_t)v) << 16);
 }
 
-// round to nearest even; NaN stays NaN
+// round to nearest even; NaN stays NaN (the conversion instruction: one in place of the seven of integer arithmetic that gave the
+// same bits, which the norms and epilogues of small steps waited for one after the other)
 __device__ __forceinline__ bf16_t f32_to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (bf16_t)((u >> 16) | 0x0040u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (bf16_t)(u >> 16);
+    return __builtin_bit_cast(bf16_t, (__bf16)f);
 }
 
 template <typename T> struct Elem;
@@ -89,16 +87,51 @@ __device__ __forceinline__ float tanh_fast(float x) {
     return 1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * 2.8853900817779268f) + 1.f);
 }
 
+// Exchanges between the lanes of a wavefront by instructions of the vector unit (row permutations, swaps of rows and of halves)
+// in place of __shfl_xor, which goes through LDS: a butterfly of six steps takes some 60 cycles, by LDS some 700, and in
+// kernels of a few microseconds nothing else runs meanwhile. Every lane of a group that exchanges has to be active.
+//
+// lane_sum<OFF>(v): v + (v of lane ^ OFF); lane_max likewise. The same values meet as by __shfl_xor, so the same bits.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int OFF>
+__device__ __forceinline__ void lane_pair(float v, float& a, float& b) {       // {a, b} = {v, v of lane ^ OFF}, in either order
+    static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8 || OFF == 16 || OFF == 32, "a power of two below 64");
+    if constexpr (OFF == 32) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        a = __uint_as_float(p[0]), b = __uint_as_float(p[1]);
+    } else if constexpr (OFF == 16) {
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        a = __uint_as_float(p[0]), b = __uint_as_float(p[1]);
+    } else {
+        a = v;
+        if constexpr (OFF == 8) b = dpp_move<0x128>(v);                         // row_ror:8
+        else if constexpr (OFF == 4) b = dpp_move<0x1b>(dpp_move<0x141>(v));    // row_half_mirror, then quad_perm [3,2,1,0]
+        else if constexpr (OFF == 2) b = dpp_move<0x4e>(v);                     // quad_perm [2,3,0,1]
+        else b = dpp_move<0xb1>(v);                                             // quad_perm [1,0,3,2]
+    }
+}
+template <int OFF>
+__device__ __forceinline__ float lane_sum(float v) {
+    float a, b;
+    lane_pair<OFF>(v, a, b);
+    return a + b;
+}
+template <int OFF>
+__device__ __forceinline__ float lane_max(float v) {
+    float a, b;
+    lane_pair<OFF>(v, a, b);
+    return fmaxf(a, b);
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = TM_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, TM_WAVE);
-    return v;
+    return lane_sum<1>(lane_sum<2>(lane_sum<4>(lane_sum<8>(lane_sum<16>(lane_sum<32>(v))))));
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = TM_WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, TM_WAVE));
-    return v;
+    return lane_max<1>(lane_max<2>(lane_max<4>(lane_max<8>(lane_max<16>(lane_max<32>(v))))));
 }
 
 // Sum over a block of NT threads (NT a multiple of 64, at most 1024). Every thread gets the result.

@@ -156,8 +156,8 @@ __global__ __launch_bounds__(64 * WAVES) void attn_latent_mfma_kernel(
                 sv[t][i] = v;
                 mx = fmaxf(mx, v);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, TM_WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, TM_WAVE));
+        mx = lane_max<16>(mx);
+        mx = lane_max<32>(mx);
         const float m_new = fmaxf(m, mx);
         const float ref = m_new == -INFINITY ? 0.f : m_new;               // no row seen yet: every weight is zero
         const float alpha = __builtin_amdgcn_exp2f(m - ref);
@@ -187,8 +187,8 @@ __global__ __launch_bounds__(64 * WAVES) void attn_latent_mfma_kernel(
     }
     if (!tile_ok) return;
     float total = l;
-    total += __shfl_xor(total, 16, TM_WAVE);
-    total += __shfl_xor(total, 32, TM_WAVE);
+    total = lane_sum<16>(total);
+    total = lane_sum<32>(total);
     if (!pair_ok) return;
     if (part_o) {                                                         // a chunk's share: as it is, with its maximum and sum
         const size_t at = ((size_t)(row0 - first_single) * H + head) * n_chunks + blockIdx.y;
