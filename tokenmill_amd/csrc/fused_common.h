@@ -8,6 +8,7 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 union FFrag {
     u32x4_t u;
@@ -21,6 +22,13 @@ __device__ __forceinline__ uint32_t fd_pack(float a, float b) {
 
 __device__ __forceinline__ float fd_round(float a) { return bf16_to_f32(f32_to_bf16(a)); }
 
+__device__ __forceinline__ f32x4_t as_f32x4(const u32x4_t u) { return __builtin_bit_cast(f32x4_t, u); }
+
+// A buffer of `bytes` at `base` (the same in every lane): loads beyond it read as zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t fd_buffer(const void* base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
+
 #define FD_EPI_QKV 0
 #define FD_EPI_SILU 1
 #define FD_KCH 8            // k-steps of one register group of matrix loads, per wavefront (one group in all)
@@ -30,6 +38,12 @@ __device__ __forceinline__ float fd_round(float a) { return bf16_to_f32(f32_to_b
 
 // rows of x a block keeps in LDS for M tokens
 __host__ __device__ __forceinline__ int fused_rows(int M) { return M <= 4 ? 4 : (M <= 8 ? 8 : 16); }
+
+// 4-element vectors a thread holds where one round of loads covers a row: rows of up to 1,024 in 4 or 8 rows of x
+__host__ __device__ constexpr int fused_row_vectors(int threads) { return 2048 / threads; }
+
+// Elements between the rows of x in LDS: whole k-steps (zeros beyond K) and the padding.
+__host__ __device__ __forceinline__ int fused_x_stride(int K) { return (K + 31) / 32 * 32 + FD_XPAD; }
 
 struct FusedArgs {
     // norm + product

@@ -17,209 +17,196 @@
 #include "api.h"
 #include "fused_common.h"
 
-// ROWS: rows of a strip (16 or 8). Short strips leave rows of the MFMA tile empty (their lanes load
-// nothing) and double the number of units, for matrices that would otherwise give fewer blocks
-// than the chip has CUs. A block takes the units u = blockIdx.x, + gridDim.x, ...: the norm is
-// computed once and serves all of them.
+// ROWS: rows of a strip (16 or 8). Short strips leave rows of the MFMA tile empty (their lanes load what the others load)
+// and double the number of units, for matrices that would otherwise give fewer blocks than the chip has CUs.
+// WAVES: wavefronts that split the K of a unit (4, or 8 for a long K). UNITS: units a block multiplies at once, each by WAVES
+// wavefronts of its own; with more units than that times the grid a block goes on to the next ones, after one norm for all.
 // PIPE: a wavefront's K range is longer than one group of FD_KCH steps, and two register groups take
 // turns so that loads are always in flight (more registers; not worth them when one group holds it all).
-// WAVES: wavefronts of a block (4, or 8 for a long K: they split K, and the norm's rows, between them).
-template <int EPI, int ROWS, bool PIPE, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void fused_norm_gemm_kernel(const FusedArgs a,
-                                                                                        const int n_units) {
+//
+// These launches are bound by the trips to memory that wait for each other and by what runs between them, not by bytes: marks of
+// the clock inside the kernel showed 0.5 us for the positions (by scalar loads) before the first vector load, the residual rows
+// waited for BEHIND the matrix that was asked for first (loads come back in their order), and 1.2 us for the norm itself, of
+// which the sum's exchange through LDS was half. So everything that hangs on nothing is asked for at once, in the order it is
+// needed: positions and slots, residual rows, norm weights, the matrix, the bias; the rotary rows as soon as the positions are
+// there; the norm runs while the matrix is on its way. Loads are unconditional: what lies beyond a row, a strip or a wavefront's
+// range of k reads as zero by the bounds of its buffer descriptor.
+//
+// PLAIN: the norm's weights are bfloat16 and the threads that share a row hold all of it in one round of loads (launch_fused_shape):
+// straight code from the loads to LDS. The other way takes any K and either type.
+template <int EPI, int ROWS, bool PIPE, int WAVES, int UNITS, bool PLAIN>
+__global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) void fused_norm_gemm_kernel(const FusedArgs a,
+                                                                                                       const int n_units) {
     constexpr int KCH = PIPE ? FD_KCH_PIPE : FD_KCH;
-    constexpr int THREADS = 64 * WAVES;
+    constexpr int THREADS = 64 * WAVES * UNITS, RC = PLAIN ? fused_row_vectors(THREADS) : FD_RC;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    bf16_t* xs = (bf16_t*)smem_raw;                                  // [4, 8 or 16 rows][K + FD_XPAD]
-    __shared__ float red[WAVES][2][64][4 + 1];
+    bf16_t* xs = (bf16_t*)smem_raw;                                  // [4, 8 or 16 rows][fused_x_stride]
+    __shared__ f32x4_t red[UNITS][WAVES][2][64];
     const int K = a.K, M = a.M;
-    const int xstride = K + FD_XPAD;
-    const int wave = threadIdx.x / TM_WAVE, lane = threadIdx.x % TM_WAVE;
-    const int r = lane % 16, g = lane / 16;
-
-    auto unit_of = [&](int u) { return fused_unit_of<EPI, ROWS>(a, u, r); };
-
     const int ksteps = (K + 31) / 32;
     const int per = (ksteps + WAVES - 1) / WAVES;
+    const int xstride = fused_x_stride(K);
+    const int block_wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;
+    const int slot_of_block = block_wave / WAVES, wave = block_wave % WAVES;      // which of the block's units, which part of its K
+    const int r = lane % 16, g = lane / 16;
     const int ks0 = wave * per;
     const int ks1 = ks0 + per < ksteps ? ks0 + per : ksteps;
-    int u = blockIdx.x;
-    FusedUnit cu = unit_of(u);
+
     // The matrix comes in strip order: the 16-byte piece of lane (r, g) for k-step ks of strip s lies at
     // ((s * ksteps + ks) * 4 + g) * ROWS + r pieces, so a wavefront's load is one run of ROWS * 64 bytes
     // and a strip is one run of memory; rows and k beyond the matrix are zeros there.
     constexpr int FRAG = 32 * ROWS;                                  // bfloat16 values of a (strip, k-step)
-    const int lane_off = (g * ROWS + (r < ROWS ? r : 0)) * 8;
-    auto strip_pointer = [&](int strip) { return a.W + (size_t)strip * ksteps * FRAG + lane_off; };
-    const bf16_t* wA = strip_pointer(cu.sA);
-    const bf16_t* wB = strip_pointer(cu.sB);
-    auto load_group = [&](auto& ga, auto& gb, int base, bool rows_ok) {
+    const int lane_off = (g * ROWS + (r < ROWS ? r : 0)) * 16;
+    FusedUnit cu;
+    __amdgpu_buffer_rsrc_t wA, wB;                                   // this wavefront's strips, up to the end of its k
+    auto take_unit = [&](int u) {
+        const bool live = u < n_units;                               // (the same in every lane)
+        cu = fused_unit_of<EPI, ROWS>(a, live ? u : 0, r);
+        const int bytes = live && ks1 > ks0 ? ks1 * FRAG * 2 : 0;
+        wA = fd_buffer(a.W + (size_t)cu.sA * ksteps * FRAG, bytes);
+        wB = fd_buffer(a.W + (size_t)cu.sB * ksteps * FRAG, bytes);
+    };
+    auto load_group = [&](auto& ga, auto& gb, int base) {
 #pragma unroll
         for (int j = 0; j < KCH; ++j) {
-            const bool in = rows_ok && base + j < ks1;
-            ga[j].u = in ? *(const u32x4_t*)(wA + (size_t)(base + j) * FRAG) : u32x4_t{0, 0, 0, 0};
-            gb[j].u = in ? *(const u32x4_t*)(wB + (size_t)(base + j) * FRAG) : u32x4_t{0, 0, 0, 0};
+            const int at = lane_off + (base + j) * (FRAG * 2);
+            ga[j].u = __builtin_amdgcn_raw_buffer_load_b128(wA, at, 0, 0);
+            gb[j].u = __builtin_amdgcn_raw_buffer_load_b128(wB, at, 0, 0);
         }
     };
-    // What the epilogue will need from memory is asked for long before it is used, and in an order
-    // that lets the long loads go first in effect: loads come back in the order they were issued, so
-    // the token's position and cache slot (a few bytes from the cache, and the rotary row's address
-    // hangs on the position) are asked for BEFORE the matrix, and can be waited for while the matrix
-    // is still on its way; the bias and the rotary row follow the matrix and are not looked at (not
-    // even widened) until the epilogue.
+
+    // --- everything that hangs on nothing, in the order it is needed ---
     const int tok = r;                                               // the epilogue's token of this lane
     const bool epi_lane = wave == 0 && tok < M && 4 * g < ROWS;
-    // The positions are read at addresses that are the same in every lane, which makes them scalar
-    // loads: those are counted apart from the vector loads, so waiting for them does not wait for the
-    // matrix. Each lane then picks its token's.
-    int tok_pos = 0;
+    int tok_pos = 0, tok_slot = 0;
     if constexpr (EPI == FD_EPI_QKV) {
+        const int t = tok < M ? tok : 0;
+        tok_pos = a.positions[t];
+        tok_slot = (a.slots ? a.slots : a.positions)[t];
+    }
+    // A row of the residual stream is shared by tpr threads of one wavefront (256 threads: 16 rows x 16 threads, 8 x 32, or 4 x 64);
+    // each keeps its first RC vectors in registers between the two passes. Rows beyond M are the last one again, for
+    // tokens that do not exist.
+    constexpr int LOG_THREADS = THREADS == 256 ? 8 : 9;
+    static_assert(THREADS == 1 << LOG_THREADS, "4 or 8 wavefronts");
+    const int mpad = fused_rows(M);
+    const int tshift = LOG_THREADS - (mpad == 4 ? 2 : mpad == 8 ? 3 : 4) < 6 ? LOG_THREADS - (mpad == 4 ? 2 : mpad == 8 ? 3 : 4) : 6;
+    const int tpr = 1 << tshift;
+    const int row = threadIdx.x >> tshift, sub = threadIdx.x & (tpr - 1);
+    const int step = 4 * tpr;
+    const __amdgpu_buffer_rsrc_t rbuf = fd_buffer(a.resid, M * K * 4);
+    const __amdgpu_buffer_rsrc_t nbuf = fd_buffer(a.norm_w, a.norm_w_f32 ? 0 : K * 2);
+    const int row0 = (row < M ? row : M - 1) * K;
+    auto resid_at = [&](int c) {                                     // (beyond the row: a place beyond the buffer)
+        return as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(rbuf, c < K ? (row0 + c) * 4 : 0x7ffffff0, 0, 0));
+    };
+    f32x4_t cache[RC];
+    u32x2_t wraw[RC];                                                // bfloat16 weights of the norm
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int pos_i = a.positions[i < M ? i : 0];
-            tok_pos = tok == i ? pos_i : tok_pos;
-        }
+    for (int j = 0; j < RC; ++j) cache[j] = resid_at(sub * 4 + j * step);
+    if constexpr (PLAIN) {
+#pragma unroll
+        for (int j = 0; j < RC; ++j) wraw[j] = __builtin_amdgcn_raw_buffer_load_b64(nbuf, (sub * 4 + j * step) * 2, 0, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
-    // matrix loads of the first group go out before the norm is computed
     FFrag fa[KCH], fb[KCH], fa2[PIPE ? KCH : 1], fb2[PIPE ? KCH : 1];
-    load_group(fa, fb, ks0, cu.rows_ok);
-    if constexpr (PIPE) load_group(fa2, fb2, ks0 + KCH, cu.rows_ok);
+    int u0 = blockIdx.x;
+    take_unit(u0 + slot_of_block * gridDim.x);
+    load_group(fa, fb, ks0);
+    if constexpr (PIPE) load_group(fa2, fb2, ks0 + KCH);
     __builtin_amdgcn_sched_barrier(0);
 
     struct EpilogueInputs {
-        union {
-            f32x4_t f;              // four rows of a strip as loaded: a 32-bit bias, or
-            uint2 h;                // a bfloat16 one (only the kind there is gets loaded and read)
-        } bias[2];
+        f32x4_t bias_f[2];          // four rows of a strip as loaded: a 32-bit bias, or
+        u32x2_t bias_h[2];          // a bfloat16 one
         f32x4_t cos, sin;
-        int slot;                   // (every lane loads, the lanes without a token from entry 0; what came is
-    };                              // looked at only where it is meant: a load under a test is waited for where the test ends)
+    };
     const int bias_kind = !a.bias ? 0 : (a.bias_f32 ? 2 : 1);       // the same for every lane
-    auto epilogue_inputs = [&](const FusedUnit& t) {
-        EpilogueInputs e;
+    auto epilogue_inputs = [&]() {
+        EpilogueInputs e{};
         if constexpr (EPI == FD_EPI_QKV) {
             // lanes beyond the strip's rows (4 g >= ROWS) have no epilogue: they read what group 0 reads
             const int ge = 4 * g < ROWS ? 4 * g : 0;
-            const int ia = t.nA + ge, ib = t.nB + ge;               // (the bias is 16-byte aligned)
-            if (bias_kind == 2) {
-                e.bias[0].f = *(const f32x4_t*)((const float*)a.bias + ia);
-                e.bias[1].f = *(const f32x4_t*)((const float*)a.bias + ib);
-            } else if (bias_kind == 1) {
-                e.bias[0].h = *(const uint2*)((const bf16_t*)a.bias + ia);
-                e.bias[1].h = *(const uint2*)((const bf16_t*)a.bias + ib);
-            }
+            const int ia = cu.nA + ge, ib = cu.nB + ge;             // (the bias is 16-byte aligned)
+            const int width = (a.H + 2 * a.KVH) * a.D;
+            const __amdgpu_buffer_rsrc_t bf = fd_buffer(a.bias, bias_kind == 2 ? width * 4 : 0), bh = fd_buffer(a.bias, bias_kind == 1 ? width * 2 : 0);
+            e.bias_f[0] = as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(bf, ia * 4, 0, 0));
+            e.bias_f[1] = as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(bf, ib * 4, 0, 0));
+            e.bias_h[0] = __builtin_amdgcn_raw_buffer_load_b64(bh, ia * 2, 0, 0);
+            e.bias_h[1] = __builtin_amdgcn_raw_buffer_load_b64(bh, ib * 2, 0, 0);
             // value heads have no rotary row: they read that of the first pair and do not use it
-            const int jt = t.head < a.H + a.KVH ? t.jt : 0;
-            const size_t at = (size_t)tok_pos * (a.D / 2) + ROWS * jt + (4 * g < ROWS ? 4 * g : 0);
+            const int jt = cu.head < a.H + a.KVH ? cu.jt : 0;
+            const size_t at = (size_t)tok_pos * (a.D / 2) + ROWS * jt + ge;
             e.cos = *(const f32x4_t*)(a.cos_t + at);
             e.sin = *(const f32x4_t*)(a.sin_t + at);
-            e.slot = (a.slots ? a.slots : a.positions)[tok < M ? tok : 0];
         }
         return e;
     };
-    EpilogueInputs e_next = epilogue_inputs(cu);
 
-    // x = norm(resid) into LDS. A row is shared by TPR threads of one wavefront (256 threads: 16 rows x 16
-    // threads, 8 x 32, or 4 x 64); each keeps its first FD_RC vectors in registers between the two passes.
-    const int mpad = fused_rows(M);
-    {
-        const int tpr = THREADS / mpad < TM_WAVE ? THREADS / mpad : TM_WAVE;
-        const int row = threadIdx.x / tpr, sub = threadIdx.x % tpr;
+    // --- x = norm(resid) into LDS, while the matrix is on its way ---
+    EpilogueInputs e_next;
+    if (row < mpad) {                                                // (the same in every lane of a wavefront)
         bf16_t* xrow = xs + (size_t)row * xstride;
-        const int step = 4 * tpr;
-        if (row < M) {
-            const float* src = a.resid + (size_t)row * K;
-            // The norm's weights of the first group are asked for with the row itself: they depend on
-            // nothing, and asked for after the sum of squares they would cost a trip to memory of their
-            // own. (Two kinds of loads behind one run-time test would each be waited for singly: the
-            // test on the weights' type stands outside the loops.)
-            const bool w16 = !a.norm_w_f32;
-            auto widen = [](const uint2 wv) {
-                return f32x4_t{__uint_as_float(wv.x << 16), __uint_as_float(wv.x & 0xffff0000u),
-                               __uint_as_float(wv.y << 16), __uint_as_float(wv.y & 0xffff0000u)};
-            };
-            uint2 wraw[FD_RC];
-            if (w16) {
+        auto squares = [](const f32x4_t v) { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3]; };
+        float ss = 0.f;
 #pragma unroll
-                for (int j = 0; j < FD_RC; ++j) {
-                    const int c = sub * 4 + j * step;
-                    wraw[j] = c < K ? *(const uint2*)((const bf16_t*)a.norm_w + c) : uint2{0u, 0u};
-                }
-            }
-            f32x4_t cache[FD_RC];
-            float ss = 0.f;
+        for (int j = 0; j < RC; ++j) ss += squares(cache[j]);
+        __builtin_amdgcn_sched_barrier(0);
+        e_next = epilogue_inputs();                                  // (the positions came before the rows)
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!PLAIN) {
+            // the rest of a long row in groups of RC loads that are in flight together
+            for (int c0 = sub * 4 + RC * step; c0 - sub * 4 < K; c0 += RC * step) {
+                f32x4_t v[RC];
 #pragma unroll
-            for (int j = 0; j < FD_RC; ++j) {
-                const int c = sub * 4 + j * step;
-                cache[j] = c < K ? *(const f32x4_t*)(src + c) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-                ss += cache[j][0] * cache[j][0] + cache[j][1] * cache[j][1] + cache[j][2] * cache[j][2] +
-                      cache[j][3] * cache[j][3];
-            }
-            // the rest of a long row in groups of FD_RC loads that are in flight together
-            for (int c0 = sub * 4 + FD_RC * step; c0 < K; c0 += FD_RC * step) {
-                f32x4_t v[FD_RC];
+                for (int j = 0; j < RC; ++j) v[j] = resid_at(c0 + j * step);
 #pragma unroll
-                for (int j = 0; j < FD_RC; ++j)
-                    v[j] = c0 + j * step < K ? *(const f32x4_t*)(src + c0 + j * step) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int j = 0; j < FD_RC; ++j)
-                    ss += v[j][0] * v[j][0] + v[j][1] * v[j][1] + v[j][2] * v[j][2] + v[j][3] * v[j][3];
-            }
-            for (int off = 1; off < tpr; off <<= 1) ss += __shfl_xor(ss, off, TM_WAVE);
-            const float rs = rsqrtf(ss / (float)K + a.eps);
-            auto emit = [&](int c, const f32x4_t v, const f32x4_t w) {
-                uint2 pk;
-                pk.x = fd_pack(w[0] * fd_round(v[0] * rs), w[1] * fd_round(v[1] * rs));
-                pk.y = fd_pack(w[2] * fd_round(v[2] * rs), w[3] * fd_round(v[3] * rs));
-                *(uint2*)(xrow + c) = pk;
-            };
-            {
-                f32x4_t w[FD_RC];
-                if (w16) {
-#pragma unroll
-                    for (int j = 0; j < FD_RC; ++j) w[j] = widen(wraw[j]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < FD_RC; ++j) {
-                        const int c = sub * 4 + j * step;
-                        w[j] = c < K ? *(const f32x4_t*)((const float*)a.norm_w + c) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < FD_RC; ++j) {
-                    const int c = sub * 4 + j * step;
-                    if (c < K) emit(c, cache[j], w[j]);
-                }
-            }
-            // the rest of a long row: the values again and their weights, a group in flight together
-            for (int c0 = sub * 4 + FD_RC * step; c0 < K; c0 += FD_RC * step) {
-                f32x4_t v[FD_RC], w[FD_RC];
-                if (w16) {
-                    uint2 raw[FD_RC];
-#pragma unroll
-                    for (int j = 0; j < FD_RC; ++j) {
-                        const bool in = c0 + j * step < K;
-                        v[j] = in ? *(const f32x4_t*)(src + c0 + j * step) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-                        raw[j] = in ? *(const uint2*)((const bf16_t*)a.norm_w + c0 + j * step) : uint2{0u, 0u};
-                    }
-#pragma unroll
-                    for (int j = 0; j < FD_RC; ++j) w[j] = widen(raw[j]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < FD_RC; ++j) {
-                        const bool in = c0 + j * step < K;
-                        v[j] = in ? *(const f32x4_t*)(src + c0 + j * step) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-                        w[j] = in ? *(const f32x4_t*)((const float*)a.norm_w + c0 + j * step) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < FD_RC; ++j)
-                    if (c0 + j * step < K) emit(c0 + j * step, v[j], w[j]);
+                for (int j = 0; j < RC; ++j) ss += squares(v[j]);
             }
         }
-        // rows M..mpad-1 of x stay as they are, and the lanes of tokens beyond mpad read rows below it
-        // again: they only feed result columns of tokens that do not exist, which no lane stores
+        ss = lane_sum<8>(lane_sum<4>(lane_sum<2>(lane_sum<1>(ss))));
+        if (tpr >= 32) ss = lane_sum<16>(ss);
+        if (tpr >= 64) ss = lane_sum<32>(ss);
+        const float rs = rsqrtf(ss / (float)K + a.eps);
+        auto emit = [&](int c, const f32x4_t v, const f32x4_t w) {
+            uint2 pk;
+            pk.x = fd_pack(w[0] * fd_round(v[0] * rs), w[1] * fd_round(v[1] * rs));
+            pk.y = fd_pack(w[2] * fd_round(v[2] * rs), w[3] * fd_round(v[3] * rs));
+            *(uint2*)(xrow + (c < K ? c : xstride - 4)) = pk;         // (what lies beyond the row: into the padding, which nobody reads)
+        };
+        auto widen = [](const u32x2_t wv) {
+            return f32x4_t{__uint_as_float(wv.x << 16), __uint_as_float(wv.x & 0xffff0000u),
+                           __uint_as_float(wv.y << 16), __uint_as_float(wv.y & 0xffff0000u)};
+        };
+        if constexpr (PLAIN) {
+#pragma unroll
+            for (int j = 0; j < RC; ++j) emit(sub * 4 + j * step, cache[j], widen(wraw[j]));
+        } else {
+            // groups of values (the first from the registers, the others read again) and their weights
+            const __amdgpu_buffer_rsrc_t wbuf = fd_buffer(a.norm_w, a.norm_w_f32 ? K * 4 : 0);
+            for (int c0 = sub * 4; c0 - sub * 4 < K; c0 += RC * step) {
+                f32x4_t w[RC];
+                if (a.norm_w_f32) {
+#pragma unroll
+                    for (int j = 0; j < RC; ++j)
+                        w[j] = as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(wbuf, c0 + j * step < K ? (c0 + j * step) * 4 : 0x7ffffff0, 0, 0));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < RC; ++j) wraw[j] = __builtin_amdgcn_raw_buffer_load_b64(nbuf, (c0 + j * step) * 2, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < RC; ++j) w[j] = widen(wraw[j]);
+                }
+                if (c0 != sub * 4) {
+#pragma unroll
+                    for (int j = 0; j < RC; ++j) cache[j] = resid_at(c0 + j * step);
+                }
+#pragma unroll
+                for (int j = 0; j < RC; ++j) emit(c0 + j * step, cache[j], w[j]);
+            }
+        }
+        for (int c = K + sub; c < xstride - FD_XPAD; c += tpr) xrow[c] = 0;      // whole k-steps
+    } else {
+        e_next = epilogue_inputs();
     }
     __syncthreads();
 
@@ -227,10 +214,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void fused_norm_gem
     f32x4_t accA, accB;
     auto multiply_group = [&](const auto& ga, const auto& gb, int base) {
 #pragma unroll
-        for (int j = 0; j < KCH; ++j) {
-            const int k = (base + j) * 32;
+        for (int j = 0; j < KCH; ++j) {                              // (steps beyond ks1: zeros of the matrix)
             FFrag xf;
-            xf.u = (base + j < ks1 && k + 8 * g < K) ? *(const u32x4_t*)(xr + k) : u32x4_t{0, 0, 0, 0};
+            xf.u = *(const u32x4_t*)(xr + (base + j < ksteps ? base + j : 0) * 32);
             accA = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[j].b, xf.b, accA, 0, 0, 0);
             accB = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gb[j].b, xf.b, accB, 0, 0, 0);
         }
@@ -244,49 +230,41 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void fused_norm_gem
             // always in flight while one is multiplied
             for (int base = ks0; base < ks1; base += 2 * KCH) {
                 multiply_group(fa, fb, base);
-                if (base + 2 * KCH < ks1) load_group(fa, fb, base + 2 * KCH, cu.rows_ok);
+                if (base + 2 * KCH < ks1) load_group(fa, fb, base + 2 * KCH);
                 if (base + KCH >= ks1) break;
                 multiply_group(fa2, fb2, base + KCH);
-                if (base + 3 * KCH < ks1) load_group(fa2, fb2, base + 3 * KCH, cu.rows_ok);
+                if (base + 3 * KCH < ks1) load_group(fa2, fb2, base + 3 * KCH);
             }
         } else {
             for (int base = ks0; base < ks1; base += KCH) {
-                if (base != ks0) load_group(fa, fb, base, cu.rows_ok);
+                if (base != ks0) load_group(fa, fb, base);
                 multiply_group(fa, fb, base);
             }
         }
         // partial sums of the wavefronts, added in wavefront order
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            red[wave][0][lane][i] = accA[i];
-            red[wave][1][lane][i] = accB[i];
-        }
+        red[slot_of_block][wave][0][lane] = accA;
+        red[slot_of_block][wave][1][lane] = accB;
         __syncthreads();
 
-        // the next unit's first loads go out before this unit's epilogue
-        const int un = u + gridDim.x;
-        const bool more = un < n_units;
+        // the next units' first loads go out before these units' epilogue
         const FusedUnit done = cu;
+        const bool done_live = u0 + slot_of_block * (int)gridDim.x < n_units;
+        u0 += UNITS * gridDim.x;
+        const bool more = u0 < n_units;
         if (more) {
-            cu = unit_of(un);
-            wA = strip_pointer(cu.sA);
-            wB = strip_pointer(cu.sB);
-            load_group(fa, fb, ks0, cu.rows_ok);
-            if constexpr (PIPE) load_group(fa2, fb2, ks0 + KCH, cu.rows_ok);
-            e_next = epilogue_inputs(cu);
+            take_unit(u0 + slot_of_block * gridDim.x);
+            load_group(fa, fb, ks0);
+            if constexpr (PIPE) load_group(fa2, fb2, ks0 + KCH);
+            e_next = epilogue_inputs();
         }
 
-        if (epi_lane) {
+        if (epi_lane && done_live) {
+            accA = red[slot_of_block][0][0][lane];
+            accB = red[slot_of_block][0][1][lane];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float sa = red[0][0][lane][i], sb = red[0][1][lane][i];
-#pragma unroll
-                for (int w = 1; w < WAVES; ++w) {
-                    sa += red[w][0][lane][i];
-                    sb += red[w][1][lane][i];
-                }
-                accA[i] = sa;
-                accB[i] = sb;
+            for (int w = 1; w < WAVES; ++w) {
+                accA += red[slot_of_block][w][0][lane];
+                accB += red[slot_of_block][w][1][lane];
             }
             // lane: token r, rows nA + 4g + i and nB + 4g + i
             if (EPI == FD_EPI_SILU) {
@@ -308,13 +286,13 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void fused_norm_gem
             } else {
                 f32x4_t bA = {0.f, 0.f, 0.f, 0.f}, bB = {0.f, 0.f, 0.f, 0.f};
                 if (bias_kind == 2) {
-                    bA = e.bias[0].f;
-                    bB = e.bias[1].f;
+                    bA = e.bias_f[0];
+                    bB = e.bias_f[1];
                 } else if (bias_kind == 1) {
-                    bA = f32x4_t{__uint_as_float(e.bias[0].h.x << 16), __uint_as_float(e.bias[0].h.x & 0xffff0000u),
-                                 __uint_as_float(e.bias[0].h.y << 16), __uint_as_float(e.bias[0].h.y & 0xffff0000u)};
-                    bB = f32x4_t{__uint_as_float(e.bias[1].h.x << 16), __uint_as_float(e.bias[1].h.x & 0xffff0000u),
-                                 __uint_as_float(e.bias[1].h.y << 16), __uint_as_float(e.bias[1].h.y & 0xffff0000u)};
+                    bA = f32x4_t{__uint_as_float(e.bias_h[0].x << 16), __uint_as_float(e.bias_h[0].x & 0xffff0000u),
+                                 __uint_as_float(e.bias_h[0].y << 16), __uint_as_float(e.bias_h[0].y & 0xffff0000u)};
+                    bB = f32x4_t{__uint_as_float(e.bias_h[1].x << 16), __uint_as_float(e.bias_h[1].x & 0xffff0000u),
+                                 __uint_as_float(e.bias_h[1].y << 16), __uint_as_float(e.bias_h[1].y & 0xffff0000u)};
                 }
                 float xA[4], xB[4];
 #pragma unroll
@@ -322,7 +300,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void fused_norm_gem
                     xA[i] = fd_round(accA[i] + bA[i]);
                     xB[i] = fd_round(accB[i] + bB[i]);
                 }
-                const int slot = a.slots ? e.slot : -1;
+                const int slot = a.slots ? tok_slot : -1;
                 if (done.head < a.H + a.KVH) {
                     const int half = a.D / 2;
                     const int j0 = ROWS * done.jt + 4 * g;                       // pair index of element 0
@@ -355,39 +333,54 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void fused_norm_gem
         }
         if (!more) break;
         __syncthreads();                                                 // the sums have been read: red is free again
-        u = un;
     }
 }
 
-static int fused_lds_bytes(int M, int K) { return fused_rows(M) * (K + FD_XPAD) * (int)sizeof(bf16_t); }
+// Dynamic LDS of a launch: the normed rows.
+static int fused_lds_bytes(int M, int K) { return fused_rows(M) * fused_x_stride(K) * (int)sizeof(bf16_t); }
 
-template <int EPI, int ROWS, bool PIPE, int WAVES>
-static int launch_fused_shape(const FusedArgs& a, int n_units, int blocks, hipStream_t stream) {
+template <int EPI, int ROWS, bool PIPE, int WAVES, int UNITS, bool PLAIN>
+static int launch_fused_kernel(const FusedArgs& a, int n_units, int blocks, hipStream_t stream) {
     const int lds = fused_lds_bytes(a.M, a.K);
-    if (lds + (int)sizeof(float) * WAVES * 2 * 64 * 5 + 1024 > 160 * 1024) return TM_ERR_ARG;
+    if (lds + (int)sizeof(f32x4_t) * UNITS * WAVES * 2 * 64 + 1024 > 160 * 1024) return TM_ERR_ARG;
     static int raised = 0;          // largest dynamic LDS size this kernel has been allowed so far
     if (lds > 48 * 1024 && lds > raised) {
-        if (hipFuncSetAttribute((const void*)fused_norm_gemm_kernel<EPI, ROWS, PIPE, WAVES>,
+        if (hipFuncSetAttribute((const void*)fused_norm_gemm_kernel<EPI, ROWS, PIPE, WAVES, UNITS, PLAIN>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
             return TM_ERR_LAUNCH;
         raised = lds;
     }
-    fused_norm_gemm_kernel<EPI, ROWS, PIPE, WAVES><<<blocks, 64 * WAVES, lds, stream>>>(a, n_units);
+    fused_norm_gemm_kernel<EPI, ROWS, PIPE, WAVES, UNITS, PLAIN><<<blocks, 64 * WAVES * UNITS, lds, stream>>>(a, n_units);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
 
-// A long K gets 8 wavefronts a block (shorter K ranges, a faster norm); whether a wavefront's range
-// needs more than one register group of loads decides the pipelined variant.
+template <int EPI, int ROWS, bool PIPE, int WAVES, int UNITS>
+static int launch_fused_shape(const FusedArgs& a, int n_units, int blocks, hipStream_t stream) {
+    constexpr int THREADS = 64 * WAVES * UNITS;
+    const int share = THREADS / fused_rows(a.M), tpr = share < TM_WAVE ? share : TM_WAVE;
+    if (WAVES == 4 && !a.norm_w_f32 && a.K <= fused_row_vectors(THREADS) * 4 * tpr)
+        return launch_fused_kernel<EPI, ROWS, PIPE, WAVES, UNITS, WAVES == 4>(a, n_units, blocks, stream);
+    return launch_fused_kernel<EPI, ROWS, PIPE, WAVES, UNITS, false>(a, n_units, blocks, stream);
+}
+
+// A long K gets 8 wavefronts a unit (shorter K ranges, a faster norm); whether a wavefront's range
+// needs more than one register group of loads decides the pipelined variant. With a shorter K a block that has several units
+// takes two at a time, so that the second's matrix is on its way with the first's.
 template <int EPI, int ROWS>
 static int launch_fused(const FusedArgs& a, int n_units, int blocks, hipStream_t stream) {
     const int ksteps = (a.K + 31) / 32;
     if (a.K >= 2048) {
-        return (ksteps + 7) / 8 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 8>(a, n_units, blocks, stream)
-                                         : launch_fused_shape<EPI, ROWS, false, 8>(a, n_units, blocks, stream);
+        return (ksteps + 7) / 8 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 8, 1>(a, n_units, blocks, stream)
+                                         : launch_fused_shape<EPI, ROWS, false, 8, 1>(a, n_units, blocks, stream);
     }
-    return (ksteps + 3) / 4 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 4>(a, n_units, blocks, stream)
-                                     : launch_fused_shape<EPI, ROWS, false, 4>(a, n_units, blocks, stream);
+    if constexpr (EPI == FD_EPI_SILU) {
+        if (n_units > blocks)
+            return (ksteps + 3) / 4 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 4, 2>(a, n_units, blocks, stream)
+                                             : launch_fused_shape<EPI, ROWS, false, 4, 2>(a, n_units, blocks, stream);
+    }
+    return (ksteps + 3) / 4 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 4, 1>(a, n_units, blocks, stream)
+                                     : launch_fused_shape<EPI, ROWS, false, 4, 1>(a, n_units, blocks, stream);
 }
 
 static bool fused_common_ok(int M, int K, const void* resid, const void* W) {
