@@ -22,15 +22,9 @@
 // apart (measured on an MI355X: 15% more bytes a second from HBM). Both give the same bits.
 #include "common.h"
 #include "api.h"
+#include "fused_common.h"
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-
-union Frag {
-    u32x4_t u;
-    bf16x8_t b;
-};
+typedef FFrag Frag;
 
 __device__ __forceinline__ Frag load_frag(const bf16_t* row, int k, int K, bool row_ok) {
     Frag f;
@@ -72,23 +66,173 @@ __device__ __forceinline__ float bias_at(const void* bias, int flags, int n) {
     return (flags & SK_BIAS_F32) ? ((const float*)bias)[n] : bf16_to_f32(((const bf16_t*)bias)[n]);
 }
 
+// --- at most 16 tokens, a strip's K split over wavefronts -------------------------------------------------------------------
+// The output and down projections of decode steps. Such a launch waits for memory once and then for the loads of a CU to pass its
+// address unit, 16 cycles an instruction whatever its lanes bring: with a strip of four rows a lane in four brought a part of
+// the matrix and with one token a lane in sixteen a part of the activations, and every load stood under a test of its own (a down
+// projection of 4,864 -> 896: 16 wavefronts of ten and ten loads, 2.1 us of the address unit for 39 KB a block).
+//
+// So an MFMA tile holds several ranges of K at once. The 16 rows of the A operand are the ROWS rows of the strip for each of
+// SA = 16 / ROWS ranges, the 16 columns of the B operand are TOKS tokens for each of SB = 16 / TOKS ranges; what is computed where a
+// range meets itself counts, the rest is dropped. VW is the number of ranges, a wavefront has SA of them and multiplies one
+// load of the matrix by NB = SA / SB loads of activations, each into accumulators of its own. Which k a range has (as many k-steps as
+// every other, in order) and the order in which the VW sums are added are those of gemm_skinny_kernel with VW wavefronts, so the
+// bits are the same for any number of tokens. Loads are unconditional: what lies beyond the strip, a token or a range
+// reads as zero by the bounds of its buffer descriptor.
+template <int ROWS, int TOKS, int VW, int CH, typename TC, bool PACKED>
+__global__ __launch_bounds__(64 * VW * ROWS / 16) void gemm_few_kernel(const bf16_t* __restrict__ A, int lda,
+                                                                       const bf16_t* __restrict__ W,
+                                                                       const void* __restrict__ bias, int flags,
+                                                                       TC* __restrict__ C, int ldc, int M, int N, int K,
+                                                                       float* __restrict__ accum, int ldacc) {
+    constexpr int SA = 16 / ROWS, SB = 16 / TOKS, NB = SA / SB;
+    static_assert(SA >= SB && VW % SA == 0, "whole wavefronts, and no range of the activations without one of the matrix");
+    constexpr int BEYOND = 0x7ffffff0;
+    __shared__ f32x4_t red[VW][ROWS / 4][16];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;
+    const int r = lane % 16, g = lane / 16;
+    const int n0 = blockIdx.x * ROWS;
+    const int ksteps = (K + 31) / 32, per = (ksteps + VW - 1) / VW;
+    const int range0 = wave * SA;                       // this wavefront's first range
+
+    // what the epilogue (wavefront 0: lane = token lane % 16, rows n0 + 4 (lane / 16) + i) reads from memory is asked for first
+    const int tok = r, nf = n0 + 4 * g;
+    const bool epi = wave == 0 && 4 * g < ROWS && tok < M && nf < N;
+    const bool fast = accum && N % 4 == 0 && ldacc % 4 == 0 && ((uintptr_t)accum % 16) == 0;      // the same in every lane
+    f32x4_t current = {0.f, 0.f, 0.f, 0.f}, offset = {0.f, 0.f, 0.f, 0.f};
+    if (wave == 0) {
+        if (fast) current = *(const f32x4_t*)(accum + (epi ? (size_t)tok * ldacc + nf : 0));
+        if (bias) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) offset[i] = bias_at(bias, flags, nf + i < N ? nf + i : 0);
+        }
+    }
+
+    // the matrix: lane (r, g) has row r % ROWS, eight k at 8 g of a k-step of range r / ROWS
+    constexpr int FRAG = 32 * ROWS;                     // packed: bfloat16 values of a (strip, k-step)
+    const __amdgpu_buffer_rsrc_t wbuf = PACKED ? fd_buffer(W + (size_t)blockIdx.x * ksteps * FRAG, ksteps * FRAG * 2)
+                                               : fd_buffer(W + (size_t)n0 * K, (N - n0 < ROWS ? N - n0 : ROWS) * K * 2);
+    const int w_ks = (range0 + r / ROWS) * per;         // its first k-step ...
+    const int w_end = w_ks + per < ksteps ? w_ks + per : ksteps;
+    const int w_k = PACKED ? w_end : (w_end * 32 < K ? w_end * 32 : K) - 8 * g;     // ... and the first that is not its own (in k-steps or k)
+    auto w_at = [&](int j) {
+        const int ks = w_ks + j;
+        if (PACKED) return ks < w_k ? ((ks * 4 + g) * ROWS + r % ROWS) * 16 : BEYOND;
+        return ks * 32 < w_k ? ((r % ROWS) * K + ks * 32 + 8 * g) * 2 : BEYOND;
+    };
+    // the activations: lane (r, g) has token r % TOKS, eight k at 8 g of a k-step of range b SB + r / TOKS
+    const __amdgpu_buffer_rsrc_t abuf = fd_buffer(A, ((M - 1) * lda + K) * 2);
+    int a_k[NB], a_end[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int ks = (range0 + b * SB + r / TOKS) * per, end = ks + per < ksteps ? ks + per : ksteps;
+        a_k[b] = ks * 32 + 8 * g;
+        a_end[b] = r % TOKS < M ? (end * 32 < K ? end * 32 : K) : 0;
+    }
+    const int a_row = (r % TOKS) * lda;
+
+    f32x4_t acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // CH k-steps of every range at a time, every load issued before the first product
+    for (int base = 0; base < per; base += CH) {
+        Frag wf[CH], af[NB][CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const int k = a_k[b] + (base + j) * 32;
+                af[b][j].u = __builtin_amdgcn_raw_buffer_load_b128(abuf, base + j < per && k < a_end[b] ? (a_row + k) * 2 : BEYOND, 0, 0);
+            }
+            wf[j].u = __builtin_amdgcn_raw_buffer_load_b128(wbuf, base + j < per ? w_at(base + j) : BEYOND, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j].b, af[b][j].b, acc[b], 0, 0, 0);
+    }
+    // lane: rows 4 g + i of the tile, so range 4 g / ROWS of the matrix; columns of range r / TOKS in each of the NB groups
+    const int range = 4 * g / ROWS;
+    f32x4_t own = acc[0];
+#pragma unroll
+    for (int b = 1; b < NB; ++b)
+        if (range / SB == b) own = acc[b];
+    if (range % SB == r / TOKS) red[range0 + range][g % (ROWS / 4)][r % TOKS] = own;
+    __syncthreads();
+    if (!epi) return;
+    f32x4_t v = red[0][g][tok];
+#pragma unroll
+    for (int w = 1; w < VW; ++w) v += red[w][g][tok];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (bias) v[i] += offset[i];
+        if (flags & SK_RELU2) {
+            v[i] = fmaxf(v[i], 0.f);
+            v[i] *= v[i];
+        }
+    }
+    if (accum) {                // the rounded result goes into the 32-bit residual stream (each element has one owner)
+        float* dst = accum + (size_t)tok * ldacc + nf;
+        if (fast) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) current[i] += bf16_to_f32(f32_to_bf16(v[i]));
+            *(f32x4_t*)dst = current;
+        } else {
+            for (int i = 0; i < 4 && nf + i < N; ++i) dst[i] += bf16_to_f32(f32_to_bf16(v[i]));
+        }
+    } else {
+        const float out[4] = {v[0], v[1], v[2], v[3]};
+        store4<TC>(C + (size_t)tok * ldc + nf, out, N - nf);
+    }
+}
+
+// Ranges of K: 4, or 16 for a long K over few strips. `rows`: of a strip (16, 8 or 4).
+template <typename TC, bool PACKED>
+static int launch_few(const void* A, int lda, const void* W, int rows, const void* bias, int flags, void* C, int ldc, int M, int N,
+                      int K, float* accum, int ldacc, hipStream_t stream) {
+    if ((size_t)M * lda * 2 >= 0x7ffffff0u && M > 1) {          // rows so far apart that an offset does not hold it: one by one (the same bits)
+        for (int m = 0; m < M; ++m) {
+            const int rc = launch_few<TC, PACKED>((const bf16_t*)A + (size_t)m * lda, lda, W, rows, bias, flags, C ? (TC*)C + (size_t)m * ldc : nullptr,
+                                                  ldc, 1, N, K, accum ? accum + (size_t)m * ldacc : nullptr, ldacc, stream);
+            if (rc) return rc;
+        }
+        return TM_OK;
+    }
+    const int strips = (N + rows - 1) / rows;
+    const bool long_k = K >= 2048 && !(rows == 16 && strips >= 256);
+#define TM_FEW(ROWS_, TOKS_, VW_, CH_)                                                                                \
+    gemm_few_kernel<ROWS_, TOKS_, VW_, CH_, TC, PACKED><<<strips, 4 * VW_ * ROWS_, 0, stream>>>(                      \
+        (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc)
+    if (rows == 4) {
+        if (M <= 4) { if (long_k) TM_FEW(4, 4, 16, 10); else TM_FEW(4, 4, 4, 7); }
+        else if (M <= 8) { if (long_k) TM_FEW(4, 8, 16, 10); else TM_FEW(4, 8, 4, 7); }
+        else { if (long_k) TM_FEW(4, 16, 16, 5); else TM_FEW(4, 16, 4, 7); }
+    } else if (rows == 8) {
+        if (M <= 8) { if (long_k) TM_FEW(8, 8, 16, 10); else TM_FEW(8, 8, 4, 8); }
+        else { if (long_k) TM_FEW(8, 16, 16, 10); else TM_FEW(8, 16, 4, 8); }
+    } else {
+        if (long_k) TM_FEW(16, 16, 16, 10); else TM_FEW(16, 16, 4, 16);
+    }
+#undef TM_FEW
+    TM_CHECK_LAUNCH();
+    return TM_OK;
+}
+
 // NT: tiles of 16 tokens. WAVES: wavefronts per block. SPLIT: they share a strip and split K.
 // SILU: W is [2 * N, K] = [gate; up] and the output is silu(gate) * up, N wide.
-// ROWS: rows of W in a strip (16, 8 or 4). A short strip leaves rows of the MFMA tile empty (their
-// lanes load nothing), which costs nothing here, and gives a matrix with few rows enough strips,
-// and so enough blocks, to have loads in flight on every CU of the chip.
-// PACKED: W is in strip order, strips of ROWS rows, rows and k beyond the matrix zero-filled; with SILU
+// PACKED: W is in strip order, strips of 16 rows, rows and k beyond the matrix zero-filled; with SILU
 // the up rows' strips start at strip `up_strip0` (each half packed by itself).
-template <int NT, int WAVES, bool SPLIT, bool SILU, typename TC, int ROWS = 16, bool PACKED = false>
+template <int NT, int WAVES, bool SPLIT, bool SILU, typename TC, bool PACKED = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* __restrict__ A, int lda,
                                                                  const bf16_t* __restrict__ W,
                                                                  const void* __restrict__ bias, int flags,
                                                                  TC* __restrict__ C, int ldc, int M, int N, int K,
                                                                  float* __restrict__ accum, int ldacc,
                                                                  int up_strip0 = 0) {
-    constexpr int NACC = SILU ? 2 : 1;
+    constexpr int NACC = SILU ? 2 : 1, ROWS = 16;
     // k-steps in flight per wavefront (fewer where 16 wavefronts share the register file)
-    constexpr int KCH = (WAVES > 4 && SILU && NT > 2) ? 4 : ((WAVES > 4 && NT == 1 && !SILU) ? 12 : ((WAVES > 4 || NT > 2 || SILU) ? 8 : 16));
+    constexpr int KCH = (WAVES > 4 && SILU && NT > 2) ? 4 : ((WAVES > 4 || NT > 2 || SILU) ? 8 : 16);
     __shared__ float red[SPLIT ? WAVES : 1][64][4 + 1];        // one accumulator tile at a time
     const int wave = threadIdx.x / TM_WAVE, lane = threadIdx.x % TM_WAVE;
     const int r = lane % 16, g = lane / 16;
@@ -103,11 +247,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
         ks1 = ks0 + per < ksteps ? ks0 + per : ksteps;
     }
     constexpr int FRAG = 32 * ROWS;             // packed: bfloat16 values of a (strip, k-step)
-    const bool w_ok = r < ROWS && (PACKED || n0 + r < N);
+    const bool w_ok = PACKED || n0 + r < N;
     const bf16_t* wrow;
     const bf16_t* urow = nullptr;
     if constexpr (PACKED) {
-        const int lane_off = (g * ROWS + (r < ROWS ? r : 0)) * 8;
+        const int lane_off = (g * ROWS + r) * 8;
         wrow = W + (size_t)strip * ksteps * FRAG + lane_off;
         if (SILU) urow = W + (size_t)(up_strip0 + strip) * ksteps * FRAG + lane_off;
     } else {
@@ -133,7 +277,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
     const int nf = n0 + 4 * g;                  // this lane's output features nf + i (i = 0..3) of token 16t + r
     const bool acc_fast = accum && nf + 4 <= N && (ldacc % 4) == 0 && ((uintptr_t)accum % 16) == 0;
     f32x4_t resid_cur[NT];
-    if (acc_fast && (!SPLIT || wave == 0) && 4 * g < ROWS) {
+    if (acc_fast && (!SPLIT || wave == 0)) {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
             resid_cur[t] = 16 * t + r < M ? *(const f32x4_t*)(accum + (size_t)(16 * t + r) * ldacc + nf) : f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -193,7 +337,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
         if (wave != 0) return;
     }
     if (n0 >= N) return;
-    if (4 * g >= ROWS) return;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         const int tok = 16 * t + r;
@@ -234,30 +377,19 @@ template <int NT, bool SILU, typename TC>
 static int launch_skinny(const void* A, int lda, const void* W, const void* bias, int flags, void* C, int ldc,
                          int M, int N, int K, float* accum, int ldacc, hipStream_t stream) {
     const int strips = (N + 15) / 16;
-    if (NT == 1 && !SILU && strips < 192) {    // few rows and few tokens: short strips, so that every CU gets a block
-        const bool r8 = (N + 7) / 8 >= 192;
-        const int n_strips = r8 ? (N + 7) / 8 : (N + 3) / 4;
-#define TM_SHORT(WV, RW)                                                                                         \
-    gemm_skinny_kernel<1, WV, true, false, TC, RW><<<n_strips, 64 * WV, 0, stream>>>(                            \
-        (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc)
-        if (K < 2048) {
-            if (r8) TM_SHORT(4, 8); else TM_SHORT(4, 4);
-        } else {
-            if (r8) TM_SHORT(16, 8); else TM_SHORT(16, 4);
-        }
-#undef TM_SHORT
-        TM_CHECK_LAUNCH();
-        return TM_OK;
+    if constexpr (NT == 1 && !SILU) {
+        if (strips < 2048) return launch_few<TC, false>(A, lda, W, tm_skinny_strip_rows(N, K), bias, flags, C, ldc, M, N, K, accum, ldacc, stream);
     }
     if (strips >= 2048) {                      // many rows: a strip per wavefront
         gemm_skinny_kernel<NT, 4, false, SILU, TC><<<(strips + 3) / 4, 256, 0, stream>>>(
             (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc);
-    } else if (strips >= 256 || K < 2048) {    // a block of 4 wavefronts per strip
-        gemm_skinny_kernel<NT, 4, true, SILU, TC><<<strips, 256, 0, stream>>>(
-            (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc);
-    } else {                                   // few rows, long K: 16 wavefronts per strip
-        gemm_skinny_kernel<NT, 16, true, SILU, TC><<<strips, 1024, 0, stream>>>(
-            (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc);
+    } else if constexpr (NT > 1 || SILU) {
+        if (strips >= 256 || K < 2048)         // a block of 4 wavefronts per strip
+            gemm_skinny_kernel<NT, 4, true, SILU, TC><<<strips, 256, 0, stream>>>(
+                (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc);
+        else                                   // few rows, long K: 16 wavefronts per strip
+            gemm_skinny_kernel<NT, 16, true, SILU, TC><<<strips, 1024, 0, stream>>>(
+                (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc);
     }
     TM_CHECK_LAUNCH();
     return TM_OK;
@@ -309,15 +441,16 @@ extern "C" int tm_skinny_strip_rows(int N, int K) {
     return (N + 7) / 8 >= 192 ? 8 : 4;
 }
 
-template <bool SILU, typename TC, int ROWS>
-static int launch_skinny_packed(const void* A, int lda, const void* W, const void* bias, int flags, void* C, int ldc,
-                                int M, int N, int K, float* accum, int ldacc, int up_strip0, hipStream_t stream) {
-    const int strips = (N + ROWS - 1) / ROWS;
+template <bool SILU, typename TC>
+static int launch_skinny_packed(const void* A, int lda, const void* W, int rows, const void* bias, int flags, void* C, int ldc,
+                                int M, int N, int K, float* accum, int ldacc, hipStream_t stream) {
+    const int strips = (N + 15) / 16;
 #define TM_PACKED(WV, SPL, BLOCKS)                                                                               \
-    gemm_skinny_kernel<1, WV, SPL, SILU, TC, ROWS, true><<<BLOCKS, 64 * WV, 0, stream>>>(                        \
-        (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc, up_strip0)
-    if (ROWS == 16 && strips >= 2048) TM_PACKED(4, false, (strips + 3) / 4);      // many rows: a strip per wavefront
-    else if (K < 2048 || (ROWS == 16 && strips >= 256)) TM_PACKED(4, true, strips);
+    gemm_skinny_kernel<1, WV, SPL, SILU, TC, true><<<BLOCKS, 64 * WV, 0, stream>>>(                              \
+        (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc, strips)
+    if (rows == 16 && strips >= 2048) TM_PACKED(4, false, (strips + 3) / 4);      // many rows: a strip per wavefront
+    else if constexpr (!SILU) return launch_few<TC, true>(A, lda, W, rows, bias, flags, C, ldc, M, N, K, accum, ldacc, stream);
+    else if (K < 2048 || strips >= 256) TM_PACKED(4, true, strips);
     else TM_PACKED(16, true, strips);
 #undef TM_PACKED
     TM_CHECK_LAUNCH();
@@ -338,18 +471,9 @@ extern "C" int tm_gemm_skinny_packed(const void* A, int lda, const void* W, int 
         (rows != 16 && rows != 8 && rows != 4) || (silu && (rows != 16 || bias)))
         return TM_ERR_ARG;
     const int flags = (bias_dtype == TM_F32 ? SK_BIAS_F32 : 0) | (relu2 ? SK_RELU2 : 0);    // the kernel's flags
-    const int up_strip0 = (N + 15) / 16;
-#define TM_PACKED_ROWS(SILU_, TC_)                                                                               \
-    switch (rows) {                                                                                              \
-        case 16: return launch_skinny_packed<SILU_, TC_, 16>(A, lda, W, bias, flags, C, ldc, M, N, K, accum, ldacc, up_strip0, stream); \
-        case 8: if (!SILU_) return launch_skinny_packed<false, TC_, 8>(A, lda, W, bias, flags, C, ldc, M, N, K, accum, ldacc, 0, stream); break; \
-        default: if (!SILU_) return launch_skinny_packed<false, TC_, 4>(A, lda, W, bias, flags, C, ldc, M, N, K, accum, ldacc, 0, stream); break; \
-    }
-    if (out_dtype == TM_BF16) {
-        if (silu) { TM_PACKED_ROWS(true, bf16_t) } else { TM_PACKED_ROWS(false, bf16_t) }
-    } else if (out_dtype == TM_F32 && !silu) {
-        TM_PACKED_ROWS(false, float)
-    }
-#undef TM_PACKED_ROWS
+    if (out_dtype == TM_BF16)
+        return silu ? launch_skinny_packed<true, bf16_t>(A, lda, W, rows, bias, flags, C, ldc, M, N, K, accum, ldacc, stream)
+                    : launch_skinny_packed<false, bf16_t>(A, lda, W, rows, bias, flags, C, ldc, M, N, K, accum, ldacc, stream);
+    if (out_dtype == TM_F32 && !silu) return launch_skinny_packed<false, float>(A, lda, W, rows, bias, flags, C, ldc, M, N, K, accum, ldacc, stream);
     return TM_ERR_ARG;
 }
