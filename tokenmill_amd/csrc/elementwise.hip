@@ -5,6 +5,7 @@
 // are 32-bit; a bfloat16 result is rounded once, where the tensor is stored.
 #include "common.h"
 #include "api.h"
+#include "fused_common.h"
 
 // ------------------------------------------------------------------------------------------
 // embedding rows -> 32-bit residual stream           (reference src/infer/model/qwen2.py:46)
@@ -172,7 +173,23 @@ template <> struct Vec4<bf16_t> {
 
 #define ADD_NORM_MAX_PARTS 8       // most partial sums the vector kernel adds (more: the plain kernel)
 
-template <typename T, typename WT, int THREADS>
+// four elements at an offset (in elements) of a row; beyond its end: zeros
+template <typename T> __device__ __forceinline__ ew_f32x4 row4(const T* row, int hidden, int at);
+template <> __device__ __forceinline__ ew_f32x4 row4<float>(const float* row, int hidden, int at) {
+    return as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(fd_buffer(row, hidden * 4), at * 4, 0, 0));
+}
+template <> __device__ __forceinline__ ew_f32x4 row4<bf16_t>(const bf16_t* row, int hidden, int at) {
+    const u32x2_t u = __builtin_amdgcn_raw_buffer_load_b64(fd_buffer(row, hidden * 2), at * 2, 0, 0);
+    return ew_f32x4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                    __uint_as_float(u.y & 0xffff0000u)};
+}
+
+// A block a row. The launch is a trip to memory, a sum over the block and a store, so everything is asked for at once: the row, what is
+// to be added, the weights. PARTS: 0, or the partial sums there is room for (2, 4 or 8; one that does not exist is part 0 again,
+// not counted). GROUPS: 4-element groups a thread has.
+// Before, with the weights asked for behind the sum, eight parts read whatever their number and the sums exchanged through LDS twice:
+// 64 rows of 896, 8 / 2 parts, 4.9 us a launch in a step, 2,048 rows with 2 parts 7.8; now 4.0 / 3.5 and 6.4.
+template <typename T, typename WT, int THREADS, int GROUPS, int PARTS>
 __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(float* __restrict__ resid, const Pending<T> pending,
                                                               const int* __restrict__ rows,
                                                               const WT* __restrict__ weight, T* __restrict__ out,
@@ -181,51 +198,80 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(float* __restr
     const int r = blockIdx.x;
     const size_t src = rows ? (size_t)rows[r] : (size_t)r;
     float* x = resid + src * hidden;
-    const T* d = pending.delta ? pending.delta + src * hidden : nullptr;
-    const float* ps = pending.parts ? pending.parts + src * hidden : nullptr;
+    const T* d = !PARTS && pending.delta ? pending.delta + src * hidden : nullptr;
+    const float* ps = PARTS ? pending.parts + src * hidden : nullptr;
     T* o = out + (size_t)r * hidden;
-    const int groups = hidden / 4;
-    ew_f32x4 v[4];
+    ew_f32x4 v[GROUPS], w[GROUPS], part[GROUPS][PARTS ? PARTS : 1];
+    auto at = [&](int i) { return 4 * ((int)threadIdx.x + i * THREADS); };
+    auto load = [&](int i) {
+        v[i] = row4(x, hidden, at(i));
+        if constexpr (PARTS > 0) {
+#pragma unroll
+            for (int p = 0; p < PARTS; ++p) part[i][p] = row4(ps + (size_t)(p < pending.n_parts ? p : 0) * pending.stride, hidden, at(i));
+        } else {
+            part[i][0] = row4(d, d ? hidden : 0, at(i));
+        }
+        if constexpr (GROUPS < 4) w[i] = row4(weight, hidden, at(i));
+    };
     float ss = 0.f;
+    auto add = [&](int i) {
+        if constexpr (PARTS > 0) {                                  // the parts in their order
+            ew_f32x4 sum = part[i][0];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int gidx = threadIdx.x + i * THREADS;
-        v[i] = ew_f32x4{0.f, 0.f, 0.f, 0.f};
-        if (gidx < groups) {
-            v[i] = Vec4<float>::load(x + 4 * gidx);
-            if (d) {
-                v[i] += Vec4<T>::load(d + 4 * gidx);
-                if (!rows) Vec4<float>::store(x + 4 * gidx, v[i]);
-            } else if (ps) {
-                // all parts asked for at once (a part that does not exist: part 0 again, not counted), then added in order
-                ew_f32x4 part[ADD_NORM_MAX_PARTS];
+            for (int p = 1; p < PARTS; ++p)
+                if (p < pending.n_parts) sum += part[i][p];
 #pragma unroll
-                for (int p = 0; p < ADD_NORM_MAX_PARTS; ++p)
-                    part[p] = Vec4<float>::load(ps + (size_t)(p < pending.n_parts ? p : 0) * pending.stride + 4 * gidx);
-                ew_f32x4 sum = part[0];
+            for (int k = 0; k < 4; ++k) v[i][k] += Elem<T>::round(sum[k]);
+        } else {
+            if (d) v[i] += part[i][0];
+        }
+        ss += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
+    };
+    if constexpr (GROUPS * (PARTS + 2) <= 12) {
 #pragma unroll
-                for (int p = 1; p < ADD_NORM_MAX_PARTS; ++p)
-                    if (p < pending.n_parts) sum += part[p];
+        for (int i = 0; i < GROUPS; ++i) load(i);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int k = 0; k < 4; ++k) v[i][k] += Elem<T>::round(sum[k]);
-                if (!rows) Vec4<float>::store(x + 4 * gidx, v[i]);
-            }
-            ss += v[i][0] * v[i][0] + v[i][1] * v[i][1] + v[i][2] * v[i][2] + v[i][3] * v[i][3];
+        for (int i = 0; i < GROUPS; ++i) add(i);
+    } else {                                                        // (more than the registers hold)
+#pragma unroll
+        for (int i = 0; i < GROUPS; ++i) {
+            load(i);
+            add(i);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    ss = block_sum<THREADS>(ss, red);
+    ss = wave_sum(ss);
+    if (threadIdx.x % TM_WAVE == 0) red[threadIdx.x / TM_WAVE] = ss;
+    __syncthreads();
+    ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < THREADS / TM_WAVE; ++i) ss += red[i];
     const float rs = rsqrtf(ss / (float)hidden + eps);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int gidx = threadIdx.x + i * THREADS;
-        if (gidx < groups) {
-            const ew_f32x4 w = Vec4<WT>::load(weight + 4 * gidx);
+    for (int i = 0; i < GROUPS; ++i) {
+        if (at(i) < hidden) {
             ew_f32x4 y;
+            if constexpr (GROUPS == 4) w[i] = row4(weight, hidden, at(i));               // (no registers for it before)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) y[k] = w[k] * Elem<T>::round(v[i][k] * rs);   // rounded BEFORE the weight multiplies
-            Vec4<T>::store(o + 4 * gidx, y);
+            for (int k = 0; k < 4; ++k) y[k] = w[i][k] * Elem<T>::round(v[i][k] * rs);   // rounded BEFORE the weight multiplies
+            Vec4<T>::store(o + at(i), y);
+            if (!rows && (PARTS || d)) Vec4<float>::store(x + at(i), v[i]);
         }
     }
+}
+
+template <typename T, typename WT, int THREADS, int GROUPS>
+static void launch_add_rmsnorm_vec(float* resid, const Pending<T>& pending, const int* rows, const WT* weight, T* out, int R, int hidden,
+                                   float eps, hipStream_t stream) {
+    if (!pending.parts)
+        add_rmsnorm_vec_kernel<T, WT, THREADS, GROUPS, 0><<<R, THREADS, 0, stream>>>(resid, pending, rows, weight, out, hidden, eps);
+    else if (pending.n_parts <= 2)
+        add_rmsnorm_vec_kernel<T, WT, THREADS, GROUPS, 2><<<R, THREADS, 0, stream>>>(resid, pending, rows, weight, out, hidden, eps);
+    else if (pending.n_parts <= 4)
+        add_rmsnorm_vec_kernel<T, WT, THREADS, GROUPS, 4><<<R, THREADS, 0, stream>>>(resid, pending, rows, weight, out, hidden, eps);
+    else
+        add_rmsnorm_vec_kernel<T, WT, THREADS, GROUPS, ADD_NORM_MAX_PARTS><<<R, THREADS, 0, stream>>>(resid, pending, rows, weight, out, hidden, eps);
 }
 
 template <typename T, typename WT>
@@ -239,15 +285,18 @@ static void launch_add_rmsnorm(float* resid, const void* delta, const float* par
     // a thread for every 4-element group where 1,024 reach (measured on an MI355X, 64 rows with 4 partial sums: width
     // 3,584 6.5 us with 256 threads, 4.9 with 512, 4.5 with 1,024; width 5,120 5.7 with 512, 5.1 with 1,024; width 896
     // 3.4 us with any); from the width alone: the sum of squares has one order per model
-    const int threads = hidden <= 1024 ? 256 : hidden <= 2048 ? 512 : 1024;
-    if (vec && threads == 256)
-        add_rmsnorm_vec_kernel<T, WT, 256><<<R, 256, 0, stream>>>(resid, pending, rows, (const WT*)weight, (T*)out, hidden, eps);
-    else if (vec && threads == 512)
-        add_rmsnorm_vec_kernel<T, WT, 512><<<R, 512, 0, stream>>>(resid, pending, rows, (const WT*)weight, (T*)out, hidden, eps);
-    else if (vec)
-        add_rmsnorm_vec_kernel<T, WT, 1024><<<R, 1024, 0, stream>>>(resid, pending, rows, (const WT*)weight, (T*)out, hidden, eps);
-    else
+    if (!vec)
         add_rmsnorm_kernel<T, WT><<<R, 256, 0, stream>>>(resid, pending, rows, (const WT*)weight, (T*)out, hidden, eps);
+    else if (hidden <= 1024)
+        launch_add_rmsnorm_vec<T, WT, 256, 1>(resid, pending, rows, (const WT*)weight, (T*)out, R, hidden, eps, stream);
+    else if (hidden <= 2048)
+        launch_add_rmsnorm_vec<T, WT, 512, 1>(resid, pending, rows, (const WT*)weight, (T*)out, R, hidden, eps, stream);
+    else if (hidden <= 4096)
+        launch_add_rmsnorm_vec<T, WT, 1024, 1>(resid, pending, rows, (const WT*)weight, (T*)out, R, hidden, eps, stream);
+    else if (hidden <= 8192)
+        launch_add_rmsnorm_vec<T, WT, 1024, 2>(resid, pending, rows, (const WT*)weight, (T*)out, R, hidden, eps, stream);
+    else
+        launch_add_rmsnorm_vec<T, WT, 1024, 4>(resid, pending, rows, (const WT*)weight, (T*)out, R, hidden, eps, stream);
 }
 
 static int add_rmsnorm_any(float* resid, const void* delta, const float* parts, int n_parts, size_t stride, const int* rows,
