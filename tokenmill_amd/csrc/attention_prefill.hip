@@ -200,8 +200,11 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     float scale_log2, float cap_in, float cap_out, int window, int keep, const float* __restrict__ sink,
     const bf16_t* __restrict__ cgate, int ldcg) {
     constexpr int NDC = D / 32, NDT = D / 16;
-    __shared__ float s_m[KS][16], s_l[KS][16];
-    __shared__ float s_o[KS][16][D + 1];
+    // the wavefronts' partials of all heads: rows of d four floats apart from a multiple of 64, so that 16 lanes of a store or load
+    // of 16 bytes meet no bank twice
+    __shared__ float s_m[KS][HPW][16], s_l[KS][HPW][16];
+    extern __shared__ __align__(16) float s_o[];                     // [KS][HPW][16][D + 4]
+    auto partial_at = [&](int w, int hh, int col, int d) { return s_o + (size_t)((w * HPW + hh) * 16 + col) * (D + 4) + d; };
     // the wavefront index in a scalar register: everything derived from it (its key blocks, their
     // pages, the branches on them) stays wave-uniform
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE);
@@ -217,30 +220,42 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     const int other = n_tiles - 1 - (int)blockIdx.x;
     const int n_mine = (pair && other > (int)blockIdx.x) ? 2 : 1;
 
-#pragma unroll 1
-    for (int which = 0; which < n_mine; ++which) {
-        const int* tl = tiles + (size_t)(which ? other : (int)blockIdx.x) * 4;
-        const int s = tl[0], row0 = tl[1], valid = tl[2], pos0 = tl[3];
-        const int* table = block_tables + (size_t)s * table_width;
-        const TileView tv = tile_view(pos0, valid, r, window, keep);
-        const int kb0 = tv.first_key / 32, kb1 = tv.last_key / 32;
-        const int first_tile = tv.first_key / 16, last_tile = tv.last_key / 16;
-        BlockWalk walk;
+    // A tile begins with three trips to memory (its entry in the table, its queries and pages, its first keys). Those of the second
+    // tile are made while the first one's partials meet.
+    int row0, valid, pos0, kb, kb1, kept_tiles, first_tile, last_tile;
+    const int* table;
+    TileView tv;
+    BlockWalk walk;
+    PFrag qf[HPW][NDC];
+    KVBlock<D> ba, bb;
+    int2 pages;
+    auto begin = [&](int tile) {                                     // up to the queries and the pages
+        const int* tl = tiles + (size_t)tile * 4;
+        const int s = tl[0];
+        row0 = tl[1], valid = tl[2], pos0 = tl[3];
+        table = block_tables + (size_t)s * table_width;
+        tv = tile_view(pos0, valid, r, window, keep);
+        const int kb0 = tv.first_key / 32;
+        kb1 = tv.last_key / 32;
+        first_tile = tv.first_key / 16, last_tile = tv.last_key / 16;
         walk.kept = tv.first_key > 0 ? (tv.keep + 31) / 32 : 0;
-        const int kept_tiles = tv.first_key > 0 ? (tv.keep + 15) / 16 : 0;
+        kept_tiles = tv.first_key > 0 ? (tv.keep + 15) / 16 : 0;
         const int behind = kb0 > walk.kept ? kb0 : walk.kept;        // the first block >= behind of this wavefront:
         walk.resume = behind + ((wave - behind) & (KS - 1));
-
-        PFrag qf[HPW][NDC];
+        kb = wave < walk.kept ? wave : walk.resume;
+        pages = lane_pages<KS>(kb, walk, lane, kept_tiles, first_tile, last_tile, table, page_shift);
+        // (columns beyond the tile's tokens are its last token again, heads beyond the group its last head: nobody reads their results)
+        const bf16_t* qrow = q + (size_t)(row0 + (r < valid ? r : valid - 1)) * q_stride + 8 * g;
 #pragma unroll
         for (int hh = 0; hh < HPW; ++hh)
 #pragma unroll
-            for (int c = 0; c < NDC; ++c) {
-                if (hh < nh && r < valid)
-                    qf[hh][c].u = *(const u32x4_t*)(q + (size_t)(row0 + r) * q_stride + (size_t)(h0 + hh) * D + 32 * c + 8 * g);
-                else
-                    qf[hh][c].u = u32x4_t{0, 0, 0, 0};
-            }
+            for (int c = 0; c < NDC; ++c) qf[hh][c].u = *(const u32x4_t*)(qrow + (size_t)(h0 + (hh < nh ? hh : nh - 1)) * D + 32 * c);
+    };
+    begin(blockIdx.x);
+    load_kv_block<D>(ba, pages, 0, k_pool, v_pool, kvh, KVH, page_shift, off);
+
+#pragma unroll 1
+    for (int which = 0; which < n_mine; ++which) {
         HeadState<D, HPW> st;
 #pragma unroll
         for (int hh = 0; hh < HPW; ++hh) {
@@ -252,11 +267,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
 
         // Two register sets take turns: one is worked on while the other's loads are in flight. The
         // load after the last block repeats it, unused, so that no load hides behind a branch.
-        int kb = wave < walk.kept ? wave : walk.resume;
-        KVBlock<D> ba, bb;
-        int2 pages = lane_pages<KS>(kb, walk, lane, kept_tiles, first_tile, last_tile, table, page_shift);
         int slot = 0;                                                // block kb is slot `slot` of `pages`
-        if (kb <= kb1) load_kv_block<D>(ba, pages, 0, k_pool, v_pool, kvh, KVH, page_shift, off);
         while (kb <= kb1) {
             if (slot == 31) {                                        // the next block starts a new set of pages
                 pages = lane_pages<KS>(walk.at<KS>(kb, kb + KS), walk, lane, kept_tiles, first_tile, last_tile, table, page_shift);
@@ -277,56 +288,60 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
             ++slot;
         }
 
-        // merge the wavefronts' partials head by head, in wavefront order; lane: d = 16 dt + 4 g + i of token r
+        // The wavefronts' partials meet in LDS, all heads at once, and are added in wavefront order. (A head at a time, 17 KB of LDS and two
+        // barriers each, this took 5 of a tile's 13 to 15 us at 2,048 tokens.)
+        const int done_row0 = row0, done_valid = valid;
+        const bool more = which + 1 < n_mine;
+        if (more) begin(other);
 #pragma unroll
         for (int hh = 0; hh < HPW; ++hh) {
             if (hh >= nh) continue;                                  // block-uniform
-            float lsum = st.l[hh];
-            lsum = lane_sum<16>(lsum);
-            lsum = lane_sum<32>(lsum);
-            // a gate per channel: this thread's pieces, on their way while the partials meet
-            constexpr int GP = (16 * (D / 2) + 64 * KS - 1) / (64 * KS);
-            uint32_t gv[GP];
-#pragma unroll
-            for (int u = 0; u < GP; ++u) {
-                const int idx = threadIdx.x + u * 64 * KS, col = idx / (D / 2) < valid ? idx / (D / 2) : valid - 1;
-                gv[u] = cgate ? *(const uint32_t*)(cgate + (size_t)(row0 + col) * ldcg + (size_t)(h0 + hh) * D + 2 * (idx % (D / 2))) : 0u;
-            }
+            const float lsum = lane_sum<32>(lane_sum<16>(st.l[hh]));
             if (g == 0) {
-                s_m[wave][r] = st.m[hh];
-                s_l[wave][r] = lsum;
+                s_m[wave][hh][r] = st.m[hh];
+                s_l[wave][hh][r] = lsum;
             }
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) s_o[wave][r][16 * dt + 4 * g + i] = st.o[hh][dt][i];
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < GP; ++u) {
-                const int idx = threadIdx.x + u * 64 * KS;
-                const int col = idx / (D / 2), d = 2 * (idx % (D / 2));
-                if (col >= valid) continue;
-                float mm = s_m[0][col];
-#pragma unroll
-                for (int w = 1; w < KS; ++w) mm = fmaxf(mm, s_m[w][col]);
-                float ll = 0.f, o0 = 0.f, o1 = 0.f;
-#pragma unroll
-                for (int w = 0; w < KS; ++w) {
-                    const float f = (s_m[w][col] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(s_m[w][col] - mm);
-                    ll = fmaf(s_l[w][col], f, ll);
-                    o0 = fmaf(s_o[w][col][d], f, o0);
-                    o1 = fmaf(s_o[w][col][d + 1], f, o1);
-                }
-                if (sink) ll += __builtin_amdgcn_exp2f(sink[h0 + hh] * 1.4426950408889634f - mm);      // a term of the denominator without a key
-                const float inv = 1.f / ll;
-                if (cgate) {
-                    o0 *= sigmoid_fast(__uint_as_float(gv[u] << 16));
-                    o1 *= sigmoid_fast(__uint_as_float(gv[u] & 0xffff0000u));
-                }
-                *(uint32_t*)(out + (size_t)(row0 + col) * out_stride + (size_t)(h0 + hh) * D + d) = pk_bf16(o0 * inv, o1 * inv);
-            }
-            __syncthreads();
+            for (int dt = 0; dt < NDT; ++dt) *(f32x4_t*)partial_at(wave, hh, r, 16 * dt + 4 * g) = st.o[hh][dt];    // lane: d = 16 dt + 4 g + i of token r
         }
+        if (more) load_kv_block<D>(ba, pages, 0, k_pool, v_pool, kvh, KVH, page_shift, off);
+        __syncthreads();
+        // a thread: four channels of a token and head
+        for (int idx = threadIdx.x; idx < nh * 16 * (D / 4); idx += 64 * KS) {
+            const int d = 4 * (idx % (D / 4)), col = idx / (D / 4) % 16, hh = idx / (16 * (D / 4));
+            if (col >= done_valid) continue;
+            uint2 gp = {0u, 0u};
+            if (cgate) {                                             // a gate per channel
+                const bf16_t* gate = cgate + (size_t)(done_row0 + col) * ldcg + (size_t)(h0 + hh) * D + d;
+                gp = uint2{*(const uint32_t*)gate, *(const uint32_t*)(gate + 2)};
+            }
+            float mm = s_m[0][hh][col];
+#pragma unroll
+            for (int w = 1; w < KS; ++w) mm = fmaxf(mm, s_m[w][hh][col]);
+            float ll = 0.f;
+            f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < KS; ++w) {
+                const float mw = s_m[w][hh][col];
+                const float f = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - mm);
+                const f32x4_t ow = *(const f32x4_t*)partial_at(w, hh, col, d);
+                ll = fmaf(s_l[w][hh][col], f, ll);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = fmaf(ow[i], f, o[i]);
+            }
+            if (sink) ll += __builtin_amdgcn_exp2f(sink[h0 + hh] * 1.4426950408889634f - mm);      // a term of the denominator without a key
+            const float inv = 1.f / ll;
+            if (cgate) {
+                o[0] *= sigmoid_fast(__uint_as_float(gp.x << 16));
+                o[1] *= sigmoid_fast(__uint_as_float(gp.x & 0xffff0000u));
+                o[2] *= sigmoid_fast(__uint_as_float(gp.y << 16));
+                o[3] *= sigmoid_fast(__uint_as_float(gp.y & 0xffff0000u));
+            }
+            uint32_t* dst = (uint32_t*)(out + (size_t)(done_row0 + col) * out_stride + (size_t)(h0 + hh) * D + d);
+            dst[0] = pk_bf16(o[0] * inv, o[1] * inv);                // (the rows are 4-byte aligned, no more)
+            dst[1] = pk_bf16(o[2] * inv, o[3] * inv);
+        }
+        if (more) __syncthreads();                                   // the partials have been read
     }
 }
 
@@ -337,7 +352,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
 template <int D> struct PrefillShape { static constexpr int HPW = D <= 64 ? 4 : 2, KS = D <= 64 ? 8 : 4; };
 
 template <int D, int HPW>
-static void launch_split_keys(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
+static int launch_split_keys(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                               const int* block_tables, int table_width, const int* tiles, int n_tiles, int H, int KVH,
                               int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep, const float* sink,
                               const bf16_t* cgate, int ldcg, hipStream_t stream) {
@@ -346,9 +361,16 @@ static void launch_split_keys(const void* q, int q_stride, void* out, int out_st
     // fold the table in two once the folded launch still gives every CU a block
     const int pair = (long long)(n_tiles / 2) * KVH * splits >= 256 ? 1 : 0;
     dim3 grid(pair ? (n_tiles + 1) / 2 : n_tiles, KVH * splits);
-    attn_prefill_mfma_kernel<D, HPW, KS><<<grid, 64 * KS, 0, stream>>>(
+    constexpr int lds = KS * HPW * 16 * (D + 4) * (int)sizeof(float);          // at most 139,264 bytes
+    if (lds > 64 * 1024) {
+        static const hipError_t raised = hipFuncSetAttribute((const void*)attn_prefill_mfma_kernel<D, HPW, KS>,
+                                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (raised != hipSuccess) return TM_ERR_LAUNCH;
+    }
+    attn_prefill_mfma_kernel<D, HPW, KS><<<grid, 64 * KS, lds, stream>>>(
         (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
         table_width, tiles, n_tiles, pair, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
+    return TM_OK;
 }
 
 // softcap > 0: a score s (scaled) becomes softcap * tanh(s / softcap) before the softmax; sink (float32 [H]) or null: one more term
@@ -371,15 +393,16 @@ extern "C" int tm_attn_prefill_mfma_cap(const void* q, int q_stride, void* out, 
     while ((1 << page_shift) < page) ++page_shift;
     const float scale_log2 = scale * 1.4426950408889634f;
     if ((long long)KVH * ((G + 1) / 2) > 65535) return TM_ERR_ARG;
+    int rc = TM_OK;
 #define TM_SPLIT_ARGS q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, tiles, n_tiles, H, KVH, \
                       page_shift, scale_log2, cap_in, cap_out, window, keep, sink, (const bf16_t*)cgate, ldcg, stream
 #define TM_PREFILL_CASE(DD)                                                                                       \
     case DD: {                                                                                                    \
         constexpr int HPW = PrefillShape<DD>::HPW;                                                                \
         if (HPW > 2 && G > 2 && (long long)n_tiles * KVH * ((G + 1) / 2) <= TM_PREFILL_ONE_ROUND)                 \
-            launch_split_keys<DD, 2>(TM_SPLIT_ARGS);                                                              \
+            rc = launch_split_keys<DD, 2>(TM_SPLIT_ARGS);                                                         \
         else                                                                                                      \
-            launch_split_keys<DD, HPW>(TM_SPLIT_ARGS);                                                            \
+            rc = launch_split_keys<DD, HPW>(TM_SPLIT_ARGS);                                                       \
         break;                                                                                                    \
     }
     switch (D) {
@@ -392,6 +415,7 @@ extern "C" int tm_attn_prefill_mfma_cap(const void* q, int q_stride, void* out, 
     }
 #undef TM_PREFILL_CASE
 #undef TM_SPLIT_ARGS
+    if (rc) return rc;
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
