@@ -47,33 +47,35 @@ struct BlockWalk {
     __device__ __forceinline__ int at(int from, int b) const { return from < kept && b >= kept ? resume + (b - kept) / KS * KS : b; }
 };
 
-// The pages of the next 32 key blocks of a wavefront (blocks kb, kb + KS, ... of its walk), one 16-key tile per
-// lane: lane 2 i + t holds the page of tile t of the i-th of them. A tile that holds no key any
+// Where the next 32 key blocks of a wavefront (blocks kb, kb + KS, ... of its walk) lie, one 16-key tile per
+// lane: lane 2 i + t holds the places of tile t of the i-th of them, of its keys in units of 64 bytes of the key pool and of its
+// values in units of 32 bytes of the value pool (a tile is whole runs of both). 64 lanes work them out at once; the scalar
+// unit needed 47 instructions a tile, in a loop that waits for its results. A tile that holds no key any
 // query of this wavefront may see (beyond the newest key, or wholly behind the window) is replaced
 // by the nearest tile that does: its table entry may name no page. The caller masks every score of
 // such a tile by the key's real position and clears its values (the tile in its place may hold keys beyond the newest one).
-template <int KS>
-__device__ __forceinline__ int2 lane_pages(int kb, const BlockWalk& walk, int lane, int kept_tiles, int first_tile, int last_tile,
-                                           const int* __restrict__ table, int page_shift) {
+struct TilePlaces {
+    uint32_t k, v;
+};
+template <int D, int KS>
+__device__ __forceinline__ TilePlaces lane_pages(int kb, const BlockWalk& walk, int lane, int kept_tiles, int first_tile, int last_tile,
+                                                 const int* __restrict__ table, int kvh, int KVH, int page_shift) {
     int tile = 2 * walk.at<KS>(kb, kb + (lane >> 1) * KS) + (lane & 1);
     tile = (tile < first_tile && tile >= kept_tiles) ? first_tile : (tile > last_tile ? last_tile : tile);
     const int tile0 = 16 * tile;
-    return int2{table[tile0 >> page_shift], tile0 & ((1 << page_shift) - 1)};
+    const uint32_t page = (uint32_t)table[tile0 >> page_shift], in_page = (uint32_t)(tile0 & ((1 << page_shift) - 1));
+    return TilePlaces{(((page << page_shift) + in_page) * KVH + kvh) * (D / 32), ((page * KVH + kvh) * D << (page_shift - 4)) + in_page / 16};
 }
 
-// Loads one block of 32 keys (two tiles of 16); slot = which of the 32 blocks held in `pages`.
+// Loads one block of 32 keys (two tiles of 16); slot = which of the 32 blocks held in `places`.
 template <int D>
-__device__ __forceinline__ void load_kv_block(KVBlock<D>& blk, int2 pages, int slot,
-                                              const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
-                                              int kvh, int KVH, int page_shift, LaneOffsets off) {
+__device__ __forceinline__ void load_kv_block(KVBlock<D>& blk, const TilePlaces& places, int slot, const bf16_t* __restrict__ k_pool,
+                                              const bf16_t* __restrict__ v_pool, int page_shift, LaneOffsets off) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const int pg = __builtin_amdgcn_readlane(pages.x, 2 * slot + t);                    // wave-uniform
-        const int in_page = __builtin_amdgcn_readlane(pages.y, 2 * slot + t);
-        const __amdgpu_buffer_rsrc_t kbuf =
-            uniform_buffer(k_pool + ((((size_t)pg << page_shift) + in_page) * KVH + kvh) * D);
-        const __amdgpu_buffer_rsrc_t vbuf =
-            uniform_buffer(v_pool + ((((size_t)pg * KVH + kvh) * D) << page_shift) + in_page);
+        const uint32_t k_at = __builtin_amdgcn_readlane(places.k, 2 * slot + t), v_at = __builtin_amdgcn_readlane(places.v, 2 * slot + t);
+        const __amdgpu_buffer_rsrc_t kbuf = uniform_buffer((const char*)k_pool + ((uint64_t)k_at << 6));
+        const __amdgpu_buffer_rsrc_t vbuf = uniform_buffer((const char*)v_pool + ((uint64_t)v_at << 5));
 #pragma unroll
         for (int c = 0; c < D / 32; ++c)
             blk.k[t][c].u = __builtin_amdgcn_raw_buffer_load_b128(kbuf, off.k, 64 * c, 0);
@@ -84,7 +86,7 @@ __device__ __forceinline__ void load_kv_block(KVBlock<D>& blk, int2 pages, int s
 }
 
 // One block of 32 keys against the wavefront's heads.
-template <int D, int HPW>
+template <int D, int HPW, bool CAP>
 __device__ __forceinline__ void attend_block(KVBlock<D>& blk, HeadState<D, HPW>& st, const PFrag (&qf)[HPW][D / 32],
                                              int key0, int nh, const TileView& tv, int g, float scale_log2, float cap_in, float cap_out) {
     constexpr int NDC = D / 32, NDT = D / 16;
@@ -117,25 +119,27 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, HeadState<D, HPW>&
             for (int c = 0; c < NDC; ++c)
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.k[t][c].b, qf[hh][c].b, acc, 0, 0, 0);
             // capped scores: cap * tanh(score * scale / cap), kept in units of 1 / scale like the plain ones
-            if (cap_in > 0.f) {
+            if constexpr (CAP) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[i] = cap_out * tanh_fast(acc[i] * cap_in);
             }
             sc[hh][t] = acc;
         }
     }
+    if (edge) {                                                  // (which keys a column sees is worked out once for all heads)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int kj = key0 + 16 * t + 4 * g + i;
+                const bool mine = (kj <= tv.my_pos) & ((kj >= tv.my_lo) | (kj < tv.keep));
+#pragma unroll
+                for (int hh = 0; hh < HPW; ++hh) sc[hh][t][i] = mine ? sc[hh][t][i] : -INFINITY;
+            }
+    }
 #pragma unroll
     for (int hh = 0; hh < HPW; ++hh) {
         if (hh >= nh) continue;                                  // wave-uniform
-        if (edge) {
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int kj = key0 + 16 * t + 4 * g + i;
-                    if (!tv.mine(kj)) sc[hh][t][i] = -INFINITY;
-                }
-        }
         // this lane's largest score of the block (scale > 0: the maximum commutes with it)
         float lm = max3(-INFINITY, sc[hh][0][0], sc[hh][0][1]);
         lm = max3(lm, sc[hh][0][2], sc[hh][0][3]);
@@ -192,7 +196,7 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, HeadState<D, HPW>&
 // With pair != 0 a block takes tile b and then tile n_tiles - 1 - b: in a table sorted by the
 // number of keys a tile sees, the longest goes with the shortest and every block has the same work
 // (the lower triangle of a prompt, folded).
-template <int D, int HPW, int KS>
+template <int D, int HPW, int KS, bool CAP>
 __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
@@ -228,7 +232,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     BlockWalk walk;
     PFrag qf[HPW][NDC];
     KVBlock<D> ba, bb;
-    int2 pages;
+    TilePlaces pages;
     auto begin = [&](int tile) {                                     // up to the queries and the pages
         const int* tl = tiles + (size_t)tile * 4;
         const int s = tl[0];
@@ -243,7 +247,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
         const int behind = kb0 > walk.kept ? kb0 : walk.kept;        // the first block >= behind of this wavefront:
         walk.resume = behind + ((wave - behind) & (KS - 1));
         kb = wave < walk.kept ? wave : walk.resume;
-        pages = lane_pages<KS>(kb, walk, lane, kept_tiles, first_tile, last_tile, table, page_shift);
+        pages = lane_pages<D, KS>(kb, walk, lane, kept_tiles, first_tile, last_tile, table, kvh, KVH, page_shift);
         // (columns beyond the tile's tokens are its last token again, heads beyond the group its last head: nobody reads their results)
         const bf16_t* qrow = q + (size_t)(row0 + (r < valid ? r : valid - 1)) * q_stride + 8 * g;
 #pragma unroll
@@ -252,7 +256,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
             for (int c = 0; c < NDC; ++c) qf[hh][c].u = *(const u32x4_t*)(qrow + (size_t)(h0 + (hh < nh ? hh : nh - 1)) * D + 32 * c);
     };
     begin(blockIdx.x);
-    load_kv_block<D>(ba, pages, 0, k_pool, v_pool, kvh, KVH, page_shift, off);
+    load_kv_block<D>(ba, pages, 0, k_pool, v_pool, page_shift, off);
 
 #pragma unroll 1
     for (int which = 0; which < n_mine; ++which) {
@@ -270,20 +274,20 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
         int slot = 0;                                                // block kb is slot `slot` of `pages`
         while (kb <= kb1) {
             if (slot == 31) {                                        // the next block starts a new set of pages
-                pages = lane_pages<KS>(walk.at<KS>(kb, kb + KS), walk, lane, kept_tiles, first_tile, last_tile, table, page_shift);
+                pages = lane_pages<D, KS>(walk.at<KS>(kb, kb + KS), walk, lane, kept_tiles, first_tile, last_tile, table, kvh, KVH, page_shift);
                 slot = -1;
             }
-            load_kv_block<D>(bb, pages, slot + 1, k_pool, v_pool, kvh, KVH, page_shift, off);
-            attend_block<D, HPW>(ba, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
+            load_kv_block<D>(bb, pages, slot + 1, k_pool, v_pool, page_shift, off);
+            attend_block<D, HPW, CAP>(ba, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
             kb = walk.at<KS>(kb, kb + KS);
             ++slot;
             if (kb > kb1) break;
             if (slot == 31) {
-                pages = lane_pages<KS>(walk.at<KS>(kb, kb + KS), walk, lane, kept_tiles, first_tile, last_tile, table, page_shift);
+                pages = lane_pages<D, KS>(walk.at<KS>(kb, kb + KS), walk, lane, kept_tiles, first_tile, last_tile, table, kvh, KVH, page_shift);
                 slot = -1;
             }
-            load_kv_block<D>(ba, pages, slot + 1, k_pool, v_pool, kvh, KVH, page_shift, off);
-            attend_block<D, HPW>(bb, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
+            load_kv_block<D>(ba, pages, slot + 1, k_pool, v_pool, page_shift, off);
+            attend_block<D, HPW, CAP>(bb, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
             kb = walk.at<KS>(kb, kb + KS);
             ++slot;
         }
@@ -304,7 +308,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) *(f32x4_t*)partial_at(wave, hh, r, 16 * dt + 4 * g) = st.o[hh][dt];    // lane: d = 16 dt + 4 g + i of token r
         }
-        if (more) load_kv_block<D>(ba, pages, 0, k_pool, v_pool, kvh, KVH, page_shift, off);
+        if (more) load_kv_block<D>(ba, pages, 0, k_pool, v_pool, page_shift, off);
         __syncthreads();
         // a thread: four channels of a token and head
         for (int idx = threadIdx.x; idx < nh * 16 * (D / 4); idx += 64 * KS) {
@@ -351,7 +355,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
 // (512 tokens at the 0.5B shape: 13.4 to 9.8 us; a head's arithmetic is the same either way, so its bits are).
 template <int D> struct PrefillShape { static constexpr int HPW = D <= 64 ? 4 : 2, KS = D <= 64 ? 8 : 4; };
 
-template <int D, int HPW>
+template <int D, int HPW, bool CAP>
 static int launch_split_keys(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                               const int* block_tables, int table_width, const int* tiles, int n_tiles, int H, int KVH,
                               int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep, const float* sink,
@@ -363,11 +367,11 @@ static int launch_split_keys(const void* q, int q_stride, void* out, int out_str
     dim3 grid(pair ? (n_tiles + 1) / 2 : n_tiles, KVH * splits);
     constexpr int lds = KS * HPW * 16 * (D + 4) * (int)sizeof(float);          // at most 139,264 bytes
     if (lds > 64 * 1024) {
-        static const hipError_t raised = hipFuncSetAttribute((const void*)attn_prefill_mfma_kernel<D, HPW, KS>,
+        static const hipError_t raised = hipFuncSetAttribute((const void*)attn_prefill_mfma_kernel<D, HPW, KS, CAP>,
                                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (raised != hipSuccess) return TM_ERR_LAUNCH;
     }
-    attn_prefill_mfma_kernel<D, HPW, KS><<<grid, 64 * KS, lds, stream>>>(
+    attn_prefill_mfma_kernel<D, HPW, KS, CAP><<<grid, 64 * KS, lds, stream>>>(
         (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
         table_width, tiles, n_tiles, pair, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
     return TM_OK;
@@ -400,9 +404,9 @@ extern "C" int tm_attn_prefill_mfma_cap(const void* q, int q_stride, void* out, 
     case DD: {                                                                                                    \
         constexpr int HPW = PrefillShape<DD>::HPW;                                                                \
         if (HPW > 2 && G > 2 && (long long)n_tiles * KVH * ((G + 1) / 2) <= TM_PREFILL_ONE_ROUND)                 \
-            rc = launch_split_keys<DD, 2>(TM_SPLIT_ARGS);                                                         \
+            rc = softcap > 0.f ? launch_split_keys<DD, 2, true>(TM_SPLIT_ARGS) : launch_split_keys<DD, 2, false>(TM_SPLIT_ARGS); \
         else                                                                                                      \
-            rc = launch_split_keys<DD, HPW>(TM_SPLIT_ARGS);                                                       \
+            rc = softcap > 0.f ? launch_split_keys<DD, HPW, true>(TM_SPLIT_ARGS) : launch_split_keys<DD, HPW, false>(TM_SPLIT_ARGS); \
         break;                                                                                                    \
     }
     switch (D) {
