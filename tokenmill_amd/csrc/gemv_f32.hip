@@ -36,8 +36,10 @@ struct GemvArgs {
     float* v_pool;              // [pages, KVH, D, page]
 };
 
-// AHEAD: steps of 16 k a wavefront asks for at once
-template <int EPI, int RT, int WAVES, int AHEAD>
+// GROUP: steps of 16 k whose products meet in sums of their own before they join the running one. AHEAD: groups a wavefront asks for
+// at once: with one, a wavefront of the 0.5B shape waited for memory two or three times in a launch of 6 to 7 us (o 6.2 to 5.8, q|k|v 7.2
+// to 6.8, down 7.3 either way, gate|up, whose blocks a CU hide each other's waits, 12.9 either way).
+template <int EPI, int RT, int WAVES, int GROUP, int AHEAD>
 __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArgs a) {
     static_assert(EPI == GM_PLAIN || RT == 1, "");
     __shared__ __align__(16) f32x4_t red[WAVES][RT][TM_WAVE];
@@ -74,42 +76,63 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
         const int n = (at < end ? at : end - 1) + (EPI != GM_PLAIN && r >= 8 ? far : 0);
         pw[t] = a.W + (size_t)n * a.K + 4 * g;
     }
-    // what the epilogue waits for otherwise
+    // What the epilogue waits for otherwise: the positions are asked for before the matrix (loads come back in their order), the
+    // rotary rows, whose place hangs on them, behind its first round.
     int pos = 0, slot = -1;
+    f32x4_t bias0 = {0.f, 0.f, 0.f, 0.f}, bias1 = bias0, cosv = bias0, sinv = bias0;
+    const int ge = EPI == GM_PLAIN ? g : g % 2;                 // (SiLU, q|k|v: lanes beyond the tile's eight rows have no epilogue)
     if constexpr (EPI == GM_QKV) {
-        pos = a.positions[r < a.M ? r : a.M - 1];
-        slot = a.slots ? a.slots[r < a.M ? r : a.M - 1] : -1;
+        const int row = r < a.M ? r : a.M - 1;
+        pos = a.positions[row];
+        slot = (a.slots ? a.slots : a.positions)[row];
+        if (a.bias) {
+            bias0 = *(const f32x4_t*)(a.bias + n0[0] + 4 * ge);
+            bias1 = *(const f32x4_t*)(a.bias + n0[0] + far + 4 * ge);
+        }
     }
     f32x4_t sum[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) sum[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int s = s0; s < s1; s += AHEAD) {
-        f32x4_t w[RT][AHEAD], x[AHEAD];
+    for (int s = s0; s < s1; s += GROUP * AHEAD) {
+        f32x4_t w[RT][GROUP * AHEAD], x[GROUP * AHEAD];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
+        for (int i = 0; i < GROUP * AHEAD; ++i) {
             const int at = 16 * (s + i < s1 ? s + i : s1 - 1);  // (no load under a test: beyond the end the last step again)
 #pragma unroll
             for (int t = 0; t < RT; ++t) w[t][i] = *(const f32x4_t*)(pw[t] + at);
             x[i] = *(const f32x4_t*)(pa + at);
         }
         __builtin_amdgcn_sched_barrier(0);
-        // four sums a tile, of every fourth k, that join the running one here: short chains of roundings
-        f32x4_t acc[RT][4];
-#pragma unroll
-        for (int t = 0; t < RT; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[t][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
-            if (s + i >= s1) break;                             // the same for the whole wavefront
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int t = 0; t < RT; ++t)
-                    acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i][e], x[i][e], acc[t][e], 0, 0, 0);
+        if constexpr (EPI == GM_QKV) {
+            if (s == s0) {
+                const size_t at = (size_t)pos * (a.D / 2) + j0 + 4 * ge;
+                cosv = *(const f32x4_t*)(a.cos_t + at);
+                sinv = *(const f32x4_t*)(a.sin_t + at);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int t = 0; t < RT; ++t) sum[t] += (acc[t][0] + acc[t][1]) + (acc[t][2] + acc[t][3]);
+        for (int j = 0; j < AHEAD; ++j) {
+            if (s + j * GROUP >= s1) break;                     // the same for the whole wavefront
+            // four sums a tile, of every fourth k, that join the running one here: short chains of roundings
+            f32x4_t acc[RT][4];
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[t][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = j * GROUP; i < (j + 1) * GROUP; ++i) {
+                if (s + i >= s1) break;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int t = 0; t < RT; ++t)
+                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i][e], x[i][e], acc[t][e], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) sum[t] += (acc[t][0] + acc[t][1]) + (acc[t][2] + acc[t][3]);
+        }
     }
 #pragma unroll
     for (int t = 0; t < RT; ++t) red[wave][t][lane] = sum[t];
@@ -144,18 +167,17 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
         if (r >= a.M) return;
         f32x4_t x = total(0, lane), y = total(0, lane + 32);
         if (a.bias) {
-            x += *(const f32x4_t*)(a.bias + n0[0] + 4 * g);
-            y += *(const f32x4_t*)(a.bias + n0[0] + far + 4 * g);
+            x += bias0;
+            y += bias1;
         }
+        if (!a.slots) slot = -1;
         const int d = j0 + 4 * g;
         if (head < a.H + a.KVH) {
-            const size_t at = (size_t)pos * (a.D / 2) + d;
-            const f32x4_t c = *(const f32x4_t*)(a.cos_t + at), s = *(const f32x4_t*)(a.sin_t + at);
             f32x4_t y1, y2;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float p, q;
-                rotate_pair(x[e], y[e], c[e], s[e], p, q);
+                rotate_pair(x[e], y[e], cosv[e], sinv[e], p, q);
                 y1[e] = p;
                 y2[e] = q;
             }
@@ -187,13 +209,15 @@ extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, con
            (!bias || gm_aligned16(bias));
 }
 
-// Up to a block a CU, eight wavefronts split K and ask for four steps at a time; more blocks than that have four wavefronts with
-// seven (0.5B shape, eight rows: down 7.1 us against 8.2 to 9.0 for the other combinations of 4, 8, 16 and 4, 7; gate|up 12.1
-// against 12.0 to 13.7, head 126 against 127 to 131).
+// Up to a block a CU, eight wavefronts split K into groups of four steps, two or three of them at a time; more blocks than that have four
+// wavefronts with groups of seven, two at a time where a block has one tile (two tiles, of the head: the registers of two groups leave
+// too few wavefronts a CU).
 #define GM_LAUNCH(EPI, RT, units, split)                                                                                    \
     do {                                                                                                                    \
-        if ((units) * (split) <= 256) gemv_mfma_f32_kernel<EPI, RT, 8, 4><<<dim3(units, split), 512, 0, stream>>>(a);       \
-        else gemv_mfma_f32_kernel<EPI, RT, 4, 7><<<dim3(units, split), 256, 0, stream>>>(a);                                \
+        const int per_ = ((a.K / 16 + (split) - 1) / (split) + 7) / 8;                                                      \
+        if ((units) * (split) <= 256 && per_ <= 8) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2><<<dim3(units, split), 512, 0, stream>>>(a); \
+        else if ((units) * (split) <= 256) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3><<<dim3(units, split), 512, 0, stream>>>(a); \
+        else gemv_mfma_f32_kernel<EPI, RT, 4, 7, RT == 1 ? 2 : 1><<<dim3(units, split), 256, 0, stream>>>(a);               \
     } while (0)
 
 extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,
