@@ -39,7 +39,7 @@ int tm_gemm_f32_mfma(const float* A, int lda, const float* W, const float* bias,
 // Products of prompt-sized steps on the bfloat16 matrix unit (gemm_tile.hip), W row-major [rows, K]; K a multiple of 64, rows of
 // whole 16-byte pieces (tm_gemm_tile_takes): silu(gate) * up of gate|up; q|k|v with bias, rotation over the whole head (head
 // sizes that are multiples of 64) and cache write; 32-bit partial sums [parts][M][N] of a product whose K is split
-// (tm_tile_linear_parts says over how many parts, 0: the library's product is the better one).
+// (tm_tile_linear_parts says over how many parts, 0: the library's product is the better one); a plain product in either type.
 int tm_gemm_tile_takes(const void* A, int lda, const void* W, int M, int N, int K);
 int tm_gemm_tile_shape(int M, int N, int K, int splits);        // which of its tiles it runs with (for tests)
 int tm_tile_gate_up_silu(const void* A, int lda, int M, int K, const void* W, void* act, int I, hipStream_t stream);
@@ -47,6 +47,7 @@ int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void* W, const 
                      const float* cos_t, const float* sin_t, const int* positions, const int* slots, void* k_pool, void* v_pool,
                      int page, hipStream_t stream);
 int tm_tile_linear_parts(int M, int N, int K);
+int tm_tile_linear(const void* A, int lda, int M, int K, const void* W, int N, void* C, int ldc, int out_dtype, hipStream_t stream);
 int tm_tile_linear_split(const void* A, int lda, int M, int K, const void* W, int N, float* parts, hipStream_t stream);
 
 // The same for the true 32-bit path (K a multiple of 32, tm_tile_f32_takes); tm_tile_f32_linear_split with one part stores the product.
@@ -383,6 +384,12 @@ int tm_moe_up_act_mfma(const void* x, int ldx, const int* slot_pair, int top, co
 // The per-head products and the experts' products on the matrix unit (grouped_mfma.hip), bfloat16; the matrices as
 // [groups, N, K] with k contiguous. The *_takes functions say whether the operands come in whole 16-byte pieces.
 int tm_heads_matmul_mfma_takes(const void* A, int lda, int a_off, const void* W, int K);
+int tm_latent_rows(const void* pool, const int* table, int table_width, int page, int first, int count, int lo, int hi, int Lk, int Dr,
+                   void* latent, void* shared, hipStream_t stream);
+int tm_attn_heads_takes(int Dn, int Dr, int Dv);
+int tm_attn_heads(const void* q, int ldq, const void* qr, const void* kv, const void* vt, void* out, const int* blocks, int n_blocks,
+                  const float* gate, int ldg, const float* sink, int H, int Dn, int Dr, int Dv, int R, float scale, int window,
+                  hipStream_t stream);
 int tm_heads_matmul_mfma(const void* A, int lda, int a_off, const void* W, void* C, int ldc, int c_off, const float* gate, int ldg,
                          int T, int H, int K, int N, int tail, int rot, const float* cos_t, const float* sin_t, const int* positions,
                          int half_pairs, hipStream_t stream);

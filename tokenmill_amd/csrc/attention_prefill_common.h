@@ -2,21 +2,11 @@
 // wavefront's heads, and what a wavefront knows about the tile of query tokens it works on.
 #pragma once
 #include "common.h"
+#include "fused_common.h"
 
 #define PF_SLACK 8.f        // how far (log2 units) a score may exceed the running reference before it moves
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-
-union PFrag {
-    u32x4_t u;
-    bf16x8_t b;
-};
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef FFrag PFrag;
 
 // two floats -> packed bfloat16 (round to nearest even, one instruction on gfx950)
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {

@@ -29,6 +29,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t fd_buffer(const void* base, in
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
 }
 
+// 16 bytes a lane from base + voff (bytes) to LDS at lds (bytes, wave-uniform) + 16 * lane
+__device__ __forceinline__ void fd_load_lds(uint32_t lds, uint32_t voff, const void* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "m0", "memory");
+}
+
 #define FD_EPI_QKV 0
 #define FD_EPI_SILU 1
 #define FD_KCH 8            // k-steps of one register group of matrix loads, per wavefront (one group in all)

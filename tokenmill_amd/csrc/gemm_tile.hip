@@ -1,5 +1,5 @@
 // Matrix products of prompt-sized steps on the bfloat16 matrix unit, each with its layer's own epilogue: gate|up with SiLU*up;
-// q|k|v with bias, rotation and cache write; 32-bit partial sums of a product A W^T whose K is split over groups of blocks (or is
+// q|k|v with bias, rotation and cache write; a plain store; 32-bit partial sums of a product A W^T whose K is split over groups of blocks (or is
 // not, one part); the products of experts. The same kernel on the 32-bit matrix unit is the true 32-bit path's.
 //
 // A block of four wavefronts computes a tile of BM rows by BN matrix rows, BM x BN / 4 a wavefront, k in steps of 64. Both
@@ -23,7 +23,7 @@
 
 #include <type_traits>
 
-enum { GT_SILU = 0, GT_QKV = 1, GT_PARTS = 2, GT_EXPERT_SILU = 3, GT_EXPERT_CLAMPED = 4, GT_EXPERT_RELU2 = 5, GT_EXPERT_DOWN = 6 };
+enum { GT_SILU = 0, GT_QKV = 1, GT_PARTS = 2, GT_STORE = 3, GT_EXPERT_SILU = 4, GT_EXPERT_CLAMPED = 5, GT_EXPERT_RELU2 = 6, GT_EXPERT_DOWN = 7 };
 
 struct TileArgs {
     const void* A;              // [M, K], rows lda apart
@@ -75,11 +75,6 @@ __device__ __forceinline__ void gt_store8(T* dst, const float (&v)[8]) {
     } else {
         *(u32x4_t*)dst = u32x4_t{fd_pack(v[0], v[1]), fd_pack(v[2], v[3]), fd_pack(v[4], v[5]), fd_pack(v[6], v[7])};
     }
-}
-
-// 16 bytes a lane from base + voff (bytes) to LDS at lds (bytes, wave-uniform) + 16 * lane
-__device__ __forceinline__ void gt_load_lds(uint32_t lds, uint32_t voff, const void* base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "m0", "memory");
 }
 
 // two values rounded to the tensors' type and back, by one conversion
@@ -218,7 +213,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
             }
         }
     };
-    auto issue_one = [&](uint32_t dst, int i) { gt_load_lds(dst + i * 4096, voff[i], i < BM / 32 ? (const void*)lA : (const void*)lW); };
+    auto issue_one = [&](uint32_t dst, int i) { fd_load_lds(dst + i * 4096, voff[i], i < BM / 32 ? (const void*)lA : (const void*)lW); };
     auto issued = [&]() {
         lA += l_more ? 128 : 0;
         lW += l_more ? 128 : 0;
@@ -432,6 +427,10 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                         *(f32x4_t*)(dst + c1) = f32x4_t{y[0], y[1], y[2], y[3]};
                         *(f32x4_t*)(dst + c1 + 4) = f32x4_t{y[4], y[5], y[6], y[7]};
                     }
+                } else if (EPI == GT_STORE) {
+                    T* dst = (T*)a.C + (size_t)m * a.ldc;
+                    if (ok0) gt_store8(dst + c0, x);
+                    if (ok1) gt_store8(dst + c1, y);
                 } else if (EPI == GT_EXPERT_RELU2) {
                     T* dst = (T*)a.C + (size_t)m * a.ldc;
 #pragma unroll
@@ -683,6 +682,17 @@ extern "C" int tm_tile_linear_split(const void* A, int lda, int M, int K, const 
         return gt_few_wide(N, K) ? gt_launch<bf16_t, GT_PARTS, 2, 4, 2, 2, GT_FEW_WIDE_RING, 2>(a, stream)
                                  : gt_launch<bf16_t, GT_PARTS, 1, 4, 4, 1, GT_FEW_RING, 2>(a, stream);
     return gt_go<GT_PARTS>(a, gt_choose(M, N, K, splits), stream);
+}
+
+// C[m, n] = A W^T, rows ldc apart, in bfloat16 (out_dtype 1) or, with ldc = N, float32 (0)
+extern "C" int tm_tile_linear(const void* A, int lda, int M, int K, const void* W, int N, void* C, int ldc, int out_dtype, hipStream_t stream) {
+    if (!gt_aligned(C) || ldc < N || ldc % 8 || (out_dtype != TM_BF16 && out_dtype != TM_F32) || (out_dtype == TM_F32 && ldc != N) ||
+        !tm_gemm_tile_takes(A, lda, W, M, N, K))
+        return TM_ERR_ARG;
+    TileArgs a{};
+    a.A = A; a.W = W; a.C = C;
+    a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.splits = 1;
+    return out_dtype == TM_F32 ? gt_go<GT_PARTS>(a, gt_choose(M, N, K, 1), stream) : gt_go<GT_STORE>(a, gt_choose(M, N, K, 1), stream);
 }
 
 // --- the same in 32-bit ---------------------------------------------------------------------------------------------------

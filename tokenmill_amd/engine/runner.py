@@ -271,7 +271,8 @@ class ModelRunner:
             num_logit_rows=R, num_decode=ND,
             max_decode_context=(self.max_positions if ND else 0) if shape is not None else
             max([s0 + 1 for s0, n in zip(starts, q_lens) if n == 1], default=0),
-            prefill_tiles=d(tiles_s).view(n_tiles, 4))
+            prefill_tiles=d(tiles_s).view(n_tiles, 4),
+            portions_known=bool(self.pools.states))        # (such a model's portions are never replayed)
         return ctx, list(range(R_real))
 
     @staticmethod

@@ -1643,6 +1643,73 @@ def attn_latent_mfma(qa: torch.Tensor, out: torch.Tensor, pool: torch.Tensor, bl
     return out
 
 
+def tile_linear_takes(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Does the tiled product take a [M, K] (rows a stride apart) and w [N, K]?"""
+    return bool(a.is_cuda and a.dtype == w.dtype == torch.bfloat16 and a.dim() == w.dim() == 2 and a.stride(1) == 1 and w.is_contiguous()
+                and library().tm_gemm_tile_takes(_p(a), c_int(a.stride(0) if a.shape[0] > 1 else a.shape[1]), _p(w), c_int(a.shape[0]),
+                                                 c_int(w.shape[0]), c_int(w.shape[1])))
+
+
+def tile_linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+    """out[m, n] = sum_k a[m, k] w[n, k], bfloat16 operands, out of either type, by the tiled product of prompt-sized steps."""
+    _gpu(a, w, out)
+    _need(tile_linear_takes(a, w) and a.shape[1] == w.shape[1], "tile_linear: bfloat16 operands in whole 16-byte pieces, K a multiple of 64")
+    _need(out.dtype in (torch.bfloat16, torch.float32) and tuple(out.shape) == (a.shape[0], w.shape[0]) and out.is_contiguous(),
+          "tile_linear: out is contiguous [M, N]")
+    _check(library().tm_tile_linear(_p(a), c_int(a.stride(0) if a.shape[0] > 1 else a.shape[1]), c_int(a.shape[0]), c_int(a.shape[1]), _p(w),
+                                    c_int(w.shape[0]), _p(out), c_int(w.shape[0]), c_int(code(out.dtype)), _stream()), "tile_linear")
+    return out
+
+
+def latent_rows(pool: torch.Tensor, table: torch.Tensor, first: int, lo: int, hi: int, Lk: int, Dr: int, latent: torch.Tensor,
+                shared: torch.Tensor) -> None:
+    """Rows of one request (``table``: its block table, int32 [W]) gathered from a cache of shared latents: row i of ``latent`` [n, Lk]
+    and ``shared`` [n, Dr] is that of position first + i; positions outside lo .. hi give zeros."""
+    _gpu(pool, table, latent, shared)
+    page = _check_latent_pool(pool, Lk + Dr, torch.bfloat16, "latent_rows")
+    n = latent.shape[0]
+    _need(table.dtype == torch.int32 and table.dim() == 1 and table.is_contiguous(), "latent_rows: a table is contiguous int32 [W]")
+    _need(tuple(latent.shape) == (n, Lk) and tuple(shared.shape) == (n, Dr) and latent.is_contiguous() and shared.is_contiguous()
+          and latent.dtype == shared.dtype == torch.bfloat16, f"latent_rows: bfloat16 [n, {Lk}] and [n, {Dr}]")
+    _need(first >= 0 and lo >= 0 and (hi < lo or hi // page < table.shape[0]), "latent_rows: positions beyond the block table")
+    _check(library().tm_latent_rows(_p(pool), _p(table), c_int(table.shape[0]), c_int(page), c_int(first), c_int(n), c_int(lo), c_int(hi), c_int(Lk),
+                                    c_int(Dr), _p(latent), _p(shared), _stream()), "latent_rows")
+
+
+def attn_heads_takes(Dn: int, Dr: int, Dv: int) -> bool:
+    """Is there a kernel for keys of Dn channels of a head and Dr shared ones, and values of Dv?"""
+    return bool(library().tm_attn_heads_takes(c_int(Dn), c_int(Dr), c_int(Dv)))
+
+
+def attn_heads(q: torch.Tensor, qr: torch.Tensor, kv: torch.Tensor, vt: torch.Tensor, out: torch.Tensor, blocks: torch.Tensor, H: int, Dn: int,
+               Dr: int, Dv: int, scale: float, window: int = 0, gate: torch.Tensor | None = None, sink: torch.Tensor | None = None) -> torch.Tensor:
+    """Attention of prompt portions with keys and values per head. q [T, H (Dn + Dr)], of which a head's last Dr channels stand rotated in
+    qr [T, H Dr]; kv flat: keys [R, H Dn] and behind them the channels that the heads share [R, Dr]; vt [H Dv, R]: the values,
+    transposed. ``blocks`` (int32 [n, 4]): (first row of q, queries (at most 64), position of the first, row of position 0 in kv and vt); the
+    rows of every block of 64 keys that a query's window touches exist. Rows of ``out`` [T, H Dv] that no block names are left alone;
+    the others are multiplied by sigmoid(gate[t, h]) (float32 [T, >= H]) if there is one."""
+    _gpu(q, qr, kv, vt, out, blocks, gate, sink)
+    _check_sink(sink, H)
+    T, R = q.shape[0], vt.shape[1]
+    _need(attn_heads_takes(Dn, Dr, Dv), "attention(heads): sizes the kernel does not run")
+    _need(all(t.dtype == torch.bfloat16 for t in (q, qr, kv, vt, out)), "attention(heads): bfloat16 only")
+    _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] >= H * (Dn + Dr) and tuple(qr.shape) == (T, H * Dr) and qr.is_contiguous()
+          and tuple(out.shape) == (T, H * Dv) and out.is_contiguous(), "attention(heads): q [T, H (Dn + Dr)], qr [T, H Dr] and out [T, H Dv]")
+    _need(R > 0 and R % 64 == 0 and kv.dim() == 1 and kv.numel() == R * (H * Dn + Dr) and kv.is_contiguous() and tuple(vt.shape) == (H * Dv, R)
+          and vt.is_contiguous(), "attention(heads): kv flat [R (H Dn + Dr)], vt [H Dv, R], R a multiple of 64")
+    _need(blocks.dtype == torch.int32 and blocks.dim() == 2 and blocks.shape[1] == 4 and blocks.is_contiguous(), "attention(heads): blocks is int32 [n, 4]")
+    _need(window >= 0, "attention(heads): window must be >= 0")
+    ldg = 0
+    if gate is not None:
+        _need(gate.dtype == torch.float32 and gate.dim() == 2 and gate.shape[0] == T and gate.shape[1] >= H and gate.stride(1) == 1,
+              "attention(heads): gate is float32 [T, >= H]")
+        ldg = gate.stride(0) if T > 1 else max(gate.stride(0), H)
+    _check(library().tm_attn_heads(_p(q), c_int(q.stride(0) if T > 1 else max(q.stride(0), q.shape[1])), _p(qr), _p(kv), _p(vt), _p(out), _p(blocks),
+                                   c_int(blocks.shape[0]), _p(gate), c_int(ldg), _p(sink), c_int(H), c_int(Dn), c_int(Dr), c_int(Dv), c_int(R),
+                                   c_float(scale), c_int(window), _stream()), "attn_heads")
+    return out
+
+
 # -------------------------------------------------------------------------------------------- experts by table
 
 MOE_TILE_ROWS = 32

@@ -22,10 +22,15 @@ import torch
 
 from tokenmill_amd import profiling
 from tokenmill_amd.hip import ops
-from tokenmill_amd.parts.base import KVCacheSpec, KVCacheView, Mixer, StepContext, as_tensor
+from tokenmill_amd.parts.base import KVCacheSpec, KVCacheView, Mixer, StepContext, as_tensor, portion_blocks
 from tokenmill_amd.parts.linear import Linear
 from tokenmill_amd.parts.position import RotaryEmbedding
 from tokenmill_amd.weights.loader import TensorSpec
+
+
+# Portions run with keys and values per head where one of their tokens sees at least so many rows and all see at most so many.
+HEADS_SEEN_ROWS = 384
+HEADS_MOST_ROWS = 8192
 
 
 class LatentAttention(Mixer):
@@ -139,16 +144,50 @@ class LatentAttention(Mixer):
         seen, pairs = self.visible_pairs(step)
         return seen * self.row * e + step.num_tokens * H * (self.row + Lk) * e, 2 * pairs * H * (self.row + Lk)
 
-    def _attend(self, qa, latent, step: StepContext, cache: KVCacheView, group) -> None:
+    def _by_heads(self, q, step: StepContext) -> bool:
+        """Do the step's portions run with keys and values per head, made from the visible rows, in place of queries and results moved
+        onto the latent? A (query, row) pair costs a third that way, and a token's rows are walked by two wavefronts side by side; it is
+        three launches more, which a short prompt has no use for. Where the host knows the portions (a step that a graph replays is
+        sized for others too), and while the keys and values stay a passing buffer (8,192 rows of the 2k shapes: 70 MB). A step of the
+        2k Lusolix shape, onto the latent / by heads, us: prompts of 100 / 250 / 400 / 800 / 1,500 tokens 2,470 / 2,483 / 2,682 / 3,377 /
+        4,268 and 2,597 / 2,576 / 2,638 / 2,607 / 3,005 (up to 2,600 the launches are the time), 64 tokens behind 600 / 1,000 cached ones
+        2,779 / 3,248 and 2,561 / 2,567."""
+        if not step.portions_known or step.num_decode >= q.shape[0] or q.dtype != torch.bfloat16 or self.uk_nt is None \
+                or not ops.attn_heads_takes(self.head_dim, self.rot_dim, self.v_head_dim):
+            return False
+        seen = max(a + n for a, n in zip(step.start_positions, step.q_lens[:step.num_seqs - step.num_decode]))
+        if min(seen, self.window or seen) < HEADS_SEEN_ROWS:
+            return False
+        H, Dn, Lk = self.num_heads, self.head_dim, self.kv_rank
+        return portion_blocks(step, self.window or 0, q.device)[2] <= HEADS_MOST_ROWS and Lk % 64 == 0 and Lk >= 256 and H * Dn % 8 == 0
+
+    def _attend_by_heads(self, q, out, gate, step: StepContext, cache: KVCacheView, group, cos, sin) -> None:
+        """The portions' rows of ``out`` [T, H Dv], gated."""
+        H, Dn, Dr, Dv, Lk = self.num_heads, self.head_dim, self.rot_dim, self.v_head_dim, self.kv_rank
+        blocks, gathers, rows = portion_blocks(step, self.window or 0, q.device)
+        T, bf16 = q.shape[0] - step.num_decode, dict(dtype=torch.bfloat16, device=q.device)
+        latent, kv = torch.empty((rows, Lk), **bf16), torch.empty(rows * (H * Dn + Dr), **bf16)
+        keys, shared = kv[:rows * H * Dn].view(rows, H * Dn), kv[rows * H * Dn:].view(rows, Dr)
+        vt, qr = torch.empty((H * Dv, rows), **bf16), torch.empty((T, H * Dr), **bf16)
+        for s, first, count, lo, hi, at in gathers:
+            ops.latent_rows(cache.k, group.block_tables[s], first, lo, hi, Lk, Dr, latent[at:at + count], shared[at:at + count])
+        ops.tile_linear(latent, self.uk.view(H * Dn, Lk), keys)
+        ops.tile_linear(self.uv_nt.view(H * Dv, Lk), latent, vt)
+        ops.rotate_heads(q[:T, Dn:], Dn + Dr, qr, Dr, H, Dr, cos, sin, step.positions[:T], half_pairs=self.half_pairs)
+        ops.attn_heads(q[:T], qr, kv, vt, out[:T], blocks, H, Dn, Dr, Dv, self.scale, self.window or 0,
+                       gate=gate[:T] if gate is not None else None, sink=self.sink)
+
+    def _attend(self, qa, latent, step: StepContext, cache: KVCacheView, group, singles_only: bool = False) -> None:
         """Prompt portions and single tokens (the step's last ``num_decode`` rows) on the matrix unit where its kernel takes
         the sizes; the 32-bit path and every other size through the kernel that takes a token and a head a wavefront."""
         H, Lk, row, T = self.num_heads, self.kv_rank, self.row, qa.shape[0]
         tiles, first_single = step.prefill_tiles, T - step.num_decode
-        if not ops.attn_latent_mfma_takes(qa.dtype, Lk, row, H) or (first_single > 0 and (tiles is None or not tiles.shape[0])):
+        if not ops.attn_latent_mfma_takes(qa.dtype, Lk, row, H) or (
+                first_single > 0 and not singles_only and (tiles is None or not tiles.shape[0])):
             ops.attn_latent(qa, latent, cache.k, group.block_tables, step.seq_of_token, step.positions, H, Lk, row, self.scale,
                             self.window or 0, sink=self.sink)
             return
-        if first_single > 0:
+        if first_single > 0 and not singles_only:
             ops.attn_latent_mfma(qa, latent, cache.k, group.block_tables, tiles, step.seq_of_token, step.positions, 0, 0, H, Lk, row,
                                  self.scale, self.window or 0, sink=self.sink)
         if step.num_decode > 0:
@@ -177,23 +216,38 @@ class LatentAttention(Mixer):
             else:
                 ops.latent_prepare(low, Lq, 0, 0, self.q_norm, None, self.norm_eps, None, None, None, None, cq, None)
             q = self.uq.forward(cq)
-            qa = torch.empty((T, H * row), dtype=x.dtype, device=x.device)
-            if self.uk_nt is not None and ops.heads_matmul_mfma_takes(q, Dn + Dr, self.uk_nt):
-                # the heads' rotated channels go beside their part on the latent in the same launch
-                ops.heads_matmul_mfma(q, Dn + Dr, self.uk_nt, qa, row, tail=Dr, cos=cos, sin=sin, positions=step.positions,
-                                      half_pairs=half)
-            else:
-                ops.heads_matmul(q, Dn + Dr, self.uk, qa, row)
-                if Dr:
-                    ops.rotate_heads(q[:, Dn:], Dn + Dr, qa[:, Lk:], row, H, Dr, cos, sin, step.positions, half_pairs=half)
-        latent = torch.empty((T, H * Lk), dtype=x.dtype, device=x.device)
-        with profiling.label("attention", lambda: self.cost("attention", step, T)):
-            self._attend(qa, latent, step, cache, group)
+        gate = low[:, self.gate_at:] if self.output_gate else None
+        out = torch.empty((T, H * Dv), dtype=x.dtype, device=x.device)
+        done = 0                                                    # rows of out that are there: the portions', or none
+        if self._by_heads(q, step):
+            done = T - step.num_decode
+            with profiling.label("attention", lambda: self.cost("attention", step, T)):
+                self._attend_by_heads(q, out, gate, step, cache, group, cos, sin)
+        if done < T:
+            self._onto_latent(q, out, gate, step, cache, group, cos, sin, done)
         with profiling.label("o_proj", lambda: self.cost("o_proj", step, T)):
-            out = torch.empty((T, H * Dv), dtype=x.dtype, device=x.device)
-            gate = low[:, self.gate_at:] if self.output_gate else None
-            if ops.heads_matmul_mfma_takes(latent, Lk, self.uv_nt):
-                ops.heads_matmul_mfma(latent, Lk, self.uv_nt, out, Dv, gate=gate)
-            else:
-                ops.heads_matmul(latent, Lk, self.uv, out, Dv, gate=gate)
             return self.o.forward(out)
+
+    def _onto_latent(self, q, out, gate, step: StepContext, cache: KVCacheView, group, cos, sin, first: int) -> None:
+        """Rows ``first`` and up of ``out``, gated: the queries moved onto the latent, the attention over it, its result onto the values."""
+        T, H, Dn, Dr, Dv, Lk, row = q.shape[0], self.num_heads, self.head_dim, self.rot_dim, self.v_head_dim, self.kv_rank, self.row
+        half = self.half_pairs
+        qa = torch.empty((T, H * row), dtype=q.dtype, device=q.device)
+        latent = torch.empty((T, H * Lk), dtype=q.dtype, device=q.device)
+        q1, qa1, latent1, out1, positions = q[first:], qa[first:], latent[first:], out[first:], step.positions[first:]
+        with profiling.label("qkv", lambda: self.cost("qkv", step, T)):
+            if self.uk_nt is not None and ops.heads_matmul_mfma_takes(q1, Dn + Dr, self.uk_nt):
+                # the heads' rotated channels go beside their part on the latent in the same launch
+                ops.heads_matmul_mfma(q1, Dn + Dr, self.uk_nt, qa1, row, tail=Dr, cos=cos, sin=sin, positions=positions, half_pairs=half)
+            else:
+                ops.heads_matmul(q1, Dn + Dr, self.uk, qa1, row)
+                if Dr:
+                    ops.rotate_heads(q1[:, Dn:], Dn + Dr, qa1[:, Lk:], row, H, Dr, cos, sin, positions, half_pairs=half)
+        with profiling.label("attention", lambda: self.cost("attention", step, T)):
+            self._attend(qa, latent, step, cache, group, singles_only=first > 0)
+        with profiling.label("o_proj", lambda: self.cost("o_proj", step, T)):
+            gate1 = gate[first:] if gate is not None else None
+            if ops.heads_matmul_mfma_takes(latent1, Lk, self.uv_nt):
+                ops.heads_matmul_mfma(latent1, Lk, self.uv_nt, out1, Dv, gate=gate1)
+            else:
+                ops.heads_matmul(latent1, Lk, self.uv, out1, Dv, gate=gate1)

@@ -119,6 +119,37 @@ class StepContext:
     # the q_len > 1 entries cut into tiles of at most 16 tokens: int32 [n, 4] =
     # (request index, first row, tokens, position of the first token)
     prefill_tiles: torch.Tensor | None = None
+    # do q_lens and start_positions hold whenever a step of this layout runs? (a step that a graph may replay is laid out once for many
+    # requests: kernels and buffers must not be sized by them)
+    portions_known: bool = False
+
+
+def portion_blocks(step: StepContext, window: int, device):
+    """The step's portions for a kernel that takes blocks of 64 queries of one portion beside its visible rows gathered in order:
+    (blocks int32 [n, 4] on the device = (first row, queries, position of the first, gathered row of position 0), those with the most keys
+    first; a portion's gathered rows as (request, position of its first row, rows, oldest and newest position in the cache, first row);
+    all gathered rows). Positions are gathered in whole blocks of 64. Made once per step and window and shared by the step's layers."""
+    made = getattr(step, "_portion_blocks", None)
+    if made is None:
+        made = step._portion_blocks = {}
+    if window not in made:
+        blocks, gathers, rows, row = [], [], 0, 0
+        for s in range(step.num_seqs - step.num_decode):
+            start, n = step.start_positions[s], step.q_lens[s]
+            lo = max(0, start - window + 1) if window else 0
+            first = lo // 64 * 64
+            count = -(-(start + n) // 64) * 64 - first
+            gathers.append((s, first, count, lo, start + n - 1, rows))
+            for at in range(0, n, 64):
+                pos, m = start + at, min(64, n - at)
+                blocks.append((pos + m - (max(0, pos - window + 1) if window else 0), (row + at, m, pos, rows - first)))
+            rows += count
+            row += n
+        if row != step.num_tokens - step.num_decode:
+            raise ValueError("the step's portions do not cover its rows")
+        blocks.sort(key=lambda b: -b[0])
+        made[window] = torch.tensor([b for _, b in blocks], dtype=torch.int32, pin_memory=True).to(device, non_blocking=True), gathers, rows
+    return made[window]
 
 
 def step_segments(step: StepContext, size: int, device, portions_only: bool = False):
