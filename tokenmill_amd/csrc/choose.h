@@ -48,6 +48,13 @@ constexpr int TM_TILE_FEW_COLUMNS = 64 * 256;
 inline int tm_split_rows(int hidden) { return hidden < 3072 ? TM_SKINNY_ROWS : hidden <= 4096 ? 4 : TM_STREAM_ROWS; }
 // (what that does not take, such as a projection with a bias, is streamed where splitting its K over groups of blocks pays:
 // tm_stream_linear_parts in gemm_stream.hip; else it is the library's)
+// Plain products of prompts that run tiled in place of the library's untimed choice: where the tiles met or beat it (cold matrices, library /
+// tiled, 300 / 600 / 1,000 / 1,500 / 2,048 / 3,001 rows, us: 2,048 -> 2,048 10.9 / 13.7 / 15.5 / 19.0 / 21.1 / 26.1 to 9.4 / 12.3 / 13.4 / 17.5 /
+// 19.2 / 25.6; 1,024 -> 1,024 6.4 / 8.7 / 9.0 / 9.8 / 10.5 / 11.7 to 5.8 / 6.1 / 6.1 / 8.8 / 8.1 / 11.3; 4,096 -> 1,024 13.4 / 17.5 / 18.3 / 21.4 /
+// 25.4 / 28.3 to 13.8 / 14.7 / 14.8 / 20.9 / 21.9 / 28.4; 3,584 -> 3,584 19.5 / 26.5 / 30.7 / 38.5 / 46.8 / 70.7 to 18.0 / 24.7 / 27.1 / 37.6 / 44.5 /
+// 61.0), and a call of it costs the host half. Beyond them the library is up to 10% better at some sizes: 2,048 -> 8,192 43.5 to 45.0 and 49.2
+// to 52.7 at 1,500 and 2,048 rows, 768 -> 3,072 12.5 to 13.2 and 14.3 to 15.8, 8,192 -> 2,048 level, 4,864 -> 896 24.6 to 28.2 at 1,500.
+inline bool tm_tile_plain(int M, int N, int K) { return M >= 256 && M <= 3072 && N >= 512 && N <= 4096 && K >= 1024 && K <= 4096; }
 // most rows one launch of the skinny product takes at all
 constexpr int TM_SKINNY_MAX_ROWS = 64;
 // most rows the 32-bit matrix-vector product takes

@@ -178,6 +178,10 @@ struct Products {
         }
         if (skinny && M <= TM_SKINNY_ROWS)
             return tm_gemm_skinny(x, ldx, L.w, L.bias, L.bias_dtype, out, ldc, M, L.N, L.K, out_dtype, ep, nullptr, 0, stream);
+        // (a program that times the library's candidates keeps the library's)
+        if (!L.bias && !L.library_first && tune.candidates < 2 && tm_tile_plain(M, L.N, L.K) && tile_ok(L, x, ldx, M, dtype) && aligned(out, 16) &&
+            ldc % 8 == 0 && (out_dtype == TM_BF16 || ldc == L.N))
+            return tm_tile_linear(x, ldx, M, L.K, L.w, L.N, out, ldc, out_dtype, stream);
         {
             const int rc = library(L, x, ldx, M, out, ldc, out_dtype);
             if (rc != TM_ERR_UNSUPPORTED) return then_act(rc);
