@@ -1,0 +1,62 @@
+"""The 32-bit attention of prompt portions where its weights' reference moves rarely, often and not at all, and over grids of one to
+several rounds of the chip."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from tokenmill_amd.hip import ops as o
+    return o
+
+
+def attend(ops, q, k, v, H, KVH, D, page, scale):
+    n = q.shape[0]
+    pages = -(-n // page)
+    kp, vp = torch.zeros(pages * page, KVH, D, device=DEV), torch.zeros(pages * page, KVH, D, device=DEV)
+    kp[:n], vp[:n] = k, v
+    tiles = torch.tensor([(0, j, min(16, n - j), j) for j in reversed(range(0, n, 16))], dtype=torch.int32, device=DEV)
+    out = torch.full((n, H * D), 3.0, device=DEV)
+    ops.attn_prefill_f32(q.reshape(n, H * D).contiguous(), out, kp.view(pages, page, KVH, D),
+                         vp.view(pages, page, KVH, D).permute(0, 2, 3, 1).contiguous(),
+                         torch.arange(pages, dtype=torch.int32, device=DEV).view(1, -1), tiles, H, KVH, D, scale, 0)
+    return out.view(n, H, D)
+
+
+@pytest.mark.parametrize("D", [16, 64, 128])
+@pytest.mark.parametrize("step", [0.0, 0.05, 0.49, 3.0, -0.3, -8.0])     # how much a key's score exceeds the one before it
+@pytest.mark.parametrize("n,H", [(17, 1), (300, 14), (300, 30)])
+def test_moving_reference(ops, D, step, n, H):
+    torch.manual_seed(n + D)
+    q, k, v = (torch.randn(n, h, D, device=DEV) for h in (H, 1, 1))
+    q[..., 0], k[..., 0] = D ** 0.5, step * torch.arange(n, device=DEV)[:, None]
+    got = attend(ops, q, k, v, H, 1, D, 16, D ** -0.5)
+    s = torch.einsum("qhd,kd->hqk", q.double().cpu(), k[:, 0].double().cpu()) * D ** -0.5
+    top = s.abs().max()
+    s = s.masked_fill(torch.ones(n, n).triu(1).bool(), float("-inf"))
+    want = torch.einsum("hqk,kd->qhd", s.softmax(-1), v[:, 0].double().cpu())
+    # a score of magnitude S is the running sum of D products that round by up to 2^-24 S each, at random (deviation 2^-24 S / 3^0.5):
+    # the difference of two scores is off by at most 5 deviations of 2 D of them, 2^-24 S 4.1 D^0.5, and a result by
+    # a quarter of that times the distance of two values, below 8; weights and their sums add 2e-6
+    bound = 2 ** -24 * top * 4.1 * D ** 0.5 * 2 + 2e-6
+    assert (got.cpu() - want).abs().max() < bound
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_no_number_reaches_those_that_see_it(ops, bad):
+    torch.manual_seed(1)
+    n, H, D = 100, 2, 64
+    q, k, v = (torch.randn(n, h, D, device=DEV) for h in (H, 1, 1))
+    q[..., 0] = q[..., 0].abs() + 1
+    k[70, 0, 0] = bad
+    got = attend(ops, q, k, v, H, 1, D, 16, D ** -0.5)
+    assert got[:70].isfinite().all() and not got[70:].isfinite().any()
+    k[70, 0, 0] = float("-inf")                                          # a key of weight zero
+    got = attend(ops, q, k, v, H, 1, D, 16, D ** -0.5)
+    k[70, 0, 0] = -1e6
+    assert torch.equal(got, attend(ops, q, k, v, H, 1, D, 16, D ** -0.5))

@@ -10,7 +10,11 @@
 //   Which wavefront takes a key block hangs on the key's position only, so a token's result depends
 //   on its request only. The longest tile of a 2,048-token prompt walks 32 key blocks a wavefront
 //   instead of 128; the heads of a kv head run in blocks of their own and share its keys through the
-//   second-level cache.
+//   second-level cache (two heads a wavefront were no faster).
+//   The matrix instructions of a 1,000-token prompt of the 0.5B shape (14 heads of 64) take 12 us a layer. What stood beside them: the newest
+//   tiles' blocks met on the same CUs (52 us; 38 dealt out as below), accumulators that the vector unit had to fetch back and a
+//   branch for a cap (35), and sums rescaled at every block, expf, loads without a scalar base (29). The next block's keys and
+//   values are on their way while a block is multiplied.
 //
 //   S^T = K Q^T   A = keys  [16 keys x 4 d]   B = Q^T [4 d x 16 tokens]   (D / 4 steps; which d a step
 //                 multiplies is free as long as keys and queries agree: the lanes of group g = lane / 16
@@ -21,24 +25,45 @@
 //                 (register i of the same lane) and what one 16-byte load of V[d][4 g .. 4 g + 3] gives.
 #include "common.h"
 #include "api.h"
-
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
+#include "fused_common.h"
 
 #define AF_SPLIT 4          // wavefronts of a block; each takes every fourth key block
+#define AF_ROUND 256        // blocks that come to rest on CUs of their own before the first CU gets a second one
 
+// A column's reference moves only when its maximum has grown by more than this (weights up to e^8 cost 32-bit sums nothing), so
+// most blocks rescale no sums.
+#define AF_GROWTH 8.f
+
+// e^x for x <= AF_GROWTH: two to the rounded x log2(e), corrected by what the rounding left out (6 instructions where expf takes 13,
+// that also look after arguments that cannot come here)
+__device__ __forceinline__ float exp_weight(float x) {
+    const float p = x * 1.44269504f, e = __builtin_amdgcn_exp2f(p);
+    const float left = __builtin_fmaf(p, -1.90465421e-9f, __builtin_fmaf(p, -0.693147182f, x));
+    return p < -150.f ? 0.f : __builtin_fmaf(e, left, e);           // (-inf, a key not to be seen: 0)
+}
+
+// What a wavefront loads of a block of 16 keys.
 template <int D>
-__global__ __launch_bounds__(64 * AF_SPLIT) void attn_prefill_f32_kernel(
+struct KVBlock32 {
+    f32x4_t k[D / 16], v[D / 16];
+};
+
+template <int D, bool CAP>
+__global__ __launch_bounds__(64 * AF_SPLIT, 2) void attn_prefill_f32_kernel(
     const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
     const float* __restrict__ k_pool, const float* __restrict__ v_pool, const int* __restrict__ block_tables,
     int table_width, const int* __restrict__ tiles, int H, int KVH, int page_shift, float scale, int window, int keep, float softcap,
     const float* __restrict__ sink, const float* __restrict__ cgate, int ldcg) {
-    constexpr int DQ = D / 4;           // values of a key (or query) a lane holds
     constexpr int NDT = D / 16;         // 16-row tiles of d
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE);
     const int lane = threadIdx.x % TM_WAVE, r = lane % 16, g = lane / 16;
-    const int h = blockIdx.y;
-    const int kvh = h / (H / KVH);
-    const int* tl = tiles + (size_t)blockIdx.x * 4;
+    // The newest tile walks the most keys, and a prompt's blocks are mostly all on the chip at once, so it is where they lie that balances
+    // them: the tiles (newest first) go over the CUs, and in every second round of the CUs the other way round.
+    const int round = blockIdx.x / AF_ROUND, in_round = blockIdx.x % AF_ROUND;
+    const int left = (int)gridDim.x - round * AF_ROUND, items = left < AF_ROUND ? left : AF_ROUND;
+    const int item = round * AF_ROUND + (round & 1 ? items - 1 - in_round : in_round);
+    const int tile = item / H, h = item % H, kvh = h / (H / KVH);
+    const int* tl = tiles + (size_t)tile * 4;
     const int s = tl[0], row0 = tl[1], valid = tl[2], pos0 = tl[3];
     const int* table = block_tables + (size_t)s * table_width;
     const int page = 1 << page_shift;
@@ -48,14 +73,12 @@ __global__ __launch_bounds__(64 * AF_SPLIT) void attn_prefill_f32_kernel(
     const int first_key = (window > 0 && pos0 - window + 1 > 0) ? pos0 - window + 1 : 0;
     const int last_lo = (window > 0 && last_key - window + 1 > 0) ? last_key - window + 1 : 0;
 
-    float qf[DQ];
+    // (columns beyond the tile's tokens: its last one again, not stored)
+    const float* qrow = q + (size_t)(row0 + (r < valid ? r : valid - 1)) * q_stride + (size_t)h * D + 4 * g;
+    f32x4_t qf[NDT];
 #pragma unroll
-    for (int c = 0; c < DQ; c += 4) {
-        f32x4_t t = {0.f, 0.f, 0.f, 0.f};
-        if (r < valid) t = *(const f32x4_t*)(q + (size_t)(row0 + r) * q_stride + (size_t)h * D + 4 * c + 4 * g);
-        qf[c] = t[0]; qf[c + 1] = t[1]; qf[c + 2] = t[2]; qf[c + 3] = t[3];
-    }
-    float m = -INFINITY, l = 0.f;       // running maximum of the scaled scores of this lane's column; this lane's share of the sum
+    for (int c = 0; c < NDT; ++c) qf[c] = *(const f32x4_t*)(qrow + 16 * c);
+    float m = -3.402823466e38f, l = 0.f; // the reference of the weights of this lane's column; this lane's share of their sum
     f32x4_t o[NDT];
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -64,116 +87,130 @@ __global__ __launch_bounds__(64 * AF_SPLIT) void attn_prefill_f32_kernel(
     const int kb_first = first_key >> 4, kb_last = last_key >> 4;
     const int kb_kept = keep > 0 && first_key > 0 ? (keep + 15) >> 4 : 0;
     auto behind_gap = [&](int b) { return (b >= kb_kept && b < kb_first) ? kb_first + ((wave - kb_first) & (AF_SPLIT - 1)) : b; };
-    int kb = behind_gap(wave);
-    // a key block's page id is asked for one block ahead (always at an entry this tile may see)
-    int pg_next = table[((kb <= kb_last ? kb : kb_last) << 4) >> page_shift];
-    for (int next; kb <= kb_last; kb = next) {
+    // (behind the wavefront's last block the newest one there is again, unused: always at an entry this tile may see)
+    auto page_of = [&](int b) { return table[((b <= kb_last ? b : kb_last) << 4) >> page_shift]; };
+    const uint32_t k_lane = ((uint32_t)r * KVH * D + 4 * g) * 4, v_lane = (((uint32_t)r << page_shift) + 4 * g) * 4;
+    auto load = [&](KVBlock32<D>& blk, int b, int pg) {
+        const int in_page = ((b <= kb_last ? b : kb_last) << 4) & (page - 1);
+        // keys: lane (r, g) holds K[key0 + r][16 c + 4 g .. + 3]; values: V[d = 16 dt + r][key0 + 4 g .. + 3]
+        // (the page's and the key's place by the scalar unit, a lane's own place in them all along the same)
+        const auto kr = fd_buffer(k_pool + ((((size_t)pg << page_shift) + in_page) * KVH + kvh) * D, 0x7fffffff);
+        const auto vr = fd_buffer(v_pool + ((((size_t)pg * KVH + kvh) * D) << page_shift) + in_page, 0x7fffffff);
+#pragma unroll
+        for (int c = 0; c < NDT; ++c) blk.k[c] = as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(kr, k_lane + 64 * c, 0, 0));
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) blk.v[dt] = as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(vr, v_lane, (64 * dt) << page_shift, 0));
+    };
+    int kb = behind_gap(wave), next = behind_gap(kb + AF_SPLIT);
+    int pg_next = page_of(next);
+    auto attend = [&](KVBlock32<D>& now, KVBlock32<D>& then) {
         const int key0 = kb << 4;
-        const int pg = pg_next;
-        next = behind_gap(kb + AF_SPLIT);
-        pg_next = table[((next <= kb_last ? next : kb) << 4) >> page_shift];
-        const int in_page = key0 & (page - 1);
-        // keys: lane (r, g) holds K[key0 + r][16 c + 4 g .. + 3], c = 0 .. D/16 - 1
-        const float* kr = k_pool + ((((size_t)pg << page_shift) + in_page + r) * KVH + kvh) * D + 4 * g;
-        float kf[DQ];
-#pragma unroll
-        for (int c = 0; c < DQ; c += 4) {
-            const f32x4_t t = *(const f32x4_t*)(kr + 4 * c);
-            kf[c] = t[0]; kf[c + 1] = t[1]; kf[c + 2] = t[2]; kf[c + 3] = t[3];
-        }
-        // values: lane (r, g) holds V[d = 16 dt + r][key0 + 4 g .. + 3]
-        const float* vr = v_pool + ((((size_t)pg * KVH + kvh) * D + r) << page_shift) + in_page + 4 * g;
-        f32x4_t vf[NDT];
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) vf[dt] = *(const f32x4_t*)(vr + ((size_t)(16 * dt) << page_shift));
+        const int after = behind_gap(next + AF_SPLIT);
+        load(then, next, pg_next);                      // the next block, and the page of the one behind it
+        pg_next = page_of(after);
+        __builtin_amdgcn_sched_barrier(0);
         // values of keys nobody may see yet (beyond the newest key) can hold anything: clear them
         if (key0 + 15 > last_key) {
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (key0 + 4 * g + i > last_key) vf[dt][i] = 0.f;
+                    if (key0 + 4 * g + i > last_key) now.v[dt][i] = 0.f;
         }
         f32x4_t sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < DQ; ++c) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c], qf[c], sc, 0, 0, 0);
+        for (int c = 0; c < NDT; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[c][e], qf[c][e], sc, 0, 0, 0);
         // sc[i] = score of key key0 + 4 g + i for this lane's token
-        const bool edge = (key0 + 15 > pos0) || (key0 < last_lo);
+        bool hidden[4] = {false, false, false, false};
+        if (key0 + 15 > pos0 || key0 < last_lo)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int kj = key0 + 4 * g + i;
+                hidden[i] = kj > my_pos || (kj < my_lo && kj >= keep);
+            }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             sc[i] *= scale;
-            if (softcap > 0.f) sc[i] = softcap * tanhf(sc[i] / softcap);
-            if (edge) {
-                const int kj = key0 + 4 * g + i;
-                if (kj > my_pos || (kj < my_lo && kj >= keep)) sc[i] = -INFINITY;
-            }
+            if (CAP) sc[i] = softcap * tanhf(sc[i] / softcap);
+            sc[i] = hidden[i] ? -INFINITY : sc[i];
         }
         float bm = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
         bm = lane_max<16>(bm);
         bm = lane_max<32>(bm);
-        const float m_new = fmaxf(m, bm);
-        // a column that has seen no key yet keeps m = -inf; its weights and its correction are zeros
-        // (every lane stays in step: the matrix instructions below are wave-wide)
-        const float m_ref = (m_new == -INFINITY) ? 0.f : m_new;
-        const float corr = expf(m - m_ref);                 // exp(-inf) = 0 on the column's first visible block
-        m = m_new;
-        l *= corr;
+        // (a column that has seen no key yet keeps the lowest number: -inf scores less that are -inf, their weights zeros. Whether a
+        // column's reference moves hangs on that column alone)
+        const bool grew = bm > m + AF_GROWTH;
+        if (__builtin_expect(__any(grew), 0)) {
+            const float corr = grew ? exp_weight(m - bm) : 1.f;
+            m = grew ? bm : m;
+            l *= corr;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[dt][i] *= corr;
+        }
         f32x4_t pr;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            pr[i] = expf(sc[i] - m_ref);
+            pr[i] = exp_weight(sc[i] - m);
             l += pr[i];
         }
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[dt][i] *= corr;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[dt][i], pr[i], o[dt], 0, 0, 0);
-        }
+            for (int dt = 0; dt < NDT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.v[dt][i], pr[i], o[dt], 0, 0, 0);
+        kb = next;
+        next = after;
+    };
+    KVBlock32<D> ba, bb;
+    load(ba, kb, page_of(kb));
+    while (kb <= kb_last) {
+        attend(ba, bb);
+        if (kb > kb_last) break;
+        attend(bb, ba);
     }
-    // o[dt][i] = sum for d = 16 dt + 4 g + i of token r; the column's sum is spread over its four lanes
-    l = lane_sum<16>(l);
-    l = lane_sum<32>(l);
-    // the four wavefronts' partial results meet in LDS; a wavefront that had no key block brings m = -inf, l = 0, o = 0
+    // o[dt][i] = sum for d = 16 dt + 4 g + i of token r; the column's sum is spread over its four lanes.
+    // The four wavefronts' partial results meet in LDS; a wavefront that had no key block brings the lowest number as its reference, l = 0, o = 0
     __shared__ float m_s[AF_SPLIT][16], l_s[AF_SPLIT][16];
     __shared__ __attribute__((aligned(16))) float o_s[AF_SPLIT][16][D + 4];
+    const float own = lane_sum<32>(lane_sum<16>(l));
     if (g == 0) {
         m_s[wave][r] = m;
-        l_s[wave][r] = l;
+        l_s[wave][r] = own;
     }
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) *(f32x4_t*)&o_s[wave][r][16 * dt + 4 * g] = o[dt];
     __syncthreads();
     const int tok = threadIdx.x >> 4;
-    if (tok < valid) {
-        float mw[AF_SPLIT], sw[AF_SPLIT], top = -INFINITY, sum = 0.f;
+    if (tok >= valid) return;
+    float mw[AF_SPLIT], sw[AF_SPLIT], top = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < AF_SPLIT; ++w) {
+        mw[w] = m_s[w][tok];
+        top = fmaxf(top, mw[w]);
+    }
+#pragma unroll
+    for (int w = 0; w < AF_SPLIT; ++w) {
+        sw[w] = expf(mw[w] - top);                                      // a token always sees its own key: top is finite
+        sum += l_s[w][tok] * sw[w];
+    }
+    if (sink) sum += expf(sink[h] - top);                                 // a term of the denominator without a key
+    const float inv = 1.f / sum;
+    float* orow = out + (size_t)(row0 + tok) * out_stride + (size_t)h * D;
+    for (int d = (threadIdx.x & 15) * 4; d < D; d += 64) {
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < AF_SPLIT; ++w) {
-            mw[w] = m_s[w][tok];
-            top = fmaxf(top, mw[w]);
+            const f32x4_t part = *(const f32x4_t*)&o_s[w][tok][d];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] += part[i] * sw[w];
         }
+        if (cgate)                                                      // a gate per channel
 #pragma unroll
-        for (int w = 0; w < AF_SPLIT; ++w) {
-            sw[w] = (mw[w] == -INFINITY) ? 0.f : expf(mw[w] - top);     // a token always sees its own key: top is finite
-            sum += l_s[w][tok] * sw[w];
-        }
-        if (sink) sum += expf(sink[h] - top);                             // a term of the denominator without a key
-        const float inv = 1.f / sum;
-        float* orow = out + (size_t)(row0 + tok) * out_stride + (size_t)h * D;
-        for (int d = (threadIdx.x & 15) * 4; d < D; d += 64) {
-            f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int w = 0; w < AF_SPLIT; ++w) {
-                const f32x4_t part = *(const f32x4_t*)&o_s[w][tok][d];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[i] += part[i] * sw[w];
-            }
-            if (cgate)                                                  // a gate per channel
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[i] *= 1.f / (1.f + expf(-cgate[(size_t)(row0 + tok) * ldcg + (size_t)h * D + d + i]));
-            *(f32x4_t*)(orow + d) = f32x4_t{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
-        }
+            for (int i = 0; i < 4; ++i) acc[i] *= 1.f / (1.f + expf(-cgate[(size_t)(row0 + tok) * ldcg + (size_t)h * D + d + i]));
+        *(f32x4_t*)(orow + d) = f32x4_t{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
     }
 }
 
@@ -197,12 +234,15 @@ extern "C" int tm_attn_prefill_f32_cap(const void* q, int q_stride, void* out, i
     if (H > 65535) return TM_ERR_ARG;
     int page_shift = 0;
     while ((1 << page_shift) < page) ++page_shift;
-    dim3 grid(n_tiles, H);
+    const unsigned grid = n_tiles * H;
+#define TM_PREFILL_F32_GO(DD, CAP)                                                                                \
+    attn_prefill_f32_kernel<DD, CAP><<<grid, 64 * AF_SPLIT, 0, stream>>>(                                         \
+        (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pool, (const float*)v_pool,           \
+        block_tables, table_width, tiles, H, KVH, page_shift, scale, window, keep, softcap, sink, (const float*)cgate, ldcg)
 #define TM_PREFILL_F32_CASE(DD)                                                                                   \
     case DD:                                                                                                      \
-        attn_prefill_f32_kernel<DD><<<grid, 64 * AF_SPLIT, 0, stream>>>(                                          \
-            (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pool, (const float*)v_pool,       \
-            block_tables, table_width, tiles, H, KVH, page_shift, scale, window, keep, softcap, sink, (const float*)cgate, ldcg); \
+        if (softcap > 0.f) TM_PREFILL_F32_GO(DD, true);                                                           \
+        else TM_PREFILL_F32_GO(DD, false);                                                                        \
         break
     switch (D) {
         TM_PREFILL_F32_CASE(16);
@@ -217,6 +257,7 @@ extern "C" int tm_attn_prefill_f32_cap(const void* q, int q_stride, void* out, i
             return TM_ERR_ARG;
     }
 #undef TM_PREFILL_F32_CASE
+#undef TM_PREFILL_F32_GO
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
