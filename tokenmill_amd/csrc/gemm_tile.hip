@@ -36,6 +36,7 @@ struct TileArgs {
     int I;                      // SiLU: columns of the result
     // q|k|v
     int H, KVH, D, page_shift;
+    uint32_t head_inverse;      // gt_inverse(D / 64): a unit's head without a division, some thirty instructions in front of the first load
     const float* cos_t;         // [positions, D / 2]
     const float* sin_t;
     const int* positions;       // [M]
@@ -104,6 +105,15 @@ __device__ __forceinline__ void gt_wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
 
+// ... until those of at most `left` steps (and MOST), NL a step, are on their way
+template <int MOST, int NL>
+__device__ __forceinline__ void gt_wait_steps(int left) {
+    if constexpr (MOST > 0) {
+        if (left < MOST) return gt_wait_steps<MOST - 1, NL>(left);
+    }
+    gt_wait_loads<MOST * NL>();
+}
+
 // Tile p of the launch. The blocks of one XCD (b % 8) walk a run of neighbouring tiles, `band` row tiles of a column tile first,
 // so that what an XCD's blocks read at a time overlaps in its L2. False: no further tile.
 template <bool GROUPED>
@@ -145,6 +155,9 @@ __device__ __forceinline__ bool gt_next(const TileArgs& a, int BM, int& p, GtPla
     return false;
 }
 
+// q|k|v: the head of unit u, u / (D / 64)
+__device__ __forceinline__ int gt_head(const TileArgs& a, int u) { return (int)__umulhi((uint32_t)(2 * u + 1), a.head_inverse); }
+
 // the matrix row that row q of unit u holds
 template <int EPI>
 __device__ __forceinline__ int gt_matrix_row(const TileArgs& a, int u, int q) {
@@ -156,7 +169,7 @@ __device__ __forceinline__ int gt_matrix_row(const TileArgs& a, int u, int q) {
         return n;
     }
     if (EPI == GT_QKV) {
-        const int per_head = a.D / 64, head = u / per_head;
+        const int per_head = a.D / 64, head = gt_head(a, u);
         n = head * a.D + 32 * (u - head * per_head) + (q & 31) + (q >= 32 ? a.D / 2 : 0);
     } else {
         n = 64 * u + q;
@@ -170,6 +183,11 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     extern __shared__ __align__(16) unsigned char gt_smem[];
     constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, ROWS = BM + BN;
     constexpr bool GROUPED = EPI >= GT_EXPERT_SILU, GATED = EPI == GT_SILU || EPI == GT_EXPERT_SILU || EPI == GT_EXPERT_CLAMPED;
+    // Behind a block's last tile there is nothing to load. Tiles of a middle size load nothing then; the others load the same bytes
+    // again, which keeps one loop and its waits: the smallest are bound by the length of a step and by their code's way into the CU (with
+    // a second loop 896 -> 896 at 77 rows 4.1 to 4.3 us), the largest have no register left for it. What it gives the middle ones, 896 wide,
+    // 2,048 rows: gate|up 40.6 to 40.2 us, down 27.8 to 27.5, o level.
+    constexpr bool QUIET = sizeof(T) == 2 && MT >= 2 && MT <= 5;
     constexpr int STAGE = ROWS * 128, NL = ROWS / 32;               // bytes of a buffer; loads a wavefront makes for it
     static_assert(BM % 32 == 0 && BN % 64 == 0 && NT % 4 == 0, "");
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)gt_smem;
@@ -187,10 +205,12 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     bool l_more = true;
     auto next_load_tile = [&]() {
         GtPlace at_;
-        if (!l_more || !gt_next<GROUPED>(a, BM, l_p, at_)) {             // no further tile: the same bytes again, never multiplied
+        if (!l_more || !gt_next<GROUPED>(a, BM, l_p, at_)) {             // no further tile: nothing, or the same bytes again, never multiplied
             l_more = false;
-            lA = (const unsigned char*)a.A;
-            lW = (const unsigned char*)a.W;
+            if constexpr (!QUIET) {
+                lA = (const unsigned char*)a.A;
+                lW = (const unsigned char*)a.W;
+            }
             return;
         }
         l_p += gridDim.x;
@@ -215,8 +235,8 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     };
     auto issue_one = [&](uint32_t dst, int i) { fd_load_lds(dst + i * 4096, voff[i], i < BM / 32 ? (const void*)lA : (const void*)lW); };
     auto issued = [&]() {
-        lA += l_more ? 128 : 0;
-        lW += l_more ? 128 : 0;
+        lA += QUIET || l_more ? 128 : 0;
+        lW += QUIET || l_more ? 128 : 0;
     };
 
     // --- the multiplying side ---
@@ -320,29 +340,62 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                 slot[i] = a.slots ? a.slots[m < a.M ? m : a.M - 1] : -1;
             }
         };
+        constexpr int UNITS = NT / 4;
+        constexpr bool BIAS_EARLY = EPI == GT_QKV && MT <= 5 && UNITS == 1;
+        u32x4_t bias0[UNITS], bias1[UNITS], bias2[UNITS], bias3[UNITS];     // eight and eight values: 32-bit, or bfloat16 in bias0 and bias2
+        auto read_bias = [&](int un) {
+            const int u = at_.tn * (BN / 64) + wn * UNITS + un, head = gt_head(a, u);
+            const int c = head * a.D + 32 * (u - head * (a.D / 64)) + 8 * g, at = c + a.D / 2 < a.N ? c : 0;
+            const size_t size = a.bias_f32 ? 4 : 2;
+            const unsigned char *lo = (const unsigned char*)a.bias + at * size, *hi = lo + a.D / 2 * size;
+            bias0[un] = bias1[un] = bias2[un] = bias3[un] = u32x4_t{0, 0, 0, 0};
+            if (a.bias) {
+                bias0[un] = *(const u32x4_t*)lo;
+                bias2[un] = *(const u32x4_t*)hi;
+                if (a.bias_f32) {
+                    bias1[un] = *(const u32x4_t*)(lo + 16);
+                    bias3[un] = *(const u32x4_t*)(hi + 16);
+                }
+            }
+        };
         if constexpr (EPI == GT_QKV && MT <= 5) read_places();
+        // (marks of the clock inside the kernel: the bias, asked for at the end and cold, took 1,800 to 2,800 of a tile's 15,000 to 33,000 cycles in
+        // front of the rotary rows' trip. With it here and a unit's head found without a division, 896 -> 1,152 at 77 / 544 / 2,048
+        // rows 8.3 / 8.8 / 16.5 to 7.8 / 8.2 / 14.6 us)
+        if constexpr (BIAS_EARLY) read_bias(0);
         int block = 0;
         // the loads are ST steps ahead: those of the last ST steps are the next tile's
+        auto step = [&](auto LOADS, int left) {                     // left (without loads): this tile's steps from here on
+            half_step(std::integral_constant<int, 0>{}, buf, std::false_type{}, 0u);
+            // the next step's rows have arrived (this wavefront's, then everybody's), and this step's have been read
+            if constexpr (decltype(LOADS)::value) gt_wait_loads<(ST - 2) * NL>();
+            else gt_wait_steps<ST - 2, NL>(left - 2);
+            __builtin_amdgcn_s_barrier();
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + wave * 1024);
+            buf = buf + 1 == ST ? 0 : buf + 1;
+            asm volatile("" ::: "memory");
+            half_step(std::integral_constant<int, 1>{}, buf, LOADS, dst);
+            if constexpr (decltype(LOADS)::value) issued();
+            if constexpr (ES == 4) {
+                if (++block == joins) {
+                    block = 0;
+                    join();
+                }
+            }
+        };
 #pragma unroll 1
         for (int part = 0; part < 2; ++part) {
-            if (part) next_load_tile();
+            if (part) {
+                next_load_tile();
+                if (QUIET && !l_more) break;
+            }
 #pragma unroll 1
-            for (int s = part ? ST : steps - ST; s > 0; --s) {
-                half_step(std::integral_constant<int, 0>{}, buf, std::false_type{}, 0u);
-                // the next step's rows have arrived (this wavefront's, then everybody's), and this step's have been read
-                gt_wait_loads<(ST - 2) * NL>();
-                __builtin_amdgcn_s_barrier();
-                const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + wave * 1024);
-                buf = buf + 1 == ST ? 0 : buf + 1;
-                asm volatile("" ::: "memory");
-                half_step(std::integral_constant<int, 1>{}, buf, std::true_type{}, dst);
-                issued();
-                if constexpr (ES == 4) {
-                    if (++block == joins) {
-                        block = 0;
-                        join();
-                    }
-                }
+            for (int s = part ? ST : steps - ST; s > 0; --s) step(std::true_type{}, 0);
+        }
+        if constexpr (QUIET) {
+            if (!l_more) {
+#pragma unroll 1
+                for (int s = ST; s > 0; --s) step(std::false_type{}, s);
             }
         }
         // --- the tile's results ---
@@ -360,7 +413,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                 ok0 = ok1 = c0 < a.I;
             } else if (EPI == GT_QKV) {
                 const int per_head = a.D / 64;
-                head = u / per_head;
+                head = gt_head(a, u);
                 d0 = 32 * (u - head * per_head) + 8 * g;
                 c0 = head * a.D + d0;
                 c1 = c0 + a.D / 2;
@@ -375,19 +428,15 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
             constexpr int AHEAD = EPI != GT_QKV ? 1 : MT <= 5 ? MT : 4;
             f32x4_t bias[4], cs[AHEAD][2], sn[AHEAD][2];
             if constexpr (EPI == GT_QKV) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int at = (ok0 ? (e < 2 ? c0 : c1) : 0) + 4 * (e & 1);
-                    bias[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-                    if (!a.bias) continue;
-                    if (a.bias_f32) {
-                        bias[e] = *(const f32x4_t*)((const float*)a.bias + at);
-                    } else {
-                        const uint2 u = *(const uint2*)((const bf16_t*)a.bias + at);
-                        bias[e] = f32x4_t{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                                          __uint_as_float(u.y & 0xffff0000u)};
-                    }
-                }
+                if constexpr (!BIAS_EARLY) read_bias(un);
+                auto widen = [](uint32_t lo, uint32_t hi) {
+                    return f32x4_t{__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u)};
+                };
+                const u32x4_t lo = bias0[un], hi = bias2[un];
+                bias[0] = a.bias_f32 ? as_f32x4(lo) : widen(lo[0], lo[1]);
+                bias[1] = a.bias_f32 ? as_f32x4(bias1[un]) : widen(lo[2], lo[3]);
+                bias[2] = a.bias_f32 ? as_f32x4(hi) : widen(hi[0], hi[1]);
+                bias[3] = a.bias_f32 ? as_f32x4(bias3[un]) : widen(hi[2], hi[3]);
             }
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
@@ -606,6 +655,9 @@ extern "C" int tm_gemm_tile_takes(const void* A, int lda, const void* W, int M, 
            (long long)M * lda * 2 < (1ll << 32) && (long long)N * K * 2 < (1ll << 32) && (long long)M * N < (1ll << 40);
 }
 
+// 2^31 / d rounded up: the upper half of its product with 2 u + 1 is u / d (u (d - 1) + d below 2^31)
+static uint32_t gt_inverse(int d) { return (uint32_t)(((1ull << 31) + d - 1) / d); }
+
 // act[m, i] = silu(gate) * up with gate|up = A W^T, W [2 I, K] (gate rows, then up rows)
 extern "C" int tm_tile_gate_up_silu(const void* A, int lda, int M, int K, const void* W, void* act, int I, hipStream_t stream) {
     if (I <= 0 || I % 8 || !gt_aligned(act) || !tm_gemm_tile_takes(A, lda, W, M, 2 * I, K)) return TM_ERR_ARG;
@@ -628,7 +680,7 @@ extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void
     a.A = A; a.W = W; a.C = q;
     a.bias = bias_dtype == TM_NONE ? nullptr : bias; a.bias_f32 = bias_dtype == TM_F32;
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = H * D; a.splits = 1;
-    a.H = H; a.KVH = KVH; a.D = D; a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots;
+    a.H = H; a.KVH = KVH; a.D = D; a.head_inverse = gt_inverse(D / 64); a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots;
     a.k_pool = k_pool; a.v_pool = v_pool;
     while ((1 << a.page_shift) < page) ++a.page_shift;
     return gt_go<GT_QKV>(a, gt_choose(M, N, K, 1), stream);
@@ -734,7 +786,7 @@ extern "C" int tm_tile_f32_qkv_rope(const void* A, int lda, int M, int K, const 
     TileArgs a{};
     a.A = A; a.W = W; a.C = q; a.bias = bias; a.bias_f32 = 1;
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = H * D; a.splits = 1;
-    a.H = H; a.KVH = KVH; a.D = D; a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots; a.k_pool = k_pool; a.v_pool = v_pool;
+    a.H = H; a.KVH = KVH; a.D = D; a.head_inverse = gt_inverse(D / 64); a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots; a.k_pool = k_pool; a.v_pool = v_pool;
     while ((1 << a.page_shift) < page) ++a.page_shift;
     return gt_go_f32<GT_QKV>(a, stream);
 }
