@@ -76,3 +76,36 @@ def test_gate_up_behind_its_norm_at_the_edges_of_its_rounds(ops, M, K, I, norm32
     # gate, up and the result are rounded to 8 bits, and an element of x may round the other way
     assert (out.double() - want).abs().max() < 3 * 2.0 ** -8 * want.abs().max()
     assert ((out.double() - want).norm() / want.norm()) < 2.0 ** -7
+
+
+@pytest.mark.parametrize("bias_dtype", [torch.float32, BF, None])
+@pytest.mark.parametrize("M,K,H,KVH,D", [(9, 8, 2, 1, 32), (16, 1000, 14, 2, 64), (17, 1024, 3, 1, 64), (33, 904, 66, 1, 128), (48, 776, 4, 2, 96), (64, 936, 14, 2, 64),
+                                         (49, 40, 70, 1, 128)])
+def test_qkv_of_9_to_64_rows_at_the_edges_of_what_a_wavefront_brings(ops, M, K, H, KVH, D, bias_dtype):
+    """Rows that end inside a piece of 64 lanes and inside a k-step, ranges of k that some wavefronts do not have, one unit a block and more
+    (more units than CUs), a token whose numbers are none."""
+    torch.manual_seed(M + K)
+    N = (H + 2 * KVH) * D
+    x, w = torch.randn(M, K, device=DEV).to(BF), (torch.randn(N, K, device=DEV) * K ** -0.5).to(BF)
+    x[3, K - 1] = float("inf")
+    b = None if bias_dtype is None else torch.randn(N, device=DEV).to(bias_dtype)
+    angle = torch.rand(40, D // 2, device=DEV) * 6
+    positions = torch.randint(0, 40, (M,), dtype=torch.int32, device=DEV)
+    slots = torch.randperm(5 * 16)[:M].to(torch.int32).to(DEV)
+    kp, vp = torch.zeros(5, 16, KVH, D, dtype=BF, device=DEV), torch.zeros(5, KVH, D, 16, dtype=BF, device=DEV)
+    out = torch.empty(M, H * D, dtype=BF, device=DEV)
+    assert ops.panel_fits(M, K)
+    ops.panel_qkv_rope(x, ops.pack_weight(w, ops.fused_qkv_strip_rows(H, KVH, D, K)), b, out, H, KVH, D, angle.cos(), angle.sin(), positions, slots, kp, vp)
+    y = x.double() @ w.double().T + (0 if b is None else b.double())
+    y = y.to(BF).double().view(M, H + 2 * KVH, D)
+    c, s = angle.double().cos()[positions.long()][:, None], angle.double().sin()[positions.long()][:, None]
+    lo, hi = y[:, :H + KVH].chunk(2, -1)
+    turned = torch.cat([lo * c - hi * s, hi * c + lo * s], -1)
+    at = slots.long()
+    got = torch.cat([out.view(M, H, D), kp.view(-1, KVH, D)[at], vp.permute(0, 3, 1, 2).reshape(-1, KVH, D)[at]], 1).double()
+    want = torch.cat([turned, y[:, H + KVH:]], 1)
+    rest = [t for t in range(M) if t != 3]
+    assert not got[3, :H + KVH].isfinite().any() and got[rest].isfinite().all()
+    # a projection may round the other way (2^-7 of itself, in both terms of a rotation), and the result is rounded (2^-8)
+    scale = torch.cat([torch.cat([lo.abs() + hi.abs()] * 2, -1), y[:, H + KVH:].abs()], 1)[rest]
+    assert ((got[rest] - want[rest]).abs() <= 2.0 ** -6 * scale + 1e-5).all()

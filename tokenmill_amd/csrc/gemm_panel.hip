@@ -24,16 +24,23 @@
 #define PN_KCH 8            // k-steps a wavefront holds: K <= 4 * 8 * 32 = 1024
 
 // NT: 16-row tiles of x a block takes (1..4). ROWS: rows of a matrix strip (16 or 8).
+//
+// The launch is a trip to memory, the input's way through LDS, 2 x 7 products a tile and two reductions, so what runs beside the trip is
+// what it is made of: a division for every 16-byte piece of the input, the positions waited for by scalar loads before the matrix was
+// asked for, sums exchanged a float at a time. Now everything is asked for at once in the order it is needed (positions, the
+// input by whole rows, the matrix, the bias; the rotary rows once the positions are there), unconditionally within the bounds of buffer
+// descriptors, and the sums go through LDS 16 bytes a lane. The same bits.
+// 896 -> 1,152, cold matrices, launches in a row: 9 to 48 rows 5.2 to 4.0 us, 64 rows 6.8 to 4.7.
 template <int ROWS, int NT>
 __global__ __launch_bounds__(64 * PN_WAVES, 1) void gemm_panel_kernel(const FusedArgs a, const int n_units) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     // the tokens of this block: all of them, or (gridDim.y > 1) the NT tiles from tok0 on
     const int tok0 = blockIdx.y * (NT * 16);
     const int K = a.K, M = a.M - tok0 < NT * 16 ? a.M - tok0 : NT * 16;
-    const int xstride = K + FD_XPAD;
-    bf16_t* xs = (bf16_t*)smem_raw;                                  // [NT * 16][K + FD_XPAD]
-    float* red = (float*)(smem_raw + (size_t)NT * 16 * xstride * sizeof(bf16_t));   // [waves][2][NT][64][5]
-    auto red_at = [&](int w, int ab, int t, int l) { return red + ((((size_t)w * 2 + ab) * NT + t) * 64 + l) * 5; };
+    const int xstride = fused_x_stride(K);
+    bf16_t* xs = (bf16_t*)smem_raw;                                  // [NT * 16][xstride]
+    f32x4_t* red = (f32x4_t*)(smem_raw + (size_t)NT * 16 * xstride * sizeof(bf16_t));   // [waves][2][NT][64]
+    auto red_at = [&](int w, int ab, int t) -> f32x4_t& { return red[((w * 2 + ab) * NT + t) * 64 + (int)threadIdx.x % TM_WAVE]; };
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;
     const int r = lane % 16, g = lane / 16;
 
@@ -41,98 +48,78 @@ __global__ __launch_bounds__(64 * PN_WAVES, 1) void gemm_panel_kernel(const Fuse
     const int per = (ksteps + PN_WAVES - 1) / PN_WAVES;
     const int ks0 = wave * per;
     const int ks1 = ks0 + per < ksteps ? ks0 + per : ksteps;
-    int u = blockIdx.x;
-    FusedUnit cu = fused_unit_of<FD_EPI_QKV, ROWS>(a, u, r);
 
-    // This wavefront's epilogue is that of row tile `wave`: token 16 wave + r. Its position comes by
-    // scalar loads (addresses the same in every lane), which are counted apart from the vector loads.
+    // This wavefront's epilogue is that of row tile `wave`: token 16 wave + r.
     const int tile = wave;
     const int tok = 16 * tile + r;
-    const bool epi_wave = tile < NT;
-    const bool epi_lane = epi_wave && tok < M && 4 * g < ROWS;
-    int tok_pos = 0;
-    if (epi_wave) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int ti = 16 * tile + i;
-            const int pos_i = a.positions[tok0 + (ti < M ? ti : 0)];
-            tok_pos = r == i ? pos_i : tok_pos;
-        }
-    }
+    const bool epi_lane = tile < NT && tok < M && 4 * g < ROWS;
+    const int tok_pos = a.positions[tok0 + (tok < M ? tok : 0)];
+    const int tok_slot = (a.slots ? a.slots : a.positions)[tok0 + (tok < M ? tok : 0)];
 
-    // the matrix first: it has the longest way
+    // x: a wavefront takes every fourth row, two pieces of 16 bytes a lane (K <= 1024); block b starts at its row b, so that the blocks do
+    // not all want the same line at the same time. Beyond the row, and rows beyond M: zeros.
+    constexpr int XR = 4 * NT;                                       // rows a wavefront brings
+    const int turn = blockIdx.x % XR;
+    auto x_row = [&](int i) { return wave + PN_WAVES * (i + turn < XR ? i + turn : i + turn - XR); };
+    u32x4_t v[XR][2];
+#pragma unroll
+    for (int i = 0; i < XR; ++i) {
+        const int row = x_row(i);
+        const __amdgpu_buffer_rsrc_t b = fd_buffer(a.X + (size_t)(tok0 + (row < M ? row : 0)) * a.ldx, row < M ? K * 2 : 0);
+        v[i][0] = __builtin_amdgcn_raw_buffer_load_b128(b, lane * 16, 0, 0);
+        v[i][1] = __builtin_amdgcn_raw_buffer_load_b128(b, lane * 16 + 1024, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // the matrix: this wavefront's range of k of the unit's two strips, zeros beyond it
     constexpr int FRAG = 32 * ROWS;
-    const int lane_off = (g * ROWS + (r < ROWS ? r : 0)) * 8;
-    auto strip_pointer = [&](int strip) { return a.W + (size_t)strip * ksteps * FRAG + lane_off; };
-    const bf16_t* wA = strip_pointer(cu.sA);
-    const bf16_t* wB = strip_pointer(cu.sB);
+    const int lane_off = (g * ROWS + (r < ROWS ? r : 0)) * 16;
     FFrag fa[PN_KCH], fb[PN_KCH];
-    auto load_group = [&]() {
+    auto load_group = [&](const FusedUnit& t) {
+        const int bytes = ks1 > ks0 ? ks1 * FRAG * 2 : 0;
+        const __amdgpu_buffer_rsrc_t wA = fd_buffer(a.W + (size_t)t.sA * ksteps * FRAG, bytes), wB = fd_buffer(a.W + (size_t)t.sB * ksteps * FRAG, bytes);
 #pragma unroll
         for (int j = 0; j < PN_KCH; ++j) {
-            const bool in = cu.rows_ok && ks0 + j < ks1;
-            fa[j].u = in ? *(const u32x4_t*)(wA + (size_t)(ks0 + j) * FRAG) : u32x4_t{0, 0, 0, 0};
-            fb[j].u = in ? *(const u32x4_t*)(wB + (size_t)(ks0 + j) * FRAG) : u32x4_t{0, 0, 0, 0};
+            fa[j].u = __builtin_amdgcn_raw_buffer_load_b128(wA, lane_off + (ks0 + j) * (FRAG * 2), 0, 0);
+            fb[j].u = __builtin_amdgcn_raw_buffer_load_b128(wB, lane_off + (ks0 + j) * (FRAG * 2), 0, 0);
         }
     };
-    load_group();
 
-    // what the epilogue needs from memory, asked for now and kept as loaded (every lane loads, from
-    // entries that exist; the lanes without an epilogue do not look at what came)
+    // what the epilogue needs from memory, kept as loaded (every lane loads, from entries that exist; the lanes without an
+    // epilogue do not look at what came)
     struct EpilogueInputs {
         f32x4_t bias_f[2];
-        uint2 bias_h[2];
+        u32x2_t bias_h[2];
         f32x4_t cos, sin;
-        int slot;
     };
     const int bias_kind = !a.bias ? 0 : (a.bias_f32 ? 2 : 1);
     auto epilogue_inputs = [&](const FusedUnit& t) {
         EpilogueInputs e;
         const int ge = 4 * g < ROWS ? 4 * g : 0;
-        const int ia = t.nA + ge, ib = t.nB + ge;
-        if (bias_kind == 2) {
-            e.bias_f[0] = *(const f32x4_t*)((const float*)a.bias + ia);
-            e.bias_f[1] = *(const f32x4_t*)((const float*)a.bias + ib);
-        } else if (bias_kind == 1) {
-            e.bias_h[0] = *(const uint2*)((const bf16_t*)a.bias + ia);
-            e.bias_h[1] = *(const uint2*)((const bf16_t*)a.bias + ib);
-        }
+        const int ia = t.nA + ge, ib = t.nB + ge, width = (a.H + 2 * a.KVH) * a.D;
+        const __amdgpu_buffer_rsrc_t bf = fd_buffer(a.bias, bias_kind == 2 ? width * 4 : 0), bh = fd_buffer(a.bias, bias_kind == 1 ? width * 2 : 0);
+        e.bias_f[0] = as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(bf, ia * 4, 0, 0));
+        e.bias_f[1] = as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(bf, ib * 4, 0, 0));
+        e.bias_h[0] = __builtin_amdgcn_raw_buffer_load_b64(bh, ia * 2, 0, 0);
+        e.bias_h[1] = __builtin_amdgcn_raw_buffer_load_b64(bh, ib * 2, 0, 0);
         const int jt = t.head < a.H + a.KVH ? t.jt : 0;          // value heads have no rotary row
         const size_t at = (size_t)tok_pos * (a.D / 2) + ROWS * jt + ge;
         e.cos = *(const f32x4_t*)(a.cos_t + at);
         e.sin = *(const f32x4_t*)(a.sin_t + at);
-        e.slot = (a.slots ? a.slots : a.positions)[tok0 + (tok < M ? tok : 0)];
         return e;
     };
-    EpilogueInputs e_next = epilogue_inputs(cu);
+    int u = blockIdx.x;
+    FusedUnit cu = fused_unit_of<FD_EPI_QKV, ROWS>(a, u, r);
+    load_group(cu);
+    __builtin_amdgcn_sched_barrier(0);
+    EpilogueInputs e_next = epilogue_inputs(cu);                     // (the positions came before the rows of x)
+    __builtin_amdgcn_sched_barrier(0);
 
-    // x into LDS, 16 bytes a thread and load, every load of a thread in flight at once (K <= 1024: at most
-    // 8 NT of them); block b starts at row b
-    {
-        const int per_row = K / 8;
-        const int pieces = M * per_row;
-        const int row_shift = blockIdx.x % M;
-        constexpr int XL = 8 * NT;
-        u32x4_t v[XL];
 #pragma unroll
-        for (int i = 0; i < XL; ++i) {
-            const int p = threadIdx.x + i * 64 * PN_WAVES;
-            const int pc = p < pieces ? p : 0;
-            int row = pc / per_row + row_shift;
-            row = row < M ? row : row - M;
-            v[i] = *(const u32x4_t*)(a.X + (size_t)(tok0 + row) * a.ldx + (pc % per_row) * 8);
-        }
-#pragma unroll
-        for (int i = 0; i < XL; ++i) {
-            const int p = threadIdx.x + i * 64 * PN_WAVES;
-            if (p < pieces) {
-                int row = p / per_row + row_shift;
-                row = row < M ? row : row - M;
-                *(u32x4_t*)(xs + (size_t)row * xstride + (p % per_row) * 8) = v[i];
-            }
-        }
-        // rows M .. 16 NT - 1 of x stay as they are: they only feed result columns of tokens that do
-        // not exist, which no lane stores
+    for (int i = 0; i < XR; ++i) {
+        bf16_t* row = xs + (size_t)x_row(i) * xstride;
+        if (8 * lane < xstride - FD_XPAD) *(u32x4_t*)(row + 8 * lane) = v[i][0];
+        if (8 * lane + 512 < xstride - FD_XPAD) *(u32x4_t*)(row + 8 * lane + 512) = v[i][1];
     }
     __syncthreads();
 
@@ -146,24 +133,21 @@ __global__ __launch_bounds__(64 * PN_WAVES, 1) void gemm_panel_kernel(const Fuse
         }
 #pragma unroll
         for (int j = 0; j < PN_KCH; ++j) {
-            const int k = (ks0 + j) * 32 + 8 * g;
-            const bool in = ks0 + j < ks1 && k < K;
+            if (ks0 + j >= ks1) break;                               // (the same in every lane)
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 FFrag xf;
-                xf.u = in ? *(const u32x4_t*)(xs + (size_t)(16 * t + r) * xstride + k) : u32x4_t{0, 0, 0, 0};
+                xf.u = *(const u32x4_t*)(xs + (size_t)(16 * t + r) * xstride + (ks0 + j) * 32 + 8 * g);
                 accA[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[j].b, xf.b, accA[t], 0, 0, 0);
                 accB[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j].b, xf.b, accB[t], 0, 0, 0);
             }
         }
         // partial sums of the wavefronts, added in wavefront order by the wavefront that owns the tile
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                red_at(wave, 0, t, lane)[i] = accA[t][i];
-                red_at(wave, 1, t, lane)[i] = accB[t][i];
-            }
+        for (int t = 0; t < NT; ++t) {
+            red_at(wave, 0, t) = accA[t];
+            red_at(wave, 1, t) = accB[t];
+        }
         __syncthreads();
 
         // the next unit's matrix goes out before this unit's epilogue
@@ -172,24 +156,16 @@ __global__ __launch_bounds__(64 * PN_WAVES, 1) void gemm_panel_kernel(const Fuse
         const FusedUnit done = cu;
         if (more) {
             cu = fused_unit_of<FD_EPI_QKV, ROWS>(a, un, r);
-            wA = strip_pointer(cu.sA);
-            wB = strip_pointer(cu.sB);
-            load_group();
+            load_group(cu);
             e_next = epilogue_inputs(cu);
         }
 
         if (epi_lane) {
-            float sA[4], sB[4];
+            f32x4_t sA = red_at(0, 0, tile), sB = red_at(0, 1, tile);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float va = red_at(0, 0, tile, lane)[i], vb = red_at(0, 1, tile, lane)[i];
-#pragma unroll
-                for (int w = 1; w < PN_WAVES; ++w) {
-                    va += red_at(w, 0, tile, lane)[i];
-                    vb += red_at(w, 1, tile, lane)[i];
-                }
-                sA[i] = va;
-                sB[i] = vb;
+            for (int w = 1; w < PN_WAVES; ++w) {
+                sA += red_at(w, 0, tile);
+                sB += red_at(w, 1, tile);
             }
             // lane: token tok, rows nA + 4g + i and nB + 4g + i
             f32x4_t bA = {0.f, 0.f, 0.f, 0.f}, bB = {0.f, 0.f, 0.f, 0.f};
@@ -208,7 +184,7 @@ __global__ __launch_bounds__(64 * PN_WAVES, 1) void gemm_panel_kernel(const Fuse
                 xA[i] = fd_round(sA[i] + bA[i]);
                 xB[i] = fd_round(sB[i] + bB[i]);
             }
-            const int slot = a.slots ? e.slot : -1;
+            const int slot = a.slots ? tok_slot : -1;
             if (done.head < a.H + a.KVH) {
                 const int half = a.D / 2;
                 const int j0 = ROWS * done.jt + 4 * g;                       // pair index of element 0
@@ -245,14 +221,16 @@ __global__ __launch_bounds__(64 * PN_WAVES, 1) void gemm_panel_kernel(const Fuse
 }
 
 static int panel_lds_bytes(int tiles, int K) {
-    return tiles * 16 * (K + FD_XPAD) * (int)sizeof(bf16_t) + PN_WAVES * 2 * tiles * 64 * 5 * (int)sizeof(float);
+    return tiles * 16 * fused_x_stride(K) * (int)sizeof(bf16_t) + PN_WAVES * 2 * tiles * 64 * (int)sizeof(f32x4_t);
 }
 
 // Can the panel products take M tokens of width K? (x and the partial sums must fit a block's LDS, and
 // a wavefront holds its whole share of K in registers.)
 extern "C" int tm_gemm_panel_fits(int M, int K) {
     if (M <= 0 || M > 64 || K <= 0 || (K % 8) || K > PN_WAVES * PN_KCH * 32) return 0;
-    return panel_lds_bytes((M + 15) / 16, K) + 1024 <= 160 * 1024 ? 1 : 0;
+    // (20 bytes a sum's lane, what the kernel's LDS once took: which rows of which widths come here is a row's bits)
+    const int tiles = (M + 15) / 16;
+    return tiles * 16 * (K + FD_XPAD) * (int)sizeof(bf16_t) + PN_WAVES * 2 * tiles * 64 * 20 + 1024 <= 160 * 1024 ? 1 : 0;
 }
 
 template <int ROWS, int NT>
