@@ -287,14 +287,16 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     // One half of a step: the products of half `half`, and spread between them the reads of the other half's operands (from
     // buffer `from`) and, with dst, the loads of the step ST ahead. The order is the program's: the barriers between the groups
     // keep the compiler from gathering the reads.
-    constexpr int READS = MT + NT, PRODUCTS = MT * NT;
-    auto multiply = [&](const GtFrag& w, const GtFrag& x, f32x4_t& c) {
-        if constexpr (ES == 4) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(w.f[e], x.f[e], c, 0, 0, 0);
-        } else {
-            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.b, x.b, c, 0, 0, 0);
-        }
+    // 32-bit fragments are multiplied a quarter at a time, each quarter over all accumulators before the next, so that no instruction waits
+    // for the one before it (against all four quarters of a pair in a row: gate|up of 100 / 1,000 / 1,500 rows of 896 35.9 / 146 / 220 to
+    // 34.1 / 143 / 213 us, q|k|v of 300 20.6 to 19.5; the order of an accumulator's sums is the same).
+    constexpr int READS = MT + NT, QUARTERS = ES == 4 ? 4 : 1, PRODUCTS = MT * NT * QUARTERS;
+    auto multiply = [&](int half, int i) {
+        const int n = i % (MT * NT), e = i / (MT * NT);
+        const GtFrag &w = fb[half][n % NT], &x = fa[half][n / NT];
+        f32x4_t& c = acc[n / NT][n % NT];
+        if constexpr (ES == 4) c = __builtin_amdgcn_mfma_f32_16x16x4f32(w.f[e], x.f[e], c, 0, 0, 0);
+        else c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.b, x.b, c, 0, 0, 0);
     };
     auto half_step = [&](auto HALF, int from, auto LOADS, uint32_t dst) {
         constexpr int half = decltype(HALF)::value, other = 1 - half;
@@ -310,8 +312,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                 for (int i = q * NL / READS; i < (q + 1) * NL / READS; ++i) issue_one(dst, i);
             }
 #pragma unroll
-            for (int n = q * PRODUCTS / READS; n < (q + 1) * PRODUCTS / READS; ++n)
-                multiply(fb[half][n % NT], fa[half][n / NT], acc[n / NT][n % NT]);
+            for (int i = q * PRODUCTS / READS; i < (q + 1) * PRODUCTS / READS; ++i) multiply(half, i);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -753,7 +754,7 @@ extern "C" int tm_tile_linear(const void* A, int lda, int M, int K, const void* 
 // every load and read, and small tiles leave the fewest CUs idle in a last round: three blocks a CU, one shape (gate|up of 1,000 /
 // 4,096 rows 154 / 537 us; two blocks a CU 159 / 566, 128 x 64 160 / 523, 64 x 128 160 / 524, 128 x 128 189 / 562; 111 / 455 at the
 // unit's peak). Against the kernel of gemm_f32_mfma.hip (16 k at a time through registers), 0.5B shape, 1,000 rows, in us a layer:
-// gate|up with SiLU*up 192 to 154, q|k|v with rotation 50 to 33, o and down 197 to 88.
+// gate|up with SiLU*up 192 to 143, q|k|v with rotation 50 to 33, o and down 197 to 89.
 
 #define GT_F32 float, EPI, 1, 4, 4, 1, 3, 3
 constexpr int GT_F32_TILE = 64, GT_F32_STEP = 32, GT_F32_RING = 3;
