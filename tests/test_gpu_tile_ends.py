@@ -32,7 +32,7 @@ def test_the_last_tile_of_every_block(shape, K):
 
 
 def test_a_units_head_without_a_division():
-    """The host's inverse and the kernel's upper half of a 64-bit product, as numbers."""
+    """unit_inverse and unit_head of csrc/fused_common.h: the host's inverse and the kernel's upper half of a 64-bit product, as numbers."""
     for d in range(1, 17):
         inverse = ((1 << 31) + d - 1) // d
         assert inverse < 1 << 32

@@ -41,6 +41,11 @@ __device__ __forceinline__ void fd_load_lds(uint32_t lds, uint32_t voff, const v
 #define FD_XPAD 16          // padding of an LDS row of x, in elements: with K a multiple of 32 the rows are 32 bytes more than a multiple of 64 apart, which the operand loads read free of bank conflicts (with 8 they take twice as long)
 #define FD_RC 8             // 4-element vectors of a residual row a thread keeps in registers
 
+// A unit's head without a division, which is some thirty instructions in a row in front of a kernel's first loads: the host's
+// 2^31 / d rounded up (d: units a head has), the upper half of whose product with 2 u + 1 is u / d (for u (d - 1) + d below 2^31).
+__host__ __device__ __forceinline__ uint32_t unit_inverse(int d) { return (uint32_t)(((1ull << 31) + d - 1) / d); }
+__device__ __forceinline__ int unit_head(int u, uint32_t inverse) { return (int)__umulhi((uint32_t)(2 * u + 1), inverse); }
+
 // rows of x a block keeps in LDS for M tokens
 __host__ __device__ __forceinline__ int fused_rows(int M) { return M <= 4 ? 4 : (M <= 8 ? 8 : 16); }
 
@@ -66,6 +71,7 @@ struct FusedArgs {
     // QKV epilogue
     bf16_t* q_out;          // [M, H*D]
     int H, KVH, D;
+    uint32_t head_inverse;  // unit_inverse of the units a head has
     const float* cos_t;     // [max_pos, D/2]
     const float* sin_t;
     const int* positions;   // [M]
@@ -95,9 +101,8 @@ __device__ __forceinline__ FusedUnit fused_unit_of(const FusedArgs& a, int u, in
     t.jt = 0;
     t.rows_ok = r < ROWS;
     if (EPI == FD_EPI_QKV) {
-        const int per_head = a.D / (2 * ROWS);
-        t.head = u / per_head;
-        t.jt = u % per_head;
+        t.head = unit_head(u, a.head_inverse);
+        t.jt = u - t.head * (a.D / (2 * ROWS));
         if (t.head < a.H + a.KVH) {                                  // the two halves of ROWS rotary pairs
             t.nA = t.head * a.D + ROWS * t.jt;
             t.nB = t.nA + a.D / 2;

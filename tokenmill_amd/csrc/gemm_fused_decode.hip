@@ -417,7 +417,9 @@ extern "C" int tm_fused_norm_qkv_rope(const float* resid, const void* norm_w, in
     a.page_shift = 0;
     while ((1 << a.page_shift) < page) ++a.page_shift;
     const int units16 = (H + 2 * KVH) * (D / 32);
-    if (tm_fused_qkv_strip_rows(H, KVH, D, K) == 16) return launch_fused<FD_EPI_QKV, 16>(a, units16, units16, stream);
+    const int rows = tm_fused_qkv_strip_rows(H, KVH, D, K);
+    a.head_inverse = unit_inverse(D / (2 * rows));
+    if (rows == 16) return launch_fused<FD_EPI_QKV, 16>(a, units16, units16, stream);
     return launch_fused<FD_EPI_QKV, 8>(a, 2 * units16, 2 * units16, stream);
 }
 

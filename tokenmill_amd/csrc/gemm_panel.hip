@@ -291,6 +291,8 @@ extern "C" int tm_panel_qkv_rope(const void* X, int ldx, int M, int K, const voi
     a.page_shift = 0;
     while ((1 << a.page_shift) < page) ++a.page_shift;
     const int units16 = (H + 2 * KVH) * (D / 32);
-    if (tm_fused_qkv_strip_rows(H, KVH, D, K) == 16) return launch_panel<16>(a, units16, stream);
+    const int rows = tm_fused_qkv_strip_rows(H, KVH, D, K);
+    a.head_inverse = unit_inverse(D / (2 * rows));
+    if (rows == 16) return launch_panel<16>(a, units16, stream);
     return launch_panel<8>(a, 2 * units16, stream);
 }

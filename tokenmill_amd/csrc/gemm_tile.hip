@@ -36,7 +36,7 @@ struct TileArgs {
     int I;                      // SiLU: columns of the result
     // q|k|v
     int H, KVH, D, page_shift;
-    uint32_t head_inverse;      // gt_inverse(D / 64): a unit's head without a division, some thirty instructions in front of the first load
+    uint32_t head_inverse;      // unit_inverse(D / 64)
     const float* cos_t;         // [positions, D / 2]
     const float* sin_t;
     const int* positions;       // [M]
@@ -155,9 +155,6 @@ __device__ __forceinline__ bool gt_next(const TileArgs& a, int BM, int& p, GtPla
     return false;
 }
 
-// q|k|v: the head of unit u, u / (D / 64)
-__device__ __forceinline__ int gt_head(const TileArgs& a, int u) { return (int)__umulhi((uint32_t)(2 * u + 1), a.head_inverse); }
-
 // the matrix row that row q of unit u holds
 template <int EPI>
 __device__ __forceinline__ int gt_matrix_row(const TileArgs& a, int u, int q) {
@@ -169,7 +166,7 @@ __device__ __forceinline__ int gt_matrix_row(const TileArgs& a, int u, int q) {
         return n;
     }
     if (EPI == GT_QKV) {
-        const int per_head = a.D / 64, head = gt_head(a, u);
+        const int per_head = a.D / 64, head = unit_head(u, a.head_inverse);
         n = head * a.D + 32 * (u - head * per_head) + (q & 31) + (q >= 32 ? a.D / 2 : 0);
     } else {
         n = 64 * u + q;
@@ -345,7 +342,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
         constexpr bool BIAS_EARLY = EPI == GT_QKV && MT <= 5 && UNITS == 1;
         u32x4_t bias0[UNITS], bias1[UNITS], bias2[UNITS], bias3[UNITS];     // eight and eight values: 32-bit, or bfloat16 in bias0 and bias2
         auto read_bias = [&](int un) {
-            const int u = at_.tn * (BN / 64) + wn * UNITS + un, head = gt_head(a, u);
+            const int u = at_.tn * (BN / 64) + wn * UNITS + un, head = unit_head(u, a.head_inverse);
             const int c = head * a.D + 32 * (u - head * (a.D / 64)) + 8 * g, at = c + a.D / 2 < a.N ? c : 0;
             const size_t size = a.bias_f32 ? 4 : 2;
             const unsigned char *lo = (const unsigned char*)a.bias + at * size, *hi = lo + a.D / 2 * size;
@@ -414,7 +411,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                 ok0 = ok1 = c0 < a.I;
             } else if (EPI == GT_QKV) {
                 const int per_head = a.D / 64;
-                head = gt_head(a, u);
+                head = unit_head(u, a.head_inverse);
                 d0 = 32 * (u - head * per_head) + 8 * g;
                 c0 = head * a.D + d0;
                 c1 = c0 + a.D / 2;
@@ -656,9 +653,6 @@ extern "C" int tm_gemm_tile_takes(const void* A, int lda, const void* W, int M, 
            (long long)M * lda * 2 < (1ll << 32) && (long long)N * K * 2 < (1ll << 32) && (long long)M * N < (1ll << 40);
 }
 
-// 2^31 / d rounded up: the upper half of its product with 2 u + 1 is u / d (u (d - 1) + d below 2^31)
-static uint32_t gt_inverse(int d) { return (uint32_t)(((1ull << 31) + d - 1) / d); }
-
 // act[m, i] = silu(gate) * up with gate|up = A W^T, W [2 I, K] (gate rows, then up rows)
 extern "C" int tm_tile_gate_up_silu(const void* A, int lda, int M, int K, const void* W, void* act, int I, hipStream_t stream) {
     if (I <= 0 || I % 8 || !gt_aligned(act) || !tm_gemm_tile_takes(A, lda, W, M, 2 * I, K)) return TM_ERR_ARG;
@@ -681,7 +675,7 @@ extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void
     a.A = A; a.W = W; a.C = q;
     a.bias = bias_dtype == TM_NONE ? nullptr : bias; a.bias_f32 = bias_dtype == TM_F32;
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = H * D; a.splits = 1;
-    a.H = H; a.KVH = KVH; a.D = D; a.head_inverse = gt_inverse(D / 64); a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots;
+    a.H = H; a.KVH = KVH; a.D = D; a.head_inverse = unit_inverse(D / 64); a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots;
     a.k_pool = k_pool; a.v_pool = v_pool;
     while ((1 << a.page_shift) < page) ++a.page_shift;
     return gt_go<GT_QKV>(a, gt_choose(M, N, K, 1), stream);
@@ -787,7 +781,7 @@ extern "C" int tm_tile_f32_qkv_rope(const void* A, int lda, int M, int K, const 
     TileArgs a{};
     a.A = A; a.W = W; a.C = q; a.bias = bias; a.bias_f32 = 1;
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = H * D; a.splits = 1;
-    a.H = H; a.KVH = KVH; a.D = D; a.head_inverse = gt_inverse(D / 64); a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots; a.k_pool = k_pool; a.v_pool = v_pool;
+    a.H = H; a.KVH = KVH; a.D = D; a.head_inverse = unit_inverse(D / 64); a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots; a.k_pool = k_pool; a.v_pool = v_pool;
     while ((1 << a.page_shift) < page) ++a.page_shift;
     return gt_go_f32<GT_QKV>(a, stream);
 }
