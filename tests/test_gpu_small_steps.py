@@ -78,6 +78,29 @@ def test_gate_up_behind_its_norm_at_the_edges_of_its_rounds(ops, M, K, I, norm32
     assert ((out.double() - want).norm() / want.norm()) < 2.0 ** -7
 
 
+@pytest.mark.parametrize("norm32", [False, True])
+@pytest.mark.parametrize("K", [136, 904, 1032, 2040])
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+def test_gate_up_of_a_token_has_the_same_bits_whatever_the_matrix_height(ops, M, K, norm32):
+    """A block with one unit and one with two at a time (narrow and wide results) add a row's squares in the same order. Rows of ties: their
+    elements times the norm's factor lie within a last bit of the middle of two bfloat16 numbers, so the factor's last bit shows."""
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    narrow, wide = 64, 4872
+    w = (torch.randn(2, wide, K, generator=g, device=DEV) * K ** -0.5).to(BF)
+    few = ops.pack_weight(w[:, :narrow].reshape(2 * narrow, K), 16, [narrow, narrow])
+    many = ops.pack_weight(w.view(2 * wide, K), 16, [wide, wide])
+    nw = torch.rand(K, generator=g, device=DEV) + 0.5
+    nw = nw if norm32 else nw.to(BF)
+    for _ in range(8):
+        resid = 0.5 + (2 * torch.randint(0, 128, (M, K), generator=g, device=DEV).double() + 1) / 512
+        resid[:, 5] = (K * (1 - 1e-6) - (resid * resid).sum(-1) + resid[:, 5] ** 2).sqrt()         # the factor is 1
+        resid = resid.float()
+        a, b = torch.empty(M, narrow, dtype=BF, device=DEV), torch.empty(M, wide, dtype=BF, device=DEV)
+        ops.fused_norm_gate_up_silu(resid, nw, 1e-6, few, a)
+        ops.fused_norm_gate_up_silu(resid, nw, 1e-6, many, b)
+        assert torch.equal(a, b[:, :narrow])
+
+
 @pytest.mark.parametrize("bias_dtype", [torch.float32, BF, None])
 @pytest.mark.parametrize("M,K,H,KVH,D", [(9, 8, 2, 1, 32), (16, 1000, 14, 2, 64), (17, 1024, 3, 1, 64), (33, 904, 66, 1, 128), (48, 776, 4, 2, 96), (64, 936, 14, 2, 64),
                                          (49, 40, 70, 1, 128)])

@@ -96,15 +96,24 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
+// {lo, hi} = v of the lower numbered of lane and lane ^ OFF, and of the other one
+template <int OFF>
+__device__ __forceinline__ void lane_halves(float v, float& lo, float& hi) {
+    static_assert(OFF == 16 || OFF == 32, "rows of 16 lanes, or halves of the wavefront");
+    const uint32_t u = __float_as_uint(v);
+    if constexpr (OFF == 32) {
+        const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        lo = __uint_as_float(p[0]), hi = __uint_as_float(p[1]);
+    } else {
+        const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        lo = __uint_as_float(p[0]), hi = __uint_as_float(p[1]);
+    }
+}
 template <int OFF>
 __device__ __forceinline__ void lane_pair(float v, float& a, float& b) {       // {a, b} = {v, v of lane ^ OFF}, in either order
     static_assert(OFF == 1 || OFF == 2 || OFF == 4 || OFF == 8 || OFF == 16 || OFF == 32, "a power of two below 64");
-    if constexpr (OFF == 32) {
-        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        a = __uint_as_float(p[0]), b = __uint_as_float(p[1]);
-    } else if constexpr (OFF == 16) {
-        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        a = __uint_as_float(p[0]), b = __uint_as_float(p[1]);
+    if constexpr (OFF >= 16) {
+        lane_halves<OFF>(v, a, b);
     } else {
         a = v;
         if constexpr (OFF == 8) b = dpp_move<0x128>(v);                         // row_ror:8

@@ -148,9 +148,29 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
     if (row < mpad) {                                                // (the same in every lane of a wavefront)
         bf16_t* xrow = xs + (size_t)row * xstride;
         auto squares = [](const f32x4_t v) { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3]; };
-        float ss = 0.f;
+        // With two units a block twice as many threads share a row of more than four: vector j of a thread of one unit's wavefronts lies
+        // with the lower half of the row's lanes for an even j and with the upper half for an odd one. They exchange the squares and add
+        // them in that thread's order, so that a row's factor has the same bits whatever the matrix's height.
+        const int halves = UNITS == 1 || mpad == 4 ? 1 : 2;
+        auto add_squares = [&](float ss, const f32x4_t (&v)[RC]) {
+            if (halves == 1) {
 #pragma unroll
-        for (int j = 0; j < RC; ++j) ss += squares(cache[j]);
+                for (int j = 0; j < RC; ++j) ss += squares(v[j]);
+            } else {
+                float lo[RC], hi[RC];
+                if (mpad == 8) {
+#pragma unroll
+                    for (int j = 0; j < RC; ++j) lane_halves<32>(squares(v[j]), lo[j], hi[j]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < RC; ++j) lane_halves<16>(squares(v[j]), lo[j], hi[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < RC; ++j) ss = (ss + lo[j]) + hi[j];
+            }
+            return ss;
+        };
+        float ss = add_squares(0.f, cache);
         __builtin_amdgcn_sched_barrier(0);
         e_next = epilogue_inputs();                                  // (the positions came before the rows)
         __builtin_amdgcn_sched_barrier(0);
@@ -160,13 +180,12 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
                 f32x4_t v[RC];
 #pragma unroll
                 for (int j = 0; j < RC; ++j) v[j] = resid_at(c0 + j * step);
-#pragma unroll
-                for (int j = 0; j < RC; ++j) ss += squares(v[j]);
+                ss = add_squares(ss, v);
             }
         }
         ss = lane_sum<8>(lane_sum<4>(lane_sum<2>(lane_sum<1>(ss))));
-        if (tpr >= 32) ss = lane_sum<16>(ss);
-        if (tpr >= 64) ss = lane_sum<32>(ss);
+        if (tpr >= 32 * halves) ss = lane_sum<16>(ss);
+        if (tpr >= 64 * halves) ss = lane_sum<32>(ss);
         const float rs = rsqrtf(ss / (float)K + a.eps);
         auto emit = [&](int c, const f32x4_t v, const f32x4_t w) {
             uint2 pk;
