@@ -60,3 +60,22 @@ def test_no_number_reaches_those_that_see_it(ops, bad):
     got = attend(ops, q, k, v, H, 1, D, 16, D ** -0.5)
     k[70, 0, 0] = -1e6
     assert torch.equal(got, attend(ops, q, k, v, H, 1, D, 16, D ** -0.5))
+
+
+def test_weights_over_the_whole_range_of_the_exponential(ops):
+    """Token t sees keys of score 0, among them its block's, so that 0 is the weights' reference, and one key (64) of a score of its own from
+    -86 up to where the reference would move, whose value alone is not 0: the result is e^s 2^30 / (t + e^s)."""
+    D, n, H = 16, 144, 64
+    s = torch.linspace(-86.0, 7.9, (n - 80) * H, device=DEV).view(n - 80, H)
+    q, k, v = torch.zeros(n, H, D, device=DEV), torch.zeros(n, 1, D, device=DEV), torch.zeros(n, 1, D, device=DEV)
+    q[80:, :, 0], k[64, 0, 0], v[64, 0] = s, 1.0, 2.0 ** 30
+    got = attend(ops, q, k, v, H, 1, D, 16, 1.0)[80:].double()
+    e = s.double().exp()
+    want = (e / (torch.arange(80, n, device=DEV)[:, None] + e) * 2.0 ** 30)[..., None]
+    units = ((got - want) / want) * 2.0 ** 24                            # of half a last place
+    # the exponential instruction is good to a last place (2 units), its argument, below 1/2, is rounded (0.4 units of the result); the sum, its
+    # inverse and the product with it round once each (3)
+    assert units.abs().max() <= 6
+    # no roundings lean one way over a range: a correction of the wrong size or sign does (by up to 8 units at -86)
+    for part in units.flatten().chunk(8):
+        assert part.mean().abs() <= 0.5, part.mean()
