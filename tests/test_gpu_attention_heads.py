@@ -132,3 +132,65 @@ def test_portions_by_heads(size, case, page, sink, gate, half, monkeypatch):
     # keys, values, weights, results and queries are rounded to 8 bits on the way: 2 ** -9 each at most, of which the sums keep less
     assert err < 2.0 ** -7 and err < 1.25 * err_latent + 1e-3, (float(err), float(err_latent))
     assert (got.double() - want).abs().max() < 2.0 ** -5 * want.abs().max()
+
+
+def _attended(size, window, entries, n_singles, taken, monkeypatch):
+    """The attention's result for entries (seed, cached tokens, tokens), the last ``n_singles`` single tokens: row by row the same inputs for
+    the same seed, whatever stands beside it (the products in front, which may round by the step's size, are given)."""
+    from tokenmill_amd.hip import ops
+
+    H, Dn, Dr, Dv, Lq, Lk = SIZES[size]
+    part, hidden = _part(size, False, True, False)
+    part.window, page = window, 16
+    part.rotary.max_positions = 10000
+    g = torch.Generator().manual_seed(1)
+    part.load({name: (torch.randn(spec.shape, generator=g) * 0.06 + (1.0 if spec.init == "ones" else 0.0)).to(BF).to(DEV)
+               for name, spec in part.tensor_specs("m.").items()}, "m.")
+    pages = [-(-(a + n) // page) for _, a, n in entries]
+    tables = torch.zeros(len(entries), max(pages), dtype=torch.int32)
+    for s, n in enumerate(pages):
+        tables[s, :n] = torch.arange(sum(pages[:s]), sum(pages[:s + 1]))
+    pool = torch.zeros(sum(pages), page, 1, Lk + Dr, dtype=BF, device=DEV)
+    low, q = [], []
+    for s, (seed, a, n) in enumerate(entries):
+        g = torch.Generator().manual_seed(seed)
+        pool.view(-1, Lk + Dr)[sum(pages[:s]) * page:][:a] = torch.randn(a, Lk + Dr, generator=g).to(BF).to(DEV)
+        low.append(torch.randn(n, Lq + Lk + Dr + H, generator=g).to(DEV))
+        q.append(torch.randn(n, H * (Dn + Dr), generator=g).to(BF).to(DEV))
+    low, q = torch.cat(low), torch.cat(q)
+    part.down = types.SimpleNamespace(forward=lambda x, out_dtype: low)
+    part.uq = types.SimpleNamespace(forward=lambda cq: q)
+    part.o = types.SimpleNamespace(forward=lambda out: out)
+    split = len(entries) - n_singles
+    step = _step([(a, n) for _, a, n in entries[:split]], [a + 1 for _, a, _ in entries[split:]], tables, page, window)
+    real = ops.attn_heads
+    with monkeypatch.context() as m:
+        m.setattr(ops, "attn_heads", lambda *a, **k: taken.append(a[5].shape[0]) or real(*a, **k))
+        out = part.forward(torch.zeros(step.num_tokens, hidden, dtype=BF, device=DEV), step, types.SimpleNamespace(k=pool, v=None, group=0, write=True))
+    return list(out.split([n for _, _, n in entries]))
+
+
+@pytest.mark.parametrize("size", list(SIZES))
+@pytest.mark.parametrize("window", [None, 500])
+def test_a_portions_bits_do_not_depend_on_its_neighbours(size, window, monkeypatch):
+    """Portions of either form, several of each, between each other and beside single tokens, and more rows than pass at once: each alone
+    gives what it gives in the step."""
+    from tokenmill_amd.parts import attention_latent
+
+    monkeypatch.setattr(attention_latent, "HEADS_MOST_ROWS", 1200)
+    entries = [(11, 0, 100), (12, 0, 400), (14, 20, 33), (13, 700, 3), (15, 300, 200), (16, 0, 500), (17, 600, 1), (18, 40, 1), (19, 1300, 1)]
+    taken: list[int] = []
+    together = _attended(size, window, entries, 3, taken, monkeypatch)
+    # blocks of 64 queries: of the 400 and the 3 tokens (448 and 704 rows, 512 in the window), then of the 200 and the 500 (512 rows each)
+    assert taken == [7 + 1, 4 + 8]
+    for i, (entry, got) in enumerate(zip(entries, together)):
+        alone, = _attended(size, window, [entry], int(i >= 6), [], monkeypatch)
+        assert torch.equal(got, alone), i
+
+
+@pytest.mark.parametrize("cached,tokens,heads", [(0, 383, False), (0, 384, True), (382, 2, True), (381, 2, False), (4000, 2, True), (8190, 2, True),
+                                                 (8191, 2, False)])
+def test_a_portions_own_rows_choose_its_form(cached, tokens, heads, monkeypatch):
+    taken: list[int] = []
+    _attended("1k", None, [(5, cached, tokens)], 0, taken, monkeypatch)
+    assert bool(taken) == heads

@@ -3,7 +3,8 @@
 // kernel multiplies queries of Dn + Dr channels by them. Against the attention over the latent itself (latent_mfma.hip: a
 // query of Lk + Dr channels, a result of Lk, each row of the cache read by every head) a (query, key) pair costs Dn + Dr + Dv in
 // place of 2 Lk + Dr products, 320 for 1,088 at Lk 512, and moving a row costs once what moving a query and its result onto the
-// latent did; so it is the way for portions whose tokens are not few beside the rows they see.
+// latent did. Few queries gain most: over the latent a tile of them has four blocks that walk all rows one after the other (2 tokens behind
+// 4,000 rows at 2k sizes 611 to 119 us a layer).
 //
 // A block: 64 queries of a head; its four wavefronts are two groups of 32 queries by two halves of every 64 keys. Keys (64 rows of
 // Dn + Dr, the last Dr shared by the heads) and transposed values (Dv rows of 64) come straight into LDS, 16 bytes a lane, two buffers

@@ -22,13 +22,23 @@ import torch
 
 from tokenmill_amd import profiling
 from tokenmill_amd.hip import ops
-from tokenmill_amd.parts.base import KVCacheSpec, KVCacheView, Mixer, StepContext, as_tensor, portion_blocks
+from tokenmill_amd.parts.base import KVCacheSpec, KVCacheView, Mixer, StepContext, as_tensor, portion_blocks, portion_rows, portion_tiles
 from tokenmill_amd.parts.linear import Linear
 from tokenmill_amd.parts.position import RotaryEmbedding
 from tokenmill_amd.weights.loader import TensorSpec
 
 
-# Portions run with keys and values per head where one of their tokens sees at least so many rows and all see at most so many.
+# A portion runs with keys and values per head where one of its tokens sees at least so many rows, up to so many of its own; portions pass
+# together while their rows are no more. A (query, row) pair costs a third of what it costs over the latent, and a token's rows are walked by two
+# wavefronts side by side; it is two launches more and one for each further portion, which short prompts have no use for. Beyond, keys and values would be no passing
+# buffer any more (8,192 rows of the 2k shapes: 70 MB). Whole steps of the 2k Lusolix shape, onto the latent / by heads, us: prompts of 100 / 250 /
+# 400 / 800 / 1,500 tokens 2,470 / 2,483 / 2,682 / 3,377 / 4,268 and 2,597 / 2,576 / 2,638 / 2,607 / 3,005 (up to 2,600 the launches are the
+# time). The number of tokens decides nothing: a portion of up to 16 is one tile, four blocks, over the latent, that walk its rows one
+# after the other. The mixer of one layer without a window, GPU time, us, 2 / 16 / 64 / 256 tokens behind 500, 1,000, 4,000 and 7,900 cached ones: over the
+# latent 105 / 124 / 148 / 180, 179 / 193 / 221 / 253, 611 / 622 / 644 / 675, 1,164 / 1,180 / 1,199 / 1,232; by heads 46 / 56 / 65 / 70, 56 /
+# 61 / 77 / 81, 119 / 124 / 133 / 141, 196 / 201 / 210 / 212. Portions in one step, 1 / 4 / 7 / 24: of 500 tokens 146 / 270 / 417 / 1,214 and 65 / 113 /
+# 174 / 548; of 2 tokens behind 4,000 614 / 620 / 622 / 642 and 118 / 261 / 481 / 1,437. (Many of the last kind would be better off over the latent,
+# but a step of the scheduler holds one request that goes on inside its prompt, and the choice is to hang on a portion alone.)
 HEADS_SEEN_ROWS = 384
 HEADS_MOST_ROWS = 8192
 
@@ -144,55 +154,79 @@ class LatentAttention(Mixer):
         seen, pairs = self.visible_pairs(step)
         return seen * self.row * e + step.num_tokens * H * (self.row + Lk) * e, 2 * pairs * H * (self.row + Lk)
 
-    def _by_heads(self, q, step: StepContext) -> bool:
-        """Do the step's portions run with keys and values per head, made from the visible rows, in place of queries and results moved
-        onto the latent? A (query, row) pair costs a third that way, and a token's rows are walked by two wavefronts side by side; it is
-        three launches more, which a short prompt has no use for. Where the host knows the portions (a step that a graph replays is
-        sized for others too), and while the keys and values stay a passing buffer (8,192 rows of the 2k shapes: 70 MB). A step of the
-        2k Lusolix shape, onto the latent / by heads, us: prompts of 100 / 250 / 400 / 800 / 1,500 tokens 2,470 / 2,483 / 2,682 / 3,377 /
-        4,268 and 2,597 / 2,576 / 2,638 / 2,607 / 3,005 (up to 2,600 the launches are the time), 64 tokens behind 600 / 1,000 cached ones
-        2,779 / 3,248 and 2,561 / 2,567."""
+    def _by_heads(self, q, step: StepContext) -> list[tuple[int, ...]]:
+        """Which of the step's portions run with keys and values per head, made from their visible rows, in place of queries and results
+        moved onto the latent: groups of requests whose rows fit the passing buffer together. A portion's own tokens and rows decide,
+        never its neighbours'."""
+        H, Dn, Lk, window = self.num_heads, self.head_dim, self.kv_rank, self.window or 0
         if not step.portions_known or step.num_decode >= q.shape[0] or q.dtype != torch.bfloat16 or self.uk_nt is None \
-                or not ops.attn_heads_takes(self.head_dim, self.rot_dim, self.v_head_dim):
-            return False
-        seen = max(a + n for a, n in zip(step.start_positions, step.q_lens[:step.num_seqs - step.num_decode]))
-        if min(seen, self.window or seen) < HEADS_SEEN_ROWS:
-            return False
-        H, Dn, Lk = self.num_heads, self.head_dim, self.kv_rank
-        return portion_blocks(step, self.window or 0, q.device)[2] <= HEADS_MOST_ROWS and Lk % 64 == 0 and Lk >= 256 and H * Dn % 8 == 0
+                or Lk % 64 or Lk < 256 or H * Dn % 8 or not ops.attn_heads_takes(Dn, self.rot_dim, self.v_head_dim):
+            return []
+        groups, held = [], HEADS_MOST_ROWS
+        for s, (_, n, start, _, rows) in enumerate(portion_rows(step, window)):
+            if min(start + n, window or start + n) < HEADS_SEEN_ROWS or rows > HEADS_MOST_ROWS:
+                continue
+            if held + rows > HEADS_MOST_ROWS:
+                groups.append(())
+                held = 0
+            groups[-1] += (s,)
+            held += rows
+        return groups
 
-    def _attend_by_heads(self, q, out, gate, step: StepContext, cache: KVCacheView, group, cos, sin) -> None:
-        """The portions' rows of ``out`` [T, H Dv], gated."""
+    def _attend_by_heads(self, q, out, gate, step: StepContext, cache: KVCacheView, group, cos, sin, which: tuple[int, ...]) -> None:
+        """The rows of ``out`` [T, H Dv] of the portions ``which``, gated."""
         H, Dn, Dr, Dv, Lk = self.num_heads, self.head_dim, self.rot_dim, self.v_head_dim, self.kv_rank
-        blocks, gathers, rows = portion_blocks(step, self.window or 0, q.device)
-        T, bf16 = q.shape[0] - step.num_decode, dict(dtype=torch.bfloat16, device=q.device)
+        blocks, gathers, rows = portion_blocks(step, which, self.window or 0, q.device)
+        portions, bf16 = portion_rows(step, self.window or 0), dict(dtype=torch.bfloat16, device=q.device)
+        span = slice(portions[which[0]][0], portions[which[-1]][0] + portions[which[-1]][1])       # (rows of other portions between: left alone)
         latent, kv = torch.empty((rows, Lk), **bf16), torch.empty(rows * (H * Dn + Dr), **bf16)
         keys, shared = kv[:rows * H * Dn].view(rows, H * Dn), kv[rows * H * Dn:].view(rows, Dr)
-        vt, qr = torch.empty((H * Dv, rows), **bf16), torch.empty((T, H * Dr), **bf16)
+        vt, qr = torch.empty((H * Dv, rows), **bf16), torch.empty((span.stop - span.start, H * Dr), **bf16)
         for s, first, count, lo, hi, at in gathers:
             ops.latent_rows(cache.k, group.block_tables[s], first, lo, hi, Lk, Dr, latent[at:at + count], shared[at:at + count])
         ops.tile_linear(latent, self.uk.view(H * Dn, Lk), keys)
         ops.tile_linear(self.uv_nt.view(H * Dv, Lk), latent, vt)
-        ops.rotate_heads(q[:T, Dn:], Dn + Dr, qr, Dr, H, Dr, cos, sin, step.positions[:T], half_pairs=self.half_pairs)
-        ops.attn_heads(q[:T], qr, kv, vt, out[:T], blocks, H, Dn, Dr, Dv, self.scale, self.window or 0,
-                       gate=gate[:T] if gate is not None else None, sink=self.sink)
+        ops.rotate_heads(q[span, Dn:], Dn + Dr, qr, Dr, H, Dr, cos, sin, step.positions[span], half_pairs=self.half_pairs)
+        ops.attn_heads(q[span], qr, kv, vt, out[span], blocks, H, Dn, Dr, Dv, self.scale, self.window or 0,
+                       gate=gate[span] if gate is not None else None, sink=self.sink)
 
-    def _attend(self, qa, latent, step: StepContext, cache: KVCacheView, group, singles_only: bool = False) -> None:
-        """Prompt portions and single tokens (the step's last ``num_decode`` rows) on the matrix unit where its kernel takes
-        the sizes; the 32-bit path and every other size through the kernel that takes a token and a head a wavefront."""
-        H, Lk, row, T = self.num_heads, self.kv_rank, self.row, qa.shape[0]
-        tiles, first_single = step.prefill_tiles, T - step.num_decode
-        if not ops.attn_latent_mfma_takes(qa.dtype, Lk, row, H) or (
-                first_single > 0 and not singles_only and (tiles is None or not tiles.shape[0])):
-            ops.attn_latent(qa, latent, cache.k, group.block_tables, step.seq_of_token, step.positions, H, Lk, row, self.scale,
-                            self.window or 0, sink=self.sink)
+    @staticmethod
+    def _latent_runs(step: StepContext, T: int, groups) -> list[tuple[int, int, tuple[int, ...] | None]]:
+        """Runs of rows that no group holds: (first row, row behind the last, their portions' requests, None: the whole step's)."""
+        if not groups:
+            return [(0, T, None)]
+        taken = {s for which in groups for s in which}
+        runs = []
+        for s, (row, n, _, _, _) in enumerate(portion_rows(step, 0)):
+            if s in taken:
+                continue
+            if runs and runs[-1][1] == row:
+                runs[-1] = (runs[-1][0], row + n, runs[-1][2] + (s,))
+            else:
+                runs.append((row, row + n, (s,)))
+        if step.num_decode:
+            first = T - step.num_decode
+            if runs and runs[-1][1] == first:
+                runs[-1] = (runs[-1][0], T, runs[-1][2])
+            else:
+                runs.append((first, T, ()))
+        return runs
+
+    def _attend(self, qa, latent, first: int, tiles, singles: int, step: StepContext, cache: KVCacheView, group) -> None:
+        """Prompt portions (``tiles``) and ``singles`` single tokens behind them, rows ``first`` and up of the step, on the matrix unit
+        where its kernel takes the sizes; the 32-bit path and every other size through the kernel that takes a token and a head a
+        wavefront."""
+        H, Lk, row, n = self.num_heads, self.kv_rank, self.row, qa.shape[0]
+        seq, positions = step.seq_of_token[first:first + n], step.positions[first:first + n]
+        if not ops.attn_latent_mfma_takes(qa.dtype, Lk, row, H) or (n > singles and (tiles is None or not tiles.shape[0])):
+            ops.attn_latent(qa, latent, cache.k, group.block_tables, seq, positions, H, Lk, row, self.scale, self.window or 0, sink=self.sink)
             return
-        if first_single > 0 and not singles_only:
-            ops.attn_latent_mfma(qa, latent, cache.k, group.block_tables, tiles, step.seq_of_token, step.positions, 0, 0, H, Lk, row,
-                                 self.scale, self.window or 0, sink=self.sink)
-        if step.num_decode > 0:
-            ops.attn_latent_mfma(qa, latent, cache.k, group.block_tables, None, step.seq_of_token, step.positions, first_single,
-                                 step.num_decode, H, Lk, row, self.scale, self.window or 0, most_context=step.max_decode_context,
+        if n > singles:
+            ops.attn_latent_mfma(qa, latent, cache.k, group.block_tables, tiles, seq, positions, 0, 0, H, Lk, row, self.scale,
+                                 self.window or 0, sink=self.sink)
+        if singles > 0:
+            ops.attn_latent_mfma(qa, latent, cache.k, group.block_tables, None, seq, positions, n - singles, singles, H, Lk, row, self.scale,
+                                 self.window or 0, most_context=step.max_decode_context,
                                  bound=self.rotary.max_positions if self.rotary is not None else 1 << 20, sink=self.sink)
 
     def forward(self, x, step: StepContext, cache: KVCacheView, residual: torch.Tensor | None = None):
@@ -218,36 +252,37 @@ class LatentAttention(Mixer):
             q = self.uq.forward(cq)
         gate = low[:, self.gate_at:] if self.output_gate else None
         out = torch.empty((T, H * Dv), dtype=x.dtype, device=x.device)
-        done = 0                                                    # rows of out that are there: the portions', or none
-        if self._by_heads(q, step):
-            done = T - step.num_decode
+        groups = self._by_heads(q, step)
+        for which in groups:
             with profiling.label("attention", lambda: self.cost("attention", step, T)):
-                self._attend_by_heads(q, out, gate, step, cache, group, cos, sin)
-        if done < T:
-            self._onto_latent(q, out, gate, step, cache, group, cos, sin, done)
+                self._attend_by_heads(q, out, gate, step, cache, group, cos, sin, which)
+        for first, stop, which in self._latent_runs(step, T, groups):
+            self._onto_latent(q, out, gate, step, cache, group, cos, sin, first, stop, which)
         with profiling.label("o_proj", lambda: self.cost("o_proj", step, T)):
             return self.o.forward(out)
 
-    def _onto_latent(self, q, out, gate, step: StepContext, cache: KVCacheView, group, cos, sin, first: int) -> None:
-        """Rows ``first`` and up of ``out``, gated: the queries moved onto the latent, the attention over it, its result onto the values."""
-        T, H, Dn, Dr, Dv, Lk, row = q.shape[0], self.num_heads, self.head_dim, self.rot_dim, self.v_head_dim, self.kv_rank, self.row
+    def _onto_latent(self, q, out, gate, step: StepContext, cache: KVCacheView, group, cos, sin, first: int, stop: int, which) -> None:
+        """Rows first .. stop - 1 of ``out``, gated: the queries moved onto the latent, the attention over it, its result onto the values.
+        ``which``: the requests whose portions they are, beside single tokens (None: the whole step)."""
+        n, T, H, Dn, Dr, Dv, Lk, row = stop - first, q.shape[0], self.num_heads, self.head_dim, self.rot_dim, self.v_head_dim, self.kv_rank, self.row
         half = self.half_pairs
-        qa = torch.empty((T, H * row), dtype=q.dtype, device=q.device)
-        latent = torch.empty((T, H * Lk), dtype=q.dtype, device=q.device)
-        q1, qa1, latent1, out1, positions = q[first:], qa[first:], latent[first:], out[first:], step.positions[first:]
-        with profiling.label("qkv", lambda: self.cost("qkv", step, T)):
-            if self.uk_nt is not None and ops.heads_matmul_mfma_takes(q1, Dn + Dr, self.uk_nt):
+        qa = torch.empty((n, H * row), dtype=q.dtype, device=q.device)
+        latent = torch.empty((n, H * Lk), dtype=q.dtype, device=q.device)
+        q, out, positions = q[first:stop], out[first:stop], step.positions[first:stop]
+        with profiling.label("qkv", lambda: self.cost("qkv", step, n)):
+            if self.uk_nt is not None and ops.heads_matmul_mfma_takes(q, Dn + Dr, self.uk_nt):
                 # the heads' rotated channels go beside their part on the latent in the same launch
-                ops.heads_matmul_mfma(q1, Dn + Dr, self.uk_nt, qa1, row, tail=Dr, cos=cos, sin=sin, positions=positions, half_pairs=half)
+                ops.heads_matmul_mfma(q, Dn + Dr, self.uk_nt, qa, row, tail=Dr, cos=cos, sin=sin, positions=positions, half_pairs=half)
             else:
-                ops.heads_matmul(q1, Dn + Dr, self.uk, qa1, row)
+                ops.heads_matmul(q, Dn + Dr, self.uk, qa, row)
                 if Dr:
-                    ops.rotate_heads(q1[:, Dn:], Dn + Dr, qa1[:, Lk:], row, H, Dr, cos, sin, positions, half_pairs=half)
-        with profiling.label("attention", lambda: self.cost("attention", step, T)):
-            self._attend(qa, latent, step, cache, group, singles_only=first > 0)
-        with profiling.label("o_proj", lambda: self.cost("o_proj", step, T)):
-            gate1 = gate[first:] if gate is not None else None
-            if ops.heads_matmul_mfma_takes(latent1, Lk, self.uv_nt):
-                ops.heads_matmul_mfma(latent1, Lk, self.uv_nt, out1, Dv, gate=gate1)
+                    ops.rotate_heads(q[:, Dn:], Dn + Dr, qa[:, Lk:], row, H, Dr, cos, sin, positions, half_pairs=half)
+        with profiling.label("attention", lambda: self.cost("attention", step, n)):
+            tiles = step.prefill_tiles if which is None else portion_tiles(step, which, q.device) if which else None
+            self._attend(qa, latent, first, tiles, max(0, stop - (T - step.num_decode)), step, cache, group)
+        with profiling.label("o_proj", lambda: self.cost("o_proj", step, n)):
+            gate = gate[first:stop] if gate is not None else None
+            if ops.heads_matmul_mfma_takes(latent, Lk, self.uv_nt):
+                ops.heads_matmul_mfma(latent, Lk, self.uv_nt, out, Dv, gate=gate)
             else:
-                ops.heads_matmul(latent1, Lk, self.uv, out1, Dv, gate=gate1)
+                ops.heads_matmul(latent, Lk, self.uv, out, Dv, gate=gate)

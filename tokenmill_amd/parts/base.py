@@ -124,32 +124,63 @@ class StepContext:
     portions_known: bool = False
 
 
-def portion_blocks(step: StepContext, window: int, device):
-    """The step's portions for a kernel that takes blocks of 64 queries of one portion beside its visible rows gathered in order:
-    (blocks int32 [n, 4] on the device = (first row, queries, position of the first, gathered row of position 0), those with the most keys
-    first; a portion's gathered rows as (request, position of its first row, rows, oldest and newest position in the cache, first row);
-    all gathered rows). Positions are gathered in whole blocks of 64. Made once per step and window and shared by the step's layers."""
-    made = getattr(step, "_portion_blocks", None)
-    if made is None:
-        made = step._portion_blocks = {}
-    if window not in made:
-        blocks, gathers, rows, row = [], [], 0, 0
-        for s in range(step.num_seqs - step.num_decode):
-            start, n = step.start_positions[s], step.q_lens[s]
-            lo = max(0, start - window + 1) if window else 0
-            first = lo // 64 * 64
-            count = -(-(start + n) // 64) * 64 - first
-            gathers.append((s, first, count, lo, start + n - 1, rows))
+def portion_rows(step: StepContext, window: int) -> list[tuple[int, int, int, int, int]]:
+    """The step's portions: (first row of the step, tokens, position of the first, position of the first row to be gathered for it, rows to
+    be gathered). Positions are gathered in whole blocks of 64 from the oldest that a token sees."""
+    out, row = [], 0
+    for start, n in zip(step.start_positions, step.q_lens[:step.num_seqs - step.num_decode]):
+        first = (max(0, start - window + 1) if window else 0) // 64 * 64
+        out.append((row, n, start, first, -(-(start + n) // 64) * 64 - first))
+        row += n
+    if row != step.num_tokens - step.num_decode:
+        raise ValueError("the step's portions do not cover its rows")
+    return out
+
+
+def _made_once(step: StepContext, key, make):
+    """What the layers of a step share beside the step itself."""
+    held = getattr(step, "_made", None)
+    if held is None:
+        held = step._made = {}
+    if key not in held:
+        held[key] = make()
+    return held[key]
+
+
+def _table(entries, device) -> torch.Tensor:
+    """Entries (keys seen, (four numbers)) as int32 [n, 4] on the device, those with the most keys first."""
+    return torch.tensor([e for _, e in sorted(entries, key=lambda e: -e[0])], dtype=torch.int32, pin_memory=True).to(device, non_blocking=True)
+
+
+def portion_blocks(step: StepContext, which: tuple[int, ...], window: int, device):
+    """The portions of the requests ``which`` for a kernel that takes blocks of 64 queries of one portion beside its visible rows gathered in
+    order: (blocks int32 [n, 4] on the device = (row, queries, position of the first, gathered row of position 0), rows counted from
+    the first portion's; a portion's gathered rows as (request, position of its first row, rows, oldest and newest position in the cache,
+    first row); all gathered rows). Made once per step and shared by its layers."""
+    def make():
+        portions = portion_rows(step, window)
+        base, blocks, gathers, rows = portions[which[0]][0], [], [], 0
+        for s in which:
+            row, n, start, first, count = portions[s]
+            gathers.append((s, first, count, max(0, start - window + 1) if window else 0, start + n - 1, rows))
             for at in range(0, n, 64):
                 pos, m = start + at, min(64, n - at)
-                blocks.append((pos + m - (max(0, pos - window + 1) if window else 0), (row + at, m, pos, rows - first)))
+                blocks.append((pos + m - (max(0, pos - window + 1) if window else 0), (row - base + at, m, pos, rows - first)))
             rows += count
-            row += n
-        if row != step.num_tokens - step.num_decode:
-            raise ValueError("the step's portions do not cover its rows")
-        blocks.sort(key=lambda b: -b[0])
-        made[window] = torch.tensor([b for _, b in blocks], dtype=torch.int32, pin_memory=True).to(device, non_blocking=True), gathers, rows
-    return made[window]
+        return _table(blocks, device), gathers, rows
+
+    return _made_once(step, ("blocks", which, window), make)
+
+
+def portion_tiles(step: StepContext, which: tuple[int, ...], device) -> torch.Tensor:
+    """``prefill_tiles`` of the portions of the requests ``which`` alone, rows counted from the first portion's."""
+    def make():
+        portions = portion_rows(step, 0)
+        base = portions[which[0]][0]
+        return _table([(start + at + min(16, n - at), (s, row - base + at, min(16, n - at), start + at))
+                       for s in which for row, n, start, _, _ in [portions[s]] for at in range(0, n, 16)], device)
+
+    return _made_once(step, ("tiles", which), make)
 
 
 def step_segments(step: StepContext, size: int, device, portions_only: bool = False):
