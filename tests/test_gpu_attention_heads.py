@@ -158,9 +158,10 @@ def _attended(size, window, entries, n_singles, taken, monkeypatch):
         low.append(torch.randn(n, Lq + Lk + Dr + H, generator=g).to(DEV))
         q.append(torch.randn(n, H * (Dn + Dr), generator=g).to(BF).to(DEV))
     low, q = torch.cat(low), torch.cat(q)
-    part.down = types.SimpleNamespace(forward=lambda x, out_dtype: low)
-    part.uq = types.SimpleNamespace(forward=lambda cq: q)
-    part.o = types.SimpleNamespace(forward=lambda out: out)
+    free = dict(cost=lambda rows, out_bytes=2: (0, 0), weight=part.uq.weight)
+    part.down = types.SimpleNamespace(forward=lambda x, out_dtype: low, **free)
+    part.uq = types.SimpleNamespace(forward=lambda cq: q, **free)
+    part.o = types.SimpleNamespace(forward=lambda out: out, **free)
     split = len(entries) - n_singles
     step = _step([(a, n) for _, a, n in entries[:split]], [a + 1 for _, a, _ in entries[split:]], tables, page, window)
     real = ops.attn_heads
@@ -194,3 +195,16 @@ def test_a_portions_own_rows_choose_its_form(cached, tokens, heads, monkeypatch)
     taken: list[int] = []
     _attended("1k", None, [(5, cached, tokens)], 0, taken, monkeypatch)
     assert bool(taken) == heads
+
+
+@pytest.mark.parametrize("entries,n_singles", [([(1, 0, 100)], 0), ([(1, 0, 100), (2, 0, 400), (3, 20, 30), (4, 500, 1)], 1)])
+def test_a_profile_counts_a_layer_once(entries, n_singles, monkeypatch):
+    from tokenmill_amd import profiling
+
+    counted = []
+    real = LatentAttention.cost
+    monkeypatch.setattr(LatentAttention, "cost", lambda self, label, step, rows: counted.append((label, rows)) or real(self, label, step, rows))
+    with profiling.collect(trace=False):
+        _attended("1k", None, entries, n_singles, [], monkeypatch)
+    T = sum(n for _, _, n in entries)
+    assert sorted(counted) == [("attention", T), ("o_proj", T), ("qkv", T)]

@@ -253,23 +253,27 @@ class LatentAttention(Mixer):
         gate = low[:, self.gate_at:] if self.output_gate else None
         out = torch.empty((T, H * Dv), dtype=x.dtype, device=x.device)
         groups = self._by_heads(q, step)
+        cost = lambda: self.cost("attention", step, T)              # (the whole step's: counted with the first piece)
         for which in groups:
-            with profiling.label("attention", lambda: self.cost("attention", step, T)):
+            with profiling.label("attention", cost):
                 self._attend_by_heads(q, out, gate, step, cache, group, cos, sin, which)
+            cost = None
         for first, stop, which in self._latent_runs(step, T, groups):
-            self._onto_latent(q, out, gate, step, cache, group, cos, sin, first, stop, which)
+            self._onto_latent(q, out, gate, step, cache, group, cos, sin, first, stop, which, cost)
+            cost = None
         with profiling.label("o_proj", lambda: self.cost("o_proj", step, T)):
             return self.o.forward(out)
 
-    def _onto_latent(self, q, out, gate, step: StepContext, cache: KVCacheView, group, cos, sin, first: int, stop: int, which) -> None:
+    def _onto_latent(self, q, out, gate, step: StepContext, cache: KVCacheView, group, cos, sin, first: int, stop: int, which, cost) -> None:
         """Rows first .. stop - 1 of ``out``, gated: the queries moved onto the latent, the attention over it, its result onto the values.
-        ``which``: the requests whose portions they are, beside single tokens (None: the whole step)."""
+        ``which``: the requests whose portions they are, beside single tokens (None: the whole step). ``cost``: the attention's, for a
+        profile, or None; the two products' are counted by the caller."""
         n, T, H, Dn, Dr, Dv, Lk, row = stop - first, q.shape[0], self.num_heads, self.head_dim, self.rot_dim, self.v_head_dim, self.kv_rank, self.row
         half = self.half_pairs
         qa = torch.empty((n, H * row), dtype=q.dtype, device=q.device)
         latent = torch.empty((n, H * Lk), dtype=q.dtype, device=q.device)
         q, out, positions = q[first:stop], out[first:stop], step.positions[first:stop]
-        with profiling.label("qkv", lambda: self.cost("qkv", step, n)):
+        with profiling.label("qkv"):
             if self.uk_nt is not None and ops.heads_matmul_mfma_takes(q, Dn + Dr, self.uk_nt):
                 # the heads' rotated channels go beside their part on the latent in the same launch
                 ops.heads_matmul_mfma(q, Dn + Dr, self.uk_nt, qa, row, tail=Dr, cos=cos, sin=sin, positions=positions, half_pairs=half)
@@ -277,10 +281,10 @@ class LatentAttention(Mixer):
                 ops.heads_matmul(q, Dn + Dr, self.uk, qa, row)
                 if Dr:
                     ops.rotate_heads(q[:, Dn:], Dn + Dr, qa[:, Lk:], row, H, Dr, cos, sin, positions, half_pairs=half)
-        with profiling.label("attention", lambda: self.cost("attention", step, n)):
+        with profiling.label("attention", cost):
             tiles = step.prefill_tiles if which is None else portion_tiles(step, which, q.device) if which else None
             self._attend(qa, latent, first, tiles, max(0, stop - (T - step.num_decode)), step, cache, group)
-        with profiling.label("o_proj", lambda: self.cost("o_proj", step, n)):
+        with profiling.label("o_proj"):
             gate = gate[first:stop] if gate is not None else None
             if ops.heads_matmul_mfma_takes(latent, Lk, self.uv_nt):
                 ops.heads_matmul_mfma(latent, Lk, self.uv_nt, out, Dv, gate=gate)
