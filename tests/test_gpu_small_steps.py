@@ -132,3 +132,27 @@ def test_qkv_of_9_to_64_rows_at_the_edges_of_what_a_wavefront_brings(ops, M, K, 
     # a projection may round the other way (2^-7 of itself, in both terms of a rotation), and the result is rounded (2^-8)
     scale = torch.cat([torch.cat([lo.abs() + hi.abs()] * 2, -1), y[:, H + KVH:].abs()], 1)[rest]
     assert ((got[rest] - want[rest]).abs() <= 2.0 ** -6 * scale + 1e-5).all()
+
+
+@pytest.mark.parametrize("norm32", [False, True])
+@pytest.mark.parametrize("M,K,H,KVH", [(1, 896, 14, 2), (8, 896, 4, 2), (4, 904, 4, 2), (16, 1544, 4, 2), (3, 2048, 4, 2), (2, 3584, 28, 4)])
+def test_an_infinite_norm_weight_gives_infinite_values(ops, M, K, H, KVH, norm32):
+    """x has an infinity in one channel: it meets that channel's column of the matrix and nothing else, least of all the zeros that stand
+    for k-steps a wavefront does not have."""
+    D = 64
+    torch.manual_seed(K)
+    N = (H + 2 * KVH) * D
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).to(BF)
+    packed = ops.pack_weight(w, ops.fused_qkv_strip_rows(H, KVH, D, K))
+    angle = torch.rand(40, D // 2, device=DEV)
+    positions = torch.arange(M, dtype=torch.int32, device=DEV)
+    for at in (3, 37, K // 4, K // 2 + 5, K - 1):
+        resid, nw = torch.randn(M, K, device=DEV) + 0.1, torch.rand(K, device=DEV) + 0.5
+        nw[at] = float("inf")
+        nw = nw if norm32 else nw.to(BF)
+        kp, vp = torch.zeros(1, 16, KVH, D, dtype=BF, device=DEV), torch.zeros(1, KVH, D, 16, dtype=BF, device=DEV)
+        out = torch.empty(M, H * D, dtype=BF, device=DEV)
+        ops.fused_norm_qkv_rope(resid, nw, 1e-6, packed, None, out, H, KVH, D, angle.cos(), angle.sin(), positions, positions, kp, vp)
+        x = (resid[:, at:at + 1].sign() * float("inf")).double()
+        want = (x @ w[-KVH * D:, at:at + 1].double().T).view(M, KVH, D)
+        assert torch.equal(vp[0, :, :, :M].permute(2, 0, 1).double(), want), at

@@ -17,6 +17,9 @@
 #include "api.h"
 #include "fused_common.h"
 
+// Elements between the rows of x in LDS: whole k-steps, one of zeros and the padding.
+__host__ __device__ __forceinline__ int fused_norm_stride(int K) { return fused_x_stride(K) + 32; }
+
 // ROWS: rows of a strip (16 or 8). Short strips leave rows of the MFMA tile empty (their lanes load what the others load)
 // and double the number of units, for matrices that would otherwise give fewer blocks than the chip has CUs.
 // WAVES: wavefronts that split the K of a unit (4, or 8 for a long K). UNITS: units a block multiplies at once, each by WAVES
@@ -40,12 +43,12 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
     constexpr int KCH = PIPE ? FD_KCH_PIPE : FD_KCH;
     constexpr int THREADS = 64 * WAVES * UNITS, RC = PLAIN ? fused_row_vectors(THREADS) : FD_RC;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    bf16_t* xs = (bf16_t*)smem_raw;                                  // [4, 8 or 16 rows][fused_x_stride]
+    bf16_t* xs = (bf16_t*)smem_raw;                                  // [4, 8 or 16 rows][fused_norm_stride]
     __shared__ f32x4_t red[UNITS][WAVES][2][64];
     const int K = a.K, M = a.M;
     const int ksteps = (K + 31) / 32;
     const int per = (ksteps + WAVES - 1) / WAVES;
-    const int xstride = fused_x_stride(K);
+    const int xstride = fused_norm_stride(K);
     const int block_wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;
     const int slot_of_block = block_wave / WAVES, wave = block_wave % WAVES;      // which of the block's units, which part of its K
     const int r = lane % 16, g = lane / 16;
@@ -223,7 +226,7 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
                 for (int j = 0; j < RC; ++j) emit(c0 + j * step, cache[j], w[j]);
             }
         }
-        for (int c = K + sub; c < xstride - FD_XPAD; c += tpr) xrow[c] = 0;      // whole k-steps
+        for (int c = K + sub; c < xstride - FD_XPAD; c += tpr) xrow[c] = 0;      // whole k-steps, and one of zeros
     } else {
         e_next = epilogue_inputs();
     }
@@ -233,9 +236,9 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
     f32x4_t accA, accB;
     auto multiply_group = [&](const auto& ga, const auto& gb, int base) {
 #pragma unroll
-        for (int j = 0; j < KCH; ++j) {                              // (steps beyond ks1: zeros of the matrix)
+        for (int j = 0; j < KCH; ++j) {                              // (steps beyond ks1: zeros by the zeros behind the row; an infinity of x would not do)
             FFrag xf;
-            xf.u = *(const u32x4_t*)(xr + (base + j < ksteps ? base + j : 0) * 32);
+            xf.u = *(const u32x4_t*)(xr + (base + j < ks1 ? base + j : ksteps) * 32);
             accA = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[j].b, xf.b, accA, 0, 0, 0);
             accB = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gb[j].b, xf.b, accB, 0, 0, 0);
         }
@@ -356,12 +359,12 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
 }
 
 // Dynamic LDS of a launch: the normed rows.
-static int fused_lds_bytes(int M, int K) { return fused_rows(M) * fused_x_stride(K) * (int)sizeof(bf16_t); }
+static int fused_lds_bytes(int M, int K) { return fused_rows(M) * fused_norm_stride(K) * (int)sizeof(bf16_t); }
 
 template <int EPI, int ROWS, bool PIPE, int WAVES, int UNITS, bool PLAIN>
 static int launch_fused_kernel(const FusedArgs& a, int n_units, int blocks, hipStream_t stream) {
     const int lds = fused_lds_bytes(a.M, a.K);
-    if (lds + (int)sizeof(f32x4_t) * UNITS * WAVES * 2 * 64 + 1024 > 160 * 1024) return TM_ERR_ARG;
+    if (lds + (int)sizeof(f32x4_t) * UNITS * WAVES * 2 * 64 > 160 * 1024) return TM_ERR_ARG;
     static int raised = 0;          // largest dynamic LDS size this kernel has been allowed so far
     if (lds > 48 * 1024 && lds > raised) {
         if (hipFuncSetAttribute((const void*)fused_norm_gemm_kernel<EPI, ROWS, PIPE, WAVES, UNITS, PLAIN>,
