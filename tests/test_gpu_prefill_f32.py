@@ -79,3 +79,17 @@ def test_weights_over_the_whole_range_of_the_exponential(ops):
     # no roundings lean one way over a range: a correction of the wrong size or sign does (by up to 8 units at -86)
     for part in units.flatten().chunk(8):
         assert part.mean().abs() <= 0.5, part.mean()
+
+
+def test_more_tiles_than_one_launch_holds(ops):
+    """A table of 2^18 + 300 tiles at 64 heads (more than 2^32 threads), all the same but for the last, and so one with the last alone."""
+    H, D = 64, 16
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, kp, vp = (torch.randn(*shape, generator=g, device=DEV) for shape in ((2, H * D), (1, 16, 1, D), (1, 1, D, 16)))
+    tables = torch.zeros(1, 1, dtype=torch.int32, device=DEV)
+    tiles = torch.tensor([[0, 0, 1, 0]], dtype=torch.int32, device=DEV).repeat((1 << 18) + 300, 1)
+    tiles[-1] = torch.tensor([0, 1, 1, 1], device=DEV)
+    many, few = torch.full_like(q, 5.0), torch.empty_like(q)
+    ops.attn_prefill_f32(q, many, kp, vp, tables, tiles, H, 1, D, 0.25, 0)
+    ops.attn_prefill_f32(q, few, kp, vp, tables, tiles[-2:].contiguous(), H, 1, D, 0.25, 0)
+    assert torch.equal(many, few)

@@ -269,7 +269,7 @@ extern "C" int tm_attn_heads(const void* q, int ldq, const void* qr, const void*
     if (n_blocks <= 0) return TM_OK;
     if (!tm_attn_heads_takes(Dn, Dr, Dv) || H <= 0 || R <= 0 || R % 64 || window < 0 || !(scale > 0.f) || !blocks || ldq < H * (Dn + Dr) || ldq % 8 ||
         !ah_aligned(q) || !ah_aligned(qr) || !ah_aligned(kv) || !ah_aligned(vt) || !ah_aligned(out) || (gate && ldg < H) ||
-        (long long)R * (H * Dn + Dr) * 2 >= (1ll << 32) || (long long)H * Dv * R * 2 >= (1ll << 32) || (long long)n_blocks * H > 0x7fffffffLL)
+        (long long)R * (H * Dn + Dr) * 2 >= (1ll << 32) || (long long)H * Dv * R * 2 >= (1ll << 32) || (long long)n_blocks * H > 0xffffff)
         return TM_ERR_ARG;
     HeadsArgs a{(const bf16_t*)q, (const bf16_t*)qr, (const bf16_t*)kv, (const bf16_t*)vt, (bf16_t*)out, blocks, gate, sink,
                 (uint32_t)((long long)R * H * Dn * 2), ldq, ldg, H, R, window, scale * 1.4426950408889634f};

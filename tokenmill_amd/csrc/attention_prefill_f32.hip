@@ -235,15 +235,20 @@ extern "C" int tm_attn_prefill_f32_cap(const void* q, int q_stride, void* out, i
     if (H > 65535) return TM_ERR_ARG;
     int page_shift = 0;
     while ((1 << page_shift) < page) ++page_shift;
-    const unsigned grid = n_tiles * H;
+    // (a launch has fewer than 2^32 threads: tables beyond that go in pieces)
+    const int most = (1 << 23) / H;
 #define TM_PREFILL_F32_GO(DD, CAP)                                                                                \
-    attn_prefill_f32_kernel<DD, CAP><<<grid, 64 * AF_SPLIT, 0, stream>>>(                                         \
-        (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pool, (const float*)v_pool,           \
-        block_tables, table_width, tiles, H, KVH, page_shift, scale, window, keep, softcap, sink, (const float*)cgate, ldcg)
+    for (int t = 0; t < n_tiles; t += most)                                                                       \
+        attn_prefill_f32_kernel<DD, CAP><<<(n_tiles - t < most ? n_tiles - t : most) * H, 64 * AF_SPLIT, 0, stream>>>( \
+            (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pool, (const float*)v_pool,       \
+            block_tables, table_width, tiles + (size_t)t * 4, H, KVH, page_shift, scale, window, keep, softcap, sink, (const float*)cgate, ldcg)
 #define TM_PREFILL_F32_CASE(DD)                                                                                   \
     case DD:                                                                                                      \
-        if (softcap > 0.f) TM_PREFILL_F32_GO(DD, true);                                                           \
-        else TM_PREFILL_F32_GO(DD, false);                                                                        \
+        if (softcap > 0.f) {                                                                                      \
+            TM_PREFILL_F32_GO(DD, true);                                                                          \
+        } else {                                                                                                  \
+            TM_PREFILL_F32_GO(DD, false);                                                                         \
+        }                                                                                                         \
         break
     switch (D) {
         TM_PREFILL_F32_CASE(16);
