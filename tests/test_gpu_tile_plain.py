@@ -28,18 +28,26 @@ def test_plain_product(M, N, K, out_dtype):
     assert ((out[:M].double() - want).abs() <= bound + 1e-6).all() and (out[M] == 7).all()
 
 
-@pytest.mark.parametrize("M", [255, 256, 1500, 3072, 3073])
-@pytest.mark.parametrize("N,K", [(512, 1024), (4096, 1024), (1360, 4096), (4104, 1024)])
-def test_a_linear_on_both_sides_of_the_line(M, N, K):
-    g = torch.Generator(device=DEV).manual_seed(M)
+@pytest.mark.parametrize("N,K,tiled", [(512, 1024, {256, 640, 1024, 1200, 2048, 2560}), (504, 1024, set()), (512, 960, set()),
+                                       (2048, 1216, {256, 640, 1024, 1200, 2048, 2560}), (2056, 1216, set()), (1024, 2304, {640, 1024}), (512, 4096, set()),
+                                       (1360, 2304, {1200, 2048}), (1024, 2368, set()), (1032, 1280, set()), (2056, 2304, set()), (4096, 1024, set())])
+def test_a_linear_on_both_sides_of_the_lines(N, K, tiled):
+    """The ranges of rows that a plain product of each size runs tiled in: at their ends and one beyond."""
+    from tokenmill_amd import profiling
+
+    g = torch.Generator(device=DEV).manual_seed(N)
     lin = Linear(K, N, "w", bias=False)
     lin.load({"w.weight": (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(BF)}, "")
     lin.prepare(False)
-    x = torch.randn(M, K, generator=g, device=DEV).to(BF)
-    want = x.double() @ lin.weight.double().T
-    for out_dtype in (BF, torch.float32):
-        got = lin.forward(x, out_dtype=out_dtype)
-        assert (got.double() - want).norm() < (2.0 ** -8 if out_dtype == BF else 1e-6) * want.norm()
-        tiled = torch.empty_like(got)
-        if 256 <= M <= 3072 and N <= 4096:
-            assert torch.equal(got, ops.tile_linear(x, lin.weight, tiled))
+    for M in (255, 256, 639, 640, 1024, 1025, 1199, 1200, 2048, 2049, 2560, 2561):
+        x = torch.randn(M, K, generator=g, device=DEV).to(BF)
+        want = x.double() @ lin.weight.double().T
+        for out_dtype in (BF, torch.float32):
+            with profiling.collect() as seen:
+                got = lin.forward(x, out_dtype=out_dtype)
+            ran = any("gemm_tile_kernel" in name for name in seen["kernels"])
+            inside = M in tiled or (len(tiled) == 6 and M in (639, 1025, 1199, 2049))
+            assert ran == inside, (M, seen["kernels"])
+            assert (got.double() - want).norm() < (2.0 ** -8 if out_dtype == BF else 1e-6) * want.norm()
+            if inside:
+                assert torch.equal(got, ops.tile_linear(x, lin.weight, torch.empty_like(got)))

@@ -48,13 +48,20 @@ constexpr int TM_TILE_FEW_COLUMNS = 64 * 256;
 inline int tm_split_rows(int hidden) { return hidden < 3072 ? TM_SKINNY_ROWS : hidden <= 4096 ? 4 : TM_STREAM_ROWS; }
 // (what that does not take, such as a projection with a bias, is streamed where splitting its K over groups of blocks pays:
 // tm_stream_linear_parts in gemm_stream.hip; else it is the library's)
-// Plain products of prompts that run tiled in place of the library's untimed choice: where the tiles met or beat it (cold matrices, library /
-// tiled, 300 / 600 / 1,000 / 1,500 / 2,048 / 3,001 rows, us: 2,048 -> 2,048 10.9 / 13.7 / 15.5 / 19.0 / 21.1 / 26.1 to 9.4 / 12.3 / 13.4 / 17.5 /
-// 19.2 / 25.6; 1,024 -> 1,024 6.4 / 8.7 / 9.0 / 9.8 / 10.5 / 11.7 to 5.8 / 6.1 / 6.1 / 8.8 / 8.1 / 11.3; 4,096 -> 1,024 13.4 / 17.5 / 18.3 / 21.4 /
-// 25.4 / 28.3 to 13.8 / 14.7 / 14.8 / 20.9 / 21.9 / 28.4; 3,584 -> 3,584 19.5 / 26.5 / 30.7 / 38.5 / 46.8 / 70.7 to 18.0 / 24.7 / 27.1 / 37.6 / 44.5 /
-// 61.0), and a call of it costs the host half. Beyond them the library is up to 10% better at some sizes: 2,048 -> 8,192 43.5 to 45.0 and 49.2
-// to 52.7 at 1,500 and 2,048 rows, 768 -> 3,072 12.5 to 13.2 and 14.3 to 15.8, 8,192 -> 2,048 level, 4,864 -> 896 24.6 to 28.2 at 1,500.
-inline bool tm_tile_plain(int M, int N, int K) { return M >= 256 && M <= 3072 && N >= 512 && N <= 4096 && K >= 1024 && K <= 4096; }
+// Plain products of prompts that run tiled in place of the library's untimed choice, in three ranges of sizes where that is the better one (cold
+// matrices, time of the tiled product over the library's, 60 sizes drawn from each range, any / multiples of 64: mean, worst):
+//   256 to 2,560 rows, 512 to 2,048 columns, K below 1,280      0.81, 1.09 / 0.84, 1.09
+//   640 to 1,024 rows, up to 1,024 columns, K up to 2,304       0.80, 1.00 / 0.88, 1.02
+//   1,200 to 2,048 rows, 1,360 to 2,048 columns, K up to 2,304  0.86, 1.04 / 0.93, 1.06
+// and a call takes 8.6 us of the host for the library's 14.2. Beyond them the library is better as often as not, by up to a third: 4,096 -> 512 at
+// 300 / 1,000 rows 11.0 / 14.8 us to 15.5 / 16.9, 4,096 -> 1,024 at 300 / 3,001 15.2 / 31 to 18.5 / 35.8, 1,792 -> 2,560 at 500 1.33
+// times its time, 2,048 -> 1,360 at 777 to 1,024 1.11 to 1.18, 1,536 -> 4,096 at 1,200 1.14; also 768 -> 3,072 12.5 to 13.2 and 14.3 to 15.8 at
+// 1,500 and 2,048 rows, 4,864 -> 896 24.6 to 28.2 at 1,500.
+inline bool tm_tile_plain(int M, int N, int K) {
+    if (K < 1024 || N < 512) return false;
+    return (M >= 256 && M <= 2560 && N <= 2048 && K < 1280) || (M >= 640 && M <= 1024 && N <= 1024 && K <= 2304) ||
+           (M >= 1200 && M <= 2048 && N >= 1360 && N <= 2048 && K <= 2304);
+}
 // most rows one launch of the skinny product takes at all
 constexpr int TM_SKINNY_MAX_ROWS = 64;
 // most rows the 32-bit matrix-vector product takes
