@@ -37,8 +37,7 @@ struct GemvArgs {
 };
 
 // GROUP: steps of 16 k whose products meet in sums of their own before they join the running one. AHEAD: groups a wavefront asks for
-// at once: with one, a wavefront of the 0.5B shape waited for memory two or three times in a launch of 6 to 7 us (o 6.2 to 5.8, q|k|v 7.2
-// to 6.8, down 7.3 either way, gate|up, whose blocks a CU hide each other's waits, 12.9 either way).
+// at once: with one, a wavefront of the 0.5B shape waited for memory two times in a launch of 6 to 7 us (o 6.2 to 5.8, q|k|v 7.2 to 6.8).
 template <int EPI, int RT, int WAVES, int GROUP, int AHEAD>
 __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArgs a) {
     static_assert(EPI == GM_PLAIN || RT == 1, "");
@@ -209,15 +208,17 @@ extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, con
            (!bias || gm_aligned16(bias));
 }
 
-// Up to a block a CU, eight wavefronts split K into groups of four steps, two or three of them at a time; more blocks than that have four
-// wavefronts with groups of seven, two at a time where a block has one tile (two tiles, of the head: the registers of two groups leave
-// too few wavefronts a CU).
+// Up to a block a CU, eight wavefronts split K into groups of four steps; more blocks than that have four wavefronts with groups of seven, whose
+// blocks a CU hide each other's waits. A wavefront of the eight that has up to three groups asks for all of them at once; with more it
+// asks for a group at a time: what it asks for beyond its end is loads that others wait for (K cut into 16 steps a wavefront, 2,048 -> 2,048,
+// 1 / 8 / 16 rows, us: two rounds of three groups 9.4 / 11.5 / 13.5, four of one 7.7 / 8.6 / 10.0).
 #define GM_LAUNCH(EPI, RT, units, split)                                                                                    \
     do {                                                                                                                    \
         const int per_ = ((a.K / 16 + (split) - 1) / (split) + 7) / 8;                                                      \
-        if ((units) * (split) <= 256 && per_ <= 8) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2><<<dim3(units, split), 512, 0, stream>>>(a); \
-        else if ((units) * (split) <= 256) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3><<<dim3(units, split), 512, 0, stream>>>(a); \
-        else gemv_mfma_f32_kernel<EPI, RT, 4, 7, RT == 1 ? 2 : 1><<<dim3(units, split), 256, 0, stream>>>(a);               \
+        if ((units) * (split) > 256) gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1><<<dim3(units, split), 256, 0, stream>>>(a);     \
+        else if (per_ <= 4 || per_ > 12) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1><<<dim3(units, split), 512, 0, stream>>>(a); \
+        else if (per_ <= 8) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2><<<dim3(units, split), 512, 0, stream>>>(a);              \
+        else gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3><<<dim3(units, split), 512, 0, stream>>>(a);                             \
     } while (0)
 
 extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,
