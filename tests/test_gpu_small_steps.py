@@ -42,6 +42,24 @@ def test_few_tokens_against_64_bits_and_against_many_tokens(ops, N, K):
         assert torch.equal(acc, resid[:M] + out.to(BF).float())
 
 
+@pytest.mark.parametrize("N", [388, 1540, 3076])                     # strips of 4, 8 and 16 rows
+@pytest.mark.parametrize("K", [456, 640, 776, 1000, 1160, 1416, 2040, 2056, 2824, 3080, 3592, 4104, 4616, 5640, 6152, 12296])
+def test_every_depth_of_a_round(ops, N, K):
+    """Ranges of 4 to 16 k-steps in four parts and of 5 to 25 in sixteen, one to three rounds of each depth there is a kernel for."""
+    torch.manual_seed(K + N)
+    a = torch.randn(17, K, device=DEV).to(BF)
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).to(BF)
+    packed = ops.pack_weight(w, ops.skinny_strip_rows(N, K))
+    many = torch.empty(17, N, dtype=torch.float32, device=DEV)       # the kernel of more than 16 rows
+    ops.gemm_skinny(a, w, None, many)
+    assert (many - a.double() @ w.double().T).abs().max() < 1e-4
+    for M in (3, 8, 16):
+        for matrix in (packed, w):
+            out = torch.empty(M, N, dtype=torch.float32, device=DEV)
+            ops.gemm_skinny(a[:M], matrix, None, out)
+            assert torch.equal(out, many[:M]), (M, matrix is w)
+
+
 @pytest.mark.parametrize("M", [3, 7, 12])
 @pytest.mark.parametrize("N", [896, 1536])
 def test_what_is_no_number_stays_with_its_token_and_its_row(ops, M, N):

@@ -144,7 +144,12 @@ __global__ __launch_bounds__(64 * VW * ROWS / 16) void gemm_few_kernel(const bf1
                 const int k = a_k[b] + (base + j) * 32;
                 af[b][j].u = __builtin_amdgcn_raw_buffer_load_b128(abuf, base + j < per && k < a_end[b] ? (a_row + k) * 2 : BEYOND, 0, 0);
             }
-            wf[j].u = __builtin_amdgcn_raw_buffer_load_b128(wbuf, base + j < per ? w_at(base + j) : BEYOND, 0, 0);
+            if constexpr (PACKED) wf[j].u = __builtin_amdgcn_raw_buffer_load_b128(wbuf, base + j < per ? w_at(base + j) : BEYOND, 0, 0);
+        }
+        if constexpr (!PACKED) {                                     // (both halves of a line of the matrix one after the other)
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < CH; ++j) wf[j].u = __builtin_amdgcn_raw_buffer_load_b128(wbuf, base + j < per ? w_at(base + j) : BEYOND, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -187,6 +192,15 @@ __global__ __launch_bounds__(64 * VW * ROWS / 16) void gemm_few_kernel(const bf1
     }
 }
 
+// K-steps a round, for ranges of `per` of them: of the four depths a shape has kernels for, ascending, the last sets the rounds and the first
+// that does with as many is taken. What a round asks for beyond a range reads as zero, but passes the address unit all the same: with
+// one depth a shape (7, 8, 10 or 16) 896 -> 9,728 took 6.7 / 7.0 / 7.8 us at 1 / 8 / 16 tokens where it takes 5.1 / 5.5 / 6.7, 1,024 -> 1,024 and
+// 2,048 -> 2,048 at 16 tokens 4.4 and 5.8 where they take 3.7 and 4.9.
+static int few_depth(int per, int a, int b, int c, int d) {
+    const int rounds = (per + d - 1) / d;
+    return a * rounds >= per ? a : b * rounds >= per ? b : c * rounds >= per ? c : d;
+}
+
 // Ranges of K: 4, or 16 for a long K over few strips. `rows`: of a strip (16, 8 or 4).
 template <typename TC, bool PACKED>
 static int launch_few(const void* A, int lda, const void* W, int rows, const void* bias, int flags, void* C, int ldc, int M, int N,
@@ -201,19 +215,37 @@ static int launch_few(const void* A, int lda, const void* W, int rows, const voi
     }
     const int strips = (N + rows - 1) / rows;
     const bool long_k = K >= 2048 && !(rows == 16 && strips >= 256);
+    const int ksteps = (K + 31) / 32, per = long_k ? (ksteps + 15) / 16 : (ksteps + 3) / 4;
 #define TM_FEW(ROWS_, TOKS_, VW_, CH_)                                                                                \
     gemm_few_kernel<ROWS_, TOKS_, VW_, CH_, TC, PACKED><<<strips, 4 * VW_ * ROWS_, 0, stream>>>(                      \
         (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc)
-    if (rows == 4) {
-        if (M <= 4) { if (long_k) TM_FEW(4, 4, 16, 10); else TM_FEW(4, 4, 4, 7); }
-        else if (M <= 8) { if (long_k) TM_FEW(4, 8, 16, 10); else TM_FEW(4, 8, 4, 7); }
-        else { if (long_k) TM_FEW(4, 16, 16, 5); else TM_FEW(4, 16, 4, 7); }
-    } else if (rows == 8) {
-        if (M <= 8) { if (long_k) TM_FEW(8, 8, 16, 10); else TM_FEW(8, 8, 4, 8); }
-        else { if (long_k) TM_FEW(8, 16, 16, 10); else TM_FEW(8, 16, 4, 8); }
-    } else {
-        if (long_k) TM_FEW(16, 16, 16, 10); else TM_FEW(16, 16, 4, 16);
+#define TM_FEW_DEEP(ROWS_, TOKS_, VW_, A_, B_, C_, D_)                                                                \
+    switch (few_depth(per, A_, B_, C_, D_)) {                                                                         \
+        case A_: TM_FEW(ROWS_, TOKS_, VW_, A_); break;                                                                \
+        case B_: TM_FEW(ROWS_, TOKS_, VW_, B_); break;                                                                \
+        case C_: TM_FEW(ROWS_, TOKS_, VW_, C_); break;                                                                \
+        default: TM_FEW(ROWS_, TOKS_, VW_, D_);                                                                       \
     }
+    if (rows == 4 && long_k) {
+        if (M <= 4) { TM_FEW_DEEP(4, 4, 16, 4, 6, 8, 10) }
+        else if (M <= 8) { TM_FEW_DEEP(4, 8, 16, 4, 6, 8, 10) }
+        else { TM_FEW_DEEP(4, 16, 16, 4, 5, 6, 8) }
+    } else if (rows == 4) {
+        if (M <= 4) { TM_FEW_DEEP(4, 4, 4, 4, 6, 7, 8) }
+        else if (M <= 8) { TM_FEW_DEEP(4, 8, 4, 4, 6, 7, 8) }
+        else { TM_FEW_DEEP(4, 16, 4, 4, 6, 7, 8) }
+    } else if (rows == 8 && long_k) {
+        if (M <= 8) { TM_FEW_DEEP(8, 8, 16, 4, 6, 9, 11) }
+        else { TM_FEW_DEEP(8, 16, 16, 4, 6, 9, 11) }
+    } else if (rows == 8) {
+        if (M <= 8) { TM_FEW_DEEP(8, 8, 4, 4, 6, 7, 8) }
+        else { TM_FEW_DEEP(8, 16, 4, 4, 6, 7, 8) }
+    } else if (long_k) {
+        TM_FEW_DEEP(16, 16, 16, 5, 6, 8, 10)
+    } else {
+        TM_FEW_DEEP(16, 16, 4, 7, 8, 10, 14)
+    }
+#undef TM_FEW_DEEP
 #undef TM_FEW
     TM_CHECK_LAUNCH();
     return TM_OK;
