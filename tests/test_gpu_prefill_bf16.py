@@ -1,0 +1,40 @@
+"""The bfloat16 attention of prompt portions that splits keys: one, two and more heads of a kv head a wavefront give a head the same bits."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV, BF = "cuda:0", torch.bfloat16
+
+
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("n,window,softcap", [(1, 0, 0.0), (17, 0, 0.0), (333, 0, 0.0), (333, 70, 0.0), (260, 0, 20.0), (2100, 0, 0.0)])
+def test_a_heads_bits_do_not_depend_on_the_heads_beside_it(D, n, window, softcap):
+    from tokenmill_amd.hip import ops
+
+    H, page = 7, 16
+    g = torch.Generator(device=DEV).manual_seed(n + D)
+    pages = -(-n // page)
+    q = torch.randn(n, H * D, generator=g, device=DEV).to(BF)
+    k, v = torch.randn(pages, page, 1, D, generator=g, device=DEV).to(BF), torch.randn(pages, 1, D, page, generator=g, device=DEV).to(BF)
+    tables = torch.randperm(pages, generator=torch.Generator().manual_seed(n)).int().to(DEV).view(1, -1)
+    tiles = torch.tensor([(0, j, min(16, n - j), j) for j in reversed(range(0, n, 16))], dtype=torch.int32, device=DEV)
+
+    def attend(lo, hi):
+        out = torch.full((n, (hi - lo) * D), 3.0, dtype=BF, device=DEV)
+        ops.attn_prefill_mfma(q[:, lo * D:hi * D].contiguous(), out, k, v, tables, tiles, hi - lo, 1, D, D ** -0.5, window, softcap=softcap)
+        return out.view(n, hi - lo, D)
+
+    every = attend(0, H)
+    for lo, hi in ((0, 1), (6, 7), (2, 4), (3, 6)):
+        assert torch.equal(attend(lo, hi), every[:, lo:hi]), (lo, hi)
+    keys, values = k[tables[0].long()].view(-1, D)[:n].double(), v[tables[0].long()].permute(0, 3, 1, 2).reshape(-1, D)[:n].double()
+    s = torch.einsum("qhd,kd->hqk", q.view(n, H, D).double(), keys) * D ** -0.5
+    if softcap:
+        s = softcap * torch.tanh(s / softcap)
+    far = torch.arange(n, device=DEV)[:, None] - torch.arange(n, device=DEV)
+    s = s.masked_fill((far < 0) | (far >= (window or n)), float("-inf"))
+    want = torch.einsum("hqk,kd->qhd", s.softmax(-1), values)
+    # weights and results are rounded to 8 bits: 2^-9 of the largest value each, the capped score's fast tanh adds below that
+    assert (every.double() - want).abs().max() < 3 * 2.0 ** -9 * values.abs().max()

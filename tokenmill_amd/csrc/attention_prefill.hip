@@ -352,7 +352,9 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
 // Heads a wavefront takes and wavefronts a block has, by head size (registers decide). Up to head size 64 a
 // wavefront can hold four heads, which quarters the loads of a long prompt's keys; a short step, whose blocks of
 // two heads a wavefront still fit the chip in one round, takes those instead: twice the blocks, half as long
-// (512 tokens at the 0.5B shape: 13.4 to 9.8 us; a head's arithmetic is the same either way, so its bits are).
+// (512 tokens at the 0.5B shape: 13.4 to 9.8 us). A kv head of one or two heads takes no more than it has: places that stand empty cost
+// queries, room for partials in LDS and with it blocks a CU (8 heads of 64 and as many kv heads, 17 / 512 / 2,048 tokens, four places 5.9 / 9.2 /
+// 40.6 us, one 4.1 / 7.0 / 34.8). A head's arithmetic is the same either way, so its bits are.
 template <int D> struct PrefillShape { static constexpr int HPW = D <= 64 ? 4 : 2, KS = D <= 64 ? 8 : 4; };
 
 template <int D, int HPW, bool CAP>
@@ -403,7 +405,9 @@ extern "C" int tm_attn_prefill_mfma_cap(const void* q, int q_stride, void* out, 
 #define TM_PREFILL_CASE(DD)                                                                                       \
     case DD: {                                                                                                    \
         constexpr int HPW = PrefillShape<DD>::HPW;                                                                \
-        if (HPW > 2 && G > 2 && (long long)n_tiles * KVH * ((G + 1) / 2) <= TM_PREFILL_ONE_ROUND)                 \
+        if (G == 1)                                                                                               \
+            rc = softcap > 0.f ? launch_split_keys<DD, 1, true>(TM_SPLIT_ARGS) : launch_split_keys<DD, 1, false>(TM_SPLIT_ARGS); \
+        else if (HPW > 2 && (G == 2 || (long long)n_tiles * KVH * ((G + 1) / 2) <= TM_PREFILL_ONE_ROUND))          \
             rc = softcap > 0.f ? launch_split_keys<DD, 2, true>(TM_SPLIT_ARGS) : launch_split_keys<DD, 2, false>(TM_SPLIT_ARGS); \
         else                                                                                                      \
             rc = softcap > 0.f ? launch_split_keys<DD, HPW, true>(TM_SPLIT_ARGS) : launch_split_keys<DD, HPW, false>(TM_SPLIT_ARGS); \
