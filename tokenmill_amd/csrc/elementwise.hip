@@ -209,9 +209,9 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(float* __restr
 #pragma unroll
             for (int p = 0; p < PARTS; ++p) part[i][p] = row4(ps + (size_t)(p < pending.n_parts ? p : 0) * pending.stride, hidden, at(i));
         } else {
-            part[i][0] = row4(d, d ? hidden : 0, at(i));
+            if (d) part[i][0] = row4(d, hidden, at(i));
         }
-        if constexpr (GROUPS < 4) w[i] = row4(weight, hidden, at(i));
+        if constexpr (GROUPS < 4 || PARTS == 0) w[i] = row4(weight, hidden, at(i));
     };
     float ss = 0.f;
     auto add = [&](int i) {
@@ -234,8 +234,10 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(float* __restr
 #pragma unroll
         for (int i = 0; i < GROUPS; ++i) add(i);
     } else {                                                        // (more than the registers hold)
+        const int first = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~(TM_WAVE - 1));
 #pragma unroll
         for (int i = 0; i < GROUPS; ++i) {
+            if (4 * (first + i * THREADS) >= hidden) break;         // (a group that the wavefront does not have: its loads take their time too)
             load(i);
             add(i);
             __builtin_amdgcn_sched_barrier(0);
@@ -252,7 +254,7 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(float* __restr
     for (int i = 0; i < GROUPS; ++i) {
         if (at(i) < hidden) {
             ew_f32x4 y;
-            if constexpr (GROUPS == 4) w[i] = row4(weight, hidden, at(i));               // (no registers for it before)
+            if constexpr (GROUPS == 4 && PARTS > 0) w[i] = row4(weight, hidden, at(i));  // (no registers for it before)
 #pragma unroll
             for (int k = 0; k < 4; ++k) y[k] = w[i][k] * Elem<T>::round(v[i][k] * rs);   // rounded BEFORE the weight multiplies
             Vec4<T>::store(o + at(i), y);
@@ -287,6 +289,8 @@ static void launch_add_rmsnorm(float* resid, const void* delta, const float* par
     // 3.4 us with any); from the width alone: the sum of squares has one order per model
     if (!vec)
         add_rmsnorm_kernel<T, WT><<<R, 256, 0, stream>>>(resid, pending, rows, (const WT*)weight, (T*)out, hidden, eps);
+    else if (hidden <= 512)                                         // (wavefronts without a group add nothing: the same sum)
+        launch_add_rmsnorm_vec<T, WT, 128, 1>(resid, pending, rows, (const WT*)weight, (T*)out, R, hidden, eps, stream);
     else if (hidden <= 1024)
         launch_add_rmsnorm_vec<T, WT, 256, 1>(resid, pending, rows, (const WT*)weight, (T*)out, R, hidden, eps, stream);
     else if (hidden <= 2048)
