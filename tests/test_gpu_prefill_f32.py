@@ -93,3 +93,29 @@ def test_more_tiles_than_one_launch_holds(ops):
     ops.attn_prefill_f32(q, many, kp, vp, tables, tiles, H, 1, D, 0.25, 0)
     ops.attn_prefill_f32(q, few, kp, vp, tables, tiles[-2:].contiguous(), H, 1, D, 0.25, 0)
     assert torch.equal(many, few)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("window,keep,softcap", [(1, 0, 0.0), (16, 0, 0.0), (64, 0, 9.0), (128, 0, 0.0), (129, 0, 0.0), (40, 88, 0.0), (41, 88, 0.0), (20, 33, 9.0)])
+def test_windows_on_both_sides_of_a_short_walk(ops, D, window, keep, softcap):
+    """Walks without a block ahead (a window and what is kept beside it of at most 128 keys) and with one."""
+    n, H, KVH, page = 300, 6, 2, 16
+    g = torch.Generator(device=DEV).manual_seed(window + D)
+    q = torch.randn(n, H, D, generator=g, device=DEV)
+    pages = -(-n // page)
+    k, v = torch.randn(pages, page, KVH, D, generator=g, device=DEV), torch.randn(pages, KVH, D, page, generator=g, device=DEV)
+    tables = torch.randperm(pages, generator=torch.Generator().manual_seed(D)).int().to(DEV).view(1, -1)
+    tiles = torch.tensor([(0, j, min(16, n - j), j) for j in reversed(range(0, n, 16))], dtype=torch.int32, device=DEV)
+    out = torch.full((n, H * D), 3.0, device=DEV)
+    ops.attn_prefill_f32(q.view(n, H * D), out, k, v, tables, tiles, H, KVH, D, D ** -0.5, window, softcap=softcap, keep=keep)
+    keys = k[tables[0].long()].view(-1, KVH, D)[:n].double().repeat_interleave(H // KVH, 1)
+    values = v[tables[0].long()].permute(0, 3, 1, 2).reshape(-1, KVH, D)[:n].double().repeat_interleave(H // KVH, 1)
+    s = torch.einsum("qhd,khd->hqk", q.double(), keys) * D ** -0.5
+    if softcap:
+        s = softcap * torch.tanh(s / softcap)
+    place = torch.arange(n, device=DEV)
+    far = place[:, None] - place
+    s = s.masked_fill((far < 0) | ((far >= window) & (place >= keep)), float("-inf"))
+    want = torch.einsum("hqk,khd->qhd", s.softmax(-1), values).reshape(n, H * D)
+    # scores are sums of D products of unit size (their roundings 2^-24 D^0.5 of some 10), weights and sums of up to 129 values below 6
+    assert (out.double() - want).abs().max() < 2.0 ** -24 * (10 * D ** 0.5 + 200)

@@ -14,7 +14,7 @@
 //   The matrix instructions of a 1,000-token prompt of the 0.5B shape (14 heads of 64) take 12 us a layer. What stood beside them: the newest
 //   tiles' blocks met on the same CUs (52 us; 38 dealt out as below), accumulators that the vector unit had to fetch back and a
 //   branch for a cap (35), and sums rescaled at every block, expf, loads without a scalar base (30). The next block's keys and
-//   values are on their way while a block is multiplied.
+//   values are on their way while a block is multiplied (but in short windows).
 //
 //   S^T = K Q^T   A = keys  [16 keys x 4 d]   B = Q^T [4 d x 16 tokens]   (D / 4 steps; which d a step
 //                 multiplies is free as long as keys and queries agree: the lanes of group g = lane / 16
@@ -28,6 +28,10 @@
 #include "fused_common.h"
 
 #define AF_SPLIT 4          // wavefronts of a block; each takes every fourth key block
+// Keys a token sees at most where a wavefront's walk is two or three blocks: the block ahead is one that nobody wants then, and without its
+// registers a CU holds more blocks (14 heads of 64, a window of 64 / 128, 1,000 tokens, with it 12.2 / 14.9 us, without 10.5 / 13.1; 3,000
+// 25.9 / 33.4 and 22.9 / 29.9; at 256 keys 44.9 with it)
+#define AF_SHORT_WALK 128
 #define AF_ROUND 256        // blocks that come to rest on CUs of their own before the first CU gets a second one
 
 // A column's reference moves only when its maximum has grown by more than this (weights up to e^8 cost 32-bit sums nothing), so
@@ -43,14 +47,14 @@ __device__ __forceinline__ float exp_weight(float x) {
     return x < -104.f ? 0.f : __builtin_ldexpf(__builtin_amdgcn_exp2f(part), (int)whole);
 }
 
-// What a wavefront loads of a block of 16 keys.
+// What a wavefront loads of a block of 16 keys. AHEAD (below): the next block's are on their way while a block is multiplied.
 template <int D>
 struct KVBlock32 {
     f32x4_t k[D / 16], v[D / 16];
 };
 
-template <int D, bool CAP>
-__global__ __launch_bounds__(64 * AF_SPLIT, 2) void attn_prefill_f32_kernel(
+template <int D, bool CAP, bool AHEAD>
+__global__ __launch_bounds__(64 * AF_SPLIT, AHEAD ? 2 : 1) void attn_prefill_f32_kernel(
     const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
     const float* __restrict__ k_pool, const float* __restrict__ v_pool, const int* __restrict__ block_tables,
     int table_width, const int* __restrict__ tiles, int H, int KVH, int page_shift, float scale, int window, int keep, float softcap,
@@ -103,12 +107,18 @@ __global__ __launch_bounds__(64 * AF_SPLIT, 2) void attn_prefill_f32_kernel(
         for (int dt = 0; dt < NDT; ++dt) blk.v[dt] = as_f32x4(__builtin_amdgcn_raw_buffer_load_b128(vr, v_lane, (64 * dt) << page_shift, 0));
     };
     int kb = behind_gap(wave), next = behind_gap(kb + AF_SPLIT);
-    int pg_next = page_of(next);
+    int pg = page_of(kb), pg_next = page_of(next);
     auto attend = [&](KVBlock32<D>& now, KVBlock32<D>& then) {
         const int key0 = kb << 4;
         const int after = behind_gap(next + AF_SPLIT);
-        load(then, next, pg_next);                      // the next block, and the page of the one behind it
-        pg_next = page_of(after);
+        if constexpr (AHEAD) {
+            load(then, next, pg_next);                  // the next block, and the page of the one behind it
+            pg_next = page_of(after);
+        } else {
+            load(now, kb, pg);
+            pg = pg_next;
+            pg_next = page_of(after);
+        }
         __builtin_amdgcn_sched_barrier(0);
         // values of keys nobody may see yet (beyond the newest key) can hold anything: clear them
         if (key0 + 15 > last_key) {
@@ -166,11 +176,15 @@ __global__ __launch_bounds__(64 * AF_SPLIT, 2) void attn_prefill_f32_kernel(
         next = after;
     };
     KVBlock32<D> ba, bb;
-    load(ba, kb, page_of(kb));
-    while (kb <= kb_last) {
-        attend(ba, bb);
-        if (kb > kb_last) break;
-        attend(bb, ba);
+    if constexpr (AHEAD) {
+        load(ba, kb, pg);
+        while (kb <= kb_last) {
+            attend(ba, bb);
+            if (kb > kb_last) break;
+            attend(bb, ba);
+        }
+    } else {
+        while (kb <= kb_last) attend(ba, ba);
     }
     // o[dt][i] = sum for d = 16 dt + 4 g + i of token r; the column's sum is spread over its four lanes.
     // The four wavefronts' partial results meet in LDS; a wavefront that had no key block brings the lowest number as its reference, l = 0, o = 0
@@ -237,17 +251,18 @@ extern "C" int tm_attn_prefill_f32_cap(const void* q, int q_stride, void* out, i
     while ((1 << page_shift) < page) ++page_shift;
     // (a launch has fewer than 2^32 threads: tables beyond that go in pieces)
     const int most = (1 << 23) / H;
-#define TM_PREFILL_F32_GO(DD, CAP)                                                                                \
+    const bool short_walk = window > 0 && (long long)window + keep <= AF_SHORT_WALK;
+#define TM_PREFILL_F32_GO(DD, CAP, AHEAD)                                                                         \
     for (int t = 0; t < n_tiles; t += most)                                                                       \
-        attn_prefill_f32_kernel<DD, CAP><<<(n_tiles - t < most ? n_tiles - t : most) * H, 64 * AF_SPLIT, 0, stream>>>( \
+        attn_prefill_f32_kernel<DD, CAP, AHEAD><<<(n_tiles - t < most ? n_tiles - t : most) * H, 64 * AF_SPLIT, 0, stream>>>( \
             (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pool, (const float*)v_pool,       \
             block_tables, table_width, tiles + (size_t)t * 4, H, KVH, page_shift, scale, window, keep, softcap, sink, (const float*)cgate, ldcg)
 #define TM_PREFILL_F32_CASE(DD)                                                                                   \
     case DD:                                                                                                      \
-        if (softcap > 0.f) {                                                                                      \
-            TM_PREFILL_F32_GO(DD, true);                                                                          \
+        if (short_walk) {                                                                                         \
+            if (softcap > 0.f) { TM_PREFILL_F32_GO(DD, true, false); } else { TM_PREFILL_F32_GO(DD, false, false); } \
         } else {                                                                                                  \
-            TM_PREFILL_F32_GO(DD, false);                                                                         \
+            if (softcap > 0.f) { TM_PREFILL_F32_GO(DD, true, true); } else { TM_PREFILL_F32_GO(DD, false, true); } \
         }                                                                                                         \
         break
     switch (D) {
