@@ -24,9 +24,9 @@ inline int tm_skinny_rows(int hidden) { return hidden <= 1024 ? TM_SKINNY_ROWS :
 inline int tm_from_norm_rows(int hidden) { const int s = tm_skinny_rows(hidden); return s < 8 ? s : 8; }
 // q|k|v keeps the normed input in LDS behind a norm of its own up to this many rows where it fits (a width of at
 // most 1,024): its matrix is small enough that the copy of the input is most of any kernel's work (measured at the
-// 0.5B shape, 64 rows: 10.9 us against 14.9 us streamed). gate|up had such a kernel too; the stream product, with
-// the tiles of tokens dealt to two groups of blocks beyond 32 rows, is as fast or faster at every row count (0.5B
-// shape, a decode step of 12 / 24 / 32 / 48 requests: 1.07 / 1.29 / 1.34 / 1.54 ms against 1.08 / 1.32 / 1.38 / 1.54 ms).
+// 0.5B shape, 16 / 32 / 64 rows: 3.7 / 3.8 / 4.4 us against 5.5 / 6.6 / 8.4 streamed). gate|up had such a kernel too; the stream product, with
+// the tiles of tokens dealt to two groups of blocks beyond 32 rows, was as fast or faster at every row count while the kernel took twice its
+// present time (0.5B shape, a decode step of 12 / 24 / 32 / 48 requests: 1.07 / 1.29 / 1.34 / 1.54 ms against 1.08 / 1.32 / 1.38 / 1.54 ms).
 constexpr int TM_PANEL_QKV_ROWS = 64;
 // up to this many rows the products stream the packed matrix once for several row tiles, with their epilogues
 constexpr int TM_STREAM_ROWS = 64;

@@ -89,17 +89,14 @@ struct FusedUnit {
     int nA, nB;             // first rows of the strips
     int sA, sB;             // their indices in the packed matrix
     int head, jt;           // QKV: the head and which slice of it
-    bool rows_ok;           // this lane's rows exist
 };
-
 
 // Unit u of a product whose strips have ROWS rows.
 template <int EPI, int ROWS>
-__device__ __forceinline__ FusedUnit fused_unit_of(const FusedArgs& a, int u, int r) {
+__device__ __forceinline__ FusedUnit fused_unit_of(const FusedArgs& a, int u) {
     FusedUnit t;
     t.head = 0;
     t.jt = 0;
-    t.rows_ok = r < ROWS;
     if (EPI == FD_EPI_QKV) {
         t.head = unit_head(u, a.head_inverse);
         t.jt = u - t.head * (a.D / (2 * ROWS));

@@ -9,9 +9,9 @@
 //                   (reference src/infer/model/layers.py:142-147,60-64; src/infer/kv/paged_cache.py:40-43)
 //   SiLU epilogue : act = silu(x Wgate^T) * (x Wup^T)          (reference src/infer/model/layers.py:163-164)
 //
-// A block owns two strips of 16 matrix rows whose results meet in the epilogue (the two halves of a
-// rotary pair; gate and up). Its four wavefronts split K; partial sums are added through LDS in
-// wavefront order. Everything is rounded where the unfused path stores a bfloat16 tensor, so both
+// A unit is two strips of 16 or 8 matrix rows whose results meet in the epilogue (the two halves of a rotary pair; gate and up). Four or
+// eight wavefronts split its K; partial sums are added through LDS in wavefront order. A block takes one unit or two at a
+// time, and the next ones after them, behind one norm. Everything is rounded where the unfused path stores a bfloat16 tensor, so both
 // paths agree up to the order of 32-bit sums.
 #include "common.h"
 #include "api.h"
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
     __amdgpu_buffer_rsrc_t wA, wB;                                   // this wavefront's strips, up to the end of its k
     auto take_unit = [&](int u) {
         const bool live = u < n_units;                               // (the same in every lane)
-        cu = fused_unit_of<EPI, ROWS>(a, live ? u : 0, r);
+        cu = fused_unit_of<EPI, ROWS>(a, live ? u : 0);
         const int bytes = live && ks1 > ks0 ? ks1 * FRAG * 2 : 0;
         wA = fd_buffer(a.W + (size_t)cu.sA * ksteps * FRAG, bytes);
         wB = fd_buffer(a.W + (size_t)cu.sB * ksteps * FRAG, bytes);

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(64 * PN_WAVES, 1) void gemm_panel_kernel(const Fuse
         return e;
     };
     int u = blockIdx.x;
-    FusedUnit cu = fused_unit_of<FD_EPI_QKV, ROWS>(a, u, r);
+    FusedUnit cu = fused_unit_of<FD_EPI_QKV, ROWS>(a, u);
     load_group(cu);
     __builtin_amdgcn_sched_barrier(0);
     EpilogueInputs e_next = epilogue_inputs(cu);                     // (the positions came before the rows of x)
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(64 * PN_WAVES, 1) void gemm_panel_kernel(const Fuse
         const bool more = un < n_units;
         const FusedUnit done = cu;
         if (more) {
-            cu = fused_unit_of<FD_EPI_QKV, ROWS>(a, un, r);
+            cu = fused_unit_of<FD_EPI_QKV, ROWS>(a, un);
             load_group(cu);
             e_next = epilogue_inputs(cu);
         }
