@@ -36,10 +36,9 @@ struct GemvArgs {
     float* v_pool;              // [pages, KVH, D, page]
 };
 
-// AHEAD: steps of 16 k a wavefront asks for at once; their products meet in sums of their own before they join the running one.
-// (Two or three such groups asked for at once were no faster where they cover a wavefront's K, and what lies beyond it is loads that the others
-// wait for: 2,048 -> 2,048 at 1 / 16 rows 7.6 / 10.0 us with one, 9.4 / 13.5 with three.)
-template <int EPI, int RT, int WAVES, int AHEAD>
+// GROUP: steps of 16 k whose products meet in sums of their own before they join the running one. AHEAD: groups a wavefront asks for
+// at once: with one, a wavefront of the 0.5B shape waited for memory two times in a launch of 6 to 7 us (o 6.2 to 5.8, q|k|v 7.2 to 6.8).
+template <int EPI, int RT, int WAVES, int GROUP, int AHEAD>
 __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArgs a) {
     static_assert(EPI == GM_PLAIN || RT == 1, "");
     __shared__ __align__(16) f32x4_t red[WAVES][RT][TM_WAVE];
@@ -93,11 +92,11 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     f32x4_t sum[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) sum[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int s = s0; s < s1; s += AHEAD) {
-        f32x4_t w[RT][AHEAD], x[AHEAD];
+    for (int s = s0; s < s1; s += GROUP * AHEAD) {
+        f32x4_t w[RT][GROUP * AHEAD], x[GROUP * AHEAD];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
+        for (int i = 0; i < GROUP * AHEAD; ++i) {
             const int at = 16 * (s + i < s1 ? s + i : s1 - 1);  // (no load under a test: beyond the end the last step again)
 #pragma unroll
             for (int t = 0; t < RT; ++t) w[t][i] = *(const f32x4_t*)(pw[t] + at);
@@ -112,23 +111,27 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        // four sums a tile, of every fourth k, that join the running one here: short chains of roundings
-        f32x4_t acc[RT][4];
 #pragma unroll
-        for (int t = 0; t < RT; ++t)
+        for (int j = 0; j < AHEAD; ++j) {
+            if (s + j * GROUP >= s1) break;                     // the same for the whole wavefront
+            // four sums a tile, of every fourth k, that join the running one here: short chains of roundings
+            f32x4_t acc[RT][4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[t][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < RT; ++t)
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
-            if (s + i >= s1) break;                             // the same for the whole wavefront
+                for (int e = 0; e < 4; ++e) acc[t][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int i = j * GROUP; i < (j + 1) * GROUP; ++i) {
+                if (s + i >= s1) break;
 #pragma unroll
-                for (int t = 0; t < RT; ++t)
-                    acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i][e], x[i][e], acc[t][e], 0, 0, 0);
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int t = 0; t < RT; ++t)
+                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i][e], x[i][e], acc[t][e], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) sum[t] += (acc[t][0] + acc[t][1]) + (acc[t][2] + acc[t][3]);
         }
-#pragma unroll
-        for (int t = 0; t < RT; ++t) sum[t] += (acc[t][0] + acc[t][1]) + (acc[t][2] + acc[t][3]);
     }
 #pragma unroll
     for (int t = 0; t < RT; ++t) red[wave][t][lane] = sum[t];
@@ -205,13 +208,17 @@ extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, con
            (!bias || gm_aligned16(bias));
 }
 
-// Up to a block a CU, eight wavefronts split K and ask for four steps at a time; more blocks than that have four wavefronts with
-// seven (0.5B shape, eight rows: down 7.1 us against 8.2 to 9.0 for the other combinations of 4, 8, 16 and 4, 7; gate|up 12.1
-// against 12.0 to 13.7, head 126 against 127 to 131).
+// Up to a block a CU, eight wavefronts split K into groups of four steps; more blocks than that have four wavefronts with groups of seven, whose
+// blocks a CU hide each other's waits. A wavefront of the eight that has up to three groups asks for all of them at once; with more it
+// asks for a group at a time: what it asks for beyond its end is loads that others wait for (K cut into 16 steps a wavefront, 2,048 -> 2,048,
+// 1 / 8 / 16 rows, us: two rounds of three groups 9.4 / 11.5 / 13.5, four of one 7.7 / 8.6 / 10.0).
 #define GM_LAUNCH(EPI, RT, units, split)                                                                                    \
     do {                                                                                                                    \
-        if ((units) * (split) <= 256) gemv_mfma_f32_kernel<EPI, RT, 8, 4><<<dim3(units, split), 512, 0, stream>>>(a);       \
-        else gemv_mfma_f32_kernel<EPI, RT, 4, 7><<<dim3(units, split), 256, 0, stream>>>(a);                                \
+        const int per_ = ((a.K / 16 + (split) - 1) / (split) + 7) / 8;                                                      \
+        if ((units) * (split) > 256) gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1><<<dim3(units, split), 256, 0, stream>>>(a);     \
+        else if (per_ <= 4 || per_ > 12) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1><<<dim3(units, split), 512, 0, stream>>>(a); \
+        else if (per_ <= 8) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2><<<dim3(units, split), 512, 0, stream>>>(a);              \
+        else gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3><<<dim3(units, split), 512, 0, stream>>>(a);                             \
     } while (0)
 
 extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,
