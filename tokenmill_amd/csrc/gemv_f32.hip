@@ -211,7 +211,9 @@ extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, con
 // Up to a block a CU, eight wavefronts split K into groups of four steps; more blocks than that have four wavefronts with groups of seven, whose
 // blocks a CU hide each other's waits. A wavefront of the eight that has up to three groups asks for all of them at once; with more it
 // asks for a group at a time: what it asks for beyond its end is loads that others wait for (K cut into 16 steps a wavefront, 2,048 -> 2,048,
-// 1 / 8 / 16 rows, us: two rounds of three groups 9.4 / 11.5 / 13.5, four of one 7.7 / 8.6 / 10.0).
+// 1 / 8 / 16 rows, us: two rounds of three groups 9.4 / 11.5 / 13.5, four of one 7.7 / 8.6 / 10.0). Steps of the 0.5B shape with 1 / 8 / 16 requests
+// take 1,133 / 1,258 / 1,422 us so and 1,149 / 1,259 / 1,432 with a group at a time everywhere; launches in a row alone show no difference, and 3%
+// the other way where the groups are a quarter longer than K (2,816 -> 1,024 in four parts 4.7 to 4.8).
 #define GM_LAUNCH(EPI, RT, units, split)                                                                                    \
     do {                                                                                                                    \
         const int per_ = ((a.K / 16 + (split) - 1) / (split) + 7) / 8;                                                      \
