@@ -118,6 +118,10 @@ int tm_attn_decode_mfma_cap(const void* q, int q_stride, void* out, int out_stri
                             int max_chunks, int S, int H, int KVH, int D, int page, float scale, int window, int keep, float softcap,
                             const float* sink, const void* cgate, int ldcg, hipStream_t stream);
 
+int tm_attn_decode_whole(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool, const int* block_tables,
+                         int table_width, const int* context_lens, int max_chunks, int S, int H, int KVH, int D, int page, float scale, int window,
+                         int keep, float softcap, const float* sink, const void* cgate, int ldcg, hipStream_t stream);
+
 // The same work behind a short convolution over time (attention_prepare_conv.hip): see the head of that file.
 int tm_conv_norm_rope_store(const void* proj, int ld, int dtype, const void* conv_w, void* conv_state, int taps, const int* cu_q_lens,
                             const int* state_slots, const int* seq_of_token, int T, int first_single, int n_portions, void* q_out, int H,

@@ -4,7 +4,7 @@
 //   one MFMA tile, so the keys and values of a kv head are read once for all of them
 //   (the reference folds the group into query rows the same way: src/infer/model/layers.py:110-124).
 //   A wavefront always takes 64 consecutive keys, aligned to a multiple of 64 positions, and gets
-//   their unnormalised partial (max, sum, weighted values) in 32-bit. Two ways to cover a context:
+//   their unnormalised partial (max, sum, weighted values) in 32-bit. Three ways to cover a context:
 //
 //   block kernel : one block of 8 (16 for head size 32) wavefronts per (request, kv head); wavefront
 //                  w takes keys [64 (i W + w), +64) for i = 0, 1, ...; the partials are merged
@@ -14,6 +14,8 @@
 //                  the cache at speed: blocks of four wavefronts take chunks of 256 positions and
 //                  write partials to scratch memory; a second kernel adds the partials of a request
 //                  in ascending chunk order.
+//   whole kernel : where contexts are a few chunks long: the split kernels' partials and their order of
+//                  additions, in one block per (request, kv head).
 //
 //   Which keys meet in which partial and in which order partials are added depends on positions
 //   only, so within either way what a request gets does not depend on which other requests are in
@@ -24,6 +26,7 @@
 //   O^T = V^T P^T (16 d x 32 keys), and P^T comes straight from the S^T accumulators.
 #include "common.h"
 #include "api.h"
+#include "choose.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
@@ -528,6 +531,144 @@ __global__ __launch_bounds__(64 * AD_MERGE_WAVES) void attn_decode_merge_long_ke
     if (two) orow[lane + 64] = f32_to_bf16(o1 / ll);
 }
 
+// ------------------------------------------------------------------------------------------------
+// whole kernel: the split kernels' work in one launch, grid (S, KVH), for contexts of a few chunks
+// ------------------------------------------------------------------------------------------------
+// A block takes all chunks of a (request, kv head): wavefront w the 64 keys of run w, w + WAVES, ...; the partials of the runs
+// meet in LDS and are added as the split kernels add them (four runs to a chunk, every fourth chunk to a sum, the four sums in
+// order), with the same bits.
+//
+// Short contexts are bound by the trips to memory that wait for each other, of which the split kernels have two more (partials out and
+// in again, behind a launch); against that stands what one CU takes out of the caches, 55 to 60 GB/s whatever is asked for at once,
+// where the split kernels use a CU a chunk. Hence one round of loads, as many wavefronts as the context has runs (at most 16, 88
+// registers up to head size 64, 8 beyond and where pairs are so many that CUs hold two blocks). The partials meet in two passes of four elements a
+// thread: with one element a thread in one pass head size 128 took 1.6 us longer, with four elements in one pass 16 wavefronts spilled.
+// The rule and what it measured stand in choose.h (tm_decode_whole).
+template <int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attn_decode_whole_kernel(
+    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
+    const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
+    int table_width, const int* __restrict__ context_lens, int chunks, int H, int KVH, int page_shift, float scale_log2,
+    float cap_in, float cap_out, int window, int keep, const float* __restrict__ sink, const bf16_t* __restrict__ cgate, int ldcg) {
+    constexpr int NDT = D / 16, ROW = D + 4;
+    extern __shared__ __align__(16) float s_whole[];
+    const int s = blockIdx.x, kvh = blockIdx.y;
+    const int G = H / KVH;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;
+    const int r = lane % 16, g = lane / 16;
+    const int runs = 4 * chunks;
+    f32x2_t* s_ml = (f32x2_t*)s_whole;                               // [runs][16]: maximum and sum
+    f32x2_t* s_chunk = s_ml + runs * 16;                             // [chunks][16]: the same of a chunk
+    float* s_o = (float*)(s_chunk + chunks * 16);                    // [runs][G][ROW]
+    const int* table = block_tables + (size_t)s * table_width;
+    const int ctx = context_lens[s];
+    int entry[4];
+    load_table_entries(entry, table, table_width, wave * AD_WKEYS, page_shift);
+    Bf16x8Bits qreg[D / 32];
+    load_q_operand<D>(qreg, q + (size_t)s * q_stride, G, kvh, r, g);
+    const int p = ctx - 1;
+    const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
+    for (int run = wave; run < runs; run += WAVES) {
+        const int wbase = run * AD_WKEYS;
+        float m = -INFINITY, l = 0.f;
+        if (wbase < ctx && (wbase + AD_WKEYS > lo || wbase < keep)) {       // else nothing of the run is visible
+            f32x4_t o[NDT];
+            Keys64<D> kv;
+            load_keys64<D>(kv, k_pool, v_pool, entry, wbase, ctx, keep, lo, kvh, KVH, page_shift, r, g);
+            attend_keys64<D>(kv, qreg, wbase, ctx, keep, lo, scale_log2, cap_in, cap_out, g, m, l, o);
+            if (r < G) {
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt) *(f32x4_t*)(s_o + ((size_t)run * G + r) * ROW + 16 * dt + 4 * g) = o[dt];
+            }
+        }
+        if (g == 0) s_ml[run * 16 + r] = f32x2_t{m, l};
+        if (run + WAVES < runs) load_table_entries(entry, table, table_width, wbase + WAVES * AD_WKEYS, page_shift);
+    }
+    __syncthreads();
+    const int c1 = ctx <= chunks * AD_CHUNK ? (ctx - 1) / AD_CHUNK : chunks - 1;      // the last chunk that counts
+    // the runs of a chunk, four elements of a head a thread (what a chunk has takes the place of its first run's)
+    constexpr int PIECES = D / 4;
+    for (int idx = threadIdx.x; idx < (c1 + 1) * G * PIECES; idx += 64 * WAVES) {
+        const int cn = idx / PIECES, d = idx % PIECES * 4, c = cn / G, n = cn - c * G;
+        f32x2_t ml[4];
+        f32x4_t v[4], oc = {0.f, 0.f, 0.f, 0.f};
+        float* at = s_o + ((size_t)4 * c * G + n) * ROW + d;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            ml[w] = s_ml[(4 * c + w) * 16 + n];
+            v[w] = *(const f32x4_t*)(at + (size_t)w * G * ROW);
+        }
+        float mc = -INFINITY, lc = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) mc = fmaxf(mc, ml[w][0]);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const bool in = ml[w][0] != -INFINITY;                   // (nothing was stored where nothing is visible)
+            const float f = in ? __builtin_amdgcn_exp2f(ml[w][0] - mc) : 0.f;
+            lc = fmaf(ml[w][1], f, lc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) oc[i] = fmaf(in ? v[w][i] : 0.f, f, oc[i]);
+        }
+        *(f32x4_t*)at = oc;
+        if (d == 0) s_chunk[c * 16 + n] = f32x2_t{mc, lc};
+    }
+    __syncthreads();
+    // the chunks
+    for (int idx = threadIdx.x; idx < G * PIECES; idx += 64 * WAVES) {
+        const int n = idx / PIECES, d = idx % PIECES * 4;
+        float mm = -INFINITY;
+        for (int c = 0; c <= c1; ++c) mm = fmaxf(mm, s_chunk[c * 16 + n][0]);
+        float ll[4] = {0.f, 0.f, 0.f, 0.f};
+        f32x4_t oo[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) oo[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int cb = 0; cb <= c1; cb += 4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int c = cb + j < c1 ? cb + j : c1;
+                const f32x2_t ml = s_chunk[c * 16 + n];
+                const f32x4_t oc = *(const f32x4_t*)(s_o + ((size_t)4 * c * G + n) * ROW + d);
+                const float f = cb + j > c1 || ml[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[0] - mm);
+                ll[j] = fmaf(ml[1], f, ll[j]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) oo[j][i] = fmaf(oc[i], f, oo[j][i]);
+            }
+        }
+        float lsum = ll[0];
+        f32x4_t osum = oo[0];
+#pragma unroll
+        for (int j = 1; j < 4; ++j) {
+            lsum += ll[j];
+            osum += oo[j];
+        }
+        if (sink) lsum += __builtin_amdgcn_exp2f(sink[kvh * G + n] * 1.4426950408889634f - mm);     // a term of the denominator without a key
+        const size_t at = (size_t)(kvh * G + n) * D + d;
+        if (cgate) {                                                 // a gate per channel
+            const uint2 gp = *(const uint2*)(cgate + (size_t)s * ldcg + at);
+            osum[0] *= sigmoid_fast(__uint_as_float(gp.x << 16));
+            osum[1] *= sigmoid_fast(__uint_as_float(gp.x & 0xffff0000u));
+            osum[2] *= sigmoid_fast(__uint_as_float(gp.y << 16));
+            osum[3] *= sigmoid_fast(__uint_as_float(gp.y & 0xffff0000u));
+        }
+        *(uint2*)(out + (size_t)s * out_stride + at) = uint2{pack_bf16(osum[0] / lsum, osum[1] / lsum), pack_bf16(osum[2] / lsum, osum[3] / lsum)};
+    }
+}
+
+template <int D, int WAVES>
+static int launch_whole(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
+                        const int* block_tables, int table_width, const int* context_lens, int chunks, int S, int H, int KVH,
+                        int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep, const float* sink,
+                        const bf16_t* cgate, int ldcg, hipStream_t stream) {
+    static const hipError_t allowed = hipFuncSetAttribute((const void*)attn_decode_whole_kernel<D, WAVES>,
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)TM_DECODE_WHOLE_LDS);
+    if (allowed != hipSuccess) return TM_ERR_LAUNCH;
+    attn_decode_whole_kernel<D, WAVES><<<dim3(S, KVH), 64 * WAVES, tm_decode_whole_lds(chunks, H / KVH, D), stream>>>(
+        (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
+        table_width, context_lens, chunks, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
+    TM_CHECK_LAUNCH();
+    return TM_OK;
+}
+
 template <int D>
 static int launch_decode(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
                          const void* v_pool, const int* block_tables, int table_width, const int* context_lens,
@@ -564,6 +705,14 @@ static int launch_decode(const void* q, int q_stride, void* out, int out_stride,
     return TM_OK;
 }
 
+static bool decode_args_ok(const void* q, int q_stride, const void* out, int out_stride, int table_width, int max_chunks, int H, int KVH, int D,
+                           int page, float scale, int window, int keep, float softcap, const void* cgate, int ldcg) {
+    if (!(softcap >= 0.f) || keep < 0 || (cgate && (ldcg < H * D || ldcg % 4 || (uintptr_t)cgate % 8))) return false;
+    return !(H <= 0 || KVH <= 0 || H % KVH || H / KVH > 16 || page < 16 || (page & (page - 1)) || max_chunks <= 0 ||
+             !(scale > 0.f) || max_chunks > 65535 || KVH > 65535 || window < 0 || table_width <= 0 || (q_stride % 8) ||
+             ((uintptr_t)q % 16) || (out_stride % 4) || ((uintptr_t)out % 8) || q_stride < H * D || out_stride < H * D);
+}
+
 // q: first decode row (one row per request, rows q_stride apart); out likewise; block_tables and
 // context_lens: first decode request. part_o: float [S, H, max_chunks, D] and part_ml: [S, H, max_chunks, 2]
 // are scratch for the split kernels, which run when both are given (the caller gives them when the
@@ -578,12 +727,8 @@ extern "C" int tm_attn_decode_mfma_cap(const void* q, int q_stride, void* out, i
                                        int H, int KVH, int D, int page, float scale, int window, int keep, float softcap,
                                        const float* sink, const void* cgate, int ldcg, hipStream_t stream) {
     if (S <= 0) return TM_OK;
-    if (!(softcap >= 0.f) || keep < 0 || (cgate && (ldcg < H * D || ldcg % 4 || (uintptr_t)cgate % 8))) return TM_ERR_ARG;
+    if (!decode_args_ok(q, q_stride, out, out_stride, table_width, max_chunks, H, KVH, D, page, scale, window, keep, softcap, cgate, ldcg)) return TM_ERR_ARG;
     if (window == 0) keep = 0;
-    if (H <= 0 || KVH <= 0 || H % KVH || H / KVH > 16 || page < 16 || (page & (page - 1)) || max_chunks <= 0 ||
-        !(scale > 0.f) || max_chunks > 65535 || KVH > 65535 || window < 0 || table_width <= 0 || (q_stride % 8) ||
-        ((uintptr_t)q % 16) || (out_stride % 4) || ((uintptr_t)out % 8) || q_stride < H * D || out_stride < H * D)
-        return TM_ERR_ARG;
 #define TM_DECODE_CASE(DD)                                                                                        \
     case DD:                                                                                                      \
         return launch_decode<DD>(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width,         \
@@ -598,6 +743,48 @@ extern "C" int tm_attn_decode_mfma_cap(const void* q, int q_stride, void* out, i
             return TM_ERR_ARG;
     }
 #undef TM_DECODE_CASE
+}
+
+// The same by the whole kernel, for contexts of at most max_chunks chunks that its LDS holds (tm_decode_whole in choose.h says where it is
+// the better one). No scratch memory; the bits of the split kernels.
+template <int D>
+static int launch_whole_waves(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
+                              const int* block_tables, int table_width, const int* context_lens, int chunks, int S, int H, int KVH, int page,
+                              float scale, int window, int keep, float softcap, const float* sink, const bf16_t* cgate, int ldcg, hipStream_t stream) {
+    int page_shift = 0;
+    while ((1 << page_shift) < page) ++page_shift;
+    const float cap_in = softcap > 0.f ? scale / softcap : 0.f;
+#define TM_WHOLE(W)                                                                                                              \
+    launch_whole<D, W>(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, chunks, S, H, KVH, \
+                       page_shift, scale * 1.4426950408889634f, cap_in, softcap * 1.4426950408889634f, window, keep, sink, cgate, ldcg, stream)
+    if (chunks == 1) return TM_WHOLE(4);
+    if constexpr (D > 64) return TM_WHOLE(8);               // (12 and 16 wavefronts do not have the registers)
+    else return chunks == 2 || S * KVH > 256 ? TM_WHOLE(8) : chunks == 3 ? TM_WHOLE(12) : TM_WHOLE(16);
+#undef TM_WHOLE
+}
+
+extern "C" int tm_attn_decode_whole(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
+                                    const int* block_tables, int table_width, const int* context_lens, int max_chunks, int S, int H, int KVH,
+                                    int D, int page, float scale, int window, int keep, float softcap, const float* sink, const void* cgate,
+                                    int ldcg, hipStream_t stream) {
+    if (S <= 0) return TM_OK;
+    if (!decode_args_ok(q, q_stride, out, out_stride, table_width, max_chunks, H, KVH, D, page, scale, window, keep, softcap, cgate, ldcg) ||
+        tm_decode_whole_lds(max_chunks, H / KVH, D) > TM_DECODE_WHOLE_LDS)
+        return TM_ERR_ARG;
+    if (window == 0) keep = 0;
+#define TM_WHOLE_CASE(DD)                                                                                                                  \
+    case DD:                                                                                                                               \
+        return launch_whole_waves<DD>(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, max_chunks,  \
+                                      S, H, KVH, page, scale, window, keep, softcap, sink, (const bf16_t*)cgate, ldcg, stream)
+    switch (D) {
+        TM_WHOLE_CASE(32);
+        TM_WHOLE_CASE(64);
+        TM_WHOLE_CASE(96);
+        TM_WHOLE_CASE(128);
+        default:
+            return TM_ERR_ARG;
+    }
+#undef TM_WHOLE_CASE
 }
 
 extern "C" int tm_attn_decode_mfma(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,

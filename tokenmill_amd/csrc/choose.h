@@ -3,6 +3,7 @@
 // program (step_program.hip) is the only code that applies them; the Python side reads the numbers through
 // tm_rule() where it sizes a buffer or checks an argument, and never decides by them.
 #pragma once
+#include <stddef.h>
 
 // --- matrix products (bfloat16) ----------------------------------------------------------------------
 // up to this many rows the kernels that stream the matrix once win: the products over packed matrices with
@@ -75,9 +76,33 @@ constexpr int TM_DECODE_SPLIT_PAIRS = 192;  // below this many (request, kv head
 inline int tm_decode_chunks(int max_context) { return (max_context + TM_DECODE_CHUNK - 1) / TM_DECODE_CHUNK; }
 
 // Does a decode step of `requests` single tokens split its contexts over blocks (and need the scratch
-// memory for their partial results)?
+// memory for their partial results), where the whole kernel below does not take it?
 inline bool tm_decode_splits(int requests, int kv_heads, int max_context) {
     return requests * kv_heads < TM_DECODE_SPLIT_PAIRS && tm_decode_chunks(max_context) > 1;
+}
+
+// Does one block take all of a (request, kv head)'s context (attn_decode_whole_kernel; asked before the other)? Where there are few pairs two launches
+// less a trip to memory stand against one CU's share of the caches, where there are many the chunks would share CUs anyway, and against
+// the block kernel (one chunk, or 192 pairs and more) it merges in one pass. Us, split or block kernel to whole, by head size D:
+//   2 to 16 pairs, D 64   100 / 300 / 500 / 700 / 1,000 keys   5.7 / 6.6 / 6.6 / 6.7 / 6.6 to 4.5 / 5.6 / 6.1 / 7.2 / 8.5
+//   16 and 32,     D 128  100 / 300 / 500 / 700                8.6 / 8.8 / 9.0 / 9.4 to 5.2 / 7.6 / 9.3 / 11.4
+//   64,            D 32   300 / 700 / 1,000                    5.8 / 6.3 / 6.4 to 5.0 / 6.1 / 6.9
+//   96,            D 64   300 / 700 / 1,000 / 1,085            7.6 / 9.3 / 9.8 / 10.1 to 6.0 / 7.8 / 9.3 / 10.1
+//   128,           D 64   the same                             8.1 / 10.1 / 10.6 / 12.0 to 6.2 / 8.0 / 9.6 / 10.5
+//   96 and 128,    D 128  300 / 700 / 1,000                    9.7 / 12.8 / 14.2 and 10.1 / 14.2 / 16.1 to 7.8 / 11.7 / 16.6 and 7.9 / 12.2 / 18.5
+//   256,           D 64   300 / 700 / 1,085                    8.2 / 10.9 / 15.8 to 6.9 / 9.8 / 14.3
+//   192 and 400,   D 128  the same                             11.5 / 17.9 / 25.2 and 21.5 / 34.7 / 46.6 to 8.3 / 14.4 / 21.9 and 14.6 / 27.0 / 40.2
+constexpr int TM_DECODE_MANY_PAIRS = 96;
+constexpr int TM_DECODE_WHOLE_KEYS = 1280;
+constexpr size_t TM_DECODE_WHOLE_LDS = 160 * 1024;
+// its LDS: of the four runs of every chunk the maximum and sum of 16 heads and the values of the heads there are, and the former of every chunk
+inline size_t tm_decode_whole_lds(int chunks, int group, int head_size) { return (size_t)chunks * (32 + 4 * (32 + group * (head_size + 4))) * 4; }
+inline bool tm_decode_whole(int requests, int heads, int kv_heads, int head_size, int max_context) {
+    const int pairs = requests * kv_heads;
+    if (tm_decode_whole_lds(tm_decode_chunks(max_context), heads / kv_heads, head_size) > TM_DECODE_WHOLE_LDS) return false;
+    if (pairs >= TM_DECODE_SPLIT_PAIRS) return max_context <= TM_DECODE_WHOLE_KEYS;
+    if (pairs >= TM_DECODE_MANY_PAIRS) return max_context <= (head_size <= 64 ? TM_DECODE_WHOLE_KEYS : 768);
+    return max_context <= (head_size <= 32 ? 768 : head_size <= 64 ? 576 : 400);
 }
 
 // --- prefill attention (bfloat16) ---------------------------------------------------------------------

@@ -169,5 +169,7 @@ int tm_linear_run(const TmLinear* L, int x_dtype, const void* x, int ldx, int M,
 int tm_rule(const char* name);
 // Chunks a decode step's contexts are split into, or 0 if this step does not split them.
 int tm_decode_split_chunks(int requests, int kv_heads, int max_context);
+// 1 if one block a (request, kv head) takes all chunks of such a step (tm_attn_decode_whole; asked before the other)
+int tm_decode_takes_whole(int requests, int heads, int kv_heads, int head_size, int max_context);
 
 }  // extern "C"

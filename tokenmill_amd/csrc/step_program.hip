@@ -220,7 +220,7 @@ bool decode_in_chunks(const TmProgram* p, const TmAttentionOp& a, int num_decode
     if (num_decode <= 0) return false;
     if (p->dtype == TM_F32)         // (beyond that many pairs the generic kernel's blocks of one (token, head) pair fill the chip)
         return num_decode * a.KVH < TM_DECODE_SPLIT_PAIRS && tm_attn_decode_f32_takes(nullptr, a.H * a.D, a.k_pool, a.v_pool, a.H, a.KVH, a.D, a.page);
-    return tm_decode_splits(num_decode, a.KVH, context);
+    return tm_decode_splits(num_decode, a.KVH, context) && !tm_decode_whole(num_decode, a.H, a.KVH, a.D, context);
 }
 
 // chunks of such a step
@@ -499,7 +499,12 @@ struct Run {
             char* out_dec = (char*)attn + (size_t)tp * HD * es;
             if (nd && dtype == TM_BF16 && head_mfma && page_ok && a.H / a.KVH <= 16 && q_ok) {
                 const bool split = decode_in_chunks(p, a, nd, s->max_decode_context);
-                rc = tm_attn_decode_mfma_cap(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
+                if (tm_decode_whole(nd, a.H, a.KVH, a.D, s->max_decode_context))
+                    rc = tm_attn_decode_whole(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
+                                              s->context_lens + (S - nd), tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page,
+                                              a.scale, a.window, a.keep, a.softcap, a.sink, cg_dec, cgate_ld, stream);
+                else
+                    rc = tm_attn_decode_mfma_cap(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
                                              s->context_lens + (S - nd), split ? part_o : nullptr, split ? part_ml : nullptr,
                                              tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep,
                                              a.softcap, a.sink, cg_dec, cgate_ld, stream);
@@ -844,6 +849,10 @@ int tm_rule(const char* name) {
     if (!strcmp(name, "decode_chunk")) return TM_DECODE_CHUNK;
     if (!strcmp(name, "decode_split_pairs")) return TM_DECODE_SPLIT_PAIRS;
     return -1;
+}
+
+int tm_decode_takes_whole(int requests, int heads, int kv_heads, int head_size, int max_context) {
+    return requests > 0 && kv_heads > 0 && max_context > 0 && tm_decode_whole(requests, heads, kv_heads, head_size, max_context) ? 1 : 0;
 }
 
 int tm_decode_split_chunks(int requests, int kv_heads, int max_context) {

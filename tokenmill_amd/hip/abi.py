@@ -101,5 +101,7 @@ def bound():
     lib.tm_rule.argtypes = [c_char_p]
     lib.tm_decode_split_chunks.restype = c_int
     lib.tm_decode_split_chunks.argtypes = [c_int, c_int, c_int]
+    lib.tm_decode_takes_whole.restype = c_int
+    lib.tm_decode_takes_whole.argtypes = [c_int, c_int, c_int, c_int, c_int]
     lib._tm_program_bound = True
     return lib

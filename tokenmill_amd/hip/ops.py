@@ -615,15 +615,16 @@ def attn_decode_mfma(q: torch.Tensor, out: torch.Tensor, k_pool: torch.Tensor, v
                      block_tables: torch.Tensor, context_lens: torch.Tensor, H: int, KVH: int, D: int, scale: float,
                      window: int, max_context: int, workspace: tuple[torch.Tensor, torch.Tensor] | None = None,
                      split: bool | None = None, softcap: float = 0.0, sink: torch.Tensor | None = None, keep: int = 0,
-                     channel_gate: torch.Tensor | None = None):
+                     channel_gate: torch.Tensor | None = None, whole: bool | None = None):
     """Attention of one new token per request over its cache (the token's own key included); ``softcap`` > 0: a scaled
     score s becomes softcap * tanh(s / softcap); ``sink`` (float32 [H]): one more term exp(sink[h]) in the denominator;
     ``keep``: with a window, the first keys of a request that every token sees beside it; ``channel_gate`` (a view [S, >= H*D] of q's
     type): channel c of the result is multiplied by sigmoid of it.
     q: [S, >= H*D] rows (unit inner stride), out [S, H*D] view; block_tables int32 [S, W];
     context_lens int32 [S] (new token counted); max_context >= every context length. ``split``: None runs
-    the kernel the library's rule names for this many requests (contexts split over blocks and merged, or one
-    block a request and kv head); True / False name it (each kernel alone, in tests)."""
+    the kernel the library's rule names for this many requests (contexts split over blocks and merged, one
+    block a request and kv head, or, for short contexts, the split kernels' work in one block); True / False name
+    one of the first two, ``whole`` the third (each kernel alone, in tests)."""
     _gpu(q, out, k_pool, v_pool, block_tables, context_lens, sink)
     _check_sink(sink, H)
     S = q.shape[0]
@@ -644,6 +645,15 @@ def attn_decode_mfma(q: torch.Tensor, out: torch.Tensor, k_pool: torch.Tensor, v
     from tokenmill_amd.hip.abi import bound
     chunks = -(-max_context // rule("decode_chunk"))
     part_o = part_ml = None
+    if whole is None:
+        whole = split is None and bool(bound().tm_decode_takes_whole(S, H, KVH, D, max_context))
+    if whole:
+        _need(out_stride % 4 == 0 and out.data_ptr() % 8 == 0, "attn_decode: out rows must be 8-byte aligned")
+        _check(library().tm_attn_decode_whole(_p(q), c_int(q_stride), _p(out), c_int(out_stride), _p(k_pool), _p(v_pool),
+                                              _p(block_tables), c_int(W), _p(context_lens), c_int(chunks), c_int(S), c_int(H),
+                                              c_int(KVH), c_int(D), c_int(page), c_float(scale), c_int(window), c_int(keep),
+                                              c_float(softcap), _p(sink), _p(cgate), c_int(ldcg), _stream()), "attn_decode_whole")
+        return out
     if split is None:                                             # few (request, kv head) pairs: contexts split over blocks
         split = bool(bound().tm_decode_split_chunks(S, KVH, max_context))
     if split and chunks > 1:
