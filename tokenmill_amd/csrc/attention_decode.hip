@@ -27,6 +27,7 @@
 #include "common.h"
 #include "api.h"
 #include "choose.h"
+#include "ahead.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
@@ -324,13 +325,19 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_block_kernel(
 // ------------------------------------------------------------------------------------------------
 // split kernels: grid (S, KVH, chunks) with four wavefronts, then the merge
 // ------------------------------------------------------------------------------------------------
-template <int D>
+template <int D, bool AHEAD>
 __global__ __launch_bounds__(256) void attn_decode_split_kernel(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables, int table_width,
     const int* __restrict__ context_lens, float* __restrict__ part_o, float* __restrict__ part_ml,
-    int max_chunks, int H, int KVH, int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep) {
+    int max_chunks, int H, int KVH, int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep,
+    const TmAhead ahead) {
     constexpr int NDT = D / 16;
+    if constexpr (AHEAD) {
+        ahead_with(q, q_stride, k_pool, v_pool, block_tables, table_width, context_lens, part_o, part_ml, H, KVH, page_shift, scale_log2, cap_in, cap_out,
+                   window, keep);
+        if ((int)blockIdx.z >= max_chunks) return tm_bring_ahead(ahead, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), 4);
+    }
     __shared__ float s_m[4][16], s_l[4][16];
     __shared__ float s_o[4][16][D + 1];
     const int s = blockIdx.x, kvh = blockIdx.y, chunk = blockIdx.z;
@@ -544,13 +551,19 @@ __global__ __launch_bounds__(64 * AD_MERGE_WAVES) void attn_decode_merge_long_ke
 // registers up to head size 64, 8 beyond and where pairs are so many that CUs hold two blocks). The partials meet in two passes of four elements a
 // thread: with one element a thread in one pass head size 128 took 1.6 us longer, with four elements in one pass 16 wavefronts spilled.
 // The rule and what it measured stand in choose.h (tm_decode_whole).
-template <int D, int WAVES>
+template <int D, int WAVES, bool AHEAD>
 __global__ __launch_bounds__(64 * WAVES) void attn_decode_whole_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
     int table_width, const int* __restrict__ context_lens, int chunks, int H, int KVH, int page_shift, float scale_log2,
-    float cap_in, float cap_out, int window, int keep, const float* __restrict__ sink, const bf16_t* __restrict__ cgate, int ldcg) {
+    float cap_in, float cap_out, int window, int keep, const float* __restrict__ sink, const bf16_t* __restrict__ cgate, int ldcg,
+    const TmAhead ahead) {
     constexpr int NDT = D / 16, ROW = D + 4;
+    if constexpr (AHEAD) {
+        ahead_with(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, chunks, H, KVH, page_shift, scale_log2, cap_in,
+                   cap_out, window, keep, sink, cgate, ldcg);
+        if (blockIdx.z) return tm_bring_ahead(ahead, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), WAVES);
+    }
     extern __shared__ __align__(16) float s_whole[];
     const int s = blockIdx.x, kvh = blockIdx.y;
     const int G = H / KVH;
@@ -654,17 +667,29 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_whole_kernel(
     }
 }
 
-template <int D, int WAVES>
+// Layers of `pairs` blocks of a grid that has `own` of them, with those that bring matrices ahead.
+static int ahead_layers(TmAhead& ahead, int pairs, int own) {
+    const int more = ahead.n ? (ahead.blocks + pairs - 1) / pairs : 0;
+    if (own + more > 65535) {                                       // (no room in the grid)
+        ahead.n = 0;
+        return own;
+    }
+    ahead.first = pairs * own;
+    ahead.blocks = pairs * more;
+    return own + more;
+}
+
+template <int D, int WAVES, bool AHEAD>
 static int launch_whole(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                         const int* block_tables, int table_width, const int* context_lens, int chunks, int S, int H, int KVH,
                         int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep, const float* sink,
-                        const bf16_t* cgate, int ldcg, hipStream_t stream) {
-    static const hipError_t allowed = hipFuncSetAttribute((const void*)attn_decode_whole_kernel<D, WAVES>,
+                        const bf16_t* cgate, int ldcg, TmAhead& ahead, hipStream_t stream) {
+    static const hipError_t allowed = hipFuncSetAttribute((const void*)attn_decode_whole_kernel<D, WAVES, AHEAD>,
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)TM_DECODE_WHOLE_LDS);
     if (allowed != hipSuccess) return TM_ERR_LAUNCH;
-    attn_decode_whole_kernel<D, WAVES><<<dim3(S, KVH), 64 * WAVES, tm_decode_whole_lds(chunks, H / KVH, D), stream>>>(
+    attn_decode_whole_kernel<D, WAVES, AHEAD><<<dim3(S, KVH, ahead_layers(ahead, S * KVH, 1)), 64 * WAVES, tm_decode_whole_lds(chunks, H / KVH, D), stream>>>(
         (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
-        table_width, context_lens, chunks, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
+        table_width, context_lens, chunks, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg, ahead);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
@@ -674,7 +699,7 @@ static int launch_decode(const void* q, int q_stride, void* out, int out_stride,
                          const void* v_pool, const int* block_tables, int table_width, const int* context_lens,
                          float* part_o, float* part_ml, int max_chunks, int S, int H, int KVH, int page,
                          float scale, int window, int keep, float softcap, const float* sink, const bf16_t* cgate, int ldcg,
-                         hipStream_t stream) {
+                         TmAhead& ahead, hipStream_t stream) {
     int page_shift = 0;
     while ((1 << page_shift) < page) ++page_shift;
     const float scale_log2 = scale * 1.4426950408889634f;
@@ -691,9 +716,10 @@ static int launch_decode(const void* q, int q_stride, void* out, int out_stride,
         TM_CHECK_LAUNCH();
         return TM_OK;
     }
-    attn_decode_split_kernel<D><<<dim3(S, KVH, max_chunks), 256, 0, stream>>>(
+    const dim3 grid(S, KVH, ahead_layers(ahead, S * KVH, max_chunks));
+    (ahead.n ? attn_decode_split_kernel<D, true> : attn_decode_split_kernel<D, false>)<<<grid, 256, 0, stream>>>(
         (const bf16_t*)q, q_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables, table_width,
-        context_lens, part_o, part_ml, max_chunks, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep);
+        context_lens, part_o, part_ml, max_chunks, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, ahead);
     TM_CHECK_LAUNCH();
     if (max_chunks <= TM_WAVE)
         attn_decode_merge_kernel<<<dim3(S, H), 64 * AD_MERGE_WAVES, 0, stream>>>(
@@ -721,11 +747,11 @@ static bool decode_args_ok(const void* q, int q_stride, const void* out, int out
 // exp(sink[h]) in the denominator of head h's softmax, with no key behind it (added once, where a request's partials meet); with a window, `keep`: the first
 // keys of a request that every token sees beside its window; cgate (rows ldcg apart, a row a request) or null: channel c of the result is
 // multiplied by sigmoid(cgate[c]).
-extern "C" int tm_attn_decode_mfma_cap(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
+int attn_decode_ahead(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
                                        const void* v_pool, const int* block_tables, int table_width,
                                        const int* context_lens, float* part_o, float* part_ml, int max_chunks, int S,
                                        int H, int KVH, int D, int page, float scale, int window, int keep, float softcap,
-                                       const float* sink, const void* cgate, int ldcg, hipStream_t stream) {
+                                       const float* sink, const void* cgate, int ldcg, TmAhead ahead, hipStream_t stream) {
     if (S <= 0) return TM_OK;
     if (!decode_args_ok(q, q_stride, out, out_stride, table_width, max_chunks, H, KVH, D, page, scale, window, keep, softcap, cgate, ldcg)) return TM_ERR_ARG;
     if (window == 0) keep = 0;
@@ -733,7 +759,7 @@ extern "C" int tm_attn_decode_mfma_cap(const void* q, int q_stride, void* out, i
     case DD:                                                                                                      \
         return launch_decode<DD>(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width,         \
                                  context_lens, part_o, part_ml, max_chunks, S, H, KVH, page, scale, window, keep, softcap, sink,  \
-                                 (const bf16_t*)cgate, ldcg, stream)
+                                 (const bf16_t*)cgate, ldcg, ahead, stream)
     switch (D) {
         TM_DECODE_CASE(32);
         TM_DECODE_CASE(64);
@@ -745,28 +771,37 @@ extern "C" int tm_attn_decode_mfma_cap(const void* q, int q_stride, void* out, i
 #undef TM_DECODE_CASE
 }
 
+extern "C" int tm_attn_decode_mfma_cap(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
+                                       const void* v_pool, const int* block_tables, int table_width,
+                                       const int* context_lens, float* part_o, float* part_ml, int max_chunks, int S,
+                                       int H, int KVH, int D, int page, float scale, int window, int keep, float softcap,
+                                       const float* sink, const void* cgate, int ldcg, hipStream_t stream) {
+    return attn_decode_ahead(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, part_o, part_ml, max_chunks, S, H,
+                             KVH, D, page, scale, window, keep, softcap, sink, cgate, ldcg, TmAhead{}, stream);
+}
+
 // The same by the whole kernel, for contexts of at most max_chunks chunks that its LDS holds (tm_decode_whole in choose.h says where it is
 // the better one). No scratch memory; the bits of the split kernels.
 template <int D>
 static int launch_whole_waves(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                               const int* block_tables, int table_width, const int* context_lens, int chunks, int S, int H, int KVH, int page,
-                              float scale, int window, int keep, float softcap, const float* sink, const bf16_t* cgate, int ldcg, hipStream_t stream) {
+                              float scale, int window, int keep, float softcap, const float* sink, const bf16_t* cgate, int ldcg, TmAhead& ahead, hipStream_t stream) {
     int page_shift = 0;
     while ((1 << page_shift) < page) ++page_shift;
     const float cap_in = softcap > 0.f ? scale / softcap : 0.f;
 #define TM_WHOLE(W)                                                                                                              \
-    launch_whole<D, W>(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, chunks, S, H, KVH, \
-                       page_shift, scale * 1.4426950408889634f, cap_in, softcap * 1.4426950408889634f, window, keep, sink, cgate, ldcg, stream)
+    (ahead.n ? launch_whole<D, W, true> : launch_whole<D, W, false>)(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, chunks, S, H, KVH, \
+                       page_shift, scale * 1.4426950408889634f, cap_in, softcap * 1.4426950408889634f, window, keep, sink, cgate, ldcg, ahead, stream)
     if (chunks == 1) return TM_WHOLE(4);
     if constexpr (D > 64) return TM_WHOLE(8);               // (12 and 16 wavefronts do not have the registers)
     else return chunks == 2 || S * KVH > 256 ? TM_WHOLE(8) : chunks == 3 ? TM_WHOLE(12) : TM_WHOLE(16);
 #undef TM_WHOLE
 }
 
-extern "C" int tm_attn_decode_whole(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
+int attn_decode_whole_ahead(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                                     const int* block_tables, int table_width, const int* context_lens, int max_chunks, int S, int H, int KVH,
                                     int D, int page, float scale, int window, int keep, float softcap, const float* sink, const void* cgate,
-                                    int ldcg, hipStream_t stream) {
+                                    int ldcg, TmAhead ahead, hipStream_t stream) {
     if (S <= 0) return TM_OK;
     if (!decode_args_ok(q, q_stride, out, out_stride, table_width, max_chunks, H, KVH, D, page, scale, window, keep, softcap, cgate, ldcg) ||
         tm_decode_whole_lds(max_chunks, H / KVH, D) > TM_DECODE_WHOLE_LDS)
@@ -775,7 +810,7 @@ extern "C" int tm_attn_decode_whole(const void* q, int q_stride, void* out, int 
 #define TM_WHOLE_CASE(DD)                                                                                                                  \
     case DD:                                                                                                                               \
         return launch_whole_waves<DD>(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, max_chunks,  \
-                                      S, H, KVH, page, scale, window, keep, softcap, sink, (const bf16_t*)cgate, ldcg, stream)
+                                      S, H, KVH, page, scale, window, keep, softcap, sink, (const bf16_t*)cgate, ldcg, ahead, stream)
     switch (D) {
         TM_WHOLE_CASE(32);
         TM_WHOLE_CASE(64);
@@ -785,6 +820,14 @@ extern "C" int tm_attn_decode_whole(const void* q, int q_stride, void* out, int 
             return TM_ERR_ARG;
     }
 #undef TM_WHOLE_CASE
+}
+
+extern "C" int tm_attn_decode_whole(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
+                                    const int* block_tables, int table_width, const int* context_lens, int max_chunks, int S, int H, int KVH,
+                                    int D, int page, float scale, int window, int keep, float softcap, const float* sink, const void* cgate,
+                                    int ldcg, hipStream_t stream) {
+    return attn_decode_whole_ahead(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, max_chunks, S, H, KVH, D, page,
+                                   scale, window, keep, softcap, sink, cgate, ldcg, TmAhead{}, stream);
 }
 
 extern "C" int tm_attn_decode_mfma(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,

@@ -117,3 +117,9 @@ __device__ __forceinline__ FusedUnit fused_unit_of(const FusedArgs& a, int u) {
     }
     return t;
 }
+
+// Blocks of the gate|up product that starts at the norm: one round, each with the same number of pairs of strips (tm_fused_norm_gate_up_silu).
+inline int fused_gate_up_blocks(int I) {
+    const int units = (I + 15) / 16, per_block = (units + 255) / 256;
+    return (units + per_block - 1) / per_block;
+}

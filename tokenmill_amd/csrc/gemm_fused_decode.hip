@@ -16,6 +16,9 @@
 #include "common.h"
 #include "api.h"
 #include "fused_common.h"
+#include "ahead.h"
+
+#include <type_traits>
 
 // Elements between the rows of x in LDS: whole k-steps, one of zeros and the padding.
 __host__ __device__ __forceinline__ int fused_norm_stride(int K) { return fused_x_stride(K) + 32; }
@@ -37,10 +40,17 @@ __host__ __device__ __forceinline__ int fused_norm_stride(int K) { return fused_
 //
 // PLAIN: the norm's weights are bfloat16 and the threads that share a row hold all of it in one round of loads (launch_fused_shape):
 // straight code from the loads to LDS. The other way takes any K and either type.
-template <int EPI, int ROWS, bool PIPE, int WAVES, int UNITS, bool PLAIN>
+template <int EPI, int ROWS, bool PIPE, int WAVES, int UNITS, bool PLAIN, bool AHEAD>
 __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) void fused_norm_gemm_kernel(const FusedArgs a,
-                                                                                                       const int n_units) {
+                                                                                                       const int n_units, const int blocks,
+                                                                                                       const TmAhead ahead) {
     constexpr int KCH = PIPE ? FD_KCH_PIPE : FD_KCH;
+    if constexpr (AHEAD) {
+        ahead_with(a.resid, a.norm_w, a.norm_w_f32, a.eps, a.M, a.K, a.W, n_units);
+        if constexpr (EPI == FD_EPI_QKV) ahead_with(a.bias, a.bias_f32, a.H, a.KVH, a.D, a.head_inverse, a.cos_t, a.sin_t, a.positions, a.slots);
+        else ahead_with(a.up_strip0, a.act_out, a.I);
+        if ((int)blockIdx.x >= blocks) return tm_bring_ahead(ahead, blockIdx.x, WAVES * UNITS);
+    }
     constexpr int THREADS = 64 * WAVES * UNITS, RC = PLAIN ? fused_row_vectors(THREADS) : FD_RC;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t* xs = (bf16_t*)smem_raw;                                  // [4, 8 or 16 rows][fused_norm_stride]
@@ -114,7 +124,7 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
     __builtin_amdgcn_sched_barrier(0);
     FFrag fa[KCH], fb[KCH], fa2[PIPE ? KCH : 1], fb2[PIPE ? KCH : 1];
     int u0 = blockIdx.x;
-    take_unit(u0 + slot_of_block * gridDim.x);
+    take_unit(u0 + slot_of_block * blocks);
     load_group(fa, fb, ks0);
     if constexpr (PIPE) load_group(fa2, fb2, ks0 + KCH);
     __builtin_amdgcn_sched_barrier(0);
@@ -270,11 +280,11 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
 
         // the next units' first loads go out before these units' epilogue
         const FusedUnit done = cu;
-        const bool done_live = u0 + slot_of_block * (int)gridDim.x < n_units;
-        u0 += UNITS * gridDim.x;
+        const bool done_live = u0 + slot_of_block * blocks < n_units;
+        u0 += UNITS * blocks;
         const bool more = u0 < n_units;
         if (more) {
-            take_unit(u0 + slot_of_block * gridDim.x);
+            take_unit(u0 + slot_of_block * blocks);
             load_group(fa, fb, ks0);
             if constexpr (PIPE) load_group(fa2, fb2, ks0 + KCH);
             e_next = epilogue_inputs();
@@ -361,48 +371,53 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
 // Dynamic LDS of a launch: the normed rows.
 static int fused_lds_bytes(int M, int K) { return fused_rows(M) * fused_norm_stride(K) * (int)sizeof(bf16_t); }
 
-template <int EPI, int ROWS, bool PIPE, int WAVES, int UNITS, bool PLAIN>
-static int launch_fused_kernel(const FusedArgs& a, int n_units, int blocks, hipStream_t stream) {
+template <int EPI, int ROWS, bool PIPE, int WAVES, int UNITS, bool PLAIN, bool AHEAD>
+static int launch_fused_kernel(const FusedArgs& a, int n_units, int blocks, TmAhead& ahead, hipStream_t stream) {
     const int lds = fused_lds_bytes(a.M, a.K);
     if (lds + (int)sizeof(f32x4_t) * UNITS * WAVES * 2 * 64 > 160 * 1024) return TM_ERR_ARG;
     static int raised = 0;          // largest dynamic LDS size this kernel has been allowed so far
     if (lds > 48 * 1024 && lds > raised) {
-        if (hipFuncSetAttribute((const void*)fused_norm_gemm_kernel<EPI, ROWS, PIPE, WAVES, UNITS, PLAIN>,
+        if (hipFuncSetAttribute((const void*)fused_norm_gemm_kernel<EPI, ROWS, PIPE, WAVES, UNITS, PLAIN, AHEAD>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
             return TM_ERR_LAUNCH;
         raised = lds;
     }
-    fused_norm_gemm_kernel<EPI, ROWS, PIPE, WAVES, UNITS, PLAIN><<<blocks, 64 * WAVES * UNITS, lds, stream>>>(a, n_units);
+    ahead.first = blocks;
+    fused_norm_gemm_kernel<EPI, ROWS, PIPE, WAVES, UNITS, PLAIN, AHEAD><<<blocks + (ahead.n ? ahead.blocks : 0), 64 * WAVES * UNITS, lds, stream>>>(
+        a, n_units, blocks, ahead);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
 
 template <int EPI, int ROWS, bool PIPE, int WAVES, int UNITS>
-static int launch_fused_shape(const FusedArgs& a, int n_units, int blocks, hipStream_t stream) {
+static int launch_fused_shape(const FusedArgs& a, int n_units, int blocks, TmAhead& ahead, hipStream_t stream) {
     constexpr int THREADS = 64 * WAVES * UNITS;
     const int share = THREADS / fused_rows(a.M), tpr = share < TM_WAVE ? share : TM_WAVE;
-    if (WAVES == 4 && !a.norm_w_f32 && a.K <= fused_row_vectors(THREADS) * 4 * tpr)
-        return launch_fused_kernel<EPI, ROWS, PIPE, WAVES, UNITS, WAVES == 4>(a, n_units, blocks, stream);
-    return launch_fused_kernel<EPI, ROWS, PIPE, WAVES, UNITS, false>(a, n_units, blocks, stream);
+    auto go = [&](auto PLAIN) {
+        return ahead.n ? launch_fused_kernel<EPI, ROWS, PIPE, WAVES, UNITS, decltype(PLAIN)::value, true>(a, n_units, blocks, ahead, stream)
+                       : launch_fused_kernel<EPI, ROWS, PIPE, WAVES, UNITS, decltype(PLAIN)::value, false>(a, n_units, blocks, ahead, stream);
+    };
+    if (WAVES == 4 && !a.norm_w_f32 && a.K <= fused_row_vectors(THREADS) * 4 * tpr) return go(std::integral_constant<bool, WAVES == 4>{});
+    return go(std::false_type{});
 }
 
 // A long K gets 8 wavefronts a unit (shorter K ranges, a faster norm); whether a wavefront's range
 // needs more than one register group of loads decides the pipelined variant. With a shorter K a block that has several units
 // takes two at a time, so that the second's matrix is on its way with the first's.
 template <int EPI, int ROWS>
-static int launch_fused(const FusedArgs& a, int n_units, int blocks, hipStream_t stream) {
+static int launch_fused(const FusedArgs& a, int n_units, int blocks, TmAhead& ahead, hipStream_t stream) {
     const int ksteps = (a.K + 31) / 32;
     if (a.K >= 2048) {
-        return (ksteps + 7) / 8 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 8, 1>(a, n_units, blocks, stream)
-                                         : launch_fused_shape<EPI, ROWS, false, 8, 1>(a, n_units, blocks, stream);
+        return (ksteps + 7) / 8 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 8, 1>(a, n_units, blocks, ahead, stream)
+                                         : launch_fused_shape<EPI, ROWS, false, 8, 1>(a, n_units, blocks, ahead, stream);
     }
     if constexpr (EPI == FD_EPI_SILU) {
         if (n_units > blocks)
-            return (ksteps + 3) / 4 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 4, 2>(a, n_units, blocks, stream)
-                                             : launch_fused_shape<EPI, ROWS, false, 4, 2>(a, n_units, blocks, stream);
+            return (ksteps + 3) / 4 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 4, 2>(a, n_units, blocks, ahead, stream)
+                                             : launch_fused_shape<EPI, ROWS, false, 4, 2>(a, n_units, blocks, ahead, stream);
     }
-    return (ksteps + 3) / 4 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 4, 1>(a, n_units, blocks, stream)
-                                     : launch_fused_shape<EPI, ROWS, false, 4, 1>(a, n_units, blocks, stream);
+    return (ksteps + 3) / 4 > FD_KCH ? launch_fused_shape<EPI, ROWS, true, 4, 1>(a, n_units, blocks, ahead, stream)
+                                     : launch_fused_shape<EPI, ROWS, false, 4, 1>(a, n_units, blocks, ahead, stream);
 }
 
 static bool fused_common_ok(int M, int K, const void* resid, const void* W) {
@@ -421,10 +436,10 @@ extern "C" int tm_fused_qkv_strip_rows(int H, int KVH, int D, int K) {
 // q_out[M, H*D], K cache, V cache <- rope(norm(resid) Wqkv^T + b).  Needs M <= 16, D % 32 == 0, a
 // rotary table over the whole head, page a power of two. W: the [(H + 2 KVH) D, K] matrix packed in
 // strips of tm_fused_qkv_strip_rows(H, KVH, D, K) rows.
-extern "C" int tm_fused_norm_qkv_rope(const float* resid, const void* norm_w, int norm_w_dtype, float eps, int M,
+int fused_norm_qkv_rope_ahead(const float* resid, const void* norm_w, int norm_w_dtype, float eps, int M,
                                       int K, const void* W, const void* bias, int bias_dtype, void* q_out, int H,
                                       int KVH, int D, const float* cos_t, const float* sin_t, const int* positions,
-                                      const int* slots, void* k_pool, void* v_pool, int page, hipStream_t stream) {
+                                      const int* slots, void* k_pool, void* v_pool, int page, TmAhead ahead, hipStream_t stream) {
     if (M == 0) return TM_OK;
     if (!fused_common_ok(M, K, resid, W) || H <= 0 || KVH <= 0 || D <= 0 || D % 32 || !cos_t || !sin_t || !positions ||
         !q_out || ((uintptr_t)q_out % 8) || page <= 0 || (page & (page - 1)) || !(eps > 0.f))
@@ -441,14 +456,22 @@ extern "C" int tm_fused_norm_qkv_rope(const float* resid, const void* norm_w, in
     const int units16 = (H + 2 * KVH) * (D / 32);
     const int rows = tm_fused_qkv_strip_rows(H, KVH, D, K);
     a.head_inverse = unit_inverse(D / (2 * rows));
-    if (rows == 16) return launch_fused<FD_EPI_QKV, 16>(a, units16, units16, stream);
-    return launch_fused<FD_EPI_QKV, 8>(a, 2 * units16, 2 * units16, stream);
+    if (rows == 16) return launch_fused<FD_EPI_QKV, 16>(a, units16, units16, ahead, stream);
+    return launch_fused<FD_EPI_QKV, 8>(a, 2 * units16, 2 * units16, ahead, stream);
+}
+
+extern "C" int tm_fused_norm_qkv_rope(const float* resid, const void* norm_w, int norm_w_dtype, float eps, int M,
+                                      int K, const void* W, const void* bias, int bias_dtype, void* q_out, int H,
+                                      int KVH, int D, const float* cos_t, const float* sin_t, const int* positions,
+                                      const int* slots, void* k_pool, void* v_pool, int page, hipStream_t stream) {
+    return fused_norm_qkv_rope_ahead(resid, norm_w, norm_w_dtype, eps, M, K, W, bias, bias_dtype, q_out, H, KVH, D, cos_t, sin_t, positions, slots, k_pool, v_pool, page,
+        TmAhead{}, stream);
 }
 
 // act[M, I] <- silu(norm(resid) Wg^T) * (norm(resid) Wu^T).  Needs M <= 16. W: Wg [I, K] and Wu [I, K]
 // each packed in strips of 16 rows, Wu behind Wg.
-extern "C" int tm_fused_norm_gate_up_silu(const float* resid, const void* norm_w, int norm_w_dtype, float eps, int M,
-                                          int K, const void* W, void* act_out, int I, hipStream_t stream) {
+int fused_norm_gate_up_silu_ahead(const float* resid, const void* norm_w, int norm_w_dtype, float eps, int M,
+                                          int K, const void* W, void* act_out, int I, TmAhead ahead, hipStream_t stream) {
     if (M == 0) return TM_OK;
     if (!fused_common_ok(M, K, resid, W) || I <= 0 || !act_out || ((uintptr_t)act_out % 8) || (I % 4) || !(eps > 0.f))
         return TM_ERR_ARG;
@@ -461,6 +484,11 @@ extern "C" int tm_fused_norm_gate_up_silu(const float* resid, const void* norm_w
     // shape's 1,184 as 237 blocks of five (the same as 256 blocks of four or five).
     const int units = (I + 15) / 16;
     a.up_strip0 = units;
-    const int per_block = (units + 255) / 256;
-    return launch_fused<FD_EPI_SILU, 16>(a, units, (units + per_block - 1) / per_block, stream);
+    return launch_fused<FD_EPI_SILU, 16>(a, units, fused_gate_up_blocks(I), ahead, stream);
+}
+
+extern "C" int tm_fused_norm_gate_up_silu(const float* resid, const void* norm_w, int norm_w_dtype, float eps, int M,
+                                          int K, const void* W, void* act_out, int I, hipStream_t stream) {
+    return fused_norm_gate_up_silu_ahead(resid, norm_w, norm_w_dtype, eps, M, K, W, act_out, I,
+        TmAhead{}, stream);
 }

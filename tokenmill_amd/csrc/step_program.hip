@@ -14,6 +14,8 @@
 #include "api.h"
 #include "choose.h"
 #include "step_program.h"
+#include "ahead.h"
+#include "fused_common.h"
 
 #include <stdint.h>
 #include <string.h>
@@ -244,6 +246,7 @@ struct Run {
     int dtype;
     int from_norm_rows;                 // rows up to which q|k|v and gate|up start at the norm (tm_from_norm_rows)
     bool labels;
+    int first_op, last_op;              // the operations of this run
     // what crosses between operations
     float* resid;
     const void* delta;                  // product output still to be added to the residual stream
@@ -357,6 +360,61 @@ struct Run {
     // x = norm(resid + delta), resid updated
     int normed(const TmNorm& n) { return add_norm(n, nullptr, x, s->T); }
 
+    // Do q|k|v of attention operation `a` and gate|up of `f` run by the kernels that start at the norm, where their input is a whole residual stream?
+    bool starts_at_norm(const TmAttentionOp& a) const {
+        return dtype == TM_BF16 && a.qkv.dtype == TM_BF16 && a.D % 32 == 0 && a.norm.w && a.rot == a.D && a.cos_t && a.sin_t &&
+               fused_decode_ok(resid, a.qkv, s->T, from_norm_rows) && is_pow2(a.page) && (!a.qkv.bias || aligned(a.qkv.bias, 16));
+    }
+    bool starts_at_norm(const TmFfnOp& f) const {
+        return dtype == TM_BF16 && f.gate_up.dtype == TM_BF16 && !f.gate_up.bias && f.I % 4 == 0 && f.norm.w && f.gate_up.packed_parts == 2 &&
+               f.gate_up.packed_rows == 16 && fused_decode_ok(resid, f.gate_up, s->T, from_norm_rows);
+    }
+
+    // Which matrices a kernel of a layer brings ahead (ahead.h), in steps whose products start at the norm: q|k|v's the first strips of every block of
+    // gate|up, the attention's o and the rest of gate|up, gate|up's down and the next layer's q|k|v. So each has about 10 MB for the time
+    // its own blocks take, and all of a layer is in the second-level caches (32 MB) when it is used; a layer of more than that brings nothing.
+    // Steps of the 0.5B shape, us: one request of 300 keys 677 to 620, eight of 2,048 788 to 737, four of 1,000 753 to 683, four of up to 16,000 837
+    // to 821. Without the share of q|k|v's / without o / without the rest of gate|up / without the next q|k|v the first takes 641 / 628 / 642 / 633,
+    // with all of it by the attention 658. Blocks: about as many as the kernel leaves CUs for, half of that and up beside q|k|v's 72 (72 / 96 / 144
+    // of them 638 / 626 / 620), beside the attention 72 / 144 / 200 619 / 623 / 628 (eight requests 746 / 741 / 745 to 740), beside gate|up's
+    // 152 blocks 64 / 104 / 208 642 / 619 / 646.
+    enum { AHEAD_OF_QKV, AHEAD_OF_ATTENTION, AHEAD_OF_GATE_UP };
+    TmAhead ahead(int op, int host) const {
+        constexpr size_t MOST = 32u << 20;
+        TmAhead h;
+        const int at = host == AHEAD_OF_GATE_UP ? op - 1 : op;      // the layer's attention
+        if (!accumulate || at < first_op || at + 1 >= last_op || p->ops[at].kind != OP_ATTENTION || p->ops[at + 1].kind != OP_FEED_FORWARD) return h;
+        const TmAttentionOp& a = p->ops[at].att;
+        const TmFfnOp& f = p->ops[at + 1].ffn;
+        const TmAttentionOp* next = at + 2 < last_op && p->ops[at + 2].kind == OP_ATTENTION ? &p->ops[at + 2].att : nullptr;
+        auto strip = [](const TmLinear& L) { return (size_t)L.packed_rows * ((L.K + 31) / 32) * 64; };
+        auto few = [&](const TmLinear& L) { return L.dtype == TM_BF16 && L.packed && L.packed_parts == 1 && L.K % 8 == 0; };
+        if (!starts_at_norm(a) || !starts_at_norm(f) || !few(a.o) || !few(f.down)) return h;
+        if (next && !starts_at_norm(*next)) next = nullptr;
+        const int units = (f.I + 15) / 16, blocks = fused_gate_up_blocks(f.I), half = (units + blocks - 1) / blocks / 2;
+        auto strips = [](const TmLinear& L) { return (L.N + L.packed_rows - 1) / L.packed_rows; };
+        if (strip(f.gate_up) * 2 * units + strip(a.o) * strips(a.o) + strip(f.down) * strips(f.down) +
+                (next ? strip(next->qkv) * strips(next->qkv) : 0) > MOST)
+            return h;
+        if (host == AHEAD_OF_QKV) {
+            h.blocks = 120;
+            h.add(f.gate_up.packed, (int)strip(f.gate_up), units, true, blocks, 0, half > 0 ? half : 1);
+        } else if (host == AHEAD_OF_ATTENTION) {
+            h.blocks = 104;
+            h.add(a.o.packed, (int)strip(a.o), strips(a.o), false, strips(a.o));
+            h.add(f.gate_up.packed, (int)strip(f.gate_up), units, true, blocks, half > 0 ? half : 1);
+        } else {
+            h.blocks = 256 - blocks > 96 ? 96 : 256 - blocks;
+            if (h.blocks < 32) return h;
+            h.add(f.down.packed, (int)strip(f.down), strips(f.down), false, strips(f.down));
+            if (next) {
+                const int head_units = next->D / (2 * next->qkv.packed_rows), all = (next->H + 2 * next->KVH) * head_units;
+                h.add(next->qkv.packed, (int)strip(next->qkv), all, true, all, 0, 1, head_units, next->H + next->KVH);
+            }
+        }
+        return h;
+    }
+
     int embedding(int op, const TmEmbedOp& e) {
         Label l(this, op, TM_LABEL_EMBED);
         if (!resid) return TM_ERR_ARG;
@@ -383,6 +441,7 @@ struct Run {
         const void* q = nullptr;
         int q_stride = 0;
         int rc = TM_OK;
+        bool after_norm = false;            // q|k|v started at the norm, as gate|up will
         if (qkv_in) {                       // projected, encoded and stored by the caller
             q = qkv_in;
             q_stride = qkv_in_stride > 0 ? qkv_in_stride : QKV;
@@ -394,13 +453,13 @@ struct Run {
             Label l(this, op, TM_LABEL_QKV);
             const bool own_norm = x_in == nullptr;
             // 1. the kernel that starts at the norm (at most 16 tokens)
-            if (own_norm && dtype == TM_BF16 && a.qkv.dtype == TM_BF16 && a.D % 32 == 0 && delta == nullptr && !pending_sums && a.norm.w &&
-                tables_fusable && fused_decode_ok(resid, a.qkv, T, from_norm_rows) && is_pow2(a.page) && bias_ok) {
-                rc = tm_fused_norm_qkv_rope(resid, a.norm.w, a.norm.w_dtype, a.norm.eps, T, hidden, a.qkv.packed, a.qkv.bias,
-                                            a.qkv.bias_dtype, qkv, a.H, a.KVH, a.D, a.cos_t, a.sin_t, s->positions, slots, kp, vp,
-                                            a.page, stream);
+            if (own_norm && delta == nullptr && !pending_sums && starts_at_norm(a)) {
+                rc = fused_norm_qkv_rope_ahead(resid, a.norm.w, a.norm.w_dtype, a.norm.eps, T, hidden, a.qkv.packed, a.qkv.bias,
+                                               a.qkv.bias_dtype, qkv, a.H, a.KVH, a.D, a.cos_t, a.sin_t, s->positions, slots, kp, vp,
+                                               a.page, ahead(op, AHEAD_OF_QKV), stream);
                 q = qkv;
                 q_stride = HD;
+                after_norm = true;
                 ++p->taken[TM_QKV_FROM_NORM];
             } else {
                 const void* xn = x_in;
@@ -499,15 +558,16 @@ struct Run {
             char* out_dec = (char*)attn + (size_t)tp * HD * es;
             if (nd && dtype == TM_BF16 && head_mfma && page_ok && a.H / a.KVH <= 16 && q_ok) {
                 const bool split = decode_in_chunks(p, a, nd, s->max_decode_context);
+                const TmAhead matrices = after_norm ? ahead(op, AHEAD_OF_ATTENTION) : TmAhead{};
                 if (tm_decode_whole(nd, a.H, a.KVH, a.D, s->max_decode_context))
-                    rc = tm_attn_decode_whole(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
-                                              s->context_lens + (S - nd), tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page,
-                                              a.scale, a.window, a.keep, a.softcap, a.sink, cg_dec, cgate_ld, stream);
+                    rc = attn_decode_whole_ahead(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
+                                                 s->context_lens + (S - nd), tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page,
+                                                 a.scale, a.window, a.keep, a.softcap, a.sink, cg_dec, cgate_ld, matrices, stream);
                 else
-                    rc = tm_attn_decode_mfma_cap(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
-                                             s->context_lens + (S - nd), split ? part_o : nullptr, split ? part_ml : nullptr,
-                                             tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep,
-                                             a.softcap, a.sink, cg_dec, cgate_ld, stream);
+                    rc = attn_decode_ahead(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
+                                           s->context_lens + (S - nd), split ? part_o : nullptr, split ? part_ml : nullptr,
+                                           tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep,
+                                           a.softcap, a.sink, cg_dec, cgate_ld, matrices, stream);
                 done_decode = true;
             } else if (nd && dtype == TM_F32 && decode_in_chunks(p, a, nd, s->max_decode_context) &&
                        tm_attn_decode_f32_takes(q_dec, q_stride, a.k_pool, a.v_pool, a.H, a.KVH, a.D, a.page)) {
@@ -552,9 +612,9 @@ struct Run {
             const bool own_norm = x_in == nullptr;
             const bool plain = f.gate_up.dtype == dtype && f.gate_up.bias == nullptr;
             const bool two_parts = f.gate_up.packed_parts == 2 && f.gate_up.packed_rows == 16;
-            if (own_norm && dtype == TM_BF16 && plain && f.I % 4 == 0 && delta == nullptr && !pending_sums && f.norm.w && two_parts &&
-                fused_decode_ok(resid, f.gate_up, T, from_norm_rows)) {
-                rc = tm_fused_norm_gate_up_silu(resid, f.norm.w, f.norm.w_dtype, f.norm.eps, T, hidden, f.gate_up.packed, act, f.I, stream);
+            if (own_norm && delta == nullptr && !pending_sums && starts_at_norm(f)) {
+                rc = fused_norm_gate_up_silu_ahead(resid, f.norm.w, f.norm.w_dtype, f.norm.eps, T, hidden, f.gate_up.packed, act, f.I,
+                                                   ahead(op, AHEAD_OF_GATE_UP), stream);
                 ++p->taken[TM_GATE_UP_FROM_NORM];
             } else {
                 const void* xn = x_in;
@@ -780,6 +840,7 @@ int tm_program_run(const TmProgram* p, int first, int count, const TmStep* s, Tm
     r.products.skinny_rows = tm_skinny_rows(p->hidden);
     r.from_norm_rows = tm_from_norm_rows(p->hidden);
     r.labels = (flags & TM_RUN_LABELS) != 0;
+    r.first_op = first; r.last_op = first + count;
     r.resid = io->resid; r.delta = io->delta; r.x_in = io->x; r.qkv_in = io->qkv; r.accumulate = io->accumulate != 0;
     r.qkv_in_stride = io->qkv_stride; r.gate_in = io->qkv ? io->gate : nullptr; r.gate_ld = io->ldg;
     if (r.gate_in && r.gate_ld < p->ops[first].att.H) return TM_ERR_ARG;
@@ -849,6 +910,24 @@ int tm_rule(const char* name) {
     if (!strcmp(name, "decode_chunk")) return TM_DECODE_CHUNK;
     if (!strcmp(name, "decode_split_pairs")) return TM_DECODE_SPLIT_PAIRS;
     return -1;
+}
+
+int tm_ahead_runs(int strip_bytes, int units, int two, int blocks, int first_round, int last_round, int head_units, int rot_heads, int die,
+                  int* strips, int* runs, int room) {
+    if (strip_bytes <= 0 || units <= 0 || blocks <= 0 || die < 0 || die > 7) return -1;
+    TmAhead a;
+    a.add(nullptr, 64, 8, false, 8);                                // (another matrix in front)
+    const int before = a.total();
+    a.add(nullptr, strip_bytes, units, two != 0, blocks, first_round, last_round, head_units, rot_heads);
+    int n = 0;
+    for (int e = before; e < a.total(); ++e) {
+        int matrix, strip, run;
+        if (!ahead_run(a, die, e, matrix, strip, run)) continue;
+        if (matrix != 1 || n == room) return -1;
+        strips[n] = strip;
+        runs[n++] = run;
+    }
+    return n;
 }
 
 int tm_decode_takes_whole(int requests, int heads, int kv_heads, int head_size, int max_context) {
