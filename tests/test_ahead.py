@@ -6,20 +6,21 @@ import pytest
 import torch
 
 
-def _runs(strip_bytes, units, two, blocks, first, last, head_units, rot_heads, die):
+def _lines(name, *args):
     from tokenmill_amd.hip.abi import bound
-    room = 1 << 16
-    strips, runs = (ctypes.c_int * room)(), (ctypes.c_int * room)()
-    n = bound().tm_ahead_runs(*(ctypes.c_int(x) for x in (strip_bytes, units, two, blocks, first, last, head_units, rot_heads, die)), strips, runs, ctypes.c_int(room))
+    room = 1 << 20
+    at = (ctypes.c_longlong * room)()
+    n = getattr(bound(), name)(*(ctypes.c_int(x) for x in args), at, ctypes.c_int(room))
     assert n >= 0
-    return list(zip(strips[:n], runs[:n]))
+    return at[:n]
 
 
-# (bytes of a strip, units, two strips a unit, blocks of the product, units of a head, heads of q and k)
-@pytest.mark.parametrize("strip_bytes,units,two,blocks,head_units,rot_heads", [
-    (28672, 304, 1, 152, 0, 0), (7168, 224, 0, 224, 0, 0), (38912, 224, 0, 224, 0, 0), (14336, 72, 1, 72, 4, 16), (8192, 1, 0, 1, 0, 0), (64, 9, 0, 9, 0, 0),
-    (8256, 13, 1, 5, 0, 0), (16384, 257, 1, 129, 0, 0), (24576, 700, 1, 234, 0, 0), (1024, 30, 1, 30, 2, 11)])
-def test_every_line_is_brought_once_by_the_die_that_reads_it(strip_bytes, units, two, blocks, head_units, rot_heads):
+# (bytes of a strip, units, two strips a unit, blocks of the product, neighbours to a block, units of a head, heads of q and k)
+@pytest.mark.parametrize("strip_bytes,units,two,blocks,together,head_units,rot_heads", [
+    (28672, 304, 1, 152, 0, 0, 0), (28672, 304, 1, 152, 1, 0, 0), (7168, 224, 0, 224, 0, 0, 0), (38912, 224, 0, 224, 0, 0, 0), (14336, 72, 1, 72, 0, 4, 16),
+    (8192, 1, 0, 1, 0, 0, 0), (64, 9, 0, 9, 0, 0, 0), (8256, 13, 1, 5, 0, 0, 0), (8256, 13, 1, 5, 1, 0, 0), (16384, 257, 1, 129, 0, 0, 0),
+    (24576, 700, 1, 234, 0, 0, 0), (1024, 30, 1, 30, 0, 2, 11)])
+def test_every_line_of_a_packed_matrix_is_brought_once_by_the_die_that_reads_it(strip_bytes, units, two, blocks, together, head_units, rot_heads):
     rounds = -(-units // blocks)
     want = {}                                            # strip -> the die of the block that multiplies it
     for u in range(units):
@@ -29,21 +30,38 @@ def test_every_line_is_brought_once_by_the_die_that_reads_it(strip_bytes, units,
         else:
             pair = (u, units + u) if two else (u,)
         for strip in pair:
-            want[strip] = u % blocks % 8
-    seen = {}
+            want[strip] = (u // rounds if together else u % blocks) % 8
+    seen = set()
     for first, last in {(0, 1), (1, rounds)} if rounds > 1 else {(0, rounds)}:
         for die in range(8):
-            for strip, run in _runs(strip_bytes, units, two, blocks, first, last, head_units, rot_heads, die):
-                assert (strip, run) not in seen and want[strip] == die
-                seen[strip, run] = die
-    assert len(seen) == len(want) * -(-strip_bytes // 8192)
-    assert all(0 <= run and run * 8192 < strip_bytes for _, run in seen)
+            for at in _lines("tm_ahead_packed", strip_bytes, units, two, blocks, together, first, last, head_units, rot_heads, die):
+                strip, off = divmod(at, strip_bytes)
+                assert at not in seen and want[strip] == die and off % 128 == 0
+                seen.add(at)
+    assert len(seen) == len(want) * -(-strip_bytes // 128)
+
+
+# (rows of a half, K, rows of a column tile, parts of K, 64 k a part, halves)
+@pytest.mark.parametrize("row_end,K,rows,parts,lines,two", [(4864, 896, 32, 1, 14, 1), (896, 4864, 64, 4, 19, 0), (896, 4864, 64, 5, 16, 0), (896, 896, 64, 2, 7, 0),
+                                                            (1152, 896, 64, 1, 14, 0), (1400, 512, 32, 1, 8, 1), (100, 256, 128, 1, 4, 0), (72, 320, 64, 1, 5, 1)])
+def test_every_line_of_a_row_major_matrix_is_brought_once(row_end, K, rows, parts, lines, two):
+    seen, all_lines, tiles = set(), K // 64, -(-row_end // rows)
+    for die in range(8):
+        for at in _lines("tm_ahead_row_major", row_end, K, rows, parts, lines, two, die):
+            line, off = divmod(at, 128)
+            assert off == 0 and 0 <= line < (1 + two) * row_end * all_lines and at not in seen
+            row, k = divmod(line, all_lines)
+            column = k // lines * tiles + row % row_end // rows             # in the order of the product's tiles, of which a die has a run
+            assert die * tiles * parts // 8 <= column < (die + 1) * tiles * parts // 8
+            seen.add(at)
+    assert len(seen) == (1 + two) * row_end * all_lines
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("width,heads,kv_heads,inside,layers", [(896, 14, 2, 4864, 3), (512, 8, 2, 1400, 3), (256, 4, 4, 5000, 2), (1024, 8, 1, 4096, 2)])
-@pytest.mark.parametrize("contexts", [[1], [300, 17, 256], [40] * 8, [700, 5, 2100, 64, 513]])
-def test_a_step_has_the_bits_of_its_operations_one_by_one(width, heads, kv_heads, inside, layers, contexts):
+@pytest.mark.parametrize("contexts,portions", [([1], []), ([300, 17, 256], []), ([40] * 8, []), ([700, 5, 2100, 64, 513], []), ([90] * 12, []), ([300, 600] * 8, []),
+                                               ([50] * 33, []), ([], [30]), ([], [77]), ([], [150, 90]), ([], [600]), ([20, 700], [100]), ([300] * 10, [241, 241])])
+def test_a_step_has_the_bits_of_its_operations_one_by_one(width, heads, kv_heads, inside, layers, contexts, portions):
     """Operations run one by one know no operation behind them, so nothing is brought ahead."""
     from conftest import qwen2_config
     from tokenmill_amd import EngineConfig, LLMEngine
@@ -57,21 +75,20 @@ def test_a_step_has_the_bits_of_its_operations_one_by_one(width, heads, kv_heads
     g = torch.Generator(device="cuda").manual_seed(1)
     tensors = {name: (torch.randn(spec.drawn_shape(), generator=g, device="cuda") * 0.02).bfloat16() for name, spec in sorted(model.tensor_specs().items())}
     model.load(tensors, torch.bfloat16, torch.device("cuda:0"))
-    engine = LLMEngine(EngineConfig(dtype="bfloat16", block_size=16, num_blocks=sum(-(-c // 16) for c in contexts) + 4, watermark=0.0, max_model_len=2200,
-                                    max_num_seqs=16, max_num_batched_tokens=4096, hip_graphs=False), model=model)
-    caches = [engine.cache.allocate(f"r{i}", c) for i, c in enumerate(contexts)]
-    ids = [torch.randint(0, 512, (c,), generator=torch.Generator().manual_seed(c)).tolist() for c in contexts]
-    for cache, prompt in zip(caches, ids):
-        if len(prompt) > 1:
-            engine.runner.step([StepEntry(cache, 0, prompt[:-1], [len(prompt) - 2])])
-    step = engine.runner.prepare([StepEntry(cache, len(prompt) - 1, prompt[-1:], [0]) for cache, prompt in zip(caches, ids)])[0]
+    requests = [(0, n) for n in portions] + [(c - 1, 1) for c in contexts]            # (cached tokens, tokens of the step)
+    engine = LLMEngine(EngineConfig(dtype="bfloat16", block_size=16, num_blocks=sum(-(-(a + b) // 16) for a, b in requests) + 4, watermark=0.0,
+                                    max_model_len=2200, max_num_seqs=64, max_num_batched_tokens=4096, hip_graphs=False), model=model)
+    caches = [engine.cache.allocate(f"r{i}", a + b) for i, (a, b) in enumerate(requests)]
+    ids = [torch.randint(0, 512, (a + b,), generator=torch.Generator().manual_seed(a + b)).tolist() for a, b in requests]
+    for cache, prompt, (a, _) in zip(caches, ids, requests):
+        if a:
+            engine.runner.step([StepEntry(cache, 0, prompt[:a], [a - 1])])
+    step = engine.runner.prepare([StepEntry(cache, a, prompt[a:], [b - 1]) for cache, prompt, (a, b) in zip(caches, ids, requests)])[0]
     program = engine.runner.program
-    before = program.counters()
     want = program.run(step).clone()
-    assert program.counters()["gate_up_from_norm"] - before["gate_up_from_norm"] == layers
-    T = step.num_tokens
+    T, R = step.num_tokens, step.num_logit_rows
     flow = Flow(resid=torch.empty((T, width), dtype=torch.float32, device="cuda"), accumulate=True)
-    flow.logits = torch.empty((T, 512), dtype=torch.float32, device="cuda")
+    flow.logits = torch.empty((R, 512), dtype=torch.float32, device="cuda")
     (native,) = program.steps
     for op in range(native.first, native.first + native.count):
         program.run_ops(op, 1, step, flow)

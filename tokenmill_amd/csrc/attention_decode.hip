@@ -333,13 +333,13 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
     int max_chunks, int H, int KVH, int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep,
     const TmAhead ahead) {
     constexpr int NDT = D / 16;
+    __shared__ float s_m[4][16], s_l[4][16];
+    __shared__ float s_o[4][16][D + 1];
     if constexpr (AHEAD) {
         ahead_with(q, q_stride, k_pool, v_pool, block_tables, table_width, context_lens, part_o, part_ml, H, KVH, page_shift, scale_log2, cap_in, cap_out,
                    window, keep);
         if ((int)blockIdx.z >= max_chunks) return tm_bring_ahead(ahead, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), 4);
     }
-    __shared__ float s_m[4][16], s_l[4][16];
-    __shared__ float s_o[4][16][D + 1];
     const int s = blockIdx.x, kvh = blockIdx.y, chunk = blockIdx.z;
     const int G = H / KVH;
     const int wave = threadIdx.x / TM_WAVE, lane = threadIdx.x % TM_WAVE;
@@ -559,12 +559,12 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_whole_kernel(
     float cap_in, float cap_out, int window, int keep, const float* __restrict__ sink, const bf16_t* __restrict__ cgate, int ldcg,
     const TmAhead ahead) {
     constexpr int NDT = D / 16, ROW = D + 4;
+    extern __shared__ __align__(16) float s_whole[];
     if constexpr (AHEAD) {
         ahead_with(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, chunks, H, KVH, page_shift, scale_log2, cap_in,
                    cap_out, window, keep, sink, cgate, ldcg);
         if (blockIdx.z) return tm_bring_ahead(ahead, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), WAVES);
     }
-    extern __shared__ __align__(16) float s_whole[];
     const int s = blockIdx.x, kvh = blockIdx.y;
     const int G = H / KVH;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;

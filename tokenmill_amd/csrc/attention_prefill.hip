@@ -19,6 +19,7 @@
 #include "api.h"
 #include "attention_prefill_common.h"
 #include "choose.h"
+#include "ahead.h"
 
 template <int D>
 struct KVBlock {
@@ -196,18 +197,21 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, HeadState<D, HPW>&
 // With pair != 0 a block takes tile b and then tile n_tiles - 1 - b: in a table sorted by the
 // number of keys a tile sees, the longest goes with the shortest and every block has the same work
 // (the lower triangle of a prompt, folded).
-template <int D, int HPW, int KS, bool CAP>
+template <int D, int HPW, int KS, bool CAP, bool AHEAD>
 __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
     int table_width, const int* __restrict__ tiles, int n_tiles, int pair, int H, int KVH, int page_shift,
     float scale_log2, float cap_in, float cap_out, int window, int keep, const float* __restrict__ sink,
-    const bf16_t* __restrict__ cgate, int ldcg) {
+    const bf16_t* __restrict__ cgate, int ldcg, const TmAheadArg<AHEAD> ahead) {
     constexpr int NDC = D / 32, NDT = D / 16;
     // the wavefronts' partials of all heads: rows of d four floats apart from a multiple of 64, so that 16 lanes of a store or load
     // of 16 bytes meet no bank twice
     __shared__ float s_m[KS][HPW][16], s_l[KS][HPW][16];
     extern __shared__ __align__(16) float s_o[];                     // [KS][HPW][16][D + 4]
+    if constexpr (AHEAD) {
+        if (blockIdx.z) return tm_bring_ahead(ahead, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), KS);
+    }
     auto partial_at = [&](int w, int hh, int col, int d) { return s_o + (size_t)((w * HPW + hh) * 16 + col) * (D + 4) + d; };
     // the wavefront index in a scalar register: everything derived from it (its key blocks, their
     // pages, the branches on them) stays wave-uniform
@@ -361,32 +365,39 @@ template <int D, int HPW, bool CAP>
 static int launch_split_keys(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                               const int* block_tables, int table_width, const int* tiles, int n_tiles, int H, int KVH,
                               int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep, const float* sink,
-                              const bf16_t* cgate, int ldcg, hipStream_t stream) {
+                              const bf16_t* cgate, int ldcg, TmAhead& ahead, hipStream_t stream) {
     constexpr int KS = PrefillShape<D>::KS;
     const int splits = (H / KVH + HPW - 1) / HPW;
     // fold the table in two once the folded launch still gives every CU a block
     const int pair = (long long)(n_tiles / 2) * KVH * splits >= 256 ? 1 : 0;
     dim3 grid(pair ? (n_tiles + 1) / 2 : n_tiles, KVH * splits);
     constexpr int lds = KS * HPW * 16 * (D + 4) * (int)sizeof(float);          // at most 139,264 bytes
-    if (lds > 64 * 1024) {
-        static const hipError_t raised = hipFuncSetAttribute((const void*)attn_prefill_mfma_kernel<D, HPW, KS, CAP>,
-                                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (raised != hipSuccess) return TM_ERR_LAUNCH;
-    }
-    attn_prefill_mfma_kernel<D, HPW, KS, CAP><<<grid, 64 * KS, lds, stream>>>(
-        (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
-        table_width, tiles, n_tiles, pair, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
-    return TM_OK;
+    const bool far = (long long)grid.x * grid.y >= 256;              // (more blocks than CUs: none to spare)
+    if (far) ahead.n = 0;
+    grid.z = 1 + (far ? 0 : ahead_spare_layers(ahead, grid.x * grid.y, grid.x * grid.y));
+    auto go = [&](auto AHEAD) {
+        constexpr bool with = decltype(AHEAD)::value;
+        if (lds > 64 * 1024) {
+            static const hipError_t raised = hipFuncSetAttribute((const void*)attn_prefill_mfma_kernel<D, HPW, KS, CAP, with>,
+                                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            if (raised != hipSuccess) return TM_ERR_LAUNCH;
+        }
+        attn_prefill_mfma_kernel<D, HPW, KS, CAP, with><<<grid, 64 * KS, lds, stream>>>(
+            (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
+            table_width, tiles, n_tiles, pair, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg, ahead_arg<with>(ahead));
+        return TM_OK;
+    };
+    return ahead.n ? go(std::true_type{}) : go(std::false_type{});
 }
 
 // softcap > 0: a score s (scaled) becomes softcap * tanh(s / softcap) before the softmax; sink (float32 [H]) or null: one more term
 // exp(sink[h]) in the denominator of head h's softmax, with no key behind it; with a window, `keep`: the first keys of a request that
 // every query sees beside its window; cgate (rows of the flat batch, ldcg apart) or null: channel c of the result is multiplied by
 // sigmoid(cgate[c])
-extern "C" int tm_attn_prefill_mfma_cap(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
+int attn_prefill_ahead(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
                                         const void* v_pool, const int* block_tables, int table_width, const int* tiles,
                                         int n_tiles, int H, int KVH, int D, int page, float scale, int window, int keep, float softcap,
-                                        const float* sink, const void* cgate, int ldcg, hipStream_t stream) {
+                                        const float* sink, const void* cgate, int ldcg, TmAhead& ahead, hipStream_t stream) {
     if (n_tiles <= 0) return TM_OK;
     if (!(softcap >= 0.f) || keep < 0 || (cgate && (ldcg < H * D || ldcg % 2 || (uintptr_t)cgate % 4))) return TM_ERR_ARG;
     const float cap_in = softcap > 0.f ? scale / softcap : 0.f, cap_out = softcap > 0.f ? softcap / scale : 0.f;
@@ -401,7 +412,7 @@ extern "C" int tm_attn_prefill_mfma_cap(const void* q, int q_stride, void* out, 
     if ((long long)KVH * ((G + 1) / 2) > 65535) return TM_ERR_ARG;
     int rc = TM_OK;
 #define TM_SPLIT_ARGS q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, tiles, n_tiles, H, KVH, \
-                      page_shift, scale_log2, cap_in, cap_out, window, keep, sink, (const bf16_t*)cgate, ldcg, stream
+                      page_shift, scale_log2, cap_in, cap_out, window, keep, sink, (const bf16_t*)cgate, ldcg, ahead, stream
 #define TM_PREFILL_CASE(DD)                                                                                       \
     case DD: {                                                                                                    \
         constexpr int HPW = PrefillShape<DD>::HPW;                                                                \
@@ -426,6 +437,15 @@ extern "C" int tm_attn_prefill_mfma_cap(const void* q, int q_stride, void* out, 
     if (rc) return rc;
     TM_CHECK_LAUNCH();
     return TM_OK;
+}
+
+extern "C" int tm_attn_prefill_mfma_cap(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
+                                        const void* v_pool, const int* block_tables, int table_width, const int* tiles,
+                                        int n_tiles, int H, int KVH, int D, int page, float scale, int window, int keep, float softcap,
+                                        const float* sink, const void* cgate, int ldcg, hipStream_t stream) {
+    TmAhead none;
+    return attn_prefill_ahead(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, tiles, n_tiles, H, KVH, D, page, scale, window, keep,
+                              softcap, sink, cgate, ldcg, none, stream);
 }
 
 extern "C" int tm_attn_prefill_mfma(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,

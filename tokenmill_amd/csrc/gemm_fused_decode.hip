@@ -45,6 +45,7 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
                                                                                                        const int n_units, const int blocks,
                                                                                                        const TmAhead ahead) {
     constexpr int KCH = PIPE ? FD_KCH_PIPE : FD_KCH;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
     if constexpr (AHEAD) {
         ahead_with(a.resid, a.norm_w, a.norm_w_f32, a.eps, a.M, a.K, a.W, n_units);
         if constexpr (EPI == FD_EPI_QKV) ahead_with(a.bias, a.bias_f32, a.H, a.KVH, a.D, a.head_inverse, a.cos_t, a.sin_t, a.positions, a.slots);
@@ -52,7 +53,6 @@ __global__ __launch_bounds__(64 * WAVES * UNITS, WAVES * UNITS == 4 ? 2 : 1) voi
         if ((int)blockIdx.x >= blocks) return tm_bring_ahead(ahead, blockIdx.x, WAVES * UNITS);
     }
     constexpr int THREADS = 64 * WAVES * UNITS, RC = PLAIN ? fused_row_vectors(THREADS) : FD_RC;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
     bf16_t* xs = (bf16_t*)smem_raw;                                  // [4, 8 or 16 rows][fused_norm_stride]
     __shared__ f32x4_t red[UNITS][WAVES][2][64];
     const int K = a.K, M = a.M;

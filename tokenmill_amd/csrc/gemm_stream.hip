@@ -27,6 +27,7 @@
 #include "common.h"
 #include "api.h"
 #include "fused_common.h"
+#include "ahead.h"
 
 #define ST_EPI_QKV 0
 #define ST_EPI_SILU 1
@@ -425,6 +426,12 @@ static void stream_plain_shape(int N, int K, int* parts, int* ks, int* us) {
     while (p > 1 && ksteps / (p * 4) < 4) p /= 2;
     *parts = p;
     stream_config(n_units * p, ks, us);
+}
+
+int stream_gate_up_units(int I) {
+    int ks, us;
+    stream_config((I + 15) / 16, &ks, &us);
+    return us;
 }
 
 template <int EPI, int NT, int KS, int US>

@@ -20,6 +20,7 @@
 #include "common.h"
 #include "api.h"
 #include "fused_common.h"
+#include "ahead.h"
 
 #include <type_traits>
 
@@ -51,6 +52,7 @@ struct TileArgs {
     int src_div, tile_rows;
     const float* pair_weight;   // clamped gate: [pairs], multiplies the products of slot i by pair_weight[row_src[i]]; or null
     float limit, alpha;
+    int grid;                   // blocks that walk tiles
 };
 
 // Where a tile lies.
@@ -145,12 +147,12 @@ __device__ __forceinline__ bool gt_place(const TileArgs& a, int BM, int p, GtPla
     return true;
 }
 
-// ... or the next one behind it (the block's tiles are gridDim.x apart) that has a row
+// ... or the next one behind it (the block's tiles are `stride` apart) that has a row
 template <bool GROUPED>
-__device__ __forceinline__ bool gt_next(const TileArgs& a, int BM, int& p, GtPlace& at) {
+__device__ __forceinline__ bool gt_next(const TileArgs& a, int BM, int stride, int& p, GtPlace& at) {
     while (gt_place<GROUPED>(a, BM, p, at)) {
         if (!GROUPED || at.m0 < at.end) return true;
-        p += gridDim.x;
+        p += stride;
     }
     return false;
 }
@@ -175,9 +177,14 @@ __device__ __forceinline__ int gt_matrix_row(const TileArgs& a, int u, int q) {
 }
 
 // MT, NT: 16-row tiles of A and of the matrix a wavefront multiplies; WM x WN = 4 wavefronts; ST: buffers of the ring
-template <typename T, int EPI, int MT, int NT, int WM, int WN, int ST, int OCC>
-__global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
+template <typename T, int EPI, int MT, int NT, int WM, int WN, int ST, int OCC, bool BRINGS = false>
+__global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a, const TmAheadArg<BRINGS> ahead) {
     extern __shared__ __align__(16) unsigned char gt_smem[];
+    if constexpr (BRINGS) {
+        ahead_with(a.A, a.W, a.M, a.N, a.K, a.lda, a.tiles_m, a.tiles_n, a.splits, a.band, a.D, a.head_inverse, a.positions, a.slots, a.bias, a.bias_f32);
+        if ((int)blockIdx.x >= a.grid) return tm_bring_ahead(ahead, blockIdx.x, 4);
+    }
+    const int stride = BRINGS ? a.grid : gridDim.x;
     constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, ROWS = BM + BN;
     constexpr bool GROUPED = EPI >= GT_EXPERT_SILU, GATED = EPI == GT_SILU || EPI == GT_EXPERT_SILU || EPI == GT_EXPERT_CLAMPED;
     // Behind a block's last tile there is nothing to load. Tiles of a middle size load nothing then; the others load the same bytes
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     bool l_more = true;
     auto next_load_tile = [&]() {
         GtPlace at_;
-        if (!l_more || !gt_next<GROUPED>(a, BM, l_p, at_)) {             // no further tile: nothing, or the same bytes again, never multiplied
+        if (!l_more || !gt_next<GROUPED>(a, BM, stride, l_p, at_)) {             // no further tile: nothing, or the same bytes again, never multiplied
             l_more = false;
             if constexpr (!QUIET) {
                 lA = (const unsigned char*)a.A;
@@ -210,7 +217,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
             }
             return;
         }
-        l_p += gridDim.x;
+        l_p += stride;
         const int k0 = at_.sp * per;
         lA = (const unsigned char*)a.A + (size_t)k0 * 128;
         lW = (const unsigned char*)a.W + (size_t)k0 * 128 + (GROUPED ? (size_t)at_.group * a.N * a.K * ES : 0);
@@ -239,7 +246,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
     // --- the multiplying side ---
     GtPlace at_;
     int p = blockIdx.x;
-    if (!gt_next<GROUPED>(a, BM, p, at_)) return;
+    if (!gt_next<GROUPED>(a, BM, stride, p, at_)) return;
     next_load_tile();
 #pragma unroll
     for (int s = 0; s < ST; ++s) {                                  // (every part of K has at least ST steps)
@@ -544,8 +551,8 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a) {
                 }
             }
         }
-        p += gridDim.x;
-        if (!gt_next<GROUPED>(a, BM, p, at_)) break;
+        p += stride;
+        if (!gt_next<GROUPED>(a, BM, stride, p, at_)) break;
         clear();
     }
     gt_wait_loads<0>();                                             // nothing of the ring is in flight when the block ends
@@ -610,7 +617,7 @@ static int gt_choose(int M, int N, int K, int splits, double* cost = nullptr) {
 }
 
 template <typename T, int EPI, int MT, int NT, int WM, int WN, int ST, int OCC>
-static int gt_launch(TileArgs& a, hipStream_t stream) {
+static int gt_launch(TileArgs& a, hipStream_t stream, TmAhead* ahead = nullptr) {
     constexpr int BM = 16 * MT * WM, BN = 16 * NT * WN, LDS = (BM + BN) * 128 * ST;
     static_assert(LDS * OCC <= 160 * 1024, "");
     static const hipError_t allowed = hipFuncSetAttribute((const void*)gemm_tile_kernel<T, EPI, MT, NT, WM, WN, ST, OCC>,
@@ -626,15 +633,28 @@ static int gt_launch(TileArgs& a, hipStream_t stream) {
     a.band = GROUPED ? 2 : (a.tiles_m + bands - 1) / bands;
     const int chunk = (a.tiles_m * a.tiles_n * a.splits + 7) / 8;
     const int grid = 8 * chunk < GT_CUS * OCC ? 8 * chunk : GT_CUS * OCC;
-    gemm_tile_kernel<T, EPI, MT, NT, WM, WN, ST, OCC><<<grid, 256, LDS, stream>>>(a);
+    a.grid = grid;
+    // (only q|k|v's small tiles leave CUs idle)
+    if constexpr (EPI == GT_QKV && sizeof(T) == 2 && BM * BN <= 64 * 128) {
+        if (const int more = ahead ? ahead_spare_layers(*ahead, 8, grid) : 0) {
+            static const hipError_t raised = hipFuncSetAttribute((const void*)gemm_tile_kernel<T, EPI, MT, NT, WM, WN, ST, OCC, true>,
+                                                                 hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+            if (raised != hipSuccess) return TM_ERR_LAUNCH;
+            gemm_tile_kernel<T, EPI, MT, NT, WM, WN, ST, OCC, true><<<grid + 8 * more, 256, LDS, stream>>>(a, *ahead);
+            TM_CHECK_LAUNCH();
+            return TM_OK;
+        }
+    }
+    if (ahead) ahead->n = 0;
+    gemm_tile_kernel<T, EPI, MT, NT, WM, WN, ST, OCC><<<grid, 256, LDS, stream>>>(a, TmNoAhead{});
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
 
 template <int EPI>
-static int gt_go(TileArgs& a, int shape, hipStream_t stream) {
+static int gt_go(TileArgs& a, int shape, hipStream_t stream, TmAhead* ahead = nullptr) {
     switch (shape) {
-#define GT_CASE(id, MT, NT, WM, WN, ST, OCC, s1, e1, s2, e2) case id: return gt_launch<bf16_t, EPI, MT, NT, WM, WN, ST, OCC>(a, stream);
+#define GT_CASE(id, MT, NT, WM, WN, ST, OCC, s1, e1, s2, e2) case id: return gt_launch<bf16_t, EPI, MT, NT, WM, WN, ST, OCC>(a, stream, ahead);
         GT_SHAPES(GT_CASE)
     }
     return TM_ERR_ARG;
@@ -664,9 +684,9 @@ extern "C" int tm_tile_gate_up_silu(const void* A, int lda, int M, int K, const 
 
 // q (rotated, [M, H D]), and k and v to the cache, of q|k|v = A W^T + bias; head sizes of whole units (64), rotated over the
 // whole head; slots (null: nothing is stored) as in tm_rope_kv_write
-extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void* W, const void* bias, int bias_dtype, void* q, int H,
+int tile_qkv_rope_ahead(const void* A, int lda, int M, int K, const void* W, const void* bias, int bias_dtype, void* q, int H,
                                 int KVH, int D, const float* cos_t, const float* sin_t, const int* positions, const int* slots,
-                                void* k_pool, void* v_pool, int page, hipStream_t stream) {
+                                void* k_pool, void* v_pool, int page, TmAhead& ahead, hipStream_t stream) {
     const int N = (H + 2 * KVH) * D;
     if (H <= 0 || KVH <= 0 || D <= 0 || D % 64 || !gt_aligned(q) || !cos_t || !sin_t || !positions || page <= 0 || (page & (page - 1)) ||
         (bias && bias_dtype != TM_NONE && !gt_aligned(bias)) || !gt_aligned(cos_t) || !gt_aligned(sin_t) || (slots && (!gt_aligned(k_pool) || !v_pool)) || !tm_gemm_tile_takes(A, lda, W, M, N, K))
@@ -678,7 +698,14 @@ extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void
     a.H = H; a.KVH = KVH; a.D = D; a.head_inverse = unit_inverse(D / 64); a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots;
     a.k_pool = k_pool; a.v_pool = v_pool;
     while ((1 << a.page_shift) < page) ++a.page_shift;
-    return gt_go<GT_QKV>(a, gt_choose(M, N, K, 1), stream);
+    return gt_go<GT_QKV>(a, gt_choose(M, N, K, 1), stream, &ahead);
+}
+
+extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void* W, const void* bias, int bias_dtype, void* q, int H,
+                                int KVH, int D, const float* cos_t, const float* sin_t, const int* positions, const int* slots,
+                                void* k_pool, void* v_pool, int page, hipStream_t stream) {
+    TmAhead none;
+    return tile_qkv_rope_ahead(A, lda, M, K, W, bias, bias_dtype, q, H, KVH, D, cos_t, sin_t, positions, slots, k_pool, v_pool, page, none, stream);
 }
 
 // Parts that a plain product's K is split into, whose 32-bit sums the next norm adds; 0: the library's product is the better one.
@@ -729,6 +756,23 @@ extern "C" int tm_tile_linear_split(const void* A, int lda, int M, int K, const 
         return gt_few_wide(N, K) ? gt_launch<bf16_t, GT_PARTS, 2, 4, 2, 2, GT_FEW_WIDE_RING, 2>(a, stream)
                                  : gt_launch<bf16_t, GT_PARTS, 1, 4, 4, 1, GT_FEW_RING, 2>(a, stream);
     return gt_go<GT_PARTS>(a, gt_choose(M, N, K, splits), stream);
+}
+
+TmTilePieces tile_pieces_gate_up(int M, int I, int K) {
+    const int shape = gt_choose(M, 2 * I, K, 1);
+    return shape < 0 ? TmTilePieces{} : TmTilePieces{gt_shapes[shape].BN / 2, 1, K / 64};
+}
+TmTilePieces tile_pieces_qkv(int M, int N, int K) {
+    const int shape = gt_choose(M, N, K, 1);
+    return shape < 0 ? TmTilePieces{} : TmTilePieces{gt_shapes[shape].BN, 1, K / 64};
+}
+TmTilePieces tile_pieces_split(int M, int N, int K) {
+    const int parts = tm_tile_linear_parts(M, N, K);
+    if (parts < 1) return {};
+    const int shape = gt_few(M, K) ? 0 : gt_choose(M, N, K, parts);
+    if (shape < 0) return {};
+    const int columns = gt_few(M, K) ? (gt_few_wide(N, K) ? 128 : 64) : gt_shapes[shape].BN;
+    return {columns, parts, (K / 64 + parts - 1) / parts};
 }
 
 // C[m, n] = A W^T, rows ldc apart, in bfloat16 (out_dtype 1) or, with ldc = N, float32 (0)

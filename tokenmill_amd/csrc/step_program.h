@@ -169,10 +169,11 @@ int tm_linear_run(const TmLinear* L, int x_dtype, const void* x, int ldx, int M,
 int tm_rule(const char* name);
 // Chunks a decode step's contexts are split into, or 0 if this step does not split them.
 int tm_decode_split_chunks(int requests, int kv_heads, int max_context);
-// The runs of 64 lines of a packed matrix (ahead.h) that the blocks of a compute die bring ahead: their strips and places in it; how many, or -1
-// if `room` is too little (for tests, on the host).
-int tm_ahead_runs(int strip_bytes, int units, int two, int blocks, int first_round, int last_round, int head_units, int rot_heads, int die,
-                  int* strips, int* runs, int room);
+// The lines of a matrix that the blocks of a compute die bring ahead (ahead.h: TmAhead::packed and ::row_major), in bytes from its start; how many, or
+// -1 if `room` is too little (for tests, on the host).
+int tm_ahead_packed(int strip_bytes, int units, int two, int blocks, int together, int first_round, int last_round, int head_units, int rot_heads,
+                    int die, long long* at, int room);
+int tm_ahead_row_major(int row_end, int K, int rows, int parts, int lines, int two, int die, long long* at, int room);
 // 1 if one block a (request, kv head) takes all chunks of such a step (tm_attn_decode_whole; asked before the other)
 int tm_decode_takes_whole(int requests, int heads, int kv_heads, int head_size, int max_context);
 

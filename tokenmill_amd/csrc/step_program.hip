@@ -238,6 +238,19 @@ int program_chunks(const TmProgram* p, int num_decode, int context) {
     return 0;
 }
 
+// The lines that a die's blocks bring of the second of two matrices.
+int ahead_lines(const TmAhead& a, int die, long long* at, int room) {
+    int n = 0;
+    for (int e = a.m[0].end; e < a.total(); ++e)
+        for (int lane = 0; lane < TM_WAVE; ++lane) {
+            const int line = ahead_line<true>(a.m[1], die, e - a.m[0].end, lane);
+            if (line < 0) continue;
+            if (n == room) return -1;
+            at[n++] = line;
+        }
+    return n;
+}
+
 struct Run {
     const TmProgram* p;
     const TmStep* s;
@@ -247,6 +260,7 @@ struct Run {
     int from_norm_rows;                 // rows up to which q|k|v and gate|up start at the norm (tm_from_norm_rows)
     bool labels;
     int first_op, last_op;              // the operations of this run
+    bool brought = false;               // q|k|v of this layer had room for matrices that follow
     // what crosses between operations
     float* resid;
     const void* delta;                  // product output still to be added to the residual stream
@@ -398,20 +412,85 @@ struct Run {
             return h;
         if (host == AHEAD_OF_QKV) {
             h.blocks = 120;
-            h.add(f.gate_up.packed, (int)strip(f.gate_up), units, true, blocks, 0, half > 0 ? half : 1);
+            h.packed(f.gate_up.packed, (int)strip(f.gate_up), units, true, blocks, false, 0, half > 0 ? half : 1);
         } else if (host == AHEAD_OF_ATTENTION) {
             h.blocks = 104;
-            h.add(a.o.packed, (int)strip(a.o), strips(a.o), false, strips(a.o));
-            h.add(f.gate_up.packed, (int)strip(f.gate_up), units, true, blocks, half > 0 ? half : 1);
+            h.packed(a.o.packed, (int)strip(a.o), strips(a.o), false, strips(a.o));
+            h.packed(f.gate_up.packed, (int)strip(f.gate_up), units, true, blocks, false, half > 0 ? half : 1);
         } else {
             h.blocks = 256 - blocks > 96 ? 96 : 256 - blocks;
             if (h.blocks < 32) return h;
-            h.add(f.down.packed, (int)strip(f.down), strips(f.down), false, strips(f.down));
+            h.packed(f.down.packed, (int)strip(f.down), strips(f.down), false, strips(f.down));
             if (next) {
                 const int head_units = next->D / (2 * next->qkv.packed_rows), all = (next->H + 2 * next->KVH) * head_units;
-                h.add(next->qkv.packed, (int)strip(next->qkv), all, true, all, 0, 1, head_units, next->H + next->KVH);
+                h.packed(next->qkv.packed, (int)strip(next->qkv), all, true, all, false, 0, 1, head_units, next->H + next->KVH);
             }
         }
+        return h;
+    }
+
+    // The same in steps of more tokens, whose products run behind a norm of their own, each matrix as the kernel that will take it reads it. There is more
+    // to gain: 896 -> 2 x 4,864 at 64 / 77 / 512 rows takes 8.6 / 8.7 / 16.9 us from cold, 5.8 / 5.6 / 13.5 out of the caches, 4,864 -> 896 6.7 / 6.2 / 12.9 and
+    // 4.7 / 4.8 / 8.9. Beyond 64 tokens q|k|v's tiles leave CUs idle and bring o and gate|up, the attention down and the next q|k|v, or all of it
+    // where q|k|v has no room; beside decoding requests q|k|v brings only in steps of up to 320 tokens, since their attention would put out
+    // more than it is late (130 / 304 / 490 / 512 tokens 1,341 / 1,450 / 1,822 / 1,778 us to 1,264 / 1,416 / 1,859 / 1,813). Up to 64 tokens everything in front of the
+    // products is short: o and down beside the attention, with the one-launch decode attention gate|up too (32 requests of 1,000 keys, split, 1,012
+    // without, 1,000 so, 1,031 with gate|up; 64 and 40 requests, whole, 1,272 and 995, 1,261 and 979, 1,243 and 960); q|k|v's panel and the norms,
+    // 3 to 5 us long, were slower by what they brought. Steps of the 0.5B shape, us, without to so: prompts of 30 / 77 / 150 / 300 / 600 tokens 896 / 1,054 /
+    // 1,155 / 1,352 / 1,812 to 886 / 962 / 1,071 / 1,230 / 1,733, 30 requests beside two portions of 241 1,906 to 1,751, 12 / 16 / 40 / 64 requests 945 / 993 /
+    // 995 / 1,272 to 910 / 970 / 958 / 1,242.
+    void bring_gate_up(TmAhead& h, const TmFfnOp& f) const {
+        const TmLinear& L = f.gate_up;
+        if (L.dtype != TM_BF16 || L.bias || s->T <= from_norm_rows) return;
+        if (f.I % 8 == 0 && tile_ok(L, x, p->hidden, s->T, dtype) && (s->T > TM_STREAM_ROWS || 2 * f.I <= TM_TILE_FEW_COLUMNS)) {
+            if (const TmTilePieces t = tile_pieces_gate_up(s->T, f.I, L.K); t.parts) h.row_major(L.w, f.I, L.K, t.rows, 1, t.steps, true);
+        } else if (L.packed_parts == 2 && L.packed_rows == 16 && stream_ok(L, x, p->hidden, s->T, dtype, from_norm_rows)) {
+            const int units = (f.I + 15) / 16, each = stream_gate_up_units(f.I);
+            h.packed(L.packed, 16 * ((L.K + 31) / 32) * 64, units, true, (units + each - 1) / each, true);
+        }
+    }
+    void bring_projection(TmAhead& h, const TmLinear& L) const {
+        if (L.dtype != TM_BF16 || L.bias || L.N != p->hidden || !sums) return;
+        if (tile_ok(L, x, L.K, s->T, dtype, tm_split_rows(p->hidden)) && tile_parts(L, s->T)) {
+            if (const TmTilePieces t = tile_pieces_split(s->T, L.N, L.K); t.parts) h.row_major(L.w, L.N, L.K, t.rows, t.parts, t.steps, false);
+        } else if (L.packed_parts == 1 && packed_ok(L, x, L.K, s->T, dtype, products.skinny_rows)) {
+            const int strips = (L.N + L.packed_rows - 1) / L.packed_rows;
+            h.packed(L.packed, L.packed_rows * ((L.K + 31) / 32) * 64, strips, false, strips);
+        }
+    }
+    void bring_qkv(TmAhead& h, const TmAttentionOp& a) const {
+        const TmLinear& L = a.qkv;
+        if (L.dtype != TM_BF16 || a.rot != a.D || a.D % 32 || !is_pow2(a.page)) return;
+        if (panel_ok(L, x, p->hidden, s->T, dtype, from_norm_rows, TM_PANEL_QKV_ROWS)) {
+            const int head_units = a.D / (2 * L.packed_rows), units = (a.H + 2 * a.KVH) * head_units;
+            h.packed(L.packed, L.packed_rows * ((L.K + 31) / 32) * 64, units, true, units, false, 0, 1, head_units, a.H + a.KVH);
+        } else if (a.D % 64 == 0 && tile_ok(L, x, p->hidden, s->T, dtype)) {
+            if (const TmTilePieces t = tile_pieces_qkv(s->T, L.N, L.K); t.parts) h.row_major(L.w, L.N, L.K, t.rows, 1, t.steps, false);
+        }
+    }
+    TmAhead ahead_behind_norm(int op, int host) const {
+        constexpr size_t MOST = 32u << 20;
+        constexpr int MIXED_ROWS = 320;
+        TmAhead h;
+        if (dtype != TM_BF16 || !accumulate || !resid || s->T <= from_norm_rows || op + 1 >= last_op || p->ops[op].kind != OP_ATTENTION || p->ops[op + 1].kind != OP_FEED_FORWARD) return h;
+        const TmAttentionOp& a = p->ops[op].att;
+        const TmFfnOp& f = p->ops[op + 1].ffn;
+        const TmAttentionOp* next = op + 2 < last_op && p->ops[op + 2].kind == OP_ATTENTION ? &p->ops[op + 2].att : nullptr;
+        auto bytes = [](const TmLinear& L) { return (size_t)L.N * L.K * 2; };
+        if (bytes(a.o) + bytes(f.gate_up) + bytes(f.down) + (next ? bytes(next->qkv) : 0) > MOST) return h;
+        const bool few = s->T <= TM_STREAM_ROWS;
+        if (host == AHEAD_OF_QKV) {
+            if (s->num_decode > 0 && s->T > MIXED_ROWS) return h;
+            h.blocks = 120;
+            bring_projection(h, a.o);
+            bring_gate_up(h, f);
+            return h;
+        }
+        h.blocks = 104;
+        if (!brought) bring_projection(h, a.o);
+        if (!brought && (!few || (s->num_decode == s->T && tm_decode_whole(s->T, a.H, a.KVH, a.D, s->max_decode_context)))) bring_gate_up(h, f);
+        bring_projection(h, f.down);
+        if (next && !few) bring_qkv(h, *next);
         return h;
     }
 
@@ -442,6 +521,8 @@ struct Run {
         int q_stride = 0;
         int rc = TM_OK;
         bool after_norm = false;            // q|k|v started at the norm, as gate|up will
+        TmAhead matrices;
+        brought = false;
         if (qkv_in) {                       // projected, encoded and stored by the caller
             q = qkv_in;
             q_stride = qkv_in_stride > 0 ? qkv_in_stride : QKV;
@@ -487,8 +568,10 @@ struct Run {
                 } else if (tables_fusable && a.D % 64 == 0 && tile_ok(a.qkv, xn, hidden, T, dtype) && is_pow2(a.page) && bias_ok &&
                            aligned(a.cos_t, 16) && aligned(a.sin_t, 16) && (!a.write || aligned(a.k_pool, 16))) {
                     // 4. more tokens: rotation and cache write in the epilogue of a product over the row-major matrix
-                    rc = tm_tile_qkv_rope(xn, hidden, T, hidden, a.qkv.w, a.qkv.bias, a.qkv.bias_dtype, qkv, a.H, a.KVH, a.D, a.cos_t,
-                                          a.sin_t, s->positions, slots, kp, vp, a.page, stream);
+                    matrices = ahead_behind_norm(op, AHEAD_OF_QKV);
+                    rc = tile_qkv_rope_ahead(xn, hidden, T, hidden, a.qkv.w, a.qkv.bias, a.qkv.bias_dtype, qkv, a.H, a.KVH, a.D, a.cos_t,
+                                             a.sin_t, s->positions, slots, kp, vp, a.page, matrices, stream);
+                    brought = matrices.n > 0;
                     q = qkv;
                     q_stride = HD;
                     ++p->taken[TM_QKV_PLAIN];
@@ -531,10 +614,11 @@ struct Run {
             const bool page_ok = a.page >= 16 && is_pow2(a.page);
             const bool head_mfma = a.D == 32 || a.D == 64 || a.D == 96 || a.D == 128;
             const bool q_ok = aligned(q, 16) && q_stride % 8 == 0;
-            bool done_prefill = false, done_decode = false;
+            bool done_prefill = false, done_decode = false, gone = false;
             const void* cg = cgate_in;      // a gate per channel, applied where a kernel stores its result
             const void* cg_dec = cg ? (const char*)cg + (size_t)tp * cgate_ld * es : nullptr;
             cgate_in = nullptr;
+            matrices = after_norm ? ahead(op, AHEAD_OF_ATTENTION) : ahead_behind_norm(op, AHEAD_OF_ATTENTION);
             if (tp && s->n_tiles > 0 && s->prefill_tiles && dtype == TM_BF16 && head_mfma && page_ok && q_ok) {
                 if (tm_prefill_shares_keys(a.D, a.H, a.KVH, s->n_tiles) && tm_attn_prefill_shared_takes(a.H, a.KVH, a.D) &&
                     HD % 4 == 0 && aligned(attn, 8)) {
@@ -543,8 +627,9 @@ struct Run {
                                                     s->n_tiles, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep, a.softcap, a.sink, cg, cgate_ld, stream);
                 } else {
                     ++p->taken[TM_PREFILL_SPLIT_KEYS];
-                    rc = tm_attn_prefill_mfma_cap(q, q_stride, attn, HD, a.k_pool, a.v_pool, tables, W, s->prefill_tiles,
-                                                  s->n_tiles, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep, a.softcap, a.sink, cg, cgate_ld, stream);
+                    rc = attn_prefill_ahead(q, q_stride, attn, HD, a.k_pool, a.v_pool, tables, W, s->prefill_tiles, s->n_tiles, a.H, a.KVH, a.D, a.page,
+                                            a.scale, a.window, a.keep, a.softcap, a.sink, cg, cgate_ld, matrices, stream);
+                    if (matrices.n) gone = true;
                 }
                 done_prefill = true;
             } else if (tp && s->n_tiles > 0 && s->prefill_tiles && dtype == TM_F32 && a.D % 16 == 0 && a.D >= 16 &&
@@ -558,7 +643,8 @@ struct Run {
             char* out_dec = (char*)attn + (size_t)tp * HD * es;
             if (nd && dtype == TM_BF16 && head_mfma && page_ok && a.H / a.KVH <= 16 && q_ok) {
                 const bool split = decode_in_chunks(p, a, nd, s->max_decode_context);
-                const TmAhead matrices = after_norm ? ahead(op, AHEAD_OF_ATTENTION) : TmAhead{};
+                if (gone) matrices.n = 0;       // (the prompt portions' attention had room for them)
+                else if (tp) matrices = after_norm ? ahead(op, AHEAD_OF_ATTENTION) : ahead_behind_norm(op, AHEAD_OF_ATTENTION);
                 if (tm_decode_whole(nd, a.H, a.KVH, a.D, s->max_decode_context))
                     rc = attn_decode_whole_ahead(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
                                                  s->context_lens + (S - nd), tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page,
@@ -912,22 +998,21 @@ int tm_rule(const char* name) {
     return -1;
 }
 
-int tm_ahead_runs(int strip_bytes, int units, int two, int blocks, int first_round, int last_round, int head_units, int rot_heads, int die,
-                  int* strips, int* runs, int room) {
+int tm_ahead_packed(int strip_bytes, int units, int two, int blocks, int together, int first_round, int last_round, int head_units, int rot_heads,
+                    int die, long long* at, int room) {
     if (strip_bytes <= 0 || units <= 0 || blocks <= 0 || die < 0 || die > 7) return -1;
     TmAhead a;
-    a.add(nullptr, 64, 8, false, 8);                                // (another matrix in front)
-    const int before = a.total();
-    a.add(nullptr, strip_bytes, units, two != 0, blocks, first_round, last_round, head_units, rot_heads);
-    int n = 0;
-    for (int e = before; e < a.total(); ++e) {
-        int matrix, strip, run;
-        if (!ahead_run(a, die, e, matrix, strip, run)) continue;
-        if (matrix != 1 || n == room) return -1;
-        strips[n] = strip;
-        runs[n++] = run;
-    }
-    return n;
+    a.packed(nullptr, 64, 8, false, 8);                             // (another matrix in front)
+    a.packed(nullptr, strip_bytes, units, two != 0, blocks, together != 0, first_round, last_round, head_units, rot_heads);
+    return ahead_lines(a, die, at, room);
+}
+
+int tm_ahead_row_major(int row_end, int K, int rows, int parts, int lines, int two, int die, long long* at, int room) {
+    if (row_end <= 0 || K < 64 || rows <= 0 || parts <= 0 || lines <= 0 || die < 0 || die > 7) return -1;
+    TmAhead a;
+    a.packed(nullptr, 64, 8, false, 8);
+    a.row_major(nullptr, row_end, K, rows, parts, lines, two != 0);
+    return ahead_lines(a, die, at, room);
 }
 
 int tm_decode_takes_whole(int requests, int heads, int kv_heads, int head_size, int max_context) {
