@@ -260,6 +260,12 @@ struct Run {
     int from_norm_rows;                 // rows up to which q|k|v and gate|up start at the norm (tm_from_norm_rows)
     bool labels;
     int first_op, last_op;              // the operations of this run
+    struct Known {
+        int what, N, K;
+        TmTilePieces pieces;
+    };
+    mutable Known known[8];             // (see pieces)
+    mutable int n_known = 0;
     bool brought = false;               // q|k|v of this layer had room for matrices that follow
     // what crosses between operations
     float* resid;
@@ -439,11 +445,20 @@ struct Run {
     // 3 to 5 us long, were slower by what they brought. Steps of the 0.5B shape, us, without to so: prompts of 30 / 77 / 150 / 300 / 600 tokens 896 / 1,054 /
     // 1,155 / 1,352 / 1,812 to 886 / 962 / 1,071 / 1,230 / 1,733, 30 requests beside two portions of 241 1,906 to 1,751, 12 / 16 / 40 / 64 requests 945 / 993 /
     // 995 / 1,272 to 910 / 970 / 958 / 1,242.
+    // How the tiled product takes a matrix in this step (0: gate|up, 1: q|k|v, 2: K in parts), asked once for all layers of a size: the rule weighs up to 88
+    // ways to cut it.
+    TmTilePieces pieces(int what, int N, int K) const {
+        for (int i = 0; i < n_known; ++i)
+            if (known[i].what == what && known[i].N == N && known[i].K == K) return known[i].pieces;
+        const TmTilePieces t = what == 0 ? tile_pieces_gate_up(s->T, N, K) : what == 1 ? tile_pieces_qkv(s->T, N, K) : tile_pieces_split(s->T, N, K);
+        known[n_known < 8 ? n_known++ : 7] = {what, N, K, t};
+        return t;
+    }
     void bring_gate_up(TmAhead& h, const TmFfnOp& f) const {
         const TmLinear& L = f.gate_up;
         if (L.dtype != TM_BF16 || L.bias || s->T <= from_norm_rows) return;
         if (f.I % 8 == 0 && tile_ok(L, x, p->hidden, s->T, dtype) && (s->T > TM_STREAM_ROWS || 2 * f.I <= TM_TILE_FEW_COLUMNS)) {
-            if (const TmTilePieces t = tile_pieces_gate_up(s->T, f.I, L.K); t.parts) h.row_major(L.w, f.I, L.K, t.rows, 1, t.steps, true);
+            if (const TmTilePieces t = pieces(0, f.I, L.K); t.parts) h.row_major(L.w, f.I, L.K, t.rows, 1, t.steps, true);
         } else if (L.packed_parts == 2 && L.packed_rows == 16 && stream_ok(L, x, p->hidden, s->T, dtype, from_norm_rows)) {
             const int units = (f.I + 15) / 16, each = stream_gate_up_units(f.I);
             h.packed(L.packed, 16 * ((L.K + 31) / 32) * 64, units, true, (units + each - 1) / each, true);
@@ -451,8 +466,8 @@ struct Run {
     }
     void bring_projection(TmAhead& h, const TmLinear& L) const {
         if (L.dtype != TM_BF16 || L.bias || L.N != p->hidden || !sums) return;
-        if (tile_ok(L, x, L.K, s->T, dtype, tm_split_rows(p->hidden)) && tile_parts(L, s->T)) {
-            if (const TmTilePieces t = tile_pieces_split(s->T, L.N, L.K); t.parts) h.row_major(L.w, L.N, L.K, t.rows, t.parts, t.steps, false);
+        if (tile_ok(L, x, L.K, s->T, dtype, tm_split_rows(p->hidden)) && !L.act && pieces(2, L.N, L.K).parts) {
+            if (const TmTilePieces t = pieces(2, L.N, L.K); t.parts <= TM_MAX_SUMS) h.row_major(L.w, L.N, L.K, t.rows, t.parts, t.steps, false);
         } else if (L.packed_parts == 1 && packed_ok(L, x, L.K, s->T, dtype, products.skinny_rows)) {
             const int strips = (L.N + L.packed_rows - 1) / L.packed_rows;
             h.packed(L.packed, L.packed_rows * ((L.K + 31) / 32) * 64, strips, false, strips);
@@ -465,7 +480,7 @@ struct Run {
             const int head_units = a.D / (2 * L.packed_rows), units = (a.H + 2 * a.KVH) * head_units;
             h.packed(L.packed, L.packed_rows * ((L.K + 31) / 32) * 64, units, true, units, false, 0, 1, head_units, a.H + a.KVH);
         } else if (a.D % 64 == 0 && tile_ok(L, x, p->hidden, s->T, dtype)) {
-            if (const TmTilePieces t = tile_pieces_qkv(s->T, L.N, L.K); t.parts) h.row_major(L.w, L.N, L.K, t.rows, 1, t.steps, false);
+            if (const TmTilePieces t = pieces(1, L.N, L.K); t.parts) h.row_major(L.w, L.N, L.K, t.rows, 1, t.steps, false);
         }
     }
     TmAhead ahead_behind_norm(int op, int host) const {
