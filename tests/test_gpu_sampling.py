@@ -62,3 +62,35 @@ def test_top_k_at_the_bound_of_the_widest_rows(k):
         z = torch.where(kept, logits.double() / 0.9, torch.tensor(float("-inf"), dtype=torch.float64)).softmax(1).cumsum(1)
         for r, t in enumerate(got):                             # the token in whose share of the mass u lies, to 32-bit sums of k weights
             assert (z[r, t - 1] if t else 0.0) - 1e-5 <= u[r] <= z[r, t] + 1e-5
+
+
+@pytest.mark.parametrize("vocab", [V, 151936, 4097, 1 << 20])
+@pytest.mark.parametrize("where", ["spread", "one share", "steps", "level", "not numbers", "small"])
+def test_lists_give_the_tokens_of_the_launches_over_all_chunks(where, vocab):
+    """Rows with k from 1 to beyond what the bound covers, with and without top-p, greedy ones and ones without top-k among them: through lists,
+    where thousands of equal entries do not fit one and unbounded rows have none, and without."""
+    from tokenmill_amd.hip import ops
+    most = ops.sample_list_k(vocab)
+    ks = [2, 7, 20, 50, most // 2, most, 1, 0, most + 1, 4 * most + 9]
+    R = 3 * len(ks)
+    g = torch.Generator().manual_seed(vocab)
+    logits = torch.randn(R, vocab, generator=g) * (0.01 if where == "small" else 2)
+    if where == "one share":
+        chunk = -(-vocab // (-(-vocab // 4096) if vocab <= 256 * 4096 else 256))
+        logits[:, torch.cat([torch.arange(chunk + 256 * j, min(vocab, chunk + 256 * j + 64)) for j in range(8) if chunk + 256 * j < vocab])] += 12
+    elif where == "steps":
+        logits = (logits * 2).round() / 2
+    elif where == "level":
+        logits = torch.where(torch.rand(R, vocab, generator=g) < 0.3, 1.5, 0.25)
+    elif where == "not numbers":
+        logits = logits.masked_fill(torch.rand(R, vocab, generator=g) < 0.6, float("nan"))
+    logits = logits.cuda()
+    f = lambda x: torch.tensor(x, dtype=torch.float32, device="cuda")       # noqa: E731
+    rows = [(ks[r % len(ks)], (1.0, 0.9, 0.5)[r // len(ks)]) for r in range(R)]
+    args = (f([0.0 if r == 4 else 0.8 for r in range(R)]), torch.tensor([k for k, _ in rows], dtype=torch.int32, device="cuda"), f([p for _, p in rows]),
+            f([(r * 0.137) % 1 for r in range(R)]))
+    want, got = (torch.full((R,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    ops.sample_rows(logits, *args, want)
+    for _ in range(2):                                                       # (the second call finds what the first left in the scratch memory)
+        ops.sample_rows(logits, *args, got, small_top_k=True)
+        assert got.tolist() == want.tolist()

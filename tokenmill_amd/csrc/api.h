@@ -419,6 +419,7 @@ int tm_argmax_rows(const float* logits, int R, int V, int* out, float* work_v, i
 int tm_argmax_rows_static_max_pairs(void);
 int tm_argmax_rows_static(const float* logits, int R, int V, int* out, hipStream_t stream);
 
+int tm_sample_list_k(int V);
 size_t tm_sample_work_bytes(int R, int V);
 int tm_sample_rows(const float* logits, int R, int V, const float* temperature, const int* top_k,
                    const float* top_p, const float* u, int* out, void* work, size_t work_bytes, int stages,

@@ -10,6 +10,7 @@
 #include "api.h"
 
 #include <mutex>
+#include <type_traits>
 
 #define SM_NT 1024
 
@@ -216,6 +217,7 @@ extern "C" int tm_argmax_rows_static(const float* logits, int R, int V, int* out
 //   3. top-p over what top-k kept, if some row asks for it: the same descent with fixed-point
 //      weights exp(z - zmax) * 2^32 instead of counts (the first level's histogram sums to the
 //      kept mass Z, so the limit p * Z needs no pass of its own);
+//   (2 to 4 where every row's k is small: one launch that gathers what may count into a list a row, and a block a row on it)
 //   4. the kept mass of every chunk (sample_chunk_mass_kernel), then one block per row that walks
 //      the chunks in vocabulary order to the one holding u * total and finds the token in it
 //      (sample_pick_kernel).
@@ -405,7 +407,7 @@ __global__ __launch_bounds__(SR_NT) void sample_bound_kernel(const float* __rest
                                                              const float* __restrict__ wave_v, int NB, int V,
                                                              const float* __restrict__ temperature, const int* __restrict__ top_k,
                                                              const float* __restrict__ top_p, float* __restrict__ rowmax,
-                                                             int* __restrict__ rowarg, RowState* __restrict__ state) {
+                                                             int* __restrict__ rowarg, RowState* __restrict__ state, int* __restrict__ counts) {
     __shared__ uint32_t s_key[SR_NT];
     __shared__ ArgMax s_best[SR_NT / TM_WAVE];
     __shared__ uint32_t s_bound;
@@ -444,7 +446,32 @@ __global__ __launch_bounds__(SR_NT) void sample_bound_kernel(const float* __rest
         if (larger < rp.k && larger + level >= rp.k) s_bound = key;        // (threads that write it write one value)
     }
     __syncthreads();
-    if (t == 0) state[row].bound = s_bound;
+    if (t == 0) {
+        state[row].bound = s_bound;
+        counts[row] = 0;
+    }
+}
+
+// The entries of a chunk that match the buckets picked so far, in a thread's share of it, into a histogram in LDS.
+template <bool BY_MASS>
+__device__ __forceinline__ void add_chunk(const float* __restrict__ row, int V, int chunk, int c, const RowParams& rp, int level, uint32_t floor_key,
+                                          uint32_t prefix, uint32_t mask, unsigned long long* s_hist) {
+    const int lo = c * chunk, hi = lo + chunk < V ? lo + chunk : V;
+    const int shift = level_shift(level);
+    const uint32_t digit_mask = (uint32_t)(level_bins(level) - 1);
+    for (int i = lo + threadIdx.x; i < hi; i += 8 * SR_NT) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = row[i + j * SR_NT < hi ? i + j * SR_NT : i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float z = v[j] * rp.inv_t;
+            if (i + j * SR_NT >= hi || !(z == z)) continue;
+            const uint32_t key = order_key(z);
+            if (key < floor_key || (key & mask) != prefix) continue;
+            atomicAdd(&s_hist[(key >> shift) & digit_mask], BY_MASS ? fix_weight(expf(z - rp.zmax)) : 1ull);
+        }
+    }
 }
 
 // One level of a descent: the chunk's entries that match the buckets picked so far, into the row's
@@ -489,23 +516,7 @@ __global__ __launch_bounds__(SR_NT) void sample_hist_kernel(const float* __restr
     if (__syncthreads_and(skip)) return;                 // nothing of this chunk counts
     for (int b = threadIdx.x; b < SR_BINS; b += SR_NT) s_hist[b] = 0ull;
     __syncthreads();
-    const float* row = logits + (size_t)r * V;
-    const int lo = c * chunk, hi = lo + chunk < V ? lo + chunk : V;
-    const int shift = level_shift(level);
-    const uint32_t digit_mask = (uint32_t)(level_bins(level) - 1);
-    for (int i = lo + threadIdx.x; i < hi && !skip; i += 8 * SR_NT) {
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = row[i + j * SR_NT < hi ? i + j * SR_NT : i];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float z = v[j] * rp.inv_t;
-            if (i + j * SR_NT >= hi || !(z == z)) continue;
-            const uint32_t key = order_key(z);
-            if (key < floor_key || (key & mask) != prefix) continue;
-            atomicAdd(&s_hist[(key >> shift) & digit_mask], BY_MASS ? fix_weight(expf(z - rp.zmax)) : 1ull);
-        }
-    }
+    if (!skip) add_chunk<BY_MASS>(logits + (size_t)r * V, V, chunk, c, rp, level, floor_key, prefix, mask, s_hist);
     __syncthreads();
     unsigned long long* dst = (BY_MASS ? hist_p : hist_k) + (size_t)level * SR_BINS;
     for (int b = threadIdx.x; b < SR_BINS; b += SR_NT)
@@ -556,6 +567,38 @@ __device__ __forceinline__ void block_sums(float& w, int& n, float* s_w /* SR_NT
     }
 }
 
+// What top-p leaves of what top-k kept: pk is the smallest key the nucleus reaches, limit = p * mass, above = mass of larger keys; the entries with that key
+// stay while the mass before them is at most p of the kept mass (reference src/infer/sampling.py:20-23: ties in sorted order, which here is
+// vocabulary order; the first always stays).
+__device__ __forceinline__ void cut_nucleus(RowKeep& keep, const RowParams& rp, uint32_t pk, unsigned long long limit, unsigned long long above) {
+    if (rp.need_k && pk < keep.p_key) return;
+    const unsigned long long w = fix_weight(expf(key_value(pk) - rp.zmax));
+    const unsigned long long room = limit > above ? limit - above : 0ull;
+    const unsigned long long fit = w ? room / w + 1ull : 0x7fffffffull;
+    const int by_mass = fit > 0x7fffffffull ? 0x7fffffff : (int)fit;
+    const bool same = rp.need_k && pk == keep.p_key;
+    keep.tie_budget = same && keep.tie_budget < by_mass ? keep.tie_budget : by_mass;
+    keep.p_key = pk;
+    keep.ties_matter = 1;
+}
+
+// The kept weight and the ties of a thread's share of a chunk.
+__device__ __forceinline__ void chunk_share(const float* __restrict__ row, int V, int chunk, int c, const RowParams& rp, const RowKeep& keep, float& w,
+                                            int& ties) {
+    const int lo = c * chunk, hi = lo + chunk < V ? lo + chunk : V;
+    for (int i = lo + threadIdx.x; i < hi; i += 8 * SR_NT) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = row[i + j * SR_NT < hi ? i + j * SR_NT : i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            bool tie = false;
+            if (i + j * SR_NT < hi) w += entry_weight(v[j], rp, keep, tie);
+            ties += tie;
+        }
+    }
+}
+
 __global__ __launch_bounds__(SR_NT) void sample_chunk_mass_kernel(const float* __restrict__ logits, int V, int chunk,
                                                                   const float* __restrict__ temperature,
                                                                   const int* __restrict__ top_k,
@@ -580,52 +623,287 @@ __global__ __launch_bounds__(SR_NT) void sample_chunk_mass_kernel(const float* _
     unsigned long long dropped = 0;
     if (rp.need_k) {
         const KEdge e = rp.need_p && (stages & 2) ? row_state[r].edge : k_edge(hist_k, rp, s_scan, s_res, (stages & 1) ? row_state[r].k : nullptr);
-        keep.p_key = e.key;
-        keep.ties_matter = 1;
-        keep.tie_budget = e.budget;
+        keep = RowKeep{e.key, 1, e.budget};
         dropped = e.dropped;
     }
     if (rp.need_p) {
-        // the smallest key the nucleus reaches; the entries with that key stay while the mass before them
-        // is at most p of the kept mass (reference src/infer/sampling.py:20-23: ties in sorted order, which
-        // here is vocabulary order; the first always stays): limit = p * mass, above = mass of larger keys
         unsigned long long limit = 0, above = 0;
         uint32_t mask;
         const uint32_t pk = descend(hist_p, 3, true, (double)rp.p, limit, above, mask, s_scan, s_res,
                                     (stages & 2) ? row_state[r].p : nullptr, dropped);
-        if (!rp.need_k || pk >= keep.p_key) {
-            const unsigned long long w = fix_weight(expf(key_value(pk) - rp.zmax));
-            const unsigned long long room = limit > above ? limit - above : 0ull;
-            const unsigned long long fit = w ? room / w + 1ull : 0x7fffffffull;
-            const int by_mass = fit > 0x7fffffffull ? 0x7fffffff : (int)fit;
-            const bool same = rp.need_k && pk == keep.p_key;
-            keep.tie_budget = same && keep.tie_budget < by_mass ? keep.tie_budget : by_mass;
-            keep.p_key = pk;
-            keep.ties_matter = 1;
-        }
+        cut_nucleus(keep, rp, pk, limit, above);
     }
     if (c == 0 && threadIdx.x == 0) row_keep[r] = keep;
-    const float* row = logits + (size_t)r * V;
-    const int lo = c * chunk, hi = lo + chunk < V ? lo + chunk : V;
     float w = 0.f;
     int ties = 0;
-    const bool skip = share_below(wave_v, (size_t)r * NB + c, rp.inv_t, keep.p_key);
+    if (!share_below(wave_v, (size_t)r * NB + c, rp.inv_t, keep.p_key)) chunk_share(logits + (size_t)r * V, V, chunk, c, rp, keep, w, ties);
+    block_sums(w, ties, s_w, s_n);
+    if (threadIdx.x == 0) {
+        chunk_weight[(size_t)r * NB + c] = w;
+        chunk_ties[(size_t)r * NB + c] = ties;
+    }
+}
+
+// --- rows whose top-k is small -----------------------------------------------------------------------------------------------
+//
+// What reaches the bound of sample_bound_kernel is little more than the k entries (k = 50 of 151,936: 60 to 70), so where every row of a call has such
+// a k the entries are gathered into a list a row, one read of the shares that hold any, and a block a row finds in the list where top-k and
+// top-p end, by counting, and sums the chunks' masses in the order of sample_chunk_mass_kernel. Seven launches over all chunks (six levels and the
+// masses, 84 us for 64 rows of 151,936 with both filters, most of it launches whose blocks find nothing) are two of 14.6 and 15.4: a whole call 110.9 to 58.2 us, of one / eight
+// rows 60.1 / 63.7 to 36.7 / 41.8, with k = 50 alone 73.6 / 42.8 / 45.4 to 57.7 / 36.3 / 41.5. A row whose list does not hold what
+// reaches the bound (thousands of equal logits), or that has no bound, is worked out by its block alone from the row itself, level by level
+// as the launches do it: slow, right, and rare.
+#define SR_LIST 512
+
+__global__ __launch_bounds__(SR_NT) void sample_gather_kernel(const float* __restrict__ logits, int V, int chunk, const float* __restrict__ temperature,
+                                                              const int* __restrict__ top_k, const float* __restrict__ top_p,
+                                                              const float* __restrict__ rowmax, const float* __restrict__ wave_v,
+                                                              const RowState* __restrict__ row_state, uint2* __restrict__ lists, int* __restrict__ counts) {
+    __shared__ uint2 s_list[SR_LIST];
+    __shared__ int s_n, s_base;
+    const int r = blockIdx.x, c = blockIdx.y;
+    const RowParams rp = row_params(r, V, temperature, top_k, top_p, rowmax);
+    const uint32_t bound = row_state[r].bound;
+    if (!rp.need_k || bound == 0u) return;               // block-uniform
+    const bool skip = share_below(wave_v, (size_t)r * gridDim.y + c, rp.inv_t, bound);
+    if (threadIdx.x == 0) s_n = 0;
+    if (__syncthreads_and(skip)) return;
+    const float* row = logits + (size_t)r * V;
+    const int lo = c * chunk, hi = lo + chunk < V ? lo + chunk : V;
     for (int i = lo + threadIdx.x; i < hi && !skip; i += 8 * SR_NT) {
         float v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = row[i + j * SR_NT < hi ? i + j * SR_NT : i];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            bool tie = false;
-            if (i + j * SR_NT < hi) w += entry_weight(v[j], rp, keep, tie);
-            ties += tie;
+            const float z = v[j] * rp.inv_t;
+            if (i + j * SR_NT >= hi || !(z == z)) continue;
+            const uint32_t key = order_key(z);
+            if (key < bound) continue;
+            const int at = atomicAdd(&s_n, 1);
+            if (at < SR_LIST) s_list[at] = uint2{key, (uint32_t)(i + j * SR_NT)};
         }
     }
-    block_sums(w, ties, s_w, s_n);
-    if (threadIdx.x == 0) {
-        chunk_weight[(size_t)r * NB + c] = w;
-        chunk_ties[(size_t)r * NB + c] = ties;
+    __syncthreads();
+    const int n = s_n;
+    if (threadIdx.x == 0 && n) s_base = atomicAdd(&counts[r], n);
+    __syncthreads();
+    const int base = n ? s_base : 0;
+    for (int i = threadIdx.x; i < n && i < SR_LIST && base + i < SR_LIST; i += SR_NT) lists[(size_t)r * SR_LIST + base + i] = s_list[i];
+}
+
+// The same from the row itself, by one block.
+__device__ void select_from_row(const float* __restrict__ row, int V, int chunk, int NB, const RowParams& rp, unsigned long long* __restrict__ hist,
+                                unsigned long long* s_hist, unsigned long long* s_scan, unsigned long long* s_res, float* s_w, int* s_n,
+                                float* __restrict__ chunk_weight, int* __restrict__ chunk_ties, RowKeep& keep) {
+    keep = RowKeep{0u, 0, 0};
+    unsigned long long dropped = 0, limit = 0, above = 0;
+    uint32_t mask, floor_key = 0;
+    auto levels = [&](auto BY_MASS, unsigned long long* h, double frac) {
+        constexpr bool by_mass = decltype(BY_MASS)::value;
+        for (int level = 0; level < 3; ++level) {
+            limit = (unsigned long long)rp.k;
+            const uint32_t prefix = descend(h, level, by_mass, frac, limit, above, mask, s_scan, s_res, nullptr, dropped);
+            for (int b = threadIdx.x; b < SR_BINS; b += SR_NT) s_hist[b] = 0ull;
+            __syncthreads();
+            for (int c = 0; c < NB; ++c) add_chunk<by_mass>(row, V, chunk, c, rp, level, floor_key, prefix, mask, s_hist);
+            __syncthreads();
+            for (int b = threadIdx.x; b < SR_BINS; b += SR_NT) h[(size_t)level * SR_BINS + b] = s_hist[b];
+            __threadfence_block();
+            __syncthreads();
+        }
+    };
+    if (rp.need_k) {
+        levels(std::false_type{}, hist, -1.0);
+        const KEdge e = k_edge(hist, rp, s_scan, s_res, nullptr);
+        keep = RowKeep{e.key, 1, e.budget};
+        floor_key = e.key;
+        dropped = e.dropped;
     }
+    if (rp.need_p) {
+        unsigned long long* h = hist + 3 * SR_BINS;
+        levels(std::true_type{}, h, (double)rp.p);
+        const uint32_t pk = descend(h, 3, true, (double)rp.p, limit, above, mask, s_scan, s_res, nullptr, dropped);
+        cut_nucleus(keep, rp, pk, limit, above);
+    }
+    for (int c = 0; c < NB; ++c) {
+        float w = 0.f;
+        int ties = 0;
+        chunk_share(row, V, chunk, c, rp, keep, w, ties);
+        block_sums(w, ties, s_w, s_n);
+        if (threadIdx.x == 0) {
+            chunk_weight[c] = w;
+            chunk_ties[c] = ties;
+        }
+    }
+}
+
+__global__ __launch_bounds__(SR_NT) void sample_select_kernel(const float* __restrict__ logits, int V, int chunk, int NB,
+                                                              const float* __restrict__ temperature, const int* __restrict__ top_k,
+                                                              const float* __restrict__ top_p, const float* __restrict__ rowmax,
+                                                              const RowState* __restrict__ row_state, const uint2* __restrict__ lists,
+                                                              const int* __restrict__ counts, unsigned long long* __restrict__ hist_all,
+                                                              float* __restrict__ chunk_weight, int* __restrict__ chunk_ties,
+                                                              RowKeep* __restrict__ row_keep) {
+    __shared__ unsigned long long s_hist[SR_BINS];       // (the list's weights lie in it)
+    __shared__ uint32_t s_key[SR_LIST], s_idx[SR_LIST];
+    __shared__ unsigned long long s_scan[SR_NT / TM_WAVE], s_res[2];
+    __shared__ float s_w[SR_NT / TM_WAVE];
+    __shared__ int s_n[SR_NT / TM_WAVE];
+    __shared__ int s_begin[256];
+    __shared__ RowKeep s_keep;
+    __shared__ unsigned long long s_limit;
+    constexpr int GROUP = 8;
+    const int r = blockIdx.x, t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / TM_WAVE), lane = t % TM_WAVE;
+    const RowParams rp = row_params(r, V, temperature, top_k, top_p, rowmax);
+    if (rp.greedy) return;                               // block-uniform
+    const int n = counts[r];
+    const bool listed = rp.need_k && row_state[r].bound != 0u && n >= rp.k && n <= SR_LIST;
+    chunk_weight += (size_t)r * NB;
+    chunk_ties += (size_t)r * NB;
+    if (!listed) {
+        RowKeep keep;
+        select_from_row(logits + (size_t)r * V, V, chunk, NB, rp, hist_all + (size_t)r * SR_HIST_PER_ROW, s_hist, s_scan, s_res, s_w, s_n, chunk_weight,
+                        chunk_ties, keep);
+        if (t == 0) row_keep[r] = keep;
+        return;
+    }
+    // the list by vocabulary order
+    uint2 mine[SR_LIST / SR_NT];
+    for (int c = t; c < NB; c += SR_NT) s_begin[c] = n;
+#pragma unroll
+    for (int j = 0; j < SR_LIST / SR_NT; ++j) {
+        const int i = t + j * SR_NT;
+        mine[j] = lists[(size_t)r * SR_LIST + (i < n ? i : 0)];
+        s_idx[i] = i < n ? mine[j].y : 0xffffffffu;      // (what pads the list to whole groups is behind all, smaller than all, and weighs nothing)
+    }
+    __syncthreads();
+    const int padded = (n + GROUP - 1) / GROUP * GROUP;
+    int place[SR_LIST / SR_NT];
+#pragma unroll
+    for (int j = 0; j < SR_LIST / SR_NT; ++j) place[j] = 0;
+    for (int i0 = 0; i0 < padded; i0 += GROUP) {
+        uint32_t other[GROUP];
+#pragma unroll
+        for (int i = 0; i < GROUP; ++i) other[i] = s_idx[i0 + i];
+#pragma unroll
+        for (int i = 0; i < GROUP; ++i)
+#pragma unroll
+            for (int j = 0; j < SR_LIST / SR_NT; ++j) place[j] += other[i] < mine[j].y;
+    }
+    __syncthreads();
+    unsigned long long* s_weight = s_hist;
+    for (int i = n + t; i < padded; i += SR_NT) {
+        s_key[i] = 0u;
+        s_weight[i] = 0ull;
+    }
+#pragma unroll
+    for (int j = 0; j < SR_LIST / SR_NT; ++j) {
+        if (t + j * SR_NT >= n) continue;
+        s_key[place[j]] = mine[j].x;
+        s_idx[place[j]] = mine[j].y;
+        s_weight[place[j]] = fix_weight(expf(key_value(mine[j].x) - rp.zmax));
+    }
+    __syncthreads();
+    // of every entry: how many are larger, their mass, and how many are equal
+    int larger[SR_LIST / SR_NT], equal[SR_LIST / SR_NT];
+    unsigned long long above[SR_LIST / SR_NT];
+    uint32_t key[SR_LIST / SR_NT];
+#pragma unroll
+    for (int j = 0; j < SR_LIST / SR_NT; ++j) {
+        larger[j] = equal[j] = 0;
+        above[j] = 0ull;
+        key[j] = t + j * SR_NT < n ? s_key[t + j * SR_NT] : 0u;
+    }
+    for (int i0 = 0; i0 < padded; i0 += GROUP) {
+        uint32_t other[GROUP];
+        unsigned long long w[GROUP];
+#pragma unroll
+        for (int i = 0; i < GROUP; ++i) other[i] = s_key[i0 + i], w[i] = s_weight[i0 + i];
+#pragma unroll
+        for (int i = 0; i < GROUP; ++i)
+#pragma unroll
+            for (int j = 0; j < SR_LIST / SR_NT; ++j) {
+                larger[j] += other[i] > key[j];
+                equal[j] += other[i] == key[j];
+                above[j] += other[i] > key[j] ? w[i] : 0ull;
+            }
+    }
+    // the k-th largest; the mass from it up, without the ties that do not stay, times p
+#pragma unroll
+    for (int j = 0; j < SR_LIST / SR_NT; ++j) {
+        if (t + j * SR_NT >= n || larger[j] >= rp.k || larger[j] + equal[j] < rp.k) continue;
+        const unsigned long long w = s_weight[t + j * SR_NT];
+        const int budget = rp.k - larger[j];
+        const unsigned long long dropped = (unsigned long long)(equal[j] - budget) * w, total = above[j] + (unsigned long long)equal[j] * w;
+        s_keep = RowKeep{key[j], 1, budget};             // (threads that write them write the same)
+        s_limit = (unsigned long long)((double)(total > dropped ? total - dropped : 0ull) * (double)rp.p);
+    }
+    __syncthreads();
+    if (rp.need_p) {
+        const unsigned long long limit = s_limit;
+        const RowKeep kept = s_keep;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < SR_LIST / SR_NT; ++j) {
+            if (t + j * SR_NT >= n || key[j] < kept.p_key) continue;
+            if (above[j] > limit || above[j] + (unsigned long long)equal[j] * s_weight[t + j * SR_NT] <= limit) continue;
+            RowKeep keep = kept;
+            cut_nucleus(keep, rp, key[j], limit, above[j]);
+            s_keep = keep;
+        }
+        __syncthreads();
+    }
+    const RowKeep keep = s_keep;
+    if (t == 0) row_keep[r] = keep;
+    // the chunks' masses: lanes and wavefronts have the entries that are theirs in sample_chunk_mass_kernel, added as there
+    for (int i = t; i < n; i += SR_NT) {
+        const int c = (int)s_idx[i] / chunk;
+        if (i == 0 || (int)s_idx[i - 1] / chunk != c) s_begin[c] = i;
+    }
+    __syncthreads();
+    for (int c = t; c < NB; c += SR_NT)
+        if (s_begin[c] == n) {
+            chunk_weight[c] = 0.f;
+            chunk_ties[c] = 0;
+        }
+    for (int c0 = 0; c0 < NB; c0 += TM_WAVE) {
+        // of the chunks that have entries, a wavefront takes every fourth
+        unsigned long long left = __ballot(c0 + lane < NB && s_begin[c0 + lane < NB ? c0 + lane : 0] < n);
+        for (int turn = 0; left; left &= left - 1, ++turn) {
+            if (turn % (SR_NT / TM_WAVE) != wave) continue;
+            const int c = c0 + __builtin_ctzll(left), lo = c * chunk, hi = lo + chunk;
+            float w[SR_NT / TM_WAVE];
+            int ties = 0;
+#pragma unroll
+            for (int v = 0; v < SR_NT / TM_WAVE; ++v) w[v] = 0.f;
+            for (int i = s_begin[c]; i < n && (int)s_idx[i] < hi; ++i) {     // the same in every lane
+                const int off = (int)s_idx[i] - lo;
+                const uint32_t k = s_key[i];
+                ties += k == keep.p_key;
+                const float e = k > keep.p_key ? expf(key_value(k) - rp.zmax) : 0.f;
+#pragma unroll
+                for (int v = 0; v < SR_NT / TM_WAVE; ++v)
+                    if (off % SR_NT == v * TM_WAVE + lane) w[v] += e;
+            }
+#pragma unroll
+            for (int v = 0; v < SR_NT / TM_WAVE; ++v) w[v] = lane_sum<1>(lane_sum<2>(lane_sum<4>(lane_sum<8>(lane_sum<16>(lane_sum<32>(w[v]))))));
+            float sum = w[0];
+#pragma unroll
+            for (int v = 1; v < SR_NT / TM_WAVE; ++v) sum += w[v];
+            if (lane == 0) {
+                chunk_weight[c] = sum;
+                chunk_ties[c] = ties;
+            }
+        }
+    }
+}
+
+// The largest k for which the calls of a vocabulary may say that their rows' entries fit a list: three quarters of the shares whose maxima bound them
+// (up to 1.4 entries a share reach it then).
+extern "C" int tm_sample_list_k(int V) {
+    const int NB = tm_argmax_work_chunks(V), shares = NB * (AM_NT / TM_WAVE) <= SR_NT ? NB * (AM_NT / TM_WAVE) : NB;
+    return V > 0 && NB > 1 ? shares * 3 / 4 : 0;
 }
 
 // Of `ties` ties that follow `seen` earlier ones, how many stay.
@@ -733,13 +1011,9 @@ __global__ __launch_bounds__(SR_NT) void sample_pick_kernel(const float* __restr
         bool tie = false;
         wj[j] = i < hi ? entry_weight(raw[j], rp, keep, tie) : 0.f;
         tie_bits |= (tie ? 1u : 0u) << j;
-        float w = wj[j];
-        int n = tie;
-#pragma unroll
-        for (int off = TM_WAVE / 2; off > 0; off >>= 1) {
-            w += __shfl_xor(w, off, TM_WAVE);
-            n += __shfl_xor(n, off, TM_WAVE);
-        }
+        // (by the vector unit and a ballot: through LDS the launch took 2 us longer)
+        const float w = lane_sum<1>(lane_sum<2>(lane_sum<4>(lane_sum<8>(lane_sum<16>(lane_sum<32>(wj[j]))))));
+        const int n = __popcll(__ballot(tie));
         if (lane == 0) {
             s_pw[wave][j] = w;
             s_pn[wave][j] = n;
@@ -808,11 +1082,13 @@ static size_t sample_hist_bytes(int R) { return (size_t)R * SR_HIST_PER_ROW * si
 extern "C" size_t tm_sample_work_bytes(int R, int V) {
     const size_t NB = (size_t)tm_argmax_work_chunks(V);
     const size_t per_chunk = (size_t)R * NB * 4;         // part_v, part_i, chunk_weight, chunk_ties, wave_v
-    return sample_hist_bytes(R) + (size_t)R * sizeof(RowState) + (4 + AM_NT / TM_WAVE) * per_chunk + (size_t)R * (sizeof(RowKeep) + 8);
+    return sample_hist_bytes(R) + (size_t)R * sizeof(RowState) + (size_t)R * SR_LIST * sizeof(uint2) + (4 + AM_NT / TM_WAVE) * per_chunk +
+           (size_t)R * (sizeof(RowKeep) + 12);
 }
 
 // stages: bit 0 = some row may use top-k, bit 1 = some row may use top-p (3 if the caller does not
-// know: rows that use neither skip those launches' work). Calls on one `work` must not overlap.
+// know: rows that use neither skip those launches' work); bit 2 = every row that is not greedy uses a top-k of at most tm_sample_list_k(V): the
+// entries go through a list a row (a row that uses none, or a larger one, is right all the same, and slow). Calls on one `work` must not overlap.
 extern "C" int tm_sample_rows(const float* logits, int R, int V, const float* temperature, const int* top_k,
                               const float* top_p, const float* u, int* out, void* work, size_t work_bytes,
                               int stages, hipStream_t stream) {
@@ -825,6 +1101,7 @@ extern "C" int tm_sample_rows(const float* logits, int R, int V, const float* te
     unsigned long long* hist = (unsigned long long*)w;
     w += sample_hist_bytes(R);
     RowState* state = (RowState*)w;     w += (size_t)R * sizeof(RowState);
+    uint2* lists = (uint2*)w;           w += (size_t)R * SR_LIST * sizeof(uint2);
     float* part_v = (float*)w;          w += (size_t)R * NB * 4;
     int* part_i = (int*)w;              w += (size_t)R * NB * 4;
     float* wave_v = (float*)w;          w += (size_t)R * NB * (AM_NT / TM_WAVE) * 4;
@@ -832,12 +1109,25 @@ extern "C" int tm_sample_rows(const float* logits, int R, int V, const float* te
     int* chunk_ties = (int*)w;          w += (size_t)R * NB * 4;
     RowKeep* row_keep = (RowKeep*)w;    w += (size_t)R * sizeof(RowKeep);
     float* rowmax = (float*)w;          w += (size_t)R * 4;
-    int* rowarg = (int*)w;
+    int* rowarg = (int*)w;              w += (size_t)R * 4;
+    int* counts = (int*)w;
     const dim3 grid(R, NB);
-    argmax_partial_kernel<<<grid, AM_NT, 0, stream>>>(logits, V, chunk, part_v, part_i, hist, SR_HIST_PER_ROW, wave_v);
+    const bool listed = (stages & 4) && NB > 1;
+    argmax_partial_kernel<<<grid, AM_NT, 0, stream>>>(logits, V, chunk, part_v, part_i, listed ? nullptr : hist, SR_HIST_PER_ROW, wave_v);
     TM_CHECK_LAUNCH();
-    sample_bound_kernel<<<R, SR_NT, 0, stream>>>(part_v, part_i, wave_v, NB, V, temperature, top_k, top_p, rowmax, rowarg, state);
+    sample_bound_kernel<<<R, SR_NT, 0, stream>>>(part_v, part_i, wave_v, NB, V, temperature, top_k, top_p, rowmax, rowarg, state, counts);
     TM_CHECK_LAUNCH();
+    if (listed) {
+        sample_gather_kernel<<<grid, SR_NT, 0, stream>>>(logits, V, chunk, temperature, top_k, top_p, rowmax, wave_v, state, lists, counts);
+        TM_CHECK_LAUNCH();
+        sample_select_kernel<<<R, SR_NT, 0, stream>>>(logits, V, chunk, NB, temperature, top_k, top_p, rowmax, state, lists, counts, hist, chunk_weight,
+                                                      chunk_ties, row_keep);
+        TM_CHECK_LAUNCH();
+        sample_pick_kernel<<<R, SR_NT, 0, stream>>>(logits, V, chunk, NB, temperature, top_k, top_p, rowmax, rowarg,
+                                                    chunk_weight, chunk_ties, row_keep, u, out);
+        TM_CHECK_LAUNCH();
+        return TM_OK;
+    }
     if (stages & 1)
         for (int level = 0; level < 3; ++level) {
             sample_hist_kernel<false><<<grid, SR_NT, 0, stream>>>(logits, V, chunk, temperature, top_k, top_p, rowmax,

@@ -385,12 +385,20 @@ def argmax_rows(logits: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
 _sample_work: dict[int, torch.Tensor] = {}
 
 
+def sample_list_k(vocab: int) -> int:
+    """The largest top-k of rows whose entries the sampler gathers into lists (``sample_rows``)."""
+    return int(library().tm_sample_list_k(c_int(vocab)))
+
+
 def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
-                u: torch.Tensor, out: torch.Tensor, uses_top_k: bool = True, uses_top_p: bool = True) -> torch.Tensor:
+                u: torch.Tensor, out: torch.Tensor, uses_top_k: bool = True, uses_top_p: bool = True,
+                small_top_k: bool = False) -> torch.Tensor:
     """One token per row: argmax where temperature <= 1e-5 or top_k == 1, else the inverse CDF at
     u of softmax(logits / temperature) after the top-k / top-p filters, in vocabulary order.
     ``uses_top_k`` / ``uses_top_p``: False if the caller knows that no row asks for that filter (its
-    launches are then left out; a row that asks for none skips their work either way)."""
+    launches are then left out; a row that asks for none skips their work either way). ``small_top_k``: True if the caller
+    knows that every row that is not greedy has a top-k of 1 to ``sample_list_k(V)``: what reaches it is then gathered into
+    a list a row (the same tokens in fewer launches)."""
     _gpu(logits, temperature, top_k, top_p, u, out)
     R, V = logits.shape
     _need(logits.dtype == torch.float32 and logits.is_contiguous(), "sample: logits must be contiguous float32 [R, V]")
@@ -406,7 +414,7 @@ def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Te
     if work is None or work.numel() < need:            # kept and grown: one sampling call at a time per device
         work = _sample_work[logits.device.index] = torch.empty(need, dtype=torch.uint8, device=logits.device)
     _check(lib.tm_sample_rows(_p(logits), c_int(R), c_int(V), _p(temperature), _p(top_k), _p(top_p), _p(u), _p(out),
-                              _p(work), ctypes.c_size_t(work.numel()), c_int((1 if uses_top_k else 0) | (2 if uses_top_p else 0)),
+                              _p(work), ctypes.c_size_t(work.numel()), c_int((1 if uses_top_k else 0) | (2 if uses_top_p else 0) | (4 if small_top_k else 0)),
                               _stream()), "sample_rows")
     return out
 

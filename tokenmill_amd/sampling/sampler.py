@@ -119,7 +119,9 @@ class Sampler:
         host[3] = ks                                              # int32 bits travel in the same copy
         dev = host.to(logits.device, non_blocking=True)
         vocab = logits.shape[1]
+        most = ops.sample_list_k(vocab)
         ops.sample_rows(logits, dev[0], dev[3].view(torch.int32), dev[1], dev[2], out,
                         uses_top_k=any(not p.greedy and 0 < p.top_k < vocab for p in params),
-                        uses_top_p=any(not p.greedy and p.top_p < 1.0 for p in params))
+                        uses_top_p=any(not p.greedy and p.top_p < 1.0 for p in params),
+                        small_top_k=all(p.greedy or 0 < p.top_k <= most for p in params))
         return out
