@@ -48,6 +48,23 @@ def test_products_plain_and_in_parts(M, N, K):
     assert (sums.double().sum(0) - ref).abs().max() <= _bound(K)
 
 
+@pytest.mark.parametrize("N,K", [(20, 48), (36, 16 * 57), (896, 896), (40, 16 * 431), (2048, 5632), (8200, 912), (9000, 112)])
+def test_a_row_is_the_same_whatever_rows_are_beside_it(N, K):
+    """Odd numbers of steps, runs of one group and of several with a rest, one tile and two; up to four, up to eight and more rows."""
+    lib = library()
+    a, w, ref = _operands(16, N, K, N + K)
+
+    def product(rows):
+        out = torch.full((rows, N), float("nan"), device="cuda")
+        assert lib.tm_gemv_f32_mfma(_ptr(a), I(K), _ptr(w), _ptr(None), _ptr(out), I(N), I(rows), I(N), I(K), _stream()) == 0
+        return out
+
+    most = product(16)
+    assert (most.double() - ref).abs().max() <= _bound(K)
+    for rows in (1, 4, 5, 8, 9):
+        assert torch.equal(product(rows), most[:rows]), rows
+
+
 def test_a_long_k_is_split():
     assert library().tm_gemv_f32_parts(896, 4864) == 4 and library().tm_gemv_f32_parts(896, 896) == 1
 

@@ -4,16 +4,24 @@
 //
 // Such a product is bound by reading its matrix once (35 MB for gate|up of the 0.5B shape) and, where that is small, by the trips to
 // memory. A block takes RT tiles of 16 matrix rows (SiLU and q|k|v: one, of 8 rows and the 8 that meet them, twice the blocks);
-// its wavefronts split K into runs of steps of 16 k and ask for several steps of matrix and activations at once, in the matrix
-// instruction's own layout (lane (r, g): 16 bytes of row r at 4 g), so nothing goes through LDS but the wavefronts' sums at the
-// end, added in wavefront order. The activations come from the second-level cache. Which k goes where depends on the matrix
-// alone: a row's result does not depend on the other rows. Non-temporal loads cost a tenth here: a line's two halves are
-// asked for by two instructions.
-// Before, a wavefront had 256 k of four rows, a lane 4 k each, and summed over the lanes by shuffles, 6 x 32 of them a wavefront:
-// 19.0 us a product of the 0.5B shape on average, with SiLU*up and rotation in kernels behind it; now gate|up takes 12 us (2.9
-// TB/s), down 7, q|k|v and o 5, the head 126 (4.3 TB/s).
+// its wavefronts split K into runs of steps of 16 k and ask for several steps of matrix and activations at once, so nothing goes through
+// LDS but the wavefronts' sums at the end, added in halves. The activations come from the second-level cache. Which k goes where
+// depends on the matrix alone: a row's result does not depend on the other rows.
+//
+// The matrix instruction wants 16 bytes of row r at 4 g in lane (r, g), 64 bytes of each of sixteen rows. A CU takes such loads in at half
+// the rate of whole lines (a line costs it the same either way; 30 to 40 KB a us against 130 a block alone on its CU), so two steps are loaded
+// as a pair, 128 bytes of eight rows an instruction, and the lanes r and r + 8 exchange what belongs to the other, which is eight
+// instructions of the vector unit a pair. Up to eight rows of activations are one load a pair, and whole lines that
+// nobody reads again pass the caches by (non-temporal: the head 98 to 85 us, down 6.7 to 6.5). Against a load a step, cold matrices,
+// 1 / 8 / 16 rows, us: gate|up of the 0.5B shape 10.9 / 12.3 / 14.4 to 9.0 / 10.2 / 12.2, down 6.4 / 7.2 / 8.6 to 5.7 / 6.5 / 7.8, o
+// 4.7 / 5.5 / 6.5 to 4.4 / 4.9 / 5.8, q|k|v 5.3 / 6.2 / 7.2 to 5.1 / 5.7 / 6.5, the head 119 / 129 / 140 to 81 / 85 / 98 (6.4 TB/s at
+// 8 rows); 3,584 -> 2 x 18,944 103 / 128 / - to 85 / 101 / -.
+// Before that, a wavefront had 256 k of four rows, a lane 4 k each, and summed over the lanes by shuffles, 6 x 32 of them a wavefront:
+// 19.0 us a product of the 0.5B shape on average, with SiLU*up and rotation in kernels behind it.
 #include "common.h"
 #include "api.h"
+
+#include <type_traits>
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -36,9 +44,28 @@ struct GemvArgs {
     float* v_pool;              // [pages, KVH, D, page]
 };
 
+// A pair of steps as it is loaded (lane (r, g): row r % 8, or 8 + r % 8, step r / 8 of the two) to the matrix instruction's
+// layout (row r): the lanes of the other half of a row of sixteen hold what is missing.
+__device__ __forceinline__ f32x4_t turned(f32x4_t v) {
+    f32x4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[e]), 0x128, 0xf, 0xf, false));
+    return o;
+}
+__device__ __forceinline__ f32x4_t fragment(int step, f32x4_t lo, f32x4_t hi) {
+    f32x4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int l = __float_as_int(lo[e]), h = __float_as_int(hi[e]);
+        o[e] = __int_as_float(step ? __builtin_amdgcn_update_dpp(h, l, 0x128, 0xf, 0x3, false) : __builtin_amdgcn_update_dpp(l, h, 0x128, 0xf, 0xc, false));
+    }
+    return o;
+}
+
 // GROUP: steps of 16 k whose products meet in sums of their own before they join the running one. AHEAD: groups a wavefront asks for
 // at once: with one, a wavefront of the 0.5B shape waited for memory two times in a launch of 6 to 7 us (o 6.2 to 5.8, q|k|v 7.2 to 6.8).
-template <int EPI, int RT, int WAVES, int GROUP, int AHEAD>
+// OVER8: more than eight rows of activations.
+template <int EPI, int RT, int WAVES, int GROUP, int AHEAD, bool OVER8>
 __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArgs a) {
     static_assert(EPI == GM_PLAIN || RT == 1, "");
     __shared__ __align__(16) f32x4_t red[WAVES][RT][TM_WAVE];
@@ -64,16 +91,24 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     const int steps = a.K / 16;
     const int per_block = (steps + gridDim.y - 1) / gridDim.y;
     const int b0 = blockIdx.y * per_block, b1 = b0 + per_block < steps ? b0 + per_block : steps;
-    const int per = (per_block + WAVES - 1) / WAVES;
+    // (Whole pairs: whole lines. With the wavefronts' sums added in halves the results are as near to 64 bits as with equal runs added in a
+    // row, rms 896 -> 896 1.014 to 0.993e-7, 4,864 -> 896 1.187 to 1.145e-7, 18,944 -> 3,584 1.518 to 1.488e-7.)
+    const int per = (per_block + 2 * WAVES - 1) / (2 * WAVES) * 2;
     const int s0 = b0 + wave * per, s1 = s0 + per < b1 ? s0 + per : b1;
-    const float* pa = a.A + (size_t)(r < a.M ? r : a.M - 1) * a.lda + 4 * g;
-    const float* pw[RT];
+    // rows r % 8 and 8 + r % 8 (rows beyond the matrix, the half or the input: its last one, never stored)
+    const int r8 = r % 8, second = r / 8;
+    const float* pa[2];
+    const float* pw[RT][2];
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-        // (rows beyond the matrix, or the half: its last one, never stored)
-        const int end = EPI == GM_SILU ? a.I : a.N, at = n0[t] + (EPI == GM_PLAIN ? r : r % 8);
-        const int n = (at < end ? at : end - 1) + (EPI != GM_PLAIN && r >= 8 ? far : 0);
-        pw[t] = a.W + (size_t)n * a.K + 4 * g;
+    for (int h = 0; h < 2; ++h) {
+        const int row = r8 + 8 * h;
+        pa[h] = a.A + (size_t)(row < a.M ? row : a.M - 1) * a.lda + 4 * g;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int end = EPI == GM_SILU ? a.I : a.N, at = n0[t] + (EPI == GM_PLAIN ? row : r8);
+            const int n = (at < end ? at : end - 1) + (EPI != GM_PLAIN ? h * far : 0);
+            pw[t][h] = a.W + (size_t)n * a.K + 4 * g;
+        }
     }
     // What the epilogue waits for otherwise: the positions are asked for before the matrix (loads come back in their order), the
     // rotary rows, whose place hangs on them, behind its first round.
@@ -92,15 +127,19 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     f32x4_t sum[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) sum[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int s = s0; s < s1; s += GROUP * AHEAD) {
-        f32x4_t w[RT][GROUP * AHEAD], x[GROUP * AHEAD];
+    auto groups = [&](auto AT_ONCE, int s) {
+        constexpr int GROUPS = decltype(AT_ONCE)::value, PAIRS = (GROUP * GROUPS + 1) / 2;
+        f32x4_t w[RT][PAIRS][2], x[PAIRS][OVER8 ? 2 : 1];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < GROUP * AHEAD; ++i) {
-            const int at = 16 * (s + i < s1 ? s + i : s1 - 1);  // (no load under a test: beyond the end the last step again)
+        for (int i = 0; i < PAIRS; ++i) {
+            const int step = s + 2 * i + second, at = 16 * (step < s1 ? step : s1 - 1);  // (no load under a test: beyond the end the last step again)
 #pragma unroll
-            for (int t = 0; t < RT; ++t) w[t][i] = *(const f32x4_t*)(pw[t] + at);
-            x[i] = *(const f32x4_t*)(pa + at);
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int t = 0; t < RT; ++t) w[t][i][h] = __builtin_nontemporal_load((const f32x4_t*)(pw[t][h] + at));
+                if (h == 0 || OVER8) x[i][h] = *(const f32x4_t*)(pa[h] + at);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (EPI == GM_QKV) {
@@ -112,7 +151,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int j = 0; j < AHEAD; ++j) {
+        for (int j = 0; j < GROUPS; ++j) {
             if (s + j * GROUP >= s1) break;                     // the same for the whole wavefront
             // four sums a tile, of every fourth k, that join the running one here: short chains of roundings
             f32x4_t acc[RT][4];
@@ -123,15 +162,27 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
 #pragma unroll
             for (int i = j * GROUP; i < (j + 1) * GROUP; ++i) {
                 if (s + i >= s1) break;
+                const f32x4_t xf = OVER8 ? fragment(i % 2, x[i / 2][0], x[i / 2][OVER8 ? 1 : 0]) : i % 2 ? turned(x[i / 2][0]) : x[i / 2][0];
+                f32x4_t wf[RT];
+#pragma unroll
+                for (int t = 0; t < RT; ++t) wf[t] = fragment(i % 2, w[t][i / 2][0], w[t][i / 2][1]);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
                     for (int t = 0; t < RT; ++t)
-                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i][e], x[i][e], acc[t][e], 0, 0, 0);
+                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[t][e], xf[e], acc[t][e], 0, 0, 0);
             }
 #pragma unroll
             for (int t = 0; t < RT; ++t) sum[t] += (acc[t][0] + acc[t][1]) + (acc[t][2] + acc[t][3]);
         }
+    };
+    // what is left when no AHEAD groups are is one group less (two tiles have no registers for the second loop: it takes the head from 98 to
+    // 151 us at 16 rows, and what they ask for beyond the end is the last step again)
+    int s = s0;
+    constexpr int LEAST = RT == 1 ? GROUP * (AHEAD - 1) : 0;
+    for (; s + LEAST < s1; s += GROUP * AHEAD) groups(std::integral_constant<int, AHEAD>{}, s);
+    if constexpr (LEAST > 0) {
+        if (s < s1) groups(std::integral_constant<int, AHEAD - 1>{}, s);
     }
 #pragma unroll
     for (int t = 0; t < RT; ++t) red[wave][t][lane] = sum[t];
@@ -139,10 +190,14 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     // lane (r, g): row r of A, rows 4 g .. + 3 of the tile
     if (EPI == GM_PLAIN ? wave >= RT : wave > 0 || g >= 2) return;
     auto total = [&](int t, int of) {
-        f32x4_t v = red[0][t][of];
+        f32x4_t v[WAVES];
 #pragma unroll
-        for (int w = 1; w < WAVES; ++w) v += red[w][t][of];
-        return v;
+        for (int w = 0; w < WAVES; ++w) v[w] = red[w][t][of];
+#pragma unroll
+        for (int n = WAVES / 2; n > 0; n /= 2)
+#pragma unroll
+            for (int w = 0; w < n; ++w) v[w] += v[w + n];
+        return v[0];
     };
     if constexpr (EPI == GM_PLAIN) {
         const int n = n0[0] + 16 * wave + 4 * g;
@@ -209,19 +264,27 @@ extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, con
 }
 
 // Up to a block a CU, eight wavefronts split K into groups of four steps; more blocks than that have four wavefronts with groups of seven, whose
-// blocks a CU hide each other's waits. A wavefront of the eight that has up to three groups asks for all of them at once; with more it
-// asks for a group at a time: what it asks for beyond its end is loads that others wait for (K cut into 16 steps a wavefront, 2,048 -> 2,048,
-// 1 / 8 / 16 rows, us: two rounds of three groups 9.4 / 11.5 / 13.5, four of one 7.7 / 8.6 / 10.0). Steps of the 0.5B shape with 1 / 8 / 16 requests
-// take 1,133 / 1,258 / 1,422 us so and 1,149 / 1,259 / 1,432 with a group at a time everywhere; launches in a row alone show no difference, and 3%
-// the other way where the groups are a quarter longer than K (2,816 -> 1,024 in four parts 4.7 to 4.8).
-#define GM_LAUNCH(EPI, RT, units, split)                                                                                    \
-    do {                                                                                                                    \
-        const int per_ = ((a.K / 16 + (split) - 1) / (split) + 7) / 8;                                                      \
-        if ((units) * (split) > 256) gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1><<<dim3(units, split), 256, 0, stream>>>(a);     \
-        else if (per_ <= 4 || per_ > 12) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1><<<dim3(units, split), 512, 0, stream>>>(a); \
-        else if (per_ <= 8) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2><<<dim3(units, split), 512, 0, stream>>>(a);              \
-        else gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3><<<dim3(units, split), 512, 0, stream>>>(a);                             \
-    } while (0)
+// blocks a CU hide each other's waits. A wavefront of the eight that has up to three groups asks for all of them at once; with more, of
+// up to four rows two groups at a time and of more rows one (K cut into 32 to 56 steps a wavefront, one group / two, us: 18,944 -> 3,584, 1 / 4 / 8 /
+// 16 rows 50.5 / 43.6, 50.7 / 47.3, 52.4 / 54.4, 67.7 / 69.5; 5,632 -> 2,048 10.7 / 9.7, 10.8 / 10.1, 11.0 / 11.6, 13.1 / 14.3). One of the four
+// asks for two groups where it has them: a group at a time leaves half a pair's line, and gate|up of the 0.5B shape takes 12.2 us so for 10.2.
+template <int EPI, int RT, bool OVER8>
+static void gm_launch_rows(const GemvArgs& a, int units, int split, hipStream_t stream) {
+    const int steps = (a.K / 16 + split - 1) / split, per = (steps + 15) / 16 * 2;
+    const dim3 grid(units, split);
+    if (units * split > 256) {
+        if (steps <= 4 * 7) gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1, OVER8><<<grid, 256, 0, stream>>>(a);
+        else gemv_mfma_f32_kernel<EPI, RT, 4, 7, 2, OVER8><<<grid, 256, 0, stream>>>(a);
+    } else if (per <= 4 || (per > 12 && a.M > 4)) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1, OVER8><<<grid, 512, 0, stream>>>(a);
+    else if (per <= 8 || per > 12) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2, OVER8><<<grid, 512, 0, stream>>>(a);
+    else gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3, OVER8><<<grid, 512, 0, stream>>>(a);
+}
+
+template <int EPI, int RT>
+static void gm_launch(const GemvArgs& a, int units, int split, hipStream_t stream) {
+    if (a.M > 8) gm_launch_rows<EPI, RT, true>(a, units, split, stream);
+    else gm_launch_rows<EPI, RT, false>(a, units, split, stream);
+}
 
 extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,
                                 hipStream_t stream) {
@@ -230,8 +293,8 @@ extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const f
     a.A = A; a.W = W; a.bias = bias; a.C = C; a.lda = lda; a.ldc = ldc; a.M = M; a.N = N; a.K = K;
     // two tiles a block read the activations once for both, where that still gives every CU a block
     const int two = (N + 31) / 32, one = (N + 15) / 16;
-    if (two >= 256) GM_LAUNCH(GM_PLAIN, 2, two, 1);
-    else GM_LAUNCH(GM_PLAIN, 1, one, 1);
+    if (two >= 256) gm_launch<GM_PLAIN, 2>(a, two, 1, stream);
+    else gm_launch<GM_PLAIN, 1>(a, one, 1, stream);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
@@ -250,7 +313,7 @@ extern "C" int tm_gemv_f32_mfma_split(const float* A, int lda, const float* W, f
     GemvArgs a{};
     a.A = A; a.W = W; a.parts = parts; a.lda = lda; a.M = M; a.N = N; a.K = K;
     const int units = (N + 15) / 16;
-    GM_LAUNCH(GM_PLAIN, 1, units, tm_gemv_f32_parts(N, K));
+    gm_launch<GM_PLAIN, 1>(a, units, tm_gemv_f32_parts(N, K), stream);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
@@ -260,7 +323,7 @@ extern "C" int tm_gemv_f32_gate_up_silu(const float* A, int lda, const float* W,
     if (I <= 0 || I % 4 || !gm_aligned16(act) || !tm_gemv_f32_mfma_takes(A, lda, W, nullptr, M, 2 * I, K)) return TM_ERR_ARG;
     GemvArgs a{};
     a.A = A; a.W = W; a.C = act; a.lda = lda; a.ldc = I; a.M = M; a.N = 2 * I; a.K = K; a.I = I;
-    GM_LAUNCH(GM_SILU, 1, (I + 7) / 8, 1);
+    gm_launch<GM_SILU, 1>(a, (I + 7) / 8, 1, stream);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
@@ -277,7 +340,7 @@ extern "C" int tm_gemv_f32_qkv_rope(const float* A, int lda, const float* W, con
     a.A = A; a.W = W; a.bias = bias; a.C = q; a.lda = lda; a.ldc = H * D; a.M = M; a.N = N; a.K = K;
     a.H = H; a.KVH = KVH; a.D = D; a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots; a.k_pool = k_pool; a.v_pool = v_pool;
     while ((1 << a.page_shift) < page) ++a.page_shift;
-    GM_LAUNCH(GM_QKV, 1, N / 16, 1);
+    gm_launch<GM_QKV, 1>(a, N / 16, 1, stream);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
