@@ -94,10 +94,21 @@ __device__ __forceinline__ void gt_round2(float& a, float& b) {
 // the division for every bfloat16 x, in seven instructions for eleven: at one wavefront a SIMD an epilogue's instructions are
 // its time (2,048 rows of 896 -> 2 x 4,864, in a step: 4.3 us more than the one-instruction exponential and reciprocal, whose
 // error is 3e-6 of the value at the far end where this one's is 1.3e-7; with the division itself 6.1 us more).
+//
+// exp(-x) after Cody and Waite: -x log2(e) from the constant's two parts, its whole number to the exponent, 2 to the rest by the hardware. x is
+// held to +-128, where that ends in infinity and zero, in place of the two comparisons and choices that expf has behind it; the same
+// bits for every bfloat16 x (gate|up with SiLU*up, launches in a row, 896 -> 2 x 4,864 at 300 / 541 / 1,024 / 2,048 rows 11.0 / 14.9 /
+// 25.3 / 39.7 to 10.7 / 14.7 / 24.6 / 38.8 us).
+__device__ __forceinline__ float gt_exp_minus(float x) {
+#pragma clang fp contract(off)
+    const float c = __builtin_amdgcn_fmed3f(x, -128.f, 128.f), t = c * -1.44269502f, n = __builtin_rintf(t);
+    const float rest = fmaf(c, -1.92596299e-8f, fmaf(c, -1.44269502f, -t));
+    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - n) + rest), (int)n);
+}
 template <typename T>
 __device__ __forceinline__ float gt_silu(float x) {
-    const float e = expf(-x);
-    if constexpr (sizeof(T) == 4) return x / (1.f + e);
+    if constexpr (sizeof(T) == 4) return x / (1.f + expf(-x));
+    const float e = gt_exp_minus(x);
     const float n = 0.25f * x, d = fmaf(e, 0.25f, 0.25f), r = __builtin_amdgcn_rcpf(d), q = n * r;
     return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
 }
