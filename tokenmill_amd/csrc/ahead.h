@@ -198,7 +198,21 @@ int tile_qkv_rope_ahead(const void* A, int lda, int M, int K, const void* W, con
                         TmAhead& ahead, hipStream_t stream);
 int attn_prefill_ahead(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool, const int* block_tables,
                        int table_width, const int* tiles, int n_tiles, int H, int KVH, int D, int page, float scale, int window, int keep, float softcap,
-                       const float* sink, const void* cgate, int ldcg, TmAhead& ahead, hipStream_t stream);
+                       const float* sink, const void* cgate, int ldcg, TmAhead& ahead, hipStream_t stream, struct TmDecodes* beside = nullptr);
+
+// Single decoded tokens that a launch over prompt portions attends too (choose.h: tm_prefill_takes_decodes), of the same pools, strides and options; as
+// attn_decode_whole_ahead's arguments.
+struct TmDecodes {
+    const void* q;
+    void* out;
+    const int* tables;
+    const int* context_lens;
+    const void* cgate;
+    int n, chunks;
+    float cap_out;              // (attn_prefill_ahead's own)
+};
+bool decode_args_ok(const void* q, int q_stride, const void* out, int out_stride, int table_width, int max_chunks, int H, int KVH, int D, int page,
+                    float scale, int window, int keep, float softcap, const void* cgate, int ldcg);
 
 // What the blocks of the tiled products read of their matrix at a time (gemm_tile.hip): rows of a column tile (gate|up: of either half), and K in
 // so many parts of so many steps of 64.

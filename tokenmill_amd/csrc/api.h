@@ -107,6 +107,11 @@ int tm_attn_paged_generic_ext(const void* q, int q_stride, void* out, int out_st
 int tm_attn_prefill_mfma_cap(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                              const int* block_tables, int table_width, const int* tiles, int n_tiles, int H, int KVH, int D, int page,
                              float scale, int window, int keep, float softcap, const float* sink, const void* cgate, int ldcg, hipStream_t stream);
+// ... with single decoded tokens in the same launch (attention_prefill.hip: head sizes up to 64)
+int tm_attn_prefill_decodes(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool, const int* block_tables,
+                            int table_width, const int* tiles, int n_tiles, const void* qd, void* outd, const int* tables, const int* context_lens,
+                            int chunks, int n, int H, int KVH, int D, int page, float scale, int window, int keep, float softcap, const float* sink,
+                            const void* cgate, const void* cgated, int ldcg, hipStream_t stream);
 int tm_attn_prefill_shared_cap(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                                const int* block_tables, int table_width, const int* tiles, int n_tiles, int H, int KVH, int D, int page,
                                float scale, int window, int keep, float softcap, const float* sink, const void* cgate, int ldcg, hipStream_t stream);

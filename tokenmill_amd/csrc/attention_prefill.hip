@@ -20,6 +20,9 @@
 #include "attention_prefill_common.h"
 #include "choose.h"
 #include "ahead.h"
+#include "attention_decode_keys.h"
+
+#include <algorithm>
 
 template <int D>
 struct KVBlock {
@@ -197,20 +200,49 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, HeadState<D, HPW>&
 // With pair != 0 a block takes tile b and then tile n_tiles - 1 - b: in a table sorted by the
 // number of keys a tile sees, the longest goes with the shortest and every block has the same work
 // (the lower triangle of a prompt, folded).
-template <int D, int HPW, int KS, bool CAP, bool AHEAD>
+// DECODES: `decodes.layers` layers of the grid in front attend single decoded tokens, a (request, kv head) a block (attend_whole). On its own that
+// is a launch, or two, that waits for its trips to memory, behind one that leaves CUs without a block or their matrix units idle; the blocks in front
+// are the first to get a CU, so a launch that does not fit the chip at once has its long blocks last. Prompt portions, tokens decoded beside them, us of
+// both launches and of one (0.5B shape): 2 of 241 tokens behind 482, 30 of contexts to 1,000 17.2 to 12.1; 1 of 100, 4 of 300 10.2 to 5.9; 1 of 400 behind
+// 1,000, 60 of 1,500 25.4 to 15.2; 4 of 400, 60 of 1,000 26.2 to 20.1; 2 of 256, 100 of 800 16.7 to 16.3.
+struct KernelDecodes {
+    const bf16_t* q;
+    bf16_t* out;
+    const int* tables;
+    const int* context_lens;
+    const bf16_t* cgate;
+    int n, pairs, layers, chunks;
+    float cap_out;
+};
+struct NoDecodes {};
+template <bool DECODES>
+using DecodesArg = std::conditional_t<DECODES, KernelDecodes, NoDecodes>;
+
+template <int D, int HPW, int KS, bool CAP, bool AHEAD, bool DECODES>
 __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
     int table_width, const int* __restrict__ tiles, int n_tiles, int pair, int H, int KVH, int page_shift,
     float scale_log2, float cap_in, float cap_out, int window, int keep, const float* __restrict__ sink,
-    const bf16_t* __restrict__ cgate, int ldcg, const TmAheadArg<AHEAD> ahead) {
+    const bf16_t* __restrict__ cgate, int ldcg, const TmAheadArg<AHEAD> ahead, const DecodesArg<DECODES> decodes) {
     constexpr int NDC = D / 32, NDT = D / 16;
     // the wavefronts' partials of all heads: rows of d four floats apart from a multiple of 64, so that 16 lanes of a store or load
     // of 16 bytes meet no bank twice
     __shared__ float s_m[KS][HPW][16], s_l[KS][HPW][16];
     extern __shared__ __align__(16) float s_o[];                     // [KS][HPW][16][D + 4]
+    int layer = blockIdx.z;
+    if constexpr (DECODES) {
+        if (layer < decodes.layers) {
+            const int pair = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * layer), of = pair / decodes.n;
+            if (pair >= decodes.pairs) return;
+            return attend_whole<D, KS>(s_o, pair - of * decodes.n, of, decodes.q, q_stride, decodes.out, out_stride, k_pool, v_pool, decodes.tables,
+                                       table_width, decodes.context_lens, decodes.chunks, H, KVH, page_shift, scale_log2, cap_in, decodes.cap_out, window,
+                                       keep, sink, decodes.cgate, ldcg);
+        }
+        layer -= decodes.layers;
+    }
     if constexpr (AHEAD) {
-        if (blockIdx.z) return tm_bring_ahead(ahead, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), KS);
+        if (layer) return tm_bring_ahead(ahead, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), KS);
     }
     auto partial_at = [&](int w, int hh, int col, int d) { return s_o + (size_t)((w * HPW + hh) * 16 + col) * (D + 4) + d; };
     // the wavefront index in a scalar register: everything derived from it (its key blocks, their
@@ -356,7 +388,8 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
 // Heads a wavefront takes and wavefronts a block has, by head size (registers decide). Up to head size 64 a
 // wavefront can hold four heads, which quarters the loads of a long prompt's keys; a short step, whose blocks of
 // two heads a wavefront still fit the chip in one round, takes those instead: twice the blocks, half as long
-// (512 tokens at the 0.5B shape: 13.4 to 9.8 us). A kv head of one or two heads takes no more than it has: places that stand empty cost
+// (512 tokens at the 0.5B shape: 13.4 to 9.8 us; one a CU with the blocks of decoded tokens too, or those of four heads: 482 tokens beside 30 of
+// 1,000 keys 16.5 to 12.1). A kv head of one or two heads takes no more than it has: places that stand empty cost
 // queries, room for partials in LDS and with it blocks a CU (8 heads of 64 and as many kv heads, 17 / 512 / 2,048 tokens, four places 5.9 / 9.2 /
 // 40.6 us, one 4.1 / 7.0 / 34.8). A head's arithmetic is the same either way, so its bits are.
 template <int D> struct PrefillShape { static constexpr int HPW = D <= 64 ? 4 : 2, KS = D <= 64 ? 8 : 4; };
@@ -365,29 +398,43 @@ template <int D, int HPW, bool CAP>
 static int launch_split_keys(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                               const int* block_tables, int table_width, const int* tiles, int n_tiles, int H, int KVH,
                               int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep, const float* sink,
-                              const bf16_t* cgate, int ldcg, TmAhead& ahead, hipStream_t stream) {
+                              const bf16_t* cgate, int ldcg, TmAhead& ahead, const TmDecodes* beside, hipStream_t stream) {
     constexpr int KS = PrefillShape<D>::KS;
     const int splits = (H / KVH + HPW - 1) / HPW;
     // fold the table in two once the folded launch still gives every CU a block
     const int pair = (long long)(n_tiles / 2) * KVH * splits >= 256 ? 1 : 0;
     dim3 grid(pair ? (n_tiles + 1) / 2 : n_tiles, KVH * splits);
     constexpr int lds = KS * HPW * 16 * (D + 4) * (int)sizeof(float);          // at most 139,264 bytes
-    const bool far = (long long)grid.x * grid.y >= 256;              // (more blocks than CUs: none to spare)
+    const long long layer = (long long)grid.x * grid.y;
+    const int pairs = beside ? beside->n * KVH : 0, front = beside ? (int)((pairs + layer - 1) / layer) : 0;
+    const bool far = layer + pairs >= 256;                           // (more blocks than CUs: none to spare)
     if (far) ahead.n = 0;
-    grid.z = 1 + (far ? 0 : ahead_spare_layers(ahead, grid.x * grid.y, grid.x * grid.y));
-    auto go = [&](auto AHEAD) {
-        constexpr bool with = decltype(AHEAD)::value;
-        if (lds > 64 * 1024) {
-            static const hipError_t raised = hipFuncSetAttribute((const void*)attn_prefill_mfma_kernel<D, HPW, KS, CAP, with>,
-                                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    grid.z = 1 + front + (far ? 0 : ahead_spare_layers(ahead, layer, layer + pairs));
+    if (front) ahead.first = (int)layer * (1 + front);
+    auto go = [&](auto AHEAD, auto DECODES) {
+        constexpr bool with = decltype(AHEAD)::value, decode = decltype(DECODES)::value;
+        DecodesArg<decode> decodes;
+        int bytes = lds;
+        if constexpr (decode) {
+            decodes = {(const bf16_t*)beside->q, (bf16_t*)beside->out, beside->tables, beside->context_lens, (const bf16_t*)beside->cgate, beside->n, pairs,
+                       front, beside->chunks, beside->cap_out};
+            bytes = std::max(bytes, (int)tm_decode_whole_lds(beside->chunks, H / KVH, D));
+        }
+        constexpr int most = decode ? std::max(lds, TM_DECODE_BESIDE_LDS) : lds;
+        if (most > 64 * 1024) {
+            static const hipError_t raised = hipFuncSetAttribute((const void*)attn_prefill_mfma_kernel<D, HPW, KS, CAP, with, decode>,
+                                                                 hipFuncAttributeMaxDynamicSharedMemorySize, most);
             if (raised != hipSuccess) return TM_ERR_LAUNCH;
         }
-        attn_prefill_mfma_kernel<D, HPW, KS, CAP, with><<<grid, 64 * KS, lds, stream>>>(
+        attn_prefill_mfma_kernel<D, HPW, KS, CAP, with, decode><<<grid, 64 * KS, bytes, stream>>>(
             (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
-            table_width, tiles, n_tiles, pair, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg, ahead_arg<with>(ahead));
+            table_width, tiles, n_tiles, pair, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg, ahead_arg<with>(ahead), decodes);
         return TM_OK;
     };
-    return ahead.n ? go(std::true_type{}) : go(std::false_type{});
+    if constexpr (D <= 64) {
+        if (beside) return ahead.n ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
+    }
+    return ahead.n ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
 }
 
 // softcap > 0: a score s (scaled) becomes softcap * tanh(s / softcap) before the softmax; sink (float32 [H]) or null: one more term
@@ -397,7 +444,14 @@ static int launch_split_keys(const void* q, int q_stride, void* out, int out_str
 int attn_prefill_ahead(const void* q, int q_stride, void* out, int out_stride, const void* k_pool,
                                         const void* v_pool, const int* block_tables, int table_width, const int* tiles,
                                         int n_tiles, int H, int KVH, int D, int page, float scale, int window, int keep, float softcap,
-                                        const float* sink, const void* cgate, int ldcg, TmAhead& ahead, hipStream_t stream) {
+                                        const float* sink, const void* cgate, int ldcg, TmAhead& ahead, hipStream_t stream, TmDecodes* beside) {
+    if (beside) {
+        if (n_tiles <= 0 || beside->n <= 0 || D > 64 ||
+            !decode_args_ok(beside->q, q_stride, beside->out, out_stride, table_width, beside->chunks, H, KVH, D, page, scale, window, keep, softcap, beside->cgate, ldcg) ||
+            tm_decode_whole_lds(beside->chunks, H / KVH, D) > TM_DECODE_BESIDE_LDS || (long long)beside->n * KVH > 32768)
+            return TM_ERR_ARG;
+        beside->cap_out = softcap * 1.4426950408889634f;
+    }
     if (n_tiles <= 0) return TM_OK;
     if (!(softcap >= 0.f) || keep < 0 || (cgate && (ldcg < H * D || ldcg % 2 || (uintptr_t)cgate % 4))) return TM_ERR_ARG;
     const float cap_in = softcap > 0.f ? scale / softcap : 0.f, cap_out = softcap > 0.f ? softcap / scale : 0.f;
@@ -412,13 +466,13 @@ int attn_prefill_ahead(const void* q, int q_stride, void* out, int out_stride, c
     if ((long long)KVH * ((G + 1) / 2) > 65535) return TM_ERR_ARG;
     int rc = TM_OK;
 #define TM_SPLIT_ARGS q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, tiles, n_tiles, H, KVH, \
-                      page_shift, scale_log2, cap_in, cap_out, window, keep, sink, (const bf16_t*)cgate, ldcg, ahead, stream
+                      page_shift, scale_log2, cap_in, cap_out, window, keep, sink, (const bf16_t*)cgate, ldcg, ahead, beside, stream
 #define TM_PREFILL_CASE(DD)                                                                                       \
     case DD: {                                                                                                    \
         constexpr int HPW = PrefillShape<DD>::HPW;                                                                \
         if (G == 1)                                                                                               \
             rc = softcap > 0.f ? launch_split_keys<DD, 1, true>(TM_SPLIT_ARGS) : launch_split_keys<DD, 1, false>(TM_SPLIT_ARGS); \
-        else if (HPW > 2 && (G == 2 || (long long)n_tiles * KVH * ((G + 1) / 2) <= TM_PREFILL_ONE_ROUND))          \
+        else if (HPW > 2 && (G == 2 || ((long long)n_tiles * ((G + 1) / 2) + (beside ? beside->n : 0)) * KVH <= TM_PREFILL_ONE_ROUND)) \
             rc = softcap > 0.f ? launch_split_keys<DD, 2, true>(TM_SPLIT_ARGS) : launch_split_keys<DD, 2, false>(TM_SPLIT_ARGS); \
         else                                                                                                      \
             rc = softcap > 0.f ? launch_split_keys<DD, HPW, true>(TM_SPLIT_ARGS) : launch_split_keys<DD, HPW, false>(TM_SPLIT_ARGS); \
@@ -454,4 +508,16 @@ extern "C" int tm_attn_prefill_mfma(const void* q, int q_stride, void* out, int 
                                     hipStream_t stream) {
     return tm_attn_prefill_mfma_cap(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, tiles, n_tiles, H, KVH, D,
                                     page, scale, window, 0, 0.f, nullptr, nullptr, 0, stream);
+}
+
+// The same with single decoded tokens beside them: qd their queries and outd their results (a row a request, in the strides of q and out), of requests with
+// block tables `tables`, context_lens and contexts of at most `chunks` chunks of 256.
+extern "C" int tm_attn_prefill_decodes(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
+                                       const int* block_tables, int table_width, const int* tiles, int n_tiles, const void* qd, void* outd, const int* tables,
+                                       const int* context_lens, int chunks, int n, int H, int KVH, int D, int page, float scale, int window, int keep,
+                                       float softcap, const float* sink, const void* cgate, const void* cgated, int ldcg, hipStream_t stream) {
+    TmAhead none;
+    TmDecodes decodes{qd, outd, tables, context_lens, cgated, n, chunks, 0.f};
+    return attn_prefill_ahead(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, tiles, n_tiles, H, KVH, D, page, scale, window, keep,
+                              softcap, sink, cgate, ldcg, none, stream, &decodes);
 }

@@ -105,6 +105,16 @@ inline bool tm_decode_whole(int requests, int heads, int kv_heads, int head_size
     return max_context <= (head_size <= 32 ? 768 : head_size <= 64 ? 576 : 400);
 }
 
+// Do a mixed step's prompt portions, of n_tiles tiles, have its decoded tokens beside them in one launch (attn_prefill_mfma_kernel with DECODES)?
+// The whole kernel's rule does not hold here: what its blocks take longer than the split kernels' they take beside the portions'. Of two blocks a CU the
+// registers hold one, so as many pairs as CUs are the most; contexts end where a block's eight wavefronts have three rounds of keys (16 of 1,500 keys
+// beside 1 portion of 100 tokens, the least there is to gain: 12.8 to 13.0 us; beside 2 of 256 14.3 to 13.0).
+constexpr int TM_DECODE_BESIDE_LDS = 139264, TM_DECODE_BESIDE_KEYS = 1536;
+inline bool tm_prefill_takes_decodes(int requests, int heads, int kv_heads, int head_size, int max_context) {
+    return requests > 0 && head_size <= 64 && max_context <= TM_DECODE_BESIDE_KEYS && requests * kv_heads <= 256 &&
+           tm_decode_whole_lds(tm_decode_chunks(max_context), heads / kv_heads, head_size) <= TM_DECODE_BESIDE_LDS;
+}
+
 // --- prefill attention (bfloat16) ---------------------------------------------------------------------
 // Two kernels: one whose wavefronts each load their own key blocks and split a tile's keys among them (many
 // short chains: best for short prompts and for small head sizes), and one that stages a tile's keys and values

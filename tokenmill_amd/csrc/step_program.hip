@@ -642,9 +642,13 @@ struct Run {
                                                     s->n_tiles, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep, a.softcap, a.sink, cg, cgate_ld, stream);
                 } else {
                     ++p->taken[TM_PREFILL_SPLIT_KEYS];
+                    TmDecodes decodes{(const char*)q + (size_t)tp * q_stride * es, (char*)attn + (size_t)tp * HD * es, tables + (size_t)(S - nd) * W,
+                                      s->context_lens + (S - nd), cg_dec, nd, tm_decode_chunks(s->max_decode_context), 0.f};
+                    const bool both = nd && a.H / a.KVH <= 16 && tm_prefill_takes_decodes(nd, a.H, a.KVH, a.D, s->max_decode_context);
                     rc = attn_prefill_ahead(q, q_stride, attn, HD, a.k_pool, a.v_pool, tables, W, s->prefill_tiles, s->n_tiles, a.H, a.KVH, a.D, a.page,
-                                            a.scale, a.window, a.keep, a.softcap, a.sink, cg, cgate_ld, matrices, stream);
+                                            a.scale, a.window, a.keep, a.softcap, a.sink, cg, cgate_ld, matrices, stream, both ? &decodes : nullptr);
                     if (matrices.n) gone = true;
+                    done_decode = both;
                 }
                 done_prefill = true;
             } else if (tp && s->n_tiles > 0 && s->prefill_tiles && dtype == TM_F32 && a.D % 16 == 0 && a.D >= 16 &&
@@ -656,7 +660,7 @@ struct Run {
             if (rc) return rc;
             const char* q_dec = (const char*)q + (size_t)tp * q_stride * es;
             char* out_dec = (char*)attn + (size_t)tp * HD * es;
-            if (nd && dtype == TM_BF16 && head_mfma && page_ok && a.H / a.KVH <= 16 && q_ok) {
+            if (nd && !done_decode && dtype == TM_BF16 && head_mfma && page_ok && a.H / a.KVH <= 16 && q_ok) {
                 const bool split = decode_in_chunks(p, a, nd, s->max_decode_context);
                 if (gone) matrices.n = 0;       // (the prompt portions' attention had room for them)
                 else if (tp) matrices = after_norm ? ahead(op, AHEAD_OF_ATTENTION) : ahead_behind_norm(op, AHEAD_OF_ATTENTION);
@@ -670,7 +674,7 @@ struct Run {
                                            tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page, a.scale, a.window, a.keep,
                                            a.softcap, a.sink, cg_dec, cgate_ld, matrices, stream);
                 done_decode = true;
-            } else if (nd && dtype == TM_F32 && decode_in_chunks(p, a, nd, s->max_decode_context) &&
+            } else if (nd && !done_decode && dtype == TM_F32 && decode_in_chunks(p, a, nd, s->max_decode_context) &&
                        tm_attn_decode_f32_takes(q_dec, q_stride, a.k_pool, a.v_pool, a.H, a.KVH, a.D, a.page)) {
                 rc = tm_attn_decode_f32((const float*)q_dec, q_stride, (float*)out_dec, HD, (const float*)a.k_pool, (const float*)a.v_pool,
                                         tables + (size_t)(S - nd) * W, W, s->context_lens + (S - nd), part_o, part_ml,
