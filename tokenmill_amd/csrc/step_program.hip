@@ -438,8 +438,9 @@ struct Run {
     // The same in steps of more tokens, whose products run behind a norm of their own, each matrix as the kernel that will take it reads it. There is more
     // to gain: 896 -> 2 x 4,864 at 64 / 77 / 512 rows takes 8.6 / 8.7 / 16.9 us from cold, 5.8 / 5.6 / 13.5 out of the caches, 4,864 -> 896 6.7 / 6.2 / 12.9 and
     // 4.7 / 4.8 / 8.9. Beyond 64 tokens q|k|v's tiles leave CUs idle and bring o and gate|up, the attention down and the next q|k|v, or all of it
-    // where q|k|v has no room; beside decoding requests q|k|v brings only in steps of up to 320 tokens, since their attention would put out
-    // more than it is late (130 / 304 / 490 / 512 tokens 1,341 / 1,450 / 1,822 / 1,778 us to 1,264 / 1,416 / 1,859 / 1,813). Up to 64 tokens everything in front of the
+    // where q|k|v has no room; beside decoding requests whose attention is a launch of its own q|k|v brings only in steps of up to 320 tokens, since that
+    // would put out more than it is late (130 / 304 / 490 / 512 tokens 1,341 / 1,450 / 1,822 / 1,778 us to 1,264 / 1,416 / 1,859 / 1,813; where they are attended
+    // in the portions' launch 512 / 530 / 780 tokens 1,674 / 1,845 / 2,201 to 1,631 / 1,808 / 2,128). Up to 64 tokens everything in front of the
     // products is short: o and down beside the attention, with the one-launch decode attention gate|up too (32 requests of 1,000 keys, split, 1,012
     // without, 1,000 so, 1,031 with gate|up; 64 and 40 requests, whole, 1,272 and 995, 1,261 and 979, 1,243 and 960); q|k|v's panel and the norms,
     // 3 to 5 us long, were slower by what they brought. Steps of the 0.5B shape, us, without to so: prompts of 30 / 77 / 150 / 300 / 600 tokens 896 / 1,054 /
@@ -483,6 +484,11 @@ struct Run {
             if (const TmTilePieces t = pieces(1, L.N, L.K); t.parts) h.row_major(L.w, L.N, L.K, t.rows, 1, t.steps, false);
         }
     }
+    // Are a mixed step's decoded tokens attended in the launch of its portions (where that is the kernel that splits keys)?
+    bool beside_portions(const TmAttentionOp& a) const {
+        return s->num_decode > 0 && s->num_decode < s->T && a.H / a.KVH <= 16 &&
+               tm_prefill_takes_decodes(s->num_decode, a.H, a.KVH, a.D, s->max_decode_context);
+    }
     TmAhead ahead_behind_norm(int op, int host) const {
         constexpr size_t MOST = 32u << 20;
         constexpr int MIXED_ROWS = 320;
@@ -495,7 +501,7 @@ struct Run {
         if (bytes(a.o) + bytes(f.gate_up) + bytes(f.down) + (next ? bytes(next->qkv) : 0) > MOST) return h;
         const bool few = s->T <= TM_STREAM_ROWS;
         if (host == AHEAD_OF_QKV) {
-            if (s->num_decode > 0 && s->T > MIXED_ROWS) return h;
+            if (s->num_decode > 0 && s->T > MIXED_ROWS && !beside_portions(a)) return h;
             h.blocks = 120;
             bring_projection(h, a.o);
             bring_gate_up(h, f);
@@ -644,7 +650,7 @@ struct Run {
                     ++p->taken[TM_PREFILL_SPLIT_KEYS];
                     TmDecodes decodes{(const char*)q + (size_t)tp * q_stride * es, (char*)attn + (size_t)tp * HD * es, tables + (size_t)(S - nd) * W,
                                       s->context_lens + (S - nd), cg_dec, nd, tm_decode_chunks(s->max_decode_context), 0.f};
-                    const bool both = nd && a.H / a.KVH <= 16 && tm_prefill_takes_decodes(nd, a.H, a.KVH, a.D, s->max_decode_context);
+                    const bool both = beside_portions(a);
                     rc = attn_prefill_ahead(q, q_stride, attn, HD, a.k_pool, a.v_pool, tables, W, s->prefill_tiles, s->n_tiles, a.H, a.KVH, a.D, a.page,
                                             a.scale, a.window, a.keep, a.softcap, a.sink, cg, cgate_ld, matrices, stream, both ? &decodes : nullptr);
                     if (matrices.n) gone = true;
