@@ -66,6 +66,10 @@ int tm_tile_experts(int kind, const void* A, int lda, const int* row_src, int sr
                     const int* n_tiles, int max_tiles, int tile_rows, int K, int F, const float* pair_weight, float limit, float alpha,
                     hipStream_t stream);
 
+// A wide product of at most 16 bfloat16 rows into 32-bit results (gemv_bf16.hip): K a multiple of 32, N of 4 and at least 16,384, 16-byte pieces.
+int tm_gemv_bf16_takes(const void* A, int lda, const void* W, const void* C, int ldc, int M, int N, int K);
+int tm_gemv_bf16(const void* A, int lda, const void* W, float* C, int ldc, int M, int N, int K, hipStream_t stream);
+
 // The true 32-bit path's products of at most 16 rows on the 32-bit matrix unit (gemv_f32.hip): K a multiple of 16, N of 4, 16-byte
 // pieces (tm_gemv_f32_mfma_takes). A plain product; 32-bit partial sums [parts][M][N] (tm_gemv_f32_parts says how many);
 // silu(gate) * up; q|k|v with bias, rotation over the whole head (head sizes that are multiples of 32) and cache write.

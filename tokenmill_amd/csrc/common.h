@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define TM_WAVE 64
 
 // dtype codes of the C interface
@@ -133,6 +135,35 @@ __device__ __forceinline__ float lane_max(float v) {
     float a, b;
     lane_pair<OFF>(v, a, b);
     return fmaxf(a, b);
+}
+
+// Rows as the 16-row matrix instructions want them: lane (r, g) = (lane % 16, lane / 16) holds 16 bytes of row r at place g, so a load of an
+// operand takes 64 bytes of each of sixteen rows, and a CU takes a line in at the same cost whole or half. Two operands that are the two halves of 128
+// bytes are loaded as a pair instead, lo: 16 bytes of row r % 8 at place g of its half r / 8, hi: the same of row 8 + r % 8; this is half 0 or 1 of
+// them for row r. V: four 32-bit values. Every lane is active.
+template <typename V>
+__device__ __forceinline__ V line_pair_half(int half, V lo, V hi) {
+    V o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const auto l = lo[e], h = hi[e];
+        // (row_ror:8, written to the upper or the lower eight lanes of each sixteen)
+        const int v = half ? __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, h), __builtin_bit_cast(int, l), 0x128, 0xf, 0x3, false)
+                           : __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, l), __builtin_bit_cast(int, h), 0x128, 0xf, 0xc, false);
+        o[e] = __builtin_bit_cast(std::remove_const_t<decltype(l)>, v);
+    }
+    return o;
+}
+// half 1 of rows r < 8, where nobody looks at the others
+template <typename V>
+__device__ __forceinline__ V line_pair_turned(V lo) {
+    V o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const auto l = lo[e];
+        o[e] = __builtin_bit_cast(std::remove_const_t<decltype(l)>, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, l), 0x128, 0xf, 0xf, false));
+    }
+    return o;
 }
 
 __device__ __forceinline__ float wave_sum(float v) {

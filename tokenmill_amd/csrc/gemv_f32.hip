@@ -44,24 +44,6 @@ struct GemvArgs {
     float* v_pool;              // [pages, KVH, D, page]
 };
 
-// A pair of steps as it is loaded (lane (r, g): row r % 8, or 8 + r % 8, step r / 8 of the two) to the matrix instruction's
-// layout (row r): the lanes of the other half of a row of sixteen hold what is missing.
-__device__ __forceinline__ f32x4_t turned(f32x4_t v) {
-    f32x4_t o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[e]), 0x128, 0xf, 0xf, false));
-    return o;
-}
-__device__ __forceinline__ f32x4_t fragment(int step, f32x4_t lo, f32x4_t hi) {
-    f32x4_t o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int l = __float_as_int(lo[e]), h = __float_as_int(hi[e]);
-        o[e] = __int_as_float(step ? __builtin_amdgcn_update_dpp(h, l, 0x128, 0xf, 0x3, false) : __builtin_amdgcn_update_dpp(l, h, 0x128, 0xf, 0xc, false));
-    }
-    return o;
-}
-
 // GROUP: steps of 16 k whose products meet in sums of their own before they join the running one. AHEAD: groups a wavefront asks for
 // at once: with one, a wavefront of the 0.5B shape waited for memory two times in a launch of 6 to 7 us (o 6.2 to 5.8, q|k|v 7.2 to 6.8).
 // OVER8: more than eight rows of activations.
@@ -162,10 +144,10 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
 #pragma unroll
             for (int i = j * GROUP; i < (j + 1) * GROUP; ++i) {
                 if (s + i >= s1) break;
-                const f32x4_t xf = OVER8 ? fragment(i % 2, x[i / 2][0], x[i / 2][OVER8 ? 1 : 0]) : i % 2 ? turned(x[i / 2][0]) : x[i / 2][0];
+                const f32x4_t xf = OVER8 ? line_pair_half(i % 2, x[i / 2][0], x[i / 2][OVER8 ? 1 : 0]) : i % 2 ? line_pair_turned(x[i / 2][0]) : x[i / 2][0];
                 f32x4_t wf[RT];
 #pragma unroll
-                for (int t = 0; t < RT; ++t) wf[t] = fragment(i % 2, w[t][i / 2][0], w[t][i / 2][1]);
+                for (int t = 0; t < RT; ++t) wf[t] = line_pair_half(i % 2, w[t][i / 2][0], w[t][i / 2][1]);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
