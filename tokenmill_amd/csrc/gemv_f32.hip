@@ -5,7 +5,7 @@
 // Such a product is bound by reading its matrix once (35 MB for gate|up of the 0.5B shape) and, where that is small, by the trips to
 // memory. A block takes RT tiles of 16 matrix rows (SiLU and q|k|v: one, of 8 rows and the 8 that meet them, twice the blocks);
 // its wavefronts split K into runs of steps of 16 k and ask for several steps of matrix and activations at once, so nothing goes through
-// LDS but the wavefronts' sums at the end, added in halves. The activations come from the second-level cache. Which k goes where
+// LDS but the wavefronts' sums at the end, added in wavefront order. The activations come from the second-level cache. Which k goes where
 // depends on the matrix alone: a row's result does not depend on the other rows.
 //
 // The matrix instruction wants 16 bytes of row r at 4 g in lane (r, g), 64 bytes of each of sixteen rows. A CU takes such loads in at half
@@ -13,9 +13,9 @@
 // as a pair, 128 bytes of eight rows an instruction, and the lanes r and r + 8 exchange what belongs to the other, which is eight
 // instructions of the vector unit a pair. Up to eight rows of activations are one load a pair, and whole lines that
 // nobody reads again pass the caches by (non-temporal: the head 98 to 85 us, down 6.7 to 6.5). Against a load a step, cold matrices,
-// 1 / 8 / 16 rows, us: gate|up of the 0.5B shape 10.9 / 12.3 / 14.4 to 9.0 / 10.2 / 12.2, down 6.4 / 7.2 / 8.6 to 5.7 / 6.5 / 7.8, o
-// 4.7 / 5.5 / 6.5 to 4.4 / 4.9 / 5.8, q|k|v 5.3 / 6.2 / 7.2 to 5.1 / 5.7 / 6.5, the head 119 / 129 / 140 to 81 / 85 / 98 (6.4 TB/s at
-// 8 rows); 3,584 -> 2 x 18,944 103 / 128 / - to 85 / 101 / -.
+// 1 / 8 / 16 rows, us: gate|up of the 0.5B shape 10.9 / 12.2 / 14.4 to 9.1 / 10.1 / 12.2, down 6.4 / 7.2 / 8.6 to 5.7 / 6.4 / 7.8, o
+// 4.7 / 5.5 / 6.4 to 4.5 / 5.3 / 6.2, q|k|v 5.4 / 6.2 / 7.2 to 5.3 / 6.0 / 7.0 (seven steps a wavefront: every other pair lies across two lines),
+// the head 120 / 129 / 141 to 84 / 86 / 99 (6.3 TB/s at 8 rows); 3,584 -> 2 x 18,944 103 / 128 / 159 to 85 / 101 / 127. The same bits.
 // Before that, a wavefront had 256 k of four rows, a lane 4 k each, and summed over the lanes by shuffles, 6 x 32 of them a wavefront:
 // 19.0 us a product of the 0.5B shape on average, with SiLU*up and rotation in kernels behind it.
 #include "common.h"
@@ -73,9 +73,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     const int steps = a.K / 16;
     const int per_block = (steps + gridDim.y - 1) / gridDim.y;
     const int b0 = blockIdx.y * per_block, b1 = b0 + per_block < steps ? b0 + per_block : steps;
-    // (Whole pairs: whole lines. With the wavefronts' sums added in halves the results are as near to 64 bits as with equal runs added in a
-    // row, rms 896 -> 896 1.014 to 0.993e-7, 4,864 -> 896 1.187 to 1.145e-7, 18,944 -> 3,584 1.518 to 1.488e-7.)
-    const int per = (per_block + 2 * WAVES - 1) / (2 * WAVES) * 2;
+    const int per = (per_block + WAVES - 1) / WAVES;
     const int s0 = b0 + wave * per, s1 = s0 + per < b1 ? s0 + per : b1;
     // rows r % 8 and 8 + r % 8 (rows beyond the matrix, the half or the input: its last one, never stored)
     const int r8 = r % 8, second = r / 8;
@@ -172,14 +170,10 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     // lane (r, g): row r of A, rows 4 g .. + 3 of the tile
     if (EPI == GM_PLAIN ? wave >= RT : wave > 0 || g >= 2) return;
     auto total = [&](int t, int of) {
-        f32x4_t v[WAVES];
+        f32x4_t v = red[0][t][of];
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) v[w] = red[w][t][of];
-#pragma unroll
-        for (int n = WAVES / 2; n > 0; n /= 2)
-#pragma unroll
-            for (int w = 0; w < n; ++w) v[w] += v[w + n];
-        return v[0];
+        for (int w = 1; w < WAVES; ++w) v += red[w][t][of];
+        return v;
     };
     if constexpr (EPI == GM_PLAIN) {
         const int n = n0[0] + 16 * wave + 4 * g;
@@ -252,7 +246,7 @@ extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, con
 // asks for two groups where it has them: a group at a time leaves half a pair's line, and gate|up of the 0.5B shape takes 12.2 us so for 10.2.
 template <int EPI, int RT, bool OVER8>
 static void gm_launch_rows(const GemvArgs& a, int units, int split, hipStream_t stream) {
-    const int steps = (a.K / 16 + split - 1) / split, per = (steps + 15) / 16 * 2;
+    const int steps = (a.K / 16 + split - 1) / split, per = (steps + 7) / 8;
     const dim3 grid(units, split);
     if (units * split > 256) {
         if (steps <= 4 * 7) gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1, OVER8><<<grid, 256, 0, stream>>>(a);
