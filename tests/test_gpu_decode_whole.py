@@ -59,3 +59,61 @@ def test_more_than_the_lds_holds_is_refused():
     q, k, v, tables, ctx, _ = _case(16, 1, 128, 16, [1300], 3)
     with pytest.raises(Exception):
         ops.attn_decode_mfma(q, torch.empty_like(q), k, v, tables, ctx, 16, 1, 128, 0.1, 0, 1300, whole=True)
+
+
+@pytest.mark.parametrize("H,KVH,D", [(14, 2, 64), (8, 8, 32), (28, 4, 128), (16, 1, 64), (6, 2, 96), (16, 1, 128)])
+@pytest.mark.parametrize("window,keep,softcap,options", [(0, 0, 0.0, False), (300, 70, 0.0, True), (0, 0, 20.0, False)])
+def test_among_many_a_request_has_its_bits_whatever_the_lengths_beside_it(H, KVH, D, window, keep, softcap, options):
+    """192 (request, kv head) pairs and more: by the kernel's rule one launch where all contexts are short, another beside a longer one."""
+    from tokenmill_amd.hip import ops
+    S = -(-192 // KVH) + 1
+    edges = [1, 64, 65, 255, 256, 257, 512, 700, 768, 769, 1023, 1024, 1025, 1279, 1280, 1281, 1600]
+    lens = [edges[i % len(edges)] for i in range(S - 1)] + [3000]
+    q, k, v, tables, ctx, g = _case(H, KVH, D, 16, lens, 5)
+    sink = torch.randn(H, generator=g).to(DEV) if options else None
+    gate = torch.randn(S, H * D, generator=g).bfloat16().to(DEV) if options else None
+
+    def run(longest):
+        """The requests of at most so many keys, the others at one key; the rule's kernel for the longest."""
+        cut = torch.where(ctx > longest, 1, ctx)
+        out = torch.full((S, H * D), 3.0, dtype=torch.bfloat16, device=DEV)
+        ops.attn_decode_mfma(q, out, k, v, tables, cut, H, KVH, D, D ** -0.5, window, longest, softcap=softcap, sink=sink, keep=keep, channel_gate=gate)
+        assert torch.isfinite(out.float()).all()
+        return out
+
+    most = run(3000)
+    for longest in (256, 512, 768, 1024, 1280, 1600):
+        same = (ctx <= longest)
+        assert torch.equal(run(longest)[same], most[same]), longest
+    few = ops.attn_decode_mfma(q[:S - 1], torch.empty_like(q[:S - 1]), k, v, tables[:S - 1], ctx[:S - 1], H, KVH, D, D ** -0.5, window, 1600, softcap=softcap,
+                               sink=sink, keep=keep, channel_gate=gate[:S - 1] if options else None)
+    assert torch.equal(few, most[:S - 1])
+
+
+@pytest.mark.parametrize("portions", [[], [40], [150, 90]])
+def test_a_step_of_many_requests_beside_a_longer_one(portions):
+    """The same through whole steps: 200 pairs, alone and beside prompt portions (whose launch attends them where contexts are short)."""
+    from conftest import qwen2_config
+    from tokenmill_amd import EngineConfig, LLMEngine
+    from tokenmill_amd.config.registry import architecture_name, get_architecture
+    from tokenmill_amd.engine.runner import StepEntry
+    shape = qwen2_config(num_hidden_layers=2, hidden_size=256, num_attention_heads=4, num_key_value_heads=2, intermediate_size=512, vocab_size=512,
+                         rope_theta=10000.0, rms_norm_eps=1e-6, tie_word_embeddings=True)
+    arch = get_architecture(architecture_name(shape))
+    model = arch.build_model(arch.config_from_dict(shape, None), None)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    model.load({name: (torch.randn(spec.drawn_shape(), generator=g, device="cuda") * 0.25).bfloat16() for name, spec in sorted(model.tensor_specs().items())},
+               torch.bfloat16, torch.device(DEV))
+    contexts = [(37 * i) % 1200 + 1 for i in range(99)]
+    got = []
+    for longest in (1000, 1400, 3000):
+        requests = [(0, n) for n in portions] + [(c - 1, 1) for c in contexts + [longest]]
+        engine = LLMEngine(EngineConfig(dtype="bfloat16", block_size=16, num_blocks=sum(-(-(a + b) // 16) for a, b in requests) + 4, watermark=0.0,
+                                        max_model_len=3100, max_num_seqs=128, max_num_batched_tokens=8192, hip_graphs=False), model=model)
+        caches = [engine.cache.allocate(f"r{i}", a + b) for i, (a, b) in enumerate(requests)]
+        ids = [torch.randint(0, 512, (a + b,), generator=torch.Generator().manual_seed(a + b)).tolist() for a, b in requests]
+        for cache, prompt, (a, _) in zip(caches, ids, requests):
+            if a:
+                engine.runner.step([StepEntry(cache, 0, prompt[:a], [a - 1])])
+        got.append(engine.runner.step([StepEntry(cache, a, prompt[a:], [b - 1]) for cache, prompt, (a, b) in zip(caches, ids, requests)])[:-1].clone())
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])

@@ -9,7 +9,7 @@
 //   block kernel : one block of 8 (16 for head size 32) wavefronts per (request, kv head); wavefront
 //                  w takes keys [64 (i W + w), +64) for i = 0, 1, ...; the partials are merged
 //                  through LDS in wavefront order. One launch, no scratch memory: the way for large
-//                  batches.
+//                  batches. Contexts of a few chunks (tm_decode_own_keys) a block takes as the whole kernel does.
 //   split kernels: with few requests more blocks than (request, kv head) pairs are needed to pull
 //                  the cache at speed: blocks of four wavefronts take chunks of 256 positions and
 //                  write partials to scratch memory; a second kernel adds the partials of a request
@@ -18,8 +18,9 @@
 //                  additions, in one block per (request, kv head).
 //
 //   Which keys meet in which partial and in which order partials are added depends on positions
-//   only, so within either way what a request gets does not depend on which other requests are in
-//   the batch (which way runs depends on how many there are: the two differ by rounding).
+//   only, and the split and the whole kernels have the same bits, so what a request gets does not depend on which other
+//   requests are in the batch. It depends on how many there are: from 192 (request, kv head) pairs on, a context beyond
+//   tm_decode_own_keys gets the block kernel's order (the two differ by rounding).
 //
 //   Operand layouts need no LDS: keys K[page][slot][kvh][d] give the A operand of S^T = K Q^T
 //   (16 keys x 32 d per instruction), values V[page][kvh][d][slot] give the A operand of
@@ -51,14 +52,18 @@ template <int D, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void attn_decode_block_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
-    int table_width, const int* __restrict__ context_lens, int H, int KVH, int page_shift, float scale_log2, float cap_in, float cap_out,
-    int window, int keep, const float* __restrict__ sink, const bf16_t* __restrict__ cgate, int ldcg) {
+    int table_width, const int* __restrict__ context_lens, int whole_chunks, int H, int KVH, int page_shift, float scale_log2, float cap_in,
+    float cap_out, int window, int keep, const float* __restrict__ sink, const bf16_t* __restrict__ cgate, int ldcg) {
     constexpr int NDT = D / 16;
-    __shared__ float s_m[WAVES][16], s_l[WAVES][16];
-    __shared__ float s_o[WAVES][16][16 + 1];                         // one 16-wide d tile at a time
+    extern __shared__ __align__(16) float s_block[];
     const int s = blockIdx.x, kvh = blockIdx.y;
     const int G = H / KVH;
     const int ctx = context_lens[s];
+    if (ctx <= whole_chunks * AD_CHUNK)                              // block-uniform
+        return attend_whole<D, WAVES>(s_block, s, kvh, q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, whole_chunks,
+                                      H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
+    float(*s_m)[16] = (float(*)[16])s_block, (*s_l)[16] = s_m + WAVES;
+    float(*s_o)[16][16 + 1] = (float(*)[16][16 + 1])(s_l + WAVES);   // one 16-wide d tile at a time
     const int p = ctx - 1;
     const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
     const int wave = threadIdx.x / TM_WAVE, lane = threadIdx.x % TM_WAVE;
@@ -437,9 +442,14 @@ static int launch_decode(const void* q, int q_stride, void* out, int out_stride,
     // asks for that by bringing the scratch memory
     const bool split = part_o && part_ml && max_chunks > 1;
     if (!split) {
-        attn_decode_block_kernel<D, WAVES><<<dim3(S, KVH), 64 * WAVES, 0, stream>>>(
+        const int own = tm_decode_own_keys(H / KVH, D) / AD_CHUNK, whole_chunks = own < max_chunks ? own : max_chunks;
+        const size_t block = (size_t)WAVES * 16 * (2 + 17) * sizeof(float), whole = tm_decode_whole_lds(whole_chunks, H / KVH, D);
+        static const hipError_t allowed = hipFuncSetAttribute((const void*)attn_decode_block_kernel<D, WAVES>,
+                                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)TM_DECODE_WHOLE_LDS);
+        if (allowed != hipSuccess) return TM_ERR_LAUNCH;
+        attn_decode_block_kernel<D, WAVES><<<dim3(S, KVH), 64 * WAVES, block > whole ? block : whole, stream>>>(
             (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool,
-            block_tables, table_width, context_lens, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink,
+            block_tables, table_width, context_lens, whole_chunks, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink,
             cgate, ldcg);
         TM_CHECK_LAUNCH();
         return TM_OK;

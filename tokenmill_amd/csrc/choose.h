@@ -97,10 +97,19 @@ constexpr int TM_DECODE_WHOLE_KEYS = 1280;
 constexpr size_t TM_DECODE_WHOLE_LDS = 160 * 1024;
 // its LDS: of the four runs of every chunk the maximum and sum of 16 heads and the values of the heads there are, and the former of every chunk
 inline size_t tm_decode_whole_lds(int chunks, int group, int head_size) { return (size_t)chunks * (32 + 4 * (32 + group * (head_size + 4))) * 4; }
+
+// From TM_DECODE_SPLIT_PAIRS pairs on: keys up to which a request is attended in the whole kernel's order, whatever the contexts beside it are (the
+// block kernel does so too, and takes longer contexts its own way), so that no request's bits hang on its neighbours' lengths, nor a replayed
+// step's on the engine's longest. As many chunks as leave the block kernel the blocks a CU that its registers do: two at head size 64, else one.
+inline int tm_decode_own_keys(int group, int head_size) {
+    const size_t room = head_size == 64 ? TM_DECODE_WHOLE_LDS / 2 : TM_DECODE_WHOLE_LDS;
+    const int keys = (int)(room / tm_decode_whole_lds(1, group, head_size)) * TM_DECODE_CHUNK;
+    return keys < TM_DECODE_WHOLE_KEYS ? keys : TM_DECODE_WHOLE_KEYS;
+}
 inline bool tm_decode_whole(int requests, int heads, int kv_heads, int head_size, int max_context) {
     const int pairs = requests * kv_heads;
+    if (pairs >= TM_DECODE_SPLIT_PAIRS) return max_context <= tm_decode_own_keys(heads / kv_heads, head_size);
     if (tm_decode_whole_lds(tm_decode_chunks(max_context), heads / kv_heads, head_size) > TM_DECODE_WHOLE_LDS) return false;
-    if (pairs >= TM_DECODE_SPLIT_PAIRS) return max_context <= TM_DECODE_WHOLE_KEYS;
     if (pairs >= TM_DECODE_MANY_PAIRS) return max_context <= (head_size <= 64 ? TM_DECODE_WHOLE_KEYS : 768);
     return max_context <= (head_size <= 32 ? 768 : head_size <= 64 ? 576 : 400);
 }
@@ -108,10 +117,12 @@ inline bool tm_decode_whole(int requests, int heads, int kv_heads, int head_size
 // Do a mixed step's prompt portions, of n_tiles tiles, have its decoded tokens beside them in one launch (attn_prefill_mfma_kernel with DECODES)?
 // The whole kernel's rule does not hold here: what its blocks take longer than the split kernels' they take beside the portions'. Of two blocks a CU the
 // registers hold one, so as many pairs as CUs are the most; contexts end where a block's eight wavefronts have three rounds of keys (16 of 1,500 keys
-// beside 1 portion of 100 tokens, the least there is to gain: 12.8 to 13.0 us; beside 2 of 256 14.3 to 13.0).
+// beside 1 portion of 100 tokens, the least there is to gain: 12.8 to 13.0 us; beside 2 of 256 14.3 to 13.0); where the pairs are so many that longer
+// ones are added up in another order, they end there.
 constexpr int TM_DECODE_BESIDE_LDS = 139264, TM_DECODE_BESIDE_KEYS = 1536;
 inline bool tm_prefill_takes_decodes(int requests, int heads, int kv_heads, int head_size, int max_context) {
     return requests > 0 && head_size <= 64 && max_context <= TM_DECODE_BESIDE_KEYS && requests * kv_heads <= 256 &&
+           (requests * kv_heads < TM_DECODE_SPLIT_PAIRS || max_context <= tm_decode_own_keys(heads / kv_heads, head_size)) &&
            tm_decode_whole_lds(tm_decode_chunks(max_context), heads / kv_heads, head_size) <= TM_DECODE_BESIDE_LDS;
 }
 
