@@ -97,13 +97,13 @@ def test_a_step_of_many_requests_beside_a_longer_one(portions):
     from tokenmill_amd import EngineConfig, LLMEngine
     from tokenmill_amd.config.registry import architecture_name, get_architecture
     from tokenmill_amd.engine.runner import StepEntry
-    shape = qwen2_config(num_hidden_layers=2, hidden_size=256, num_attention_heads=4, num_key_value_heads=2, intermediate_size=512, vocab_size=512,
+    shape = qwen2_config(num_hidden_layers=4, hidden_size=512, num_attention_heads=8, num_key_value_heads=2, intermediate_size=512, vocab_size=512,
                          rope_theta=10000.0, rms_norm_eps=1e-6, tie_word_embeddings=True)
     arch = get_architecture(architecture_name(shape))
     model = arch.build_model(arch.config_from_dict(shape, None), None)
     g = torch.Generator(device="cuda").manual_seed(1)
-    model.load({name: (torch.randn(spec.drawn_shape(), generator=g, device="cuda") * 0.25).bfloat16() for name, spec in sorted(model.tensor_specs().items())},
-               torch.bfloat16, torch.device(DEV))
+    model.load({name: (torch.randn(spec.drawn_shape(), generator=g, device="cuda") * 0.1 + (spec.init == "ones")).bfloat16()
+                for name, spec in sorted(model.tensor_specs().items())}, torch.bfloat16, torch.device(DEV))
     contexts = [(37 * i) % 1200 + 1 for i in range(99)]
     got = []
     for longest in (1000, 1400, 3000):
