@@ -93,3 +93,64 @@ def test_a_step_has_the_bits_of_its_operations_one_by_one(width, heads, kv_heads
     for op in range(native.first, native.first + native.count):
         program.run_ops(op, 1, step, flow)
     assert torch.equal(flow.logits, want)
+
+
+def _brought(width, heads, kv_heads, head_dim, inside, contexts, portions, graphs=False):
+    """What a step of three layers is given to bring, and which kernels it takes (counters of the step program)."""
+    from conftest import qwen2_config
+    from tokenmill_amd import EngineConfig, LLMEngine
+    from tokenmill_amd.config.registry import architecture_name, get_architecture
+    from tokenmill_amd.engine.runner import StepEntry
+    shape = qwen2_config(num_hidden_layers=3, hidden_size=width, num_attention_heads=heads, num_key_value_heads=kv_heads, head_dim=head_dim,
+                         intermediate_size=inside, vocab_size=16384, rope_theta=10000.0, rms_norm_eps=1e-6, tie_word_embeddings=True)
+    arch = get_architecture(architecture_name(shape))
+    model = arch.build_model(arch.config_from_dict(shape, None), None)
+    model.load({name: torch.full(spec.drawn_shape(), 0.01, dtype=torch.bfloat16, device="cuda") for name, spec in model.tensor_specs().items()},
+               torch.bfloat16, torch.device("cuda:0"))
+    requests = [(0, n) for n in portions] + [(c - 1, 1) for c in contexts]
+    engine = LLMEngine(EngineConfig(dtype="bfloat16", block_size=16, num_blocks=sum(-(-(a + b) // 16) for a, b in requests) + 4, watermark=0.0,
+                                    max_model_len=2200, max_num_seqs=128, max_num_batched_tokens=4096, hip_graphs=graphs), model=model)
+    entries = [StepEntry(engine.cache.allocate(f"r{i}", a + b), a, [1] * b, [b - 1]) for i, (a, b) in enumerate(requests)]
+    program = engine.runner.program
+    before = program.brought(), program.counters()
+    for _ in range(3 if graphs else 1):
+        engine.runner.step(entries)
+    after = program.brought(), program.counters()
+    return [{k: n - b[k] for k, n in a.items() if n != b[k]} for a, b in zip(after, before)]
+
+
+SMALL, LARGE = (896, 14, 2, 64, 4864), (1536, 12, 2, 128, 8960)
+NORM = {"qkv_from_norm": 3, "gate_up_from_norm": 3, "head_few": 1}
+TILED = {"qkv_plain": 3, "qkv_tiled": 3, "gate_up_plain": 3, "gate_up_tiled": 3, "project_tiled": 6, "head_few": 1}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,contexts,portions,brought,kernels", [
+    # q|k|v: half of gate|up; attention: o and the rest; gate|up: down and the next q|k|v
+    (SMALL, [300], [], {"qkv": 3, "attention": 6, "gate_up": 5}, {**NORM, "decode_whole": 3}),
+    (SMALL, [300] * 8, [], {"qkv": 3, "attention": 6, "gate_up": 5}, {**NORM, "decode_whole": 3}),
+    (SMALL, [2100] * 4, [], {"qkv": 3, "attention": 6, "gate_up": 5}, NORM),
+    (LARGE, [300], [], {}, {**NORM, "decode_whole": 3}),
+    # attention: o and down; gate|up too where it is one launch
+    (SMALL, [90] * 12, [], {"attention": 9}, {"qkv_panel": 3, "gate_up_stream": 3, "head_few": 1, "decode_whole": 3}),
+    (SMALL, [50] * 33, [], {"attention": 9, "row_major": 9}, {"qkv_panel": 3, "gate_up_plain": 3, "gate_up_tiled": 3, "project_tiled": 6, "decode_whole": 3}),
+    (SMALL, [1500] * 24, [], {"attention": 6, "row_major": 6}, {"qkv_panel": 3, "gate_up_plain": 3, "gate_up_tiled": 3, "project_tiled": 6}),
+    (SMALL, [], [30], {"attention": 6, "row_major": 6},
+     {"qkv_panel": 3, "gate_up_plain": 3, "gate_up_tiled": 3, "project_tiled": 6, "prefill_split_keys": 3, "head_few": 1}),
+    # q|k|v's tiles: o and gate|up; attention: down and the next q|k|v
+    (SMALL, [], [77], {"qkv": 6, "attention": 5, "row_major": 11}, {**TILED, "prefill_split_keys": 3}),
+    (SMALL, [300] * 10, [241, 241], {"qkv": 6, "attention": 5, "row_major": 11}, {**TILED, "prefill_split_keys": 3, "decode_beside": 3}),
+    (SMALL, [1800] * 10, [241, 241], {"attention": 11, "row_major": 11}, {**TILED, "prefill_split_keys": 3}),
+    (LARGE, [], [77], {}, {**TILED, "prefill_split_keys": 3}),
+])
+def test_which_matrices_a_step_brings_and_which_kernels_take_them(shape, contexts, portions, brought, kernels):
+    """Each matrix is brought in the order of the kernel that takes it: row-major ones are the tiled products'."""
+    got, took = _brought(*shape, contexts, portions)
+    assert got == brought and took == kernels
+
+
+@pytest.mark.gpu
+def test_a_captured_step_brings_what_an_eager_one_does():
+    got, took = _brought(*SMALL, [300] * 4, [], graphs=True)
+    runs = took["qkv_from_norm"]                                             # (layers of the runs that a capture makes)
+    assert runs >= 3 and got == {"qkv": runs, "attention": 2 * runs, "gate_up": 5 * runs // 3}

@@ -124,9 +124,22 @@ enum {
     TM_PROJECT_STREAM,          // ... over the packed matrix (gemm_stream.hip)
     TM_PROJECT_FEW_F32,         // ... 32-bit, few rows
     TM_DECODE_F32_SPLIT,        // 32-bit attention of single tokens in chunks (attention_decode_f32.hip)
+    TM_DECODE_WHOLE,            // bfloat16 attention of single tokens: contexts of a few chunks in one block each, in a launch of its own
+    TM_DECODE_BESIDE,           // ... in the launch of the prompt portions
+    TM_HEAD_FEW,                // output heads of few bfloat16 rows (gemv_bf16.hip)
     TM_PROGRAM_COUNTERS
 };
 void tm_program_counters(const TmProgram* p, long long* out);
+
+// matrices that a step's kernels were given to bring ahead (ahead.h), counted per program (TM_BROUGHT_COUNTERS numbers)
+enum {
+    TM_BROUGHT_BY_QKV = 0,
+    TM_BROUGHT_BY_ATTENTION,
+    TM_BROUGHT_BY_GATE_UP,
+    TM_BROUGHT_ROW_MAJOR,       // of all of them, those in the order of a tiled product
+    TM_BROUGHT_COUNTERS
+};
+void tm_program_brought(const TmProgram* p, long long* out);
 
 // The spans of a run that a profile tells apart. While labels are asked for (TM_RUN_LABELS), `hook(user, op,
 // label, 1)` is called on the host before the span's launches and `hook(user, op, label, 0)` after them; op is

@@ -57,7 +57,7 @@ struct TmProgram {
     void* hook_user = nullptr;
     TmTune tune{0, 3, 0};
     // how often each way of computing q|k|v and the activation was taken (for tests and curiosity)
-    mutable long long taken[TM_PROGRAM_COUNTERS] = {};
+    mutable long long taken[TM_PROGRAM_COUNTERS] = {}, brought[TM_BROUGHT_COUNTERS] = {};
 };
 
 namespace {
@@ -130,6 +130,7 @@ struct Products {
     TmTune tune;
     float* wide_in = nullptr;           // room for a product's input and output in 32-bit (see TmProgram::max_wide_in)
     float* wide_out = nullptr;
+    long long* head_few = nullptr;      // counts the heads of few rows
     int skinny_rows = TM_SKINNY_ROWS;   // rows up to which the packed products for at most 16 rows are preferred (tm_skinny_rows)
 
     int library(const TmLinear& L, const void* x, int ldx, int M, void* out, int ldc, int out_dtype) const {
@@ -174,8 +175,10 @@ struct Products {
             return then_act(tm_gemm_nt_tiled(x, ldx, L.w, L.bias, L.bias_dtype, out, ldc, M, L.N, L.K, dtype, out_dtype, stream));
         }
         const bool skinny = skinny_ok(L, x, ldx, dtype);
-        if (L.library_first && !L.bias && !L.act && out_dtype == TM_F32 && tm_gemv_bf16_takes(x, ldx, L.w, out, ldc, M, L.N, L.K))
+        if (L.library_first && !L.bias && !L.act && out_dtype == TM_F32 && tm_gemv_bf16_takes(x, ldx, L.w, out, ldc, M, L.N, L.K)) {
+            if (head_few) ++*head_few;
             return tm_gemv_bf16(x, ldx, L.w, (float*)out, ldc, M, L.N, L.K, stream);
+        }
         if (L.library_first) {
             const int rc = library(L, x, ldx, M, out, ldc, out_dtype);
             if (rc != TM_ERR_UNSUPPORTED) return then_act(rc);
@@ -437,6 +440,11 @@ struct Run {
         return h;
     }
 
+    void count(int by, const TmAhead& h) const {
+        p->brought[by] += h.n;
+        for (int i = 0; i < h.n; ++i) p->brought[TM_BROUGHT_ROW_MAJOR] += h.m[i].row_major;
+    }
+
     // The same in steps of more tokens, whose products run behind a norm of their own, each matrix as the kernel that will take it reads it. There is more
     // to gain: 896 -> 2 x 4,864 at 64 / 77 / 512 rows takes 8.6 / 8.7 / 16.9 us from cold, 5.8 / 5.6 / 13.5 out of the caches, 4,864 -> 896 6.7 / 6.2 / 12.9 and
     // 4.7 / 4.8 / 8.9. Beyond 64 tokens q|k|v's tiles leave CUs idle and bring o and gate|up, the attention down and the next q|k|v, or all of it
@@ -558,9 +566,11 @@ struct Run {
             const bool own_norm = x_in == nullptr;
             // 1. the kernel that starts at the norm (at most 16 tokens)
             if (own_norm && delta == nullptr && !pending_sums && starts_at_norm(a)) {
+                matrices = ahead(op, AHEAD_OF_QKV);
+                count(TM_BROUGHT_BY_QKV, matrices);
                 rc = fused_norm_qkv_rope_ahead(resid, a.norm.w, a.norm.w_dtype, a.norm.eps, T, hidden, a.qkv.packed, a.qkv.bias,
                                                a.qkv.bias_dtype, qkv, a.H, a.KVH, a.D, a.cos_t, a.sin_t, s->positions, slots, kp, vp,
-                                               a.page, ahead(op, AHEAD_OF_QKV), stream);
+                                               a.page, matrices, stream);
                 q = qkv;
                 q_stride = HD;
                 after_norm = true;
@@ -595,6 +605,7 @@ struct Run {
                     rc = tile_qkv_rope_ahead(xn, hidden, T, hidden, a.qkv.w, a.qkv.bias, a.qkv.bias_dtype, qkv, a.H, a.KVH, a.D, a.cos_t,
                                              a.sin_t, s->positions, slots, kp, vp, a.page, matrices, stream);
                     brought = matrices.n > 0;
+                    count(TM_BROUGHT_BY_QKV, matrices);
                     q = qkv;
                     q_stride = HD;
                     ++p->taken[TM_QKV_PLAIN];
@@ -656,7 +667,9 @@ struct Run {
                     rc = attn_prefill_ahead(q, q_stride, attn, HD, a.k_pool, a.v_pool, tables, W, s->prefill_tiles, s->n_tiles, a.H, a.KVH, a.D, a.page,
                                             a.scale, a.window, a.keep, a.softcap, a.sink, cg, cgate_ld, matrices, stream, both ? &decodes : nullptr);
                     if (matrices.n) gone = true;
+                    count(TM_BROUGHT_BY_ATTENTION, matrices);
                     done_decode = both;
+                    p->taken[TM_DECODE_BESIDE] += both;
                 }
                 done_prefill = true;
             } else if (tp && s->n_tiles > 0 && s->prefill_tiles && dtype == TM_F32 && a.D % 16 == 0 && a.D >= 16 &&
@@ -672,7 +685,10 @@ struct Run {
                 const bool split = decode_in_chunks(p, a, nd, s->max_decode_context);
                 if (gone) matrices.n = 0;       // (the prompt portions' attention had room for them)
                 else if (tp) matrices = after_norm ? ahead(op, AHEAD_OF_ATTENTION) : ahead_behind_norm(op, AHEAD_OF_ATTENTION);
-                if (tm_decode_whole(nd, a.H, a.KVH, a.D, s->max_decode_context))
+                const bool whole = tm_decode_whole(nd, a.H, a.KVH, a.D, s->max_decode_context);
+                p->taken[TM_DECODE_WHOLE] += whole;
+                if (whole || split) count(TM_BROUGHT_BY_ATTENTION, matrices);
+                if (whole)
                     rc = attn_decode_whole_ahead(q_dec, q_stride, out_dec, HD, a.k_pool, a.v_pool, tables + (size_t)(S - nd) * W, W,
                                                  s->context_lens + (S - nd), tm_decode_chunks(s->max_decode_context), nd, a.H, a.KVH, a.D, a.page,
                                                  a.scale, a.window, a.keep, a.softcap, a.sink, cg_dec, cgate_ld, matrices, stream);
@@ -726,8 +742,9 @@ struct Run {
             const bool plain = f.gate_up.dtype == dtype && f.gate_up.bias == nullptr;
             const bool two_parts = f.gate_up.packed_parts == 2 && f.gate_up.packed_rows == 16;
             if (own_norm && delta == nullptr && !pending_sums && starts_at_norm(f)) {
-                rc = fused_norm_gate_up_silu_ahead(resid, f.norm.w, f.norm.w_dtype, f.norm.eps, T, hidden, f.gate_up.packed, act, f.I,
-                                                   ahead(op, AHEAD_OF_GATE_UP), stream);
+                const TmAhead matrices = ahead(op, AHEAD_OF_GATE_UP);
+                count(TM_BROUGHT_BY_GATE_UP, matrices);
+                rc = fused_norm_gate_up_silu_ahead(resid, f.norm.w, f.norm.w_dtype, f.norm.eps, T, hidden, f.gate_up.packed, act, f.I, matrices, stream);
                 ++p->taken[TM_GATE_UP_FROM_NORM];
             } else {
                 const void* xn = x_in;
@@ -893,6 +910,10 @@ void tm_program_counters(const TmProgram* p, long long* out) {
     for (int i = 0; i < TM_PROGRAM_COUNTERS; ++i) out[i] = p ? p->taken[i] : 0;
 }
 
+void tm_program_brought(const TmProgram* p, long long* out) {
+    for (int i = 0; i < TM_BROUGHT_COUNTERS; ++i) out[i] = p ? p->brought[i] : 0;
+}
+
 // Most parts that a product's K is split into in a step of T tokens (their sums [T, hidden] are kept until the next norm).
 static int program_sums(const TmProgram* p, int T) {
     if (p->dtype == TM_BF16 && T <= TM_STREAM_ROWS) return TM_MAX_SUMS;
@@ -949,6 +970,7 @@ int tm_program_run(const TmProgram* p, int first, int count, const TmStep* s, Tm
     r.p = p; r.s = s; r.stream = stream; r.dtype = p->dtype;
     r.products.stream = stream; r.products.lib_ws = library_workspace; r.products.lib_ws_bytes = library_workspace_bytes;
     r.products.tune = p->tune;
+    r.products.head_few = &p->taken[TM_HEAD_FEW];
     if (flags & TM_RUN_TUNE_AT_ONCE) r.products.tune.after = 1;
     r.products.skinny_rows = tm_skinny_rows(p->hidden);
     r.from_norm_rows = tm_from_norm_rows(p->hidden);

@@ -64,7 +64,10 @@ RUN_LABELS, RUN_TUNE_AT_ONCE = 1, 2
 # how q|k|v, the feed-forward's activation, the projections and the attention were computed, in the order of the header's counters
 COUNTERS = ("qkv_from_norm", "qkv_panel", "qkv_stream", "qkv_plain", "gate_up_from_norm",
             "gate_up_stream", "gate_up_plain", "prefill_split_keys", "prefill_shared_keys", "qkv_tiled", "qkv_few_f32",
-            "gate_up_tiled", "gate_up_few_f32", "project_tiled", "project_stream", "project_few_f32", "decode_f32_split")
+            "gate_up_tiled", "gate_up_few_f32", "project_tiled", "project_stream", "project_few_f32", "decode_f32_split",
+            "decode_whole", "decode_beside", "head_few")
+# matrices brought ahead of their products: by which kernel, and how many of all of them in the order of a tiled product
+BROUGHT = ("qkv", "attention", "gate_up", "row_major")
 
 
 def bound():
@@ -89,6 +92,8 @@ def bound():
     lib.tm_program_workspace_bytes.argtypes = [c_void_p, c_int, c_int, c_int, c_int]
     lib.tm_program_counters.restype = None
     lib.tm_program_counters.argtypes = [c_void_p, POINTER(ctypes.c_longlong)]
+    lib.tm_program_brought.restype = None
+    lib.tm_program_brought.argtypes = [c_void_p, POINTER(ctypes.c_longlong)]
     lib.tm_program_run.restype = c_int
     lib.tm_program_run.argtypes = [c_void_p, c_int, c_int, POINTER(TmStep), POINTER(TmStream), c_void_p, c_size_t, c_void_p,
                                    c_size_t, c_void_p, c_int, c_void_p]

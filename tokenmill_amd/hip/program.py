@@ -205,6 +205,12 @@ class StepProgram:
         self._lib.tm_program_counters(self._handle, out)
         return dict(zip(abi.COUNTERS, out))
 
+    def brought(self) -> dict[str, int]:
+        """How many matrices the steps' kernels were given to bring ahead (``abi.BROUGHT``)."""
+        out = (ctypes.c_longlong * len(abi.BROUGHT))()
+        self._lib.tm_program_brought(self._handle, out)
+        return dict(zip(abi.BROUGHT, out))
+
     def _label(self, op: int, name: str, begin: bool) -> None:
         """Called by the library around a span's launches while a profile is collected."""
         if begin:
