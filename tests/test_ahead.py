@@ -119,7 +119,7 @@ def _brought(width, heads, kv_heads, head_dim, inside, contexts, portions, graph
     return [{k: n - b[k] for k, n in a.items() if n != b[k]} for a, b in zip(after, before)]
 
 
-SMALL, LARGE = (896, 14, 2, 64, 4864), (1536, 12, 2, 128, 8960)
+SMALL, WIDE_QKV, LARGE = (896, 14, 2, 64, 4864), (1024, 16, 8, 128, 3072), (1536, 12, 2, 128, 8960)
 NORM = {"qkv_from_norm": 3, "gate_up_from_norm": 3, "head_few": 1}
 TILED = {"qkv_plain": 3, "qkv_tiled": 3, "gate_up_plain": 3, "gate_up_tiled": 3, "project_tiled": 6, "head_few": 1}
 
@@ -130,6 +130,8 @@ TILED = {"qkv_plain": 3, "qkv_tiled": 3, "gate_up_plain": 3, "gate_up_tiled": 3,
     (SMALL, [300], [], {"qkv": 3, "attention": 6, "gate_up": 5}, {**NORM, "decode_whole": 3}),
     (SMALL, [300] * 8, [], {"qkv": 3, "attention": 6, "gate_up": 5}, {**NORM, "decode_whole": 3}),
     (SMALL, [2100] * 4, [], {"qkv": 3, "attention": 6, "gate_up": 5}, NORM),
+    # q|k|v has no CU to spare, gate|up room for down alone
+    (WIDE_QKV, [300], [], {"attention": 3, "gate_up": 3}, {**NORM, "decode_whole": 3}),
     (LARGE, [300], [], {}, {**NORM, "decode_whole": 3}),
     # attention: o and down; gate|up too where it is one launch
     (SMALL, [90] * 12, [], {"attention": 9}, {"qkv_panel": 3, "gate_up_stream": 3, "head_few": 1, "decode_whole": 3}),

@@ -400,12 +400,18 @@ struct Run {
     // its own blocks take, and all of a layer is in the second-level caches (32 MB) when it is used; a layer of more than that brings nothing.
     // Steps of the 0.5B shape, us: one request of 300 keys 677 to 620, eight of 2,048 788 to 737, four of 1,000 753 to 683, four of up to 16,000 837
     // to 821. Without the share of q|k|v's / without o / without the rest of gate|up / without the next q|k|v the first takes 641 / 628 / 642 / 633,
-    // with all of it by the attention 658. Blocks: about as many as the kernel leaves CUs for, half of that and up beside q|k|v's 72 (72 / 96 / 144
-    // of them 638 / 626 / 620), beside the attention 72 / 144 / 200 619 / 623 / 628 (eight requests 746 / 741 / 745 to 740), beside gate|up's
-    // 152 blocks 64 / 104 / 208 642 / 619 / 646.
+    // with all of it by the attention 658.
+    // The blocks are those the kernel leaves CUs for, and a block brings what it can for as long as the kernel's own run: beyond that the launch waits for it
+    // (beside q|k|v's 72 blocks 72 / 96 / 144 blocks of 121 / 91 / 61 KB 638 / 626 / 620 us; beside gate|up's 152, 64 / 104 of 168 / 104 KB 642 / 619;
+    // beside the attention 72 / 144 / 200 619 / 623 / 628, eight requests 746 / 741 / 745 to 740 with 104). What is more than that for the blocks there are
+    // is not brought. Layers of up to 32 MB whose q|k|v has more blocks, one request of 300 keys / eight of 2,000, us with nothing brought, with 120 and 96
+    // blocks whatever they had to bring, and so: width 1,024, heads 16 over 8 of 128, 3,072 inside (256 and 192 blocks of q|k|v and gate|up) 747 / 1,002,
+    // 733 / 1,036, 696 / 979; 16 over 16 of 64, 2,816 (192, 176) 684 / 990, 663 / 1,012, 645 / 980; 768, 12 over 12 of 64, 3,072 (144, 192) 663 / 868, 633 / 884,
+    // 616 / 841; 1,024, 16 over 4 of 64, 4,096 (96, 256) 706 / 783, 670 / 785, 654 / 769.
     enum { AHEAD_OF_QKV, AHEAD_OF_ATTENTION, AHEAD_OF_GATE_UP };
     TmAhead ahead(int op, int host) const {
         constexpr size_t MOST = 32u << 20;
+        constexpr int QKV_KB = 112, GATE_UP_KB = 116;               // a block
         TmAhead h;
         const int at = host == AHEAD_OF_GATE_UP ? op - 1 : op;      // the layer's attention
         if (!accumulate || at < first_op || at + 1 >= last_op || p->ops[at].kind != OP_ATTENTION || p->ops[at + 1].kind != OP_FEED_FORWARD) return h;
@@ -418,12 +424,14 @@ struct Run {
         if (next && !starts_at_norm(*next)) next = nullptr;
         const int units = (f.I + 15) / 16, blocks = fused_gate_up_blocks(f.I), half = (units + blocks - 1) / blocks / 2;
         auto strips = [](const TmLinear& L) { return (L.N + L.packed_rows - 1) / L.packed_rows; };
-        if (strip(f.gate_up) * 2 * units + strip(a.o) * strips(a.o) + strip(f.down) * strips(f.down) +
-                (next ? strip(next->qkv) * strips(next->qkv) : 0) > MOST)
-            return h;
+        auto bytes = [&](const TmLinear& L) { return strip(L) * strips(L); };
+        if (strip(f.gate_up) * 2 * units + bytes(a.o) + bytes(f.down) + (next ? bytes(next->qkv) : 0) > MOST) return h;
         if (host == AHEAD_OF_QKV) {
-            h.blocks = 120;
-            h.packed(f.gate_up.packed, (int)strip(f.gate_up), units, true, blocks, false, 0, half > 0 ? half : 1);
+            const int idle = 256 - (a.H + 2 * a.KVH) * a.D / (2 * a.qkv.packed_rows);
+            const int rounds = half > 0 ? half : 1, taken = rounds * blocks < units ? rounds * blocks : units;
+            h.blocks = idle < 160 ? idle : 160;
+            if (idle < 128 || strip(f.gate_up) * 2 * taken > (size_t)h.blocks * QKV_KB * 1024) return h;
+            h.packed(f.gate_up.packed, (int)strip(f.gate_up), units, true, blocks, false, 0, rounds);
         } else if (host == AHEAD_OF_ATTENTION) {
             h.blocks = 104;
             h.packed(a.o.packed, (int)strip(a.o), strips(a.o), false, strips(a.o));
@@ -431,8 +439,12 @@ struct Run {
         } else {
             h.blocks = 256 - blocks > 96 ? 96 : 256 - blocks;
             if (h.blocks < 32) return h;
-            h.packed(f.down.packed, (int)strip(f.down), strips(f.down), false, strips(f.down));
-            if (next) {
+            size_t room = (size_t)h.blocks * GATE_UP_KB * 1024;
+            if (bytes(f.down) <= room) {
+                h.packed(f.down.packed, (int)strip(f.down), strips(f.down), false, strips(f.down));
+                room -= bytes(f.down);
+            }
+            if (next && bytes(next->qkv) <= room) {
                 const int head_units = next->D / (2 * next->qkv.packed_rows), all = (next->H + 2 * next->KVH) * head_units;
                 h.packed(next->qkv.packed, (int)strip(next->qkv), all, true, all, false, 0, 1, head_units, next->H + next->KVH);
             }
