@@ -94,3 +94,50 @@ def test_lists_give_the_tokens_of_the_launches_over_all_chunks(where, vocab):
     for _ in range(2):                                                       # (the second call finds what the first left in the scratch memory)
         ops.sample_rows(logits, *args, got, small_top_k=True)
         assert got.tolist() == want.tolist()
+
+
+TOGETHER = ("few of -inf", "many of -inf", "few of the smallest", "one place of -inf", "a larger place of -inf", "steps in one place", "two steps in one place",
+            "half raised", "ascending", "descending", "one level", "one above a level", "infinite", "one place of not numbers")
+
+
+@pytest.mark.parametrize("vocab", [V, 151936, 4097, 1 << 20])
+@pytest.mark.parametrize("where", TOGETHER)
+def test_lists_of_rows_whose_large_entries_lie_together(where, vocab):
+    """Fewer finite entries than k; a level that fills all shares; more entries above the bound than a list holds, in few shares and in most, with the edge
+    of top-k inside equal ones or not: the tokens of the launches over all chunks."""
+    from tokenmill_amd.hip import ops
+    most = ops.sample_list_k(vocab)
+    ks = sorted({2, 7, 20, 50, most // 2, most})
+    R = 4 * len(ks)
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    x = torch.randn(R, vocab, generator=g, device="cuda") * 2
+    place = torch.zeros(vocab, dtype=torch.bool, device="cuda")
+    place[vocab // 5:vocab // 5 + (min(900, vocab // 3) if where == "one place of -inf" else min(4000, vocab // 2))] = True
+    if where.startswith(("few", "many")):
+        kept = torch.rand(R, vocab, generator=g, device="cuda").topk(5 if where.startswith("few") else min(700, vocab // 8), 1).indices
+        logits = torch.full_like(x, torch.finfo(torch.float32).min if "smallest" in where else float("-inf")).scatter(1, kept, x.gather(1, kept))
+    elif "place of -inf" in where:
+        logits = x.masked_fill(~place, float("-inf"))
+    elif "steps in" in where:
+        logits = ((x * (2 if where.startswith("steps") else 0.1)).round() / 2).masked_fill(~place, -9.0)
+    elif where == "half raised":
+        logits = x + 30 * (torch.arange(vocab, device="cuda") >= vocab // 2)
+    elif where in ("ascending", "descending"):
+        logits = (torch.arange(vocab, dtype=torch.float32, device="cuda") * (20 / vocab if where == "ascending" else -20 / vocab)).expand(R, vocab).contiguous()
+    elif where == "infinite":
+        logits = x.masked_fill(place, float("inf"))
+    elif where == "one place of not numbers":
+        logits = x.masked_fill(~place, float("nan"))
+    else:
+        logits = torch.full_like(x, 0.5)
+        if where.startswith("one above"):
+            logits[:, vocab // 3] = 2.0
+    f = lambda v: torch.tensor(v, dtype=torch.float32, device="cuda")       # noqa: E731
+    k = torch.tensor([ks[r % len(ks)] for r in range(R)], dtype=torch.int32, device="cuda")
+    p = f([(1.0, 0.95, 0.5, 1e-4)[r // len(ks)] for r in range(R)])
+    for u in (0.0, 0.31, 0.77, 1 - 2.0 ** -24):
+        args = (f([0.8] * R), k, p, f([u] * R))
+        want, got = (torch.full((R,), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+        ops.sample_rows(logits, *args, want)
+        ops.sample_rows(logits, *args, got, small_top_k=True)
+        assert got.tolist() == want.tolist(), u

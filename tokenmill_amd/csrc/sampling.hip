@@ -646,50 +646,194 @@ __global__ __launch_bounds__(SR_NT) void sample_chunk_mass_kernel(const float* _
 
 // --- rows whose top-k is small -----------------------------------------------------------------------------------------------
 //
-// What reaches the bound of sample_bound_kernel is little more than the k entries (k = 50 of 151,936: 60 to 70), so where every row of a call has such
+// What lies above the bound of sample_bound_kernel is little more than the k entries (k = 50 of 151,936: 60 to 70), so where every row of a call has such
 // a k the entries are gathered into a list a row, one read of the shares that hold any, and a block a row finds in the list where top-k and
-// top-p end, by counting, and sums the chunks' masses in the order of sample_chunk_mass_kernel. Seven launches over all chunks (six levels and the
-// masses, 84 us for 64 rows of 151,936 with both filters, most of it launches whose blocks find nothing) are two of 14.6 and 15.4: a whole call 110.9 to 58.2 us, of one / eight
-// rows 60.1 / 63.7 to 36.7 / 41.8, with k = 50 alone 73.6 / 42.8 / 45.4 to 57.7 / 36.3 / 41.5. A row whose list does not hold what
-// reaches the bound (thousands of equal logits), or that has no bound, is worked out by its block alone from the row itself, level by level
-// as the launches do it: slow, right, and rare.
-#define SR_LIST 512
+// top-p end, by counting, and sums the chunks' masses in the order of sample_chunk_mass_kernel. Of entries at the bound their number in every chunk is enough: a
+// level that fills the shares (a masked vocabulary with fewer than k entries left, equal logits) needs no list. Seven launches over all chunks (six levels and
+// the masses, 84 us for 64 rows of 151,936 with both filters, most of it launches whose blocks find nothing) are two of 15: a whole call of 64 / 8 / 1 rows
+// 107.6 / 62.4 / 56.9 to 57.2 / 41.8 / 36.4 us, with k = 20 47.4 / 35.6 / 31.0, with 100 70.4 / 52.4 / 45.9.
+//
+// Where the large entries lie in fewer than k shares, far more are above the bound. A chunk with more than 2 k of them gathers again, what its k-th
+// largest thread has and more, and the row's block narrows what is more than worth counting, up to SR_LIST_ALL entries, to the largest first, digit by
+// digit. 1 / 64 rows, us, by the launches and so: 30 entries in -inf 65 / 224 and 37 / 59; 4,000 in one place, the rest -inf, k = 50 60 / 113 and 52 / 64, k =
+// 100 60 / 114 and 68 / 86; half a vocabulary raised, k = 100, 60 / 124 and 63 / 90; 20,000 raised, k = 50, 58 / 91 and 50 / 61; sorted logits, k = 50 63 /
+// 113 and 59 / 74, k = 100 65 / 124 and 74 / 97, of a million with k = 112 one row 96 and 130. What a list has no room for, more than SR_LIST equal entries
+// above the bound in a chunk, is narrowed from the row itself (40,000 of two levels above a third: 65 / 137 and 224 / 246).
+#define SR_LIST 256             // entries counted, one a thread
+#define SR_LIST_ALL 16384       // entries a row's list has room for (SR_LIST of a chunk)
 
 __global__ __launch_bounds__(SR_NT) void sample_gather_kernel(const float* __restrict__ logits, int V, int chunk, const float* __restrict__ temperature,
                                                               const int* __restrict__ top_k, const float* __restrict__ top_p,
                                                               const float* __restrict__ rowmax, const float* __restrict__ wave_v,
-                                                              const RowState* __restrict__ row_state, uint2* __restrict__ lists, int* __restrict__ counts) {
+                                                              const RowState* __restrict__ row_state, uint2* __restrict__ lists, int* __restrict__ counts,
+                                                              int* __restrict__ chunk_ties) {
     __shared__ uint2 s_list[SR_LIST];
-    __shared__ int s_n, s_base;
+    __shared__ uint32_t s_best[SR_NT], s_floor;
+    __shared__ int s_n, s_ties, s_base;
     const int r = blockIdx.x, c = blockIdx.y;
     const RowParams rp = row_params(r, V, temperature, top_k, top_p, rowmax);
     const uint32_t bound = row_state[r].bound;
     if (!rp.need_k || bound == 0u) return;               // block-uniform
     const bool skip = share_below(wave_v, (size_t)r * gridDim.y + c, rp.inv_t, bound);
-    if (threadIdx.x == 0) s_n = 0;
-    if (__syncthreads_and(skip)) return;
+    if (threadIdx.x == 0) s_n = s_ties = 0;
+    if (__syncthreads_and(skip)) {
+        if (threadIdx.x == 0) chunk_ties[(size_t)r * gridDim.y + c] = 0;
+        return;
+    }
     const float* row = logits + (size_t)r * V;
     const int lo = c * chunk, hi = lo + chunk < V ? lo + chunk : V;
-    for (int i = lo + threadIdx.x; i < hi && !skip; i += 8 * SR_NT) {
-        float v[8];
+    int ties = 0;
+    uint32_t best = 0u;
+    auto gather = [&](uint32_t floor) {
+        for (int i = lo + threadIdx.x; i < hi && !skip; i += 8 * SR_NT) {
+            float v[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = row[i + j * SR_NT < hi ? i + j * SR_NT : i];
+            for (int j = 0; j < 8; ++j) v[j] = row[i + j * SR_NT < hi ? i + j * SR_NT : i];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float z = v[j] * rp.inv_t;
-            if (i + j * SR_NT >= hi || !(z == z)) continue;
-            const uint32_t key = order_key(z);
-            if (key < bound) continue;
-            const int at = atomicAdd(&s_n, 1);
-            if (at < SR_LIST) s_list[at] = uint2{key, (uint32_t)(i + j * SR_NT)};
+            for (int j = 0; j < 8; ++j) {
+                const float z = v[j] * rp.inv_t;
+                if (i + j * SR_NT >= hi || !(z == z)) continue;
+                const uint32_t key = order_key(z);
+                ties += key == bound;
+                if (key < floor) continue;
+                best = key > best ? key : best;
+                const int at = atomicAdd(&s_n, 1);
+                if (at < SR_LIST) s_list[at] = uint2{key, (uint32_t)(i + j * SR_NT)};
+            }
         }
-    }
+    };
+    gather(bound + 1);
+    if (ties) atomicAdd(&s_ties, ties);
     __syncthreads();
-    const int n = s_n;
-    if (threadIdx.x == 0 && n) s_base = atomicAdd(&counts[r], n);
+    int n = s_n;
+    if (threadIdx.x == 0) chunk_ties[(size_t)r * gridDim.y + c] = s_ties;
+    if (n > 2 * rp.k && rp.k <= SR_NT) {
+        // far more than can count: none below the k-th largest of the threads' largest does
+        s_best[threadIdx.x] = best;
+        if (threadIdx.x == 0) s_floor = bound + 1;
+        __syncthreads();
+        int larger = 0, level = 0;
+#pragma unroll 8
+        for (int i = 0; i < SR_NT; ++i) {
+            larger += s_best[i] > best;
+            level += s_best[i] == best;
+        }
+        if (best > bound && larger < rp.k && larger + level >= rp.k) s_floor = best;        // (threads that write it write one value)
+        if (threadIdx.x == 0) s_n = 0;
+        __syncthreads();
+        gather(s_floor);
+        __syncthreads();
+        n = s_n;
+    }
+    if (threadIdx.x == 0 && n) s_base = atomicAdd(&counts[r], n <= SR_LIST ? n : SR_LIST_ALL + 1);
     __syncthreads();
     const int base = n ? s_base : 0;
-    for (int i = threadIdx.x; i < n && i < SR_LIST && base + i < SR_LIST; i += SR_NT) lists[(size_t)r * SR_LIST + base + i] = s_list[i];
+    for (int i = threadIdx.x; i < n && i < SR_LIST && base + i < SR_LIST_ALL; i += SR_NT) lists[(size_t)r * SR_LIST_ALL + base + i] = s_list[i];
+}
+
+// Where narrow_list takes a row's entries from: its list, or, where that does not hold them, the row itself.
+struct Entries {
+    const uint2* list;
+    int n;                      // in the list
+    const float *row, *tops;    // tops: the largest of the shares of every chunk
+    int V, chunk, NB;
+    float inv_t;
+};
+
+// f(is there one, key, index) by every lane of a wavefront, for entries among which are all with keys of `floor` and more, 16 loads at a time. Of the row a
+// wavefront goes through those of its shares by itself that hold such a key.
+template <typename F>
+__device__ __forceinline__ void for_entries(const Entries& e, uint32_t floor, F&& f) {
+    constexpr int WAVES = SR_NT / TM_WAVE, DEEP = 16;
+    static_assert(SR_LIST_ALL % (DEEP * SR_NT) == 0, "");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE), lane = threadIdx.x % TM_WAVE;
+    const bool listed = e.n <= SR_LIST_ALL;
+    for (int c0 = 0; c0 < (listed ? 1 : e.NB); c0 += TM_WAVE) {
+        unsigned long long left = 1ull;
+        if (!listed) {
+            const float top = e.tops[(c0 + lane < e.NB ? c0 + lane : e.NB - 1) * WAVES + wave] * e.inv_t;
+            left = __ballot(c0 + lane < e.NB && !(top == top && order_key(top) < floor));
+        }
+        for (; left; left &= left - 1) {
+            const int lo = listed ? 0 : (c0 + __builtin_ctzll(left)) * e.chunk, hi = listed ? e.n : lo + e.chunk < e.V ? lo + e.chunk : e.V;
+            for (int o = lo + threadIdx.x; o - lane < hi; o += DEEP * SR_NT) {
+                uint32_t key[DEEP], at[DEEP];
+#pragma unroll
+                for (int j = 0; j < DEEP; ++j) {
+                    const int i = o + j * SR_NT < hi ? o + j * SR_NT : hi - 1;
+                    if (listed) {
+                        const uint2 x = e.list[i];
+                        key[j] = x.x, at[j] = x.y;
+                    } else {
+                        key[j] = __float_as_uint(e.row[i]), at[j] = i;
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < DEEP; ++j) {
+                    const float z = __uint_as_float(key[j]) * e.inv_t;
+                    f(o + j * SR_NT < hi && (listed || z == z), listed ? key[j] : order_key(z), (int)at[j]);
+                }
+            }
+        }
+    }
+}
+
+// More than `most` entries of a row lie above the bound (one block, all threads call): a bound that leaves at most so many above it, or fewer than k (s_key,
+// s_idx; s_ties the entries at it by chunk, where they are needed to fill up to k), from the k-th largest entry's key digit by digit.
+__device__ __forceinline__ int narrow_list(const Entries& e, const RowParams& rp, int most, uint32_t& bound, unsigned long long* s_hist, unsigned long long* s_scan,
+                                           unsigned long long* s_res, uint32_t* s_key, uint32_t* s_idx, int* s_ties, int* s_count) {
+    const int t = threadIdx.x, lane = t % TM_WAVE;
+    unsigned long long limit = (unsigned long long)rp.k, above = 0;
+    uint32_t prefix = 0, mask = 0;
+    bool exact = true;
+    for (int level = 0; level < 3; ++level) {
+        const int shift = level_shift(level);
+        const uint32_t digit_mask = (uint32_t)(level_bins(level) - 1);
+        for (int b = t; b < SR_BINS; b += SR_NT) s_hist[b] = 0ull;
+        __syncthreads();
+        for_entries(e, bound + 1 > prefix ? bound + 1 : prefix, [&](bool in, uint32_t key, int) {
+            in = in && key > bound && (key & mask) == prefix;
+            const uint32_t digit = (key >> shift) & digit_mask;
+            // equal digits of a wavefront at once (large entries share their exponents, and one counter would take them one by one)
+            unsigned long long left = __ballot(in);
+            for (int turn = 0; left && turn < 3; ++turn) {
+                const uint32_t d = __builtin_amdgcn_readlane(digit, __builtin_ctzll(left));
+                const unsigned long long same = __ballot(in && digit == d);
+                if (lane == __builtin_ctzll(same)) atomicAdd(&s_hist[d], (unsigned long long)__popcll(same));
+                left &= ~same;
+                in = in && digit != d;
+            }
+            if (in) atomicAdd(&s_hist[digit], 1ull);
+        });
+        __syncthreads();
+        uint32_t bucket;
+        pick_bucket(s_hist, level_bins(level), false, -1.0, 0ull, limit, above, bucket, s_scan, s_res);
+        const int held = (int)s_hist[bucket];
+        __syncthreads();
+        prefix |= bucket << shift;
+        mask |= digit_mask << shift;
+        if (level < 2 && above + (unsigned long long)held <= (unsigned long long)most) {      // (they hold the k-th largest: no tie at the bound is needed)
+            exact = false;
+            --prefix;
+            break;
+        }
+    }
+    bound = prefix;
+    for (int c = t; c < e.NB; c += SR_NT) s_ties[c] = 0;
+    if (t == 0) *s_count = 0;
+    __syncthreads();
+    for_entries(e, exact ? bound : bound + 1, [&](bool in, uint32_t key, int i) {
+        if (exact && in && key == bound) atomicAdd(&s_ties[i / e.chunk], 1);
+        if (in && key > bound) {
+            const int at = atomicAdd(s_count, 1);
+            if (at < SR_LIST) {                          // (no more are above the bound)
+                s_key[at] = key;
+                s_idx[at] = (uint32_t)i;
+            }
+        }
+    });
+    __syncthreads();
+    return *s_count;
 }
 
 // The same from the row itself, by one block.
@@ -741,42 +885,56 @@ __device__ void select_from_row(const float* __restrict__ row, int V, int chunk,
 __global__ __launch_bounds__(SR_NT) void sample_select_kernel(const float* __restrict__ logits, int V, int chunk, int NB,
                                                               const float* __restrict__ temperature, const int* __restrict__ top_k,
                                                               const float* __restrict__ top_p, const float* __restrict__ rowmax,
-                                                              const RowState* __restrict__ row_state, const uint2* __restrict__ lists,
-                                                              const int* __restrict__ counts, unsigned long long* __restrict__ hist_all,
-                                                              float* __restrict__ chunk_weight, int* __restrict__ chunk_ties,
-                                                              RowKeep* __restrict__ row_keep) {
+                                                              const float* __restrict__ wave_v, const RowState* __restrict__ row_state,
+                                                              const uint2* __restrict__ lists, const int* __restrict__ counts,
+                                                              unsigned long long* __restrict__ hist_all, float* __restrict__ chunk_weight,
+                                                              int* __restrict__ chunk_ties, RowKeep* __restrict__ row_keep) {
     __shared__ unsigned long long s_hist[SR_BINS];       // (the list's weights lie in it)
     __shared__ uint32_t s_key[SR_LIST], s_idx[SR_LIST];
     __shared__ unsigned long long s_scan[SR_NT / TM_WAVE], s_res[2];
     __shared__ float s_w[SR_NT / TM_WAVE];
     __shared__ int s_n[SR_NT / TM_WAVE];
-    __shared__ int s_begin[256];
+    __shared__ int s_begin[256], s_ties[256], s_total, s_count;
     __shared__ RowKeep s_keep;
     __shared__ unsigned long long s_limit;
     constexpr int GROUP = 8;
     const int r = blockIdx.x, t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / TM_WAVE), lane = t % TM_WAVE;
     const RowParams rp = row_params(r, V, temperature, top_k, top_p, rowmax);
     if (rp.greedy) return;                               // block-uniform
-    const int n = counts[r];
-    const bool listed = rp.need_k && row_state[r].bound != 0u && n >= rp.k && n <= SR_LIST;
+    int n = counts[r];
+    uint32_t bound = row_state[r].bound;
     chunk_weight += (size_t)r * NB;
     chunk_ties += (size_t)r * NB;
-    if (!listed) {
+    if (!rp.need_k || bound == 0u) {
         RowKeep keep;
         select_from_row(logits + (size_t)r * V, V, chunk, NB, rp, hist_all + (size_t)r * SR_HIST_PER_ROW, s_hist, s_scan, s_res, s_w, s_n, chunk_weight,
                         chunk_ties, keep);
         if (t == 0) row_keep[r] = keep;
         return;
     }
-    // the list by vocabulary order
+    // the list, and how many entries of every chunk are at the bound
     uint2 mine[SR_LIST / SR_NT];
-    for (int c = t; c < NB; c += SR_NT) s_begin[c] = n;
+    const int most = 2 * rp.k + 32 < SR_LIST ? 2 * rp.k + 32 : SR_LIST;     // (an entry costs 0.1 us, narrowing some 15)
+    if (n > most) {
+        const Entries e{lists + (size_t)r * SR_LIST_ALL, n, logits + (size_t)r * V, wave_v + (size_t)r * NB * (AM_NT / TM_WAVE), V, chunk, NB, rp.inv_t};
+        n = narrow_list(e, rp, most, bound, s_hist, s_scan, s_res, s_key, s_idx, s_ties, &s_count);
 #pragma unroll
-    for (int j = 0; j < SR_LIST / SR_NT; ++j) {
-        const int i = t + j * SR_NT;
-        mine[j] = lists[(size_t)r * SR_LIST + (i < n ? i : 0)];
-        s_idx[i] = i < n ? mine[j].y : 0xffffffffu;      // (what pads the list to whole groups is behind all, smaller than all, and weighs nothing)
+        for (int j = 0; j < SR_LIST / SR_NT; ++j) mine[j] = uint2{s_key[t + j * SR_NT], s_idx[t + j * SR_NT]};
+    } else {
+#pragma unroll
+        for (int j = 0; j < SR_LIST / SR_NT; ++j) mine[j] = lists[(size_t)r * SR_LIST_ALL + (t + j * SR_NT < n ? t + j * SR_NT : 0)];
+        for (int c = t; c < NB; c += SR_NT) s_ties[c] = chunk_ties[c];
     }
+    if (t == 0) s_total = 0;
+    __syncthreads();
+    for (int c = t; c < NB; c += SR_NT) {
+        s_begin[c] = n;
+        if (s_ties[c]) atomicAdd(&s_total, s_ties[c]);
+    }
+    // ... by vocabulary order
+#pragma unroll
+    for (int j = 0; j < SR_LIST / SR_NT; ++j)            // (what pads the list to whole groups is behind all, smaller than all, and weighs nothing)
+        s_idx[t + j * SR_NT] = t + j * SR_NT < n ? mine[j].y : 0xffffffffu;
     __syncthreads();
     const int padded = (n + GROUP - 1) / GROUP * GROUP;
     int place[SR_LIST / SR_NT];
@@ -839,6 +997,21 @@ __global__ __launch_bounds__(SR_NT) void sample_select_kernel(const float* __res
         s_keep = RowKeep{key[j], 1, budget};             // (threads that write them write the same)
         s_limit = (unsigned long long)((double)(total > dropped ? total - dropped : 0ull) * (double)rp.p);
     }
+    // ... which is the bound, where the list is shorter than k
+    const unsigned long long w_bound = fix_weight(expf(key_value(bound) - rp.zmax));
+    unsigned long long listed = 0ull;
+    if (n < rp.k) {
+        for (int i = 0; i < padded; i += GROUP)
+#pragma unroll
+            for (int j = 0; j < GROUP; ++j) listed += s_weight[i + j];
+        if (t == 0) {
+            const int ties = s_total, budget = rp.k - n;
+            const unsigned long long dropped = ties > budget ? (unsigned long long)(ties - budget) * w_bound : 0ull;
+            const unsigned long long total = listed + (unsigned long long)ties * w_bound;
+            s_keep = RowKeep{bound, 1, budget};
+            s_limit = (unsigned long long)((double)(total > dropped ? total - dropped : 0ull) * (double)rp.p);
+        }
+    }
     __syncthreads();
     if (rp.need_p) {
         const unsigned long long limit = s_limit;
@@ -852,9 +1025,15 @@ __global__ __launch_bounds__(SR_NT) void sample_select_kernel(const float* __res
             cut_nucleus(keep, rp, key[j], limit, above[j]);
             s_keep = keep;
         }
+        if (t == 0 && n < rp.k && listed <= limit && listed + (unsigned long long)s_total * w_bound > limit) {
+            RowKeep keep = kept;
+            cut_nucleus(keep, rp, bound, limit, listed);
+            s_keep = keep;
+        }
         __syncthreads();
     }
     const RowKeep keep = s_keep;
+    const bool at_bound = keep.p_key == bound;           // (the ties are the bound's, none of which is in the list)
     if (t == 0) row_keep[r] = keep;
     // the chunks' masses: lanes and wavefronts have the entries that are theirs in sample_chunk_mass_kernel, added as there
     for (int i = t; i < n; i += SR_NT) {
@@ -865,7 +1044,7 @@ __global__ __launch_bounds__(SR_NT) void sample_select_kernel(const float* __res
     for (int c = t; c < NB; c += SR_NT)
         if (s_begin[c] == n) {
             chunk_weight[c] = 0.f;
-            chunk_ties[c] = 0;
+            chunk_ties[c] = at_bound ? s_ties[c] : 0;
         }
     for (int c0 = 0; c0 < NB; c0 += TM_WAVE) {
         // of the chunks that have entries, a wavefront takes every fourth
@@ -893,17 +1072,17 @@ __global__ __launch_bounds__(SR_NT) void sample_select_kernel(const float* __res
             for (int v = 1; v < SR_NT / TM_WAVE; ++v) sum += w[v];
             if (lane == 0) {
                 chunk_weight[c] = sum;
-                chunk_ties[c] = ties;
+                chunk_ties[c] = at_bound ? s_ties[c] : ties;
             }
         }
     }
 }
 
 // The largest k for which the calls of a vocabulary may say that their rows' entries fit a list: three quarters of the shares whose maxima bound them
-// (up to 1.4 entries a share reach it then).
+// (up to 1.4 entries a share reach it then), and no more than counting them is worth.
 extern "C" int tm_sample_list_k(int V) {
     const int NB = tm_argmax_work_chunks(V), shares = NB * (AM_NT / TM_WAVE) <= SR_NT ? NB * (AM_NT / TM_WAVE) : NB;
-    return V > 0 && NB > 1 ? shares * 3 / 4 : 0;
+    return V > 0 && NB > 1 ? (shares * 3 / 4 < 112 ? shares * 3 / 4 : 112) : 0;
 }
 
 // Of `ties` ties that follow `seen` earlier ones, how many stay.
@@ -1082,7 +1261,7 @@ static size_t sample_hist_bytes(int R) { return (size_t)R * SR_HIST_PER_ROW * si
 extern "C" size_t tm_sample_work_bytes(int R, int V) {
     const size_t NB = (size_t)tm_argmax_work_chunks(V);
     const size_t per_chunk = (size_t)R * NB * 4;         // part_v, part_i, chunk_weight, chunk_ties, wave_v
-    return sample_hist_bytes(R) + (size_t)R * sizeof(RowState) + (size_t)R * SR_LIST * sizeof(uint2) + (4 + AM_NT / TM_WAVE) * per_chunk +
+    return sample_hist_bytes(R) + (size_t)R * sizeof(RowState) + (size_t)R * SR_LIST_ALL * sizeof(uint2) + (4 + AM_NT / TM_WAVE) * per_chunk +
            (size_t)R * (sizeof(RowKeep) + 12);
 }
 
@@ -1101,7 +1280,7 @@ extern "C" int tm_sample_rows(const float* logits, int R, int V, const float* te
     unsigned long long* hist = (unsigned long long*)w;
     w += sample_hist_bytes(R);
     RowState* state = (RowState*)w;     w += (size_t)R * sizeof(RowState);
-    uint2* lists = (uint2*)w;           w += (size_t)R * SR_LIST * sizeof(uint2);
+    uint2* lists = (uint2*)w;           w += (size_t)R * SR_LIST_ALL * sizeof(uint2);
     float* part_v = (float*)w;          w += (size_t)R * NB * 4;
     int* part_i = (int*)w;              w += (size_t)R * NB * 4;
     float* wave_v = (float*)w;          w += (size_t)R * NB * (AM_NT / TM_WAVE) * 4;
@@ -1118,10 +1297,10 @@ extern "C" int tm_sample_rows(const float* logits, int R, int V, const float* te
     sample_bound_kernel<<<R, SR_NT, 0, stream>>>(part_v, part_i, wave_v, NB, V, temperature, top_k, top_p, rowmax, rowarg, state, counts);
     TM_CHECK_LAUNCH();
     if (listed) {
-        sample_gather_kernel<<<grid, SR_NT, 0, stream>>>(logits, V, chunk, temperature, top_k, top_p, rowmax, wave_v, state, lists, counts);
+        sample_gather_kernel<<<grid, SR_NT, 0, stream>>>(logits, V, chunk, temperature, top_k, top_p, rowmax, wave_v, state, lists, counts, chunk_ties);
         TM_CHECK_LAUNCH();
-        sample_select_kernel<<<R, SR_NT, 0, stream>>>(logits, V, chunk, NB, temperature, top_k, top_p, rowmax, state, lists, counts, hist, chunk_weight,
-                                                      chunk_ties, row_keep);
+        sample_select_kernel<<<R, SR_NT, 0, stream>>>(logits, V, chunk, NB, temperature, top_k, top_p, rowmax, wave_v, state, lists, counts, hist,
+                                                      chunk_weight, chunk_ties, row_keep);
         TM_CHECK_LAUNCH();
         sample_pick_kernel<<<R, SR_NT, 0, stream>>>(logits, V, chunk, NB, temperature, top_k, top_p, rowmax, rowarg,
                                                     chunk_weight, chunk_ties, row_keep, u, out);
