@@ -73,6 +73,22 @@ def test_the_activation_is_the_one_of_the_other_products(scale):
     assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.nan_to_num(0.0), want.nan_to_num(0.0))
 
 
+def test_the_activation_of_infinities_and_what_is_no_number():
+    """One column of the matrix that is not zero: gates of every bfloat16 value down to 2^-100, both infinities and every NaN, times one; the bits of the kernel
+    behind a plain product."""
+    every = torch.arange(65536, device="cuda").sub(32768).to(torch.int16).view(torch.bfloat16)
+    gates = torch.where(every.float().abs() < 2.0 ** -100, torch.zeros_like(every), every)
+    M, n, K = 65, 65536, 256
+    a, w = torch.zeros(M, K, device="cuda", dtype=torch.bfloat16), torch.zeros(2 * n, K, device="cuda", dtype=torch.bfloat16)
+    a[:, 0], w[:n, 0], w[n:, 0] = 1.0, gates, 1.0
+    out = torch.empty(M, n, device="cuda", dtype=torch.bfloat16)
+    assert library().tm_tile_gate_up_silu(P(a.data_ptr()), I(K), I(M), I(K), P(w.data_ptr()), P(out.data_ptr()), I(n), _stream()) == 0
+    both, want = torch.cat([gates, torch.ones_like(gates)])[None].contiguous(), torch.empty(1, n, device="cuda", dtype=torch.bfloat16)
+    assert library().tm_silu_mul(P(both.data_ptr()), P(want.data_ptr()), I(1), I(1), I(n), _stream()) == 0
+    assert torch.equal(want.isnan()[0], gates.isnan() | (gates == float("-inf")))
+    assert torch.equal(out.isnan(), want.isnan().expand(M, n)) and torch.equal(out.nan_to_num(0.0), want.nan_to_num(0.0).expand(M, n))
+
+
 # (rows, heads, kv heads, head size, K, page): every tile
 QKV = [(65, 14, 2, 64, 256, 16), (333, 14, 2, 64, 896, 16), (1000, 28, 4, 128, 256, 16), (2500, 14, 2, 64, 256, 16), (70, 3, 1, 192, 256, 16),
        (66, 28, 4, 128, 512, 4), (400, 28, 4, 128, 512, 64), (600, 28, 4, 128, 512, 128), (1001, 28, 4, 128, 512, 1), (1500, 28, 4, 128, 512, 32),
