@@ -90,9 +90,8 @@ def test_among_many_a_request_has_its_bits_whatever_the_lengths_beside_it(H, KVH
     assert torch.equal(few, most[:S - 1])
 
 
-@pytest.mark.parametrize("portions", [[], [40], [150, 90]])
-def test_a_step_of_many_requests_beside_a_longer_one(portions):
-    """The same through whole steps: 200 pairs, alone and beside prompt portions (whose launch attends them where contexts are short)."""
+def _many(portions, contexts, max_model_len, graphs):
+    """The logits of a step of a small model (200 pairs and more of request and kv head)."""
     from conftest import qwen2_config
     from tokenmill_amd import EngineConfig, LLMEngine
     from tokenmill_amd.config.registry import architecture_name, get_architecture
@@ -104,16 +103,32 @@ def test_a_step_of_many_requests_beside_a_longer_one(portions):
     g = torch.Generator(device="cuda").manual_seed(1)
     model.load({name: (torch.randn(spec.drawn_shape(), generator=g, device="cuda") * 0.1 + (spec.init == "ones")).bfloat16()
                 for name, spec in sorted(model.tensor_specs().items())}, torch.bfloat16, torch.device(DEV))
-    contexts = [(37 * i) % 1200 + 1 for i in range(99)]
-    got = []
-    for longest in (1000, 1400, 3000):
-        requests = [(0, n) for n in portions] + [(c - 1, 1) for c in contexts + [longest]]
-        engine = LLMEngine(EngineConfig(dtype="bfloat16", block_size=16, num_blocks=sum(-(-(a + b) // 16) for a, b in requests) + 4, watermark=0.0,
-                                        max_model_len=3100, max_num_seqs=128, max_num_batched_tokens=8192, hip_graphs=False), model=model)
-        caches = [engine.cache.allocate(f"r{i}", a + b) for i, (a, b) in enumerate(requests)]
-        ids = [torch.randint(0, 512, (a + b,), generator=torch.Generator().manual_seed(a + b)).tolist() for a, b in requests]
-        for cache, prompt, (a, _) in zip(caches, ids, requests):
-            if a:
-                engine.runner.step([StepEntry(cache, 0, prompt[:a], [a - 1])])
-        got.append(engine.runner.step([StepEntry(cache, a, prompt[a:], [b - 1]) for cache, prompt, (a, b) in zip(caches, ids, requests)])[:-1].clone())
+    requests = [(0, n) for n in portions] + [(c - 1, 1) for c in contexts]
+    engine = LLMEngine(EngineConfig(dtype="bfloat16", block_size=16, num_blocks=sum(-(-(a + b) // 16) for a, b in requests) + 4, watermark=0.0,
+                                    max_model_len=max_model_len, max_num_seqs=128, max_num_batched_tokens=8192, hip_graphs=graphs), model=model)
+    caches = [engine.cache.allocate(f"r{i}", a + b) for i, (a, b) in enumerate(requests)]
+    ids = [torch.randint(0, 512, (a + b,), generator=torch.Generator().manual_seed(a + b)).tolist() for a, b in requests]
+    for cache, prompt, (a, _) in zip(caches, ids, requests):
+        if a:                                            # (without a graph of each prompt's shape)
+            engine.runner.forward(engine.runner.prepare([StepEntry(cache, 0, prompt[:a])])[0])
+    entries = [StepEntry(cache, a, prompt[a:], [b - 1]) for cache, prompt, (a, b) in zip(caches, ids, requests)]
+    for _ in range(4 if graphs else 1):
+        logits = engine.runner.step(entries).clone()
+    assert not graphs or engine.runner.graphs.replays > 0 or engine.runner.step_graphs.replays > 0
+    return logits
+
+
+CONTEXTS = [(37 * i) % 1200 + 1 for i in range(99)]
+
+
+@pytest.mark.parametrize("portions", [[], [40], [150, 90]])
+def test_a_step_of_many_requests_beside_a_longer_one(portions):
+    """The same through whole steps: 200 pairs, alone and beside prompt portions (whose launch attends them where contexts are short)."""
+    got = [_many(portions, CONTEXTS + [longest], 3100, False)[:-1] for longest in (1000, 1400, 3000)]
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("portions", [[], [40]])
+def test_a_replayed_step_of_many_requests_whatever_the_longest_there_may_be(portions):
+    """A graph's kernels are chosen by the engine's limit, not by the contexts there are."""
+    assert torch.equal(_many(portions, CONTEXTS, 1250, True), _many(portions, CONTEXTS, 3100, True))
