@@ -83,7 +83,10 @@ inline bool tm_decode_splits(int requests, int kv_heads, int max_context) {
 
 // Does one block take all of a (request, kv head)'s context (attn_decode_whole_kernel; asked before the other)? Where there are few pairs two launches
 // less a trip to memory stand against one CU's share of the caches, where there are many the chunks would share CUs anyway, and against
-// the block kernel (one chunk, or 192 pairs and more) it merges in one pass. Us, split or block kernel to whole, by head size D:
+// the block kernel (one chunk, or 192 pairs and more) it merges in one pass. max_context is the step's: the longest context of an eager step, and
+// of a replayed one the longest that the engine allows (max_model_len), since a graph serves whatever contexts come: with 2,048 allowed no replayed
+// step below 192 pairs takes this kernel (0.5B shape, one request of 300 keys 640 us a step for 613, 64 of up to 1,021 sampled 1,218 for 1,188).
+// Us, split or block kernel to whole, by head size D (seven heads a kv head, or one):
 //   2 to 16 pairs, D 64   100 / 300 / 500 / 700 / 1,000 keys   5.7 / 6.6 / 6.6 / 6.7 / 6.6 to 4.5 / 5.6 / 6.1 / 7.2 / 8.5
 //   16 and 32,     D 128  100 / 300 / 500 / 700                8.6 / 8.8 / 9.0 / 9.4 to 5.2 / 7.6 / 9.3 / 11.4
 //   64,            D 32   300 / 700 / 1,000                    5.8 / 6.3 / 6.4 to 5.0 / 6.1 / 6.9
@@ -92,6 +95,11 @@ inline bool tm_decode_splits(int requests, int kv_heads, int max_context) {
 //   96 and 128,    D 128  300 / 700 / 1,000                    9.7 / 12.8 / 14.2 and 10.1 / 14.2 / 16.1 to 7.8 / 11.7 / 16.6 and 7.9 / 12.2 / 18.5
 //   256,           D 64   300 / 700 / 1,085                    8.2 / 10.9 / 15.8 to 6.9 / 9.8 / 14.3
 //   192 and 400,   D 128  the same                             11.5 / 17.9 / 25.2 and 21.5 / 34.7 / 46.6 to 8.3 / 14.4 / 21.9 and 14.6 / 27.0 / 40.2
+// and of 16 heads a kv head (of 1, 4 and 8 the same way; 16 pairs of one head of 128 with 400 keys are the worst, 8.4 to 8.5):
+//   4 and 64,      D 128  200 / 400                            9.7 / 9.5 and 10.1 / 10.8 to 7.4 / 9.1 and 7.6 / 9.5
+//   128 and 192,   D 128  400 / 700                            12.5 / 16.3 and 13.1 / 17.8 to 9.8 / 13.0 and 10.4 / 15.2
+//   64 and 128,    D 64   400 / 1,000 (the former 500)         8.0 / 8.3 and 9.8 / 12.3 to 6.2 / 6.6 and 6.5 / 10.0
+//   512,           D 64   400 / 700 / 1,000 / 1,280            12.4 / 20.3 / 27.2 / 32.1 to 11.0 / 18.0 / 25.1 / 32.9 (the last by the block kernel)
 constexpr int TM_DECODE_MANY_PAIRS = 96;
 constexpr int TM_DECODE_WHOLE_KEYS = 1280;
 constexpr size_t TM_DECODE_WHOLE_LDS = 160 * 1024;
@@ -116,7 +124,8 @@ inline bool tm_decode_whole(int requests, int heads, int kv_heads, int head_size
 
 // Do a mixed step's prompt portions, of n_tiles tiles, have its decoded tokens beside them in one launch (attn_prefill_mfma_kernel with DECODES)?
 // The whole kernel's rule does not hold here: what its blocks take longer than the split kernels' they take beside the portions'. Of two blocks a CU the
-// registers hold one, so as many pairs as CUs are the most; contexts end where a block's eight wavefronts have three rounds of keys (16 of 1,500 keys
+// registers hold one, so as many pairs as CUs are the most; contexts (in a replayed step the engine's limit: with 2,048 allowed two launches, and 30 of 1,000
+// beside 2 of 241 take 1,752 us for 1,613) end where a block's eight wavefronts have three rounds of keys (16 of 1,500 keys
 // beside 1 portion of 100 tokens, the least there is to gain: 12.8 to 13.0 us; beside 2 of 256 14.3 to 13.0); where the pairs are so many that longer
 // ones are added up in another order, they end there.
 constexpr int TM_DECODE_BESIDE_LDS = 139264, TM_DECODE_BESIDE_KEYS = 1536;

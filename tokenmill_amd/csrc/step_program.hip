@@ -405,9 +405,9 @@ struct Run {
     // (beside q|k|v's 72 blocks 72 / 96 / 144 blocks of 121 / 91 / 61 KB 638 / 626 / 620 us; beside gate|up's 152, 64 / 104 of 168 / 104 KB 642 / 619;
     // beside the attention 72 / 144 / 200 619 / 623 / 628, eight requests 746 / 741 / 745 to 740 with 104). What is more than that for the blocks there are
     // is not brought. Layers of up to 32 MB whose q|k|v has more blocks, one request of 300 keys / eight of 2,000, us with nothing brought, with 120 and 96
-    // blocks whatever they had to bring, and so: width 1,024, heads 16 over 8 of 128, 3,072 inside (256 and 192 blocks of q|k|v and gate|up) 747 / 1,002,
-    // 733 / 1,036, 696 / 979; 16 over 16 of 64, 2,816 (192, 176) 684 / 990, 663 / 1,012, 645 / 980; 768, 12 over 12 of 64, 3,072 (144, 192) 663 / 868, 633 / 884,
-    // 616 / 841; 1,024, 16 over 4 of 64, 4,096 (96, 256) 706 / 783, 670 / 785, 654 / 769.
+    // blocks whatever they had to bring, and so: width 1,024, heads 16 over 8 of 128, 3,072 inside (256 and 192 blocks of q|k|v and gate|up) 719 / 991,
+    // 736 / 1,039, 700 / 982; 16 over 16 of 64, 2,816 (192, 176) 654 / 983, 664 / 1,018, 648 / 976; 768, 12 over 12 of 64, 3,072 (144, 192) 628 / 856, 634 / 878,
+    // 617 / 849; 1,024, 16 over 4 of 64, 4,096 (96, 256) 666 / 785, 664 / 773, 656 / 758; the 0.5B shape 665 / 778, 611 / 726, 611 / 726.
     enum { AHEAD_OF_QKV, AHEAD_OF_ATTENTION, AHEAD_OF_GATE_UP };
     TmAhead ahead(int op, int host) const {
         constexpr size_t MOST = 32u << 20;
@@ -468,6 +468,11 @@ struct Run {
     // 3 to 5 us long, were slower by what they brought. Steps of the 0.5B shape, us, without to so: prompts of 30 / 77 / 150 / 300 / 600 tokens 896 / 1,054 /
     // 1,155 / 1,352 / 1,812 to 886 / 962 / 1,071 / 1,230 / 1,733, 30 requests beside two portions of 241 1,906 to 1,751, 12 / 16 / 40 / 64 requests 945 / 993 /
     // 995 / 1,272 to 910 / 970 / 958 / 1,242.
+    // Steps of single tokens alone, beyond 64 requests: 96 / 128 / 192 / 256 of up to 300 keys with nothing 1,164 / 1,325 / 1,379 / 1,576, with what the
+    // attention brings 1,131 / 1,242 / 1,297 / 1,486, with q|k|v's too 1,114 / 1,223 / 1,301 / 1,465; of up to 2,000 keys, whose attention reads 50 to 130 MB
+    // a layer in between, 1,527 / 1,755 / 2,010 / 2,402 with nothing and 1,476 / 1,669 / 1,957 / 2,390 so. Of six other shapes of up to 32 MB a layer, 17 to 200 requests,
+    // prompts of 20 to 700 tokens and mixed steps, one in a hundred was slower by more than 0.3% (width 1,024, 16 over 4 heads of 64, 4,096 inside, 24 requests of up to
+    // 1,000 and 2,000 keys 1,042 and 1,082 to 1,052 and 1,099).
     // How the tiled product takes a matrix in this step (0: gate|up, 1: q|k|v, 2: K in parts), asked once for all layers of a size: the rule weighs up to 88
     // ways to cut it.
     TmTilePieces pieces(int what, int N, int K) const {
