@@ -65,6 +65,51 @@ def test_a_row_is_the_same_whatever_rows_are_beside_it(N, K):
         assert torch.equal(product(rows), most[:rows]), rows
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("K,small,large", [(912, 1868, 1872), (1440, 1180, 1184), (6896, 244, 248), (448, 3800, 3808), (400, 4256, 4260)])
+def test_whole_lines_and_a_load_a_step_have_the_same_bits(K, small, large, M):
+    """Matrices of 6.5 MB and less: odd numbers of steps, one, two and three groups a wavefront, four and eight wavefronts, K in parts."""
+    lib = library()
+    a, w, ref = _operands(M, large, K, K)
+    outs, parts, gates = [], [], []
+    for N in (small, large):
+        out = torch.full((M, N), float("nan"), device="cuda")
+        assert lib.tm_gemv_f32_mfma(_ptr(a), I(K), _ptr(w), _ptr(None), _ptr(out), I(N), I(M), I(N), I(K), _stream()) == 0
+        sums = torch.full((lib.tm_gemv_f32_parts(N, K), M, N), float("nan"), device="cuda")
+        assert lib.tm_gemv_f32_mfma_split(_ptr(a), I(K), _ptr(w), _ptr(sums), I(M), I(N), I(K), _stream()) == 0
+        n = N // 8 * 4
+        both = torch.cat([w[:n], w[large - n:]])                # (up: the last rows, of which the smaller has the end)
+        act = torch.full((M, n), float("nan"), device="cuda")
+        assert lib.tm_gemv_f32_gate_up_silu(_ptr(a), I(K), _ptr(both), _ptr(act), I(M), I(n), I(K), _stream()) == 0
+        want = torch.nn.functional.silu(ref[:, :n]) * ref[:, large - n:]
+        assert ((act.double() - want).abs() <= _bound(K) * (1.1 * ref[:, large - n:].abs() + ref[:, :n].abs() + 1) + 2.0 ** -20 * want.abs()).all()
+        assert (out.double() - ref[:, :N]).abs().max() <= _bound(K)
+        outs.append(out[:, :small]), parts.append(sums[:, :, :small])
+    assert torch.equal(*outs) and parts[0].shape == parts[1].shape and torch.equal(*parts)
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("H,more,KVH,D,K", [(14, 28, 2, 64, 896), (5, 9, 1, 128, 1456)])
+def test_qkv_by_whole_lines_has_the_bits_of_a_load_a_step(H, more, KVH, D, K, M):
+    """The same query heads with so many beside them that the matrix is read by whole lines."""
+    a, w, _ = _operands(M, (more + 2 * KVH) * D, K, H)
+    bias = torch.randn((more + 2 * KVH) * D, generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")
+    angle = torch.rand(300, D // 2, generator=torch.Generator(device="cuda").manual_seed(2), device="cuda") * 6.28
+    cos, sin, pos = angle.cos(), angle.sin(), torch.arange(M, device="cuda", dtype=torch.int32) * 7
+    got = []
+    for heads in (H, more):
+        skip = (more - heads) * D
+        rows = torch.cat([torch.arange(heads * D), torch.arange(heads * D + skip, w.shape[0])]).cuda()
+        ww, bb = w[rows].contiguous(), bias[rows].contiguous()
+        q, k, v = torch.empty(M, heads * D, device="cuda"), torch.zeros(2, 16, KVH, D, device="cuda"), torch.zeros(2, KVH, D, 16, device="cuda")
+        slots = torch.arange(M, device="cuda", dtype=torch.int32)
+        assert library().tm_gemv_f32_qkv_rope(_ptr(a), I(K), _ptr(ww), _ptr(bb), _ptr(q), I(M), I(K), I(heads), I(KVH), I(D), _ptr(cos), _ptr(sin), _ptr(pos),
+                                              _ptr(slots), _ptr(k), _ptr(v), I(16), _stream()) == 0
+        got.append((q[:, :H * D], k, v))
+    assert 4 * K * (H + 2 * KVH) * D < 6656 * 1024 <= 4 * K * (more + 2 * KVH) * D
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
 def test_a_long_k_is_split():
     assert library().tm_gemv_f32_parts(896, 4864) == 4 and library().tm_gemv_f32_parts(896, 896) == 1
 

@@ -12,10 +12,11 @@
 // the rate of whole lines (a line costs it the same either way; 30 to 40 KB a us against 130 a block alone on its CU), so two steps are loaded
 // as a pair, 128 bytes of eight rows an instruction, and the lanes r and r + 8 exchange what belongs to the other, which is eight
 // instructions of the vector unit a pair. Up to eight rows of activations are one load a pair, and whole lines that
-// nobody reads again pass the caches by (non-temporal: the head 98 to 85 us, down 6.7 to 6.5). Against a load a step, cold matrices,
-// 1 / 8 / 16 rows, us: gate|up of the 0.5B shape 10.9 / 12.2 / 14.4 to 9.1 / 10.1 / 12.2, down 6.4 / 7.2 / 8.6 to 5.7 / 6.4 / 7.8, o
-// 4.7 / 5.5 / 6.4 to 4.5 / 5.3 / 6.2, q|k|v 5.4 / 6.2 / 7.2 to 5.3 / 6.0 / 7.0 (seven steps a wavefront: every other pair lies across two lines),
-// the head 120 / 129 / 141 to 84 / 86 / 99 (6.3 TB/s at 8 rows); 3,584 -> 2 x 18,944 103 / 128 / 159 to 85 / 101 / 127. The same bits.
+// nobody reads again pass the caches by (non-temporal: the head 98 to 85 us, down 6.7 to 6.5). Against a load a step, cold matrices, us: gate|up of the 0.5B
+// shape at 1 / 8 rows 11.2 / 12.7 to 9.4 / 10.5 and at 16 rows 16% less, down 6.7 to 6.0 at one row, 9% less at 16; the head 120 / 129 to 84 / 86 (6.3 TB/s at 8
+// rows), 3,584 -> 2 x 18,944 110 to 91 at one row. Matrices of less than 6.5 MB and rows of less than 384 k are latency, and the exchange comes on top of it (K
+// from 256 to 8,192, 6 MB, against a load a step: 1 and 8 rows 7% slower to 6% faster, 9 and 16 rows up to 11% slower and 4% on the mean; 7 MB 5% faster
+// on the mean at all, K of 256 5% slower): they keep a load a step (GM_LINES). The same bits either way.
 // Before that, a wavefront had 256 k of four rows, a lane 4 k each, and summed over the lanes by shuffles, 6 x 32 of them a wavefront:
 // 19.0 us a product of the 0.5B shape on average, with SiLU*up and rotation in kernels behind it.
 #include "common.h"
@@ -46,8 +47,8 @@ struct GemvArgs {
 
 // GROUP: steps of 16 k whose products meet in sums of their own before they join the running one. AHEAD: groups a wavefront asks for
 // at once: with one, a wavefront of the 0.5B shape waited for memory two times in a launch of 6 to 7 us (o 6.2 to 5.8, q|k|v 7.2 to 6.8).
-// OVER8: more than eight rows of activations.
-template <int EPI, int RT, int WAVES, int GROUP, int AHEAD, bool OVER8>
+// LINES: two steps as a pair of lines, else a load a step. OVER8: more than eight rows of activations (the same code where there are no lines).
+template <int EPI, int RT, int WAVES, int GROUP, int AHEAD, bool LINES, bool OVER8>
 __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArgs a) {
     static_assert(EPI == GM_PLAIN || RT == 1, "");
     __shared__ __align__(16) f32x4_t red[WAVES][RT][TM_WAVE];
@@ -75,18 +76,19 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     const int b0 = blockIdx.y * per_block, b1 = b0 + per_block < steps ? b0 + per_block : steps;
     const int per = (per_block + WAVES - 1) / WAVES;
     const int s0 = b0 + wave * per, s1 = s0 + per < b1 ? s0 + per : b1;
-    // rows r % 8 and 8 + r % 8 (rows beyond the matrix, the half or the input: its last one, never stored)
+    // rows r % 8 and 8 + r % 8, or row r (rows beyond the matrix, the half or the input: its last one, never stored)
+    constexpr int HALVES = LINES ? 2 : 1;
     const int r8 = r % 8, second = r / 8;
-    const float* pa[2];
-    const float* pw[RT][2];
+    const float* pa[HALVES];
+    const float* pw[RT][HALVES];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int row = r8 + 8 * h;
+    for (int h = 0; h < HALVES; ++h) {
+        const int row = LINES ? r8 + 8 * h : r;
         pa[h] = a.A + (size_t)(row < a.M ? row : a.M - 1) * a.lda + 4 * g;
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
             const int end = EPI == GM_SILU ? a.I : a.N, at = n0[t] + (EPI == GM_PLAIN ? row : r8);
-            const int n = (at < end ? at : end - 1) + (EPI != GM_PLAIN ? h * far : 0);
+            const int n = (at < end ? at : end - 1) + (EPI != GM_PLAIN ? (LINES ? h : second) * far : 0);
             pw[t][h] = a.W + (size_t)n * a.K + 4 * g;
         }
     }
@@ -108,16 +110,19 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
 #pragma unroll
     for (int t = 0; t < RT; ++t) sum[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     auto groups = [&](auto AT_ONCE, int s) {
-        constexpr int GROUPS = decltype(AT_ONCE)::value, PAIRS = (GROUP * GROUPS + 1) / 2;
-        f32x4_t w[RT][PAIRS][2], x[PAIRS][OVER8 ? 2 : 1];
+        constexpr int GROUPS = decltype(AT_ONCE)::value, LOADS = LINES ? (GROUP * GROUPS + 1) / 2 : GROUP * GROUPS;
+        f32x4_t w[RT][LOADS][HALVES], x[LOADS][LINES && OVER8 ? 2 : 1];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < PAIRS; ++i) {
-            const int step = s + 2 * i + second, at = 16 * (step < s1 ? step : s1 - 1);  // (no load under a test: beyond the end the last step again)
+        for (int i = 0; i < LOADS; ++i) {
+            const int step = LINES ? s + 2 * i + second : s + i, at = 16 * (step < s1 ? step : s1 - 1);  // (no load under a test: beyond the end the last step again)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
+            for (int h = 0; h < HALVES; ++h) {
 #pragma unroll
-                for (int t = 0; t < RT; ++t) w[t][i][h] = __builtin_nontemporal_load((const f32x4_t*)(pw[t][h] + at));
+                for (int t = 0; t < RT; ++t) {
+                    const f32x4_t* at_w = (const f32x4_t*)(pw[t][h] + at);
+                    w[t][i][h] = LINES ? __builtin_nontemporal_load(at_w) : *at_w;
+                }
                 if (h == 0 || OVER8) x[i][h] = *(const f32x4_t*)(pa[h] + at);
             }
         }
@@ -142,10 +147,16 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
 #pragma unroll
             for (int i = j * GROUP; i < (j + 1) * GROUP; ++i) {
                 if (s + i >= s1) break;
-                const f32x4_t xf = OVER8 ? line_pair_half(i % 2, x[i / 2][0], x[i / 2][OVER8 ? 1 : 0]) : i % 2 ? line_pair_turned(x[i / 2][0]) : x[i / 2][0];
-                f32x4_t wf[RT];
+                f32x4_t xf, wf[RT];
+                if constexpr (LINES) {
+                    xf = OVER8 ? line_pair_half(i % 2, x[i / 2][0], x[i / 2][OVER8 ? 1 : 0]) : i % 2 ? line_pair_turned(x[i / 2][0]) : x[i / 2][0];
 #pragma unroll
-                for (int t = 0; t < RT; ++t) wf[t] = line_pair_half(i % 2, w[t][i / 2][0], w[t][i / 2][1]);
+                    for (int t = 0; t < RT; ++t) wf[t] = line_pair_half(i % 2, w[t][i / 2][0], w[t][i / 2][1]);
+                } else {
+                    xf = x[i][0];
+#pragma unroll
+                    for (int t = 0; t < RT; ++t) wf[t] = w[t][i][0];
+                }
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -159,7 +170,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     // what is left when no AHEAD groups are is one group less (two tiles have no registers for the second loop: it takes the head from 98 to
     // 151 us at 16 rows, and what they ask for beyond the end is the last step again)
     int s = s0;
-    constexpr int LEAST = RT == 1 ? GROUP * (AHEAD - 1) : 0;
+    constexpr int LEAST = LINES && RT == 1 ? GROUP * (AHEAD - 1) : 0;
     for (; s + LEAST < s1; s += GROUP * AHEAD) groups(std::integral_constant<int, AHEAD>{}, s);
     if constexpr (LEAST > 0) {
         if (s < s1) groups(std::integral_constant<int, AHEAD - 1>{}, s);
@@ -244,22 +255,44 @@ extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, con
 // up to four rows two groups at a time and of more rows one (K cut into 32 to 56 steps a wavefront, one group / two, us: 18,944 -> 3,584, 1 / 4 / 8 /
 // 16 rows 50.5 / 43.6, 50.7 / 47.3, 52.4 / 54.4, 67.7 / 69.5; 5,632 -> 2,048 10.7 / 9.7, 10.8 / 10.1, 11.0 / 11.6, 13.1 / 14.3). One of the four
 // asks for two groups where it has them: a group at a time leaves half a pair's line, and gate|up of the 0.5B shape takes 12.2 us so for 10.2.
-template <int EPI, int RT, bool OVER8>
+// Of the products with a load a step (GM_LINES), more than three groups a wavefront are asked for one at a time whatever the rows are (2,048 -> 2,048 cut
+// into 16 steps a wavefront, 1 / 8 / 16 rows: two rounds of three groups 9.4 / 11.5 / 13.5 us, four of one 7.7 / 8.6 / 10.0).
+constexpr size_t GM_LINES = 6656 * 1024;
+constexpr int GM_LINES_K = 384;
+
+template <int EPI, int RT, bool LINES, bool OVER8>
 static void gm_launch_rows(const GemvArgs& a, int units, int split, hipStream_t stream) {
     const int steps = (a.K / 16 + split - 1) / split, per = (steps + 7) / 8;
+    const bool long_runs = LINES && per > 12 && a.M <= 4;
     const dim3 grid(units, split);
     if (units * split > 256) {
-        if (steps <= 4 * 7) gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1, OVER8><<<grid, 256, 0, stream>>>(a);
-        else gemv_mfma_f32_kernel<EPI, RT, 4, 7, 2, OVER8><<<grid, 256, 0, stream>>>(a);
-    } else if (per <= 4 || (per > 12 && a.M > 4)) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1, OVER8><<<grid, 512, 0, stream>>>(a);
-    else if (per <= 8 || per > 12) gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2, OVER8><<<grid, 512, 0, stream>>>(a);
-    else gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3, OVER8><<<grid, 512, 0, stream>>>(a);
+        if constexpr (LINES) {
+            if (steps > 4 * 7) {
+                gemv_mfma_f32_kernel<EPI, RT, 4, 7, 2, LINES, OVER8><<<grid, 256, 0, stream>>>(a);
+                return;
+            }
+        }
+        gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1, LINES, OVER8><<<grid, 256, 0, stream>>>(a);
+        return;
+    }
+    if constexpr (LINES || RT == 1) {                           // (two tiles without lines: K of less than 384)
+        if (per > 4 && (per <= 8 || long_runs)) {
+            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2, LINES, OVER8><<<grid, 512, 0, stream>>>(a);
+            return;
+        }
+        if (per > 8 && per <= 12) {
+            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3, LINES, OVER8><<<grid, 512, 0, stream>>>(a);
+            return;
+        }
+    }
+    gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1, LINES, OVER8><<<grid, 512, 0, stream>>>(a);
 }
 
 template <int EPI, int RT>
 static void gm_launch(const GemvArgs& a, int units, int split, hipStream_t stream) {
-    if (a.M > 8) gm_launch_rows<EPI, RT, true>(a, units, split, stream);
-    else gm_launch_rows<EPI, RT, false>(a, units, split, stream);
+    if ((size_t)a.N * a.K * 4 < GM_LINES || a.K < GM_LINES_K) gm_launch_rows<EPI, RT, false, false>(a, units, split, stream);
+    else if (a.M > 8) gm_launch_rows<EPI, RT, true, true>(a, units, split, stream);
+    else gm_launch_rows<EPI, RT, true, false>(a, units, split, stream);
 }
 
 extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,
