@@ -156,3 +156,11 @@ def test_a_captured_step_brings_what_an_eager_one_does():
     got, took = _brought(*SMALL, [300] * 4, [], graphs=True)
     runs = took["qkv_from_norm"]                                             # (layers of the runs that a capture makes)
     assert runs >= 3 and got == {"qkv": runs, "attention": 2 * runs, "gate_up": 5 * runs // 3}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,heads,requests,few", [(896, 14, 16, 1), (896, 14, 17, 0), (3200, 25, 8, 1), (3200, 25, 9, 0)])
+def test_which_heads_the_kernel_of_few_rows_takes(width, heads, requests, few):
+    """Beyond eight rows a narrow head with a long K is the library's."""
+    _, took = _brought(width, heads, 1, width // heads, 512, [20] * requests, [])
+    assert took.get("head_few", 0) == few

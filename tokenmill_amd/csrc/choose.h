@@ -68,6 +68,11 @@ constexpr int TM_SKINNY_MAX_ROWS = 64;
 // most rows the 32-bit matrix-vector product takes
 constexpr int TM_GEMV_F32_ROWS = 16;
 
+// Does the kernel for wide products of few bfloat16 rows (gemv_bf16.hip) take an output head from the library? Up to eight rows at every size that it has (from
+// 16,384 x 256 to 256,000 x 8,192 the library takes 0.98 to 2.2 times its time, 1.3 on the mean); with more, K of 8,192 is 10 to 20% slower (128,256 rows: 357 to 424 us),
+// and K from 3,584 to 5,120 up to 12% in heads of less than 65,536 (50,304 x 5,120: 95 to 107; 65,536 x 5,120 and 151,936 x 5,120 2 and 18% faster).
+inline bool tm_head_few(int M, int N, int K) { return M <= 8 || K <= 3072 || (N >= 65536 && K <= 5120); }
+
 // --- decode attention ---------------------------------------------------------------------------------
 constexpr int TM_DECODE_CHUNK = 256;        // keys per block of the split decode attention
 constexpr int TM_DECODE_F32_CHUNK = 128;    // the same in the 32-bit path, whose contexts are always split below that many pairs

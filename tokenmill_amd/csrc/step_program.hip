@@ -175,7 +175,7 @@ struct Products {
             return then_act(tm_gemm_nt_tiled(x, ldx, L.w, L.bias, L.bias_dtype, out, ldc, M, L.N, L.K, dtype, out_dtype, stream));
         }
         const bool skinny = skinny_ok(L, x, ldx, dtype);
-        if (L.library_first && !L.bias && !L.act && out_dtype == TM_F32 && tm_gemv_bf16_takes(x, ldx, L.w, out, ldc, M, L.N, L.K)) {
+        if (L.library_first && !L.bias && !L.act && out_dtype == TM_F32 && tm_head_few(M, L.N, L.K) && tm_gemv_bf16_takes(x, ldx, L.w, out, ldc, M, L.N, L.K)) {
             if (head_few) ++*head_few;
             return tm_gemv_bf16(x, ldx, L.w, (float*)out, ldc, M, L.N, L.K, stream);
         }
