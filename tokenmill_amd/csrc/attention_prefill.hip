@@ -24,16 +24,34 @@
 
 #include <algorithm>
 
+// A block of 32 keys as a wavefront holds it between asking for it and using it. Row rho of operand tile t is key 8 (rho / 4) + 4 t + rho % 4,
+// so that the lane which holds rows 4 g .. 4 g + 3 of both tiles of the scores has the eight keys 8 g .. 8 g + 7 of a row of V^T in one piece.
+//
+// What bounds a long prompt is the address unit of a CU, beside its vector units: it takes 64 bytes a cycle where four neighbouring lanes ask for a
+// piece of one line, and one lane a cycle where they are in different keys, as the lanes of a score operand are (a key a lane). So keys are
+// loaded as whole rows, eight lanes a row of 64, and change lanes through LDS (attend_block), and values come 16 bytes a lane. At 8,000 tokens of the 0.5B
+// shape the first-level caches had 112 million accesses in 443,000 cycles, one a cycle and CU, and have 43 million in 385,000; keys, 77 / 512 /
+// 2,048 / 8,000 tokens, us a launch 5.0 / 8.5 / 25.7 / 212 to 4.6 / 6.9 / 23.6 / 186. (Keys by loads of half rows that lanes exchange in
+// registers, which ask for as many places: 26.1 and 215. The next block's keys through LDS behind this block's last score products, a
+// wait less: spills, 27.0 and 197.)
 template <int D>
 struct KVBlock {
-    PFrag k[2][D / 32];     // [16-key tile][d chunk]
-    u32x2_t v[D / 16][2];   // [d tile][16-key tile]: 4 keys each
+    static constexpr int PIECES = D / 8, ROW = 2 * D + 16, TILE = 16 * ROW + 128;       // 16-byte pieces of a key; bytes of a key and of a tile in LDS
+    u32x4_t k[2][D / 32];   // [16 keys][c]: piece 64 c + lane of the keys as they lie
+    PFrag v[D / 16];        // [d tile]: keys 8 g .. 8 g + 7 of row d = r
 };
 
+// Floats of LDS that a wavefront has: its partials of all heads, and before that a block's keys.
+template <int D, int HPW>
+constexpr int wave_floats() { return HPW * 16 * (D + 4) > KVBlock<D>::TILE / 2 ? HPW * 16 * (D + 4) : KVBlock<D>::TILE / 2; }
+
 // What a lane adds to a tile's (wave-uniform) base address: constant for the whole kernel.
+template <int D>
 struct LaneOffsets {
-    uint32_t k;             // bytes: key r of the tile, d = 8 g
-    uint32_t v;             // bytes: d = r, keys 4 g .. 4 g + 3 of the tile
+    uint32_t k[D / 32];     // bytes: piece 64 c + lane of the tile's keys
+    uint32_t v;             // bytes: d = r, keys 8 (g % 2) .. + 7 of tile g / 2
+    uint32_t turn[2][D / 32];   // bytes in LDS: where they go
+    uint32_t row;           // bytes in LDS: piece g of row r
 };
 
 // A raw buffer descriptor over memory that starts at a wave-uniform address: loads through it take
@@ -74,81 +92,99 @@ __device__ __forceinline__ TilePlaces lane_pages(int kb, const BlockWalk& walk, 
 // Loads one block of 32 keys (two tiles of 16); slot = which of the 32 blocks held in `places`.
 template <int D>
 __device__ __forceinline__ void load_kv_block(KVBlock<D>& blk, const TilePlaces& places, int slot, const bf16_t* __restrict__ k_pool,
-                                              const bf16_t* __restrict__ v_pool, int page_shift, LaneOffsets off) {
+                                              const bf16_t* __restrict__ v_pool, int page_shift, const LaneOffsets<D>& off) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const uint32_t k_at = __builtin_amdgcn_readlane(places.k, 2 * slot + t), v_at = __builtin_amdgcn_readlane(places.v, 2 * slot + t);
+        const uint32_t k_at = __builtin_amdgcn_readlane(places.k, 2 * slot + t);
         const __amdgpu_buffer_rsrc_t kbuf = uniform_buffer((const char*)k_pool + ((uint64_t)k_at << 6));
-        const __amdgpu_buffer_rsrc_t vbuf = uniform_buffer((const char*)v_pool + ((uint64_t)v_at << 5));
 #pragma unroll
-        for (int c = 0; c < D / 32; ++c)
-            blk.k[t][c].u = __builtin_amdgcn_raw_buffer_load_b128(kbuf, off.k, 64 * c, 0);
-#pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt)
-            blk.v[dt][t] = __builtin_amdgcn_raw_buffer_load_b64(vbuf, off.v, (32 * dt) << page_shift, 0);
+        for (int c = 0; c < D / 32; ++c) blk.k[t][c] = __builtin_amdgcn_raw_buffer_load_b128(kbuf, off.k[c], 0, 0);
     }
+    const uint32_t v0 = __builtin_amdgcn_readlane(places.v, 2 * slot), v1 = __builtin_amdgcn_readlane(places.v, 2 * slot + 1);
+    const char* vp = (const char*)v_pool + ((uint64_t)(threadIdx.x & 32 ? v1 : v0) << 5) + off.v;
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt) blk.v[dt].u = *(const u32x4_t*)(vp + ((size_t)(32 * dt) << page_shift));
 }
 
 // One block of 32 keys against the wavefront's heads.
 template <int D, int HPW, bool CAP>
-__device__ __forceinline__ void attend_block(KVBlock<D>& blk, HeadState<D, HPW>& st, const PFrag (&qf)[HPW][D / 32],
+__device__ __forceinline__ void attend_block(KVBlock<D>& blk, unsigned char* turn, const LaneOffsets<D>& off, HeadState<D, HPW>& st, const PFrag (&qf)[HPW][D / 32],
                                              int key0, int nh, const TileView& tv, int g, float scale_log2, float cap_in, float cap_out) {
     constexpr int NDC = D / 32, NDT = D / 16;
     // values of keys nobody may see (beyond the newest key, or behind every window: see lane_pages) can hold anything: clear them
     if (key0 + 31 > tv.last_key || key0 < tv.first_key) {
+        uint32_t seen[4];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int k0 = key0 + 16 * t + 4 * g;
-            const uint32_t keep0 = (tv.seen(k0) ? 0x0000ffffu : 0u) | (tv.seen(k0 + 1) ? 0xffff0000u : 0u);
-            const uint32_t keep1 = (tv.seen(k0 + 2) ? 0x0000ffffu : 0u) | (tv.seen(k0 + 3) ? 0xffff0000u : 0u);
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) {
-                blk.v[dt][t][0] &= keep0;
-                blk.v[dt][t][1] &= keep1;
-            }
+        for (int w = 0; w < 4; ++w) {
+            const int k0 = key0 + 8 * g + 2 * w;
+            seen[w] = (tv.seen(k0) ? 0x0000ffffu : 0u) | (tv.seen(k0 + 1) ? 0xffff0000u : 0u);
         }
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) blk.v[dt].u[w] &= seen[w];
     }
+    // the keys change lanes: whole rows as they were loaded, a row a lane as the matrix unit takes them (rows 16 bytes more than their values
+    // apart meet no bank twice)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int c = 0; c < NDC; ++c) *(u32x4_t*)(turn + off.turn[t][c]) = blk.k[t][c];
+    // (a wavefront's LDS instructions are done in their order; this holds the compiler to it)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    PFrag kf[2][NDC];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int c = 0; c < NDC; ++c) kf[t][c].u = *(const u32x4_t*)(turn + off.row + t * KVBlock<D>::TILE + 64 * c);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     // does any (query, key) pair of this block fall outside the causal / window limits?
     const bool edge = (key0 + 31 > tv.pos0) || (key0 < tv.last_lo);
-    // all score products first: the matrix unit works on the next head's while the vector unit
-    // does the softmax of this one
-    f32x4_t sc[HPW][2];
+    // the score products of two heads first: the matrix unit works on the next head's while the vector unit does the softmax of this
+    // one. (Of all four at once the registers do not hold the scores beside a block's keys in both orders.)
+    auto heads = [&](auto FIRST, auto COUNT) {
+        constexpr int h0 = decltype(FIRST)::value, AT_ONCE = decltype(COUNT)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4_t sc[AT_ONCE][2];
 #pragma unroll
-    for (int hh = 0; hh < HPW; ++hh) {
-        if (hh >= nh) continue;                                  // wave-uniform
+        for (int j = 0; j < AT_ONCE; ++j)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < 2; ++t) {
+                f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int c = 0; c < NDC; ++c)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.k[t][c].b, qf[hh][c].b, acc, 0, 0, 0);
-            // capped scores: cap * tanh(score * scale / cap), kept in units of 1 / scale like the plain ones
-            if constexpr (CAP) {
+                for (int c = 0; c < NDC; ++c)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][c].b, qf[h0 + j][c].b, acc, 0, 0, 0);
+                // capped scores: cap * tanh(score * scale / cap), kept in units of 1 / scale like the plain ones
+                if constexpr (CAP) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[i] = cap_out * tanh_fast(acc[i] * cap_in);
+                    for (int i = 0; i < 4; ++i) acc[i] = cap_out * tanh_fast(acc[i] * cap_in);
+                }
+                sc[j][t] = acc;
             }
-            sc[hh][t] = acc;
+        if (edge) {                                              // (which keys a column sees is worked out once for both heads)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int kj = key0 + 8 * g + 4 * t + i;
+                    const bool mine = (kj <= tv.my_pos) & ((kj >= tv.my_lo) | (kj < tv.keep));
+#pragma unroll
+                    for (int j = 0; j < AT_ONCE; ++j) sc[j][t][i] = mine ? sc[j][t][i] : -INFINITY;
+                }
         }
-    }
-    if (edge) {                                                  // (which keys a column sees is worked out once for all heads)
+        // this lane's largest scores of the block (scale > 0: the maximum commutes with it)
+        float lm[AT_ONCE];
+        bool grows = false;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int kj = key0 + 16 * t + 4 * g + i;
-                const bool mine = (kj <= tv.my_pos) & ((kj >= tv.my_lo) | (kj < tv.keep));
-#pragma unroll
-                for (int hh = 0; hh < HPW; ++hh) sc[hh][t][i] = mine ? sc[hh][t][i] : -INFINITY;
-            }
-    }
-#pragma unroll
-    for (int hh = 0; hh < HPW; ++hh) {
-        if (hh >= nh) continue;                                  // wave-uniform
-        // this lane's largest score of the block (scale > 0: the maximum commutes with it)
-        float lm = max3(-INFINITY, sc[hh][0][0], sc[hh][0][1]);
-        lm = max3(lm, sc[hh][0][2], sc[hh][0][3]);
-        lm = max3(lm, sc[hh][1][0], sc[hh][1][1]);
-        lm = max3(lm, sc[hh][1][2], sc[hh][1][3]);
+        for (int j = 0; j < AT_ONCE; ++j) {
+            lm[j] = max3(-INFINITY, sc[j][0][0], sc[j][0][1]);
+            lm[j] = max3(lm[j], sc[j][0][2], sc[j][0][3]);
+            lm[j] = max3(lm[j], sc[j][1][0], sc[j][1][1]);
+            lm[j] = max3(lm[j], sc[j][1][2], sc[j][1][3]);
+            grows |= lm[j] * scale_log2 > st.m[h0 + j] + PF_SLACK;   // (true for a column that has seen no key: m = -inf)
+        }
         // The running reference m of a column moves only when the block's maximum exceeds it by more
         // than PF_SLACK (in units of log2): until then the weights are exp2(s - m) <= 2^PF_SLACK instead of
         // <= 1, which changes nothing but their common scale (it cancels against the sum), and the
@@ -157,36 +193,53 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, HeadState<D, HPW>&
         // does not depend on the other queries of its tile. Whether any column moves is asked of the lanes'
         // own maxima first (a column's maximum exceeds the limit exactly when one of its four lanes' does), so
         // the exchange between the lanes of a column is as rare as the rescaling.
-        if (__any(lm * scale_log2 > st.m[hh] + PF_SLACK)) {          // (true for a column that has seen no key: m = -inf)
-            const float bm = column_max(lm) * scale_log2;
-            const bool grow = bm > st.m[hh] + PF_SLACK;
-            const float m_new = grow ? bm : st.m[hh];
-            const float corr = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(st.m[hh] - m_new);
-            st.m[hh] = m_new;
-            st.l[hh] *= corr;
+        if (__any(grows)) {
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
+            for (int j = 0; j < AT_ONCE; ++j) {
+                const int hh = h0 + j;
+                const float bm = column_max(lm[j]) * scale_log2;
+                const bool grow = bm > st.m[hh] + PF_SLACK;
+                const float m_new = grow ? bm : st.m[hh];
+                const float corr = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(st.m[hh] - m_new);
+                st.m[hh] = m_new;
+                st.l[hh] *= corr;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) st.o[hh][dt][i] *= corr;
-        }
-        // a column that has seen no key yet (m = -inf) gets zeros: exp2(-inf - 0)
-        const float neg_m = (st.m[hh] == -INFINITY) ? 0.f : -st.m[hh];
-        float pr[2][4];
+                for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                pr[t][i] = __builtin_amdgcn_exp2f(fmaf(sc[hh][t][i], scale_log2, neg_m));
-                st.l[hh] += pr[t][i];
+                    for (int i = 0; i < 4; ++i) st.o[hh][dt][i] *= corr;
             }
-        PFrag pt;
-        pt.u = u32x4_t{pk_bf16(pr[0][0], pr[0][1]), pk_bf16(pr[0][2], pr[0][3]), pk_bf16(pr[1][0], pr[1][1]),
-                       pk_bf16(pr[1][2], pr[1][3])};
+        }
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
-            PFrag vf;
-            vf.u = u32x4_t{blk.v[dt][0][0], blk.v[dt][0][1], blk.v[dt][1][0], blk.v[dt][1][1]};
-            st.o[hh][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.b, pt.b, st.o[hh][dt], 0, 0, 0);
+        for (int j = 0; j < AT_ONCE; ++j) {
+            const int hh = h0 + j;
+            // a column that has seen no key yet (m = -inf) gets zeros: exp2(-inf - 0)
+            const float neg_m = (st.m[hh] == -INFINITY) ? 0.f : -st.m[hh];
+            float pr[2][4];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    pr[t][i] = __builtin_amdgcn_exp2f(fmaf(sc[j][t][i], scale_log2, neg_m));
+                    st.l[hh] += pr[t][i];
+                }
+            PFrag pt;
+            pt.u = u32x4_t{pk_bf16(pr[0][0], pr[0][1]), pk_bf16(pr[0][2], pr[0][3]), pk_bf16(pr[1][0], pr[1][1]),
+                           pk_bf16(pr[1][2], pr[1][3])};
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+                st.o[hh][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk.v[dt].b, pt.b, st.o[hh][dt], 0, 0, 0);
+            }
+        }
+    };
+    using std::integral_constant;
+    if constexpr (HPW == 1) {
+        heads(integral_constant<int, 0>{}, integral_constant<int, 1>{});
+    } else {
+        if (nh >= 2) heads(integral_constant<int, 0>{}, integral_constant<int, 2>{});        // (nh is the same in every lane)
+        else heads(integral_constant<int, 0>{}, integral_constant<int, 1>{});
+        if constexpr (HPW > 2) {
+            if (nh >= 4) heads(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+            else if (nh == 3) heads(integral_constant<int, 2>{}, integral_constant<int, 1>{});
         }
     }
 }
@@ -229,7 +282,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     // the wavefronts' partials of all heads: rows of d four floats apart from a multiple of 64, so that 16 lanes of a store or load
     // of 16 bytes meet no bank twice
     __shared__ float s_m[KS][HPW][16], s_l[KS][HPW][16];
-    extern __shared__ __align__(16) float s_o[];                     // [KS][HPW][16][D + 4]
+    extern __shared__ __align__(16) float s_o[];                     // [KS][wave_floats]: [HPW][16][D + 4]
     int layer = blockIdx.z;
     if constexpr (DECODES) {
         if (layer < decodes.layers) {
@@ -244,7 +297,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     if constexpr (AHEAD) {
         if (layer) return tm_bring_ahead(ahead, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), KS);
     }
-    auto partial_at = [&](int w, int hh, int col, int d) { return s_o + (size_t)((w * HPW + hh) * 16 + col) * (D + 4) + d; };
+    auto partial_at = [&](int w, int hh, int col, int d) { return s_o + w * wave_floats<D, HPW>() + (hh * 16 + col) * (D + 4) + d; };
     // the wavefront index in a scalar register: everything derived from it (its key blocks, their
     // pages, the branches on them) stays wave-uniform
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TM_WAVE);
@@ -254,9 +307,19 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     const int kvh = blockIdx.y / splits, split = blockIdx.y % splits;
     const int h0 = kvh * G + split * HPW;
     const int nh = (G - split * HPW) < HPW ? (G - split * HPW) : HPW;
-    LaneOffsets off;
-    off.k = (uint32_t)(((size_t)r * KVH * D + 8 * g) * sizeof(bf16_t));
-    off.v = (uint32_t)((((size_t)r << page_shift) + 4 * g) * sizeof(bf16_t));
+    LaneOffsets<D> off;
+    using Block = KVBlock<D>;
+#pragma unroll
+    for (int c = 0; c < NDC; ++c) {
+        const int key = (64 * c + lane) / Block::PIECES, piece = (64 * c + lane) % Block::PIECES;
+        off.k[c] = (uint32_t)(((size_t)key * KVH * D + 8 * piece) * sizeof(bf16_t));
+#pragma unroll
+        for (int t = 0; t < 2; ++t)                                  // key 16 t + key is row 4 (. / 8) + . % 4 of tile . / 4 % 2
+            off.turn[t][c] = (uint32_t)((key / 4 % 2) * Block::TILE + (8 * t + 4 * (key / 8) + key % 4) * Block::ROW + 16 * piece);
+    }
+    off.v = (uint32_t)((((size_t)r << page_shift) + 8 * (g % 2)) * sizeof(bf16_t));
+    off.row = (uint32_t)(r * Block::ROW + 16 * g);
+    unsigned char* turn = (unsigned char*)partial_at(wave, 0, 0, 0);         // (the place of this wavefront's partials, which are stored behind the last block)
     const int other = n_tiles - 1 - (int)blockIdx.x;
     const int n_mine = (pair && other > (int)blockIdx.x) ? 2 : 1;
 
@@ -314,7 +377,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
                 slot = -1;
             }
             load_kv_block<D>(bb, pages, slot + 1, k_pool, v_pool, page_shift, off);
-            attend_block<D, HPW, CAP>(ba, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
+            attend_block<D, HPW, CAP>(ba, turn, off, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
             kb = walk.at<KS>(kb, kb + KS);
             ++slot;
             if (kb > kb1) break;
@@ -323,7 +386,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
                 slot = -1;
             }
             load_kv_block<D>(ba, pages, slot + 1, k_pool, v_pool, page_shift, off);
-            attend_block<D, HPW, CAP>(bb, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
+            attend_block<D, HPW, CAP>(bb, turn, off, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
             kb = walk.at<KS>(kb, kb + KS);
             ++slot;
         }
@@ -404,7 +467,7 @@ static int launch_split_keys(const void* q, int q_stride, void* out, int out_str
     // fold the table in two once the folded launch still gives every CU a block
     const int pair = (long long)(n_tiles / 2) * KVH * splits >= 256 ? 1 : 0;
     dim3 grid(pair ? (n_tiles + 1) / 2 : n_tiles, KVH * splits);
-    constexpr int lds = KS * HPW * 16 * (D + 4) * (int)sizeof(float);          // at most 139,264 bytes
+    constexpr int lds = KS * wave_floats<D, HPW>() * (int)sizeof(float);          // at most 139,264 bytes
     const long long layer = (long long)grid.x * grid.y;
     const int pairs = beside ? beside->n * KVH : 0, front = beside ? (int)((pairs + layer - 1) / layer) : 0;
     const bool far = layer + pairs >= 256;                           // (more blocks than CUs: none to spare)
