@@ -1114,6 +1114,25 @@ def test_stream_linear_with_k_split_over_blocks_and_the_norm_that_adds_the_parts
     assert torch.equal(o3, o1[pick.long()]) and torch.equal(r3.cpu(), resid)
 
 
+@pytest.mark.parametrize("units,ks,per", [(2, 8, 5), (2, 8, 6), (2, 8, 9), (2, 8, 12), (2, 8, 24), (2, 8, 25), (258, 4, 4), (258, 4, 5),
+                                          (258, 4, 9), (513, 2, 8), (770, 2, 9), (1026, 2, 6), (1300, 2, 13), (1540, 2, 7)])
+def test_stream_linear_by_rounds_of_four_and_of_eight(ops, units, ks, per):
+    """How many k-steps a round has hangs on the number of tokens and on the k-steps a wavefront has (`per`): every
+    number of token tiles, at the lengths where the choice turns, with one block's share of K ending within a k-step.
+    The order of a row's sum does not hang on it: the same bits in every call."""
+    torch.manual_seed(27)
+    N, K = 32 * units - 3, 32 * ks * per - 24
+    a, w = torch.randn(64, K).bfloat16(), (torch.randn(N, K) * 0.05).bfloat16()
+    Wp = ops.pack_weight(w.to(DEV), 16)
+    da = a.to(DEV)
+    outs = [ops.stream_linear(da[:M], Wp, None, torch.full((M, N), 7.0, device=DEV)) for M in (64, 48, 33, 32, 17, 16, 1)]
+    for out in outs[1:]:
+        assert torch.equal(out, outs[0][:out.shape[0]])
+    # products of two bfloat16 are exact in 32 bits: what is left is one rounding of at most the sum of the magnitudes an addition
+    a64, w64 = a.double().to(DEV), w.double().to(DEV)
+    assert ((outs[0].double() - a64 @ w64.t()).abs() <= K * 2.0 ** -24 * (a64.abs() @ w64.abs().t())).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(8, 896, 4864), (1, 64, 128), (40, 200, 120), (64, 896, 896)])
 def test_gemm_skinny_adds_into_the_residual(ops, M, N, K):
     torch.manual_seed(15)

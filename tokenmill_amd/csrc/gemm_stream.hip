@@ -10,12 +10,12 @@
 // 64 tokens.
 //
 // A block has KS x US wavefronts: US units side by side, each unit's K split over KS wavefronts. The block walks K
-// in rounds of ST_KCH k-steps per wavefront. The activations of a round (for each of the KS ranges of K a window
-// of ST_KCH k-steps, all rows) are read from the cache in whole lines by all threads together, go through LDS,
+// in rounds of KCH k-steps (4 or 8) per wavefront. The activations of a round (for each of the KS ranges of K a window
+// of KCH k-steps, all rows) are read from the cache in whole lines by all threads together, go through LDS,
 // and serve all US units from there: the cache sees them once a block, not once a wavefront, and a wavefront
 // reads them in the matrix unit's layout without asking the cache for half lines. The matrix streams from HBM
 // straight into registers: as soon as a k-step's products are issued its registers are asked for the same
-// k-step of the next round, so every wavefront keeps ST_KCH k-steps of two strips in flight while it multiplies.
+// k-step of the next round, so every wavefront keeps ST_WD k-steps of two strips in flight while it multiplies.
 // Every load is without a condition, at an address clamped into valid memory. At the end the KS partial sums of
 // a unit are added through LDS in wavefront order, tile by tile, and wavefront t mod KS of the unit does the
 // epilogue of row tile t.
@@ -32,10 +32,9 @@
 #define ST_EPI_QKV 0
 #define ST_EPI_SILU 1
 #define ST_EPI_PLAIN 2
-#define ST_KCH 4            // k-steps of a round, per wavefront
-#define ST_WD 8             // k-steps of the matrix a wavefront has in registers or on their way (a multiple of ST_KCH)
 // the matrix is read once and never again: loads that do not displace the activations in the caches
 #define ST_WLOAD(p) __builtin_nontemporal_load((const u32x4_t*)(p))
+#define ST_WD 8             // k-steps of the matrix a wavefront has in registers or on their way: one round of eight or two of four
 #define ST_XPAD 16          // padding of an LDS row of activations, in elements: rows 288 bytes apart, which the operand loads (lane (r, g): 16 bytes of row r at piece g) read free of bank conflicts; with 8 (272 bytes) they take twice as long
 
 struct StreamArgs {
@@ -90,18 +89,19 @@ __device__ __forceinline__ StreamUnit stream_unit_of(const StreamArgs& a, int u,
 }
 
 // Bytes of LDS a block needs: the activations of a round, or (whichever is more) the partial sums of two tiles.
-__host__ __device__ constexpr int stream_lds_bytes(int NT, int KS, int US) {
-    const int window = KS * NT * 16 * (ST_KCH * 32 + ST_XPAD) * 2;
+__host__ __device__ constexpr int stream_lds_bytes(int NT, int KS, int US, int KCH) {
+    const int window = KS * NT * 16 * (KCH * 32 + ST_XPAD) * 2;
     const int sums = 2 * KS * US * 2 * 64 * 4 * 4;
     return window > sums ? window : sums;
 }
 
-// NT: 16-token tiles of the activations (1..4). KS: wavefronts that split a unit's K. US: units of a block.
-template <int EPI, int NT, int KS, int US>
+// NT: 16-token tiles of the activations (1..4). KS: wavefronts that split a unit's K. US: units of a block. KCH: k-steps
+// of a round, per wavefront (4 or 8).
+template <int EPI, int NT, int KS, int US, int KCH>
 __global__ __launch_bounds__(64 * KS * US) void gemm_stream_kernel(const StreamArgs a, const int n_units) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     constexpr int WAVES = KS * US, THREADS = 64 * WAVES;
-    constexpr int XROW = ST_KCH * 32 + ST_XPAD;                      // elements of an LDS row: a window of K, padded
+    constexpr int XROW = KCH * 32 + ST_XPAD;                         // elements of an LDS row: a window of K, padded
     constexpr int ROWS_X = NT * 16;
     bf16_t* xs = (bf16_t*)smem_raw;                                  // [KS][ROWS_X][XROW]
     const FusedArgs& f = a.f;
@@ -135,9 +135,9 @@ __global__ __launch_bounds__(64 * KS * US) void gemm_stream_kernel(const StreamA
     const bf16_t* wB = f.W + (size_t)sB * ksteps * frag + ((g << shift) + rr) * 8;
     auto w_at = [&](int ks) { return (size_t)(ks < last_ks ? ks : last_ks) * frag; };
 
-    // The activations of a round: KS windows of ST_KCH k-steps (64 bytes a row each), all rows. Thread i takes the
+    // The activations of a round: KS windows of KCH k-steps (64 bytes a row each), all rows. Thread i takes the
     // 16-byte pieces i, i + THREADS, ...: consecutive lanes read one row's window as a run, whole lines at a time.
-    constexpr int PIECES_ROW = ST_KCH * 4;
+    constexpr int PIECES_ROW = KCH * 4;
     constexpr int PIECES = KS * ROWS_X * PIECES_ROW;
     constexpr int XL = (PIECES + THREADS - 1) / THREADS;
     const int k_end = K;
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(64 * KS * US) void gemm_stream_kernel(const StreamA
             const int p = threadIdx.x + i * THREADS;
             const int win = p / (ROWS_X * PIECES_ROW), in = p % (ROWS_X * PIECES_ROW);
             const int row = in / PIECES_ROW, piece = in % PIECES_ROW;
-            int k = (k_begin + (win < KS ? win : KS - 1) * per + round * ST_KCH) * 32 + piece * 8;
+            int k = (k_begin + (win < KS ? win : KS - 1) * per + round * KCH) * 32 + piece * 8;
             k = k + 8 <= k_end ? k : 0;                               // beyond the row: a piece that exists (zeroed when stored)
             xv[i] = *(const u32x4_t*)(f.X + (size_t)(tok0 + (row < M ? row : M - 1)) * f.ldx + k);
         }
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(64 * KS * US) void gemm_stream_kernel(const StreamA
             if (PIECES % THREADS == 0 || p < PIECES) {
                 const int win = p / (ROWS_X * PIECES_ROW), in = p % (ROWS_X * PIECES_ROW);
                 const int row = in / PIECES_ROW, piece = in % PIECES_ROW;
-                const int k = (k_begin + win * per + round * ST_KCH) * 32 + piece * 8;
+                const int k = (k_begin + win * per + round * KCH) * 32 + piece * 8;
                 // beyond K the packed matrix holds zeros: the activations there must be zeros too (0 * anything stays 0)
                 const u32x4_t v = k + 8 <= k_end ? xv[i] : u32x4_t{0, 0, 0, 0};
                 *(u32x4_t*)(xs + ((size_t)win * ROWS_X + row) * XROW + piece * 8) = v;
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(64 * KS * US) void gemm_stream_kernel(const StreamA
         accA[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         accB[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-    const int rounds = (per + ST_KCH - 1) / ST_KCH;                  // the same for every wavefront of the block
+    const int rounds = (per + KCH - 1) / KCH;                        // the same for every wavefront of the block
     // What the q|k|v epilogue needs from memory, where a wavefront owns one token tile (tile kw): the token's position,
     // cache slot and the bias are asked for before anything else (loads come back in the order they were issued, so
     // these are not behind the matrix), the rotary row, whose address hangs on the position, after the first round.
@@ -205,9 +205,9 @@ __global__ __launch_bounds__(64 * KS * US) void gemm_stream_kernel(const StreamA
         fb[j].u = ST_WLOAD(wB + w_at(ks0 + j));
     }
     const bf16_t* x_mine = xs + ((size_t)kw * ROWS_X + r) * XROW + 8 * g;
-    for (int round0 = 0; round0 < rounds; round0 += ST_WD / ST_KCH) {
+    for (int round0 = 0; round0 < rounds; round0 += ST_WD / KCH) {
 #pragma unroll
-        for (int sr = 0; sr < ST_WD / ST_KCH; ++sr) {
+        for (int sr = 0; sr < ST_WD / KCH; ++sr) {
             const int round = round0 + sr;
             if (round < rounds) {                                     // the same for the whole block
                 store_x(round);
@@ -220,10 +220,10 @@ __global__ __launch_bounds__(64 * KS * US) void gemm_stream_kernel(const StreamA
                         pre_sn = *(const f32x4_t*)(f.sin_t + at);
                     }
                 }
-                const int base = ks0 + round * ST_KCH;
+                const int base = ks0 + round * KCH;
 #pragma unroll
-                for (int j = 0; j < ST_KCH; ++j) {
-                    const int slot = sr * ST_KCH + j;                 // a compile-time register index
+                for (int j = 0; j < KCH; ++j) {
+                    const int slot = sr * KCH + j;                    // a compile-time register index
                     if (base + j < ks1) {                             // the same for all lanes of the wavefront
 #pragma unroll
                         for (int t = 0; t < NT; ++t) {
@@ -434,19 +434,41 @@ int stream_gate_up_units(int I) {
     return us;
 }
 
-template <int EPI, int NT, int KS, int US>
-static int launch_stream_config(const StreamArgs& a, int n_units, int kparts, int row_parts, hipStream_t stream) {
-    constexpr int lds = stream_lds_bytes(NT, KS, US);
+template <int EPI, int NT, int KS, int US, int KCH>
+static int launch_stream_rounds(const StreamArgs& a, int n_units, int kparts, int row_parts, hipStream_t stream) {
+    constexpr int lds = stream_lds_bytes(NT, KS, US, KCH);
     static bool raised = false;
     if (lds > 48 * 1024 && !raised) {
-        if (hipFuncSetAttribute((const void*)gemm_stream_kernel<EPI, NT, KS, US>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute((const void*)gemm_stream_kernel<EPI, NT, KS, US, KCH>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 lds) != hipSuccess)
             return TM_ERR_LAUNCH;
         raised = true;
     }
-    gemm_stream_kernel<EPI, NT, KS, US><<<dim3((n_units + US - 1) / US, kparts, row_parts), 64 * KS * US, lds, stream>>>(a, n_units);
+    gemm_stream_kernel<EPI, NT, KS, US, KCH><<<dim3((n_units + US - 1) / US, kparts, row_parts), 64 * KS * US, lds, stream>>>(a, n_units);
     TM_CHECK_LAUNCH();
     return TM_OK;
+}
+
+// Four k-steps a round or eight. Both add a wavefront's products in the order of K, so the results are the same bits;
+// the matrix is eight k-steps ahead with either. Eight halve the rounds, and with them the two meetings of the block
+// and the turn of the activations through LDS that each costs while nothing new is asked of HBM, but the last round
+// turns a window that may be nearly empty, and the first products wait for twice the activations. Eight pay where a
+// wavefront's last eight are at least about half used or lost among many. They need KS x NT x 8.7 KB of LDS and some
+// registers more, which they have up to 8 wavefronts a block, or with one tile of tokens. Measured on an MI355X,
+// rounds of four / eight (us): 8 rows, gate|up 7B 51.6 / 47.6, 4,096 -> 2 x 14,336 46.7 / 44.5, 2,048 -> 2 x 11,008
+// 23.4 / 18.1, 1,536 -> 2 x 8,960 18.4 / 13.3; q|k|v 7B 10.9 / 10.5; 7B down 26.9 / 25.4, 32B down 52.7 / 47.5; 64 rows,
+// 4,096 -> 2 x 14,336 51.9 / 49.2, 7B down 33.5 / 32.0. Where they lose: a wavefront with 4 or 5 k-steps at 8 rows
+// (q|k|v 0.5B 4.96 / 5.35, 0.5B down 6.94 / 7.12), with 9 to 12 at 32 rows (11,008 -> 2,048 12.9 / 13.1; 17 to 20 at
+// 8 x 1: q|k|v 32B 20.2 / 20.6), ten wavefronts at 64 rows (gate|up 7B 54.0 / 54.6; sixteen: 104 / 107), and where two
+// blocks with two tiles share a CU (gate|up 0.5B 64 rows 11.5 / 13.9).
+template <int EPI, int NT, int KS, int US>
+static int launch_stream_config(const StreamArgs& a, int n_units, int kparts, int row_parts, hipStream_t stream) {
+    if constexpr (NT == 1 || (KS * US <= 8 && KS * NT <= 16)) {
+        const int ksteps = (a.f.K + 31) / 32, per = ((ksteps + kparts - 1) / kparts + KS - 1) / KS;
+        const bool pays = NT == 1 ? per > 8 || (per + 7) % 8 >= 5 : per > 24 || (per + 7) % 8 >= 4;
+        if (row_parts == 1 && pays) return launch_stream_rounds<EPI, NT, KS, US, 8>(a, n_units, kparts, row_parts, stream);
+    }
+    return launch_stream_rounds<EPI, NT, KS, US, 4>(a, n_units, kparts, row_parts, stream);
 }
 
 template <int EPI, int NT>
