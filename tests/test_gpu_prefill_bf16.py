@@ -38,3 +38,33 @@ def test_a_heads_bits_do_not_depend_on_the_heads_beside_it(D, n, window, softcap
     want = torch.einsum("hqk,kd->qhd", s.softmax(-1), values)
     # weights and results are rounded to 8 bits: 2^-9 of the largest value each, the capped score's fast tanh adds below that
     assert (every.double() - want).abs().max() < 3 * 2.0 ** -9 * values.abs().max()
+
+
+@pytest.mark.parametrize("KVH,tiles", [(4, 64), (4, 65), (3, 86), (2, 255), (3, 170), (4, 128), (3, 171), (16, 47), (257, 1), (257, 2)])
+def test_every_piece_of_a_dealt_launch_is_somebodys(KVH, tiles):
+    """The shared-keys kernel deals the pieces (tile, kv head) of a table out from 257 on, and reverses the second 256: the same bits as
+    calls on parts of the table that are too few to be dealt, where every block takes the piece of its own place."""
+    from tokenmill_amd.hip import ops
+
+    D, G, page, n = 96, 2, 16, 16 * tiles - 3
+    H = KVH * G
+    g = torch.Generator(device=DEV).manual_seed(tiles)
+    q = torch.randn(n, H * D, generator=g, device=DEV).to(BF)
+    k, v = torch.randn(tiles, page, KVH, D, generator=g, device=DEV).to(BF), torch.randn(tiles, KVH, D, page, generator=g, device=DEV).to(BF)
+    tables = torch.arange(tiles, dtype=torch.int32, device=DEV).view(1, -1)
+    table = torch.tensor([(0, j, min(16, n - j), j) for j in reversed(range(0, n, 16))], dtype=torch.int32, device=DEV)
+
+    def attend(rows, heads, out):
+        lo, hi = heads
+        ops.attn_prefill_mfma(q.view(n, H, D)[:, lo * G:hi * G].reshape(n, -1), out, k[:, :, lo:hi].contiguous(), v[:, lo:hi].contiguous(),
+                              tables, table[rows], (hi - lo) * G, hi - lo, D, D ** -0.5, 0, shared=True)
+
+    dealt = torch.full((n, H * D), 3.0, dtype=BF, device=DEV)
+    attend(slice(0, tiles), (0, KVH), dealt)
+    wide = min(KVH, 128)
+    for lo in range(0, KVH, wide):
+        heads = (lo, min(lo + wide, KVH))
+        part = torch.full((n, (heads[1] - lo) * G * D), 3.0, dtype=BF, device=DEV)
+        for t in range(0, tiles, 256 // wide):
+            attend(slice(t, t + 256 // wide), heads, part)
+        assert torch.equal(part.view(n, -1), dealt.view(n, KVH, -1)[:, lo:heads[1]].reshape(n, -1))
