@@ -40,13 +40,16 @@ def test_a_heads_bits_do_not_depend_on_the_heads_beside_it(D, n, window, softcap
     assert (every.double() - want).abs().max() < 3 * 2.0 ** -9 * values.abs().max()
 
 
-@pytest.mark.parametrize("KVH,tiles", [(4, 64), (4, 65), (3, 86), (2, 255), (3, 170), (4, 128), (3, 171), (16, 47), (257, 1), (257, 2)])
-def test_every_piece_of_a_dealt_launch_is_somebodys(KVH, tiles):
-    """The shared-keys kernel deals the pieces (tile, kv head) of a table out from 257 on, and reverses the second 256: the same bits as
-    calls on parts of the table that are too few to be dealt, where every block takes the piece of its own place."""
+@pytest.mark.parametrize("shared,D,KVH,tiles", [(True, 96, *case) for case in ((4, 64), (4, 65), (3, 86), (2, 255), (3, 170), (4, 128), (3, 171), (16, 47),
+                                                                              (257, 1), (257, 2))]
+                         + [(False, D, *case) for D in (64, 96) for case in ((4, 65), (4, 108), (4, 109), (4, 128), (4, 129), (4, 217), (3, 87), (257, 2))])
+def test_every_piece_of_a_launch_is_somebodys(shared, D, KVH, tiles):
+    """From 257 pieces (tile, kv head, its heads) on a launch's blocks take them dealt out over all heads, in reverse among the second 256 (the
+    shared-keys kernel), or dealt or a tile from either end of the table (the other): the same bits as calls on parts of the table so few that every
+    block takes the piece of its own place."""
     from tokenmill_amd.hip import ops
 
-    D, G, page, n = 96, 2, 16, 16 * tiles - 3
+    G, page, n = 2, 16, 16 * tiles - 3
     H = KVH * G
     g = torch.Generator(device=DEV).manual_seed(tiles)
     q = torch.randn(n, H * D, generator=g, device=DEV).to(BF)
@@ -57,7 +60,7 @@ def test_every_piece_of_a_dealt_launch_is_somebodys(KVH, tiles):
     def attend(rows, heads, out):
         lo, hi = heads
         ops.attn_prefill_mfma(q.view(n, H, D)[:, lo * G:hi * G].reshape(n, -1), out, k[:, :, lo:hi].contiguous(), v[:, lo:hi].contiguous(),
-                              tables, table[rows], (hi - lo) * G, hi - lo, D, D ** -0.5, 0, shared=True)
+                              tables, table[rows], (hi - lo) * G, hi - lo, D, D ** -0.5, 0, shared=shared)
 
     dealt = torch.full((n, H * D), 3.0, dtype=BF, device=DEV)
     attend(slice(0, tiles), (0, KVH), dealt)

@@ -62,6 +62,12 @@ def test_bits_of_the_two_launches(H, KVH, D, portions, contexts, extras):
     assert not one.isnan().any() and torch.equal(one, two)
 
 
+@pytest.mark.parametrize("n", [1040, 1740, 2048])
+def test_bits_of_the_two_launches_in_every_order_of_the_pieces(n):
+    """Dealt out, and folded below and at a block a CU."""
+    test_bits_of_the_two_launches(14, 2, 64, [(0, n)], [900, 33], "plain")
+
+
 def test_what_the_launch_does_not_take_is_refused():
     lib = library()
     t = torch.zeros(1 << 16, dtype=torch.bfloat16, device="cuda")

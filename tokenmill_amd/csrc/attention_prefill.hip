@@ -23,6 +23,7 @@
 #include "attention_decode_keys.h"
 
 #include <algorithm>
+#include <limits.h>
 
 // A block of 32 keys as a wavefront holds it between asking for it and using it. Row rho of operand tile t is key 8 (rho / 4) + 4 t + rho % 4,
 // so that the lane which holds rows 4 g .. 4 g + 3 of both tiles of the scores has the eight keys 8 g .. 8 g + 7 of a row of V^T in one piece.
@@ -244,15 +245,17 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, unsigned char* tur
     }
 }
 
+enum { PF_PLAIN, PF_PAIRS, PF_DEALT };
+
 // tiles: int32 [n_tiles][4] = (request index in the step, first row of the tile in the flat batch,
 //                              tokens in the tile (1..16), position of its first token)
 // A block is KS wavefronts on the same tile and heads; wavefront j takes the key blocks kb with
 // kb % KS == j and the partial results are merged through LDS in wavefront order. Which blocks a
 // wavefront takes depends on absolute positions only, and a block in which a token sees no key
 // changes nothing for it, so a token's bits do not depend on the tile it falls into.
-// With pair != 0 a block takes tile b and then tile n_tiles - 1 - b: in a table sorted by the
-// number of keys a tile sees, the longest goes with the shortest and every block has the same work
-// (the lower triangle of a prompt, folded).
+// order: a block takes a tile and heads by its place in the grid (PF_PLAIN); tile b and then tile n_tiles - 1 - b (PF_PAIRS: in
+// a table sorted by the number of keys a tile sees, the longest goes with the shortest and every block has the same
+// work, the lower triangle of a prompt, folded); or the pieces of all heads in the order of the table (PF_DEALT).
 // DECODES: `decodes.layers` layers of the grid in front attend single decoded tokens, a (request, kv head) a block (attend_whole). On its own that
 // is a launch, or two, that waits for its trips to memory, behind one that leaves CUs without a block or their matrix units idle; the blocks in front
 // are the first to get a CU, so a launch that does not fit the chip at once has its long blocks last. Prompt portions, tokens decoded beside them, us of
@@ -275,7 +278,7 @@ template <int D, int HPW, int KS, bool CAP, bool AHEAD, bool DECODES>
 __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
-    int table_width, const int* __restrict__ tiles, int n_tiles, int pair, int H, int KVH, int page_shift,
+    int table_width, const int* __restrict__ tiles, int n_tiles, int order, int H, int KVH, int page_shift,
     float scale_log2, float cap_in, float cap_out, int window, int keep, const float* __restrict__ sink,
     const bf16_t* __restrict__ cgate, int ldcg, const TmAheadArg<AHEAD> ahead, const DecodesArg<DECODES> decodes) {
     constexpr int NDC = D / 32, NDT = D / 16;
@@ -304,7 +307,12 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     const int lane = threadIdx.x % TM_WAVE, r = lane % 16, g = lane / 16;
     const int G = H / KVH;
     const int splits = (G + HPW - 1) / HPW;
-    const int kvh = blockIdx.y / splits, split = blockIdx.y % splits;
+    int tile0 = blockIdx.x, heads = blockIdx.y;
+    if (order == PF_DEALT) {
+        heads = tile0 % (KVH * splits);
+        tile0 /= KVH * splits;
+    }
+    const int kvh = heads / splits, split = heads % splits;
     const int h0 = kvh * G + split * HPW;
     const int nh = (G - split * HPW) < HPW ? (G - split * HPW) : HPW;
     LaneOffsets<D> off;
@@ -320,8 +328,8 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     off.v = (uint32_t)((((size_t)r << page_shift) + 8 * (g % 2)) * sizeof(bf16_t));
     off.row = (uint32_t)(r * Block::ROW + 16 * g);
     unsigned char* turn = (unsigned char*)partial_at(wave, 0, 0, 0);         // (the place of this wavefront's partials, which are stored behind the last block)
-    const int other = n_tiles - 1 - (int)blockIdx.x;
-    const int n_mine = (pair && other > (int)blockIdx.x) ? 2 : 1;
+    const int other = n_tiles - 1 - tile0;
+    const int n_mine = (order == PF_PAIRS && other > tile0) ? 2 : 1;
 
     // A tile begins with three trips to memory (its entry in the table, its queries and pages, its first keys). Those of the second
     // tile are made while the first one's partials meet.
@@ -354,7 +362,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
 #pragma unroll
             for (int c = 0; c < NDC; ++c) qf[hh][c].u = *(const u32x4_t*)(qrow + (size_t)(h0 + (hh < nh ? hh : nh - 1)) * D + 32 * c);
     };
-    begin(blockIdx.x);
+    begin(tile0);
     load_kv_block<D>(ba, pages, 0, k_pool, v_pool, page_shift, off);
 
 #pragma unroll 1
@@ -457,6 +465,21 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
 // 40.6 us, one 4.1 / 7.0 / 34.8). A head's arithmetic is the same either way, so its bits are.
 template <int D> struct PrefillShape { static constexpr int HPW = D <= 64 ? 4 : 2, KS = D <= 64 ? 8 : 4; };
 
+// The order of a launch's pieces of work (a tile and the heads a wavefront takes of one kv head), of which a CU mostly holds one.
+// Two tiles a block save a block its beginning: the second tile's trips to memory are made while the first one's partials
+// meet. But a pair is as long as the longest tile, and where the pairs do not fill their last round of the 256 CUs, pieces of
+// their own, handed out longest first over all heads, are better balanced by the CUs that come free. us on an MI355X, pairs (below 256 of them:
+// tiles by heads) / dealt: 14 heads over 2 of 64, 1,040 tokens (a fill of 0.52) 14.5 / 14.5, 1,200 (0.59) 17.5 / 16.6, 1,500 (0.73) 22.4 / 19.8,
+// 2,100 (0.52) 38.9 / 31.9, 3,001 (0.73) 51.1 / 46.7, 3,400 (0.84) 57.4 / 57.4, 3,700 (0.91) 61.3 / 63.5, 4,096 (1) 64.9 / 71.5; 32 over 8 of 128, 600
+// (0.59) 33.8 / 26.3, 800 (0.78) 38.3 / 36.2, 900 (0.91) 41.5 / 41.6; 8 over 8 of 64, 1,500 (0.73) 19.0 / 15.7; 12 over 2 of 96, 1,500 (0.55) 41.6 / 30.4.
+// From 218 pairs (0.85) on pairs are better than tiles by heads too (1,900 tokens of the first 26.7 / 23.9), with fewer they are not (1,100
+// tokens 14.6 / 18.8). Head size 32, where a CU holds two blocks, stays with tiles by heads and pairs from 256 on (2,500 tokens of 12
+// heads over 2 26.4 / 28.5 dealt), and up to 256 pieces there is nothing to choose.
+static int prefill_order(int D, long long pieces, long long folded) {
+    if (D < 64 || pieces <= 256 || pieces > INT_MAX) return folded >= 256 ? PF_PAIRS : PF_PLAIN;
+    return 100 * folded < 85 * 256 * ((folded + 255) / 256) ? PF_DEALT : PF_PAIRS;
+}
+
 template <int D, int HPW, bool CAP>
 static int launch_split_keys(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                               const int* block_tables, int table_width, const int* tiles, int n_tiles, int H, int KVH,
@@ -464,9 +487,9 @@ static int launch_split_keys(const void* q, int q_stride, void* out, int out_str
                               const bf16_t* cgate, int ldcg, TmAhead& ahead, const TmDecodes* beside, hipStream_t stream) {
     constexpr int KS = PrefillShape<D>::KS;
     const int splits = (H / KVH + HPW - 1) / HPW;
-    // fold the table in two once the folded launch still gives every CU a block
-    const int pair = (long long)(n_tiles / 2) * KVH * splits >= 256 ? 1 : 0;
-    dim3 grid(pair ? (n_tiles + 1) / 2 : n_tiles, KVH * splits);
+    const long long pieces = (long long)n_tiles * KVH * splits, folded = (long long)((n_tiles + 1) / 2) * KVH * splits;
+    const int order = prefill_order(D, pieces, folded);
+    dim3 grid = order == PF_DEALT ? dim3((unsigned)pieces) : dim3(order == PF_PAIRS ? (n_tiles + 1) / 2 : n_tiles, KVH * splits);
     constexpr int lds = KS * wave_floats<D, HPW>() * (int)sizeof(float);          // at most 139,264 bytes
     const long long layer = (long long)grid.x * grid.y;
     const int pairs = beside ? beside->n * KVH : 0, front = beside ? (int)((pairs + layer - 1) / layer) : 0;
@@ -491,7 +514,7 @@ static int launch_split_keys(const void* q, int q_stride, void* out, int out_str
         }
         attn_prefill_mfma_kernel<D, HPW, KS, CAP, with, decode><<<grid, 64 * KS, bytes, stream>>>(
             (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
-            table_width, tiles, n_tiles, pair, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg, ahead_arg<with>(ahead), decodes);
+            table_width, tiles, n_tiles, order, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg, ahead_arg<with>(ahead), decodes);
         return TM_OK;
     };
     if constexpr (D <= 64) {
