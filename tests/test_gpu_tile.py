@@ -225,6 +225,33 @@ def test_few_rows_do_not_change_a_row_of_a_split_product(N, K):
     assert all(torch.equal(out, sums[64][:, :M]) for M, out in sums.items())
 
 
+# one wavefront, four, all; pairs that are held and that are not; experts without a pair, without matrices
+@pytest.mark.parametrize("T,E,real,top,rows", [(1, 1, 1, 1, 32), (128, 64, 64, 2, 64), (129, 64, 63, 2, 64), (5, 65, 65, 2, 32), (512, 256, 256, 2, 128), (513, 17, 16, 2, 64),
+                                               (3, 257, 257, 5, 32), (64, 1024, 1000, 8, 32), (64, 1024, 1024, 8, 32), (2048, 3, 3, 2, 128), (4097, 1, 1, 1, 64),
+                                               (3000, 70, 64, 4, 128), (5, 8, 0, 2, 32)])
+def test_route(T, E, real, top, rows):
+    lib = library()
+    g = torch.Generator().manual_seed(T + E)
+    table = torch.rand(T, E, generator=g).argsort(1)[:, :top].int().contiguous()
+    n = T * top
+    most = min(n, n // rows + E)
+    slot_pair, pair_slot, tiles, n_tiles = (torch.full((k,), -7, dtype=torch.int32, device="cuda") for k in (n, n, 3 * most, 1))
+    chosen = table.to("cuda")
+    assert lib.tm_moe_route_chosen(None, P(chosen.data_ptr()), I(T), I(top), I(E), I(real), I(rows), P(slot_pair.data_ptr()), P(pair_slot.data_ptr()),
+                                   P(tiles.data_ptr()), P(n_tiles.data_ptr()), _stream()) == 0
+    e = table.flatten().long()
+    count = torch.bincount(e[e < real], minlength=real)[:real].tolist()
+    want, at = [], 0
+    for x, c in enumerate(count):
+        want += [(x, at + r, min(rows, c - r)) for r in range(0, c, rows)]
+        at += c
+    assert n_tiles.item() == len(want) and [tuple(t) for t in tiles.view(-1, 3)[:len(want)].tolist()] == want
+    slots, pairs = pair_slot.cpu().long(), slot_pair.cpu().long()
+    assert (slots[e >= real] == -1).all() and slots[e < real].sort().values.tolist() == list(range(at))
+    assert torch.equal(pairs[slots[e < real]], torch.nonzero(e < real).flatten())
+    assert (e[pairs[:at]].diff() >= 0).all() if at > 1 else True
+
+
 # (tokens, experts, choices a token, K, width): experts without a token, with one, with tiles that are full and that are not
 EXPERTS = [(40, 3, 1, 192, 16), (200, 5, 2, 256, 208), (700, 4, 2, 320, 576), (130, 16, 3, 192, 192)]
 
