@@ -65,6 +65,12 @@ def test_a_row_is_the_same_whatever_rows_are_beside_it(N, K):
         assert torch.equal(product(rows), most[:rows]), rows
 
 
+@pytest.mark.parametrize("N,K", [(3580, 16 * 97), (3584, 16 * 105), (4092, 16 * 112), (3568, 16 * 97), (24000, 384), (2100, 16 * 49)])
+def test_a_row_is_the_same_where_the_blocks_nearly_fill_the_chip(N, K):
+    """From 224 blocks on two groups at a time for any rows, with a rest of every length; the shortest lines; a step of a pair that is not there."""
+    test_a_row_is_the_same_whatever_rows_are_beside_it(N, K)
+
+
 @pytest.mark.parametrize("M", [1, 8, 9, 16])
 @pytest.mark.parametrize("K,small,large", [(912, 1868, 1872), (1440, 1180, 1184), (6896, 244, 248), (448, 3800, 3808), (400, 4256, 4260)])
 def test_whole_lines_and_a_load_a_step_have_the_same_bits(K, small, large, M):

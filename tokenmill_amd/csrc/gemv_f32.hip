@@ -8,15 +8,18 @@
 // LDS but the wavefronts' sums at the end, added in wavefront order. The activations come from the second-level cache. Which k goes where
 // depends on the matrix alone: a row's result does not depend on the other rows.
 //
-// The matrix instruction wants 16 bytes of row r at 4 g in lane (r, g), 64 bytes of each of sixteen rows. A CU takes such loads in at half
-// the rate of whole lines (a line costs it the same either way; 30 to 40 KB a us against 130 a block alone on its CU), so two steps are loaded
-// as a pair, 128 bytes of eight rows an instruction, and the lanes r and r + 8 exchange what belongs to the other, which is eight
-// instructions of the vector unit a pair. Up to eight rows of activations are one load a pair, and whole lines that
-// nobody reads again pass the caches by (non-temporal: the head 98 to 85 us, down 6.7 to 6.5). Against a load a step, cold matrices, us: gate|up of the 0.5B
-// shape at 1 / 8 rows 11.2 / 12.7 to 9.4 / 10.5 and at 16 rows 16% less, down 6.7 to 6.0 at one row, 9% less at 16; the head 120 / 129 to 84 / 86 (6.3 TB/s at 8
-// rows), 3,584 -> 2 x 18,944 110 to 91 at one row. Matrices of less than 6.5 MB and rows of less than 384 k are latency, and the exchange comes on top of it (K
-// from 256 to 8,192, 6 MB, against a load a step: 1 and 8 rows 7% slower to 6% faster, 9 and 16 rows up to 11% slower and 4% on the mean; 7 MB 5% faster
-// on the mean at all, K of 256 5% slower): they keep a load a step (GM_LINES). The same bits either way.
+// The matrix instruction wants 16 bytes of row r at 4 g in lane (r, g): neighbouring lanes in different rows. A CU takes the addresses of a load
+// in four lanes at a time where these lie beside each other, and one at a time where they do not, which was most of what small products took
+// (64 clocks a load of 1 KB for 16). So four neighbouring lanes load 64 consecutive bytes, and the exchange that puts the pieces where the
+// instruction wants them (lane (4 q + p, g) holds row 4 q + g at piece p, and wants row 4 q + p at piece g) is four ds_bpermute a load, which
+// pass no memory. Matrices of 6.5 MB and more (GM_LINES) are loaded two steps at a time, 128 bytes of eight rows an instruction, whole lines that
+// pass the caches by (non-temporal), halves of lines would come from HBM twice as slowly; the step's parity lies in lane bit 4, where
+// one instruction a register changes it for the row's lowest bit. The activations go the same way; one row of them is asked for as the
+// instruction wants it, all sixteen lanes of a piece at one place. us with the loads in the instruction's order / now, cold matrices:
+// q|k|v of the 0.5B shape at 1 / 8 / 16 rows 5.66 / 4.97, 6.40 / 5.65, 7.31 / 6.47, o 4.85 / 4.38, 5.58 / 5.07, 6.51 / 5.74, down 6.34 / 6.25, 7.25 / 6.56, 8.62 / 7.53, gate|up
+// 9.5 / 9.8, 10.4 / 10.2, 12.3 / 11.2, the head 96 / 91, 102 / 96, 117 / 107 (5.1 TB/s); 3,584 -> 2 x 18,944 93.8 / 92.3, 109 / 97, 137 / 111, back 48.7 / 49.7, 60 / 57,
+// 76.6 / 64.5; 2,048 -> 2,048 7.60 / 7.15, 8.49 / 7.95, 9.87 / 8.62; 2,000 x 128 3.44 / 3.06, 3.73 / 3.15, 4.05 / 3.15. Slower: up to four rows of 384 -> 32,000 (12.7 /
+// 13.3), K of 336 and 400 that leave wavefronts part of a group (3.4 / 3.5). The same bits.
 // Before that, a wavefront had 256 k of four rows, a lane 4 k each, and summed over the lanes by shuffles, 6 x 32 of them a wavefront:
 // 19.0 us a product of the 0.5B shape on average, with SiLU*up and rotation in kernels behind it.
 #include "common.h"
@@ -47,8 +50,9 @@ struct GemvArgs {
 
 // GROUP: steps of 16 k whose products meet in sums of their own before they join the running one. AHEAD: groups a wavefront asks for
 // at once: with one, a wavefront of the 0.5B shape waited for memory two times in a launch of 6 to 7 us (o 6.2 to 5.8, q|k|v 7.2 to 6.8).
-// LINES: two steps as a pair of lines, else a load a step. OVER8: more than eight rows of activations (the same code where there are no lines).
-template <int EPI, int RT, int WAVES, int GROUP, int AHEAD, bool LINES, bool OVER8>
+// LINES: two steps as a pair of lines, else a load a step. ROWS: rows of activations that there are places for, 1, 8 (of a pair of lines: one
+// load) or 16.
+template <int EPI, int RT, int WAVES, int GROUP, int AHEAD, bool LINES, int ROWS>
 __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArgs a) {
     static_assert(EPI == GM_PLAIN || RT == 1, "");
     __shared__ __align__(16) f32x4_t red[WAVES][RT][TM_WAVE];
@@ -76,22 +80,40 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     const int b0 = blockIdx.y * per_block, b1 = b0 + per_block < steps ? b0 + per_block : steps;
     const int per = (per_block + WAVES - 1) / WAVES;
     const int s0 = b0 + wave * per, s1 = s0 + per < b1 ? s0 + per : b1;
-    // rows r % 8 and 8 + r % 8, or row r (rows beyond the matrix, the half or the input: its last one, never stored)
+    // What a lane loads: 16 bytes at 4 * piece of a step of row 4 q + g, q = r / 4; of a pair of lines of the step whose parity is g's lower
+    // bit, of rows 4 q + 2 (g / 2) + h. (Rows beyond the matrix, the half or the input: its last one, never stored.)
+    static_assert(LINES || ROWS != 8, "");
     constexpr int HALVES = LINES ? 2 : 1;
-    const int r8 = r % 8, second = r / 8;
+    constexpr bool WHOLE = GROUP == 4 && (LINES || AHEAD == 1); // a full group's operands are all turned before its first product: 4,096 -> 4,096 at 8 rows 16.1 to 15.4
+    const int q = r / 4, piece = r % 4, parity = LINES ? g % 2 : 0;
+    // where a lane gets row r at piece g from, in bytes of lanes (eight rows of a pair of lines: the other step 16 lanes on)
+    const int turn = 4 * (LINES ? 32 * (r / 2 % 2) + 16 * (r % 2) + 4 * q + g : 16 * piece + 4 * q + g);
+    const int turn_x = LINES && ROWS == 8 ? 4 * (32 * (r % 2) + 4 * (r % 8 / 2) + g) : turn;
     const float* pa[HALVES];
     const float* pw[RT][HALVES];
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) {
-        const int row = LINES ? r8 + 8 * h : r;
-        pa[h] = a.A + (size_t)(row < a.M ? row : a.M - 1) * a.lda + 4 * g;
+        const int row = LINES ? 4 * q + 2 * (g / 2) + h : 4 * q + g, of = LINES && ROWS == 8 ? 2 * q + g / 2 : row;
+        pa[h] = ROWS == 1 ? a.A + 4 * g : a.A + (size_t)(of < a.M ? of : a.M - 1) * a.lda + 4 * piece;
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
-            const int end = EPI == GM_SILU ? a.I : a.N, at = n0[t] + (EPI == GM_PLAIN ? row : r8);
-            const int n = (at < end ? at : end - 1) + (EPI != GM_PLAIN ? (LINES ? h : second) * far : 0);
-            pw[t][h] = a.W + (size_t)n * a.K + 4 * g;
+            const int end = EPI == GM_SILU ? a.I : a.N, at = n0[t] + (EPI == GM_PLAIN ? row : row % 8);
+            const int n = (at < end ? at : end - 1) + (EPI != GM_PLAIN ? row / 8 * far : 0);
+            pw[t][h] = a.W + (size_t)n * a.K + 4 * piece;
         }
     }
+    auto turned = [&](int from, f32x4_t v) {
+        f32x4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(v[e])));
+        return o;
+    };
+    auto pair_half = [&](int half, f32x4_t lo, f32x4_t hi) {    // lane bit 4, the step's parity, changes places with h
+        f32x4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(lo[e]), __float_as_uint(hi[e]), false, false)[half]);
+        return o;
+    };
     // What the epilogue waits for otherwise: the positions are asked for before the matrix (loads come back in their order), the
     // rotary rows, whose place hangs on them, behind its first round.
     int pos = 0, slot = -1;
@@ -111,11 +133,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     for (int t = 0; t < RT; ++t) sum[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     auto groups = [&](auto AT_ONCE, int s) {
         constexpr int GROUPS = decltype(AT_ONCE)::value, LOADS = LINES ? (GROUP * GROUPS + 1) / 2 : GROUP * GROUPS;
-        f32x4_t w[RT][LOADS][HALVES], x[LOADS][LINES && OVER8 ? 2 : 1];
+        f32x4_t w[RT][LOADS][HALVES], x[LOADS][LINES && ROWS == 16 ? 2 : 1];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
-            const int step = LINES ? s + 2 * i + second : s + i, at = 16 * (step < s1 ? step : s1 - 1);  // (no load under a test: beyond the end the last step again)
+            const int step = LINES ? s + 2 * i + parity : s + i, at = 16 * (step < s1 ? step : s1 - 1);  // (no load under a test: beyond the end the last step again)
+            const int one = s + 2 * i + r / 8, at_one = 16 * (one < s1 ? one : s1 - 1);      // (one row: lanes r < 8 the first step, the others the second)
 #pragma unroll
             for (int h = 0; h < HALVES; ++h) {
 #pragma unroll
@@ -123,7 +146,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
                     const f32x4_t* at_w = (const f32x4_t*)(pw[t][h] + at);
                     w[t][i][h] = LINES ? __builtin_nontemporal_load(at_w) : *at_w;
                 }
-                if (h == 0 || OVER8) x[i][h] = *(const f32x4_t*)(pa[h] + at);
+                if (h == 0 || ROWS == 16) x[i][h] = *(const f32x4_t*)(pa[h] + (ROWS == 1 && LINES ? at_one : at));
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -135,6 +158,19 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        auto operands = [&](int i, f32x4_t& xf, f32x4_t (&wf)[RT]) {
+            if constexpr (LINES) {
+                if constexpr (ROWS == 1) xf = i % 2 ? line_pair_turned(x[i / 2][0]) : x[i / 2][0];
+                else if constexpr (ROWS == 8) xf = turned(turn_x + 64 * (i % 2), x[i / 2][0]);
+                else xf = turned(turn, pair_half(i % 2, x[i / 2][0], x[i / 2][ROWS == 16 ? 1 : 0]));
+#pragma unroll
+                for (int t = 0; t < RT; ++t) wf[t] = turned(turn, pair_half(i % 2, w[t][i / 2][0], w[t][i / 2][1]));
+            } else {
+                xf = ROWS == 1 ? x[i][0] : turned(turn, x[i][0]);
+#pragma unroll
+                for (int t = 0; t < RT; ++t) wf[t] = turned(turn, w[t][i][0]);
+            }
+        };
 #pragma unroll
         for (int j = 0; j < GROUPS; ++j) {
             if (s + j * GROUP >= s1) break;                     // the same for the whole wavefront
@@ -144,19 +180,23 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
             for (int t = 0; t < RT; ++t)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[t][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            if (WHOLE && s + (j + 1) * GROUP <= s1) {
+                f32x4_t xf[GROUP], wf[GROUP][RT];
+#pragma unroll
+                for (int k = 0; k < GROUP; ++k) operands(j * GROUP + k, xf[k], wf[k]);
+#pragma unroll
+                for (int k = 0; k < GROUP; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int t = 0; t < RT; ++t)
+                            acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[k][t][e], xf[k][e], acc[t][e], 0, 0, 0);
+            } else
 #pragma unroll
             for (int i = j * GROUP; i < (j + 1) * GROUP; ++i) {
                 if (s + i >= s1) break;
                 f32x4_t xf, wf[RT];
-                if constexpr (LINES) {
-                    xf = OVER8 ? line_pair_half(i % 2, x[i / 2][0], x[i / 2][OVER8 ? 1 : 0]) : i % 2 ? line_pair_turned(x[i / 2][0]) : x[i / 2][0];
-#pragma unroll
-                    for (int t = 0; t < RT; ++t) wf[t] = line_pair_half(i % 2, w[t][i / 2][0], w[t][i / 2][1]);
-                } else {
-                    xf = x[i][0];
-#pragma unroll
-                    for (int t = 0; t < RT; ++t) wf[t] = w[t][i][0];
-                }
+                operands(i, xf, wf);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -252,47 +292,62 @@ extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, con
 
 // Up to a block a CU, eight wavefronts split K into groups of four steps; more blocks than that have four wavefronts with groups of seven, whose
 // blocks a CU hide each other's waits. A wavefront of the eight that has up to three groups asks for all of them at once; with more, of
-// up to four rows two groups at a time and of more rows one (K cut into 32 to 56 steps a wavefront, one group / two, us: 18,944 -> 3,584, 1 / 4 / 8 /
-// 16 rows 50.5 / 43.6, 50.7 / 47.3, 52.4 / 54.4, 67.7 / 69.5; 5,632 -> 2,048 10.7 / 9.7, 10.8 / 10.1, 11.0 / 11.6, 13.1 / 14.3). One of the four
+// up to four rows, or where nearly every CU has a block, two groups at a time, else one (one group / two, us: 18,944 -> 3,584, 8 / 16 rows, 224 blocks
+// 58.7 / 51.4, 65.7 / 61.4; 4,096 -> 4,096, 256 blocks 15.4 / 14.8, 17.3 / 16.5; 8,960 -> 1,536, 192 blocks 18.7 / 19.3, 22.1 / 22.9; 2,048 -> q|k|v of 2,560, 160
+// blocks 8.8 / 9.0, 9.7 / 10.3). One of the four
 // asks for two groups where it has them: a group at a time leaves half a pair's line, and gate|up of the 0.5B shape takes 12.2 us so for 10.2.
 // Of the products with a load a step (GM_LINES), more than three groups a wavefront are asked for one at a time whatever the rows are (2,048 -> 2,048 cut
 // into 16 steps a wavefront, 1 / 8 / 16 rows: two rounds of three groups 9.4 / 11.5 / 13.5 us, four of one 7.7 / 8.6 / 10.0).
 constexpr size_t GM_LINES = 6656 * 1024;
 constexpr int GM_LINES_K = 384;
 
-template <int EPI, int RT, bool LINES, bool OVER8>
+template <int EPI, int RT, bool LINES, int ROWS>
 static void gm_launch_rows(const GemvArgs& a, int units, int split, hipStream_t stream) {
     const int steps = (a.K / 16 + split - 1) / split, per = (steps + 7) / 8;
-    const bool long_runs = LINES && per > 12 && a.M <= 4;
+    const bool long_runs = LINES && per > 12 && (a.M <= 4 || units * split >= 224);
     const dim3 grid(units, split);
     if (units * split > 256) {
         if constexpr (LINES) {
             if (steps > 4 * 7) {
-                gemv_mfma_f32_kernel<EPI, RT, 4, 7, 2, LINES, OVER8><<<grid, 256, 0, stream>>>(a);
+                gemv_mfma_f32_kernel<EPI, RT, 4, 7, 2, LINES, ROWS><<<grid, 256, 0, stream>>>(a);
                 return;
             }
         }
-        gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1, LINES, OVER8><<<grid, 256, 0, stream>>>(a);
+        gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1, LINES, ROWS><<<grid, 256, 0, stream>>>(a);
         return;
     }
     if constexpr (LINES || RT == 1) {                           // (two tiles without lines: K of less than 384)
         if (per > 4 && (per <= 8 || long_runs)) {
-            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2, LINES, OVER8><<<grid, 512, 0, stream>>>(a);
+            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2, LINES, ROWS><<<grid, 512, 0, stream>>>(a);
             return;
         }
         if (per > 8 && per <= 12) {
-            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3, LINES, OVER8><<<grid, 512, 0, stream>>>(a);
+            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3, LINES, ROWS><<<grid, 512, 0, stream>>>(a);
             return;
         }
     }
-    gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1, LINES, OVER8><<<grid, 512, 0, stream>>>(a);
+    gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1, LINES, ROWS><<<grid, 512, 0, stream>>>(a);
+}
+
+template <int EPI, int RT, bool LINES>
+static void gm_launch_lines(const GemvArgs& a, int units, int split, hipStream_t stream) {
+    if (a.M == 1) {
+        gm_launch_rows<EPI, RT, LINES, 1>(a, units, split, stream);
+        return;
+    }
+    if constexpr (LINES) {
+        if (a.M <= 8) {
+            gm_launch_rows<EPI, RT, LINES, 8>(a, units, split, stream);
+            return;
+        }
+    }
+    gm_launch_rows<EPI, RT, LINES, 16>(a, units, split, stream);
 }
 
 template <int EPI, int RT>
 static void gm_launch(const GemvArgs& a, int units, int split, hipStream_t stream) {
-    if ((size_t)a.N * a.K * 4 < GM_LINES || a.K < GM_LINES_K) gm_launch_rows<EPI, RT, false, false>(a, units, split, stream);
-    else if (a.M > 8) gm_launch_rows<EPI, RT, true, true>(a, units, split, stream);
-    else gm_launch_rows<EPI, RT, true, false>(a, units, split, stream);
+    if ((size_t)a.N * a.K * 4 < GM_LINES || a.K < GM_LINES_K) gm_launch_lines<EPI, RT, false>(a, units, split, stream);
+    else gm_launch_lines<EPI, RT, true>(a, units, split, stream);
 }
 
 extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,
