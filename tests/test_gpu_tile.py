@@ -210,6 +210,47 @@ def test_the_rows_do_not_change_a_row_of_gate_up_or_of_qkv(dt):
         assert all(torch.equal(x, y[:x.shape[0]]) for x, y in zip(few, got[0]))
 
 
+# rows and matrices whose launch takes a tile between those of the table (11 to 14), and the table's where the sizes above have come to take another
+BETWEEN = [("silu", (804, 2816, 320), 5), ("silu", (321, 4864, 320), 6), ("silu", (449, 2000, 320), 7), ("silu", (1409, 1000, 320), 11),
+           ("silu", (417, 4864, 320), 12), ("silu", (804, 2816, 832), 13), ("silu", (579, 4864, 320), 14), ("qkv", (2242, 16, 16, 64, 320, 16), 4),
+           ("qkv", (1601, 16, 16, 64, 320, 16), 5), ("qkv", (707, 28, 4, 128, 320, 16), 6), ("qkv", (611, 28, 4, 128, 320, 16), 11),
+           ("qkv", (1345, 16, 16, 64, 320, 1), 12), ("qkv", (1605, 16, 16, 64, 832, 16), 13), ("qkv", (2017, 16, 16, 64, 320, 32), 14),
+           ("parts", (1860, 1536, 320), 11), ("parts", (579, 3584, 1280), 12), ("parts", (648, 3584, 1600), 13), ("parts", (2311, 896, 2112), 14),
+           ("linear", (929, 3072, 320), 11), ("linear", (1347, 3072, 320), 12), ("linear", (1606, 3072, 832), 13), ("linear", (2018, 3072, 320), 14)]
+
+
+@pytest.mark.parametrize("what,size,tile", BETWEEN)
+def test_tiles_between(what, size, tile):
+    """Against 64 bits as above, and a row's bits are those of the calls of fewer rows, which take other tiles."""
+    lib, M, K = library(), size[0], size[4] if what == "qkv" else size[2]
+    N = 2 * size[1] if what == "silu" else (size[1] + 2 * size[2]) * size[3] if what == "qkv" else size[1]
+    parts = lib.tm_tile_linear_parts(M, N, K) if what == "parts" else 1
+    assert lib.tm_gemm_tile_picked(M, N, K, parts) == tile
+    if what == "qkv":
+        return test_qkv_with_rotation_and_cache_write(*size, torch.float32, True)
+    if what == "parts":
+        return test_partial_sums_of_a_split_k(*size)
+    if what == "silu":
+        test_gate_up_silu(*size)
+    a, w, ref = _operands(M, N, K, M)
+    lead = lambda m: (P(a.data_ptr()), I(K), I(m), I(K), P(w.data_ptr()))
+
+    def product(m, dt=torch.bfloat16):
+        out = torch.full((m, size[1]), float("nan"), device="cuda", dtype=dt)
+        if what == "silu":
+            assert lib.tm_tile_gate_up_silu(*lead(m), P(out.data_ptr()), I(N // 2), _stream()) == 0
+        else:
+            assert lib.tm_tile_linear(*lead(m), I(N), P(out.data_ptr()), I(N), I(1 if dt is torch.bfloat16 else 0), _stream()) == 0
+        return out
+
+    full = product(M)
+    for m in (77, 300):
+        assert torch.equal(product(m), full[:m])
+    if what == "linear":
+        sums = product(M, torch.float32)
+        assert (sums.double() - ref).abs().max() <= 2.0 ** -24 * 5 * 4 * K ** 0.5 and torch.equal(sums.bfloat16(), full)
+
+
 # an output and a down projection of the shipped shapes and what lies around the line between the two tiles of few rows
 @pytest.mark.parametrize("N,K", [(896, 896), (896, 4864), (2048, 11008), (3584, 3584), (3584, 18944), (5120, 27648), (3072, 12864), (2944, 12864)])
 def test_few_rows_do_not_change_a_row_of_a_split_product(N, K):

@@ -591,10 +591,18 @@ __global__ __launch_bounds__(256, OCC) void gemm_tile_kernel(const TileArgs a, c
     X(8, 1, 4, 4, 1, 4, 2, 0.232, 1.01, 0.342, 1.94)       \
     X(9, 1, 4, 4, 1, 8, 1, 0.213, 1.16, 0, 0)              \
     X(10, 1, 4, 2, 2, 4, 2, 0.318, 1.02, 0.273, 0.61)
+// Tiles between those, 128 columns wide, for rows whose tiles of the table above are one round of the chip only with a larger one (gt_pick).
+// Fitted to 149 timings of eleven matrices at 100 to 4,000 rows, one round each, against what the table's choice took there.
+#define GT_BETWEEN(X)                                      \
+    X(11, 3, 4, 2, 2, 5, 1, 0.422, 2.68, 0, 0)             \
+    X(12, 5, 4, 2, 2, 4, 1, 0.488, 4.51, 0, 0)             \
+    X(13, 6, 4, 2, 2, 3, 1, 0.533, 5.60, 0, 0)             \
+    X(14, 7, 4, 2, 2, 3, 1, 0.622, 4.90, 0, 0)
 struct GtShape { int BM, BN, ST, OCC; double step, epi, step2, epi2; };
 #define GT_SHAPE(id, MT, NT, WM, WN, ST, OCC, s1, e1, s2, e2) {16 * MT * WM, 16 * NT * WN, ST, OCC, s1, e1, s2, e2},
-static const GtShape gt_shapes[] = {GT_SHAPES(GT_SHAPE)};
-constexpr int GT_N_SHAPES = sizeof(gt_shapes) / sizeof(gt_shapes[0]);
+static const GtShape gt_shapes[] = {GT_SHAPES(GT_SHAPE) GT_BETWEEN(GT_SHAPE)};
+#define GT_COUNT(...) +1
+constexpr int GT_N_SHAPES = GT_SHAPES(GT_COUNT), GT_N_ALL = sizeof(gt_shapes) / sizeof(gt_shapes[0]);
 constexpr int GT_CUS = 256;
 constexpr double GT_BYTES_US = 14e6;        // what the CUs take out of the second-level caches together
 
@@ -624,6 +632,27 @@ static int gt_choose(int M, int N, int K, int splits, double* cost = nullptr) {
         if (best < 0 || c < least) best = i, least = c;
     }
     if (cost) *cost = least;
+    return best;
+}
+
+// The tile a launch takes: the table's choice, which also says into how many parts K is cut, or a tile between where that is one round of the chip,
+// at least 7% cheaper by these figures, and not bound by the operands' way into the CUs. 25 matrices (0.5B, 1.5B, 7B and others), 70 to 3,001
+// rows: of 1,000 launches it then takes 129, which last 0.79 to 1.02 of what they did, 0.925 on the mean; nearer lines bring 1% more of that and
+// launches that last 1.05 to 1.3. us: gate|up of the 0.5B shape at 250 rows 128 x 128 13.4, 96 x 128 11.9, at 544 96 x 256 17.1, 192 x 128 15.9, at 640 128 x 256
+// 19.3, 224 x 128 17.6; q|k|v at 2,048 13.2 / 11.3; 1,792 -> q|k|v of 4,608 at 1,024 96 x 256 30.1, 160 x 128 24.2. Every tile adds a row's products in one order.
+static int gt_pick(int M, int N, int K, int splits) {
+    double least;
+    int best = gt_choose(M, N, K, splits, &least);
+    if (best < 0) return best;
+    least *= 0.93;
+    const int per = (K / 64 + splits - 1) / splits;
+    for (int i = GT_N_SHAPES; i < GT_N_ALL; ++i) {
+        const GtShape& t = gt_shapes[i];
+        const long long tiles = (long long)((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN) * splits;
+        const double cost = per * t.step + t.epi;
+        if (tiles > GT_CUS || !gt_splits_ok(t, K, splits) || (double)tiles * (t.BM + t.BN) * per * 128 / GT_BYTES_US >= 0.92 * cost) continue;
+        if (cost < least) best = i, least = cost;
+    }
     return best;
 }
 
@@ -667,11 +696,17 @@ static int gt_go(TileArgs& a, int shape, hipStream_t stream, TmAhead* ahead = nu
     switch (shape) {
 #define GT_CASE(id, MT, NT, WM, WN, ST, OCC, s1, e1, s2, e2) case id: return gt_launch<bf16_t, EPI, MT, NT, WM, WN, ST, OCC>(a, stream, ahead);
         GT_SHAPES(GT_CASE)
+        GT_BETWEEN(GT_CASE)
     }
     return TM_ERR_ARG;
 }
 
 // Which of the tiles above a product runs with.
+extern "C" int tm_gemm_tile_picked(int M, int N, int K, int splits) {
+    return M > 0 && N > 0 && K >= 256 && splits > 0 ? gt_pick(M, N, K, splits) : -1;
+}
+
+// Which of the first table's: the one that says how K is cut.
 extern "C" int tm_gemm_tile_shape(int M, int N, int K, int splits) {
     return M > 0 && N > 0 && K >= 256 && splits > 0 ? gt_choose(M, N, K, splits) : -1;
 }
@@ -690,7 +725,7 @@ extern "C" int tm_tile_gate_up_silu(const void* A, int lda, int M, int K, const 
     TileArgs a{};
     a.A = A; a.W = W; a.C = act;
     a.M = M; a.N = 2 * I; a.K = K; a.lda = lda; a.ldc = I; a.I = I; a.splits = 1;
-    return gt_go<GT_SILU>(a, gt_choose(M, 2 * I, K, 1), stream);
+    return gt_go<GT_SILU>(a, gt_pick(M, 2 * I, K, 1), stream);
 }
 
 // q (rotated, [M, H D]), and k and v to the cache, of q|k|v = A W^T + bias; head sizes of whole units (64), rotated over the
@@ -709,7 +744,7 @@ int tile_qkv_rope_ahead(const void* A, int lda, int M, int K, const void* W, con
     a.H = H; a.KVH = KVH; a.D = D; a.head_inverse = unit_inverse(D / 64); a.cos_t = cos_t; a.sin_t = sin_t; a.positions = positions; a.slots = slots;
     a.k_pool = k_pool; a.v_pool = v_pool;
     while ((1 << a.page_shift) < page) ++a.page_shift;
-    return gt_go<GT_QKV>(a, gt_choose(M, N, K, 1), stream, &ahead);
+    return gt_go<GT_QKV>(a, gt_pick(M, N, K, 1), stream, &ahead);
 }
 
 extern "C" int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void* W, const void* bias, int bias_dtype, void* q, int H,
@@ -766,21 +801,21 @@ extern "C" int tm_tile_linear_split(const void* A, int lda, int M, int K, const 
     if (gt_few(M, K))
         return gt_few_wide(N, K) ? gt_launch<bf16_t, GT_PARTS, 2, 4, 2, 2, GT_FEW_WIDE_RING, 2>(a, stream)
                                  : gt_launch<bf16_t, GT_PARTS, 1, 4, 4, 1, GT_FEW_RING, 2>(a, stream);
-    return gt_go<GT_PARTS>(a, gt_choose(M, N, K, splits), stream);
+    return gt_go<GT_PARTS>(a, gt_pick(M, N, K, splits), stream);
 }
 
 TmTilePieces tile_pieces_gate_up(int M, int I, int K) {
-    const int shape = gt_choose(M, 2 * I, K, 1);
+    const int shape = gt_pick(M, 2 * I, K, 1);
     return shape < 0 ? TmTilePieces{} : TmTilePieces{gt_shapes[shape].BN / 2, 1, K / 64};
 }
 TmTilePieces tile_pieces_qkv(int M, int N, int K) {
-    const int shape = gt_choose(M, N, K, 1);
+    const int shape = gt_pick(M, N, K, 1);
     return shape < 0 ? TmTilePieces{} : TmTilePieces{gt_shapes[shape].BN, 1, K / 64};
 }
 TmTilePieces tile_pieces_split(int M, int N, int K) {
     const int parts = tm_tile_linear_parts(M, N, K);
     if (parts < 1) return {};
-    const int shape = gt_few(M, K) ? 0 : gt_choose(M, N, K, parts);
+    const int shape = gt_few(M, K) ? 0 : gt_pick(M, N, K, parts);
     if (shape < 0) return {};
     const int columns = gt_few(M, K) ? (gt_few_wide(N, K) ? 128 : 64) : gt_shapes[shape].BN;
     return {columns, parts, (K / 64 + parts - 1) / parts};
@@ -794,7 +829,7 @@ extern "C" int tm_tile_linear(const void* A, int lda, int M, int K, const void* 
     TileArgs a{};
     a.A = A; a.W = W; a.C = C;
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.splits = 1;
-    return out_dtype == TM_F32 ? gt_go<GT_PARTS>(a, gt_choose(M, N, K, 1), stream) : gt_go<GT_STORE>(a, gt_choose(M, N, K, 1), stream);
+    return out_dtype == TM_F32 ? gt_go<GT_PARTS>(a, gt_pick(M, N, K, 1), stream) : gt_go<GT_STORE>(a, gt_pick(M, N, K, 1), stream);
 }
 
 // --- the same in 32-bit ---------------------------------------------------------------------------------------------------
