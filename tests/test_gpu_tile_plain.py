@@ -51,3 +51,23 @@ def test_a_linear_on_both_sides_of_the_lines(N, K, tiled):
             assert (got.double() - want).norm() < (2.0 ** -8 if out_dtype == BF else 1e-6) * want.norm()
             if inside:
                 assert torch.equal(got, ops.tile_linear(x, lin.weight, torch.empty_like(got)))
+
+
+@pytest.mark.parametrize("N,K,tiled", [(32000, 1024, True), (16384, 256, True), (32004, 1024, False), (32000, 1056, False), (204808, 2048, False), (204808, 1984, True)])
+def test_an_output_head_on_both_sides_of_the_lines(N, K, tiled):
+    """Rows of a head that the tiled kernel takes from the library: their ends and one beyond, sizes it does not have; a row does not depend on the others."""
+    from tokenmill_amd import profiling
+
+    g = torch.Generator(device=DEV).manual_seed(N)
+    lin = Linear(K, N, "w", bias=False, library_first=True)
+    lin.load({"w.weight": (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(BF)}, "")
+    lin.prepare(False)
+    x = torch.randn(65, K, generator=g, device=DEV).to(BF)
+    want, got = x.double() @ lin.weight.double().T, {}
+    for M in (16, 17, 33, 64, 65):
+        with profiling.collect() as seen:
+            got[M] = lin.forward(x[:M], out_dtype=torch.float32)
+        assert any("gemm_tile_kernel" in name for name in seen["kernels"]) == (tiled and 16 < M <= 64), (M, seen["kernels"])
+        assert (got[M].double() - want[:M]).norm() < 1e-6 * want[:M].norm()
+    if tiled:
+        assert torch.equal(got[64][:17], got[17]) and torch.equal(got[64][:33], got[33])

@@ -73,6 +73,12 @@ constexpr int TM_GEMV_F32_ROWS = 16;
 // and K from 3,584 to 5,120 up to 12% in heads of less than 65,536 (50,304 x 5,120: 95 to 107; 65,536 x 5,120 and 151,936 x 5,120 2 and 18% faster).
 inline bool tm_head_few(int M, int N, int K) { return M <= 8 || K <= 3072 || (N >= 65536 && K <= 5120); }
 
+// And the tiled kernel, of 17 to 64 rows? The library's time / the tiles', us, 17 / 33 / 64 rows: 151,936 x 896 65 / 53, 70 / 55, 74 / 64; 151,936 x 2,048
+// 147 / 121, 153 / 129, 158 / 137; 152,064 x 3,584 244 / 193, 201 / 201, 218 / 214; 128,256 x 4,096 198 / 185, 213 / 192, 220 / 197; 200,064 x 3,072 381 / 228,
+// 264 / 241, 285 / 258; 65,536 x 768 25.6 / 20.9, 26.7 / 22.3, 28.6 / 23.9; 50,304 x 1,024 and 32,000 x 2,048 and 4,096 level or to 3% less; 262,144 x 1,152
+// 127 / 116, 142 / 124, 147 / 139. 256,000 x 2,304 would be 1 to 4% slower, x 3,072 level. At 96 and 128 rows the tiles take 0.86 to 1.03 of the library's time.
+inline bool tm_head_tiled(int M, int N, int K) { return M > 16 && M <= 64 && (N <= 204800 || K < 2048); }
+
 // --- decode attention ---------------------------------------------------------------------------------
 constexpr int TM_DECODE_CHUNK = 256;        // keys per block of the split decode attention
 constexpr int TM_DECODE_F32_CHUNK = 128;    // the same in the 32-bit path, whose contexts are always split below that many pairs

@@ -179,6 +179,9 @@ struct Products {
             if (head_few) ++*head_few;
             return tm_gemv_bf16(x, ldx, L.w, (float*)out, ldc, M, L.N, L.K, stream);
         }
+        if (L.library_first && !L.bias && !L.act && out_dtype == TM_F32 && tune.candidates < 2 && tm_head_tiled(M, L.N, L.K) && tile_ok(L, x, ldx, M, dtype) &&
+            aligned(out, 16) && ldc == L.N)
+            return tm_tile_linear(x, ldx, M, L.K, L.w, L.N, out, ldc, out_dtype, stream);
         if (L.library_first) {
             const int rc = library(L, x, ldx, M, out, ldc, out_dtype);
             if (rc != TM_ERR_UNSUPPORTED) return then_act(rc);
