@@ -266,8 +266,8 @@ def test_few_rows_do_not_change_a_row_of_a_split_product(N, K):
     assert all(torch.equal(out, sums[64][:, :M]) for M, out in sums.items())
 
 
-# one wavefront, four, all; pairs that are held and that are not; experts without a pair, without matrices
-@pytest.mark.parametrize("T,E,real,top,rows", [(1, 1, 1, 1, 32), (128, 64, 64, 2, 64), (129, 64, 63, 2, 64), (5, 65, 65, 2, 32), (512, 256, 256, 2, 128), (513, 17, 16, 2, 64),
+# few experts; one wavefront, four, all; pairs that are held and that are not; experts without a pair, without matrices
+@pytest.mark.parametrize("T,E,real,top,rows", [(1, 1, 1, 1, 32), (1024, 16, 15, 2, 64), (1025, 16, 16, 2, 64), (100, 17, 17, 2, 32), (128, 64, 64, 2, 64), (129, 64, 63, 2, 64), (5, 65, 65, 2, 32), (512, 256, 256, 2, 128), (513, 17, 16, 2, 64),
                                                (3, 257, 257, 5, 32), (64, 1024, 1000, 8, 32), (64, 1024, 1024, 8, 32), (2048, 3, 3, 2, 128), (4097, 1, 1, 1, 64),
                                                (3000, 70, 64, 4, 128), (5, 8, 0, 2, 32)])
 def test_route(T, E, real, top, rows):

@@ -25,6 +25,7 @@
 
 #define MR_THREADS 1024
 #define MOE_MAX_EXPERTS 1024
+#define MR_FEW_EXPERTS 16
 
 // One block, bound by its trips to memory (the token, its table row) and to LDS. A pair's expert and its place in the expert's run come
 // from one pass: a thread asks for four pairs' tokens and then for their rows at once, the counter that counts a pair says its place,
@@ -136,12 +137,59 @@ __global__ __launch_bounds__(THREADS) void moe_route_kernel(const int* __restric
     }
 }
 
-// The fewest wavefronts that have a lane an expert and hold the pairs: barriers cost a block of one nothing. 1 token, 16 experts, top 2
-// 4.2 us in 16 wavefronts, 3.0 in one (2.9 with one thread laying out); 256 tokens 4.4 in 16, 3.4 in four (3.5).
+// The same for few experts and pairs: in a step the launch finds its code out of the instruction cache, and this is a quarter of it (16 experts,
+// top 2, 90 / 400 / 900 tokens between a layer's other launches, us: 4.2 / 5.2 / 7.3, the kernel above 5.2 / 6.0 / 7.4; at 1,500 10.3 / 9.3).
+__global__ __launch_bounds__(MR_THREADS) void moe_route_few_kernel(const int* __restrict__ ids, const int* __restrict__ table, int T,
+                                                                   int top, int E, int real, int tile_rows, int* __restrict__ slot_pair,
+                                                                   int* __restrict__ pair_slot, int* __restrict__ tiles,
+                                                                   int* __restrict__ n_tiles) {
+    __shared__ int cnt[MR_FEW_EXPERTS];
+    __shared__ int off[MR_FEW_EXPERTS + 1];
+    const int P = T * top;
+    for (int e = threadIdx.x; e < E; e += MR_THREADS) cnt[e] = 0;
+    __syncthreads();
+    for (int p = threadIdx.x; p < P; p += MR_THREADS) {
+        const int e = ids ? table[(size_t)ids[p / top] * top + p % top] : table[p];
+        if (e < real) atomicAdd(&cnt[e], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int at = 0, n = 0;
+        for (int e = 0; e < real; ++e) {
+            off[e] = at;
+            for (int r = 0; r < cnt[e]; r += tile_rows) {
+                tiles[3 * n] = e;
+                tiles[3 * n + 1] = at + r;
+                tiles[3 * n + 2] = min(tile_rows, cnt[e] - r);
+                ++n;
+            }
+            at += cnt[e];
+            cnt[e] = 0;
+        }
+        off[real] = at;
+        n_tiles[0] = n;
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < P; p += MR_THREADS) {
+        const int e = ids ? table[(size_t)ids[p / top] * top + p % top] : table[p];
+        if (e >= real) {                        // an expert without matrices: the pair has no slot
+            pair_slot[p] = -1;
+            continue;
+        }
+        const int slot = off[e] + atomicAdd(&cnt[e], 1);
+        slot_pair[slot] = p;
+        pair_slot[p] = slot;
+    }
+}
+
+// Otherwise the fewest wavefronts that have a lane an expert and hold the pairs (8 tokens, 64 experts, top 8 in one 3.1 us, in 16 4.4;
+// the one thread's runs and tiles 6.6).
 static int launch_moe_route(const int* ids, const int* table, int T, int top, int E, int real, int tile_rows, int* slot_pair, int* pair_slot,
                             int* tiles, int* n_tiles, hipStream_t stream) {
     static_assert(MOE_MAX_EXPERTS <= MR_THREADS, "");
-    if (E <= TM_WAVE && T * top <= 4 * TM_WAVE)
+    if (E <= MR_FEW_EXPERTS && T * top <= 2 * MR_THREADS)
+        moe_route_few_kernel<<<1, MR_THREADS, 0, stream>>>(ids, table, T, top, E, real, tile_rows, slot_pair, pair_slot, tiles, n_tiles);
+    else if (E <= TM_WAVE && T * top <= 4 * TM_WAVE)
         moe_route_kernel<TM_WAVE><<<1, TM_WAVE, 0, stream>>>(ids, table, T, top, E, real, tile_rows, slot_pair, pair_slot, tiles, n_tiles);
     else if (E <= 4 * TM_WAVE && T * top <= 16 * TM_WAVE)
         moe_route_kernel<4 * TM_WAVE><<<1, 4 * TM_WAVE, 0, stream>>>(ids, table, T, top, E, real, tile_rows, slot_pair, pair_slot, tiles, n_tiles);
