@@ -41,8 +41,8 @@ __device__ __forceinline__ void wave_keys64(const Bf16x8Bits (&qreg)[D / 32], co
     int entry[4];
     load_table_entries(entry, table, table_width, wbase, page_shift);
     Keys64<D> kv;
-    load_keys64<D>(kv, k_pool, v_pool, entry, wbase, ctx, keep, lo, kvh, KVH, page_shift, r, g);
-    attend_keys64<D>(kv, qreg, wbase, ctx, keep, lo, scale_log2, cap_in, cap_out, g, m, l, o);
+    load_keys64<D, true>(kv, k_pool, v_pool, entry, wbase, ctx, keep, lo, kvh, KVH, page_shift, r, g);
+    attend_keys64<D, true>(kv, qreg, wbase, ctx, keep, lo, scale_log2, cap_in, cap_out, g, m, l, o);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -191,8 +191,8 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
     f32x4_t o[NDT];
     {
         Keys64<D> kv;
-        load_keys64<D>(kv, k_pool, v_pool, entry, wbase, ctx, keep, lo, kvh, KVH, page_shift, r, g);
-        attend_keys64<D>(kv, qreg, wbase, ctx, keep, lo, scale_log2, cap_in, cap_out, g, m, l, o);
+        load_keys64<D, false>(kv, k_pool, v_pool, entry, wbase, ctx, keep, lo, kvh, KVH, page_shift, r, g);
+        attend_keys64<D, false>(kv, qreg, wbase, ctx, keep, lo, scale_log2, cap_in, cap_out, g, m, l, o);
     }
     if (g == 0) {
         s_m[wave][r] = m;

@@ -37,12 +37,19 @@ union Bf16x8Bits {
 // runs of four: row rho of tile t is key 32 (t / 2) + 8 (rho / 4) + 4 (t % 2) + rho % 4. The lane that holds
 // rows 4g..4g+3 of both tiles then has the keys 32b + 8g .. + 7: one 16-byte load, 64 bytes of a row an
 // instruction (4.7 TB/s), and half as many loads. The keys are whole rows of the pool either way.
+//
+// Neighbouring lanes of the first product's operand are in different rows: 64 addresses for a CU's address unit, one a cycle, where four lanes
+// beside each other in a row are one. TURN: four lanes load 64 bytes of a row (lane (4 q + p, g) row 4 q + g, piece p) and the pieces change
+// lanes in front of the product by ds_bpermute, four a load. us without / with (seven heads a kv head): the kernel of a whole context, 1 request of 300
+// keys, head sizes 64 / 128, 5.63 / 5.26, 7.54 / 6.61, 2 of 500 6.07 / 5.54, 16 of 300 6.08 / 5.76, 32 of 600, 128, 13.4 / 12.9, 64 of 1,021 11.1 / 10.8; the
+// block kernel, 128 of 2,000 25.6 / 25.1, 96 of 1,500, 128, 55.5 / 53.8. The split kernel, whose wavefronts have 64 keys and no more, has the
+// exchange in its one chain: 8 of 2,048, 128, 12.7 / 13.1, 64 level. It goes without. The same bits.
 __device__ __forceinline__ int tile_key(int t, int rho) { return 32 * (t / 2) + 8 * (rho / 4) + 4 * (t % 2) + rho % 4; }
 
 template <int D>
 struct Keys64 {
     int group_page[4];                      // page of the 16 positions [wbase + 16 q, + 16), -1 if no query may see them (wave-uniform)
-    Bf16x8Bits k[4][D / 32];                // [tile][32 d]
+    Bf16x8Bits k[4][D / 32];                // [tile][32 d], rows and pieces as loaded
     u32x4_t v[D / 16][2];                   // [16 d][32 keys]: keys 32 b + 8 g .. + 7 of row d = 16 dt + r
 };
 
@@ -59,7 +66,7 @@ __device__ __forceinline__ void load_table_entries(int (&entry)[4], const int* _
 }
 
 // Ask for the keys and values of [wbase, wbase + 64): every load is issued, nothing is waited for.
-template <int D>
+template <int D, bool TURN>
 __device__ __forceinline__ void load_keys64(Keys64<D>& kv, const bf16_t* __restrict__ k_pool,
                                             const bf16_t* __restrict__ v_pool, const int (&entry)[4], int wbase,
                                             int ctx, int keep, int lo, int kvh, int KVH, int page_shift, int r, int g) {
@@ -77,10 +84,10 @@ __device__ __forceinline__ void load_keys64(Keys64<D>& kv, const bf16_t* __restr
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
         // the 16 positions of a row's key: the pair's first 16 for rows 0..7, its second 16 for rows 8..15
-        const int key = wbase + tile_key(t, r);
-        const int page = r < 8 ? kv.group_page[2 * (t / 2)] : kv.group_page[2 * (t / 2) + 1];
+        const int row = TURN ? 4 * (r / 4) + g : r, piece = TURN ? r % 4 : g, key = wbase + tile_key(t, row);
+        const int page = row < 8 ? kv.group_page[2 * (t / 2)] : kv.group_page[2 * (t / 2) + 1];
         const size_t pg = page >= 0 ? (size_t)page : 0;
-        const bf16_t* kr = k_pool + (((pg << page_shift) + (key & page_mask)) * KVH + kvh) * D + 8 * g;
+        const bf16_t* kr = k_pool + (((pg << page_shift) + (key & page_mask)) * KVH + kvh) * D + 8 * piece;
 #pragma unroll
         for (int c = 0; c < NDC; ++c) kv.k[t][c].u = *(const u32x4_t*)(kr + 32 * c);
     }
@@ -100,18 +107,25 @@ __device__ __forceinline__ void load_keys64(Keys64<D>& kv, const bf16_t* __restr
 
 // The partial of the 64 keys in kv for the (up to 16) query heads of one kv head.
 // m is in units of score * scale * log2(e).
-template <int D>
+template <int D, bool TURN>
 __device__ __forceinline__ void attend_keys64(const Keys64<D>& kv, const Bf16x8Bits (&qreg)[D / 32], int wbase, int ctx,
                                               int keep, int lo, float scale_log2, float cap_in, float cap_out, int g, float& m, float& l,
                                               f32x4_t (&o)[D / 16]) {
     constexpr int NDC = D / 32, NDT = D / 16;
     float sc[4][4];                                                 // [tile][row 4g+i of the tile] for head r
+    const int r = threadIdx.x % 16, from = 4 * (16 * (r % 4) + 4 * (r / 4) + g);       // the lane, in bytes, that has row r's piece g
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
         f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < NDC; ++c)
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv.k[t][c].b, qreg[c].b, acc, 0, 0, 0);
+        for (int c = 0; c < NDC; ++c) {
+            Bf16x8Bits kf = kv.k[t][c];
+            if constexpr (TURN) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) kf.u[e] = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)kf.u[e]);
+            }
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.b, qreg[c].b, acc, 0, 0, 0);
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int kj = wbase + tile_key(t, 4 * g + i);
@@ -206,8 +220,8 @@ __device__ __forceinline__ void attend_whole(float* lds, int s, int kvh, const b
         if (wbase < ctx && (wbase + AD_WKEYS > lo || wbase < keep)) {       // else nothing of the run is visible
             f32x4_t o[NDT];
             Keys64<D> kv;
-            load_keys64<D>(kv, k_pool, v_pool, entry, wbase, ctx, keep, lo, kvh, KVH, page_shift, r, g);
-            attend_keys64<D>(kv, qreg, wbase, ctx, keep, lo, scale_log2, cap_in, cap_out, g, m, l, o);
+            load_keys64<D, true>(kv, k_pool, v_pool, entry, wbase, ctx, keep, lo, kvh, KVH, page_shift, r, g);
+            attend_keys64<D, true>(kv, qreg, wbase, ctx, keep, lo, scale_log2, cap_in, cap_out, g, m, l, o);
             if (r < G) {
 #pragma unroll
                 for (int dt = 0; dt < NDT; ++dt) *(f32x4_t*)(s_o + ((size_t)run * G + r) * ROW + 16 * dt + 4 * g) = o[dt];
