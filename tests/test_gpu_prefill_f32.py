@@ -47,6 +47,19 @@ def test_moving_reference(ops, D, step, n, H):
     assert (got.cpu() - want).abs().max() < bound
 
 
+@pytest.mark.parametrize("D,H,n", [(64, 12, 1008), (64, 12, 1024), (64, 64, 190), (96, 8, 1007), (96, 8, 1024), (128, 32, 255), (128, 32, 257), (80, 32, 400)])
+def test_a_tokens_bits_do_not_depend_on_the_launch(ops, D, H, n):
+    """From two or three blocks a CU on keys and values change lanes behind their loads: the bits of launches with fewer heads, and so fewer blocks."""
+    torch.manual_seed(n)
+    q, k, v = torch.randn(n, H, D, device=DEV), torch.randn(n, 2, D, device=DEV), torch.randn(n, 2, D, device=DEV)
+    full = attend(ops, q, k, v, H, 2, D, 16, D ** -0.5)
+    few = attend(ops, q[:, [0, H - 1]], k, v, 2, 2, D, 16, D ** -0.5)
+    assert torch.equal(full[:, [0, H - 1]], few)
+    s = torch.einsum("qhd,khd->hqk", q[:, [0, H - 1]].double(), k.double()) * D ** -0.5
+    want = torch.einsum("hqk,khd->qhd", s.masked_fill(torch.ones(n, n, device=DEV).triu(1).bool(), float("-inf")).softmax(-1), v.double())
+    assert (full[:, [0, H - 1]] - want).abs().max() < 2 ** -24 * s.abs().max() * 4.1 * D ** 0.5 * 2 + 2e-6      # (the bound above)
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
 def test_no_number_reaches_those_that_see_it(ops, bad):
     torch.manual_seed(1)

@@ -32,6 +32,15 @@
 // registers a CU holds more blocks (14 heads of 64, a window of 64 / 128, 1,000 tokens, with it 12.2 / 14.9 us, without 10.5 / 13.1; 3,000
 // 25.9 / 33.4 and 22.9 / 29.9; at 256 keys 44.9 with it)
 #define AF_SHORT_WALK 128
+// TURN: neighbouring lanes of the operands are in different rows, 64 addresses for a CU's address unit, one a clock, and four wavefronts
+// ask for twice what it can take while they multiply. So four lanes load 64 bytes of a row (lane (4 q + p, g) row 4 q + g, piece p) and the
+// pieces change lanes by ds_bpermute, four a load. us without / with: 28 heads over 4 of 128, 300 / 512 / 1,000 tokens 18.7 / 18.0, 38.2 / 35.4, 103 / 94;
+// 12 over 2 of 96, 800 / 1,500 26.5 / 25.2, 74.6 / 63.4; 14 over 2 of 64, 1,000 / 1,500 / 3,000 31.3 / 28.5, 59.7 / 54.3, 189 / 173. A launch of few blocks or of small heads
+// waits for the exchange instead: 14 of 64, 600 / 800 tokens 15.4 / 16.6, 22.0 / 22.0, 8 over 8 of 64, 1,000 20.3 / 22.5, 5 of 80, 2,500 59.8 / 63.0, 8 over 2
+// of 32, 3,000 56.4 / 55.9, 12 over 2 of 96, 300 10.9 / 11.8, 9 over 3 of 112, 1,500 56 / 60: head size 64 takes it from three blocks a CU, 96 and 128 from
+// two. The same bits.
+constexpr bool AF_TURNS(int D) { return D == 64 || D == 96 || D == 128; }
+constexpr int AF_TURN_BLOCKS(int D) { return D == 64 ? 768 : 512; }
 #define AF_ROUND 256        // blocks that come to rest on CUs of their own before the first CU gets a second one
 
 // A column's reference moves only when its maximum has grown by more than this (weights up to e^8 cost 32-bit sums nothing), so
@@ -53,7 +62,7 @@ struct KVBlock32 {
     f32x4_t k[D / 16], v[D / 16];
 };
 
-template <int D, bool CAP, bool AHEAD>
+template <int D, bool CAP, bool AHEAD, bool TURN>
 __global__ __launch_bounds__(64 * AF_SPLIT, AHEAD ? 2 : 1) void attn_prefill_f32_kernel(
     const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
     const float* __restrict__ k_pool, const float* __restrict__ v_pool, const int* __restrict__ block_tables,
@@ -94,7 +103,13 @@ __global__ __launch_bounds__(64 * AF_SPLIT, AHEAD ? 2 : 1) void attn_prefill_f32
     auto behind_gap = [&](int b) { return (b >= kb_kept && b < kb_first) ? kb_first + ((wave - kb_first) & (AF_SPLIT - 1)) : b; };
     // (behind the wavefront's last block the newest one there is again, unused: always at an entry this tile may see)
     auto page_of = [&](int b) { return table[((b <= kb_last ? b : kb_last) << 4) >> page_shift]; };
-    const uint32_t k_lane = ((uint32_t)r * KVH * D + 4 * g) * 4, v_lane = (((uint32_t)r << page_shift) + 4 * g) * 4;
+    const uint32_t row = TURN ? 4 * (r / 4) + g : r, piece = TURN ? r % 4 : g;
+    const uint32_t k_lane = (row * KVH * D + 4 * piece) * 4, v_lane = ((row << page_shift) + 4 * piece) * 4;
+    const int from = 4 * (16 * (r % 4) + 4 * (r / 4) + g);             // the lane, in bytes, that has row r's piece g
+    auto turn = [&](f32x4_t& v) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(v[e])));
+    };
     auto load = [&](KVBlock32<D>& blk, int b, int pg) {
         const int in_page = ((b <= kb_last ? b : kb_last) << 4) & (page - 1);
         // keys: lane (r, g) holds K[key0 + r][16 c + 4 g .. + 3]; values: V[d = 16 dt + r][key0 + 4 g .. + 3]
@@ -120,6 +135,12 @@ __global__ __launch_bounds__(64 * AF_SPLIT, AHEAD ? 2 : 1) void attn_prefill_f32
             pg_next = page_of(after);
         }
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (TURN) {
+#pragma unroll
+            for (int c = 0; c < NDT; ++c) turn(now.k[c]);
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) turn(now.v[dt]);
+        }
         // values of keys nobody may see yet (beyond the newest key) can hold anything: clear them
         if (key0 + 15 > last_key) {
 #pragma unroll
@@ -252,17 +273,20 @@ extern "C" int tm_attn_prefill_f32_cap(const void* q, int q_stride, void* out, i
     // (a launch has fewer than 2^32 threads: tables beyond that go in pieces)
     const int most = (1 << 23) / H;
     const bool short_walk = window > 0 && (long long)window + keep <= AF_SHORT_WALK;
-#define TM_PREFILL_F32_GO(DD, CAP, AHEAD)                                                                         \
+    const bool turn = AF_TURNS(D) && (long long)n_tiles * H >= AF_TURN_BLOCKS(D);
+#define TM_PREFILL_F32_GO(DD, CAP, AHEAD, TURN)                                                                   \
     for (int t = 0; t < n_tiles; t += most)                                                                       \
-        attn_prefill_f32_kernel<DD, CAP, AHEAD><<<(n_tiles - t < most ? n_tiles - t : most) * H, 64 * AF_SPLIT, 0, stream>>>( \
+        attn_prefill_f32_kernel<DD, CAP, AHEAD, TURN><<<(n_tiles - t < most ? n_tiles - t : most) * H, 64 * AF_SPLIT, 0, stream>>>( \
             (const float*)q, q_stride, (float*)out, out_stride, (const float*)k_pool, (const float*)v_pool,       \
             block_tables, table_width, tiles + (size_t)t * 4, H, KVH, page_shift, scale, window, keep, softcap, sink, (const float*)cgate, ldcg)
 #define TM_PREFILL_F32_CASE(DD)                                                                                   \
     case DD:                                                                                                      \
         if (short_walk) {                                                                                         \
-            if (softcap > 0.f) { TM_PREFILL_F32_GO(DD, true, false); } else { TM_PREFILL_F32_GO(DD, false, false); } \
+            if (softcap > 0.f) { TM_PREFILL_F32_GO(DD, true, false, false); } else { TM_PREFILL_F32_GO(DD, false, false, false); } \
+        } else if (!turn) {                                                                                       \
+            if (softcap > 0.f) { TM_PREFILL_F32_GO(DD, true, true, false); } else { TM_PREFILL_F32_GO(DD, false, true, false); } \
         } else {                                                                                                  \
-            if (softcap > 0.f) { TM_PREFILL_F32_GO(DD, true, true); } else { TM_PREFILL_F32_GO(DD, false, true); } \
+            if (softcap > 0.f) { TM_PREFILL_F32_GO(DD, true, true, AF_TURNS(DD)); } else { TM_PREFILL_F32_GO(DD, false, true, AF_TURNS(DD)); } \
         }                                                                                                         \
         break
     switch (D) {
