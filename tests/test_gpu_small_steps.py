@@ -60,6 +60,17 @@ def test_every_depth_of_a_round(ops, N, K):
             assert torch.equal(out, many[:M]), (M, matrix is w)
 
 
+@pytest.mark.parametrize("N,K", [(897, 4856), (1540, 2056), (3076, 2056), (3076, 904), (4100, 2056)])
+def test_every_number_of_few_tokens(ops, N, K):
+    """Activations whose pieces change lanes behind their loads and those that do not, on both sides of each line between them: a token's bits are one."""
+    torch.manual_seed(K + N)
+    a = torch.randn(16, K, device=DEV).to(BF)
+    packed = ops.pack_weight((torch.randn(N, K, device=DEV) * K ** -0.5).to(BF), ops.skinny_strip_rows(N, K))
+    outs = [ops.gemm_skinny(a[:M], packed, None, torch.full((M, N), float("nan"), device=DEV)) for M in range(1, 17)]
+    for M, out in enumerate(outs, 1):
+        assert torch.equal(out, outs[15][:M]), M
+
+
 @pytest.mark.parametrize("M", [3, 7, 12])
 @pytest.mark.parametrize("N", [896, 1536])
 def test_what_is_no_number_stays_with_its_token_and_its_row(ops, M, N):

@@ -79,7 +79,13 @@ __device__ __forceinline__ float bias_at(const void* bias, int flags, int n) {
 // every other, in order) and the order in which the VW sums are added are those of gemm_skinny_kernel with VW wavefronts, so the
 // bits are the same for any number of tokens. Loads are unconditional: what lies beyond the strip, a token or a range
 // reads as zero by the bounds of its buffer descriptor.
-template <int ROWS, int TOKS, int VW, int CH, typename TC, bool PACKED>
+//
+// TURN: neighbouring lanes of the B operand are different tokens, one address a clock for the CU, and the loads of activations were most of a launch
+// whose matrix lies in the caches. Four lanes beside each other load 64 bytes of a token (lane (4 q + p, g) column 4 q + g, piece p) and the
+// pieces change lanes by ds_bpermute. us without / with, matrices in the caches (brought ahead, as in a step) and cold: 4,864 -> 896 4 tokens 3.87 / 3.41
+// and 4.75 / 4.63, 8 5.05 / 4.44 and 6.15 / 5.88, 16 7.18 / 6.25 and 8.75 / 8.32; 8,960 -> 1,536 8 7.63 / 5.74 and 10.4 / 9.9; 18,944 -> 3,584 8 21.4 / 21.1
+// and 28.2 / 27.4; 896 -> 9,728 16 5.25 / 3.88 and 7.1 / 6.9. The rule is few_turns below. The same bits.
+template <int ROWS, int TOKS, int VW, int CH, typename TC, bool PACKED, bool TURN>
 __global__ __launch_bounds__(64 * VW * ROWS / 16) void gemm_few_kernel(const bf16_t* __restrict__ A, int lda,
                                                                        const bf16_t* __restrict__ W,
                                                                        const void* __restrict__ bias, int flags,
@@ -122,14 +128,16 @@ __global__ __launch_bounds__(64 * VW * ROWS / 16) void gemm_few_kernel(const bf1
     };
     // the activations: lane (r, g) has token r % TOKS, eight k at 8 g of a k-step of range b SB + r / TOKS
     const __amdgpu_buffer_rsrc_t abuf = fd_buffer(A, ((M - 1) * lda + K) * 2);
+    const int column = TURN ? 4 * (r / 4) + g : r, piece = TURN ? r % 4 : g;      // what it loads
+    const int from = 4 * (16 * (r % 4) + 4 * (r / 4) + g);                        // the lane, in bytes, that has column r's piece g
     int a_k[NB], a_end[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-        const int ks = (range0 + b * SB + r / TOKS) * per, end = ks + per < ksteps ? ks + per : ksteps;
-        a_k[b] = ks * 32 + 8 * g;
-        a_end[b] = r % TOKS < M ? (end * 32 < K ? end * 32 : K) : 0;
+        const int ks = (range0 + b * SB + column / TOKS) * per, end = ks + per < ksteps ? ks + per : ksteps;
+        a_k[b] = ks * 32 + 8 * piece;
+        a_end[b] = column % TOKS < M ? (end * 32 < K ? end * 32 : K) : 0;
     }
-    const int a_row = (r % TOKS) * lda;
+    const int a_row = (column % TOKS) * lda;
 
     f32x4_t acc[NB];
 #pragma unroll
@@ -155,7 +163,13 @@ __global__ __launch_bounds__(64 * VW * ROWS / 16) void gemm_few_kernel(const bf1
 #pragma unroll
         for (int j = 0; j < CH; ++j)
 #pragma unroll
-            for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j].b, af[b][j].b, acc[b], 0, 0, 0);
+            for (int b = 0; b < NB; ++b) {
+                if constexpr (TURN) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) af[b][j].u[e] = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)af[b][j].u[e]);
+                }
+                acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j].b, af[b][j].b, acc[b], 0, 0, 0);
+            }
     }
     // lane: rows 4 g + i of the tile, so range 4 g / ROWS of the matrix; columns of range r / TOKS in each of the NB groups
     const int range = 4 * g / ROWS;
@@ -201,6 +215,14 @@ static int few_depth(int per, int a, int b, int c, int d) {
     return a * rounds >= per ? a : b * rounds >= per ? b : c * rounds >= per ? c : d;
 }
 
+// Do the activations' pieces change lanes behind their loads? Where the loads are many (a long K; else strips of 16 rows) and the tokens fill their
+// places: with 9 of 16 and 5 of 8 tokens 4,864 -> 896 takes 6.0 for 5.7 and 4.4 for 4.3 us, with 4 of 16 4,096 -> 4,096 6.0 for 5.7 (18,944 -> 3,584 level
+// up to 5); over a short K and strips of 4 or 8 rows the exchange is longer than the wait (896 -> 896 8 tokens 3.0 / 3.4, 1,536 -> 1,536 3.2 / 3.3).
+static bool few_turns(int rows, int M, bool long_k) {
+    if (!long_k) return rows == 16 && M >= 10;
+    return rows == 4 ? 4 * M >= 3 * (M <= 4 ? 4 : M <= 8 ? 8 : 16) : M >= (rows == 8 ? 4 : 6);
+}
+
 // Ranges of K: 4, or 16 for a long K over few strips. `rows`: of a strip (16, 8 or 4).
 template <typename TC, bool PACKED>
 static int launch_few(const void* A, int lda, const void* W, int rows, const void* bias, int flags, void* C, int ldc, int M, int N,
@@ -216,16 +238,20 @@ static int launch_few(const void* A, int lda, const void* W, int rows, const voi
     const int strips = (N + rows - 1) / rows;
     const bool long_k = K >= 2048 && !(rows == 16 && strips >= 256);
     const int ksteps = (K + 31) / 32, per = long_k ? (ksteps + 15) / 16 : (ksteps + 3) / 4;
-#define TM_FEW(ROWS_, TOKS_, VW_, CH_)                                                                                \
-    gemm_few_kernel<ROWS_, TOKS_, VW_, CH_, TC, PACKED><<<strips, 4 * VW_ * ROWS_, 0, stream>>>(                      \
+    const bool turn = PACKED && few_turns(rows, M, long_k);
+#define TM_FEW(ROWS_, TOKS_, VW_, CH_, TURN_)                                                                         \
+    gemm_few_kernel<ROWS_, TOKS_, VW_, CH_, TC, PACKED, TURN_><<<strips, 4 * VW_ * ROWS_, 0, stream>>>(               \
         (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc)
-#define TM_FEW_DEEP(ROWS_, TOKS_, VW_, A_, B_, C_, D_)                                                                \
+#define TM_FEW_DEPTHS(ROWS_, TOKS_, VW_, A_, B_, C_, D_, TURN_)                                                       \
     switch (few_depth(per, A_, B_, C_, D_)) {                                                                         \
-        case A_: TM_FEW(ROWS_, TOKS_, VW_, A_); break;                                                                \
-        case B_: TM_FEW(ROWS_, TOKS_, VW_, B_); break;                                                                \
-        case C_: TM_FEW(ROWS_, TOKS_, VW_, C_); break;                                                                \
-        default: TM_FEW(ROWS_, TOKS_, VW_, D_);                                                                       \
+        case A_: TM_FEW(ROWS_, TOKS_, VW_, A_, TURN_); break;                                                         \
+        case B_: TM_FEW(ROWS_, TOKS_, VW_, B_, TURN_); break;                                                         \
+        case C_: TM_FEW(ROWS_, TOKS_, VW_, C_, TURN_); break;                                                         \
+        default: TM_FEW(ROWS_, TOKS_, VW_, D_, TURN_);                                                                \
     }
+#define TM_FEW_DEEP(ROWS_, TOKS_, VW_, A_, B_, C_, D_)                                                                \
+    if (turn) { TM_FEW_DEPTHS(ROWS_, TOKS_, VW_, A_, B_, C_, D_, (PACKED && (VW_ == 16 || ROWS_ == 16))) }            \
+    else { TM_FEW_DEPTHS(ROWS_, TOKS_, VW_, A_, B_, C_, D_, false) }
     if (rows == 4 && long_k) {
         if (M <= 4) { TM_FEW_DEEP(4, 4, 16, 4, 6, 8, 10) }
         else if (M <= 8) { TM_FEW_DEEP(4, 8, 16, 4, 6, 8, 10) }
@@ -245,6 +271,7 @@ static int launch_few(const void* A, int lda, const void* W, int rows, const voi
     } else {
         TM_FEW_DEEP(16, 16, 4, 7, 8, 10, 14)
     }
+#undef TM_FEW_DEPTHS
 #undef TM_FEW_DEEP
 #undef TM_FEW
     TM_CHECK_LAUNCH();
