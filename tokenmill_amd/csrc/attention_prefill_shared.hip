@@ -10,7 +10,7 @@
 //   Every wavefront visits all key blocks of its tokens in ascending order, in stages aligned to absolute
 //   positions (multiples of 64), so a token's result does not depend on how its prompt was cut into
 //   portions nor on the rest of the batch. (It differs by rounding from the other kernel's, whose
-//   wavefronts split the key blocks among them: which kernel runs depends on the model's shape only.)
+//   wavefronts split the key blocks among them: which kernel runs depends on the model's shape and the number of tiles.)
 //
 //   S^T = K Q^T      A = keys  [16 keys x 32 d]   from LDS, rows in tile order (see stage_row)
 //                    B = Q^T   [32 d x 16 tokens] in registers

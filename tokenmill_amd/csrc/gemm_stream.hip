@@ -388,7 +388,7 @@ __global__ __launch_bounds__(64 * KS * US) void gemm_stream_kernel(const StreamA
 // A CU holds one block of these kernels (at 128 registers a lane a CU has room for 16 wavefronts), so a launch
 // should be one round of at most 256 blocks, as close to 256 as the units allow: US = the fewest units a block
 // that leave at most 256 blocks, and two wavefronts a unit from three units a block on (four with two units,
-// eight with one). Measured on an MI355X, 8 / 32 / 64 tokens (us): gate|up 7B (1,184 units) 2 x 5 = 237 blocks:
+// eight with one). Measured on an MI355X with rounds of four k-steps, 8 / 32 / 64 tokens (us): gate|up 7B (1,184 units) 2 x 5 = 237 blocks:
 // 53 / 50 / 55 (2 x 8 = 148 blocks: 58 / 61 / 68; 2 x 6: 54 / 53 / 57; 3 x 5: 48 / 50 / 78; 1 x 4 = 296 blocks: - / 60 / 73;
 // 4 x 4: - / 70 / 100); gate|up 32B (1,728 units) 2 x 8 = 216 blocks: 95 / 98 / 101 (2 x 7 = 247: 94 / 97 / 106, a few registers spilled; 2 x 6 = 288
 // blocks, a second round: 133 / 134 / 142; 1 x 4: - / 97 / 110); gate|up 0.5B (304 units) 4 x 2: - / 9 / 13 (8 x 1: - / 14 / 21);
@@ -405,7 +405,7 @@ static void stream_config(int n_units, int* ks, int* us) {
 static void stream_plain_shape(int N, int K, int* parts, int* ks, int* us) {
     const int n_units = (N + 31) / 32, ksteps = (K + 31) / 32;
     // Wide outputs over a K that gives every wavefront four k-steps: eight groups of blocks, two wavefronts a unit, and
-    // the fewest units a block that leave at most 256 blocks. Measured on an MI355X, 8 / 32 / 64 tokens (us): 7B down
+    // the fewest units a block that leave at most 256 blocks. Measured on an MI355X with rounds of four k-steps, 8 / 32 / 64 tokens (us): 7B down
     // (112 units, K 18,944) 8 groups of 2 x 4 = 224 blocks: 27 / 29 / 34 (3 x 4: 26 / 29 / 33; 4 x 4: 26 / 29 / 41; 4 groups
     // of 4 x 2: - / 30 / 39; 8 of 2 x 8 = 112 blocks: - / 36 / 42; unsplit - / 56 / 81; the library's product with its
     // algorithm chosen by timing - / 52 / 69); 7B o: 8 / 10 / 13 (4 groups of 4 x 2: - / 10 / 13); 32B down (160 units,

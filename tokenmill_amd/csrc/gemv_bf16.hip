@@ -2,7 +2,7 @@
 // row-major matrix.
 //
 // It is bound by reading the matrix once, 272 MB at the 0.5B shape, so the loads are whole lines: two steps of 32 k of eight rows an instruction, 128 bytes of
-// each, passing the caches by; lanes exchange what belongs to rows of the other eight (line_pair_half; gemv_f32.hip has why). A block takes RT tiles of
+// each, passing the caches by; lanes exchange what belongs to rows of the other eight (line_pair_half). A block takes RT tiles of
 // 16 matrix rows, which share the activations, its wavefronts split K and their sums meet in LDS, in halves. Which k goes where depends on the matrix alone.
 // choose.h says which heads it takes (tm_head_few). Against the library's product, cold matrices, us: 151,936 x 896 at 1 / 8 rows 51 / 52 to 40 / 44, 152,064 x 3,584 226 / 239 to 164 / 170 (6.6 and 6.4 TB/s).
 #include "common.h"
