@@ -71,3 +71,62 @@ def test_every_piece_of_a_launch_is_somebodys(shared, D, KVH, tiles):
         for t in range(0, tiles, 256 // wide):
             attend(slice(t, t + 256 // wide), heads, part)
         assert torch.equal(part.view(n, -1), dealt.view(n, KVH, -1)[:, lo:heads[1]].reshape(n, -1))
+
+
+# (head size, kv heads, heads of each, tokens, page, window, softcap, shared keys) and what the bits of the result add up to (bits_of_a_prompt)
+BITS = {
+    (32, 2, 3, 300, 16, 0, 0.0, False): 273273644921,
+    (64, 2, 7, 33, 16, 0, 0.0, False): 903370577692,
+    (64, 2, 7, 700, 64, 0, 0.0, False): 263496069408,
+    (64, 1, 4, 333, 32, 70, 0.0, False): 291748353217,
+    (96, 2, 3, 260, 16, 0, 20.0, False): 543656972435,
+    (128, 4, 2, 500, 16, 0, 0.0, False): 767424335260,
+    (96, 2, 5, 260, 16, 0, 0.0, True): 154814135182,
+    (128, 4, 7, 500, 32, 90, 0.0, True): 16163658554,
+}
+
+
+def bits_of_a_prompt(D, KVH, G, n, page, window, softcap, shared):
+    """Attention over numbers made from their places; its bits weighted and added up modulo 2^40."""
+    from tokenmill_amd.hip import ops
+
+    def numbers(*size, seed):
+        i = torch.arange(torch.Size(size).numel()) * 2654435761 + seed * 40503
+        i = (i ^ (i >> 13)) * 1103515245 % 2 ** 31
+        return ((i >> 8) % 4096 - 2048).float().div(800).view(size).to(BF).to(DEV)
+
+    pages, H = -(-n // page), KVH * G
+    out = torch.empty(n, H * D, dtype=BF, device=DEV)
+    tables = torch.arange(pages - 1, -1, -1, dtype=torch.int32, device=DEV).view(1, -1)
+    tiles = torch.tensor([(0, j, min(16, n - j), j) for j in reversed(range(0, n, 16))], dtype=torch.int32, device=DEV)
+    ops.attn_prefill_mfma(numbers(n, H * D, seed=1), out, numbers(pages, page, KVH, D, seed=2), numbers(pages, KVH, D, page, seed=3), tables, tiles,
+                          H, KVH, D, D ** -0.5, window, softcap=softcap, shared=shared)
+    bits = out.view(torch.int16).long().flatten().cpu()
+    return int((bits * (torch.arange(bits.numel()) % 1000003 + 1)).sum()) % 2 ** 40
+
+
+@pytest.mark.parametrize("case", BITS)
+def test_the_bits_of_a_prompt_stay(case):
+    """The order in which keys are added up, within a block of the matrix unit too, is part of what a prompt gives: the same numbers by any way the
+    keys and values are loaded. Which keys of a block stand in which place shows in the last bits alone, and nowhere else."""
+    assert bits_of_a_prompt(*case) == BITS[case]
+
+
+@pytest.mark.parametrize("D,KVH,G", [(32, 2, 3), (64, 2, 7), (64, 2, 2), (96, 3, 2), (96, 3, 1), (128, 2, 4)])
+@pytest.mark.parametrize("n", [31, 300])
+def test_the_size_of_a_page_changes_no_bit(D, KVH, G, n):
+    """Values come in other pieces out of pages of 16 than out of longer ones."""
+    from tokenmill_amd.hip import ops
+
+    g = torch.Generator(device=DEV).manual_seed(D + n)
+    H, most = KVH * G, 64 * -(-n // 64)
+    q, k, v = (torch.randn(m, heads, D, generator=g, device=DEV).to(BF) for m, heads in ((n, H), (most, KVH), (most, KVH)))
+    tiles = torch.tensor([(0, j, min(16, n - j), j) for j in reversed(range(0, n, 16))], dtype=torch.int32, device=DEV)
+    got = []
+    for page in (16, 32, 64):
+        out = torch.full((n, H * D), 3.0, dtype=BF, device=DEV)
+        tables = torch.arange(most // page, dtype=torch.int32, device=DEV).view(1, -1)
+        ops.attn_prefill_mfma(q.view(n, -1), out, k.view(-1, page, KVH, D), v.view(-1, page, KVH, D).permute(0, 2, 3, 1).contiguous(), tables, tiles, H, KVH, D,
+                              D ** -0.5, 0)
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])

@@ -25,21 +25,27 @@
 #include <algorithm>
 #include <limits.h>
 
-// A block of 32 keys as a wavefront holds it between asking for it and using it. Row rho of operand tile t is key 8 (rho / 4) + 4 t + rho % 4,
-// so that the lane which holds rows 4 g .. 4 g + 3 of both tiles of the scores has the eight keys 8 g .. 8 g + 7 of a row of V^T in one piece.
+// A block of 32 keys as a wavefront holds it between asking for it and using it. Row rho of operand tile t is key 16 t + rho: the lane which holds
+// rows 4 g .. 4 g + 3 of both tiles of the scores has the keys 4 g .. + 3 of either, and wants the same of a row of V^T.
 //
 // What bounds a long prompt is the address unit of a CU, beside its vector units: it takes 64 bytes a cycle where four neighbouring lanes ask for a
 // piece of one line, and one lane a cycle where they are in different keys, as the lanes of a score operand are (a key a lane). So keys are
-// loaded as whole rows, eight lanes a row of 64, and change lanes through LDS (attend_block), and values come 16 bytes a lane. At 8,000 tokens of the 0.5B
-// shape the first-level caches had 112 million accesses in 443,000 cycles, one a cycle and CU, and have 43 million in 385,000; keys, 77 / 512 /
-// 2,048 / 8,000 tokens, us a launch 5.0 / 8.5 / 25.7 / 212 to 4.6 / 6.9 / 23.6 / 186. (Keys by loads of half rows that lanes exchange in
-// registers, which ask for as many places: 26.1 and 215. The next block's keys through LDS behind this block's last score products, a
+// loaded as whole rows, eight lanes a row of 64, and change lanes through LDS (attend_block). At 8,000 tokens of the 0.5B shape the first-level
+// caches had 112 million accesses in 443,000 cycles, one a cycle and CU, and have 43 million in 385,000. (Keys by loads of half rows that lanes exchange in
+// registers ask for as many places: 2,048 / 8,000 tokens 26.1 and 215 us. The next block's keys through LDS behind this block's last score products, a
 // wait less: spills, 27.0 and 197.)
+//
+// HALVES: values come as two loads of eight bytes a lane. In pages of 16 keys, whose rows of V^T lie side by side, that is the better way where a
+// wavefront has two heads of more than 64 channels or four; else they come 16 bytes a lane, half of which belong to the lane 16 on (turn_values). us a launch, keys a
+// lane and eight bytes / keys by rows and 16 bytes / by rows and eight bytes: 14 heads over 2 of 64, pages of 16, 77 / 512 / 2,048 / 8,000 tokens
+// 4.87 / 4.58 / 4.68, 7.9 / 6.4 / 6.7, 24.2 / 22.3 / 21.7, 209 / 195 / 186, pages of 64, 77 / 3,001 6.5 / 4.8 / 5.6, 87 / 49 / 60; 16 over 16, 1,500
+// 40.6 / 27.0 / 29.3; 12 over 2 of 96, 600 / 2,500 10.1 / 10.4 / 9.5, 56.7 / 57.6 / 50.7; 32 over 8 of 128, 1,500 78.2 / 78.2 / 67.6; 12 over 2 of 96, pages of 64, 700
+// 16.6 / 11.8 / 13.9. The same bits.
 template <int D>
 struct KVBlock {
-    static constexpr int PIECES = D / 8, ROW = 2 * D + 16, TILE = 16 * ROW + 128;       // 16-byte pieces of a key; bytes of a key and of a tile in LDS
+    static constexpr int PIECES = D / 8, ROW = 2 * D + 16, TILE = 16 * ROW;       // 16-byte pieces of a key; bytes of a key and of a tile in LDS
     u32x4_t k[2][D / 32];   // [16 keys][c]: piece 64 c + lane of the keys as they lie
-    PFrag v[D / 16];        // [d tile]: keys 8 g .. 8 g + 7 of row d = r
+    PFrag v[D / 16];        // [d tile]: of row d = r, keys 4 g .. + 3 of both tiles (HALVES), or 8 (g / 2) .. + 7 of tile g % 2
 };
 
 // Floats of LDS that a wavefront has: its partials of all heads, and before that a block's keys.
@@ -50,8 +56,8 @@ constexpr int wave_floats() { return HPW * 16 * (D + 4) > KVBlock<D>::TILE / 2 ?
 template <int D>
 struct LaneOffsets {
     uint32_t k[D / 32];     // bytes: piece 64 c + lane of the tile's keys
-    uint32_t v;             // bytes: d = r, keys 8 (g % 2) .. + 7 of tile g / 2
-    uint32_t turn[2][D / 32];   // bytes in LDS: where they go
+    uint32_t v;             // bytes: d = r, and the keys (KVBlock)
+    uint32_t turn[D / 32];  // bytes in LDS: where a tile's keys go
     uint32_t row;           // bytes in LDS: piece g of row r
 };
 
@@ -91,7 +97,7 @@ __device__ __forceinline__ TilePlaces lane_pages(int kb, const BlockWalk& walk, 
 }
 
 // Loads one block of 32 keys (two tiles of 16); slot = which of the 32 blocks held in `places`.
-template <int D>
+template <int D, bool HALVES>
 __device__ __forceinline__ void load_kv_block(KVBlock<D>& blk, const TilePlaces& places, int slot, const bf16_t* __restrict__ k_pool,
                                               const bf16_t* __restrict__ v_pool, int page_shift, const LaneOffsets<D>& off) {
 #pragma unroll
@@ -102,13 +108,37 @@ __device__ __forceinline__ void load_kv_block(KVBlock<D>& blk, const TilePlaces&
         for (int c = 0; c < D / 32; ++c) blk.k[t][c] = __builtin_amdgcn_raw_buffer_load_b128(kbuf, off.k[c], 0, 0);
     }
     const uint32_t v0 = __builtin_amdgcn_readlane(places.v, 2 * slot), v1 = __builtin_amdgcn_readlane(places.v, 2 * slot + 1);
-    const char* vp = (const char*)v_pool + ((uint64_t)(threadIdx.x & 32 ? v1 : v0) << 5) + off.v;
+    if constexpr (HALVES) {
+        const __amdgpu_buffer_rsrc_t b0 = uniform_buffer((const char*)v_pool + ((uint64_t)v0 << 5)), b1 = uniform_buffer((const char*)v_pool + ((uint64_t)v1 << 5));
 #pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) blk.v[dt].u = *(const u32x4_t*)(vp + ((size_t)(32 * dt) << page_shift));
+        for (int dt = 0; dt < D / 16; ++dt) {
+            const u32x2_t lo = __builtin_amdgcn_raw_buffer_load_b64(b0, off.v, (32 * dt) << page_shift, 0);
+            const u32x2_t hi = __builtin_amdgcn_raw_buffer_load_b64(b1, off.v, (32 * dt) << page_shift, 0);
+            blk.v[dt].u = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+        }
+    } else {
+        const char* vp = (const char*)v_pool + ((uint64_t)(threadIdx.x & 16 ? v1 : v0) << 5) + off.v;
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) blk.v[dt].u = *(const u32x4_t*)(vp + ((size_t)(32 * dt) << page_shift));
+    }
+}
+
+// Lane (r, g) has keys 4 g .. + 3 of one tile and the lane 16 on those of the other, each beside four that the other wants: an instruction a word
+// changes them (rows of 16 lanes: the odd ones of the first operand with the even ones of the second).
+template <int D>
+__device__ __forceinline__ void turn_values(KVBlock<D>& blk) {
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt)
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const auto both = __builtin_amdgcn_permlane16_swap(blk.v[dt].u[w], blk.v[dt].u[w + 2], false, false);
+            blk.v[dt].u[w] = both[0];
+            blk.v[dt].u[w + 2] = both[1];
+        }
 }
 
 // One block of 32 keys against the wavefront's heads.
-template <int D, int HPW, bool CAP>
+template <int D, int HPW, bool CAP, bool HALVES>
 __device__ __forceinline__ void attend_block(KVBlock<D>& blk, unsigned char* turn, const LaneOffsets<D>& off, HeadState<D, HPW>& st, const PFrag (&qf)[HPW][D / 32],
                                              int key0, int nh, const TileView& tv, int g, float scale_log2, float cap_in, float cap_out) {
     constexpr int NDC = D / 32, NDT = D / 16;
@@ -117,7 +147,7 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, unsigned char* tur
         uint32_t seen[4];
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-            const int k0 = key0 + 8 * g + 2 * w;
+            const int k0 = key0 + (HALVES ? 4 * g + 16 * (w / 2) + 2 * (w % 2) : 16 * (g % 2) + 8 * (g / 2) + 2 * w);
             seen[w] = (tv.seen(k0) ? 0x0000ffffu : 0u) | (tv.seen(k0 + 1) ? 0xffff0000u : 0u);
         }
 #pragma unroll
@@ -125,12 +155,13 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, unsigned char* tur
 #pragma unroll
             for (int w = 0; w < 4; ++w) blk.v[dt].u[w] &= seen[w];
     }
+    if constexpr (!HALVES && D <= 64) turn_values(blk);
     // the keys change lanes: whole rows as they were loaded, a row a lane as the matrix unit takes them (rows 16 bytes more than their values
     // apart meet no bank twice)
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int c = 0; c < NDC; ++c) *(u32x4_t*)(turn + off.turn[t][c]) = blk.k[t][c];
+        for (int c = 0; c < NDC; ++c) *(u32x4_t*)(turn + t * KVBlock<D>::TILE + off.turn[c]) = blk.k[t][c];
     // (a wavefront's LDS instructions are done in their order; this holds the compiler to it)
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -169,7 +200,7 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, unsigned char* tur
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int kj = key0 + 8 * g + 4 * t + i;
+                    const int kj = key0 + 16 * t + 4 * g + i;
                     const bool mine = (kj <= tv.my_pos) & ((kj >= tv.my_lo) | (kj < tv.keep));
 #pragma unroll
                     for (int j = 0; j < AT_ONCE; ++j) sc[j][t][i] = mine ? sc[j][t][i] : -INFINITY;
@@ -210,6 +241,7 @@ __device__ __forceinline__ void attend_block(KVBlock<D>& blk, unsigned char* tur
                     for (int i = 0; i < 4; ++i) st.o[hh][dt][i] *= corr;
             }
         }
+        if constexpr (!HALVES && D > 64 && h0 == 0) turn_values(blk);      // (behind the scores up to 64 channels the registers do not hold it: 22.3 to 25.2 us at 2,048)
 #pragma unroll
         for (int j = 0; j < AT_ONCE; ++j) {
             const int hh = h0 + j;
@@ -274,7 +306,7 @@ struct NoDecodes {};
 template <bool DECODES>
 using DecodesArg = std::conditional_t<DECODES, KernelDecodes, NoDecodes>;
 
-template <int D, int HPW, int KS, bool CAP, bool AHEAD, bool DECODES>
+template <int D, int HPW, int KS, bool CAP, bool AHEAD, bool DECODES, bool HALVES>
 __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
@@ -321,11 +353,9 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
     for (int c = 0; c < NDC; ++c) {
         const int key = (64 * c + lane) / Block::PIECES, piece = (64 * c + lane) % Block::PIECES;
         off.k[c] = (uint32_t)(((size_t)key * KVH * D + 8 * piece) * sizeof(bf16_t));
-#pragma unroll
-        for (int t = 0; t < 2; ++t)                                  // key 16 t + key is row 4 (. / 8) + . % 4 of tile . / 4 % 2
-            off.turn[t][c] = (uint32_t)((key / 4 % 2) * Block::TILE + (8 * t + 4 * (key / 8) + key % 4) * Block::ROW + 16 * piece);
+        off.turn[c] = (uint32_t)(key * Block::ROW + 16 * piece);
     }
-    off.v = (uint32_t)((((size_t)r << page_shift) + 8 * (g % 2)) * sizeof(bf16_t));
+    off.v = (uint32_t)((((size_t)r << page_shift) + (HALVES ? 4 * g : 8 * (g / 2))) * sizeof(bf16_t));
     off.row = (uint32_t)(r * Block::ROW + 16 * g);
     unsigned char* turn = (unsigned char*)partial_at(wave, 0, 0, 0);         // (the place of this wavefront's partials, which are stored behind the last block)
     const int other = n_tiles - 1 - tile0;
@@ -363,7 +393,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
             for (int c = 0; c < NDC; ++c) qf[hh][c].u = *(const u32x4_t*)(qrow + (size_t)(h0 + (hh < nh ? hh : nh - 1)) * D + 32 * c);
     };
     begin(tile0);
-    load_kv_block<D>(ba, pages, 0, k_pool, v_pool, page_shift, off);
+    load_kv_block<D, HALVES>(ba, pages, 0, k_pool, v_pool, page_shift, off);
 
 #pragma unroll 1
     for (int which = 0; which < n_mine; ++which) {
@@ -384,8 +414,8 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
                 pages = lane_pages<D, KS>(walk.at<KS>(kb, kb + KS), walk, lane, kept_tiles, first_tile, last_tile, table, kvh, KVH, page_shift);
                 slot = -1;
             }
-            load_kv_block<D>(bb, pages, slot + 1, k_pool, v_pool, page_shift, off);
-            attend_block<D, HPW, CAP>(ba, turn, off, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
+            load_kv_block<D, HALVES>(bb, pages, slot + 1, k_pool, v_pool, page_shift, off);
+            attend_block<D, HPW, CAP, HALVES>(ba, turn, off, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
             kb = walk.at<KS>(kb, kb + KS);
             ++slot;
             if (kb > kb1) break;
@@ -393,8 +423,8 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
                 pages = lane_pages<D, KS>(walk.at<KS>(kb, kb + KS), walk, lane, kept_tiles, first_tile, last_tile, table, kvh, KVH, page_shift);
                 slot = -1;
             }
-            load_kv_block<D>(ba, pages, slot + 1, k_pool, v_pool, page_shift, off);
-            attend_block<D, HPW, CAP>(bb, turn, off, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
+            load_kv_block<D, HALVES>(ba, pages, slot + 1, k_pool, v_pool, page_shift, off);
+            attend_block<D, HPW, CAP, HALVES>(bb, turn, off, st, qf, kb * 32, nh, tv, g, scale_log2, cap_in, cap_out);
             kb = walk.at<KS>(kb, kb + KS);
             ++slot;
         }
@@ -415,7 +445,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) *(f32x4_t*)partial_at(wave, hh, r, 16 * dt + 4 * g) = st.o[hh][dt];    // lane: d = 16 dt + 4 g + i of token r
         }
-        if (more) load_kv_block<D>(ba, pages, 0, k_pool, v_pool, page_shift, off);
+        if (more) load_kv_block<D, HALVES>(ba, pages, 0, k_pool, v_pool, page_shift, off);
         __syncthreads();
         // a thread: four channels of a token and head
         for (int idx = threadIdx.x; idx < nh * 16 * (D / 4); idx += 64 * KS) {
@@ -497,8 +527,8 @@ static int launch_split_keys(const void* q, int q_stride, void* out, int out_str
     if (far) ahead.n = 0;
     grid.z = 1 + front + (far ? 0 : ahead_spare_layers(ahead, layer, layer + pairs));
     if (front) ahead.first = (int)layer * (1 + front);
-    auto go = [&](auto AHEAD, auto DECODES) {
-        constexpr bool with = decltype(AHEAD)::value, decode = decltype(DECODES)::value;
+    auto go = [&](auto AHEAD, auto DECODES, auto PIECES) {
+        constexpr bool with = decltype(AHEAD)::value, decode = decltype(DECODES)::value, halves = decltype(PIECES)::value;
         DecodesArg<decode> decodes;
         int bytes = lds;
         if constexpr (decode) {
@@ -508,19 +538,25 @@ static int launch_split_keys(const void* q, int q_stride, void* out, int out_str
         }
         constexpr int most = decode ? std::max(lds, TM_DECODE_BESIDE_LDS) : lds;
         if (most > 64 * 1024) {
-            static const hipError_t raised = hipFuncSetAttribute((const void*)attn_prefill_mfma_kernel<D, HPW, KS, CAP, with, decode>,
+            static const hipError_t raised = hipFuncSetAttribute((const void*)attn_prefill_mfma_kernel<D, HPW, KS, CAP, with, decode, halves>,
                                                                  hipFuncAttributeMaxDynamicSharedMemorySize, most);
             if (raised != hipSuccess) return TM_ERR_LAUNCH;
         }
-        attn_prefill_mfma_kernel<D, HPW, KS, CAP, with, decode><<<grid, 64 * KS, bytes, stream>>>(
+        attn_prefill_mfma_kernel<D, HPW, KS, CAP, with, decode, halves><<<grid, 64 * KS, bytes, stream>>>(
             (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
             table_width, tiles, n_tiles, order, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg, ahead_arg<with>(ahead), decodes);
         return TM_OK;
     };
-    if constexpr (D <= 64) {
-        if (beside) return ahead.n ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
+    auto with_values = [&](auto PIECES) {
+        if constexpr (D <= 64) {
+            if (beside) return ahead.n ? go(std::true_type{}, std::true_type{}, PIECES) : go(std::false_type{}, std::true_type{}, PIECES);
+        }
+        return ahead.n ? go(std::true_type{}, std::false_type{}, PIECES) : go(std::false_type{}, std::false_type{}, PIECES);
+    };
+    if constexpr (D <= 64 ? HPW > 2 : HPW > 1) {
+        if (page_shift == 4) return with_values(std::true_type{});
     }
-    return ahead.n ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
+    return with_values(std::false_type{});
 }
 
 // softcap > 0: a score s (scaled) becomes softcap * tanh(s / softcap) before the softmax; sink (float32 [H]) or null: one more term
