@@ -1,0 +1,30 @@
+"""How launches hand out their work, as the library says on the host."""
+import ctypes
+
+import pytest
+
+from tokenmill_amd.hip.library import library
+
+THREADS = 2 ** 32                       # a dimension of a launch has fewer
+
+
+# (query heads, kv heads, head size, wavefronts of a block)
+@pytest.mark.parametrize("H,KVH,D,waves", [(2, 1, 128, 2), (28, 4, 128, 4), (40, 8, 128, 4), (16, 1, 96, 8), (48, 4, 128, 8), (12, 2, 64, 4)])
+def test_a_dealt_launch_fits_the_grid(H, KVH, D, waves):
+    """Pieces dealt out stand in the grid's x; tables beyond what that holds are taken by tiles and kv heads, as they were before pieces were dealt."""
+    lib, most = library(), (THREADS // (64 * waves) - 1) // KVH
+    deals = lambda n: lib.tm_attn_prefill_shared_deals(*map(ctypes.c_int, (H, KVH, D, n)))
+    assert deals(256 // KVH) == 0 and deals(256 // KVH + 1) == 1
+    assert deals(most) == 1 and deals(most + 1) == 0 and deals(2 ** 31 - 1) == 0
+
+
+@pytest.mark.parametrize("H,KVH,D,heads,waves", [(14, 2, 64, 4, 8), (16, 16, 64, 1, 8), (32, 8, 128, 2, 4), (12, 2, 96, 2, 4), (640, 320, 64, 1, 8)])
+def test_an_order_of_pieces_fits_the_grid(H, KVH, D, heads, waves):
+    lib, columns = library(), KVH * -(-(H // KVH) // heads)
+    order = lambda n: lib.tm_attn_prefill_order(*map(ctypes.c_int, (H, KVH, D, heads, n)))
+    for n in [*range(1, 3000, 7), *(THREADS // (64 * waves) // columns + d for d in range(-400, 400)), 2 ** 31 - 1]:
+        if order(n) == 2:
+            assert n * columns * 64 * waves < THREADS
+        elif n * columns <= 256:
+            assert order(n) == 0
+    assert any(order(n) == 2 for n in range(1, 3000))

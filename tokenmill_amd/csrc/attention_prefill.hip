@@ -23,7 +23,6 @@
 #include "attention_decode_keys.h"
 
 #include <algorithm>
-#include <limits.h>
 
 // A block of 32 keys as a wavefront holds it between asking for it and using it. Row rho of operand tile t is key 16 t + rho: the lane which holds
 // rows 4 g .. 4 g + 3 of both tiles of the scores has the keys 4 g .. + 3 of either, and wants the same of a row of V^T.
@@ -504,10 +503,17 @@ template <int D> struct PrefillShape { static constexpr int HPW = D <= 64 ? 4 : 
 // (0.59) 33.8 / 26.3, 800 (0.78) 38.3 / 36.2, 900 (0.91) 41.5 / 41.6; 8 over 8 of 64, 1,500 (0.73) 19.0 / 15.7; 12 over 2 of 96, 1,500 (0.55) 41.6 / 30.4.
 // From 218 pairs (0.85) on pairs are better than tiles by heads too (1,900 tokens of the first 26.7 / 23.9), with fewer they are not (1,100
 // tokens 14.6 / 18.8). Head size 32, where a CU holds two blocks, stays with tiles by heads and pairs from 256 on (2,500 tokens of 12
-// heads over 2 26.4 / 28.5 dealt), and up to 256 pieces there is nothing to choose.
-static int prefill_order(int D, long long pieces, long long folded) {
-    if (D < 64 || pieces <= 256 || pieces > INT_MAX) return folded >= 256 ? PF_PAIRS : PF_PLAIN;
+// heads over 2 26.4 / 28.5 dealt), and up to 256 pieces there is nothing to choose. Pieces that do not fit the grid's x are not dealt.
+static int prefill_order(int D, int threads, long long pieces, long long folded) {
+    if (D < 64 || pieces <= 256 || !fits_a_dimension(pieces, threads)) return folded >= 256 ? PF_PAIRS : PF_PLAIN;
     return 100 * folded < 85 * 256 * ((folded + 255) / 256) ? PF_DEALT : PF_PAIRS;
+}
+
+// ... of a launch (for tests), with `heads` query heads of a kv head a wavefront
+extern "C" int tm_attn_prefill_order(int H, int KVH, int D, int heads, int n_tiles) {
+    if (H <= 0 || KVH <= 0 || H % KVH || heads <= 0 || n_tiles <= 0) return -1;
+    const long long columns = (long long)KVH * ((H / KVH + heads - 1) / heads);
+    return prefill_order(D, 64 * (D <= 64 ? PrefillShape<64>::KS : PrefillShape<128>::KS), n_tiles * columns, (n_tiles / 2 + n_tiles % 2) * columns);
 }
 
 template <int D, int HPW, bool CAP>
@@ -517,9 +523,9 @@ static int launch_split_keys(const void* q, int q_stride, void* out, int out_str
                               const bf16_t* cgate, int ldcg, TmAhead& ahead, const TmDecodes* beside, hipStream_t stream) {
     constexpr int KS = PrefillShape<D>::KS;
     const int splits = (H / KVH + HPW - 1) / HPW;
-    const long long pieces = (long long)n_tiles * KVH * splits, folded = (long long)((n_tiles + 1) / 2) * KVH * splits;
-    const int order = prefill_order(D, pieces, folded);
-    dim3 grid = order == PF_DEALT ? dim3((unsigned)pieces) : dim3(order == PF_PAIRS ? (n_tiles + 1) / 2 : n_tiles, KVH * splits);
+    const long long pieces = (long long)n_tiles * KVH * splits, folded = (long long)(n_tiles / 2 + n_tiles % 2) * KVH * splits;
+    const int order = prefill_order(D, 64 * KS, pieces, folded);
+    dim3 grid = order == PF_DEALT ? dim3((unsigned)pieces) : dim3(order == PF_PAIRS ? n_tiles / 2 + n_tiles % 2 : n_tiles, KVH * splits);
     constexpr int lds = KS * wave_floats<D, HPW>() * (int)sizeof(float);          // at most 139,264 bytes
     const long long layer = (long long)grid.x * grid.y;
     const int pairs = beside ? beside->n * KVH : 0, front = beside ? (int)((pairs + layer - 1) / layer) : 0;

@@ -8,6 +8,9 @@
 
 typedef FFrag PFrag;
 
+// A dimension of a launch has fewer than 2^32 threads: do so many blocks fit one?
+inline bool fits_a_dimension(long long blocks, int threads) { return blocks < (1LL << 32) / threads; }
+
 // two floats -> packed bfloat16 (round to nearest even, one instruction on gfx950)
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
     const bf16x2_t v = __builtin_convertvector(f32x2_t{a, b}, bf16x2_t);

@@ -20,7 +20,6 @@
 #include "common.h"
 #include "api.h"
 #include "attention_prefill_common.h"
-#include <limits.h>
 
 #define PS_KEYS 64          // positions per stage
 #ifndef TM_SHARED_HPW64
@@ -340,6 +339,11 @@ __global__ __launch_bounds__(64 * WAVES, SharedPlan<D>::WAVES_PER_SIMD) void att
     }
 }
 
+static bool shared_deals(int n_tiles, int KVH, int waves) {
+    const long long pieces = (long long)n_tiles * KVH;
+    return pieces > 256 && fits_a_dimension(pieces, 64 * waves);
+}
+
 template <int D, int WAVES>
 static int launch_shared(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                          const int* block_tables, int table_width, const int* tiles, int n_tiles, int H, int KVH,
@@ -353,9 +357,8 @@ static int launch_shared(const void* q, int q_stride, void* out, int out_stride,
             return TM_ERR_LAUNCH;
         raised = true;
     }
-    const long long blocks = (long long)n_tiles * KVH;
-    const int deal = blocks > 256 && blocks <= INT_MAX;
-    const dim3 grid = deal ? dim3((unsigned)blocks) : dim3(n_tiles, KVH);
+    const int deal = shared_deals(n_tiles, KVH, WAVES);
+    const dim3 grid = deal ? dim3((unsigned)n_tiles * KVH) : dim3(n_tiles, KVH);
     attn_prefill_shared_kernel<D, WAVES><<<grid, 64 * WAVES, lds, stream>>>(
         (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
         table_width, tiles, n_tiles, deal, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
@@ -369,6 +372,18 @@ extern "C" int tm_attn_prefill_shared_takes(int H, int KVH, int D) {
     const int G = H / KVH;
     if (!(D == 32 || D == 64 || D == 96 || D == 128) || KVH > 65535) return 0;
     return G <= 8 * (D <= 64 ? SharedPlan<64>::HPW : SharedPlan<128>::HPW);
+}
+
+// Wavefronts of a block. Three of work get a fourth, idle one: with two blocks a CU every working wavefront then
+// shares its SIMD with another, which is worth more than the SIMD the idle ones hold.
+static int shared_waves(int H, int KVH, int D) {
+    const int hpw = D <= 64 ? SharedPlan<64>::HPW : SharedPlan<128>::HPW, need = (H / KVH + hpw - 1) / hpw;
+    return need <= 2 ? 2 : need <= 4 ? 4 : 8;
+}
+
+// Are a launch's pieces dealt out over the chip? (for tests)
+extern "C" int tm_attn_prefill_shared_deals(int H, int KVH, int D, int n_tiles) {
+    return n_tiles > 0 && tm_attn_prefill_shared_takes(H, KVH, D) && shared_deals(n_tiles, KVH, shared_waves(H, KVH, D));
 }
 
 // softcap > 0: a score s (scaled) becomes softcap * tanh(s / softcap) before the softmax; sink (float32 [H]) or null: one more term
@@ -386,8 +401,7 @@ extern "C" int tm_attn_prefill_shared_cap(const void* q, int q_stride, void* out
         (q_stride % 8) || ((uintptr_t)q % 16) || (out_stride % 4) || ((uintptr_t)out % 8) || q_stride < H * D ||
         out_stride < H * D || !(scale > 0.f))
         return TM_ERR_ARG;
-    const int hpw = D <= 64 ? SharedPlan<64>::HPW : SharedPlan<128>::HPW;
-    const int G = H / KVH, need = (G + hpw - 1) / hpw;
+    const int waves = shared_waves(H, KVH, D);
     int page_shift = 0;
     while ((1 << page_shift) < page) ++page_shift;
     const float scale_log2 = scale * 1.4426950408889634f;
@@ -395,10 +409,8 @@ extern "C" int tm_attn_prefill_shared_cap(const void* q, int q_stride, void* out
                        page_shift, scale_log2, cap_in, cap_out, window, keep, sink, (const bf16_t*)cgate, ldcg, stream
 #define TM_SHARED_CASE(DD)                                                          \
     case DD:                                                                        \
-        if (need <= 2) return launch_shared<DD, 2>(TM_SHARED_ARGS);                 \
-        /* three wavefronts of work get a fourth, idle one: with two blocks a CU every working wavefront then */ \
-        /* shares its SIMD with another, which is worth more than the SIMD the idle ones hold */                  \
-        if (need <= 4) return launch_shared<DD, 4>(TM_SHARED_ARGS);                 \
+        if (waves == 2) return launch_shared<DD, 2>(TM_SHARED_ARGS);                \
+        if (waves == 4) return launch_shared<DD, 4>(TM_SHARED_ARGS);                \
         return launch_shared<DD, 8>(TM_SHARED_ARGS);
     switch (D) {
         TM_SHARED_CASE(32)
