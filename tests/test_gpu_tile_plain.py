@@ -53,7 +53,9 @@ def test_a_linear_on_both_sides_of_the_lines(N, K, tiled):
                 assert torch.equal(got, ops.tile_linear(x, lin.weight, torch.empty_like(got)))
 
 
-@pytest.mark.parametrize("N,K,tiled", [(32000, 1024, True), (16384, 256, True), (32004, 1024, False), (32000, 1056, False), (204808, 2048, False), (204808, 1984, True)])
+@pytest.mark.parametrize("N,K,tiled", [(32000, 1024, True), (16384, 256, True), (32004, 1024, False), (32000, 1056, False), (204808, 2048, False), (204808, 1984, True),
+                                         (264, 512, True), (4088, 576, False), (4096, 1024, True), (4096, 1088, False), (65528, 1088, False), (65536, 1088, True),
+                                         (65536, 6144, True), (65536, 6208, False), (541200, 1984, True), (541208, 1984, False)])
 def test_an_output_head_on_both_sides_of_the_lines(N, K, tiled):
     """Rows of a head that the tiled kernel takes from the library: their ends and one beyond, sizes it does not have; a row does not depend on the others."""
     from tokenmill_amd import profiling

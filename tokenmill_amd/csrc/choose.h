@@ -73,11 +73,21 @@ constexpr int TM_GEMV_F32_ROWS = 16;
 // and K from 3,584 to 5,120 up to 12% in heads of less than 65,536 (50,304 x 5,120: 95 to 107; 65,536 x 5,120 and 151,936 x 5,120 2 and 18% faster).
 inline bool tm_head_few(int M, int N, int K) { return M <= 8 || K <= 3072 || (N >= 65536 && K <= 5120); }
 
-// And the tiled kernel, of 17 to 64 rows? The library's time / the tiles', us, 17 / 33 / 64 rows: 151,936 x 896 65 / 53, 70 / 55, 74 / 64; 151,936 x 2,048
-// 147 / 121, 153 / 129, 158 / 137; 152,064 x 3,584 244 / 193, 201 / 201, 218 / 214; 128,256 x 4,096 198 / 185, 213 / 192, 220 / 197; 200,064 x 3,072 381 / 228,
-// 264 / 241, 285 / 258; 65,536 x 768 25.6 / 20.9, 26.7 / 22.3, 28.6 / 23.9; 50,304 x 1,024 and 32,000 x 2,048 and 4,096 level or to 3% less; 262,144 x 1,152
-// 127 / 116, 142 / 124, 147 / 139. 256,000 x 2,304 would be 1 to 4% slower, x 3,072 level. At 96 and 128 rows the tiles take 0.86 to 1.03 of the library's time.
-inline bool tm_head_tiled(int M, int N, int K) { return M > 16 && M <= 64 && (N <= 204800 || K < 2048); }
+// And the tiled kernel, of 17 to 64 rows? It adds all of K up in one chain and has a block a column of tiles, so where these are few and K is long the library, which
+// then cuts K, is faster and its error against 64 bits half as large: up to 4,096 columns by K of 768 and more. The tiles' time over the library's and
+// the largest of 17, 40 and 64 rows, over 15 widths from 512 to 200,064, cold matrices (up to 4,096 columns K of 1,024 is the library's at 17 rows only):
+//   K up to 512             0.46 to 0.98, 24,576 columns at 64 rows 1.05      512 to 4,096 columns, K 2,304 to 6,144    1.0 to 2.9
+//   K 768 to 1,024          from 4,096 columns on 0.33 to 0.98, 24,576 and 50,304 columns at 64 rows 1.02 to 1.04
+//   K 1,152 to 6,144        8,192 to 50,304 columns 0.62 to 1.4, level on the mean from 16,384 on; from 65,536 on 0.52 to 1.02, 0.88 on the mean
+// us, library / tiles, 17 / 33 / 64 rows: 151,936 x 896 65 / 53, 70 / 55, 74 / 64; 151,936 x 2,048 147 / 121, 153 / 129, 158 / 137; 152,064 x 3,584
+// 244 / 193, 201 / 201, 218 / 214; 152,064 x 5,120 331 / 274, 293 / 286, 310 / 309; 32,000 x 1,024 24 / 14, 25 / 15, 25 / 16; 200,064 x 3,072 381 / 228, 264 / 241,
+// 285 / 258; 262,144 x 1,152 127 / 116, 142 / 124, 147 / 139. 256,000 x 2,304 would be 1 to 4% slower. K of 8,192 is level. From 8,192 columns on the errors are the same
+// (128,256 columns alone, from K of 1,536 on, 5 to 9% larger). At 96 and 128 rows the tiles take 0.86 to 1.03 of the library's time. Matrices of 2 GB and more stay
+// the library's.
+inline bool tm_head_tiled(int M, int N, int K) {
+    if (M <= 16 || M > 64 || (long long)N * K >= 1LL << 30) return false;
+    return K <= 512 || (K <= 1024 && N >= 4096) || (K <= 6144 && N >= 65536 && (N <= 204800 || K < 2048));
+}
 
 // --- decode attention ---------------------------------------------------------------------------------
 constexpr int TM_DECODE_CHUNK = 256;        // keys per block of the split decode attention

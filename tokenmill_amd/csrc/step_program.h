@@ -20,7 +20,7 @@ struct TmLinear {               // y = x W^T + b, W [N, K]
     int bias_dtype;             // -1 without bias
     int N, K;
     int dtype;                  // type of w
-    int library_first;          // the owner asks for the library's product at any row count (an output head)
+    int library_first;          // an output head: the library's product, but for the rows and sizes of tm_head_few and tm_head_tiled
     int act;                    // 0: none; 1: y = relu(x W^T + b)^2 (in the product's epilogue where its kernel has one)
 };
 

@@ -27,7 +27,7 @@ class Linear(Part):
         assert len(self.biases) == len(self.names)
         self.has_bias = any(self.biases)
         self.bias_init_zero = False
-        self.library_first = library_first              # a wide matrix the library reads fastest at any row count
+        self.library_first = library_first              # an output head: the library's product but for few rows of some sizes, never a packed matrix
         self.wide_bias = wide_bias                      # the bias is kept in 32-bit (a product whose 32-bit result is wanted)
         if activation not in (None, "relu2"):
             raise ValueError(f"activation '{activation}' is not one a product applies itself (relu2)")
