@@ -61,13 +61,20 @@ def test_a_row_is_the_same_whatever_rows_are_beside_it(N, K):
 
     most = product(16)
     assert (most.double() - ref).abs().max() <= _bound(K)
-    for rows in (1, 4, 5, 8, 9):
+    for rows in (1, 2, 4, 5, 8, 9, 15):
         assert torch.equal(product(rows), most[:rows]), rows
 
 
 @pytest.mark.parametrize("N,K", [(3580, 16 * 97), (3584, 16 * 105), (4092, 16 * 112), (3568, 16 * 97), (24000, 384), (2100, 16 * 49)])
 def test_a_row_is_the_same_where_the_blocks_nearly_fill_the_chip(N, K):
     """From 224 blocks on two groups at a time for any rows, with a rest of every length; the shortest lines; a step of a pair that is not there."""
+    test_a_row_is_the_same_whatever_rows_are_beside_it(N, K)
+
+
+@pytest.mark.parametrize("N,K", [(3584, 16 * 98), (4092, 896), (4092, 1536), (4092, 1792), (6144, 768), (6144, 896), (6144, 960), (9728, 896), (32800, 896), (16384, 1040),
+                                 (1536, 160), (1536, 272), (1536, 528), (8200, 272)])
+def test_a_row_is_the_same_in_either_order_of_the_lanes(N, K):
+    """Sizes at which the number of rows says whether neighbouring lanes load side by side, and sizes whose rows are half a line more than whole ones."""
     test_a_row_is_the_same_whatever_rows_are_beside_it(N, K)
 
 

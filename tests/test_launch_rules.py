@@ -28,3 +28,13 @@ def test_an_order_of_pieces_fits_the_grid(H, KVH, D, heads, waves):
         elif n * columns <= 256:
             assert order(n) == 0
     assert any(order(n) == 2 for n in range(1, 3000))
+
+
+# (columns, K, rows at which neighbouring lanes load side by side) of the 32-bit product of few rows
+@pytest.mark.parametrize("N,K,rows", [(4096, 768, range(1, 17)), (4096, 896, range(5, 17)), (4096, 1536, range(5, 17)), (4096, 1568, range(2, 17)), (3552, 1536, range(1, 17)),
+                                      (6144, 704, range(1, 17)), (6144, 768, range(5, 17)), (6144, 896, range(5, 17)), (6144, 928, range(1, 17)), (32768, 896, []),
+                                      (32800, 896, [16]), (151936, 896, [16]), (151936, 928, range(1, 17)), (9728, 912, []), (1536, 144, range(1, 17)), (1536, 176, []),
+                                      (1536, 496, []), (1536, 528, range(1, 17)), (1536, 192, range(1, 17)), (8224, 176, range(1, 17))])
+def test_lanes_of_a_32_bit_product_load_side_by_side_where_that_pays(N, K, rows):
+    """Both sides of each line: rows that are no whole lines, two groups of steps a wavefront, one row of a block alone on its CU."""
+    assert [m for m in range(1, 17) if library().tm_gemv_f32_turns(*map(ctypes.c_int, (m, N, K)))] == list(rows)

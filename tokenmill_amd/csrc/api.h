@@ -73,6 +73,7 @@ int tm_gemv_bf16(const void* A, int lda, const void* W, float* C, int ldc, int M
 // The true 32-bit path's products of at most 16 rows on the 32-bit matrix unit (gemv_f32.hip): K a multiple of 16, N of 4, 16-byte
 // pieces (tm_gemv_f32_mfma_takes). A plain product; 32-bit partial sums [parts][M][N] (tm_gemv_f32_parts says how many);
 // silu(gate) * up; q|k|v with bias, rotation over the whole head (head sizes that are multiples of 32) and cache write.
+int tm_gemv_f32_turns(int M, int N, int K);    // whether the plain product's neighbouring lanes load what lies side by side (for tests)
 int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, const void* bias, int M, int N, int K);
 int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K, hipStream_t stream);
 int tm_gemv_f32_parts(int N, int K);

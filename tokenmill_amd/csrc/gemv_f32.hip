@@ -12,14 +12,14 @@
 // in four lanes at a time where these lie beside each other, and one at a time where they do not, which was most of what small products took
 // (64 clocks a load of 1 KB for 16). So four neighbouring lanes load 64 consecutive bytes, and the exchange that puts the pieces where the
 // instruction wants them (lane (4 q + p, g) holds row 4 q + g at piece p, and wants row 4 q + p at piece g) is four ds_bpermute a load, which
-// pass no memory. Matrices of 6.5 MB and more (GM_LINES) are loaded two steps at a time, 128 bytes of eight rows an instruction, whole lines that
-// pass the caches by (non-temporal), halves of lines would come from HBM twice as slowly; the step's parity lies in lane bit 4, where
-// one instruction a register changes it for the row's lowest bit. The activations go the same way; one row of them is asked for as the
+// pass no memory; where that costs more than it gains (gm_turns) the lanes load in the instruction's order. Matrices of 6.5 MB and more (GM_LINES) are
+// loaded two steps at a time, 128 bytes of eight rows an instruction, whole lines that pass the caches by (non-temporal), halves of lines would come from HBM
+// twice as slowly; the step's parity lies in lane bit 4, where one instruction a register changes it for the row's lowest bit (in the instruction's
+// order in bit 3: line_pair_half). The activations go the same way; one row of them is asked for as the
 // instruction wants it, all sixteen lanes of a piece at one place. us with the loads in the instruction's order / now, cold matrices:
 // q|k|v of the 0.5B shape at 1 / 8 / 16 rows 5.66 / 4.97, 6.40 / 5.65, 7.31 / 6.47, o 4.85 / 4.38, 5.58 / 5.07, 6.51 / 5.74, down 6.34 / 6.25, 7.25 / 6.56, 8.62 / 7.53, gate|up
-// 9.5 / 9.8, 10.4 / 10.2, 12.3 / 11.2, the head 96 / 91, 102 / 96, 117 / 107 (5.1 TB/s); 3,584 -> 2 x 18,944 93.8 / 92.3, 109 / 97, 137 / 111, back 48.7 / 49.7, 60 / 57,
-// 76.6 / 64.5; 2,048 -> 2,048 7.60 / 7.15, 8.49 / 7.95, 9.87 / 8.62; 2,000 x 128 3.44 / 3.06, 3.73 / 3.15, 4.05 / 3.15. Slower: up to four rows of 384 -> 32,000 (12.7 /
-// 13.3), K of 336 and 400 that leave wavefronts part of a group (3.4 / 3.5). The same bits.
+// at 8 / 16 10.4 / 10.3, 12.3 / 11.2; 3,584 -> 2 x 18,944 at 8 / 16 106 / 91, 127 / 104, back at 2 / 8 46.2 / 44.5, 53.9 / 46.2; 2,048 -> 1,536 at 1 / 8 / 16
+// 7.0 / 6.6, 8.2 / 7.7, 9.7 / 8.4. The same bits.
 // Before that, a wavefront had 256 k of four rows, a lane 4 k each, and summed over the lanes by shuffles, 6 x 32 of them a wavefront:
 // 19.0 us a product of the 0.5B shape on average, with SiLU*up and rotation in kernels behind it.
 #include "common.h"
@@ -52,7 +52,7 @@ struct GemvArgs {
 // at once: with one, a wavefront of the 0.5B shape waited for memory two times in a launch of 6 to 7 us (o 6.2 to 5.8, q|k|v 7.2 to 6.8).
 // LINES: two steps as a pair of lines, else a load a step. ROWS: rows of activations that there are places for, 1, 8 (of a pair of lines: one
 // load) or 16.
-template <int EPI, int RT, int WAVES, int GROUP, int AHEAD, bool LINES, int ROWS>
+template <int EPI, int RT, int WAVES, int GROUP, int AHEAD, bool LINES, int ROWS, bool TURN>
 __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArgs a) {
     static_assert(EPI == GM_PLAIN || RT == 1, "");
     __shared__ __align__(16) f32x4_t red[WAVES][RT][TM_WAVE];
@@ -85,15 +85,15 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
     static_assert(LINES || ROWS != 8, "");
     constexpr int HALVES = LINES ? 2 : 1;
     constexpr bool WHOLE = GROUP == 4 && (LINES || AHEAD == 1); // a full group's operands are all turned before its first product: 4,096 -> 4,096 at 8 rows 16.1 to 15.4
-    const int q = r / 4, piece = r % 4, parity = LINES ? g % 2 : 0;
+    const int q = r / 4, piece = TURN ? r % 4 : g, parity = !LINES ? 0 : TURN ? g % 2 : r / 8;
     // where a lane gets row r at piece g from, in bytes of lanes (eight rows of a pair of lines: the other step 16 lanes on)
-    const int turn = 4 * (LINES ? 32 * (r / 2 % 2) + 16 * (r % 2) + 4 * q + g : 16 * piece + 4 * q + g);
+    const int turn = 4 * (16 * (r % 4) + 4 * q + g);
     const int turn_x = LINES && ROWS == 8 ? 4 * (32 * (r % 2) + 4 * (r % 8 / 2) + g) : turn;
     const float* pa[HALVES];
     const float* pw[RT][HALVES];
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) {
-        const int row = LINES ? 4 * q + 2 * (g / 2) + h : 4 * q + g, of = LINES && ROWS == 8 ? 2 * q + g / 2 : row;
+        const int row = !TURN ? (LINES ? r % 8 + 8 * h : r) : LINES ? 4 * q + 2 * (g / 2) + h : 4 * q + g, of = TURN && LINES && ROWS == 8 ? 2 * q + g / 2 : row;
         pa[h] = ROWS == 1 ? a.A + 4 * g : a.A + (size_t)(of < a.M ? of : a.M - 1) * a.lda + 4 * piece;
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
@@ -161,14 +161,15 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_mfma_f32_kernel(const GemvArg
         auto operands = [&](int i, f32x4_t& xf, f32x4_t (&wf)[RT]) {
             if constexpr (LINES) {
                 if constexpr (ROWS == 1) xf = i % 2 ? line_pair_turned(x[i / 2][0]) : x[i / 2][0];
-                else if constexpr (ROWS == 8) xf = turned(turn_x + 64 * (i % 2), x[i / 2][0]);
-                else xf = turned(turn, pair_half(i % 2, x[i / 2][0], x[i / 2][ROWS == 16 ? 1 : 0]));
+                else if constexpr (ROWS == 8) xf = TURN ? turned(turn_x + 64 * (i % 2), x[i / 2][0]) : i % 2 ? line_pair_turned(x[i / 2][0]) : x[i / 2][0];
+                else xf = TURN ? turned(turn, pair_half(i % 2, x[i / 2][0], x[i / 2][1])) : line_pair_half(i % 2, x[i / 2][0], x[i / 2][1]);
 #pragma unroll
-                for (int t = 0; t < RT; ++t) wf[t] = turned(turn, pair_half(i % 2, w[t][i / 2][0], w[t][i / 2][1]));
+                for (int t = 0; t < RT; ++t)
+                    wf[t] = TURN ? turned(turn, pair_half(i % 2, w[t][i / 2][0], w[t][i / 2][1])) : line_pair_half(i % 2, w[t][i / 2][0], w[t][i / 2][1]);
             } else {
-                xf = ROWS == 1 ? x[i][0] : turned(turn, x[i][0]);
+                xf = ROWS == 1 || !TURN ? x[i][0] : turned(turn, x[i][0]);
 #pragma unroll
-                for (int t = 0; t < RT; ++t) wf[t] = turned(turn, w[t][i][0]);
+                for (int t = 0; t < RT; ++t) wf[t] = TURN ? turned(turn, w[t][i][0]) : w[t][i][0];
             }
         };
 #pragma unroll
@@ -301,53 +302,86 @@ extern "C" int tm_gemv_f32_mfma_takes(const void* A, int lda, const void* W, con
 constexpr size_t GM_LINES = 6656 * 1024;
 constexpr int GM_LINES_K = 384;
 
-template <int EPI, int RT, bool LINES, int ROWS>
+template <int EPI, int RT, bool LINES, int ROWS, bool TURN>
 static void gm_launch_rows(const GemvArgs& a, int units, int split, hipStream_t stream) {
     const int steps = (a.K / 16 + split - 1) / split, per = (steps + 7) / 8;
-    const bool long_runs = LINES && per > 12 && (a.M <= 4 || units * split >= 224);
+    const bool long_runs = LINES && per > 12 && (a.M <= 4 || (TURN && units * split >= 224));
     const dim3 grid(units, split);
     if (units * split > 256) {
         if constexpr (LINES) {
             if (steps > 4 * 7) {
-                gemv_mfma_f32_kernel<EPI, RT, 4, 7, 2, LINES, ROWS><<<grid, 256, 0, stream>>>(a);
+                gemv_mfma_f32_kernel<EPI, RT, 4, 7, 2, LINES, ROWS, TURN><<<grid, 256, 0, stream>>>(a);
                 return;
             }
         }
-        gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1, LINES, ROWS><<<grid, 256, 0, stream>>>(a);
+        gemv_mfma_f32_kernel<EPI, RT, 4, 7, 1, LINES, ROWS, TURN><<<grid, 256, 0, stream>>>(a);
         return;
     }
     if constexpr (LINES || RT == 1) {                           // (two tiles without lines: K of less than 384)
         if (per > 4 && (per <= 8 || long_runs)) {
-            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2, LINES, ROWS><<<grid, 512, 0, stream>>>(a);
+            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 2, LINES, ROWS, TURN><<<grid, 512, 0, stream>>>(a);
             return;
         }
         if (per > 8 && per <= 12) {
-            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3, LINES, ROWS><<<grid, 512, 0, stream>>>(a);
+            gemv_mfma_f32_kernel<EPI, RT, 8, 4, 3, LINES, ROWS, TURN><<<grid, 512, 0, stream>>>(a);
             return;
         }
     }
-    gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1, LINES, ROWS><<<grid, 512, 0, stream>>>(a);
+    gemv_mfma_f32_kernel<EPI, RT, 8, 4, 1, LINES, ROWS, TURN><<<grid, 512, 0, stream>>>(a);
 }
 
-template <int EPI, int RT, bool LINES>
+template <int EPI, int RT, bool LINES, bool TURN>
 static void gm_launch_lines(const GemvArgs& a, int units, int split, hipStream_t stream) {
     if (a.M == 1) {
-        gm_launch_rows<EPI, RT, LINES, 1>(a, units, split, stream);
+        gm_launch_rows<EPI, RT, LINES, 1, TURN>(a, units, split, stream);
         return;
     }
     if constexpr (LINES) {
         if (a.M <= 8) {
-            gm_launch_rows<EPI, RT, LINES, 8>(a, units, split, stream);
+            gm_launch_rows<EPI, RT, LINES, 8, TURN>(a, units, split, stream);
             return;
         }
     }
-    gm_launch_rows<EPI, RT, LINES, 16>(a, units, split, stream);
+    gm_launch_rows<EPI, RT, LINES, 16, TURN>(a, units, split, stream);
+}
+
+// Four neighbouring lanes side by side (TURN), or the instruction's order? Lines: matrices loaded as pairs of lines; per: steps a wavefront has.
+// The exchange behind the loads costs a wavefront some hundreds of cycles a group, which it has to gain at the loads. It does not
+//  - where rows are no whole lines (K % 32 = 16), so that the four lanes' 64 bytes lie in two: pairs of lines at 2 and 8 rows, K 720, 1,296 and 1,552, 3,584 to
+//    32,000 columns, 1.03 to 1.08 of the time of the other order (M 16, 1.02 to 1.1), a load a step with K of 176 to 464 1.01 to 1.08, below and above 0.85 to 0.99;
+//  - where more blocks than CUs have wavefronts of two groups of seven at once (K 768 to 896): of the 0.5B shape's head 1.04, 1.05, 1.05, 1.02 and 1.05 at 1 / 2 / 4 / 8 / 9
+//    rows (0.99 at 16), 896 -> 16,384 1.07 to 1.11 (1.04), 896 -> 6,144 1.04, 1.06, 1.03, 0.97, 1.01, gate|up 1.02, 1.05, 1.04, 0.99 (12 rows: 0.94); K 640 0.94 to 1.03, K 960 0.8 to 0.92;
+//  - at one row where a block is alone on its CU and not short (896 -> 4,096 1.03, 1,536 -> 3,584 1.07, 8,960 -> 4,096 1.05; K 512 0.96), and up to four if a
+//    wavefront's groups are all asked for at once (1,536 -> 4,096 at 2 / 4 / 8 rows 1.06 / 1.03 / 0.99; 2,048 -> 4,096 0.97 / 0.96 / 0.92).
+// Elsewhere, over 1,000 sizes, it is 0.92 on the mean, 0.58 to 1.04.
+static bool gm_turns(int RT, bool lines, int K, int M, int blocks, int per) {
+    if (K % 32) return !lines && (RT == 2 || K < 160 || K >= 512);
+    if (!lines) return true;
+    if (blocks > 256) return per < 12 || per > 14 || (RT == 2 ? M == 16 && blocks > 1024 : M > 4);
+    return blocks < 224 || per < 7 || (M > 1 && (M > 4 || per > 12));
+}
+
+static bool gm_lines(int N, int K) { return (size_t)N * K * 4 >= GM_LINES && K >= GM_LINES_K; }
+static bool gm_launch_turns(int RT, int M, int N, int K, int units, int split) {
+    const int steps = (K / 16 + split - 1) / split, waves = units * split > 256 ? 4 : 8;
+    return gm_turns(RT, gm_lines(N, K), K, M, units * split, (steps + waves - 1) / waves);
 }
 
 template <int EPI, int RT>
 static void gm_launch(const GemvArgs& a, int units, int split, hipStream_t stream) {
-    if ((size_t)a.N * a.K * 4 < GM_LINES || a.K < GM_LINES_K) gm_launch_lines<EPI, RT, false>(a, units, split, stream);
-    else gm_launch_lines<EPI, RT, true>(a, units, split, stream);
+    const bool lines = gm_lines(a.N, a.K), turn = gm_launch_turns(RT, a.M, a.N, a.K, units, split);
+    if (lines && turn) gm_launch_lines<EPI, RT, true, true>(a, units, split, stream);
+    else if (lines) gm_launch_lines<EPI, RT, true, false>(a, units, split, stream);
+    else if (RT == 2 || turn) gm_launch_lines<EPI, RT, false, true>(a, units, split, stream);
+    else if constexpr (RT == 1) gm_launch_lines<EPI, RT, false, false>(a, units, split, stream);
+}
+
+// two tiles a block read the activations once for both, where that still gives every CU a block
+static bool gm_two_tiles(int N) { return (N + 31) / 32 >= 256; }
+
+// Do neighbouring lanes of the plain product load what lies side by side? (for tests)
+extern "C" int tm_gemv_f32_turns(int M, int N, int K) {
+    return gm_two_tiles(N) ? gm_launch_turns(2, M, N, K, (N + 31) / 32, 1) : gm_launch_turns(1, M, N, K, (N + 15) / 16, 1);
 }
 
 extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,
@@ -355,10 +389,8 @@ extern "C" int tm_gemv_f32_mfma(const float* A, int lda, const float* W, const f
     if (!tm_gemv_f32_mfma_takes(A, lda, W, bias, M, N, K) || !gm_aligned16(C) || ldc < N || ldc % 4) return TM_ERR_ARG;
     GemvArgs a{};
     a.A = A; a.W = W; a.bias = bias; a.C = C; a.lda = lda; a.ldc = ldc; a.M = M; a.N = N; a.K = K;
-    // two tiles a block read the activations once for both, where that still gives every CU a block
-    const int two = (N + 31) / 32, one = (N + 15) / 16;
-    if (two >= 256) gm_launch<GM_PLAIN, 2>(a, two, 1, stream);
-    else gm_launch<GM_PLAIN, 1>(a, one, 1, stream);
+    if (gm_two_tiles(N)) gm_launch<GM_PLAIN, 2>(a, (N + 31) / 32, 1, stream);
+    else gm_launch<GM_PLAIN, 1>(a, (N + 15) / 16, 1, stream);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
