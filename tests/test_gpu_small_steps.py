@@ -71,6 +71,26 @@ def test_every_number_of_few_tokens(ops, N, K):
         assert torch.equal(out, outs[15][:M]), M
 
 
+@pytest.mark.parametrize("N", [388, 1540, 3076, 4100])
+@pytest.mark.parametrize("K", [456, 512, 904, 2040, 2056, 2824, 3592, 4616, 6152, 12296])
+def test_rows_of_whole_pieces_have_the_bits_of_others(ops, N, K):
+    """Activations change lanes where their rows lie in whole pieces of 64 bytes, at every depth of a round; the others, and those that begin
+    beside a piece, do not."""
+    torch.manual_seed(K + N)
+    w = (torch.randn(N, K, device=DEV) * K ** -0.5).to(BF)
+    packed = ops.pack_weight(w, ops.skinny_strip_rows(N, K))
+    room = torch.randn(17, -(-K // 32) * 32 + 32, device=DEV).to(BF)
+    room[:, K:] = float("nan")                                       # what lies behind a row is nobody's
+    rows, beside = room[:16, :K], torch.empty_like(room)[:16, 8:8 + K]
+    beside.copy_(rows)
+    assert rows.stride(0) % 32 == 0 and rows.data_ptr() % 64 == 0 and beside.data_ptr() % 64
+    for M in range(1, 17):
+        outs = [ops.gemm_skinny(x[:M], packed, None, torch.full((M, N), float("nan"), device=DEV)) for x in (rows, beside, rows[:M].contiguous())]
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2]), M
+    # products of two bfloat16 are exact in 32 bits: what is left is one rounding of at most the sum of the magnitudes an addition
+    assert ((outs[0].double() - rows.double() @ w.double().T).abs() <= K * 2.0 ** -24 * (rows.double().abs() @ w.double().abs().T)).all()
+
+
 @pytest.mark.parametrize("M", [3, 7, 12])
 @pytest.mark.parametrize("N", [896, 1536])
 def test_what_is_no_number_stays_with_its_token_and_its_row(ops, M, N):

@@ -38,3 +38,13 @@ def test_an_order_of_pieces_fits_the_grid(H, KVH, D, heads, waves):
 def test_lanes_of_a_32_bit_product_load_side_by_side_where_that_pays(N, K, rows):
     """Both sides of each line: rows that are no whole lines, two groups of steps a wavefront, one row of a block alone on its CU."""
     assert [m for m in range(1, 17) if library().tm_gemv_f32_turns(*map(ctypes.c_int, (m, N, K)))] == list(rows)
+
+
+# (columns, K, row stride, tokens at which the activations' pieces change lanes) of the packed product of few tokens: strips of 4, 8 and 16 rows
+@pytest.mark.parametrize("N,K,lda,tokens", [(896, 4864, 4864, [3, 4, 6, 7, 8, *range(12, 17)]), (896, 4864, 4872, []), (896, 4856, 4864, [3, 4, 6, 7, 8, *range(12, 17)]),
+                                            (896, 4856, 4856, []), (896, 2016, 2016, []), (1536, 2048, 2048, range(4, 17)), (1536, 2016, 2016, []),
+                                            (3584, 2048, 2048, range(6, 17)), (3584, 2016, 2016, range(10, 17)), (3584, 512, 512, range(10, 17)), (3584, 480, 480, []),
+                                            (3584, 904, 904, []), (4096, 4096, 4096, range(10, 17))])
+def test_activations_change_lanes_where_that_pays(N, K, lda, tokens):
+    """Both sides of each line: a short K, places without a token, rows that are no whole pieces of 64 bytes."""
+    assert [m for m in range(1, 17) if library().tm_skinny_turns(*map(ctypes.c_int, (m, N, K, lda)))] == list(tokens)

@@ -154,6 +154,7 @@ int tm_gemm_skinny(const void* A, int lda, const void* W, const void* bias, int 
 // 16-byte loads of one k-step of one strip are then one run of R * 64 bytes. A stacked matrix whose
 // parts meet in an epilogue (gate and up) is packed part by part, each part's strips behind the other's.
 int tm_skinny_strip_rows(int N, int K);
+int tm_skinny_turns(int M, int N, int K, int lda);  // whether pieces of the activations change lanes behind their loads (for tests)
 int tm_fused_qkv_strip_rows(int H, int KVH, int D, int K);
 int tm_gemm_skinny_packed(const void* A, int lda, const void* W, int rows, const void* bias, int bias_dtype, void* C,
                           int ldc, int M, int N, int K, int out_dtype, int silu, float* accum, int ldacc,

@@ -215,12 +215,23 @@ static int few_depth(int per, int a, int b, int c, int d) {
     return a * rounds >= per ? a : b * rounds >= per ? b : c * rounds >= per ? c : d;
 }
 
-// Do the activations' pieces change lanes behind their loads? Where the loads are many (a long K; else strips of 16 rows) and the tokens fill their
-// places: with 9 of 16 and 5 of 8 tokens 4,864 -> 896 takes 6.0 for 5.7 and 4.4 for 4.3 us, with 4 of 16 4,096 -> 4,096 6.0 for 5.7 (18,944 -> 3,584 level
-// up to 5); over a short K and strips of 4 or 8 rows the exchange is longer than the wait (896 -> 896 8 tokens 3.0 / 3.4, 1,536 -> 1,536 3.2 / 3.3).
-static bool few_turns(int rows, int M, bool long_k) {
-    if (!long_k) return rows == 16 && M >= 10;
+// Do the activations' pieces change lanes behind their loads? Where the loads are many (a long K; else strips of 16 rows and K of 512 and more) and the
+// tokens fill their places: with 9 of 16 and 5 of 8 tokens 4,864 -> 896 takes 6.0 for 5.7 and 4.4 for 4.3 us, with 4 of 16 4,096 -> 4,096 6.0 for 5.7
+// (18,944 -> 3,584 level up to 5); over a short K and strips of 4 or 8 rows the exchange is longer than the wait (896 -> 896 8 tokens 3.0 / 3.4,
+// 1,536 -> 1,536 3.2 / 3.3), and over 256 -> 4,096 too (2.55 / 2.67 at 10 tokens). And where rows lie in whole pieces of 64 bytes: four lanes' loads that straddle two
+// lines are no fewer than before, and 2,056 -> 896 takes 3.9 for 4.4 us at 12 tokens, 1,032 -> 3,584 2.7 for 2.9. Where they do, over 70 matrices, the launch takes
+// 0.68 to 1.04 of the time of the other order, the matrix in the caches, and 0.86 to 1.07 cold (above 1.04 at 12 to 14 tokens of strips of 4 rows).
+static bool few_turns(int rows, int M, int K, bool long_k, const void* A, int lda) {
+    if (lda % 32 || (uintptr_t)A % 64) return false;
+    if (!long_k) return rows == 16 && M >= 10 && K >= 512;
     return rows == 4 ? 4 * M >= 3 * (M <= 4 ? 4 : M <= 8 ? 8 : 16) : M >= (rows == 8 ? 4 : 6);
+}
+static bool few_long_k(int rows, int N, int K) { return K >= 2048 && !(rows == 16 && (N + 15) / 16 >= 256); }
+
+// ... of a packed matrix and activations at a whole line (for tests)
+extern "C" int tm_skinny_turns(int M, int N, int K, int lda) {
+    const int rows = tm_skinny_strip_rows(N, K);
+    return few_turns(rows, M, K, few_long_k(rows, N, K), nullptr, lda);
 }
 
 // Ranges of K: 4, or 16 for a long K over few strips. `rows`: of a strip (16, 8 or 4).
@@ -236,9 +247,9 @@ static int launch_few(const void* A, int lda, const void* W, int rows, const voi
         return TM_OK;
     }
     const int strips = (N + rows - 1) / rows;
-    const bool long_k = K >= 2048 && !(rows == 16 && strips >= 256);
+    const bool long_k = few_long_k(rows, N, K);
     const int ksteps = (K + 31) / 32, per = long_k ? (ksteps + 15) / 16 : (ksteps + 3) / 4;
-    const bool turn = PACKED && few_turns(rows, M, long_k);
+    const bool turn = PACKED && few_turns(rows, M, K, long_k, A, lda);
 #define TM_FEW(ROWS_, TOKS_, VW_, CH_, TURN_)                                                                         \
     gemm_few_kernel<ROWS_, TOKS_, VW_, CH_, TC, PACKED, TURN_><<<strips, 4 * VW_ * ROWS_, 0, stream>>>(               \
         (const bf16_t*)A, lda, (const bf16_t*)W, bias, flags, (TC*)C, ldc, M, N, K, accum, ldacc)
