@@ -54,6 +54,22 @@ def test_one_block_has_the_bits_of_the_split_contexts(H, KVH, D, page, lens, win
     assert torch.equal(out, got[sub])
 
 
+@pytest.mark.parametrize("D", [64, 96, 128])
+@pytest.mark.parametrize("keys", [256, 257])
+def test_a_request_has_its_bits_in_either_order_of_the_key_loads(D, keys):
+    """Up to 64 keys a wavefront and up to 64 channels, or beside 128 pairs and more, keys are loaded in the order of the product, else four lanes side by side."""
+    from tokenmill_amd.hip import ops
+    lens = [keys, 1, 64, 65, 200, keys - 1] + [100] * 58
+    q, k, v, tables, ctx, _ = _case(6, 2, D, 16, lens, 11)
+
+    def run(n):
+        return ops.attn_decode_mfma(q[:n], torch.full_like(q[:n], 3.0), k, v, tables[:n], ctx[:n], 6, 2, D, D ** -0.5, 0, keys, whole=True)
+
+    most = run(64)
+    for n in (1, 6, 63):
+        assert torch.equal(run(n), most[:n]), n
+
+
 def test_more_than_the_lds_holds_is_refused():
     from tokenmill_amd.hip import ops
     q, k, v, tables, ctx, _ = _case(16, 1, 128, 16, [1300], 3)

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_block_kernel(
     const int G = H / KVH;
     const int ctx = context_lens[s];
     if (ctx <= whole_chunks * AD_CHUNK)                              // block-uniform
-        return attend_whole<D, WAVES>(s_block, s, kvh, q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, whole_chunks,
+        return attend_whole<D, WAVES, false>(s_block, s, kvh, q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, whole_chunks,
                                       H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
     float(*s_m)[16] = (float(*)[16])s_block, (*s_l)[16] = s_m + WAVES;
     float(*s_o)[16][16 + 1] = (float(*)[16][16 + 1])(s_l + WAVES);   // one 16-wide d tile at a time
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(64 * AD_MERGE_WAVES) void attn_decode_merge_long_ke
 // registers up to head size 64, 8 beyond and where pairs are so many that CUs hold two blocks). The partials meet in two passes of four elements a
 // thread: with one element a thread in one pass head size 128 took 1.6 us longer, with four elements in one pass 16 wavefronts spilled.
 // The rule and what it measured stand in choose.h (tm_decode_whole).
-template <int D, int WAVES, bool AHEAD>
+template <int D, int WAVES, bool AHEAD, bool TURN>
 __global__ __launch_bounds__(64 * WAVES) void attn_decode_whole_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_whole_kernel(
                    cap_out, window, keep, sink, cgate, ldcg);
         if (blockIdx.z) return tm_bring_ahead(ahead, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), WAVES);
     }
-    attend_whole<D, WAVES>(s_whole, blockIdx.x, blockIdx.y, q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, chunks, H,
+    attend_whole<D, WAVES, TURN>(s_whole, blockIdx.x, blockIdx.y, q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, chunks, H,
                            KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
 }
 
@@ -412,15 +412,15 @@ static int ahead_layers(TmAhead& ahead, int pairs, int own) {
     return own + more;
 }
 
-template <int D, int WAVES, bool AHEAD>
+template <int D, int WAVES, bool AHEAD, bool TURN>
 static int launch_whole(const void* q, int q_stride, void* out, int out_stride, const void* k_pool, const void* v_pool,
                         const int* block_tables, int table_width, const int* context_lens, int chunks, int S, int H, int KVH,
                         int page_shift, float scale_log2, float cap_in, float cap_out, int window, int keep, const float* sink,
                         const bf16_t* cgate, int ldcg, TmAhead& ahead, hipStream_t stream) {
-    static const hipError_t allowed = hipFuncSetAttribute((const void*)attn_decode_whole_kernel<D, WAVES, AHEAD>,
+    static const hipError_t allowed = hipFuncSetAttribute((const void*)attn_decode_whole_kernel<D, WAVES, AHEAD, TURN>,
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)TM_DECODE_WHOLE_LDS);
     if (allowed != hipSuccess) return TM_ERR_LAUNCH;
-    attn_decode_whole_kernel<D, WAVES, AHEAD><<<dim3(S, KVH, ahead_layers(ahead, S * KVH, 1)), 64 * WAVES, tm_decode_whole_lds(chunks, H / KVH, D), stream>>>(
+    attn_decode_whole_kernel<D, WAVES, AHEAD, TURN><<<dim3(S, KVH, ahead_layers(ahead, S * KVH, 1)), 64 * WAVES, tm_decode_whole_lds(chunks, H / KVH, D), stream>>>(
         (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
         table_width, context_lens, chunks, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg, ahead);
     TM_CHECK_LAUNCH();
@@ -527,12 +527,17 @@ static int launch_whole_waves(const void* q, int q_stride, void* out, int out_st
     int page_shift = 0;
     while ((1 << page_shift) < page) ++page_shift;
     const float cap_in = softcap > 0.f ? scale / softcap : 0.f;
-#define TM_WHOLE(W)                                                                                                              \
-    (ahead.n ? launch_whole<D, W, true> : launch_whole<D, W, false>)(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, chunks, S, H, KVH, \
+#define TM_WHOLE(W, TURN)                                                                                                        \
+    (ahead.n ? launch_whole<D, W, true, TURN> : launch_whole<D, W, false, TURN>)(q, q_stride, out, out_stride, k_pool, v_pool, block_tables, table_width, context_lens, chunks, S, H, KVH, \
                        page_shift, scale * 1.4426950408889634f, cap_in, softcap * 1.4426950408889634f, window, keep, sink, cgate, ldcg, ahead, stream)
-    if (chunks == 1) return TM_WHOLE(4);
-    if constexpr (D > 64) return TM_WHOLE(8);               // (12 and 16 wavefronts do not have the registers)
-    else return chunks == 2 || S * KVH > 256 ? TM_WHOLE(8) : chunks == 3 ? TM_WHOLE(12) : TM_WHOLE(16);
+    if constexpr (D > 64) {
+        if (chunks > 1) return TM_WHOLE(8, true);           // (12 and 16 wavefronts do not have the registers)
+        return tm_decode_whole_turns(D, chunks, S * KVH) ? TM_WHOLE(4, true) : TM_WHOLE(4, false);
+    } else {
+        constexpr bool turn = tm_decode_whole_turns(D, 2, 1);
+        if (chunks == 1) return TM_WHOLE(4, false);
+        return chunks == 2 || S * KVH > 256 ? TM_WHOLE(8, turn) : chunks == 3 ? TM_WHOLE(12, turn) : TM_WHOLE(16, turn);
+    }
 #undef TM_WHOLE
 }
 

@@ -40,10 +40,15 @@ union Bf16x8Bits {
 //
 // Neighbouring lanes of the first product's operand are in different rows: 64 addresses for a CU's address unit, one a cycle, where four lanes
 // beside each other in a row are one. TURN: four lanes load 64 bytes of a row (lane (4 q + p, g) row 4 q + g, piece p) and the pieces change
-// lanes in front of the product by ds_bpermute, four a load. us without / with (seven heads a kv head): the kernel of a whole context, 1 request of 300
-// keys, head sizes 64 / 128, 5.63 / 5.26, 7.54 / 6.61, 2 of 500 6.07 / 5.54, 16 of 300 6.08 / 5.76, 32 of 600, 128, 13.4 / 12.9, 64 of 1,021 11.1 / 10.8; the
-// block kernel, 128 of 2,000 25.6 / 25.1, 96 of 1,500, 128, 55.5 / 53.8. The split kernel, whose wavefronts have 64 keys and no more, has the
-// exchange in its one chain: 8 of 2,048, 128, 12.7 / 13.1, 64 level. It goes without. The same bits.
+// lanes in front of the product by ds_bpermute, four a load, which a wavefront waits for. So it pays where a CU has many keys to load: in the kernel of a whole
+// context with more than one chunk and more than 32 channels a head, with one chunk of more than 64 channels and fewer than 128 pairs. us without / with: 1 request of
+// two heads, D 64 of 300 / 600 / 1,100 keys 5.6 / 5.2, 7.3 / 6.4, 10.3 / 8.5, D 128 of 200 / 600 6.6 / 5.9, 11.1 / 9.2, 32 requests, D 64 of 320 / 768 6.5 / 6.1, 8.9 / 8.2; 64,
+// of 600 9.0 / 8.7. Where it does not: D 64 of 64 / 128 / 200 keys, 1 request 4.4 / 4.6, 4.5 / 4.7, 4.9 / 4.9; D 32, of 128 / 512 keys 1 and 64 requests
+// 4.2 / 4.3, 5.0 / 4.9, 5.0 / 5.0, 6.0 / 6.0; D 128, 64 and 90 requests of 256 keys 8.4 / 8.6, 8.8 / 9.1. The block kernel takes its requests beyond the
+// whole kernel's order so (200 of 2,500 keys, D 64 56.2 / 53.4, D 96 and D 128 100 of 40 heads over 8 171 / 168, 217 / 204) and those of the whole kernel's order without (128 and 200 of 200
+// keys, D 128 9.4 / 9.9, 15.5 / 16.1). The split kernel, whose wavefronts have 64 keys and no more, has the exchange in its one chain: 8 of 2,048, D 128, 12.7 / 13.1, 64
+// level. It goes without. The same bits.
+constexpr bool tm_decode_whole_turns(int D, int chunks, int pairs) { return D > 32 && (chunks > 1 || (D > 64 && pairs < 128)); }
 __device__ __forceinline__ int tile_key(int t, int rho) { return 32 * (t / 2) + 8 * (rho / 4) + 4 * (t % 2) + rho % 4; }
 
 template <int D>
@@ -192,7 +197,7 @@ __device__ __forceinline__ void load_q_operand(Bf16x8Bits (&qreg)[D / 32], const
 }
 
 // All chunks of a (request, kv head) by one block of WAVES wavefronts (the whole kernel of attention_decode.hip); lds: tm_decode_whole_lds bytes, 16 byte aligned.
-template <int D, int WAVES>
+template <int D, int WAVES, bool TURN>
 __device__ __forceinline__ void attend_whole(float* lds, int s, int kvh, const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out,
                                              int out_stride, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
                                              const int* __restrict__ block_tables, int table_width, const int* __restrict__ context_lens, int chunks,
@@ -220,8 +225,8 @@ __device__ __forceinline__ void attend_whole(float* lds, int s, int kvh, const b
         if (wbase < ctx && (wbase + AD_WKEYS > lo || wbase < keep)) {       // else nothing of the run is visible
             f32x4_t o[NDT];
             Keys64<D> kv;
-            load_keys64<D, true>(kv, k_pool, v_pool, entry, wbase, ctx, keep, lo, kvh, KVH, page_shift, r, g);
-            attend_keys64<D, true>(kv, qreg, wbase, ctx, keep, lo, scale_log2, cap_in, cap_out, g, m, l, o);
+            load_keys64<D, TURN>(kv, k_pool, v_pool, entry, wbase, ctx, keep, lo, kvh, KVH, page_shift, r, g);
+            attend_keys64<D, TURN>(kv, qreg, wbase, ctx, keep, lo, scale_log2, cap_in, cap_out, g, m, l, o);
             if (r < G) {
 #pragma unroll
                 for (int dt = 0; dt < NDT; ++dt) *(f32x4_t*)(s_o + ((size_t)run * G + r) * ROW + 16 * dt + 4 * g) = o[dt];

@@ -322,7 +322,7 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_mfma_kernel(
         if (layer < decodes.layers) {
             const int pair = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * layer), of = pair / decodes.n;
             if (pair >= decodes.pairs) return;
-            return attend_whole<D, KS>(s_o, pair - of * decodes.n, of, decodes.q, q_stride, decodes.out, out_stride, k_pool, v_pool, decodes.tables,
+            return attend_whole<D, KS, (D > 32)>(s_o, pair - of * decodes.n, of, decodes.q, q_stride, decodes.out, out_stride, k_pool, v_pool, decodes.tables,
                                        table_width, decodes.context_lens, decodes.chunks, H, KVH, page_shift, scale_log2, cap_in, decodes.cap_out, window,
                                        keep, sink, decodes.cgate, ldcg);
         }
