@@ -48,3 +48,11 @@ def test_lanes_of_a_32_bit_product_load_side_by_side_where_that_pays(N, K, rows)
 def test_activations_change_lanes_where_that_pays(N, K, lda, tokens):
     """Both sides of each line: a short K, places without a token, rows that are no whole pieces of 64 bytes."""
     assert [m for m in range(1, 17) if library().tm_skinny_turns(*map(ctypes.c_int, (m, N, K, lda)))] == list(tokens)
+
+
+# (token tiles, wavefronts a unit, units a block), k-steps a wavefront at which a round has eight of them
+@pytest.mark.parametrize("shape,eight", [((1, 8, 1), [6, 7, 8, *range(13, 40)]), ((1, 4, 2), [6, 7, 8, *range(9, 40)]), ((1, 2, 8), range(6, 40)), ((2, 8, 1), []), ((3, 8, 1), []),
+                                         ((2, 4, 2), [5, 6, 7, 8, *range(13, 17), *range(21, 40)]), ((4, 2, 4), [5, 6, 7, 8, *range(13, 17), *range(21, 40)]), ((4, 2, 5), [])])
+def test_rounds_of_a_streamed_product_have_eight_steps_where_that_pays(shape, eight):
+    """Both sides of each line: a second round for a few steps, two tiles of tokens with eight wavefronts a unit, more wavefronts than have the registers."""
+    assert [per for per in range(1, 40) if library().tm_stream_round(*map(ctypes.c_int, (*shape, per))) == 8] == list(eight)

@@ -191,6 +191,7 @@ int tm_stream_linear(const void* X, int ldx, int M, int K, const void* W, int ro
 // The plain product with K split over tm_stream_linear_parts(N, K) groups of blocks (a number from the matrix's shape
 // alone; 1: not worth splitting): parts[p][M][N] (float32, M * N elements apart) receives the 32-bit partial sums,
 // the bias in part 0, for tm_add_rmsnorm_parts or tm_sum_parts to add up.
+int tm_stream_round(int NT, int KS, int US, int per);   // k-steps of a round: NT token tiles, KS wavefronts a unit, US units a block, per k-steps a wavefront (for tests)
 int tm_stream_linear_parts(int N, int K);
 int tm_stream_linear_split(const void* X, int ldx, int M, int K, const void* W, int rows, int N, const void* bias,
                            int bias_dtype, float* parts, hipStream_t stream);

@@ -35,7 +35,7 @@
 // the matrix is read once and never again: loads that do not displace the activations in the caches
 #define ST_WLOAD(p) __builtin_nontemporal_load((const u32x4_t*)(p))
 #define ST_WD 8             // k-steps of the matrix a wavefront has in registers or on their way: one round of eight or two of four
-#define ST_XPAD 16          // padding of an LDS row of activations, in elements: rows 288 bytes apart, which the operand loads (lane (r, g): 16 bytes of row r at piece g) read free of bank conflicts; with 8 (272 bytes) they take twice as long
+#define ST_XPAD 16          // padding of an LDS row of activations, in elements: rows 288 bytes apart, 544 with rounds of eight, which the operand loads (lane (r, g): 16 bytes of row r at piece g) read free of bank conflicts; with 8 (272 bytes) they take twice as long
 
 struct StreamArgs {
     FusedArgs f;            // activations X [M, K], the packed matrix, and what the q|k|v and SiLU epilogues need
@@ -449,7 +449,7 @@ static int launch_stream_rounds(const StreamArgs& a, int n_units, int kparts, in
     return TM_OK;
 }
 
-// Four k-steps a round or eight. Both add a wavefront's products in the order of K, so the results are the same bits;
+// Four k-steps a round or eight, for a wavefront with `per` of them. Both add a wavefront's products in the order of K, so the results are the same bits;
 // the matrix is eight k-steps ahead with either. Eight halve the rounds, and with them the two meetings of the block
 // and the turn of the activations through LDS that each costs while nothing new is asked of HBM, but the last round
 // turns a window that may be nearly empty, and the first products wait for twice the activations. Eight pay where a
@@ -458,15 +458,24 @@ static int launch_stream_rounds(const StreamArgs& a, int n_units, int kparts, in
 // rounds of four / eight (us): 8 rows, gate|up 7B 51.6 / 47.6, 4,096 -> 2 x 14,336 46.7 / 44.5, 2,048 -> 2 x 11,008
 // 23.4 / 18.1, 1,536 -> 2 x 8,960 18.4 / 13.3; q|k|v 7B 10.9 / 10.5; 7B down 26.9 / 25.4, 32B down 52.7 / 47.5; 64 rows,
 // 4,096 -> 2 x 14,336 51.9 / 49.2, 7B down 33.5 / 32.0. Where they lose: a wavefront with 4 or 5 k-steps at 8 rows
-// (q|k|v 0.5B 4.96 / 5.35, 0.5B down 6.94 / 7.12), with 9 to 12 at 32 rows (11,008 -> 2,048 12.9 / 13.1; 17 to 20 at
-// 8 x 1: q|k|v 32B 20.2 / 20.6), ten wavefronts at 64 rows (gate|up 7B 54.0 / 54.6; sixteen: 104 / 107), and where two
+// (q|k|v 0.5B 4.96 / 5.35, 0.5B down 6.94 / 7.12); with 9 to 12 where eight wavefronts share a unit, the second round's window of all of K for one to four steps
+// (8 / 16 rows, 2,304 -> 4,608 as gate|up 8.3 / 8.7, 8.4 / 9.0, plain -> 4,096 8.5 / 8.7, 8.6 / 9.1, 3,072 -> 2,048 9.0 / 9.0, 9.2 / 9.6; 2,048 and 3,584, with 8 and 14, 0.97 to 1.0 and
+// 0.95 to 0.98); with 9 to 12 at 32 rows (11,008 -> 2,048 12.9 / 13.1); two tiles of tokens and eight wavefronts a unit (17 / 32 rows, 2,048 -> 2,048 8.8 / 8.8,
+// 9.0 / 9.3, 8,960 -> 2,048 25.0 / 27.0, 27.7 / 28.5, as gate|up 24.8 / 25.5, 27.2 / 26.4); ten wavefronts at 64 rows (gate|up 7B 54.0 / 54.6; sixteen: 104 / 107); and where two
 // blocks with two tiles share a CU (gate|up 0.5B 64 rows 11.5 / 13.9).
+static constexpr bool stream_has_eight(int NT, int KS, int US) { return NT == 1 || (KS < 8 && KS * US <= 8 && KS * NT <= 16); }
+static bool stream_eight_pay(int NT, int KS, int per) {
+    return NT == 1 ? per >= (KS == 8 ? 13 : 9) || (per >= 6 && per <= 8) : per > 24 || (per + 7) % 8 >= 4;
+}
+
+// k-steps of a round (for tests)
+extern "C" int tm_stream_round(int NT, int KS, int US, int per) { return stream_has_eight(NT, KS, US) && stream_eight_pay(NT, KS, per) ? 8 : 4; }
+
 template <int EPI, int NT, int KS, int US>
 static int launch_stream_config(const StreamArgs& a, int n_units, int kparts, int row_parts, hipStream_t stream) {
-    if constexpr (NT == 1 || (KS * US <= 8 && KS * NT <= 16)) {
+    if constexpr (stream_has_eight(NT, KS, US)) {
         const int ksteps = (a.f.K + 31) / 32, per = ((ksteps + kparts - 1) / kparts + KS - 1) / KS;
-        const bool pays = NT == 1 ? per > 8 || (per + 7) % 8 >= 5 : per > 24 || (per + 7) % 8 >= 4;
-        if (row_parts == 1 && pays) return launch_stream_rounds<EPI, NT, KS, US, 8>(a, n_units, kparts, row_parts, stream);
+        if (row_parts == 1 && stream_eight_pay(NT, KS, per)) return launch_stream_rounds<EPI, NT, KS, US, 8>(a, n_units, kparts, row_parts, stream);
     }
     return launch_stream_rounds<EPI, NT, KS, US, 4>(a, n_units, kparts, row_parts, stream);
 }
