@@ -56,3 +56,12 @@ def test_activations_change_lanes_where_that_pays(N, K, lda, tokens):
 def test_rounds_of_a_streamed_product_have_eight_steps_where_that_pays(shape, eight):
     """Both sides of each line: a second round for a few steps, two tiles of tokens with eight wavefronts a unit, more wavefronts than have the registers."""
     assert [per for per in range(1, 40) if library().tm_stream_round(*map(ctypes.c_int, (*shape, per))) == 8] == list(eight)
+
+
+# (rows, columns, K, the first table's tile, the one that runs): a tile between the table's on both sides of what says that it may be taken
+@pytest.mark.parametrize("M,N,K,table,runs", [(264, 7536, 7808, 6, 6), (231, 9096, 1728, 6, 11), (750, 3120, 4416, 6, 6), (3651, 1288, 5248, 5, 5), (3104, 1392, 11392, 5, 5),
+                                              (615, 9832, 1280, 4, 14), (311, 10144, 9920, 6, 6), (287, 11024, 2048, 7, 12), (3562, 544, 1408, 8, 8), (2325, 1160, 384, 10, 11),
+                                              (1605, 3072, 832, 5, 13), (2322, 1672, 1472, 5, 12)])
+def test_tiles_between_are_taken_where_they_pay(M, N, K, table, runs):
+    args = [ctypes.c_int(x) for x in (M, N, K, 1)]
+    assert (library().tm_gemm_tile_shape(*args), library().tm_gemm_tile_picked(*args)) == (table, runs)

@@ -606,10 +606,12 @@ constexpr int GT_N_SHAPES = GT_SHAPES(GT_COUNT), GT_N_ALL = sizeof(gt_shapes) / 
 constexpr int GT_CUS = 256;
 constexpr double GT_BYTES_US = 14e6;        // what the CUs take out of the second-level caches together
 
+static long long gt_tiles(const GtShape& t, int M, int N, int splits) { return (long long)((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN) * splits; }
+
 // Microseconds a launch takes beyond its start: rounds of blocks, or the operands' way into the CUs.
 static double gt_cost(const GtShape& t, int M, int N, int K, int splits) {
     const int per = (K / 64 + splits - 1) / splits;
-    const long long tiles = (long long)((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN) * splits;
+    const long long tiles = gt_tiles(t, M, N, splits);
     const bool pairs = t.OCC > 1 && tiles > GT_CUS;
     const long long slots = pairs ? 2 * GT_CUS : GT_CUS;
     const double compute = (double)((tiles + slots - 1) / slots) * (pairs ? per * t.step2 + t.epi2 : per * t.step + t.epi);
@@ -635,23 +637,43 @@ static int gt_choose(int M, int N, int K, int splits, double* cost = nullptr) {
     return best;
 }
 
+// What part of the table's choice's time by these figures a tile between may take at most to be taken, 0: never. Each is what timings say: 2,200 sizes for which
+// seven hundredths less were enough, at 65 to 4,096 rows, took 0.94 of their former time, but 183 of them 1.02 to 1.36. Those were
+//  - 96 rows for as many rows of tiles of 128 x 128: nothing fewer is multiplied, and the shorter step is not what the operands' way allows (278 sizes, 1.01 on the mean, to
+//    1.19); with more of those 0.92, but where the operands' way is most of the time 1.12 at the worst (0.58 of it at 128 x 128, or 16% cheaper, is where that ends);
+//  - tiles larger than those they stand in for, which had only seemed bound by the operands' way (160 rows for 128 x 128, 10 sizes, 1.31; 96 for 64 x 64, 8 sizes, 1.05;
+//    32 x 64 are, 0.85);
+//  - 224 rows by less than 12% (155 sizes, 0.99, to 1.14).
+// Of 2,200 drawn anew that take one now, 22 take more than 1.02 of their former time, 1.08 at the worst, 0.915 on the mean.
+static double gt_between_line(int i, int table, int M, int N, int K, int splits) {
+    const GtShape &t = gt_shapes[i], &of = gt_shapes[table];
+    const bool wide = of.BN == 128 && of.BM == 128;
+    if (i == 11) {
+        if (table == 8 || (wide && (M + t.BM - 1) / t.BM == (M + of.BM - 1) / of.BM)) return 0;
+        const int per = (K / 64 + splits - 1) / splits;
+        const bool way = (double)gt_tiles(of, M, N, splits) * (of.BM + of.BN) * per * 128 / GT_BYTES_US >= 0.58 * (per * of.step + of.epi);
+        return wide && way ? 0.84 : 0.93;
+    }
+    if (i == 12 && wide) return 0;
+    return i == 14 ? 0.88 : 0.93;
+}
+
 // The tile a launch takes: the table's choice, which also says into how many parts K is cut, or a tile between where that is one round of the chip,
-// at least 7% cheaper by these figures, and not bound by the operands' way into the CUs. 25 matrices (0.5B, 1.5B, 7B and others), 70 to 3,001
-// rows: of 1,000 launches it then takes 129, which last 0.79 to 1.02 of what they did, 0.925 on the mean; nearer lines bring 1% more of that and
-// launches that last 1.05 to 1.3. us: gate|up of the 0.5B shape at 250 rows 128 x 128 13.4, 96 x 128 11.9, at 544 96 x 256 17.1, 192 x 128 15.9, at 640 128 x 256
-// 19.3, 224 x 128 17.6; q|k|v at 2,048 13.2 / 11.3; 1,792 -> q|k|v of 4,608 at 1,024 96 x 256 30.1, 160 x 128 24.2. Every tile adds a row's products in one order.
+// cheaper by these figures (gt_between_line), and not bound by the operands' way into the CUs. us: gate|up of the 0.5B shape at 250 rows 128 x 128 13.4, 96 x 128 11.9,
+// at 544 96 x 256 17.1, 192 x 128 15.9, at 640 128 x 256 19.3, 224 x 128 17.6; q|k|v at 2,048 13.2 / 11.3; 1,792 -> q|k|v of 4,608 at 1,024 96 x 256 30.1, 160 x 128 24.2.
+// Every tile adds a row's products in one order.
 static int gt_pick(int M, int N, int K, int splits) {
-    double least;
-    int best = gt_choose(M, N, K, splits, &least);
-    if (best < 0) return best;
-    least *= 0.93;
+    double table_cost, least = 0;
+    const int table = gt_choose(M, N, K, splits, &table_cost);
+    if (table < 0) return table;
+    int best = table;
     const int per = (K / 64 + splits - 1) / splits;
     for (int i = GT_N_SHAPES; i < GT_N_ALL; ++i) {
         const GtShape& t = gt_shapes[i];
-        const long long tiles = (long long)((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN) * splits;
+        const long long tiles = gt_tiles(t, M, N, splits);
         const double cost = per * t.step + t.epi;
         if (tiles > GT_CUS || !gt_splits_ok(t, K, splits) || (double)tiles * (t.BM + t.BN) * per * 128 / GT_BYTES_US >= 0.92 * cost) continue;
-        if (cost < least) best = i, least = cost;
+        if (cost < gt_between_line(i, table, M, N, K, splits) * table_cost && (best == table || cost < least)) best = i, least = cost;
     }
     return best;
 }
