@@ -30,14 +30,23 @@ def _stream():
     return P(torch.cuda.current_stream().cuda_stream)
 
 
+def _product(what, size):
+    """Rows, columns, K and parts of K of a case of one of the lists."""
+    if what == "qkv":
+        M, H, KVH, D, K, _ = size
+        return M, (H + 2 * KVH) * D, K, 1
+    M, n, K = size
+    return M, 2 * n if what == "silu" else n, K, library().tm_tile_linear_parts(M, n, K) if what == "parts" else 1
+
+
 def test_the_sizes_reach_every_tile_with_every_epilogue():
     lib = library()
     few = [size for size in PARTS if size[0] <= 64 and size[2] >= 320]          # these run one of two tiles of their own
     assert {K // 64 > 200 and N >= 3072 for M, N, K in few} == {True, False}
-    for shapes in ({lib.tm_gemm_tile_shape(M, 2 * n, K, 1) for M, n, K in SILU},
-                   {lib.tm_gemm_tile_shape(M, (H + 2 * KVH) * D, K, 1) for M, H, KVH, D, K, page in QKV},
-                   {lib.tm_gemm_tile_shape(M, N, K, lib.tm_tile_linear_parts(M, N, K)) for M, N, K in PARTS if (M, N, K) not in few}):
-        assert shapes == set(range(11))
+    for what, sizes in (("silu", SILU), ("qkv", QKV), ("parts", [size for size in PARTS if size not in few]), ("linear", [])):
+        sizes = sizes + [size for of, size, _ in BETWEEN if of == what]
+        runs = {lib.tm_gemm_tile_picked(*_product(what, size)) for size in sizes}
+        assert runs >= (set(range(15)) if what != "linear" else set(range(11, 15))), what      # (plain products: test_gpu_tile_ends.py has the others)
 
 
 @pytest.mark.parametrize("M,n,K", SILU)
@@ -204,7 +213,7 @@ def test_the_rows_do_not_change_a_row_of_gate_up_or_of_qkv(dt):
         assert (lib.tm_tile_f32_gate_up_silu if f32 else lib.tm_tile_gate_up_silu)(*lead, P(act.data_ptr()), I(n), _stream()) == 0
         assert (lib.tm_tile_f32_qkv_rope(*lead, P(None), *tail) if f32 else lib.tm_tile_qkv_rope(*lead, P(None), I(-1), *tail)) == 0
         got.append((act, q, k[:M], v[:M]))
-        tiles.add(lib.tm_gemm_tile_shape(M, 2 * n, K, 1))
+        tiles.add(lib.tm_gemm_tile_picked(M, 2 * n, K, 1))
     assert len(tiles) >= 6
     for few in got[1:]:
         assert all(torch.equal(x, y[:x.shape[0]]) for x, y in zip(few, got[0]))
@@ -222,20 +231,32 @@ BETWEEN = [("silu", (804, 2816, 320), 5), ("silu", (321, 4864, 320), 6), ("silu"
 @pytest.mark.parametrize("what,size,tile", BETWEEN)
 def test_tiles_between(what, size, tile):
     """Against 64 bits as above, and a row's bits are those of the calls of fewer rows, which take other tiles."""
-    lib, M, K = library(), size[0], size[4] if what == "qkv" else size[2]
-    N = 2 * size[1] if what == "silu" else (size[1] + 2 * size[2]) * size[3] if what == "qkv" else size[1]
-    parts = lib.tm_tile_linear_parts(M, N, K) if what == "parts" else 1
+    lib = library()
+    M, N, K, parts = _product(what, size)
     assert lib.tm_gemm_tile_picked(M, N, K, parts) == tile
     if what == "qkv":
-        return test_qkv_with_rotation_and_cache_write(*size, torch.float32, True)
+        test_qkv_with_rotation_and_cache_write(*size, torch.float32, True)
     if what == "parts":
-        return test_partial_sums_of_a_split_k(*size)
+        test_partial_sums_of_a_split_k(*size)
     if what == "silu":
         test_gate_up_silu(*size)
     a, w, ref = _operands(M, N, K, M)
     lead = lambda m: (P(a.data_ptr()), I(K), I(m), I(K), P(w.data_ptr()))
 
     def product(m, dt=torch.bfloat16):
+        """A row a token of everything that the call gives."""
+        if what == "qkv":
+            _, H, KVH, D, _, page = size
+            q, (k, v) = torch.full((m, H * D), float("nan"), device="cuda", dtype=dt), torch.zeros(2, -(-M // page), page * KVH * D, device="cuda", dtype=dt)
+            cos, sin = torch.rand(2, M, D // 2, generator=torch.Generator(device="cuda").manual_seed(6), device="cuda")
+            pos = torch.arange(m, device="cuda", dtype=torch.int32)
+            assert lib.tm_tile_qkv_rope(*lead(m), P(None), I(-1), P(q.data_ptr()), I(H), I(KVH), I(D), P(cos.data_ptr()), P(sin.data_ptr()), P(pos.data_ptr()),
+                                        P(pos.data_ptr()), P(k.data_ptr()), P(v.data_ptr()), I(page), _stream()) == 0
+            return torch.cat([q, k.view(-1, KVH * D)[:m], v.view(-1, KVH * D, page).transpose(1, 2).reshape(-1, KVH * D)[:m]], 1)
+        if what == "parts":
+            sums = torch.full((parts, m, N), float("nan"), device="cuda")
+            assert lib.tm_tile_linear_split(*lead(m), I(N), P(sums.data_ptr()), _stream()) == 0
+            return sums.transpose(0, 1)
         out = torch.full((m, size[1]), float("nan"), device="cuda", dtype=dt)
         if what == "silu":
             assert lib.tm_tile_gate_up_silu(*lead(m), P(out.data_ptr()), I(N // 2), _stream()) == 0
@@ -243,8 +264,11 @@ def test_tiles_between(what, size, tile):
             assert lib.tm_tile_linear(*lead(m), I(N), P(out.data_ptr()), I(N), I(1 if dt is torch.bfloat16 else 0), _stream()) == 0
         return out
 
+    # fewer rows, which take other tiles (of the same number of parts of K)
+    few = [77, 300] if what != "parts" else [m for m in range(M - 1, 64, -1) if lib.tm_tile_linear_parts(m, N, K) == parts and lib.tm_gemm_tile_picked(m, N, K, parts) != tile][:2]
     full = product(M)
-    for m in (77, 300):
+    assert few and {lib.tm_gemm_tile_picked(m, N, K, parts) for m in few} != {tile} and not full.isnan().any()
+    for m in few:
         assert torch.equal(product(m), full[:m])
     if what == "linear":
         sums = product(M, torch.float32)

@@ -41,7 +41,9 @@ int tm_gemm_f32_mfma(const float* A, int lda, const float* W, const float* bias,
 // sizes that are multiples of 64) and cache write; 32-bit partial sums [parts][M][N] of a product whose K is split
 // (tm_tile_linear_parts says over how many parts, 0: the library's product is the better one); a plain product in either type.
 int tm_gemm_tile_takes(const void* A, int lda, const void* W, int M, int N, int K);
-int tm_gemm_tile_shape(int M, int N, int K, int splits);        // which of its tiles it runs with (for tests)
+// Which of its tiles it runs with, and which of the first eleven says how K is cut and what the choice costs (for tests).
+int tm_gemm_tile_picked(int M, int N, int K, int splits);
+int tm_gemm_tile_shape(int M, int N, int K, int splits);
 int tm_tile_gate_up_silu(const void* A, int lda, int M, int K, const void* W, void* act, int I, hipStream_t stream);
 int tm_tile_qkv_rope(const void* A, int lda, int M, int K, const void* W, const void* bias, int bias_dtype, void* q, int H, int KVH, int D,
                      const float* cos_t, const float* sin_t, const int* positions, const int* slots, void* k_pool, void* v_pool,
