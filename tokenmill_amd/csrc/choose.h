@@ -107,20 +107,22 @@ inline bool tm_decode_splits(int requests, int kv_heads, int max_context) {
 // the block kernel (one chunk, or 192 pairs and more) it merges in one pass. max_context is the step's: the longest context of an eager step, and
 // of a replayed one the longest that the engine allows (max_model_len), since a graph serves whatever contexts come: with 2,048 allowed no replayed
 // step below 192 pairs takes this kernel (0.5B shape, one request of 300 keys 640 us a step for 613, 64 of up to 1,021 sampled 1,218 for 1,188).
-// Us, split or block kernel to whole, by head size D (seven heads a kv head, or one):
-//   2 to 16 pairs, D 64   100 / 300 / 500 / 700 / 1,000 keys   5.7 / 6.6 / 6.6 / 6.7 / 6.6 to 4.5 / 5.6 / 6.1 / 7.2 / 8.5
-//   16 and 32,     D 128  100 / 300 / 500 / 700                8.6 / 8.8 / 9.0 / 9.4 to 5.2 / 7.6 / 9.3 / 11.4
-//   64,            D 32   300 / 700 / 1,000                    5.8 / 6.3 / 6.4 to 5.0 / 6.1 / 6.9
-//   96,            D 64   300 / 700 / 1,000 / 1,085            7.6 / 9.3 / 9.8 / 10.1 to 6.0 / 7.8 / 9.3 / 10.1
-//   128,           D 64   the same                             8.1 / 10.1 / 10.6 / 12.0 to 6.2 / 8.0 / 9.6 / 10.5
-//   96 and 128,    D 128  300 / 700 / 1,000                    9.7 / 12.8 / 14.2 and 10.1 / 14.2 / 16.1 to 7.8 / 11.7 / 16.6 and 7.9 / 12.2 / 18.5
+// The whole kernel's time over the split kernels', of 1 to 64 requests at 300 / 400 / 512 / 576 / 700 / 768 / 1,024 keys, the least and the most of
+//   1 to 64 pairs, D 32     0.72 to 0.85, 0.73 to 0.85, 0.72 to 0.88, 0.77 to 0.94, 0.77 to 0.96, 0.77 to 1.01, 0.85 to 1.17
+//                  D 64     0.71 to 0.84, 0.73 to 0.87, 0.74 to 0.90, 0.82 to 1.00, 0.87 to 1.04, 0.87 to 1.08, 1.00 to 1.18
+//                  D 96     0.73 to 0.88, 0.79 to 0.92, 0.83 to 1.01, 0.93 to 1.16, 0.99 to 1.22, 1.02 to 1.25, 1.23 to 1.58
+//                  D 128    0.74 to 0.84, 0.81 to 0.98, 0.86 to 1.06, 0.95 to 1.12, 1.03 to 1.23, 1.07 to 1.32, 1.28 to 1.67
+//   96 and 128,    D 32     0.74 to 0.84, 0.75 to 0.84, 0.75 to 0.84, 0.73 to 0.81, 0.78 to 0.87, 0.78 to 0.88, 0.88 to 0.97 (1,280 keys 0.88 to 0.99)
+//                  D 64     0.78 to 0.87, 0.78 to 0.89, 0.79 to 0.90, 0.76 to 0.87, 0.79 to 0.88, 0.81 to 0.92, 0.88 to 1.00 (1,280 keys 0.93 to 1.04)
+//                  D 96     0.79 to 0.89, 0.84 to 0.93, 0.91 to 1.01, 0.82 to 0.91, 0.88 to 0.96, 0.89 to 0.97, 1.10 to 1.21
+//                  D 128    0.81 to 0.90, 0.89 to 0.97, 0.90 to 0.98, 0.80 to 0.89, 0.90 to 0.97, 0.92 to 0.98, 1.08 to 1.18
+// (one, five, seven and 16 heads a kv head; one head is the worst almost everywhere). us, split / whole: one request of 14 heads over 2 of 64, 300 / 700 keys
+// 6.7 / 5.2, 6.8 / 6.7. Below 96 pairs the lines lie lower than these alone say: the split kernels' blocks leave room for matrices to be brought ahead of the
+// products behind them, and the whole kernel's do not. Steps with contexts of up to 630 keys allowed 694, us, split / whole: the 0.5B shape, 1 / 4 / 16 / 40 requests
+// 638 / 659, 658 / 681, 938 / 928, 996 / 992; 7B, of 440 allowed 504, 2 / 12 requests 3,117 / 3,108, 3,207 / 3,198. Against the block kernel, where its keys were loaded in the product's order throughout, by pairs:
 //   256,           D 64   300 / 700 / 1,085                    8.2 / 10.9 / 15.8 to 6.9 / 9.8 / 14.3
 //   192 and 400,   D 128  the same                             11.5 / 17.9 / 25.2 and 21.5 / 34.7 / 46.6 to 8.3 / 14.4 / 21.9 and 14.6 / 27.0 / 40.2
-// and of 16 heads a kv head (of 1, 4 and 8 the same way; 16 pairs of one head of 128 with 400 keys are the worst, 8.4 to 8.5):
-//   4 and 64,      D 128  200 / 400                            9.7 / 9.5 and 10.1 / 10.8 to 7.4 / 9.1 and 7.6 / 9.5
-//   128 and 192,   D 128  400 / 700                            12.5 / 16.3 and 13.1 / 17.8 to 9.8 / 13.0 and 10.4 / 15.2
-//   64 and 128,    D 64   400 / 1,000 (the former 500)         8.0 / 8.3 and 9.8 / 12.3 to 6.2 / 6.6 and 6.5 / 10.0
-//   512,           D 64   400 / 700 / 1,000 / 1,280            12.4 / 20.3 / 27.2 / 32.1 to 11.0 / 18.0 / 25.1 / 32.9 (the last by the block kernel)
+//   512,           D 64   400 / 700 / 1,000 / 1,280, 16 heads a kv head   12.4 / 20.3 / 27.2 / 32.1 to 11.0 / 18.0 / 25.1 / 32.9
 constexpr int TM_DECODE_MANY_PAIRS = 96;
 constexpr int TM_DECODE_WHOLE_KEYS = 1280;
 constexpr size_t TM_DECODE_WHOLE_LDS = 160 * 1024;

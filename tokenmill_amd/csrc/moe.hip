@@ -182,8 +182,9 @@ __global__ __launch_bounds__(MR_THREADS) void moe_route_few_kernel(const int* __
     }
 }
 
-// Otherwise the fewest wavefronts that have a lane an expert and hold the pairs (8 tokens, 64 experts, top 8 in one 3.1 us, in 16 4.4;
-// the one thread's runs and tiles 6.6).
+// Otherwise the fewest wavefronts that have a lane an expert and hold the pairs (8 tokens, 64 experts, top 8 in one 3.1 us, in 16 4.4; the one thread's runs and
+// tiles 6.6, launched again and again). Between fifteen launches of other kernels, the code out of the second-level cache, the one thread's / this, us at 8 / 90 / 400
+// tokens: 17 experts, top 2, 3.0 / 3.2, 3.5 / 3.4, 4.4 / 3.7, 24, 4, 4.1 / 3.2, 4.1 / 3.9, 6.6 / 4.1, 32, 2, 4.0 / 3.1, 4.7 / 3.1, 4.8 / 3.8, 64, 6, 6.6 / 3.2, 7.8 / 3.7, 10.9 / 4.6.
 static int launch_moe_route(const int* ids, const int* table, int T, int top, int E, int real, int tile_rows, int* slot_pair, int* pair_slot,
                             int* tiles, int* n_tiles, hipStream_t stream) {
     static_assert(MOE_MAX_EXPERTS <= MR_THREADS, "");
