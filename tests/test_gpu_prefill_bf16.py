@@ -43,13 +43,13 @@ def test_a_heads_bits_do_not_depend_on_the_heads_beside_it(D, n, window, softcap
 @pytest.mark.parametrize("shared,D,KVH,tiles", [(True, 96, *case) for case in ((4, 64), (4, 65), (3, 86), (2, 255), (3, 170), (4, 128), (3, 171), (16, 47),
                                                                               (257, 1), (257, 2))]
                          + [(False, D, *case) for D in (64, 96) for case in ((4, 65), (4, 108), (4, 109), (4, 128), (4, 129), (4, 217), (3, 87), (257, 2))])
-def test_every_piece_of_a_launch_is_somebodys(shared, D, KVH, tiles):
+def test_every_piece_of_a_launch_is_somebodys(shared, D, KVH, tiles, G=2):
     """From 257 pieces (tile, kv head, its heads) on a launch's blocks take them dealt out over all heads, in reverse among the second 256 (the
     shared-keys kernel), or dealt or a tile from either end of the table (the other): the same bits as calls on parts of the table so few that every
     block takes the piece of its own place."""
     from tokenmill_amd.hip import ops
 
-    G, page, n = 2, 16, 16 * tiles - 3
+    page, n = 16, 16 * tiles - 3
     H = KVH * G
     g = torch.Generator(device=DEV).manual_seed(tiles)
     q = torch.randn(n, H * D, generator=g, device=DEV).to(BF)
@@ -71,6 +71,12 @@ def test_every_piece_of_a_launch_is_somebodys(shared, D, KVH, tiles):
         for t in range(0, tiles, 256 // wide):
             attend(slice(t, t + 256 // wide), heads, part)
         assert torch.equal(part.view(n, -1), dealt.view(n, KVH, -1)[:, lo:heads[1]].reshape(n, -1))
+
+
+@pytest.mark.parametrize("D,KVH,G,tiles", [(96, 1, 10, 257), (96, 1, 10, 400), (128, 2, 16, 256), (128, 1, 9, 513), (96, 2, 5, 200), (128, 4, 7, 128)])
+def test_every_piece_of_a_launch_of_many_heads_is_somebodys(D, KVH, G, tiles):
+    """Blocks of four wavefronts, whose second 256 pieces stand in reverse, and of eight, whose pieces do not."""
+    test_every_piece_of_a_launch_is_somebodys(True, D, KVH, tiles, G)
 
 
 # (head size, kv heads, heads of each, tokens, page, window, softcap, shared keys) and what the bits of the result add up to (bits_of_a_prompt)

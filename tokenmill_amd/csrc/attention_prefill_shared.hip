@@ -219,12 +219,15 @@ __device__ __forceinline__ void attend_shared(const unsigned char* stage, int su
 //                              tokens in the tile (1..16), position of its first token)
 // The table is sorted by the number of keys a tile sees, most first. deal != 0: piece of work w, at place w of the grid's x,
 // is kv head w mod KVH of tile w / KVH, so that the launch as a whole starts with its longest work and each block that
-// ends is followed by the longest that is left; the second 256 pieces, which meet the first on the 256 CUs (a CU holds
-// two blocks), stand in reverse, the shortest of them beside the longest. Measured on an MI355X against blocks that took
+// ends is followed by the longest that is left; of blocks of two and four wavefronts the second 256 pieces, which meet the first on the 256 CUs (a CU holds
+// two of them), stand in reverse, the shortest of them beside the longest. Measured on an MI355X against blocks that took
 // the tiles from both ends of the table in pairs (H 28, KVH 4, D 128; us): 1,500 tokens 65.8 / 56.4, 2,048 78.3 / 74.6, 3,001
-// 138 / 112, 4,096 187 / 186, 6,000 421 / 352, 16,384 2,435 / 2,358; H 40, KVH 8: 1,024 46.3 / 41.0, 3,001 209 / 185 (376 pairs on
-// 512 places leave about half of the CUs a second block and half none); without the reversal 1,500 tokens of the first
-// take 57.8, 4,096 194. Up to 256 blocks there is nothing to deal, and a grid of tiles by kv heads is 2-3% faster (1,024 tokens 38.8 against 40.0).
+// 138 / 112 (376 pairs on 512 places leave about half of the CUs a second block and half none), 4,096 187 / 186, 6,000 421 / 352, 16,384 2,435 / 2,358; H 40, KVH 8:
+// 1,024 46.3 / 41.0, 3,001 209 / 185; without the reversal 1,500 tokens of the first
+// take 57.8, 4,096 194. Of blocks of eight wavefronts a CU holds one, and the longest piece that is left is the right one for the first CU to come free: H 36, KVH 4, D 128,
+// pairs / reversed / not: 1,595 tokens 82.7 / 69.3 / 61.3, 1,915 105 / 95 / 78, 2,075 161 / 109 / 97, 3,595 261 / 238 / 244, but 2,043, where the pairs are
+// 256, 82.4 / 106 / 86.5, and 4,091, where they are 512, 295 / 299 / 303.
+// Up to 256 blocks there is nothing to deal, and a grid of tiles by kv heads is 2-3% faster (1,024 tokens 38.8 against 40.0).
 // query heads a wavefront takes, and wavefronts a SIMD the registers are limited for, by head size
 template <int D> struct SharedPlan { static constexpr int HPW = D <= 64 ? TM_SHARED_HPW64 : 2, WAVES_PER_SIMD = D <= 64 ? TM_SHARED_OCC64 : 2; };
 
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(64 * WAVES, SharedPlan<D>::WAVES_PER_SIMD) void att
     const int G = H / KVH;
     int kvh = blockIdx.y, tile = blockIdx.x;
     if (deal) {
-        if (tile >= 256 && tile < 512) tile = 255 + ((int)gridDim.x < 512 ? (int)gridDim.x : 512) - tile;
+        if (WAVES <= 4 && tile >= 256 && tile < 512) tile = 255 + ((int)gridDim.x < 512 ? (int)gridDim.x : 512) - tile;
         kvh = tile % KVH;
         tile /= KVH;
     }
