@@ -11,11 +11,15 @@ THREADS = 2 ** 32                       # a dimension of a launch has fewer
 # (query heads, kv heads, head size, wavefronts of a block)
 @pytest.mark.parametrize("H,KVH,D,waves", [(2, 1, 128, 2), (28, 4, 128, 4), (40, 8, 128, 4), (16, 1, 96, 8), (48, 4, 128, 8), (12, 2, 64, 4)])
 def test_a_dealt_launch_fits_the_grid(H, KVH, D, waves):
-    """Pieces dealt out stand in the grid's x; tables beyond what that holds are taken by tiles and kv heads, as they were before pieces were dealt."""
+    """Pieces dealt out stand in the grid's x; tables beyond what that holds are taken by tiles and kv heads, as they were before pieces were dealt, or in pairs where
+    eight wavefronts a block fill the chip with them."""
     lib, most = library(), (THREADS // (64 * waves) - 1) // KVH
-    deals = lambda n: lib.tm_attn_prefill_shared_deals(*map(ctypes.c_int, (H, KVH, D, n)))
-    assert deals(256 // KVH) == 0 and deals(256 // KVH + 1) == 1
-    assert deals(most) == 1 and deals(most + 1) == 0 and deals(2 ** 31 - 1) == 0
+    order = lambda n: lib.tm_attn_prefill_shared_order(*map(ctypes.c_int, (H, KVH, D, n)))
+    assert order(256 // KVH) == 0 and order(256 // KVH + 1) == 2
+    for n in [*range(1, 4000, 3), *range(most - 300, most + 300), 2 ** 31 - 1]:
+        folded = -(-n // 2) * KVH
+        pairs = waves == 8 and n * KVH > 256 and 100 * folded >= 97 * 256 * -(-folded // 256)
+        assert order(n) == (1 if pairs else 2 if 256 // KVH < n <= most else 0), n
 
 
 @pytest.mark.parametrize("H,KVH,D,heads,waves", [(14, 2, 64, 4, 8), (16, 16, 64, 1, 8), (32, 8, 128, 2, 4), (12, 2, 96, 2, 4), (640, 320, 64, 1, 8)])

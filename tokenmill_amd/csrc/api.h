@@ -208,9 +208,9 @@ int tm_attn_prefill_shared(const void* q, int q_stride, void* out, int out_strid
                            const void* v_pool, const int* block_tables, int table_width, const int* tiles, int n_tiles,
                            int H, int KVH, int D, int page, float scale, int window, hipStream_t stream);
 int tm_attn_prefill_shared_takes(int H, int KVH, int D);
-// How a launch of either kernel hands out its work (for tests): 1, dealt piece by piece over the grid's x; 0, by tiles and kv heads. Of the first kernel,
-// with `heads` query heads of a kv head a wavefront: 0 by tiles, 1 two tiles a block, 2 dealt.
-int tm_attn_prefill_shared_deals(int H, int KVH, int D, int n_tiles);
+// How a launch of either kernel hands out its work (for tests): 0 by tiles and kv heads, 1 two tiles a block, 2 dealt piece by piece over the grid's x. heads: query
+// heads of a kv head a wavefront of the first kernel takes.
+int tm_attn_prefill_shared_order(int H, int KVH, int D, int n_tiles);
 int tm_attn_prefill_order(int H, int KVH, int D, int heads, int n_tiles);
 
 int tm_gemv_f32(const float* A, int lda, const float* W, const float* bias, float* C, int ldc, int M, int N, int K,

@@ -22,6 +22,7 @@
 #include "attention_prefill_common.h"
 
 #define PS_KEYS 64          // positions per stage
+enum { PS_PLAIN, PS_PAIRS, PS_DEALT };
 #ifndef TM_SHARED_HPW64
 #define TM_SHARED_HPW64 2
 #define TM_SHARED_OCC64 3
@@ -217,7 +218,8 @@ __device__ __forceinline__ void attend_shared(const unsigned char* stage, int su
 
 // tiles: int32 [n_tiles][4] = (request index in the step, first row of the tile in the flat batch,
 //                              tokens in the tile (1..16), position of its first token)
-// The table is sorted by the number of keys a tile sees, most first. deal != 0: piece of work w, at place w of the grid's x,
+// The table is sorted by the number of keys a tile sees, most first. order: a block takes a tile and a kv head by its place in the grid (PS_PLAIN); tile b and then tile
+// n_tiles - 1 - b (PS_PAIRS: the longest with the shortest); or (PS_DEALT) piece of work w, at place w of the grid's x,
 // is kv head w mod KVH of tile w / KVH, so that the launch as a whole starts with its longest work and each block that
 // ends is followed by the longest that is left; of blocks of two and four wavefronts the second 256 pieces, which meet the first on the 256 CUs (a CU holds
 // two of them), stand in reverse, the shortest of them beside the longest. Measured on an MI355X against blocks that took
@@ -225,8 +227,8 @@ __device__ __forceinline__ void attend_shared(const unsigned char* stage, int su
 // 138 / 112 (376 pairs on 512 places leave about half of the CUs a second block and half none), 4,096 187 / 186, 6,000 421 / 352, 16,384 2,435 / 2,358; H 40, KVH 8:
 // 1,024 46.3 / 41.0, 3,001 209 / 185; without the reversal 1,500 tokens of the first
 // take 57.8, 4,096 194. Of blocks of eight wavefronts a CU holds one, and the longest piece that is left is the right one for the first CU to come free: H 36, KVH 4, D 128,
-// pairs / reversed / not: 1,595 tokens 82.7 / 69.3 / 61.3, 1,915 105 / 95 / 78, 2,075 161 / 109 / 97, 3,595 261 / 238 / 244, but 2,043, where the pairs are
-// 256, 82.4 / 106 / 86.5, and 4,091, where they are 512, 295 / 299 / 303.
+// pairs / reversed / not: 1,595 tokens 82.7 / 69.3 / 61.3, 1,915 105 / 95 / 78, 2,075 161 / 109 / 97, 3,595 261 / 238 / 244; but where pairs fill their last round of
+// the chip they are the better ones, a block the less to begin: 2,043 82.4 / 106 / 86.5, 4,091 295 / 299 / 303.
 // Up to 256 blocks there is nothing to deal, and a grid of tiles by kv heads is 2-3% faster (1,024 tokens 38.8 against 40.0).
 // query heads a wavefront takes, and wavefronts a SIMD the registers are limited for, by head size
 template <int D> struct SharedPlan { static constexpr int HPW = D <= 64 ? TM_SHARED_HPW64 : 2, WAVES_PER_SIMD = D <= 64 ? TM_SHARED_OCC64 : 2; };
@@ -235,7 +237,7 @@ template <int D, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, SharedPlan<D>::WAVES_PER_SIMD) void attn_prefill_shared_kernel(
     const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out, int out_stride,
     const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables,
-    int table_width, const int* __restrict__ tiles, int n_tiles, int deal, int H, int KVH, int page_shift,
+    int table_width, const int* __restrict__ tiles, int n_tiles, int order, int H, int KVH, int page_shift,
     float scale_log2, float cap_in, float cap_out, int window, int keep, const float* __restrict__ sink,
     const bf16_t* __restrict__ cgate, int ldcg) {
     constexpr int NDC = D / 32, NDT = D / 16, THREADS = 64 * WAVES, STAGE = SharedShape<D>::STAGE, HPW = SharedPlan<D>::HPW;
@@ -244,7 +246,7 @@ __global__ __launch_bounds__(64 * WAVES, SharedPlan<D>::WAVES_PER_SIMD) void att
     const int tid = threadIdx.x, lane = tid % TM_WAVE, r = lane % 16, g = lane / 16;
     const int G = H / KVH;
     int kvh = blockIdx.y, tile = blockIdx.x;
-    if (deal) {
+    if (order == PS_DEALT) {
         if (WAVES <= 4 && tile >= 256 && tile < 512) tile = 255 + ((int)gridDim.x < 512 ? (int)gridDim.x : 512) - tile;
         kvh = tile % KVH;
         tile /= KVH;
@@ -254,97 +256,105 @@ __global__ __launch_bounds__(64 * WAVES, SharedPlan<D>::WAVES_PER_SIMD) void att
     const unsigned char* kp = (const unsigned char*)k_pool;
     const unsigned char* vp = (const unsigned char*)v_pool;
 
-    const int* tl = tiles + (size_t)tile * 4;
-    const int s = tl[0], row0 = tl[1], valid = tl[2], pos0 = tl[3];
-    const int* table = block_tables + (size_t)s * table_width;
-    const TileView tv = tile_view(pos0, valid, r, window, keep);
-    const int first_key = tv.first_key, sb1 = tv.last_key / PS_KEYS;
-    const int first_tile = first_key / 16, last_tile = tv.last_key / 16;
-    // stages: those of the kept first keys (if there is a gap behind them), then those of the windows
-    const int kept_tiles = first_key > 0 ? (tv.keep + 15) / 16 : 0, kept_stages = first_key > 0 ? (tv.keep + PS_KEYS - 1) / PS_KEYS : 0;
-    const int resume = first_key / PS_KEYS > kept_stages ? first_key / PS_KEYS : kept_stages;
-    const int sb0 = kept_stages > 0 ? 0 : resume;
+    const int other = n_tiles - 1 - tile, n_mine = WAVES == 8 && order == PS_PAIRS && other > tile ? 2 : 1;
 
-    PFrag qf[HPW][NDC];
-#pragma unroll
-    for (int hh = 0; hh < HPW; ++hh)
-#pragma unroll
-        for (int c = 0; c < NDC; ++c) {
-            if (hh < nh && r < valid)
-                qf[hh][c].u = *(const u32x4_t*)(q + (size_t)(row0 + r) * q_stride + (size_t)(h0 + hh) * D + 32 * c + 8 * g);
-            else
-                qf[hh][c].u = u32x4_t{0, 0, 0, 0};
-        }
-    HeadState<D, HPW> st;
-#pragma unroll
-    for (int hh = 0; hh < HPW; ++hh) {
-        st.m[hh] = -INFINITY;
-        st.l[hh] = 0.f;
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) st.o[hh][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
+#pragma unroll 1
+    for (int which = 0; which < n_mine; ++which) {
+        const int* tl = tiles + (size_t)(which ? other : tile) * 4;
+        const int s = tl[0], row0 = tl[1], valid = tl[2], pos0 = tl[3];
+        const int* table = block_tables + (size_t)s * table_width;
+        const TileView tv = tile_view(pos0, valid, r, window, keep);
+        const int first_key = tv.first_key, sb1 = tv.last_key / PS_KEYS;
+        const int first_tile = first_key / 16, last_tile = tv.last_key / 16;
+        // stages: those of the kept first keys (if there is a gap behind them), then those of the windows
+        const int kept_tiles = first_key > 0 ? (tv.keep + 15) / 16 : 0, kept_stages = first_key > 0 ? (tv.keep + PS_KEYS - 1) / PS_KEYS : 0;
+        const int resume = first_key / PS_KEYS > kept_stages ? first_key / PS_KEYS : kept_stages;
+        const int sb0 = kept_stages > 0 ? 0 : resume;
 
-    // The stages take turns in the two halves of LDS: while one is worked on, the next one's keys and values
-    // are on their way into registers, and are stored when the work is done. The load after the last stage
-    // repeats it, unused, so that no load hides behind a branch.
-    int base = sb0;                                              // `places` covers stages base .. base + 15
-    TilePlaces places = lane_places(base, lane, kept_tiles, first_tile, last_tile, table, page_shift, kvh, KVH, D);
-    StageCopy<D, THREADS> copy;
-    copy.load(places, 0, kp, vp, KVH, page_shift, tid);
-    copy.store(stages, tid, tv.keep - sb0 * PS_KEYS, first_key - sb0 * PS_KEYS, tv.last_key + 1 - sb0 * PS_KEYS);
-    __syncthreads();
-    int cur = 0;
-    for (int sb = sb0, next; sb <= sb1; sb = next, cur ^= 1) {
-        next = sb + 1 == kept_stages ? resume : sb + 1;
-        const int ahead = next <= sb1 ? next : sb1;
-        if (ahead - base >= 16) {
-            base = ahead;
-            places = lane_places(base, lane, kept_tiles, first_tile, last_tile, table, page_shift, kvh, KVH, D);
-        }
-        copy.load(places, ahead - base, kp, vp, KVH, page_shift, tid);
-        if (nh > 0) {                                            // wave-uniform
+        PFrag qf[HPW][NDC];
 #pragma unroll
-            for (int sub = 0; sub < 2; ++sub) {
-                const int key0 = sb * PS_KEYS + 32 * sub;
-                if (key0 > tv.last_key || (key0 + 31 < first_key && key0 >= tv.keep)) continue;     // block-uniform: nothing of it is visible
-                attend_shared<D, HPW>(stages + cur * STAGE, sub, st, qf, key0, tv, r, g, scale_log2, cap_in, cap_out);
+        for (int hh = 0; hh < HPW; ++hh)
+#pragma unroll
+            for (int c = 0; c < NDC; ++c) {
+                if (hh < nh && r < valid)
+                    qf[hh][c].u = *(const u32x4_t*)(q + (size_t)(row0 + r) * q_stride + (size_t)(h0 + hh) * D + 32 * c + 8 * g);
+                else
+                    qf[hh][c].u = u32x4_t{0, 0, 0, 0};
             }
+        HeadState<D, HPW> st;
+#pragma unroll
+        for (int hh = 0; hh < HPW; ++hh) {
+            st.m[hh] = -INFINITY;
+            st.l[hh] = 0.f;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) st.o[hh][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
-        copy.store(stages + (cur ^ 1) * STAGE, tid, tv.keep - ahead * PS_KEYS, first_key - ahead * PS_KEYS, tv.last_key + 1 - ahead * PS_KEYS);
+
+        // The stages take turns in the two halves of LDS: while one is worked on, the next one's keys and values
+        // are on their way into registers, and are stored when the work is done. The load after the last stage
+        // repeats it, unused, so that no load hides behind a branch.
+        int base = sb0;                                              // `places` covers stages base .. base + 15
+        TilePlaces places = lane_places(base, lane, kept_tiles, first_tile, last_tile, table, page_shift, kvh, KVH, D);
+        StageCopy<D, THREADS> copy;
+        copy.load(places, 0, kp, vp, KVH, page_shift, tid);
+        copy.store(stages, tid, tv.keep - sb0 * PS_KEYS, first_key - sb0 * PS_KEYS, tv.last_key + 1 - sb0 * PS_KEYS);
         __syncthreads();
-    }
-
-    // every wavefront has its heads' whole result; lane: d = 16 dt + 4 g + i of token r
-#pragma unroll
-    for (int hh = 0; hh < HPW; ++hh) {
-        if (hh >= nh) continue;                                  // wave-uniform
-        float lsum = st.l[hh];
-        lsum = lane_sum<16>(lsum);
-        lsum = lane_sum<32>(lsum);
-        if (r >= valid) continue;
-        if (sink) lsum += __builtin_amdgcn_exp2f(sink[h0 + hh] * 1.4426950408889634f - st.m[hh]);      // a term of the denominator without a key
-        const float inv = 1.f / lsum;
-        bf16_t* orow = out + (size_t)(row0 + r) * out_stride + (size_t)(h0 + hh) * D + 4 * g;
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
-            if (cgate) {                                         // a gate per channel
-                const uint2 gp = *(const uint2*)(cgate + (size_t)(row0 + r) * ldcg + (size_t)(h0 + hh) * D + 4 * g + 16 * dt);
-                st.o[hh][dt][0] *= sigmoid_fast(__uint_as_float(gp.x << 16));
-                st.o[hh][dt][1] *= sigmoid_fast(__uint_as_float(gp.x & 0xffff0000u));
-                st.o[hh][dt][2] *= sigmoid_fast(__uint_as_float(gp.y << 16));
-                st.o[hh][dt][3] *= sigmoid_fast(__uint_as_float(gp.y & 0xffff0000u));
+        int cur = 0;
+        for (int sb = sb0, next; sb <= sb1; sb = next, cur ^= 1) {
+            next = sb + 1 == kept_stages ? resume : sb + 1;
+            const int ahead = next <= sb1 ? next : sb1;
+            if (ahead - base >= 16) {
+                base = ahead;
+                places = lane_places(base, lane, kept_tiles, first_tile, last_tile, table, page_shift, kvh, KVH, D);
             }
-            uint2 pk;
-            pk.x = pk_bf16(st.o[hh][dt][0] * inv, st.o[hh][dt][1] * inv);
-            pk.y = pk_bf16(st.o[hh][dt][2] * inv, st.o[hh][dt][3] * inv);
-            *(uint2*)(orow + 16 * dt) = pk;
+            copy.load(places, ahead - base, kp, vp, KVH, page_shift, tid);
+            if (nh > 0) {                                            // wave-uniform
+#pragma unroll
+                for (int sub = 0; sub < 2; ++sub) {
+                    const int key0 = sb * PS_KEYS + 32 * sub;
+                    if (key0 > tv.last_key || (key0 + 31 < first_key && key0 >= tv.keep)) continue;     // block-uniform: nothing of it is visible
+                    attend_shared<D, HPW>(stages + cur * STAGE, sub, st, qf, key0, tv, r, g, scale_log2, cap_in, cap_out);
+                }
+            }
+            copy.store(stages + (cur ^ 1) * STAGE, tid, tv.keep - ahead * PS_KEYS, first_key - ahead * PS_KEYS, tv.last_key + 1 - ahead * PS_KEYS);
+            __syncthreads();
+        }
+
+        // every wavefront has its heads' whole result; lane: d = 16 dt + 4 g + i of token r
+#pragma unroll
+        for (int hh = 0; hh < HPW; ++hh) {
+            if (hh >= nh) continue;                                  // wave-uniform
+            float lsum = st.l[hh];
+            lsum = lane_sum<16>(lsum);
+            lsum = lane_sum<32>(lsum);
+            if (r >= valid) continue;
+            if (sink) lsum += __builtin_amdgcn_exp2f(sink[h0 + hh] * 1.4426950408889634f - st.m[hh]);      // a term of the denominator without a key
+            const float inv = 1.f / lsum;
+            bf16_t* orow = out + (size_t)(row0 + r) * out_stride + (size_t)(h0 + hh) * D + 4 * g;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+                if (cgate) {                                         // a gate per channel
+                    const uint2 gp = *(const uint2*)(cgate + (size_t)(row0 + r) * ldcg + (size_t)(h0 + hh) * D + 4 * g + 16 * dt);
+                    st.o[hh][dt][0] *= sigmoid_fast(__uint_as_float(gp.x << 16));
+                    st.o[hh][dt][1] *= sigmoid_fast(__uint_as_float(gp.x & 0xffff0000u));
+                    st.o[hh][dt][2] *= sigmoid_fast(__uint_as_float(gp.y << 16));
+                    st.o[hh][dt][3] *= sigmoid_fast(__uint_as_float(gp.y & 0xffff0000u));
+                }
+                uint2 pk;
+                pk.x = pk_bf16(st.o[hh][dt][0] * inv, st.o[hh][dt][1] * inv);
+                pk.y = pk_bf16(st.o[hh][dt][2] * inv, st.o[hh][dt][3] * inv);
+                *(uint2*)(orow + 16 * dt) = pk;
+            }
         }
     }
 }
 
-static bool shared_deals(int n_tiles, int KVH, int waves) {
-    const long long pieces = (long long)n_tiles * KVH;
-    return pieces > 256 && fits_a_dimension(pieces, 64 * waves);
+// Pairs of blocks of eight wavefronts where they fill their last round of the chip; else every piece is dealt that the grid's x holds.
+static int shared_order(int n_tiles, int KVH, int waves) {
+    const long long pieces = (long long)n_tiles * KVH, folded = (long long)(n_tiles / 2 + n_tiles % 2) * KVH;
+    if (pieces <= 256) return PS_PLAIN;
+    if (waves == 8 && 100 * folded >= 97 * 256 * ((folded + 255) / 256)) return PS_PAIRS;
+    return fits_a_dimension(pieces, 64 * waves) ? PS_DEALT : PS_PLAIN;
 }
 
 template <int D, int WAVES>
@@ -360,11 +370,11 @@ static int launch_shared(const void* q, int q_stride, void* out, int out_stride,
             return TM_ERR_LAUNCH;
         raised = true;
     }
-    const int deal = shared_deals(n_tiles, KVH, WAVES);
-    const dim3 grid = deal ? dim3((unsigned)n_tiles * KVH) : dim3(n_tiles, KVH);
+    const int order = shared_order(n_tiles, KVH, WAVES);
+    const dim3 grid = order == PS_DEALT ? dim3((unsigned)n_tiles * KVH) : dim3(order == PS_PAIRS ? n_tiles / 2 + n_tiles % 2 : n_tiles, KVH);
     attn_prefill_shared_kernel<D, WAVES><<<grid, 64 * WAVES, lds, stream>>>(
         (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_tables,
-        table_width, tiles, n_tiles, deal, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
+        table_width, tiles, n_tiles, order, H, KVH, page_shift, scale_log2, cap_in, cap_out, window, keep, sink, cgate, ldcg);
     TM_CHECK_LAUNCH();
     return TM_OK;
 }
@@ -384,9 +394,9 @@ static int shared_waves(int H, int KVH, int D) {
     return need <= 2 ? 2 : need <= 4 ? 4 : 8;
 }
 
-// Are a launch's pieces dealt out over the chip? (for tests)
-extern "C" int tm_attn_prefill_shared_deals(int H, int KVH, int D, int n_tiles) {
-    return n_tiles > 0 && tm_attn_prefill_shared_takes(H, KVH, D) && shared_deals(n_tiles, KVH, shared_waves(H, KVH, D));
+// The order of a launch's pieces (for tests)
+extern "C" int tm_attn_prefill_shared_order(int H, int KVH, int D, int n_tiles) {
+    return n_tiles > 0 && tm_attn_prefill_shared_takes(H, KVH, D) ? shared_order(n_tiles, KVH, shared_waves(H, KVH, D)) : -1;
 }
 
 // softcap > 0: a score s (scaled) becomes softcap * tanh(s / softcap) before the softmax; sink (float32 [H]) or null: one more term
