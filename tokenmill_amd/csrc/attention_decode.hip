@@ -157,8 +157,11 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_block_kernel(
 // ------------------------------------------------------------------------------------------------
 // split kernels: grid (S, KVH, chunks) with four wavefronts, then the merge
 // ------------------------------------------------------------------------------------------------
+// The split and the merge kernel begin at multiples of 8 KiB. The same instructions at other places took 796 to 817 us a step (4 requests of 16,000 keys)
+// and 715 to 726 (8 of 2,048), and the kernels beside them were the slower ones: what fits is that a layer's kernels share the sets of the instruction
+// cache, whose ways are 8 KiB, and drive each other out. Aligned: 796 to 802 and 719 to 721, whatever stands before them in this file.
 template <int D, bool AHEAD>
-__global__ __launch_bounds__(256) void attn_decode_split_kernel(
+__global__ __attribute__((aligned(8192))) __launch_bounds__(256) void attn_decode_split_kernel(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ v_pool, const int* __restrict__ block_tables, int table_width,
     const int* __restrict__ context_lens, float* __restrict__ part_o, float* __restrict__ part_ml,
@@ -233,7 +236,7 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
 // which of them count (scratch memory beyond the context holds anything: it is dropped by selects,
 // never multiplied): one trip to memory for contexts up to 4,096.
 #define AD_MERGE_WAVES 4
-__global__ __launch_bounds__(64 * AD_MERGE_WAVES) void attn_decode_merge_kernel(
+__attribute__((aligned(8192))) __global__ __launch_bounds__(64 * AD_MERGE_WAVES) void attn_decode_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ context_lens,
     bf16_t* __restrict__ out, int out_stride, int max_chunks, int H, int D, int window, int keep, const float* __restrict__ sink,
     const bf16_t* __restrict__ cgate, int ldcg) {
