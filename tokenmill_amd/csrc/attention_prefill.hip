@@ -498,12 +498,12 @@ template <int D> struct PrefillShape { static constexpr int HPW = D <= 64 ? 4 : 
 // Two tiles a block save a block its beginning: the second tile's trips to memory are made while the first one's partials
 // meet. But a pair is as long as the longest tile, and where the pairs do not fill their last round of the 256 CUs, pieces of
 // their own, handed out longest first over all heads, are better balanced by the CUs that come free. us on an MI355X, pairs (below 256 of them:
-// tiles by heads) / dealt: 14 heads over 2 of 64, 1,040 tokens (a fill of 0.52) 14.5 / 14.5, 1,200 (0.59) 17.5 / 16.6, 1,500 (0.73) 22.4 / 19.8,
-// 2,100 (0.52) 38.9 / 31.9, 3,001 (0.73) 51.1 / 46.7, 3,400 (0.84) 57.4 / 57.4, 3,700 (0.91) 61.3 / 63.5, 4,096 (1) 64.9 / 71.5; 32 over 8 of 128, 600
-// (0.59) 33.8 / 26.3, 800 (0.78) 38.3 / 36.2, 900 (0.91) 41.5 / 41.6; 8 over 8 of 64, 1,500 (0.73) 19.0 / 15.7; 12 over 2 of 96, 1,500 (0.55) 41.6 / 30.4.
-// From 218 pairs (0.85) on pairs are better than tiles by heads too (1,900 tokens of the first 26.7 / 23.9), with fewer they are not (1,100
-// tokens 14.6 / 18.8). Head size 32, where a CU holds two blocks, stays with tiles by heads and pairs from 256 on (2,500 tokens of 12
-// heads over 2 26.4 / 28.5 dealt), and up to 256 pieces there is nothing to choose. Pieces that do not fit the grid's x are not dealt.
+// tiles by heads) / dealt: 14 heads over 2 of 64, 1,040 tokens (a fill of 0.52) 13.2 / 13.3, 1,100 (0.55) 12.9 / 13.5, 1,200 (0.59) 16.2 / 15.2, 1,500 (0.73) 20.9 / 18.2,
+// 2,100 (0.52) 37.3 / 29.2, 3,001 (0.73) 48.0 / 43.9, 3,400 (0.84) 52.3 / 53.2, 3,700 (0.91) 55.6 / 58.4, 4,096 (1) 60.9 / 67.9; 32 over 8 of 128, 600
+// (0.59) 30.6 / 24.0, 800 (0.78) 34.2 / 33.8, 900 (0.91) 36.4 / 37.9; 8 over 8 of 64, 1,500 (0.73) 18.5 / 14.9; 12 over 2 of 96, 1,500 (0.55) 36.4 / 27.2.
+// From 218 pairs (0.85) on pairs are better than tiles by heads too (1,740 and 1,900 tokens of the first 24.1 / 20.5, 24.8 / 21.9), with fewer they are not (1,100
+// tokens, as the kernel was before, 14.6 / 18.8). Head size 32, where a CU holds two blocks, stays with tiles by heads and pairs from 256 on (2,500 tokens of 12
+// heads over 2, as it was, 26.4 / 28.5 dealt), and up to 256 pieces there is nothing to choose. Pieces that do not fit the grid's x are not dealt.
 static int prefill_order(int D, int threads, long long pieces, long long folded) {
     if (D < 64 || pieces <= 256 || !fits_a_dimension(pieces, threads)) return folded >= 256 ? PF_PAIRS : PF_PLAIN;
     return 100 * folded < 85 * 256 * ((folded + 255) / 256) ? PF_DEALT : PF_PAIRS;

@@ -112,7 +112,8 @@ __global__ __launch_bounds__(64 * AF_SPLIT, AHEAD ? 2 : 1) void attn_prefill_f32
     };
     auto load = [&](KVBlock32<D>& blk, int b, int pg) {
         const int in_page = ((b <= kb_last ? b : kb_last) << 4) & (page - 1);
-        // keys: lane (r, g) holds K[key0 + r][16 c + 4 g .. + 3]; values: V[d = 16 dt + r][key0 + 4 g .. + 3]
+        // keys: lane (r, g) loads K[key0 + row][16 c + 4 piece .. + 3]; values: V[d = 16 dt + row][key0 + 4 piece .. + 3]. With TURN lane (r, g) holds
+        // row r's piece g behind `turn`, without from the load on
         // (the page's and the key's place by the scalar unit, a lane's own place in them all along the same)
         const auto kr = fd_buffer(k_pool + ((((size_t)pg << page_shift) + in_page) * KVH + kvh) * D, 0x7fffffff);
         const auto vr = fd_buffer(v_pool + ((((size_t)pg * KVH + kvh) * D) << page_shift) + in_page, 0x7fffffff);

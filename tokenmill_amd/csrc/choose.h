@@ -163,7 +163,11 @@ inline bool tm_prefill_takes_decodes(int requests, int heads, int kv_heads, int 
 // short chains: best for short prompts and for small head sizes), and one that stages a tile's keys and values
 // through LDS once for all query heads of a kv head (twice the rate at head sizes above 64 from about a thousand
 // tokens on, where the first is held back by one wavefront a SIMD). The second needs at least three wavefronts'
-// worth of heads (two heads a wavefront) to fill a CU, and a launch of at least a block a CU.
+// worth of heads (two heads a wavefront) to fill a CU, and a launch of at least a block a CU. us, first / second, at 160, 192, 256, 320 and 512 of its blocks:
+// 28 heads over 4 of 128 25.5 / 26.5, 29.1 / 30.0, 38.6 / 37.5, 56.3 / 46.5, 100 / 69; 40 over 8 of 128 15.3 / 16.9, 20.7 / 18.6, 24.9 / 22.4, 32.2 / 26.7, 55.9 / 38.9; 16 over 1
+// of 128 84 / 94, 105 / 111, 168 / 144, 249 / 178, 589 / 301. With two kv heads of five to eight heads the first is, since its keys are loaded as rows, the better one
+// further on (12 over 2 of 96 19.0 / 37.4, 28.3 / 43.7, 38.9 / 56.1, 52.5 / 69.1, 108 / 107; 16 over 2 of 128 33.2 / 44.4, 39.8 / 51.8, 55.3 / 66.2, 82.6 / 81.7, 168 / 126);
+// the line has stayed for what a prompt gives: the two kernels differ by rounding.
 inline bool tm_prefill_shares_keys(int D, int H, int KVH, int n_tiles) {
     const int G = H / KVH;
     return D > 64 && G >= 5 && G <= 16 && (long long)n_tiles * KVH >= 256;
