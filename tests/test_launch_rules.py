@@ -1,8 +1,10 @@
 """How launches hand out their work, as the library says on the host."""
 import ctypes
+import struct
 
 import pytest
 
+from tokenmill_amd.csrc import build
 from tokenmill_amd.hip.library import library
 
 THREADS = 2 ** 32                       # a dimension of a launch has fewer
@@ -69,3 +71,22 @@ def test_rounds_of_a_streamed_product_have_eight_steps_where_that_pays(shape, ei
 def test_tiles_between_are_taken_where_they_pay(M, N, K, table, runs):
     args = [ctypes.c_int(x) for x in (M, N, K, 1)]
     assert (library().tm_gemm_tile_shape(*args), library().tm_gemm_tile_picked(*args)) == (table, runs)
+
+
+def test_the_decode_attentions_pair_of_kernels_begins_at_multiples_of_8_kib():
+    """Where they lie in their code object is worth 2% of a step, so it does not hang on what stands before them. Read from the code objects' symbol tables."""
+    data, found, at = build.find_library().read_bytes(), {}, 0
+    while (at := data.find(b"\x7fELF\x02", at)) >= 0:
+        if struct.unpack_from("<H", data, at + 18)[0] == 224:           # EM_AMDGPU
+            table, = struct.unpack_from("<Q", data, at + 40)
+            size, count = struct.unpack_from("<HH", data, at + 58)
+            sections = [struct.unpack_from("<IIQQQQI", data, at + table + size * i) for i in range(count)]
+            for _, kind, _, _, offset, length, link in sections:
+                for s in range(offset, offset + length, 24) if kind == 11 else ():      # SHT_DYNSYM
+                    name, info, _, _, value, _ = struct.unpack_from("<IBBHQQ", data, at + s)
+                    start = at + sections[link][4] + name
+                    if info & 15 == 2:                                                  # STT_FUNC
+                        found[data[start:data.index(b"\0", start)].decode()] = value
+        at += 4
+    pair = {name: value for name, value in found.items() if "attn_decode_split_kernel" in name or "attn_decode_merge_kernel" in name}
+    assert len(pair) == 4 * 2 + 1 and not any(value % 8192 for value in pair.values()), pair
