@@ -75,6 +75,7 @@ def test_tiles_between_are_taken_where_they_pay(M, N, K, table, runs):
 
 def test_the_decode_attentions_pair_of_kernels_begins_at_multiples_of_8_kib():
     """Where they lie in their code object is worth 2% of a step, so it does not hang on what stands before them. Read from the code objects' symbol tables."""
+    library()                                       # built if it is not there
     data, found, at = build.find_library().read_bytes(), {}, 0
     while (at := data.find(b"\x7fELF\x02", at)) >= 0:
         if struct.unpack_from("<H", data, at + 18)[0] == 224:           # EM_AMDGPU
